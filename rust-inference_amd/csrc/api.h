@@ -263,7 +263,7 @@ int ri_attention_decode_fused_bf16(void* out, float* workspace, const void* qkv,
                                    int seqs, int max_chunks, int heads, int kv_heads, int head_dim, int page_size,
                                    int window, float scale, int tiled_out, void* stream);
 
-// out[M, N] (float32) = x[M, K] (float32) . w[N, K]^T, w float32 or bfloat16; true 32-bit arithmetic.
+// out[M, N] (float32) = x[M, K] (float32) . w[N, K]^T, w float32 or bfloat16; no input is rounded, the sums are float32.
 int ri_gemm_f32(float* out, const float* x, const void* w, int w_dtype, int m, int n, int k, void* stream);
 
 // out[M, N] (out_dtype) = x[M, K] . w[N, K]^T for bfloat16 x and w, float32 accumulation, M <= 8.

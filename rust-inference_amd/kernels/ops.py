@@ -1311,7 +1311,7 @@ def attention_decode_fused_bf16(qkv, q_gain, k_gain, eps, inv_freq, k_pages, v_p
 
 # ---------------------------------------------------------------- products
 def gemm_f32(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """``x @ w.T`` in true 32-bit arithmetic; ``x`` float32 ``[M, K]``, ``w`` float32 or bfloat16 ``[N, K]``."""
+    """``x @ w.T`` with no input rounded and float32 sums; ``x`` float32 ``[M, K]``, ``w`` float32 or bfloat16 ``[N, K]``."""
     m, k = x.shape
     n = w.shape[0]
     out = torch.empty((m, n), dtype=torch.float32, device=x.device)

@@ -632,6 +632,37 @@ def test_gemm_f32_rows_do_not_depend_on_the_batch(ops):
     assert torch.equal(whole[60:], ops.gemm_f32(x[60:].contiguous(), w))
 
 
+@pytest.mark.parametrize("m,n,k", [(1, 37, 72), (33, 129, 192), (65, 130, 64), (65, 16500, 72), (33, 4100, 136)])
+def test_gemm_f32_on_the_matrix_cores(ops, m, n, k):
+    """bfloat16 weights: edges of the tiles of 32 and 64 rows, 32 to 128 columns and stages of 64 k, values over many orders of
+    magnitude.  An additions' chain of k / 32 steps and 32 products a step: (k / 32 + 32) half units of 2^-24 of the sum of
+    magnitudes at most."""
+    if EMULATED and n > 1000:
+        pytest.skip("the larger tiles run on the emulated machine of one unit, at small sizes")
+    rng = np.random.default_rng(m + n + k)
+    x, w = t(rng.normal(size=(m, k)) * 10.0 ** rng.uniform(-6, 6, size=(m, k))), t(rng.normal(size=(n, k)), torch.bfloat16)
+    got = f64(ops.gemm_f32(x, w))
+    bound = (k / 32 + 32) * 2.0 ** -24 * (np.abs(f64(x)) @ np.abs(f64(w)).T)
+    assert (np.abs(got - f64(x) @ f64(w).T) <= bound).all()
+    some = ops.gemm_f32(x[m // 2:].contiguous(), w)
+    assert np.array_equal(got[m // 2:], f64(some)), "a row's sums depend on the other rows"
+
+
+def test_gemm_f32_infinities_and_nan(ops):
+    """Numbers that have no parts: the row of x and the column of the weights they stand in become what multiply-adds make of them."""
+    rng = np.random.default_rng(3)
+    x, w = t(rng.normal(size=(40, 136))), t(rng.normal(size=(50, 136)), torch.bfloat16)
+    clean = f64(ops.gemm_f32(x, w))
+    x[3, 7], x[4, 9], x[5, 0], w[6, 11] = float("inf"), float("nan"), 3.4e38, float("-inf")
+    got, want = f64(ops.gemm_f32(x, w)), f64(x) @ f64(w).T
+    rows, cols = [i for i in range(40) if i not in (3, 4, 5)], [j for j in range(50) if j != 6]
+    assert np.array_equal(got[np.ix_(rows, cols)], clean[np.ix_(rows, cols)])
+    assert np.array_equal(got[3, cols], want[3, cols]) and np.isnan(got[4]).all()
+    assert np.array_equal(np.isnan(got[:, 6]), np.isnan(want[:, 6])) and not np.isfinite(got[:, 6]).any()
+    big = np.abs(want[5, cols]) < 3e38
+    assert np.allclose(got[5, cols][big], want[5, cols][big], rtol=1e-5)
+
+
 def test_gemm_f32_is_true_32_bit(ops):
     """Values that a reduced-precision matrix mode (tf32, bf16 inputs) would round away."""
     x = t([[1.0, 2.0 ** -12, 0.0, 0.0]]).repeat(1, 16)
