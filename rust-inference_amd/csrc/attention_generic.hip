@@ -162,6 +162,175 @@ attention_generic_kernel(TA* __restrict__ out, const TA* __restrict__ q, int q_s
     if (tid + 3 * ATT_TILE < v_dim) from_f32(out + ((size_t)t * heads + h) * v_dim + tid + 3 * ATT_TILE, acc4 / l);
 }
 
+// The same for runs of tokens: a workgroup takes `per` neighbouring tokens and the query heads of one kv head, up to 16 rows of
+// queries that share every key and value it loads; every row's sums are the other kernel's, addition by addition, so that a
+// token's result is the same bits in either.  What bounds the kernel above is that a key row is loaded again for every
+// token and head; here sixteen rows share a load, and what is left is the loads' spread (a lane a key row, a lane a value
+// channel: 64 cache lines a load).  759 tokens of three sequences, 16 heads over 8 of 128, float32: 222 us a layer with the
+// kernel above, 133 with this one.
+// head_dim and the value rows in 16-byte pieces, v_dim <= 512 / SHARES: the rows' weighted sums go to SHARES groups of threads,
+// two channels a thread, so that a weight read from LDS serves two of them; a query read from LDS serves two keys likewise.
+#define ATT_ROWS 16
+template <typename T, int SHARES>
+__global__ void __launch_bounds__(ATT_TILE)
+attention_rows_kernel(T* __restrict__ out, const T* __restrict__ q, int q_stride, const T* __restrict__ k_pages,
+                      const T* __restrict__ v_pages, const int32_t* __restrict__ tok_pos,
+                      const int32_t* __restrict__ tok_seq, const int32_t* __restrict__ page_table, int table_width, int tokens,
+                      int per, int heads, int kv_heads, int head_dim, int v_dim, int page_size, Reach reach, float scale,
+                      float softcap, const float* __restrict__ slopes, int keep_first, const float* __restrict__ sinks) {
+    constexpr int MINE = ATT_ROWS / SHARES;                 // rows whose weighted sums a thread holds
+    extern __shared__ float4 qs4[];                         // ATT_ROWS rows of head_dim floats: the queries
+    float* qs = reinterpret_cast<float*>(qs4);
+    __shared__ float4 ps4[ATT_ROWS][ATT_TILE / 4];          // this tile's weights
+    __shared__ float part[2][ATT_ROWS][ATT_TILE / RI_WAVE];
+    __shared__ float state[3][ATT_ROWS];                    // every row's running maximum, sum and this tile's factor
+    const int tid = threadIdx.x, lane = tid & (RI_WAVE - 1), wave = tid / RI_WAVE;
+    const int kvh = blockIdx.y, group = heads / kv_heads, h0 = kvh * group;
+    const int end = min((int)(blockIdx.x + 1) * per, tokens);
+    const int share = tid / (ATT_TILE / SHARES), d = tid % (ATT_TILE / SHARES);
+    const int row0 = (wave >> 1) * (ATT_ROWS / 2), at = tid & 127;               // scores: half of the rows, two keys of a tile
+    // the tokens of one sequence at a time (a workgroup's tokens are of one sequence nearly always)
+    for (int t0 = blockIdx.x * per, t1; t0 < end; t0 = t1) {
+        const int seq = tok_seq[t0], p0 = tok_pos[t0];
+        for (t1 = t0 + 1; t1 < end && tok_seq[t1] == seq && tok_pos[t1] == p0 + (t1 - t0);) ++t1;
+        const int rows = (t1 - t0) * group, last_pos = p0 + (t1 - 1 - t0);       // row r: token t0 + r / group, head h0 + r % group
+        const int32_t* table = page_table + (size_t)seq * table_width;
+        __syncthreads();
+        for (int e = tid; e < ATT_ROWS * head_dim; e += ATT_TILE) {
+            const int r = e / head_dim, c = e % head_dim;
+            qs[e] = r < rows ? to_f32(q[(size_t)(t0 + r / group) * q_stride + (size_t)(h0 + r % group) * head_dim + c]) : 0.f;
+        }
+        if (tid < ATT_ROWS) { state[0][tid] = -INFINITY; state[1][tid] = 0.f; }
+        __syncthreads();
+        float acc[2][MINE] = {};                            // channels d and d + ATT_TILE / SHARES
+        const int lo_first = reach.first(p0), lo_tile = lo_first / ATT_TILE;       // the first token sees the furthest back
+        const int kept_tiles = (min(keep_first, reach.first(last_pos)) + ATT_TILE - 1) / ATT_TILE;
+        for (int tile = 0; tile <= last_pos / ATT_TILE; ++tile) {
+            if (tile >= kept_tiles && tile < lo_tile) { tile = lo_tile - 1; continue; }
+            const int base = tile * ATT_TILE;
+            float dot[2][ATT_ROWS / 2] = {};                // keys base + at and base + at + 128 with rows row0 ..+ 8
+            const T* kr[2];
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const int j = min(base + at + 128 * u, last_pos);                  // (a key behind the last is read as the last and not seen)
+                kr[u] = k_pages + (((long)table[j / page_size] * kv_heads + kvh) * page_size + j % page_size) * (long)head_dim;
+            }
+            for (int c = 0; c < head_dim; c += Vec<T>::N) {
+                float kv[2][Vec<T>::N];
+                Vec<T>::load(kr[0] + c, kv[0]);
+                Vec<T>::load(kr[1] + c, kv[1]);
+#pragma unroll
+                for (int i = 0; i < ATT_ROWS / 2; ++i)
+#pragma unroll
+                    for (int e = 0; e < Vec<T>::N; e += 4) {
+                        const float4 qv = qs4[((row0 + i) * head_dim + c + e) / 4];
+#pragma unroll
+                        for (int u = 0; u < 2; ++u) {
+                            dot[u][i] += qv.x * kv[u][e]; dot[u][i] += qv.y * kv[u][e + 1];
+                            dot[u][i] += qv.z * kv[u][e + 2]; dot[u][i] += qv.w * kv[u][e + 3];
+                        }
+                    }
+            }
+            uint32_t seen = 0;                               // bit 8 u + i: row row0 + i sees key u of this thread
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int i = 0; i < ATT_ROWS / 2; ++i) {
+                    const int j = base + at + 128 * u, r = row0 + i, qpos = p0 + r / group, lo = reach.first(qpos);
+                    const bool valid = r < rows && (j >= lo || j < min(keep_first, lo)) && j <= qpos;
+                    float s = -INFINITY;
+                    if (valid) {
+                        s = dot[u][i] * scale;
+                        if (softcap > 0.f) s = softcap * tanhf(s / softcap);
+                        if (slopes) s -= slopes[h0 + r % group] * (float)(qpos - j);
+                        seen |= 1u << (8 * u + i);
+                    }
+                    dot[u][i] = s;
+                    const float top = wave_max(s);
+                    if (lane == 0) part[0][r][(wave & 1) + 2 * u] = top;
+                }
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < ATT_ROWS / 2; ++i) {
+                const int r = row0 + i;
+                float m_new = state[0][r];
+#pragma unroll
+                for (int w = 0; w < ATT_TILE / RI_WAVE; ++w) m_new = fmaxf(m_new, part[0][r][w]);
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    const float p = (seen >> (8 * u + i)) & 1 ? expf(dot[u][i] - m_new) : 0.f;
+                    reinterpret_cast<float*>(ps4[r])[at + 128 * u] = p;
+                    const float sum = wave_sum(p);
+                    if (lane == 0) part[1][r][(wave & 1) + 2 * u] = sum;
+                }
+            }
+            __syncthreads();
+            if (tid < ATT_ROWS) {
+                const float m = state[0][tid];
+                float m_new = m, sum = 0.f;
+#pragma unroll
+                for (int w = 0; w < ATT_TILE / RI_WAVE; ++w) {
+                    m_new = fmaxf(m_new, part[0][tid][w]);
+                    sum += part[1][tid][w];
+                }
+                const float corr = m_new > -INFINITY ? expf(m - m_new) : 1.f;      // (a row that has seen no key yet stays as it is)
+                state[1][tid] = state[1][tid] * corr + sum;
+                state[0][tid] = m_new;
+                state[2][tid] = corr;
+            }
+            __syncthreads();
+            if (d < v_dim) {
+                const bool two = d + ATT_TILE / SHARES < v_dim;
+#pragma unroll
+                for (int i = 0; i < MINE; ++i) {
+                    acc[0][i] *= state[2][share * MINE + i];
+                    acc[1][i] *= state[2][share * MINE + i];
+                }
+                const int last = min(last_pos, base + ATT_TILE - 1) - base;
+                for (int j0 = 0; j0 <= last; j0 += 8) {
+                    const int a = base + j0;
+                    float vv[2][8];
+                    const T* vp = v_pages + ((long)table[a / page_size] * kv_heads + kvh) * page_size * (long)v_dim + a % page_size +
+                                  (long)d * page_size;
+#pragma unroll
+                    for (int c = 0; c < 2; ++c) {
+                        const T* vc = vp + (c && two ? (long)(ATT_TILE / SHARES) * page_size : 0);
+                        Vec<T>::load(vc, vv[c]);
+                        if (Vec<T>::N == 4) Vec<T>::load(vc + 4, vv[c] + 4);
+                    }
+#pragma unroll
+                    for (int i = 0; i < MINE; ++i) {
+                        // (the same for the whole share: none of the eight is seen by this row)
+                        const int r = share * MINE + i, qpos = p0 + r / group, b = min(a + 7, qpos);
+                        const int lo = reach.first(qpos);
+                        if (r >= rows || a > qpos || (b < lo && a >= min(keep_first, lo))) continue;
+                        const float4 pa = ps4[r][j0 / 4], pb = ps4[r][j0 / 4 + 1];
+                        const float w[8] = {pa.x, pa.y, pa.z, pa.w, pb.x, pb.y, pb.z, pb.w};
+#pragma unroll
+                        for (int c = 0; c < 2; ++c)
+#pragma unroll
+                            for (int e = 0; e < 8; ++e) acc[c][i] += w[e] * vv[c][e];
+                    }
+                }
+            }
+            __syncthreads();                                 // before the next tile overwrites the weights
+        }
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            const int ch = d + c * (ATT_TILE / SHARES);
+            if (ch >= v_dim) continue;
+#pragma unroll
+            for (int i = 0; i < MINE; ++i) {
+                const int r = share * MINE + i;
+                if (r >= rows) continue;
+                float l = state[1][r];
+                if (sinks) l += expf(sinks[h0 + r % group] - state[0][r]);
+                from_f32(out + ((size_t)(t0 + r / group) * heads + h0 + r % group) * v_dim + ch, acc[c][i] / l);
+            }
+        }
+    }
+}
+
 template <typename T, bool VEC>
 static void launch_attention(void* out, const void* q, int q_stride, const void* k_pages, const void* v_pages,
                              const int32_t* tok_pos, const int32_t* tok_seq, const int32_t* page_table,
@@ -173,11 +342,30 @@ static void launch_attention(void* out, const void* q, int q_stride, const void*
         table_width, heads, kv_heads, head_dim, v_dim, page_size, reach, scale, softcap, slopes, keep_first, sinks);
 }
 
+template <typename T, int SHARES>
+static void launch_rows(void* out, const void* q, int q_stride, const void* k_pages, const void* v_pages, const int32_t* tok_pos,
+                        const int32_t* tok_seq, const int32_t* page_table, int table_width, int tokens, int heads, int kv_heads,
+                        int head_dim, int v_dim, int page_size, Reach reach, float scale, float softcap, const float* slopes,
+                        int keep_first, const float* sinks, hipStream_t s) {
+    const int per = ATT_ROWS / (heads / kv_heads);
+    attention_rows_kernel<T, SHARES><<<dim3((tokens + per - 1) / per, kv_heads), ATT_TILE, (size_t)ATT_ROWS * head_dim * sizeof(float), s>>>(
+        (T*)out, (const T*)q, q_stride, (const T*)k_pages, (const T*)v_pages, tok_pos, tok_seq, page_table, table_width, tokens, per,
+        heads, kv_heads, head_dim, v_dim, page_size, reach, scale, softcap, slopes, keep_first, sinks);
+}
+
+// Whether a step runs by rows of queries: runs of tokens to share keys between, and so many (token, head) pairs that the form
+// with a workgroup for each is past one round of resident workgroups (eight a compute unit).
+static bool attention_by_rows(int most_new, int tokens, int heads, int kv_heads, int head_dim, int v_dim, int page_size, int element) {
+    const int piece = 16 / element, group = heads / kv_heads;
+    return most_new >= 4 && group <= ATT_ROWS && (long)tokens * heads > 8L * ri_compute_units() && head_dim % piece == 0 &&
+           head_dim <= 256 && v_dim <= ATT_TILE && page_size % 8 == 0;
+}
+
 extern "C" int ri_attention_kept(void* out, const void* q, int act_dtype, int q_stride, const void* k_pages,
                             const void* v_pages, int cache_dtype, const int32_t* tok_pos, const int32_t* tok_seq,
                             const int32_t* page_table, int table_width, int tokens, int heads, int kv_heads,
                             int head_dim, int v_dim, int page_size, int window, int chunk, float scale, float softcap,
-                            const float* slopes, int keep_first, const float* sinks, void* stream) {
+                            const float* slopes, int keep_first, const float* sinks, int most_new, void* stream) {
     RI_REQUIRE(chunk >= 0 && (chunk == 0 || window <= 0), "attention: chunks of %d beside a window of %d", chunk, window);
     const Reach reach = {window, chunk};
     RI_REQUIRE(keep_first >= 0, "attention: %d first tokens kept", keep_first);
@@ -199,7 +387,14 @@ extern "C" int ri_attention_kept(void* out, const void* q, int act_dtype, int q_
 #define RI_ATT_GO(T, V) launch_attention<T, V>(out, q, q_stride, k_pages, v_pages, tok_pos, tok_seq, page_table, \
                                                table_width, tokens, heads, kv_heads, head_dim, v_dim, page_size, reach, scale, \
                                                softcap, slopes, window > 0 ? keep_first : 0, sinks, s)
-    if (act_dtype == RI_F32) { if (vec) RI_ATT_GO(float, true); else RI_ATT_GO(float, false); }
+    if (vec && attention_by_rows(most_new, tokens, heads, kv_heads, head_dim, v_dim, page_size, act_dtype == RI_F32 ? 4 : 2)) {
+#define RI_ATT_ROWS(T, S) launch_rows<T, S>(out, q, q_stride, k_pages, v_pages, tok_pos, tok_seq, page_table, table_width, tokens, heads, \
+                                            kv_heads, head_dim, v_dim, page_size, reach, scale, softcap, slopes, \
+                                            window > 0 ? keep_first : 0, sinks, s)
+        if (act_dtype == RI_F32) { if (v_dim <= 128) RI_ATT_ROWS(float, 4); else RI_ATT_ROWS(float, 2); }
+        else                     { if (v_dim <= 128) RI_ATT_ROWS(bf16_t, 4); else RI_ATT_ROWS(bf16_t, 2); }
+#undef RI_ATT_ROWS
+    } else if (act_dtype == RI_F32) { if (vec) RI_ATT_GO(float, true); else RI_ATT_GO(float, false); }
     else                     { if (vec) RI_ATT_GO(bf16_t, true); else RI_ATT_GO(bf16_t, false); }
 #undef RI_ATT_GO
     RI_LAUNCH_CHECK("attention");
@@ -213,5 +408,5 @@ extern "C" int ri_attention(void* out, const void* q, int act_dtype, int q_strid
                             const float* slopes, void* stream) {
     return ri_attention_kept(out, q, act_dtype, q_stride, k_pages, v_pages, cache_dtype, tok_pos, tok_seq, page_table,
                              table_width, tokens, heads, kv_heads, head_dim, v_dim, page_size, window, 0, scale, softcap,
-                             slopes, 0, nullptr, stream);
+                             slopes, 0, nullptr, 1, stream);
 }

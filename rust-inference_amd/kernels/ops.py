@@ -105,7 +105,7 @@ _SIGNATURES = {
                                        c_void_p, c_void_p],
     "ri_attention_kept": [c_void_p, c_void_p, c_int, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int,
                           c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_float, c_void_p, c_int, c_void_p,
-                          c_void_p],
+                          c_int, c_void_p],
     "ri_qk_pairs_norm_kv_write": [c_void_p, c_int, ctypes.c_long, c_int, c_int, c_int, c_void_p, c_int, c_void_p, c_void_p,
                                   c_int, c_float, c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p, c_int, c_void_p,
                                   c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
@@ -528,8 +528,10 @@ def qk_norm_rope_kv_write(qkv, q_gain, k_gain, eps, inv_freq, tok_pos, tok_seq, 
 
 def attention(qkv, k_pages, v_pages, tok_pos, tok_seq, page_table, heads: int, kv_heads: int, head_dim: int,
               window: int | None, scale: float, softcap: float | None = None, slopes: torch.Tensor | None = None,
-              keep_first: int = 0, sinks: torch.Tensor | None = None, q_off: int = 0, chunk: int | None = None) -> torch.Tensor:
+              keep_first: int = 0, sinks: torch.Tensor | None = None, q_off: int = 0, chunk: int | None = None,
+              most_new: int = 1) -> torch.Tensor:
     """Attention of every new token over its sequence's pages; q is the first ``H dh`` columns of ``qkv``.
+    ``most_new``: the most new tokens that any sequence brings (neighbours then share their loads; the results are the same bits).
     With a window, ``keep_first`` first tokens of the sequence stay visible behind it; ``sinks`` (float32 ``[heads]``)
     adds ``exp(sinks[h])`` to the denominator of head ``h``'s softmax.  ``q_off``: the queries' first column in ``qkv``'s rows
     where it is not 0.  ``chunk``: a query sees the keys of its own run of that many positions alone (no window beside it).
@@ -548,7 +550,7 @@ def attention(qkv, k_pages, v_pages, tok_pos, tok_seq, page_table, heads: int, k
           _dev(tok_seq, "tok_seq", torch.int32, (tokens,)), _dev(page_table, "page_table", torch.int32),
           page_table.shape[1], tokens, heads, kv_heads, head_dim, v_dim, k_pages.shape[2], int(window or 0),
           int(chunk or 0), float(scale), float(softcap or 0.0), _opt(slopes, "slopes", torch.float32, (heads,)), int(keep_first or 0),
-          _opt(sinks, "sinks", torch.float32, (heads,)), _stream())
+          _opt(sinks, "sinks", torch.float32, (heads,)), int(most_new), _stream())
     return out
 
 

@@ -344,6 +344,27 @@ def test_attention_prompts_pieces_and_single_tokens(ops, dtype, rel, heads, kv_h
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("heads, kv_heads, dh, vd, form", [(8, 4, 128, 128, "plain"), (10, 2, 24, 40, "window"), (8, 1, 64, 200, "chunk"),
+                                                           (8, 8, 16, 16, "kept"), (24, 2, 32, 128, "plain")])
+def test_attention_rows_of_queries_share_their_loads(ops, dtype, heads, kv_heads, dh, vd, form):
+    """Runs of tokens (whole prompts, the ends of longer sequences, single tokens among them) as rows that share keys: the same
+    bits as a workgroup for every token and head, whatever the mask."""
+    lens, new = ([11, 270, 257], [11, 7, 1]) if EMULATED else ([200, 700, 257, 3, 90], [200, 60, 1, 3, 90])
+    rng = np.random.default_rng(heads + dh)
+    _, _, kp, _, table = paged(rng, lens, kv_heads, dh, dtype=dtype, spare=12)
+    vp = t(rng.normal(size=(kp.shape[0], kv_heads, vd, 32)), dtype)
+    qkv = t(rng.normal(size=(sum(new), heads * dh + 8)), dtype)
+    seq = t([b for b, n in enumerate(new) for _ in range(n)], torch.int32)
+    pos = t([lens[b] - n + i for b, n in enumerate(new) for i in range(n)], torch.int32)
+    more = {"plain": dict(softcap=20.0), "window": dict(slopes=t(rng.uniform(0.01, 0.1, heads))), "chunk": dict(chunk=50),
+            "kept": dict(keep_first=5, sinks=t(rng.normal(size=heads)))}[form]
+    window = {"window": 37, "kept": 270}.get(form)
+    alone, shared = (f64(ops.attention(qkv, kp, vp, pos, seq, table, heads, kv_heads, dh, window, dh ** -0.5, most_new=most, **more))
+                     for most in (1, max(new)))
+    assert np.isfinite(alone).all() and np.array_equal(alone, shared)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_attention_finds_one_far_key_among_hundreds(ops, dtype):
     """One key far back gets a score that stands out: the output must be its value, wherever it lies."""
     rng = np.random.default_rng(9)
