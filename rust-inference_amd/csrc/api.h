@@ -498,8 +498,8 @@ int ri_ssd_scan(float* out, const float* xbc, int channels, int b_off, int c_off
 int ri_ssd_scan_cols_fits(int n, int vdim);
 int ri_ssd_scan_cols(float* out, const float* xbc, int channels, int b_off, int c_off, const void* proj, int act_dtype, int stride,
                      int z_off, int dt_off, const float* dt_bias, const float* a_log, const float* d_skip, float* state,
-                     const int32_t* cu_seqlens, const int32_t* slots, int seqs, int heads, int groups, int n, int vdim,
-                     void* stream);
+                     const int32_t* cu_seqlens, const int32_t* slots, int tokens, int seqs, int heads, int groups, int n,
+                     int vdim, void* stream);
 int ri_group_rms_norm(void* out, int out_dtype, const float* x, const float* gain, float eps, int rows, int width, int parts,
                       void* stream);
 

@@ -14,6 +14,7 @@
 // with one barrier a block.  The same kernel serves a step of one token.
 #include "api.h"
 #include "common.h"
+#include "walk.h"
 
 #define GLA_COLS 16
 #define GLA_SLICES 16
@@ -200,6 +201,80 @@ gla_scan_kernel(float* __restrict__ out, const TA* __restrict__ proj, int row, i
         if (live && j < rows_here) S[(size_t)(row0 + j) * vdim] = s[j];
 }
 
+// Heads of 65 to 128 key channels with a decay per channel: the walk of walk.h, the decays made beforehand.  Three sequences of up to 1,500
+// tokens, 32 heads of 128 x 128: 873 us with a thread on eight rows of a column, 292 with tiles of four rows.
+template <typename TA, int CPL, bool VEC>
+__global__ void __launch_bounds__(256)
+gla_walk_kernel(float* __restrict__ out, const TA* __restrict__ proj, int row, int q_off, int k_off, int v_off,
+                const float* __restrict__ decay, float q_scale, float* __restrict__ state, const int32_t* __restrict__ cu_seqlens,
+                const int32_t* __restrict__ slots, int heads, int dim, int vdim) {
+    constexpr int NC = 8 * CPL;
+    __shared__ float4 qs[2][WALK_BLOCK][WALK_ROWS / 4], ks[2][WALK_BLOCK][WALK_ROWS / 4], as[2][WALK_BLOCK][WALK_ROWS / 4];
+    __shared__ __attribute__((aligned(16))) float vs[2][WALK_BLOCK][NC];
+    const int seq = blockIdx.z, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int slice = lane & 31, row0 = 4 * slice, wcol = wave * 2 * CPL + (lane >> 5) * CPL, first_col = blockIdx.x * NC;
+    const int t0 = cu_seqlens[seq], t1 = cu_seqlens[seq + 1];
+    if (t0 >= t1) return;                                     // (the whole workgroup; the state stays)
+    float* sp = state + (((size_t)slots[seq] * heads + h) * dim) * vdim;
+    float st[4][CPL];
+    walk_load<CPL>(st, sp, row0, dim, first_col + wcol, vdim);
+    const int rtok = tid / 32, rrow = 4 * (tid & 31);         // the thread's piece of q, k and the decay, its element of v
+    const int vtok = tid / NC % WALK_BLOCK, vcol = min(first_col + tid % NC, vdim - 1);
+    struct Ahead { float4 q, k, a; float v; };
+    auto fetch = [&](Ahead& a, int tb) {                      // (always issued, from a token pulled back inside the sequence)
+        const size_t t = (size_t)min(tb + rtok, t1 - 1);
+        a.q = walk_rows<VEC>(proj + t * row + q_off + h * dim, rrow, dim);
+        a.k = walk_rows<VEC>(proj + t * row + k_off + h * dim, rrow, dim);
+        a.a = walk_rows<VEC>(decay + (t * heads + h) * dim, rrow, dim);
+        a.v = to_f32(proj[(size_t)min(tb + vtok, t1 - 1) * row + v_off + h * vdim + vcol]);
+    };
+    auto stage = [&](const Ahead& a, int tb, int buf) {
+        const bool in = tb + rtok < t1;
+        const float4 q = walk_keep(a.q, rrow, dim, in, 0.f);
+        qs[buf][rtok][tid & 31] = make_float4(q.x * q_scale, q.y * q_scale, q.z * q_scale, q.w * q_scale);
+        ks[buf][rtok][tid & 31] = walk_keep(a.k, rrow, dim, in, 0.f);
+        as[buf][rtok][tid & 31] = walk_keep(a.a, rrow, dim, in, 1.f);
+        if (tid < WALK_BLOCK * NC) vs[buf][vtok][tid % NC] = tb + vtok < t1 ? a.v : 0.f;
+    };
+    auto block = [&](int tb, int buf) {
+        float part[WALK_BLOCK * CPL];
+#pragma unroll
+        for (int tt = 0; tt < WALK_BLOCK; ++tt) {
+            const float4 q = qs[buf][tt][slice], k = ks[buf][tt][slice], a = as[buf][tt][slice];
+#pragma unroll
+            for (int j = 0; j < CPL; ++j) {
+                const float v = vs[buf][tt][wcol + j];
+                st[0][j] = a.x * st[0][j] + k.x * v;
+                st[1][j] = a.y * st[1][j] + k.y * v;
+                st[2][j] = a.z * st[2][j] + k.z * v;
+                st[3][j] = a.w * st[3][j] + k.w * v;
+                part[tt * CPL + j] = (st[0][j] * q.x + st[1][j] * q.y) + (st[2][j] * q.z + st[3][j] * q.w);
+            }
+        }
+        const float sum = walk_sum<CPL>(part, lane);
+        const int mine = walk_mine<CPL>(lane), tt = mine / CPL, col = first_col + wcol + mine % CPL;
+        if (mine < WALK_BLOCK * CPL && tb + tt < t1 && col < vdim) out[((size_t)(tb + tt) * heads + h) * vdim + col] = sum;
+    };
+    // two blocks are on their way in registers while a third is computed: a block is computed in less than memory's latency
+    Ahead even, odd;
+    fetch(even, t0);
+    fetch(odd, t0 + WALK_BLOCK);
+    stage(even, t0, 0);
+    __syncthreads();
+    for (int tb = t0; tb < t1; tb += 2 * WALK_BLOCK) {        // (blocks come in pairs)
+        fetch(even, tb + 2 * WALK_BLOCK);
+        block(tb, 0);
+        stage(odd, tb + WALK_BLOCK, 1);
+        __syncthreads();
+        if (tb + WALK_BLOCK >= t1) break;                     // (a step of single tokens is one block)
+        fetch(odd, tb + 3 * WALK_BLOCK);
+        block(tb + WALK_BLOCK, 1);
+        stage(even, tb + 2 * WALK_BLOCK, 0);
+        __syncthreads();
+    }
+    walk_store<CPL>(st, sp, row0, dim, first_col + wcol, vdim);
+}
+
 static int gla_scan_go(float* out, const void* proj, int act_dtype, int row, int q_off, int k_off, int v_off,
                        float* z, const float* z_bias, float tau, float q_scale, float* state,
                        const int32_t* cu_seqlens, const int32_t* slots, int seqs, int tokens, int heads, int dim,
@@ -224,12 +299,28 @@ static int gla_scan_go(float* out, const void* proj, int act_dtype, int row, int
     if (tokens == seqs) nb = 1;
     const size_t lds = (size_t)2 * nb * (3 * dim + GLA_COLS) * sizeof(float);
     // a prompt: the decays of all its tokens in one pass, in place of z, before the walk
+    const bool tiles = !head_decay && dim > 64 && dim <= WALK_ROWS;
     int z_is_decay = 0;
-    if (tokens > seqs && !head_decay) {
+    if ((tokens > seqs || tiles) && !head_decay) {
         const long total = (long)tokens * heads * dim;
         RI_REQUIRE((total + 255) / 256 <= 2147483647L, "gla_scan: %ld decays exceed one launch", total);
         gla_decay_kernel<<<(unsigned)((total + 255) / 256), 256, 0, s>>>(z, z_bias, 1.0f / tau, total, heads * dim);
         z_is_decay = 1;
+    }
+    if (tiles) {
+        const int cpl = walk_columns((long)seqs * heads * vdim, tokens == seqs);
+        const dim3 wgrid((vdim + 8 * cpl - 1) / (8 * cpl), heads, seqs);
+        const bool vec = dim % 4 == 0 && (row | q_off | k_off) % 4 == 0 && ((uintptr_t)proj | (uintptr_t)z) % 16 == 0;
+#define RI_WALK(T, CPL, VEC)                                                                                          \
+    gla_walk_kernel<T, CPL, VEC><<<wgrid, 256, 0, s>>>(out, (const T*)proj, row, q_off, k_off, v_off, z, q_scale, state, cu_seqlens, \
+                                                       slots, heads, dim, vdim)
+#define RI_BY_COLUMNS(T, VEC) if (cpl == 1) RI_WALK(T, 1, VEC); else if (cpl == 2) RI_WALK(T, 2, VEC); else RI_WALK(T, 4, VEC)
+        if (act_dtype == RI_F32) { if (vec) { RI_BY_COLUMNS(float, true); } else { RI_BY_COLUMNS(float, false); } }
+        else                     { if (vec) { RI_BY_COLUMNS(bf16_t, true); } else { RI_BY_COLUMNS(bf16_t, false); } }
+#undef RI_BY_COLUMNS
+#undef RI_WALK
+        RI_LAUNCH_CHECK("gla_scan");
+        return 0;
     }
     // key heads of 64, 128, 256 or 512: a thread's rows are a fixed number, a multiple of 4, read 16 bytes at a time
     const int fixed = (dim == 64 || dim == 128 || dim == 256 || dim == 512) ? dim / GLA_SLICES : 0;

@@ -17,6 +17,7 @@
 // how the tokens were cut into steps.  The same kernels walk a prompt and take a single step.
 #include "api.h"
 #include "common.h"
+#include "walk.h"
 
 #define SSD_MAX_TAPS 16
 
@@ -185,15 +186,15 @@ extern "C" int ri_ssd_scan(float* out, const float* xbc, int channels, int b_off
 }
 
 // ------------------------------------------------------------------ the walk, a wavefront on 16 columns
-// States of up to 128 rows: a wavefront owns 16 columns of one (sequence, head), its lanes four slices of the rows of a
-// column each (8 columns and eight slices for states above 64 rows), the rows in registers; a token's sum over the rows is the lane's own sum (four partial sums, so that no
+// States of up to 64 rows: a wavefront owns 16 columns of one (sequence, head), its lanes four slices of the rows of a
+// column each, the rows in registers; a token's sum over the rows is the lane's own sum (four partial sums, so that no
 // addition waits for the one before) and two exchanges between the lanes of a column.  A workgroup is four wavefronts
 // on columns of their own, which share the tokens staged in LDS in blocks of SSD_BLOCK (B, C, x, the step size and decay, z), the next block's loads asked
 // for before the block in work is computed.  The order of a token's additions is fixed by the sizes alone.
 #define SSD_BLOCK 8
 #define SSD_WAVES 4          // wavefronts of a workgroup: they share the staged tokens, each on columns of its own
 
-template <typename TA, int RPL, int SL>                       // RPL: rows a lane holds, a multiple of 4; SL: slices of rows, 4 or 8
+template <typename TA, int RPL, int SL>                       // RPL: rows a lane holds, a multiple of 4; SL: slices of rows, 4
 __global__ void __launch_bounds__(64 * SSD_WAVES)
 ssd_scan_cols_kernel(float* __restrict__ out, const float* __restrict__ xbc, int channels, int b_off, int c_off,
                      const TA* __restrict__ proj, int stride, int z_off, int dt_off, const float* __restrict__ dt_bias,
@@ -296,8 +297,7 @@ ssd_scan_cols_kernel(float* __restrict__ out, const float* __restrict__ xbc, int
 #pragma unroll
         for (int tt = 0; tt < SSD_BLOCK; ++tt) {
             float y = part[tt];
-            if (SL == 8) y += __shfl_xor(y, 8, RI_WAVE);      // the slices of a column
-            y += __shfl_xor(y, 16, RI_WAVE);
+            y += __shfl_xor(y, 16, RI_WAVE);                  // the slices of a column
             y += __shfl_xor(y, 32, RI_WAVE);
             if (tt < count && has_col && slice == 0) {
                 y += skip * xs[buf][tt][wcol];
@@ -315,29 +315,144 @@ ssd_scan_cols_kernel(float* __restrict__ out, const float* __restrict__ xbc, int
     }
 }
 
+// States of 65 to 128 rows: the walk of walk.h.  2,048 tokens of one sequence, 32 heads of 128 x 128: 1,130 us with a lane on 16
+// rows of a column (its reads of B and C from LDS for one column each), 310 with tiles of four rows.
+template <typename TA, int CPL, bool VEC>
+__global__ void __launch_bounds__(256)
+ssd_walk_kernel(float* __restrict__ out, const float* __restrict__ xbc, int channels, int b_off, int c_off,
+                const TA* __restrict__ proj, int stride, int z_off, int dt_off, const float* __restrict__ dt_bias,
+                const float* __restrict__ a_log, const float* __restrict__ d_skip, float* __restrict__ state,
+                const int32_t* __restrict__ cu_seqlens, const int32_t* __restrict__ slots, int heads, int groups, int n,
+                int vdim) {
+    constexpr int NC = 8 * CPL;
+    __shared__ float4 bs[2][WALK_BLOCK][WALK_ROWS / 4], cs[2][WALK_BLOCK][WALK_ROWS / 4];
+    __shared__ __attribute__((aligned(16))) float xs[2][WALK_BLOCK][NC];
+    __shared__ float zs[2][WALK_BLOCK][NC];
+    __shared__ float dts[2][64], decays[2][64];               // 64 tokens' step sizes and decays, and the next 64's
+    const int seq = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int slice = lane & 31, row0 = 4 * slice, wcol = wave * 2 * CPL + (lane >> 5) * CPL, first_col = blockIdx.z * NC;
+    const int group = h / (heads / groups), inner = heads * vdim;
+    float* sp = state + (((size_t)slots[seq] * heads + h) * n) * vdim;
+    float st[4][CPL];
+    walk_load<CPL>(st, sp, row0, n, first_col + wcol, vdim);
+    const float neg_a = -expf(a_log[h]), skip = d_skip ? d_skip[h] : 0.f, bias = dt_bias ? dt_bias[h] : 0.f;
+    const int t0 = cu_seqlens[seq], t1 = cu_seqlens[seq + 1];
+    if (t0 >= t1) return;                                     // (the whole workgroup; the state stays)
+    const int btok = tid / 32, brow = 4 * (tid & 31);         // the thread's piece of B and C, and its element of x and z
+    const int vtok = tid / NC % WALK_BLOCK, vcol = min(first_col + tid % NC, vdim - 1);
+    struct Ahead { float4 b, c; float x, z; };
+    auto fetch = [&](Ahead& a, int tb) {                      // (always issued, from a token pulled back inside the sequence)
+        const float* row = xbc + (size_t)min(tb + btok, t1 - 1) * channels + group * n;
+        a.b = walk_rows<VEC>(row + b_off, brow, n);
+        a.c = walk_rows<VEC>(row + c_off, brow, n);
+        const int t = min(tb + vtok, t1 - 1);
+        a.x = xbc[(size_t)t * channels + h * vdim + vcol];
+        a.z = to_f32(proj[(size_t)t * stride + z_off + h * vdim + vcol]);
+    };
+    auto stage = [&](const Ahead& a, int tb, int buf) {
+        const bool in = tb + btok < t1;
+        bs[buf][btok][tid & 31] = walk_keep(a.b, brow, n, in, 0.f);
+        cs[buf][btok][tid & 31] = walk_keep(a.c, brow, n, in, 0.f);
+        if (tid < WALK_BLOCK * NC) {
+            xs[buf][vtok][tid % NC] = tb + vtok < t1 ? a.x : 0.f;
+            zs[buf][vtok][tid % NC] = a.z;
+        }
+    };
+    // the step sizes of 64 tokens at once, a lane a token: softplus and the decay's exponential take a wavefront what one token's do
+    auto raw_of = [&](int first) { return to_f32(proj[(size_t)min(first + lane, t1 - 1) * stride + dt_off + h]); };
+    auto put_steps = [&](float raw, int first) {
+        raw += bias;
+        const float dt = raw > 20.f ? raw : log1pf(expf(raw));           // softplus: beyond 20 it is its argument to the last bit
+        const bool in = first + lane < t1;
+        dts[(first - t0) >> 6 & 1][lane] = in ? dt : 0.f;
+        decays[(first - t0) >> 6 & 1][lane] = in ? expf(neg_a * dt) : 1.f;
+    };
+    auto block = [&](int tb, int buf, float raw) {
+        const int at = (tb - t0) & 63, half = (tb - t0) >> 6 & 1;
+        float part[WALK_BLOCK * CPL];
+#pragma unroll
+        for (int tt = 0; tt < WALK_BLOCK; ++tt) {
+            const float dt = dts[half][at + tt], decay = decays[half][at + tt];
+            const float4 b = bs[buf][tt][slice], c = cs[buf][tt][slice];
+#pragma unroll
+            for (int j = 0; j < CPL; ++j) {
+                const float dx = dt * xs[buf][tt][wcol + j];
+                st[0][j] = decay * st[0][j] + b.x * dx;
+                st[1][j] = decay * st[1][j] + b.y * dx;
+                st[2][j] = decay * st[2][j] + b.z * dx;
+                st[3][j] = decay * st[3][j] + b.w * dx;
+                part[tt * CPL + j] = (st[0][j] * c.x + st[1][j] * c.y) + (st[2][j] * c.z + st[3][j] * c.w);
+            }
+        }
+        const float sum = walk_sum<CPL>(part, lane);
+        const int mine = walk_mine<CPL>(lane), tt = mine / CPL, col = wcol + mine % CPL;
+        if (mine < WALK_BLOCK * CPL && tb + tt < t1 && first_col + col < vdim) {
+            const float y = sum + skip * xs[buf][tt][col], z = zs[buf][tt][col];
+            out[(size_t)(tb + tt) * inner + h * vdim + first_col + col] = y * (z / (1.f + expf(-z)));
+        }
+        if (at == 64 - WALK_BLOCK && wave == 0) put_steps(raw, tb + WALK_BLOCK);
+    };
+    // two blocks are on their way in registers while a third is computed: a block is computed in less than memory's latency
+    Ahead even, odd;
+    fetch(even, t0);
+    fetch(odd, t0 + WALK_BLOCK);
+    if (wave == 0) put_steps(raw_of(t0), t0);
+    stage(even, t0, 0);
+    __syncthreads();
+    for (int tb = t0; tb < t1; tb += 2 * WALK_BLOCK) {        // (blocks come in pairs)
+        const float raw = raw_of(t0 + (((tb - t0) >> 6) + 1) * 64);
+        fetch(even, tb + 2 * WALK_BLOCK);
+        block(tb, 0, raw);
+        stage(odd, tb + WALK_BLOCK, 1);
+        __syncthreads();
+        if (tb + WALK_BLOCK >= t1) break;                     // (a step of single tokens is one block)
+        fetch(odd, tb + 3 * WALK_BLOCK);
+        block(tb + WALK_BLOCK, 1, raw);
+        stage(even, tb + 2 * WALK_BLOCK, 0);
+        __syncthreads();
+    }
+    walk_store<CPL>(st, sp, row0, n, first_col + wcol, vdim);
+}
+
 extern "C" int ri_ssd_scan_cols_fits(int n, int vdim) { return n >= 1 && n <= 128 && vdim >= 1; }
 
 extern "C" int ri_ssd_scan_cols(float* out, const float* xbc, int channels, int b_off, int c_off, const void* proj, int act_dtype,
                                 int stride, int z_off, int dt_off, const float* dt_bias, const float* a_log, const float* d_skip,
-                                float* state, const int32_t* cu_seqlens, const int32_t* slots, int seqs, int heads, int groups,
+                                float* state, const int32_t* cu_seqlens, const int32_t* slots, int tokens, int seqs, int heads, int groups,
                                 int n, int vdim, void* stream) {
-    RI_REQUIRE(seqs > 0 && heads > 0 && heads <= 65535 && groups > 0 && heads % groups == 0 && ri_ssd_scan_cols_fits(n, vdim),
+    RI_REQUIRE(tokens >= 0 && seqs > 0 && heads > 0 && heads <= 65535 && groups > 0 && heads % groups == 0 && ri_ssd_scan_cols_fits(n, vdim),
                "ssd_scan_cols: %d sequences, %d heads in %d groups, state %d x %d", seqs, heads, groups, n, vdim);
     RI_REQUIRE(b_off >= 0 && c_off >= 0 && b_off + groups * n <= channels && c_off + groups * n <= channels && heads * vdim <= channels,
                "ssd_scan_cols: columns %d and %d of %d channels", b_off, c_off, channels);
     RI_REQUIRE(z_off >= 0 && dt_off >= 0 && z_off + heads * vdim <= stride && dt_off + heads <= stride,
                "ssd_scan_cols: columns %d and %d of rows of %d", z_off, dt_off, stride);
     RI_REQUIRE(act_dtype == RI_F32 || act_dtype == RI_BF16, "ssd_scan_cols: dtype %d", act_dtype);
-    const int cols = (n > 64 ? 8 : 16) * SSD_WAVES;
+    hipStream_t s = (hipStream_t)stream;
+    if (n > 64) {
+        const int cpl = walk_columns((long)seqs * heads * vdim, tokens == seqs);
+        const dim3 grid(seqs, heads, (vdim + 8 * cpl - 1) / (8 * cpl));
+        RI_REQUIRE(grid.z <= 65535, "ssd_scan_cols: heads of %d channels", vdim);
+        const bool vec = n % 4 == 0 && (channels | b_off | c_off) % 4 == 0 && (uintptr_t)xbc % 16 == 0;
+#define RI_GO(TA, CPL, VEC)                                                                                             \
+    ssd_walk_kernel<TA, CPL, VEC><<<grid, 256, 0, s>>>(out, xbc, channels, b_off, c_off, (const TA*)proj, stride, z_off, dt_off, \
+                                                       dt_bias, a_log, d_skip, state, cu_seqlens, slots, heads, groups, n, vdim)
+#define RI_BY_COLUMNS(TA, VEC) if (cpl == 1) RI_GO(TA, 1, VEC); else if (cpl == 2) RI_GO(TA, 2, VEC); else RI_GO(TA, 4, VEC)
+        if (act_dtype == RI_F32) { if (vec) { RI_BY_COLUMNS(float, true); } else { RI_BY_COLUMNS(float, false); } }
+        else                     { if (vec) { RI_BY_COLUMNS(bf16_t, true); } else { RI_BY_COLUMNS(bf16_t, false); } }
+#undef RI_BY_COLUMNS
+#undef RI_GO
+        RI_LAUNCH_CHECK("ssd_scan_cols");
+        return 0;
+    }
+    const int cols = 16 * SSD_WAVES;
     const dim3 grid(seqs, heads, (vdim + cols - 1) / cols);
     RI_REQUIRE(grid.z <= 65535, "ssd_scan_cols: heads of %d channels", vdim);
-    hipStream_t s = (hipStream_t)stream;
 #define RI_GO(TA, RPL, SL)                                                                                              \
     ssd_scan_cols_kernel<TA, RPL, SL><<<grid, 64 * SSD_WAVES, 0, s>>>(out, xbc, channels, b_off, c_off, (const TA*)proj, stride, z_off,  \
                                                       dt_off, dt_bias, a_log, d_skip, state, cu_seqlens, slots, heads,   \
                                                       groups, n, vdim)
 #define RI_BY_ROWS(TA)                                                                                                  \
-    if (n <= 16) RI_GO(TA, 4, 4); else if (n <= 32) RI_GO(TA, 8, 4); else if (n <= 64) RI_GO(TA, 16, 4); else RI_GO(TA, 16, 8)
+    if (n <= 16) RI_GO(TA, 4, 4); else if (n <= 32) RI_GO(TA, 8, 4); else RI_GO(TA, 16, 4)
     if (act_dtype == RI_F32) { RI_BY_ROWS(float); } else { RI_BY_ROWS(bf16_t); }
 #undef RI_BY_ROWS
 #undef RI_GO

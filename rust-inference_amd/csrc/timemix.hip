@@ -17,6 +17,7 @@
 // were cut into steps.  Any number of new tokens a sequence: the same kernel walks a prompt and takes a single step.
 #include "api.h"
 #include "common.h"
+#include "walk.h"
 
 template <typename TA>
 __global__ void __launch_bounds__(256)
@@ -190,8 +191,8 @@ extern "C" int ri_timemix_scan(void* out, int out_stride, int out_off, float out
 }
 
 // ------------------------------------------------------------------ the walk, a wavefront on 16 columns
-// Heads of up to 128: a wavefront owns 16 columns of one (sequence, head), its lanes four slices of the rows of a column
-// each (8 columns and eight slices for heads above 64: a token's walk over a lane's rows is what the wavefront waits for), the rows in registers; a token's sum over the rows is the lane's own sum (four partial sums, so that no addition
+// Heads of up to 64: a wavefront owns 16 columns of one (sequence, head), its lanes four slices of the rows of a column
+// each, the rows in registers; a token's sum over the rows is the lane's own sum (four partial sums, so that no addition
 // waits for the one before) and two exchanges between the lanes of a column.  A workgroup is four wavefronts on columns of
 // their own, which share the tokens staged in LDS in blocks of TM_BLOCK (r, k, the decay, v), the next block's loads asked for before the block in work is
 // computed.  The heads' results are written as they are, float32; the norm over a head and the gate are
@@ -199,7 +200,7 @@ extern "C" int ri_timemix_scan(void* out, int out_stride, int out_off, float out
 #define TM_BLOCK 8
 #define TM_WAVES 4           // wavefronts of a workgroup: they share the staged tokens, each on columns of its own
 
-template <typename TA, int RPL, int SL>                       // RPL: rows a lane holds, a multiple of 4; SL: slices of rows, 4 or 8
+template <typename TA, int RPL, int SL>                       // RPL: rows a lane holds, a multiple of 4; SL: slices of rows, 4
 __global__ void __launch_bounds__(64 * TM_WAVES)
 timemix_scan_cols_kernel(float* __restrict__ out, const TA* __restrict__ r, const TA* __restrict__ k, const TA* __restrict__ v,
                          const float* __restrict__ z, const float* __restrict__ u,
@@ -297,8 +298,7 @@ timemix_scan_cols_kernel(float* __restrict__ out, const TA* __restrict__ r, cons
 #pragma unroll
         for (int tt = 0; tt < TM_BLOCK; ++tt) {
             float o = part[tt];
-            if (SL == 8) o += __shfl_xor(o, 8, RI_WAVE);      // the slices of a column
-            o += __shfl_xor(o, 16, RI_WAVE);
+            o += __shfl_xor(o, 16, RI_WAVE);                  // the slices of a column
             o += __shfl_xor(o, 32, RI_WAVE);
             if (tt < count && has_col && slice == 0) out[(size_t)(tb + tt) * width + (size_t)h * dim + c] = o;
         }
@@ -310,6 +310,86 @@ timemix_scan_cols_kernel(float* __restrict__ out, const TA* __restrict__ r, cons
         for (int i = 0; i < RPL; ++i)
             if (row0 + i < dim) sp[(size_t)(row0 + i) * dim] = st[i];
     }
+}
+
+// Heads of 65 to 128: the walk of walk.h.  2,048 tokens of one sequence, 8 heads of 128: 1,032 us with a lane on 16 rows of a
+// column, 200 with tiles of four rows.
+template <typename TA, int CPL, bool VEC>
+__global__ void __launch_bounds__(256)
+timemix_walk_kernel(float* __restrict__ out, const TA* __restrict__ r, const TA* __restrict__ k, const TA* __restrict__ v,
+                    const float* __restrict__ z, const float* __restrict__ u, float* __restrict__ state,
+                    const int32_t* __restrict__ cu_seqlens, const int32_t* __restrict__ slots, int heads, int dim) {
+    constexpr int NC = 8 * CPL;
+    __shared__ float4 rs[2][WALK_BLOCK][WALK_ROWS / 4], ks[2][WALK_BLOCK][WALK_ROWS / 4], ws[2][WALK_BLOCK][WALK_ROWS / 4];
+    __shared__ __attribute__((aligned(16))) float vs[2][WALK_BLOCK][NC];
+    const int seq = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int slice = lane & 31, row0 = 4 * slice, wcol = wave * 2 * CPL + (lane >> 5) * CPL, first_col = blockIdx.z * NC;
+    const int width = heads * dim;
+    float* sp = state + (((size_t)slots[seq] * heads + h) * dim) * dim;
+    float st[4][CPL], ub[4];
+    walk_load<CPL>(st, sp, row0, dim, first_col + wcol, dim);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) ub[i] = u[h * dim + min(row0 + i, dim - 1)];
+    const int t0 = cu_seqlens[seq], t1 = cu_seqlens[seq + 1];
+    const int rtok = tid / 32, rrow = 4 * (tid & 31);         // the thread's piece of r, k and the decay, its element of v
+    const int vtok = tid / NC % WALK_BLOCK, vcol = min(first_col + tid % NC, dim - 1);
+    if (t0 >= t1) return;                                     // (the whole workgroup; the state stays)
+    struct Ahead { float4 r, k, w; float v; };
+    auto fetch = [&](Ahead& a, int tb) {                      // (always issued, from a token pulled back inside the sequence)
+        const size_t at = (size_t)min(tb + rtok, t1 - 1) * width + (size_t)h * dim;
+        a.r = walk_rows<VEC>(r + at, rrow, dim);
+        a.k = walk_rows<VEC>(k + at, rrow, dim);
+        a.w = walk_rows<VEC>(z + at, rrow, dim);              // the decay itself: timemix_decay has been over z
+        a.v = to_f32(v[(size_t)min(tb + vtok, t1 - 1) * width + (size_t)h * dim + vcol]);
+    };
+    auto stage = [&](const Ahead& a, int tb, int buf) {
+        const bool in = tb + rtok < t1;
+        rs[buf][rtok][tid & 31] = walk_keep(a.r, rrow, dim, in, 0.f);
+        ks[buf][rtok][tid & 31] = walk_keep(a.k, rrow, dim, in, 0.f);
+        ws[buf][rtok][tid & 31] = walk_keep(a.w, rrow, dim, in, 1.f);
+        if (tid < WALK_BLOCK * NC) vs[buf][vtok][tid % NC] = tb + vtok < t1 ? a.v : 0.f;
+    };
+    auto block = [&](int tb, int buf) {
+        float part[WALK_BLOCK * CPL];
+#pragma unroll
+        for (int tt = 0; tt < WALK_BLOCK; ++tt) {
+            const float4 r4 = rs[buf][tt][slice], k4 = ks[buf][tt][slice], w4 = ws[buf][tt][slice];
+            const float rr[4] = {r4.x, r4.y, r4.z, r4.w}, kk[4] = {k4.x, k4.y, k4.z, k4.w}, ww[4] = {w4.x, w4.y, w4.z, w4.w};
+#pragma unroll
+            for (int j = 0; j < CPL; ++j) {
+                const float vc = vs[buf][tt][wcol + j];
+                float o[2] = {0.f, 0.f};
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float kv = kk[i] * vc;
+                    o[i >> 1] += (st[i][j] + ub[i] * kv) * rr[i];
+                    st[i][j] = ww[i] * st[i][j] + kv;
+                }
+                part[tt * CPL + j] = o[0] + o[1];
+            }
+        }
+        const float sum = walk_sum<CPL>(part, lane);
+        const int mine = walk_mine<CPL>(lane), tt = mine / CPL, col = first_col + wcol + mine % CPL;
+        if (mine < WALK_BLOCK * CPL && tb + tt < t1 && col < dim) out[(size_t)(tb + tt) * width + (size_t)h * dim + col] = sum;
+    };
+    // two blocks are on their way in registers while a third is computed: a block is computed in less than memory's latency
+    Ahead even, odd;
+    fetch(even, t0);
+    fetch(odd, t0 + WALK_BLOCK);
+    stage(even, t0, 0);
+    __syncthreads();
+    for (int tb = t0; tb < t1; tb += 2 * WALK_BLOCK) {        // (blocks come in pairs)
+        fetch(even, tb + 2 * WALK_BLOCK);
+        block(tb, 0);
+        stage(odd, tb + WALK_BLOCK, 1);
+        __syncthreads();
+        if (tb + WALK_BLOCK >= t1) break;                     // (a step of single tokens is one block)
+        fetch(odd, tb + 3 * WALK_BLOCK);
+        block(tb + WALK_BLOCK, 1);
+        stage(even, tb + 2 * WALK_BLOCK, 0);
+        __syncthreads();
+    }
+    walk_store<CPL>(st, sp, row0, dim, first_col + wcol, dim);
 }
 
 // out[t, out_off + h * dim + c] = scale * o[t, h, c] / sqrt(mean_c(o[t, h, :]^2) + eps) * gain[h * dim + c] * silu(g[t, h * dim + c]).
@@ -346,8 +426,9 @@ extern "C" int ri_timemix_scan_cols(void* out, int out_stride, int out_off, floa
                "timemix_scan_cols: %d tokens of %d sequences, %d heads of %d", tokens, seqs, heads, dim);
     RI_REQUIRE(out_off >= 0 && out_off + heads * dim <= out_stride, "timemix_scan_cols: column %d of rows of %d", out_off, out_stride);
     RI_REQUIRE(act_dtype == RI_F32 || act_dtype == RI_BF16, "timemix_scan_cols: dtype %d", act_dtype);
-    const int cols = (dim > 64 ? 8 : 16) * TM_WAVES;
+    const int cpl = walk_columns((long)seqs * heads * dim, tokens == seqs), cols = dim > 64 ? 8 * cpl : 16 * TM_WAVES;
     const dim3 grid(seqs, heads, (dim + cols - 1) / cols);
+    const bool vec = dim % 4 == 0 && ((uintptr_t)r | (uintptr_t)k | (uintptr_t)z) % 16 == 0;
     hipStream_t s = (hipStream_t)stream;
     const long total = (long)tokens * heads * dim;
     RI_REQUIRE((total + 255) / 256 <= 2147483647L, "timemix_scan_cols: %ld decays exceed one launch", total);
@@ -355,18 +436,25 @@ extern "C" int ri_timemix_scan_cols(void* out, int out_stride, int out_off, floa
 #define RI_GO(TA, ROWS, SL)                                                                                             \
     timemix_scan_cols_kernel<TA, ROWS, SL><<<grid, 64 * TM_WAVES, 0, s>>>(o, (const TA*)r, (const TA*)k, (const TA*)v, z, u, state,  \
                                                            cu_seqlens, slots, heads, dim)
+#define RI_WALK(TA, CPL, VEC)                                                                                           \
+    timemix_walk_kernel<TA, CPL, VEC><<<grid, 256, 0, s>>>(o, (const TA*)r, (const TA*)k, (const TA*)v, z, u, state, cu_seqlens, \
+                                                           slots, heads, dim)
+#define RI_BY_COLUMNS(TA, VEC) if (cpl == 1) RI_WALK(TA, 1, VEC); else if (cpl == 2) RI_WALK(TA, 2, VEC); else RI_WALK(TA, 4, VEC)
 #define RI_BY_ROWS(TA)                                                                                                  \
-    if (dim <= 16) RI_GO(TA, 4, 4); else if (dim <= 32) RI_GO(TA, 8, 4); else if (dim <= 64) RI_GO(TA, 16, 4); else RI_GO(TA, 16, 8)
+    if (dim <= 16) RI_GO(TA, 4, 4); else if (dim <= 32) RI_GO(TA, 8, 4); else if (dim <= 64) RI_GO(TA, 16, 4);             \
+    else if (vec) { RI_BY_COLUMNS(TA, true); } else { RI_BY_COLUMNS(TA, false); }
     if (act_dtype == RI_F32) {
-        RI_BY_ROWS(float);
+        RI_BY_ROWS(float)
         heads_norm_gate_kernel<float><<<dim3(tokens, heads), 64, 0, s>>>((float*)out, out_stride, out_off, out_scale, o, gain,
                                                                         (const float*)g, eps, heads, dim);
     } else {
-        RI_BY_ROWS(bf16_t);
+        RI_BY_ROWS(bf16_t)
         heads_norm_gate_kernel<bf16_t><<<dim3(tokens, heads), 64, 0, s>>>((bf16_t*)out, out_stride, out_off, out_scale, o, gain,
                                                                          (const bf16_t*)g, eps, heads, dim);
     }
 #undef RI_BY_ROWS
+#undef RI_BY_COLUMNS
+#undef RI_WALK
 #undef RI_GO
     RI_LAUNCH_CHECK("timemix_scan_cols");
     return 0;

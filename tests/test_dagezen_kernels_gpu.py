@@ -373,3 +373,98 @@ def test_talking_attention_on_the_matrix_cores_is_the_general_kernel(ops, heads,
         got = ops.talking_attention_mfma(proj, 8, k_pages, v_pages, tok_pos, cu, counts, table, heads, kv_heads, dim, window, 0.2,
                                          a, b, c)
         close(got, f64(want), 1.5e-2, "matrix cores against the general kernels")
+
+
+# ---------------------------------------------------------------- the walks over states of 65 to 128 rows
+@pytest.mark.parametrize("kind", ["ssd", "timemix", "gla"])
+@pytest.mark.parametrize("rows, cols, heads, many", [(65, 65, 2, False), (100, 33, 2, False), (128, 40, 1, False), (128, 128, 33, True)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_walks_in_tiles_of_four_rows(ops, kind, rows, cols, heads, many, dtype):
+    """Sequences that end inside a block of eight tokens, at its end and past 64 and 128 tokens, whole against the sums in 64 bits and
+    cut anywhere against whole (the same bits).  A sum runs over `rows` products and as many steps of the state as its decay
+    lets through (under ten here): (rows / 4 + 5 + 2 x 10) roundings of half a unit, against the largest result."""
+    if kind == "timemix":
+        cols = rows
+    lens = [150, 64, 17, 9, 1] if many or not EMULATED else [70, 8, 1]
+    if many and EMULATED:
+        pytest.skip("thousands of columns: minutes when emulated")
+    if many:
+        lens = lens * 2                                       # more columns than the wavefronts of one or two a lane
+    rng = np.random.default_rng(rows + cols)
+    total, slots = sum(lens), rng.permutation(len(lens))
+    width, wv = heads * rows, heads * cols
+    a, b = (rng.standard_normal((total, heads, rows)) for _ in range(2))           # read by the results, written into the state
+    v = rng.standard_normal((total, heads, cols))
+    rounded = lambda x: f64(t(x, dtype)) if kind != "ssd" else f64(t(x))
+    a, b, v = rounded(a), rounded(b), rounded(v)
+    s0 = f64(t(rng.standard_normal((len(lens), heads, rows, cols))))
+    raw = f64(t(rng.standard_normal((total, heads)), dtype))
+    z = f64(t(rng.standard_normal((total, heads, rows)) - (1 if kind == "timemix" else 0)))
+    u = f64(t(rng.standard_normal((heads, rows))))
+    if kind == "ssd":
+        dt = np.logaddexp(0.0, raw)
+        decay, b64 = np.exp(-dt)[..., None] * np.ones(rows), b * dt[..., None]
+        gate = f64(t(rng.standard_normal((total, heads, cols)), dtype))
+    elif kind == "timemix":
+        decay, b64 = np.exp(-np.exp(z)), b
+    else:
+        decay, b64 = (1.0 / (1.0 + np.exp(-z))) ** 0.5, b
+    want, at = np.zeros((total, heads, cols)), 0
+    end = np.zeros_like(s0)
+    for i, n in enumerate(lens):
+        s = s0[slots[i]].copy()
+        for k in range(at, at + n):
+            kv = b64[k][:, :, None] * v[k][:, None, :]
+            if kind == "timemix":
+                want[k] = np.einsum("hrc,hr->hc", s + u[:, :, None] * kv, a[k])
+                s = decay[k][:, :, None] * s + kv
+            else:
+                s = decay[k][:, :, None] * s + kv
+                want[k] = np.einsum("hrc,hr->hc", s, a[k])
+        end[slots[i]] = s
+        at += n
+    if kind == "ssd":
+        want *= gate / (1.0 + np.exp(-gate))
+
+    def run(pieces):
+        """Every sequence's tokens in the given number of steps."""
+        state = t(s0)
+        got, done = np.zeros_like(want), [0] * len(lens)
+        starts = np.concatenate([[0], np.cumsum(lens)])
+        for p in range(pieces):
+            take = [(i, starts[i] + done[i], starts[i] + (n * (p + 1)) // pieces) for i, n in enumerate(lens)]
+            take = [(i, x, y) for i, x, y in take if y > x]
+            rows_of = np.concatenate([np.arange(x, y) for _, x, y in take])
+            for i, x, y in take:
+                done[i] += y - x
+            cu = t(np.concatenate([[0], np.cumsum([y - x for _, x, y in take])]), torch.int32)
+            sl = t([slots[i] for i, _, _ in take], torch.int32)
+            m = len(rows_of)
+            if kind == "ssd":
+                xbc = t(np.concatenate([v[rows_of].reshape(m, -1), b[rows_of].reshape(m, -1), a[rows_of].reshape(m, -1)], 1))
+                proj = t(np.concatenate([gate[rows_of].reshape(m, -1), raw[rows_of]], 1), dtype)
+                zero = t(np.zeros(heads))
+                o = ops.ssd_scan(xbc, wv, wv + width, proj, 0, wv, zero, zero, None, state, cu, sl, heads, heads, rows, cols)
+            elif kind == "timemix":
+                out = guarded(torch.zeros((m, width), dtype=dtype, device=DEV))
+                gates = t(np.full((m, width), 30.0), dtype)                        # silu(30) = 30
+                r_, k_, v_ = (t(x[rows_of].reshape(m, -1), dtype) for x in (a, b, v))
+                ops.timemix_scan(out, 0, 1.0, r_, k_, v_, gates, t(z[rows_of].reshape(m, -1)), t(np.zeros(width)), t(u.reshape(-1)),
+                                 t(np.ones(width)), 0.0, state, cu, sl, heads, rows)
+                o = out
+            else:
+                proj = t(np.concatenate([x[rows_of].reshape(m, -1) for x in (a, b, v)], 1), dtype)
+                o = ops.gla_scan(proj, 0, width, 2 * width, t(z[rows_of].reshape(m, -1)), None, 2.0, 1.0, state, cu, sl, heads, rows, cols)
+            got[rows_of] = f64(o).reshape(m, heads, cols)
+        return got, f64(state)
+
+    if kind == "timemix":
+        want = want / np.sqrt((want * want).mean(-1, keepdims=True)) * 30.0
+    whole, state = run(1)
+    bound = (rows / 4 + 25) * 2.0 ** -24 * 4                  # (four: the largest result beside the largest term of its sum)
+    assert np.abs(state - end).max() <= bound * np.abs(end).max()
+    if kind == "timemix" and dtype == torch.bfloat16:
+        bound = 2.0 ** -8                                     # the normed heads are written in bfloat16
+    assert np.abs(whole - want).max() <= bound * np.abs(want).max()
+    cut, cut_state = run(3)
+    assert np.array_equal(cut, whole) and np.array_equal(cut_state, state)
