@@ -465,7 +465,7 @@ int ri_talking_attention_mfma(void* out, float* stats, const void* q, int q_stri
                               const void* v_pages, const int32_t* tok_pos, const int32_t* cu_seqlens, int seqs,
                               const int32_t* page_table, int table_width, int tiles, int heads, int kv_heads, int dim,
                               int page_size, int window, float scale, const float* r1, const float* r2, const float* talk,
-                              void* stream);
+                              float* bias, float* parts, int shares, int tokens, void* stream);
 
 // ---- time mixing (timemix.hip)
 int ri_shift_mix(void* out, int out_dtype, const float* x, const float* kept, const float* mu, int n_mix,

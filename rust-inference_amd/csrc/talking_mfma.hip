@@ -12,7 +12,13 @@
 // The key rows of a half page are permuted (row r of the first half is key 8 (r / 4) + r % 4, of the second that plus
 // 4), so that a lane's eight scores are eight neighbouring keys, which is how the value product wants its weights.
 // Scores, the logarithm, maxima, sums, the weights before and after the mix and the accumulators are float32.  A token's
-// sums run over its sequence's pages in order, whatever else the step holds.
+// sums run over its sequence's pages in order, whatever else the step holds, or over equal parts of them that are added.
+//
+// The distance bias of a windowed head is a number a distance: a table of window + 16 entries a head is made first, by the
+// same logarithm, and both walks read eight neighbouring entries of it for their eight keys (a logarithm a score was half
+// of what the walks took).  The second walk of a step with fewer tiles than compute units cuts every tile's pages into
+// shares, whose float32 results are added.  2,048 tokens, 32 heads of 128 over 8, a window of 1,024, us: first walk 283 ->
+// 133, second 950 -> 395 with the adding.
 #include "api.h"
 #include "common.h"
 
@@ -46,37 +52,57 @@ __device__ __forceinline__ bool tile_of(int index, const int32_t* __restrict__ c
     return false;
 }
 
+// table[h][8 + gap] = r1_h log(1 + r2_h gap) for gaps -8 .. window + 7 (those outside 0 .. window - 1 are read and not used).
+__global__ void __launch_bounds__(256)
+talking_bias_kernel(float* __restrict__ table, const float* __restrict__ r1, const float* __restrict__ r2, int heads, int window) {
+    const int e = blockIdx.x * 256 + threadIdx.x, span = window + 16;
+    if (e >= heads * span) return;
+    const int h = e / span;
+    table[e] = r1[h] * log1pf(r2[h] * (float)max(e % span - 8, 0));
+}
+
+struct __attribute__((packed, aligned(4))) TmEight { float v[8]; };
+
 // The eight scores of a lane (column = token, keys key0 .. key0 + 7) of head h for one page: raw products times the scale,
 // minus the distance bias, minus infinity where the token does not see the key.
-template <int KS>
+// TABLE: `bias` is the head's row of the table of distances, its entry for a gap of 0.
+template <int KS, bool TABLE>
 __device__ __forceinline__ void talking_scores(float (&s)[8], const TmFrag (&qf)[KS], const bf16_t* __restrict__ kp, int dim,
-                                               float scale, float b1, float b2, bool biased, int qpos, int lo, int key0) {
+                                               float scale, float b1, float b2, bool biased, int qpos, int lo, int key0,
+                                               const float* __restrict__ bias, int window) {
+    TmEight by_gap;                                            // of the gaps from the last of the eight keys up to the first's
+    TmFrag k0[KS], k1[KS];
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+        k0[ks].u = *reinterpret_cast<const uint4*>(kp + ks * 32);
+        k1[ks].u = *reinterpret_cast<const uint4*>(kp + 4 * dim + ks * 32);
+    }
+    if (TABLE) by_gap = *reinterpret_cast<const TmEight*>(bias + min(max(qpos - key0 - 7, -8), window));
+    __builtin_amdgcn_sched_barrier(0);                         // every load is asked for before the first is waited for
     tm_floatx4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
-        TmFrag k0, k1;
-        k0.u = *reinterpret_cast<const uint4*>(kp + ks * 32);
-        k1.u = *reinterpret_cast<const uint4*>(kp + 4 * dim + ks * 32);
-        s0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k0.v, qf[ks].v, s0, 0, 0, 0);
-        s1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k1.v, qf[ks].v, s1, 0, 0, 0);
+        s0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k0[ks].v, qf[ks].v, s0, 0, 0, 0);
+        s1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k1[ks].v, qf[ks].v, s1, 0, 0, 0);
     }
     const float raw[8] = {s0[0], s0[1], s0[2], s0[3], s1[0], s1[1], s1[2], s1[3]};
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
         const int key = key0 + e;
         float v = raw[e] * scale;
-        if (biased) v -= b1 * log1pf(b2 * (float)max(qpos - key, 0));
+        if (TABLE) v -= by_gap.v[7 - e];
+        else if (biased) v -= b1 * log1pf(b2 * (float)max(qpos - key, 0));
         s[e] = (key > qpos || key < lo) ? -INFINITY : v;
     }
 }
 
-template <int KS>
+template <int KS, bool TABLE>
 __global__ void __launch_bounds__(64)
 talking_stats_mfma_kernel(float* __restrict__ stats, const bf16_t* __restrict__ q, int q_stride, int q_off,
                           const bf16_t* __restrict__ k_pages, const int32_t* __restrict__ tok_pos,
                           const int32_t* __restrict__ cu_seqlens, int seqs, const int32_t* __restrict__ page_table,
                           int table_width, int heads, int kv_heads, int window, float scale, const float* __restrict__ r1,
-                          const float* __restrict__ r2) {
+                          const float* __restrict__ r2, const float* __restrict__ bias) {
     constexpr int DIM = 32 * KS;
     int seq, first, count;
     if (!tile_of(blockIdx.x, cu_seqlens, seqs, seq, first, count)) return;
@@ -93,6 +119,7 @@ talking_stats_mfma_kernel(float* __restrict__ stats, const bf16_t* __restrict__ 
         qf[ks].u = *reinterpret_cast<const uint4*>(q + (size_t)t * q_stride + q_off + (size_t)h * DIM + ks * 32 + 8 * g);
     const bool biased = r1 != nullptr;
     const float b1 = biased ? r1[h] : 0.f, b2 = biased ? r2[h] : 0.f;
+    const float* hb = TABLE ? bias + (size_t)h * (window + 16) + 8 : nullptr;
     const int pos_first = tok_pos[first], pos_last = pos_first + count - 1;
     const int lo_first = window > 0 ? max(0, pos_first - window + 1) : 0;
     const int key_row = 8 * (col >> 2) + (col & 3);
@@ -100,7 +127,7 @@ talking_stats_mfma_kernel(float* __restrict__ stats, const bf16_t* __restrict__ 
     for (int page = lo_first / TM_PAGE; page <= pos_last / TM_PAGE; ++page) {
         const bf16_t* kp = k_pages + (((long)table[page] * kv_heads + kvh) * TM_PAGE + key_row) * (long)DIM + 8 * g;
         float s[8];
-        talking_scores<KS>(s, qf, kp, DIM, scale, b1, b2, biased, qpos, lo, page * TM_PAGE + 8 * g);
+        talking_scores<KS, TABLE>(s, qf, kp, DIM, scale, b1, b2, biased, qpos, lo, page * TM_PAGE + 8 * g, hb, window);
         float mx = fmaxf(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3])), fmaxf(fmaxf(s[4], s[5]), fmaxf(s[6], s[7])));
         mx = fmaxf(mx, __shfl_xor(mx, 16, RI_WAVE));
         mx = fmaxf(mx, __shfl_xor(mx, 32, RI_WAVE));
@@ -120,17 +147,18 @@ talking_stats_mfma_kernel(float* __restrict__ stats, const bf16_t* __restrict__ 
     }
 }
 
-template <int KS, int HPW>
+template <int KS, int HPW, bool TABLE>
 __global__ void __launch_bounds__(64 * TM_WAVES)
-talking_mix_mfma_kernel(bf16_t* __restrict__ out, const float* __restrict__ stats, const bf16_t* __restrict__ q, int q_stride,
+talking_mix_mfma_kernel(bf16_t* __restrict__ out, float* __restrict__ parts, size_t part_stride, const float* __restrict__ stats, const bf16_t* __restrict__ q, int q_stride,
                         int q_off, const bf16_t* __restrict__ k_pages, const bf16_t* __restrict__ v_pages,
                         const int32_t* __restrict__ tok_pos, const int32_t* __restrict__ cu_seqlens, int seqs,
                         const int32_t* __restrict__ page_table, int table_width, int kv_heads, int window, float scale,
-                        const float* __restrict__ r1, const float* __restrict__ r2, const float* __restrict__ talk) {
+                        const float* __restrict__ r1, const float* __restrict__ r2, const float* __restrict__ talk,
+                        const float* __restrict__ bias) {
     constexpr int DIM = 32 * KS, VT = DIM / 16, HEADS = HPW * TM_WAVES;
     extern __shared__ float lds[];
     float* ps = lds;                                           // [HEADS][TM_TILE][TM_PAGE] the heads' weights of a page
-    float* tk = ps + HEADS * TM_TILE * TM_PAGE;                // [HEADS][HEADS] the mixing matrix
+    float* tk = ps + HEADS * TM_TILE * TM_PAGE;                // [HEADS][HEADS] the mixing matrix, transposed
     int seq, first, count;
     if (!tile_of(blockIdx.x, cu_seqlens, seqs, seq, first, count)) return;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -140,7 +168,7 @@ talking_mix_mfma_kernel(bf16_t* __restrict__ out, const float* __restrict__ stat
     const int lo = window > 0 ? max(0, qpos - window + 1) : 0;
     const int share = HEADS / kv_heads;
     const int32_t* table = page_table + (size_t)seq * table_width;
-    for (int e = threadIdx.x; e < HEADS * HEADS; e += 64 * TM_WAVES) tk[e] = talk ? talk[e] : (e / HEADS == e % HEADS ? 1.f : 0.f);
+    for (int e = threadIdx.x; e < HEADS * HEADS; e += 64 * TM_WAVES) tk[e % HEADS * HEADS + e / HEADS] = talk ? talk[e] : (e / HEADS == e % HEADS ? 1.f : 0.f);
     const bool biased = r1 != nullptr;
     float ms[HPW], inv_l[HPW], b1[HPW], b2[HPW];
 #pragma unroll
@@ -159,8 +187,11 @@ talking_mix_mfma_kernel(bf16_t* __restrict__ out, const float* __restrict__ stat
     const int pos_first = tok_pos[first], pos_last = pos_first + count - 1;
     const int lo_first = window > 0 ? max(0, pos_first - window + 1) : 0;
     const int key_row = 8 * (col >> 2) + (col & 3);
+    // (a share of the pages: workgroup y of gridDim.y)
+    const int page0 = lo_first / TM_PAGE, pages = pos_last / TM_PAGE + 1 - page0;
+    const int page_first = page0 + (int)((long)pages * blockIdx.y / gridDim.y), page_end = page0 + (int)((long)pages * (blockIdx.y + 1) / gridDim.y);
     __syncthreads();
-    for (int page = lo_first / TM_PAGE; page <= pos_last / TM_PAGE; ++page) {
+    for (int page = page_first; page < page_end; ++page) {
         const long phys = table[page];
         // this wavefront's heads: their weights of the page, into LDS
 #pragma unroll
@@ -172,7 +203,8 @@ talking_mix_mfma_kernel(bf16_t* __restrict__ out, const float* __restrict__ stat
             for (int ks = 0; ks < KS; ++ks)
                 qf[ks].u = *reinterpret_cast<const uint4*>(q + (size_t)t * q_stride + q_off + (size_t)h * DIM + ks * 32 + 8 * g);
             float s[8];
-            talking_scores<KS>(s, qf, kp, DIM, scale, b1[i], b2[i], biased, qpos, lo, page * TM_PAGE + 8 * g);
+            talking_scores<KS, TABLE>(s, qf, kp, DIM, scale, b1[i], b2[i], biased, qpos, lo, page * TM_PAGE + 8 * g,
+                                      TABLE ? bias + (size_t)h * (window + 16) + 8 : nullptr, window);
             float4 lo4, hi4;
             lo4.x = expf(s[0] - ms[i]) * inv_l[i]; lo4.y = expf(s[1] - ms[i]) * inv_l[i];
             lo4.z = expf(s[2] - ms[i]) * inv_l[i]; lo4.w = expf(s[3] - ms[i]) * inv_l[i];
@@ -181,9 +213,12 @@ talking_mix_mfma_kernel(bf16_t* __restrict__ out, const float* __restrict__ stat
             float* pp = ps + ((size_t)h * TM_TILE + col) * TM_PAGE + 8 * g;
             *reinterpret_cast<float4*>(pp) = lo4;
             *reinterpret_cast<float4*>(pp + 4) = hi4;
+            __builtin_amdgcn_sched_barrier(0);                 // (a head at a time: the registers are the sums')
         }
         __syncthreads();
-        // the mix for this wavefront's heads, then their value products
+        // the mix for this wavefront's heads, then their value products; a head's values are asked for together (left to itself
+        // the compiler waits for every single load)
+        TmFrag p[HPW];
         float mixed[HPW][8];
 #pragma unroll
         for (int i = 0; i < HPW; ++i)
@@ -195,30 +230,38 @@ talking_mix_mfma_kernel(bf16_t* __restrict__ out, const float* __restrict__ stat
             const float w8[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
 #pragma unroll
             for (int i = 0; i < HPW; ++i) {
-                const float c = tk[(wave * HPW + i) * HEADS + gh];
+                const float c = tk[gh * HEADS + wave * HPW + i];
 #pragma unroll
                 for (int e = 0; e < 8; ++e) mixed[i][e] += c * w8[e];
             }
         }
 #pragma unroll
+        for (int i = 0; i < HPW; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) p[i].w[e] = pack_bf16x2(mixed[i][2 * e], mixed[i][2 * e + 1]);
+#pragma unroll
         for (int i = 0; i < HPW; ++i) {
-            const int h = wave * HPW + i;
-            TmFrag p;
+            const bf16_t* vp = v_pages + ((phys * kv_heads + (wave * HPW + i) / share) * (long)DIM + col) * TM_PAGE + 8 * g;
+            TmFrag vf[VT];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) p.w[e] = pack_bf16x2(mixed[i][2 * e], mixed[i][2 * e + 1]);
-            const bf16_t* vp = v_pages + ((phys * kv_heads + h / share) * (long)DIM + col) * TM_PAGE + 8 * g;
+            for (int vt = 0; vt < VT; ++vt) vf[vt].u = *reinterpret_cast<const uint4*>(vp + (long)vt * 16 * TM_PAGE);
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int vt = 0; vt < VT; ++vt) {
-                TmFrag vf;
-                vf.u = *reinterpret_cast<const uint4*>(vp + (long)vt * 16 * TM_PAGE);
-                o[i][vt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf.v, p.v, o[i][vt], 0, 0, 0);
-            }
+            for (int vt = 0; vt < VT; ++vt)
+                o[i][vt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[vt].v, p[i].v, o[i][vt], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
         }
         __syncthreads();                                       // before the next page's weights overwrite these
     }
     if (col < count) {
 #pragma unroll
         for (int i = 0; i < HPW; ++i) {
+            if (parts) {
+                float* fp = parts + blockIdx.y * part_stride + (size_t)t * HEADS * DIM + (size_t)(wave * HPW + i) * DIM + 4 * g;
+#pragma unroll
+                for (int vt = 0; vt < VT; ++vt) *reinterpret_cast<tm_floatx4*>(fp + vt * 16) = o[i][vt];
+                continue;
+            }
             bf16_t* op = out + (size_t)t * HEADS * DIM + (size_t)(wave * HPW + i) * DIM + 4 * g;
 #pragma unroll
             for (int vt = 0; vt < VT; ++vt) {
@@ -236,13 +279,17 @@ extern "C" int ri_talking_attention_mfma_fits(int heads, int kv_heads, int dim, 
            kv_heads >= 1 && heads % kv_heads == 0;
 }
 
-// out [tokens, heads * dim] bfloat16; stats: float32 workspace [tokens][heads][2]; tiles: an upper bound on the tiles of
+// out [tokens, heads * dim] bfloat16; stats: float32 workspace [tokens][heads][2]; bias: float32 workspace [heads][window + 16], used where
+// there is a window and a bias (NULL: the logarithm a score); parts: with shares > 1, float32 [shares][tokens][heads * dim], whose sum is the
+// result (out is then not written); tiles: an upper bound on the tiles of
 // 16 tokens that the sequences' new tokens make (every sequence's count rounded up).
 extern "C" int ri_talking_attention_mfma(void* out, float* stats, const void* q, int q_stride, int q_off, const void* k_pages,
                                          const void* v_pages, const int32_t* tok_pos, const int32_t* cu_seqlens, int seqs,
                                          const int32_t* page_table, int table_width, int tiles, int heads, int kv_heads, int dim,
                                          int page_size, int window, float scale, const float* r1, const float* r2,
-                                         const float* talk, void* stream) {
+                                         const float* talk, float* bias, float* parts, int shares, int tokens, void* stream) {
+    RI_REQUIRE(shares >= 1 && shares <= 65535 && tokens > 0 && (shares == 1 || (parts && (uintptr_t)parts % 16 == 0)),
+               "talking_attention_mfma: %d shares of %d tokens", shares, tokens);
     RI_REQUIRE(seqs > 0 && tiles > 0 && ri_talking_attention_mfma_fits(heads, kv_heads, dim, page_size),
                "talking_attention_mfma: %d sequences, %d heads over %d of %d, pages of %d", seqs, heads, kv_heads, dim, page_size);
     RI_REQUIRE(q_off >= 0 && q_off + heads * dim <= q_stride && q_stride % 8 == 0 && q_off % 8 == 0 && (uintptr_t)q % 16 == 0 &&
@@ -253,25 +300,33 @@ extern "C" int ri_talking_attention_mfma(void* out, float* stats, const void* q,
     RI_REQUIRE(lds <= 64 * 1024 + 4096, "talking_attention_mfma: %d heads need %zu bytes of LDS", heads, lds);
     hipStream_t s = (hipStream_t)stream;
     const int hpw = heads / TM_WAVES;
-#define RI_STATS(KS)                                                                                                    \
-    talking_stats_mfma_kernel<KS><<<dim3(tiles, heads), 64, 0, s>>>(stats, (const bf16_t*)q, q_stride, q_off,          \
+    const bool table = bias && r1 && window > 0;
+    if (table) {
+        RI_REQUIRE((long)heads * (window + 16) < (1L << 30), "talking_attention_mfma: a window of %d", window);
+        talking_bias_kernel<<<(heads * (window + 16) + 255) / 256, 256, 0, s>>>(bias, r1, r2, heads, window);
+    }
+    if (shares == 1) parts = nullptr;
+#define RI_STATS(KS, T)                                                                                                 \
+    talking_stats_mfma_kernel<KS, T><<<dim3(tiles, heads), 64, 0, s>>>(stats, (const bf16_t*)q, q_stride, q_off,       \
                                                                      (const bf16_t*)k_pages, tok_pos, cu_seqlens, seqs, \
-                                                                     page_table, table_width, heads, kv_heads, window, scale, r1, r2)
-#define RI_MIX(KS, HPW)                                                                                                 \
+                                                                     page_table, table_width, heads, kv_heads, window, scale, r1, r2, bias)
+#define RI_MIX(KS, HPW, T)                                                                                              \
     do {                                                                                                                \
         if (lds > 64 * 1024)                                                                                            \
-            hipFuncSetAttribute((const void*)talking_mix_mfma_kernel<KS, HPW>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); \
-        talking_mix_mfma_kernel<KS, HPW><<<tiles, 64 * TM_WAVES, lds, s>>>(                                             \
-            (bf16_t*)out, stats, (const bf16_t*)q, q_stride, q_off, (const bf16_t*)k_pages, (const bf16_t*)v_pages, tok_pos, \
-            cu_seqlens, seqs, page_table, table_width, kv_heads, window, scale, r1, r2, talk);                          \
+            hipFuncSetAttribute((const void*)talking_mix_mfma_kernel<KS, HPW, T>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); \
+        talking_mix_mfma_kernel<KS, HPW, T><<<dim3(tiles, shares), 64 * TM_WAVES, lds, s>>>(                            \
+            (bf16_t*)out, parts, (size_t)tokens * heads * dim, stats, (const bf16_t*)q, q_stride, q_off, (const bf16_t*)k_pages, \
+            (const bf16_t*)v_pages, tok_pos, cu_seqlens, seqs, page_table, table_width, kv_heads, window, scale, r1, r2, talk, bias); \
     } while (0)
-#define RI_BY_HEADS(KS)                                                                                                 \
+#define RI_BY_TABLE(KS, T)                                                                                              \
     do {                                                                                                                \
-        RI_STATS(KS);                                                                                                   \
-        if (hpw == 1) RI_MIX(KS, 1); else if (hpw == 2) RI_MIX(KS, 2); else if (hpw == 3) RI_MIX(KS, 3); else RI_MIX(KS, 4); \
+        RI_STATS(KS, T);                                                                                                \
+        if (hpw == 1) RI_MIX(KS, 1, T); else if (hpw == 2) RI_MIX(KS, 2, T); else if (hpw == 3) RI_MIX(KS, 3, T); else RI_MIX(KS, 4, T); \
     } while (0)
+#define RI_BY_HEADS(KS) do { if (table) RI_BY_TABLE(KS, true); else RI_BY_TABLE(KS, false); } while (0)
     if (dim == 32) RI_BY_HEADS(1); else if (dim == 64) RI_BY_HEADS(2); else RI_BY_HEADS(4);
 #undef RI_BY_HEADS
+#undef RI_BY_TABLE
 #undef RI_MIX
 #undef RI_STATS
     RI_LAUNCH_CHECK("talking_attention_mfma");

@@ -179,7 +179,7 @@ _SIGNATURES = {
     "ri_talking_attention_mfma_fits": [c_int, c_int, c_int, c_int],
     "ri_talking_attention_mfma": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_int,
                                   c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_void_p, c_void_p, c_void_p,
-                                  c_void_p],
+                                  c_void_p, c_void_p, c_int, c_int, c_void_p],
     "ri_shift_mix": [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p],
     "ri_shift_keep": [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p],
     "ri_timemix_max_dim": [],
@@ -1789,6 +1789,9 @@ def talking_attention_mfma_fits(dtype, heads: int, kv_heads: int, dim: int, page
     return dtype == torch.bfloat16 and bool(_get("ri_talking_attention_mfma_fits")(heads, kv_heads, dim, page_size))
 
 
+TALKING_MAX_SHARES = 4           # parts of a tile's pages: past this the adding of the parts costs what the walk gains
+
+
 def talking_attention_mfma(proj, q_off: int, k_pages, v_pages, tok_pos, cu_seqlens, new_counts, page_table, heads: int,
                            kv_heads: int, dim: int, window: int | None, scale: float, r1, r2, talk) -> torch.Tensor:
     """The same attention on the matrix cores, for prompts in bfloat16: ``[T, heads * dim]``.  ``new_counts``: every
@@ -1800,13 +1803,18 @@ def talking_attention_mfma(proj, q_off: int, k_pages, v_pages, tok_pos, cu_seqle
     if tiles == 0:
         return out
     stats = torch.empty((tokens, heads, 2), dtype=torch.float32, device=proj.device)
+    # (a table of the biases a distance for windows it is small for; shares of the pages where the tiles leave compute units idle)
+    bias = torch.empty((heads, window + 16), dtype=torch.float32, device=proj.device) if window and window <= 16384 and r1 is not None else None
+    shares = max(1, min(TALKING_MAX_SHARES, compute_units() // tiles))
+    parts = torch.empty((shares, tokens, heads * dim), dtype=torch.float32, device=proj.device) if shares > 1 else None
     _call("ri_talking_attention_mfma", _dev(out, "out"), _dev(stats, "stats"), _dev(proj, "proj", torch.bfloat16), proj.shape[1],
           int(q_off), _dev(k_pages, "k_pages", torch.bfloat16), _dev(v_pages, "v_pages", torch.bfloat16),
           _dev(tok_pos, "tok_pos", torch.int32, (tokens,)), _dev(cu_seqlens, "cu_seqlens", torch.int32, (seqs + 1,)), seqs,
           _dev(page_table, "page_table", torch.int32), page_table.shape[1], tiles, heads, kv_heads, dim, k_pages.shape[2],
           int(window or 0), float(scale), _opt(r1, "r1", torch.float32, (heads,)), _opt(r2, "r2", torch.float32, (heads,)),
-          _opt(talk, "talk", torch.float32, (heads, heads)), _stream())
-    return out
+          _opt(talk, "talk", torch.float32, (heads, heads)), _opt(bias, "bias", torch.float32), _opt(parts, "parts", torch.float32), shares,
+          tokens, _stream())
+    return sum_parts(parts) if parts is not None else out
 
 
 # ---------------------------------------------------------------- time mixing
