@@ -131,6 +131,152 @@ latent_attention_mfma_kernel(bf16_t* __restrict__ out, const bf16_t* __restrict_
     }
 }
 
+// Prompts: a workgroup of eight wavefronts takes eight (token, tile of 16 heads) pairs of neighbouring tokens, which walk the same
+// pages, and brings every page into LDS once for all of them.  What bounds the kernel above on a prompt is the caches: every wavefront
+// fetches every page for itself, 69 KB for 68 MFMAs.  Here a page crosses once for eight wavefronts, and what is left is
+// reading the fragments from LDS, two cycles of it for every one of the matrix cores.  A page's key and value halves take turns: while
+// the scores are made from the keys the values are on their way into registers, and the other way round, so that two barriers a
+// page are all that is waited for.  Pieces of 16 bytes are exchanged by the row's number so that a fragment's sixteen rows meet every
+// bank equally.  A token's sums are the other kernel's.  2,048 tokens, 32 heads, keys of 576: 1,400 us with a page a wavefront, 616.
+#define LP_WAVES 8
+template <int KS, int VT>
+__global__ void __launch_bounds__(64 * LP_WAVES)
+latent_attention_shared_kernel(bf16_t* __restrict__ out, const bf16_t* __restrict__ q, int q_stride,
+                               const bf16_t* __restrict__ k_pages, const bf16_t* __restrict__ v_pages,
+                               const int32_t* __restrict__ tok_pos, const int32_t* __restrict__ tok_seq,
+                               const int32_t* __restrict__ page_table, int table_width, int tokens, int heads, int tiles,
+                               float scale_log2, const float* __restrict__ sinks) {
+    constexpr int DK = 32 * KS, RANK = 16 * VT, THREADS = 64 * LP_WAVES;
+    constexpr int KP = DK / 8, KPIECES = LM_PAGE * KP;        // 16-byte pieces of a key row and of a page's keys
+    constexpr int VP = LM_PAGE / 8, VPIECES = RANK * VP;      // ... of a value channel's row and of a page's values
+    constexpr int KN = (KPIECES + THREADS - 1) / THREADS, VN = (VPIECES + THREADS - 1) / THREADS;
+    __shared__ uint4 ks_[KPIECES], vs_[VPIECES];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, col = lane & 15, g = lane >> 4;
+    const long pairs = (long)tokens * tiles;
+    // (long prompts first: the workgroups launched last are the short ones; pairs count back from the last token's)
+    const long pair = (long)blockIdx.x * LP_WAVES + wave;
+    const bool there = pair < pairs;
+    const long mine = there ? pair : pairs - 1;
+    const int t = tokens - 1 - (int)(mine / tiles), tile = (int)(mine % tiles);
+    const int head = tile * 16 + col, hq = head < heads ? head : heads - 1;
+    const int qpos = tok_pos[t], seq = tok_seq[t];
+    // the tokens of a workgroup are of one sequence nearly always; where they are not, the sequences go one after the other
+    const int t_last = tokens - 1 - (int)((long)blockIdx.x * LP_WAVES / tiles);
+    const int t_first = tokens - 1 - (int)(min((long)blockIdx.x * LP_WAVES + LP_WAVES, pairs) - 1) / tiles;
+
+    LmFrag qf[KS];
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+        qf[ks].u = *reinterpret_cast<const uint4*>(q + (size_t)t * q_stride + (size_t)hq * DK + ks * 32 + 8 * g);
+    lm_floatx4 o[VT];
+#pragma unroll
+    for (int vt = 0; vt < VT; ++vt) o[vt] = lm_floatx4{0.f, 0.f, 0.f, 0.f};
+    float m = -INFINITY, l = 0.f;
+    const int key_row = 8 * (col >> 2) + (col & 3);
+    uint4 kn[KN], vn[VN];
+    auto fetch_keys = [&](long phys) {
+        const uint4* from = reinterpret_cast<const uint4*>(k_pages + phys * LM_PAGE * (long)DK);
+#pragma unroll
+        for (int i = 0; i < KN; ++i) kn[i] = from[min(tid + i * THREADS, KPIECES - 1)];
+    };
+    auto fetch_values = [&](long phys) {
+        const uint4* from = reinterpret_cast<const uint4*>(v_pages + phys * LM_PAGE * (long)RANK);
+#pragma unroll
+        for (int i = 0; i < VN; ++i) vn[i] = from[min(tid + i * THREADS, VPIECES - 1)];
+    };
+    // (a fragment's key rows are 0 .. 3 of every eight, or 4 .. 7; pieces stay within eight, or four where eight do not divide a row)
+    auto key_at = [](int row, int piece) { return row * KP + (piece ^ (((row >> 1 & 1) | (row >> 3 & 3) << 1) & (KP % 8 == 0 ? 7 : 3))); };
+    auto value_at = [](int row, int piece) { return row * VP + (piece ^ (row >> 2 & 3)); };
+
+    for (int from = t_last; from >= t_first;) {               // (uniform: the tokens' sequences and positions are memory's)
+        const int s_now = tok_seq[from];
+        int to = from;
+        while (to > t_first && tok_seq[to - 1] == s_now) --to;
+        const bool active = there && t <= from && t >= to;
+        const int32_t* table = page_table + (size_t)s_now * table_width;
+        const int pages = tok_pos[from] / LM_PAGE + 1;        // (positions grow with the tokens of a sequence)
+        fetch_keys(table[0]);
+        for (int page = 0; page < pages; ++page) {
+            const long phys = table[page], next = table[min(page + 1, pages - 1)];
+#pragma unroll
+            for (int i = 0; i < KN; ++i) {
+                const int e = tid + i * THREADS;
+                if (KPIECES % THREADS == 0 || e < KPIECES) ks_[key_at(e / KP, e % KP)] = kn[i];
+            }
+            fetch_values(phys);
+            __syncthreads();                                  // the keys are in place, and the page before's values have been read
+            const bool sees = active && page * LM_PAGE <= qpos;          // (the same for the whole wavefront)
+            LmFrag p;
+            float corr = 1.f;
+            if (sees) {
+                lm_floatx4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int ks = 0; ks < KS; ++ks) {
+                    LmFrag k0, k1;
+                    k0.u = ks_[key_at(key_row, ks * 4 + g)];
+                    k1.u = ks_[key_at(key_row + 4, ks * 4 + g)];
+                    s0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k0.v, qf[ks].v, s0, 0, 0, 0);
+                    s1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k1.v, qf[ks].v, s1, 0, 0, 0);
+                }
+                float s[8] = {s0[0], s0[1], s0[2], s0[3], s1[0], s1[1], s1[2], s1[3]};
+                const int key0 = page * LM_PAGE + 8 * g;
+                if (key0 + 7 > qpos) {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
+                        if (key0 + e > qpos) s[e] = -INFINITY;
+                }
+                float mx = fmaxf(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3])), fmaxf(fmaxf(s[4], s[5]), fmaxf(s[6], s[7])));
+                mx = fmaxf(mx, __shfl_xor(mx, 16, RI_WAVE));
+                mx = fmaxf(mx, __shfl_xor(mx, 32, RI_WAVE));
+                const float m_new = fmaxf(m, mx * scale_log2);        // the scale is positive; key 0 is seen by every token: finite
+                float sum = 0.f;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float a = exp2f(fmaf(s[2 * e], scale_log2, -m_new));
+                    const float b = exp2f(fmaf(s[2 * e + 1], scale_log2, -m_new));
+                    p.w[e] = pack_bf16x2(a, b);
+                    sum += a + b;
+                }
+                corr = exp2f(m - m_new);                      // 0 at the first page (m = -inf)
+                l = l * corr + sum;
+                m = m_new;
+            }
+#pragma unroll
+            for (int i = 0; i < VN; ++i) {
+                const int e = tid + i * THREADS;
+                if (VPIECES % THREADS == 0 || e < VPIECES) vs_[value_at(e / VP, e % VP)] = vn[i];
+            }
+            fetch_keys(next);
+            __syncthreads();                                  // the values are in place, and the keys have been read
+            if (sees) {
+#pragma unroll
+                for (int vt = 0; vt < VT; ++vt) {
+                    LmFrag vf;
+                    vf.u = vs_[value_at(vt * 16 + col, g)];
+                    o[vt] *= corr;
+                    o[vt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf.v, p.v, o[vt], 0, 0, 0);
+                }
+            }
+        }
+        from = to - 1;
+    }
+    if (!there) return;
+    l += __shfl_xor(l, 16, RI_WAVE);                          // a column's sum over its four lanes
+    l += __shfl_xor(l, 32, RI_WAVE);
+    if (sinks) l += exp2f(sinks[hq] * 1.4426950408889634f - m);
+    const float inv = 1.0f / l;
+    if (head < heads) {
+        bf16_t* op = out + ((size_t)t * heads + head) * RANK + 4 * g;
+#pragma unroll
+        for (int vt = 0; vt < VT; ++vt) {
+            uint2 w;
+            w.x = pack_bf16x2(o[vt][0] * inv, o[vt][1] * inv);
+            w.y = pack_bf16x2(o[vt][2] * inv, o[vt][3] * inv);
+            *reinterpret_cast<uint2*>(op + vt * 16) = w;
+        }
+    }
+}
+
 // The chunks of a token's pages, joined: the largest maximum, every chunk's sums scaled to it, the sink, the division.
 __global__ void __launch_bounds__(256)
 latent_attention_join_kernel(bf16_t* __restrict__ out, const float* __restrict__ partial, const float* __restrict__ sinks,
@@ -173,10 +319,11 @@ extern "C" int ri_latent_attention_mfma_fits(int key_dim, int rank, int page_siz
 
 // out [tokens, heads * rank] bfloat16: causal attention of every new token's heads (q [tokens, >= heads * key_dim], the
 // heads side by side) over its sequence's one key/value head of key rows of key_dim and value rows of rank.
+// shared_pages: neighbouring tokens are of one sequence for the most part, and share the pages they fetch (the results are the same bits).
 extern "C" int ri_latent_attention_mfma(void* out, const void* q, int q_stride, const void* k_pages, const void* v_pages,
                                         const int32_t* tok_pos, const int32_t* tok_seq, const int32_t* page_table,
                                         int table_width, int tokens, int heads, int key_dim, int rank, int page_size, float scale,
-                                        const float* sinks, float* partial, int chunks, int chunk_pages, void* stream) {
+                                        const float* sinks, float* partial, int chunks, int chunk_pages, int shared_pages, void* stream) {
     RI_REQUIRE(tokens > 0 && heads > 0 && ri_latent_attention_mfma_fits(key_dim, rank, page_size),
                "latent_attention_mfma: %d tokens, %d heads, keys of %d, values of %d, pages of %d", tokens, heads, key_dim, rank, page_size);
     RI_REQUIRE(q_stride >= heads * key_dim && q_stride % 8 == 0 && (uintptr_t)q % 16 == 0 && (uintptr_t)k_pages % 16 == 0 &&
@@ -197,7 +344,16 @@ extern "C" int ri_latent_attention_mfma(void* out, const void* q, int q_stride, 
                                                                           tok_pos, tok_seq, page_table, table_width, tokens, \
                                                                           heads, tiles, scale_log2, sinks, partial, chunks, \
                                                                           chunk_pages)
-    if (key_dim == 576) RI_GO(18, 32); else if (key_dim == 288) RI_GO(9, 16); else RI_GO(5, 8);
+    if (shared_pages && chunks == 1) {
+        const unsigned groups = (unsigned)((pairs + LP_WAVES - 1) / LP_WAVES);
+#define RI_SHARED(KS, VT)                                                                                               \
+    latent_attention_shared_kernel<KS, VT><<<groups, 64 * LP_WAVES, 0, s>>>((bf16_t*)out, (const bf16_t*)q, q_stride,   \
+                                                                            (const bf16_t*)k_pages, (const bf16_t*)v_pages, tok_pos, \
+                                                                            tok_seq, page_table, table_width, tokens, heads, tiles, \
+                                                                            scale_log2, sinks)
+        if (key_dim == 576) RI_SHARED(18, 32); else if (key_dim == 288) RI_SHARED(9, 16); else RI_SHARED(5, 8);
+#undef RI_SHARED
+    } else if (key_dim == 576) RI_GO(18, 32); else if (key_dim == 288) RI_GO(9, 16); else RI_GO(5, 8);
 #undef RI_GO
     if (chunks > 1)
         latent_attention_join_kernel<<<dim3(tokens, heads), 256, 0, s>>>((bf16_t*)out, partial, sinks, heads, chunks, rank);

@@ -167,7 +167,7 @@ _SIGNATURES = {
                           c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
     "ri_latent_attention_mfma_fits": [c_int, c_int, c_int],
     "ri_latent_attention_mfma": [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int,
-                                 c_int, c_int, c_int, c_float, c_void_p, c_void_p, c_int, c_int, c_void_p],
+                                 c_int, c_int, c_int, c_float, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p],
     "ri_head_products": [c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_int, c_void_p,
                          c_int, c_int, c_float, c_int, c_int, c_int, c_int, c_int, c_void_p],
     "ri_whole_norm_kv_write": [c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_float, c_void_p, c_void_p, c_void_p,
@@ -1656,6 +1656,10 @@ def latent_attention_mfma_fits(dtype, key_dim: int, rank: int, page_size: int) -
     return dtype == torch.bfloat16 and bool(_get("ri_latent_attention_mfma_fits")(key_dim, rank, page_size))
 
 
+LATENT_SHARED_FROM = 16          # new tokens a sequence brings on average from which neighbours share the pages they fetch: where a
+                                 # workgroup's tokens are of different sequences they go one sequence after the other
+
+
 def latent_attention_mfma(q, k_pages, v_pages, tok_pos, tok_seq, page_table, heads: int, scale: float, sinks,
                           max_len: int = 0) -> torch.Tensor:
     """bfloat16 ``[T, heads * rank]``: causal attention on the matrix cores of every new token's ``heads`` query rows (``q [T,
@@ -1680,7 +1684,8 @@ def latent_attention_mfma(q, k_pages, v_pages, tok_pos, tok_seq, page_table, hea
           _dev(k_pages, "k_pages", torch.bfloat16), _dev(v_pages, "v_pages", torch.bfloat16),
           _dev(tok_pos, "tok_pos", torch.int32, (tokens,)), _dev(tok_seq, "tok_seq", torch.int32, (tokens,)),
           _dev(page_table, "page_table", torch.int32), page_table.shape[1], tokens, heads, key_dim, rank, page, float(scale),
-          _opt(sinks, "sinks", torch.float32, (heads,)), _opt(partial, "partial"), chunks, chunk_pages, _stream())
+          _opt(sinks, "sinks", torch.float32, (heads,)), _opt(partial, "partial"), chunks, chunk_pages,
+          int(not max_len and tokens >= LATENT_SHARED_FROM * page_table.shape[0]), _stream())
     return out
 
 

@@ -351,6 +351,28 @@ def test_latent_attention_on_the_matrix_cores_is_the_general_kernel(ops, heads):
             close(got, f64(want), 1.2e-2, f"in chunks, sequences of up to {bound}")
 
 
+@pytest.mark.parametrize("heads, dk, rank", [(3, 160, 128), (20, 288, 256), (40, 160, 128), (130, 160, 128), (16, 576, 512)])
+def test_latent_attention_with_shared_pages_gives_the_same_bits(ops, heads, dk, rank, monkeypatch):
+    """Eight (token, tile of heads) pairs a workgroup: workgroups whose tokens are of two and three sequences, of more tiles than
+    pairs, a last one that is not full; against a wavefront that fetches its pages itself."""
+    rng = np.random.default_rng(heads + dk)
+    new, lens = [9, 1, 2, 5], [40, 1, 34, 5]
+    pages = sum(-(-n // PAGE) for n in lens) + 2
+    k_pages = guarded((torch.randn((pages, 1, PAGE, dk), device=DEV) * 0.5).to(torch.bfloat16))
+    v_pages = guarded(k_pages[:, :, :, :rank].transpose(2, 3).contiguous())
+    order = iter(rng.permutation(pages))
+    table = t([[next(order) if i < -(-n // PAGE) else -1 for i in range(2)] for n in lens], torch.int32)
+    tok_seq = t([s for s, n in enumerate(new) for _ in range(n)], torch.int32)
+    tok_pos = t([lens[s] - n + i for s, n in enumerate(new) for i in range(n)], torch.int32)
+    q = guarded((torch.randn((sum(new), heads * dk), device=DEV) * 0.5).to(torch.bfloat16))
+    sinks = t(rng.standard_normal(heads))
+    got = []
+    for least in (1 << 30, 0):
+        monkeypatch.setattr(ops, "LATENT_SHARED_FROM", least)
+        got.append(f64(ops.latent_attention_mfma(q, k_pages, v_pages, tok_pos, tok_seq, table, heads, 0.11, sinks)))
+    assert np.isfinite(got[0]).all() and np.array_equal(*got)
+
+
 @pytest.mark.parametrize("heads, kv_heads, dim, window", [(8, 2, 32, 40), (16, 16, 32, None), (8, 1, 64, 33)])
 def test_talking_attention_on_the_matrix_cores_is_the_general_kernel(ops, heads, kv_heads, dim, window):
     """bfloat16: two sequences whose pages lie in shuffled order, one that goes on from 37 cached tokens with 21 new ones
