@@ -44,6 +44,12 @@ SMALL_ONLY_ROWS = 64             # a matrix packed for small steps alone stays o
 WIDE_GATED_FILL = 0.75            # gate|up goes to the wide kernel where its workgroups fill this share of the rounds,
 WIDE_GATED_ROWS = 48             # and up to this many rows whatever they fill, if the packed kernel of 17 to 64 rows is no match:
 WIDE_GATED_BYTES = 64_000_000    # pairs larger than this (smaller ones, up to 32 tiled rows, are that kernel's)
+# 17 to 48 rows against a plain matrix of many rows (all experts' gates and ups side by side: 4 row tiles a compute unit and
+# more): the wide kernel, K whole.  98,304 x 4,096 at 17 / 32 / 48 / 64 rows: 136 / 143 / 163 / 183 us against the library's 180 / 180 / 172 / 177;
+# 24,576 x 1,024: 13 / 15 / 17 / 20 against 32 / 32 / 18 / 18; 24,576 x 4,096 37 / 41 / 49 / 58 against 52 / 51 / 51 / 51; with fewer row
+# tiles level (12,288 x 4,096 at 32 rows 23 against 24).
+WIDE_PLAIN_TILES = 4
+WIDE_PLAIN_ROWS = 48
 SPLIT_K = 4096                   # pieces of a long K (PACKED_LONG_K and more) whose sums the next norm adds
 # Which matrices get a packed copy for 2 to 16 rows (the gate|up matrix always does: its activation rides in
 # the kernel): up to 40 MB always; up to PACKED_MAX_BYTES unless the last round of workgroups (one per 16 rows)
@@ -55,6 +61,14 @@ PACKED_LONG_K = 16384
 @functools.lru_cache(maxsize=None)
 def _compute_units() -> int:
     return ops.compute_units()
+
+
+def _wide_whole_waves(n: int, m: int) -> int:
+    """Three or four row tiles a workgroup of the wide kernel with K whole: whichever has a compute unit fetch fewer rows (of
+    x for every round of workgroups, and of the matrix)."""
+    def rows(waves):
+        return -(-n // (16 * waves * _compute_units())) * (-(-m // 16) * 16 + 16 * waves)
+    return 3 if rows(3) < rows(4) else 4
 
 
 def _packed_pays(n: int, k: int) -> bool:
@@ -294,6 +308,10 @@ class Runtime:
                 x = self.normed_now(x) if later else x
                 return ops.gemm_mid_packed_bf16(x, pw.packed, pw.n, out_dtype, swiglu=pw.swiglu,
                                                 tiled_out=tiled_out and out_dtype == torch.bfloat16)
+            if (WIDE_MIN_ROWS <= m <= WIDE_PLAIN_ROWS and pw.packed is not None and not pw.swiglu and not pw.small_only
+                    and pw.n >= 16 * WIDE_PLAIN_TILES * _compute_units()):
+                x = self.normed_now(x) if later else x
+                return ops.gemm_wide_packed_bf16(x, pw.packed, pw.n, out_dtype, depth=1, waves=_wide_whole_waves(pw.n, m))
         y = self.linear(x, pw.w, None if pw.swiglu else out_dtype)
         return ops.swiglu(y, tiled_out=tiled_out) if pw.swiglu else y
 

@@ -482,3 +482,15 @@ def test_a_shared_expert_without_a_gate_is_added_as_it_is(ops):
     for dim in (48, 50):
         routed, shared = rng.normal(size=(3, 5, dim)), rng.normal(size=(2, 5, dim))
         close(ops.experts_finish(t(routed), None, t(shared), None), routed.sum(0) + shared.sum(0), F32)
+
+
+@pytest.mark.parametrize("tokens, experts, ff, limit", [(1, 1, 8, 0.0), (3, 5, 40, 1.1), (2, 2, 2056, 0.0)])
+def test_experts_activation_in_pieces_is_the_one_by_elements(ops, tokens, experts, ff, limit):
+    """Rows of a multiple of eight elements against the same numbers as float32, rounded once; experts not chosen give zeros over NaN."""
+    rng = np.random.default_rng(ff)
+    gu = t(rng.normal(size=(tokens, experts * 2 * ff)), torch.bfloat16)
+    dense = t(rng.random((tokens, experts + 1)) * (rng.random((tokens, experts + 1)) < 0.6))
+    want = ops.experts_activate(guarded(gu.float()), dense, ff, limit).to(torch.bfloat16)
+    chosen = (dense[:, :experts, None] != 0).expand(-1, -1, 2 * ff).reshape(tokens, -1)
+    got = ops.experts_activate(guarded(torch.where(chosen, gu, torch.full_like(gu, float("nan")))), dense, ff, limit)
+    assert torch.equal(got, want)
