@@ -941,6 +941,67 @@ __device__ __forceinline__ void finish_head(bf16_t* dst_lds, const HeadLoads<DH>
 // one workgroup a compute unit for steps that have one run for every compute unit and few more (a wavefront's
 // walk is then half as long, and there is no join).
 
+// Which (sequence, kv head) a workgroup takes, and the sequence's position, where sequences run whole and two workgroups and
+// more share a compute unit: a unit takes as long as its walks together, and in the launch's own order (64 sequences of 8 kv
+// heads on 256 units) they are of one sequence, the longest with itself.  The sequences are ranked by their lengths (every
+// workgroup for itself), the longest go out first, and every second round of workgroups runs the other way, so that the
+// longest meets the shortest.  Eight sequences go out side by side and then their next heads: an XCD then has whole sequences.
+// Lengths within a sixteenth of the first's stay in the launch's order: there the ranking only costs (200 sequences of 800 keys:
+// 134.5 us a layer, 136.0 with the look at them, ranked too 144.8).  64 sequences of 1,100 to 2,040 keys at 32 heads of 128:
+// 80.0 us in the launch's order, 72.3 ranked; of 30 to 4,000: 133.9, 100.6; 200 of 30 to 2,000: 194.0, 167.8.
+#define STREAM_BALANCE_MOST 256  // sequences
+template <int W>
+__device__ __forceinline__ int stream_balance(int& b, int& kvh, const int32_t* __restrict__ tok_pos, int kv_heads, int units,
+                                              const Reach& reach, int32_t* __restrict__ len) {
+    __shared__ int chosen[2];  // (len is the workgroup's LDS for its sums, which nothing has written yet)
+    constexpr int HELD = STREAM_BALANCE_MOST / 64;
+    const int n = gridDim.x, tid = threadIdx.x, lane = tid & 63;
+    const int own = tok_pos[b], first = tok_pos[0];
+    int pos[HELD], far = 0;
+#pragma unroll
+    for (int i = 0; i < HELD; ++i) pos[i] = tok_pos[min(64 * i + lane, n - 1)];
+    __builtin_amdgcn_sched_barrier(0);  // (one trip to memory for all of them)
+    // (against the first sequence's: every wavefront of every workgroup for itself, and all find the same)
+    const int first_len = first + 1 - reach.first(first);
+#pragma unroll
+    for (int i = 0; i < HELD; ++i) {
+        const int more = pos[i] + 1 - reach.first(pos[i]) - first_len;
+        far |= 16 * max(more, -more) > first_len;
+    }
+    if (!__any(far)) return own;
+    const int padded = (n + 15) & ~15;
+    if (tid < 64)
+#pragma unroll
+        for (int i = 0; i < HELD; ++i) len[64 * i + lane] = 64 * i + lane < n ? pos[i] + 1 - reach.first(pos[i]) : -1;
+    __syncthreads();
+    const int at = blockIdx.x + n * blockIdx.y, round = at / units, place = at - round * units;
+    const int unit = round * units + ((round & 1) ? min(units, n * kv_heads - round * units) - 1 - place : place);
+    const int set = unit / (8 * kv_heads), in_set = unit - set * 8 * kv_heads, wide = min(8, n - 8 * set);
+    const int rank = 8 * set + in_set % wide;
+    for (int i = tid; i < n; i += W * 64) {
+        const int mine = len[i];
+        int before = 0;
+        for (int k = 0; k < padded; k += 16)
+#pragma unroll
+            for (int d = 0; d < 16; d++) before += len[k + d] > mine || (len[k + d] == mine && k + d < i);
+        if (before == rank) {
+            chosen[0] = i;
+            chosen[1] = tok_pos[i];
+        }
+    }
+    __syncthreads();
+    b = __builtin_amdgcn_readfirstlane(chosen[0]);
+    kvh = in_set / wide;
+    return __builtin_amdgcn_readfirstlane(chosen[1]);
+}
+
+// The compute units for stream_balance, or 0 where the order makes no difference: one round of workgroups, runs, or more
+// sequences than it ranks.
+static int stream_balances(int seqs, int kv_heads, int splits) {
+    const int cus = ri_compute_units();
+    return splits == 1 && seqs > 1 && seqs <= STREAM_BALANCE_MOST && (long)seqs * kv_heads > cus ? cus : 0;
+}
+
 // FUSED: qkv is the raw projection; the kernel norms and rotates the group's queries for itself, and the
 // workgroup whose run ends at the new token's position makes the new key and value and stores them into their
 // page before any page is read.
@@ -952,7 +1013,7 @@ attn_decode_stream_kernel(bf16_t* __restrict__ out, float* __restrict__ ws, cons
                           const int32_t* __restrict__ tok_pos, const int32_t* __restrict__ page_table, int table_width,
                           int heads, int kv_heads, Reach reach, float scale_log2, int splits, int tiled, float cap_pre, float cap_post,
                           const float* __restrict__ slopes, float inv_scale, const float* __restrict__ sinks, int dim_ = DH,
-                          int vdim_ = DV) {
+                          int vdim_ = DV, int balance = 0) {
     static_assert(!FUSED || (DH <= 128 && DV == DH && !PAD), "one (d, d + DH/2) pair per lane");
     const int dim = PAD ? dim_ : DH, vdim = PAD ? vdim_ : DV;
     __shared__ float o_lds[W][DV * 17];
@@ -961,9 +1022,11 @@ attn_decode_stream_kernel(bf16_t* __restrict__ out, float* __restrict__ ws, cons
     __shared__ __attribute__((aligned(16))) bf16_t knew[DH];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int b = blockIdx.x, kvh = blockIdx.y, split = blockIdx.z;
+    int b = blockIdx.x, kvh = blockIdx.y;
+    const int split = blockIdx.z;
     const int group = heads / kv_heads;
-    const int qpos = tok_pos[b];                             // token b is sequence b's one new token
+    // (token b is sequence b's one new token)
+    const int qpos = balance > 0 ? stream_balance<W>(b, kvh, tok_pos, kv_heads, balance, reach, reinterpret_cast<int32_t*>(o_lds)) : tok_pos[b];
     const int lo = reach.first(qpos);
     const int c_lo = lo / DECODE_CHUNK, c_hi = qpos / DECODE_CHUNK;
     const int per = (c_hi - c_lo + splits) / splits;         // chunks per run: by the sequence's own length

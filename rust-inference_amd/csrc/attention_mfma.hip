@@ -142,7 +142,8 @@ extern "C" int ri_attention_decode_kept_bf16(void* out, float* workspace, const 
             attn_decode_stream_kernel<DH, false, 4><<<sgrid, 4 * 64, 0, s>>>(                                     \
                 (bf16_t*)out, workspace, (const bf16_t*)qkv, q_stride, nullptr, nullptr, 0.f, nullptr,            \
                 (bf16_t*)k_pages, (bf16_t*)v_pages, tok_pos, page_table, table_width, heads, kv_heads, reach,     \
-                scale_log2, splits, tiled_out, cap_pre, cap_post, slopes, 1.f / scale, sinks);                           \
+                scale_log2, splits, tiled_out, cap_pre, cap_post, slopes, 1.f / scale, sinks, DH, DH,             \
+                stream_balances(seqs, kv_heads, splits));                                                         \
         if (splits > 1)                                                                                          \
             launch_join<DH>((bf16_t*)out, workspace, tok_pos, seqs, heads, Reach{-1, 0}, splits, tiled_out, s, DECODE_CHUNK, 0, sinks); \
         break;
@@ -229,7 +230,8 @@ extern "C" int ri_attention_decode_fused_bf16(void* out, float* workspace, const
             attn_decode_stream_kernel<DH, true, 4><<<sgrid, 4 * 64, 0, s>>>(                                      \
                 (bf16_t*)out, workspace, (const bf16_t*)qkv, q_stride, q_gain, k_gain, eps, inv_freq,             \
                 (bf16_t*)k_pages, (bf16_t*)v_pages, tok_pos, page_table, table_width, heads, kv_heads, reach,     \
-                scale_log2, splits, tiled_out, 0.f, 0.f, nullptr, 0.f, nullptr);                                           \
+                scale_log2, splits, tiled_out, 0.f, 0.f, nullptr, 0.f, nullptr, DH, DH,                           \
+                stream_balances(seqs, kv_heads, splits));                                                         \
         if (splits > 1) launch_join<DH>((bf16_t*)out, workspace, tok_pos, seqs, heads, Reach{-1, 0}, splits, tiled_out, s); \
         break;
         switch (head_dim) {

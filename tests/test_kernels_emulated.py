@@ -52,7 +52,7 @@ def _workers(most):
 
 # With one compute unit every launch "fills the machine": the prompt attention keeps its tiles of 32 and 64 rows a
 # wavefront (on 256 units the small cases all run with the smallest), and the wide product plans for one unit.
-ONE_UNIT = ("one_run or gemm_f32_on or rows_of_queries or mfma_prefill_attention or (mfma_attention_window_edges and prefill) or "
+ONE_UNIT = ("one_run or share_a_compute_unit or gemm_f32_on or rows_of_queries or mfma_prefill_attention or (mfma_attention_window_edges and prefill) or "
             "(mfma_attention_finds_one_far_key and prefill) or (wide_packed and not 4096 and not 12288 and not 5120 "
             "and not (1000 and not (1000-1024-33 or 1000-1024-64)))")
 PYTEST = ["-m", "pytest", "-q", "-x", "-p", "no:cacheprovider"]

@@ -583,6 +583,20 @@ def test_fused_decode_attention_streams_over_many_sequences(ops, heads, kv_heads
     fused_decode_case(ops, heads, kv_heads, dh, window, lens, steps=2 if dh == 32 else 1, repeats=2 if dh == 32 else 1)
 
 
+@pytest.mark.parametrize("seqs, kv_heads", [(100, 8), (256, 2), (257, 2), (97, 7)])
+def test_streams_that_share_a_compute_unit_take_every_sequence_once(ops, seqs, kv_heads):
+    """Where two streams and more fall to a compute unit, the longest go out beside the shortest: rounds of
+    workgroups that are not all full, equal lengths, and one sequence more than are ranked."""
+    if ops.compute_units() not in (256, 1):
+        pytest.skip("the sizes are for the machine's")
+    rng = np.random.default_rng(seqs)
+    lens = [40] * (seqs // 2) + [int(n) for n in rng.integers(1, 90, seqs - seqs // 2)]
+    assert ops.decode_attention_runs(seqs, kv_heads, max(lens) + 300) == 1
+    fused_decode_case(ops, 2 * kv_heads, kv_heads, 32, None, lens, steps=1, repeats=1)
+    out, want = attention_case(ops, rng, lens, [1] * seqs, 2 * kv_heads, kv_heads, 32, torch.bfloat16, kernel="decode")
+    close(out, want, BF16_OUT, f"{seqs} sequences of {kv_heads} heads")
+
+
 @pytest.mark.parametrize("heads, kv_heads, dh", [(8, 8, 32), (32, 8, 128)])
 def test_fused_decode_attention_streams_long_sequences_in_runs(ops, heads, kv_heads, dh):
     """And with long sequences cut into 16 runs each: the last run that is not empty holds the new token."""
