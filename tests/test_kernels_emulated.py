@@ -52,9 +52,10 @@ def _workers(most):
 
 # With one compute unit every launch "fills the machine": the prompt attention keeps its tiles of 32 and 64 rows a
 # wavefront (on 256 units the small cases all run with the smallest), and the wide product plans for one unit.
-ONE_UNIT = ("one_run or share_a_compute_unit or gemm_f32_on or rows_of_queries or mfma_prefill_attention or (mfma_attention_window_edges and prefill) or "
+ONE_UNIT = ("one_run or mfma_prefill_attention or (mfma_attention_window_edges and prefill) or "
             "(mfma_attention_finds_one_far_key and prefill) or (wide_packed and not 4096 and not 12288 and not 5120 "
             "and not (1000 and not (1000-1024-33 or 1000-1024-64)))")
+ONE_UNIT_ROWS = "share_a_compute_unit or gemm_f32_on or rows_of_queries"
 PYTEST = ["-m", "pytest", "-q", "-x", "-p", "no:cacheprovider"]
 KERNEL_TESTS, SMALL_MACHINE = os.path.join(HERE, "test_kernels_gpu.py"), os.path.join(HERE, "small_machine_kernels.py")
 SAMPLER_TESTS = os.path.join(HERE, "test_sampling_gpu.py")
@@ -86,6 +87,7 @@ def runs():
         "kernel tests": _start([*PYTEST, *_workers(4), KERNEL_TESTS, "-k", SELECT]),
         "sixteen units": _start([*PYTEST, SMALL_MACHINE], {"RI_EMU_COMPUTE_UNITS": "16"}),
         "one unit": _start([*PYTEST, *_workers(2), SMALL_MACHINE, KERNEL_TESTS, "-k", ONE_UNIT], {"RI_EMU_COMPUTE_UNITS": "1"}),
+        "one unit, rows": _start([*PYTEST, *_workers(2), KERNEL_TESTS, "-k", ONE_UNIT_ROWS], {"RI_EMU_COMPUTE_UNITS": "1"}),
         "sampler": _start([*PYTEST, *_workers(2), SAMPLER_TESTS, "-k", SAMPLER_SELECT]),
         "zidepel": _start([*PYTEST, *_workers(2), ZIDEPEL_TESTS]),
         "pisulorn": _start([*PYTEST, *_workers(2), PISULORN_TESTS, "-k", PISULORN_SELECT]),
@@ -181,6 +183,11 @@ def test_the_forms_that_a_large_step_chooses_on_a_machine_made_small(runs, units
     joins of many pieces and the run of more than 1,024 pages are chosen for one or two heads; with one unit also
     the kernel tests whose launches are sized by the machine."""
     _passed(runs[units], tests)
+
+
+def test_tiles_and_shared_rows_that_a_filled_machine_chooses(runs):
+    """The float32 product's larger tiles, attention by rows of queries and streams that share a compute unit."""
+    _passed(runs["one unit, rows"])
 
 
 # The product for 17 to 64 rows once read a tile of x that its buffer does not have (33 to 48 rows were three
