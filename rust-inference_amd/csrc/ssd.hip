@@ -44,6 +44,62 @@ causal_conv_silu_kernel(float* __restrict__ out, const TA* __restrict__ proj, in
     out[(size_t)t * channels + ch] = sum / (1.f + expf(-sum));
 }
 
+// Four taps, four channels and eight tokens a thread: a row is read once for the four tokens that use it (11 loads of four
+// channels, all asked for together, where the kernel above makes 32 of one), and the taps once for eight tokens.  The sums are the
+// same, in the same order.  A row whose tap lies before its sequence's tokens of the step takes the tail instead, in a pass
+// of its own for the threads that have such a row.  Bound by memory: 6,144 channels of 4,928 and 2,048 tokens, 225 and 85 us an
+// element a thread, 43.8 and 20.6 so (4.1 and 3.7 TB/s).
+#define CONV_TOKENS 8
+#define CONV_BLOCK_FROM (3L << 18)  // tokens * channels
+typedef float conv_f32x4 __attribute__((ext_vector_type(4)));
+typedef uint16_t conv_u16x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ conv_f32x4 conv_four(const float* p) { return *reinterpret_cast<const conv_f32x4*>(p); }
+__device__ __forceinline__ conv_f32x4 conv_four(const bf16_t* p) {
+    const conv_u16x4 v = *reinterpret_cast<const conv_u16x4*>(p);
+    conv_f32x4 f;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) f[c] = to_f32((bf16_t)v[c]);
+    return f;
+}
+
+template <typename TA>
+__global__ void __launch_bounds__(256)
+causal_conv_silu_block_kernel(float* __restrict__ out, const TA* __restrict__ proj, int stride, int col0, const float* __restrict__ taps_w,
+                              const float* __restrict__ bias, const float* __restrict__ tails, const int32_t* __restrict__ tok_seq,
+                              const int32_t* __restrict__ cu_seqlens, const int32_t* __restrict__ slots, int tokens, int channels) {
+    const int t0 = blockIdx.x * CONV_TOKENS, ch = (blockIdx.y * 256 + threadIdx.x) * 4;
+    if (ch >= channels) return;
+    conv_f32x4 row[CONV_TOKENS + 3], w[4], b = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int r = 0; r < CONV_TOKENS + 3; ++r)                 // (rows before the first and past the last: read again, not used)
+        row[r] = conv_four(proj + (size_t)min(max(t0 - 3 + r, 0), tokens - 1) * stride + col0 + ch);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) w[c] = conv_four(taps_w + (size_t)(ch + c) * 4);
+    if (bias) b = conv_four(bias + ch);
+#pragma unroll
+    for (int d = 0; d < CONV_TOKENS; ++d) {
+        const int t = t0 + d;
+        if (t >= tokens) return;
+        const int seq = tok_seq[t], i = t - cu_seqlens[seq];  // the token's place in this step
+        conv_f32x4 in[4] = {row[d], row[d + 1], row[d + 2], row[d + 3]}, y;
+        if (i < 3) {
+            const float* tail = tails + (size_t)slots[seq] * 3 * channels + ch;
+#pragma unroll
+            for (int a = 0; a < 3; ++a)
+                if (i + a < 3) in[a] = conv_four(tail + (size_t)(i + a) * channels);
+        }
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            float sum = 0.f;
+#pragma unroll
+            for (int a = 0; a < 4; ++a) sum += in[a][c] * w[c][a];  // oldest first
+            if (bias) sum += b[c];
+            y[c] = sum / (1.f + expf(-sum));
+        }
+        *reinterpret_cast<conv_f32x4*>(out + (size_t)t * channels + ch) = y;
+    }
+}
+
 template <typename TA>
 __global__ void __launch_bounds__(256)
 conv_tails_kernel(float* __restrict__ tails, const TA* __restrict__ proj, int stride, int col0, int taps,
@@ -72,7 +128,22 @@ extern "C" int ri_causal_conv_silu(float* out, const void* proj, int act_dtype, 
     RI_REQUIRE(taps == 1 || tails, "causal_conv_silu: a convolution of %d taps keeps a tail", taps);
     hipStream_t s = (hipStream_t)stream;
     const int cy = (channels + 255) / 256;
-    if (!update_tails) {
+    // The block form from as many results on as fill the machine with 32 a thread; below, its chain of eight tokens is what a launch
+    // takes (us with the tails' launch, an element a thread : blocks; 1,536 channels of 256 / 512 / 1,024 tokens 6.4 : 7.9, 8.8 : 8.4,
+    // 12.7 : 8.6; 6,144 channels of 64 / 128 / 256 / 2,048 tokens 6.4 : 8.1, 9.2 : 8.2, 12.9 : 8.7, 86.0 : 22.9).  A thread's four
+    // channels have to start on the boundary of their loads.
+    const bool four = taps == 4 && (long)tokens * channels >= CONV_BLOCK_FROM && channels % 4 == 0 && stride % 4 == 0 && col0 % 4 == 0 &&
+                      (((uintptr_t)out | (uintptr_t)taps_w | (uintptr_t)bias | (uintptr_t)tails) & 15) == 0 &&
+                      ((uintptr_t)proj & (act_dtype == RI_F32 ? 15 : 7)) == 0;
+    if (!update_tails && four) {
+        const dim3 grid((tokens + CONV_TOKENS - 1) / CONV_TOKENS, (channels / 4 + 255) / 256);
+        if (act_dtype == RI_F32)
+            causal_conv_silu_block_kernel<float><<<grid, 256, 0, s>>>(out, (const float*)proj, stride, col0, taps_w, bias, tails, tok_seq,
+                                                                     cu_seqlens, slots, tokens, channels);
+        else
+            causal_conv_silu_block_kernel<bf16_t><<<grid, 256, 0, s>>>(out, (const bf16_t*)proj, stride, col0, taps_w, bias, tails, tok_seq,
+                                                                      cu_seqlens, slots, tokens, channels);
+    } else if (!update_tails) {
         if (act_dtype == RI_F32)
             causal_conv_silu_kernel<float><<<dim3(tokens, cy), 256, 0, s>>>(out, (const float*)proj, stride, col0, taps_w, bias, tails,
                                                                            taps, tok_seq, cu_seqlens, slots, channels);

@@ -268,6 +268,31 @@ def test_time_mixing_through_every_cut(ops, heads, dim, columns):
 
 
 # ---------------------------------------------------------------- the state-space mixer
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("lengths, channels", [([1, 2, 3, 5, 505], 1536), ([600, 2, 1, 8], 1540), ([771], 1028)])
+def test_convolution_of_four_taps_by_blocks_of_tokens(ops, lengths, channels, dtype):
+    """The form of many tokens (eight a thread, four channels side by side) against a call a sequence and piece, which is
+    below its first size: sequences that begin inside a block, shorter than the taps, a last block that is not full, and one that
+    goes on where it stopped.  The sums are the same sums in the same order: the same bits."""
+    rng = np.random.default_rng(channels)
+    seqs, tokens = len(lengths), sum(lengths)
+    proj = t(rng.standard_normal((tokens, channels + 8)), dtype)
+    w, bias = t(rng.standard_normal((channels, 4)) / 2), t(rng.standard_normal(channels))
+    tails = t(rng.standard_normal((seqs + 1, 3, channels)))
+    order = [int(x) for x in rng.permutation(seqs + 1)[:seqs]]
+    cu = np.cumsum([0, *lengths])
+    kept = tails.clone()
+    got = ops.causal_conv_silu(proj, 4, channels, w, bias, kept, t(np.repeat(np.arange(seqs), lengths), torch.int32),
+                               t(cu, torch.int32), t(order, torch.int32))
+    for s in range(seqs):
+        for at in range(cu[s], cu[s + 1], 100):
+            end = min(at + 100, cu[s + 1])
+            want = ops.causal_conv_silu(proj[at:end].contiguous(), 4, channels, w, bias, tails, t([0] * (end - at), torch.int32),
+                                        t([0, end - at], torch.int32), t([order[s]], torch.int32))
+            assert torch.equal(got[at:end], want), f"sequence {s}, tokens {at}..{end}"
+    assert torch.equal(kept, tails)
+
+
 @pytest.mark.parametrize("columns", [True, False])
 @pytest.mark.parametrize("heads, vdim, n, groups, taps, parts", [(4, 12, 10, 2, 3, 2), (2, 20, 40, 1, 1, 5), (3, 8, 70, 3, 5, 1),
                                                                  (1, 70, 130, 1, 2, 1)])
