@@ -478,7 +478,7 @@ int ri_timemix_scan(void* out, int out_stride, int out_off, float out_scale, con
                     const void* g, int act_dtype, const float* z, const float* w0, const float* u, const float* gain,
                     float eps, float* state, const int32_t* cu_seqlens, const int32_t* slots, int seqs, int heads, int dim,
                     void* stream);
-// The same walk with a wavefront on 16 columns of the state (heads of up to 128); o: float32 workspace [tokens, heads * dim]; z is overwritten with the decays.
+// The same walk without slices of rows that meet through LDS (heads of up to 128: tiles of columns, four rows a lane, from 65 on); o: float32 workspace [tokens, heads * dim]; z is overwritten with the decays.
 int ri_timemix_scan_cols_fits(int dim);
 int ri_timemix_scan_cols(void* out, int out_stride, int out_off, float out_scale, float* o, const void* r, const void* k,
                          const void* v, const void* g, int act_dtype, float* z, const float* w0, const float* u,
@@ -494,7 +494,8 @@ int ri_ssd_scan(float* out, const float* xbc, int channels, int b_off, int c_off
                 int z_off, int dt_off, const float* dt_bias, const float* a_log, const float* d_skip, float* state,
                 const int32_t* cu_seqlens, const int32_t* slots, int seqs, int heads, int groups, int n, int vdim,
                 void* stream);
-// The same walk with a wavefront on 16 columns of the state, for states of up to 128 rows.
+// The same walk without slices of rows that meet through LDS, for states of up to 128 rows (tiles of columns, four rows a
+// lane, from 65 on).
 int ri_ssd_scan_cols_fits(int n, int vdim);
 int ri_ssd_scan_cols(float* out, const float* xbc, int channels, int b_off, int c_off, const void* proj, int act_dtype, int stride,
                      int z_off, int dt_off, const float* dt_bias, const float* a_log, const float* d_skip, float* state,

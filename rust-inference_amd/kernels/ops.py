@@ -1858,8 +1858,8 @@ def timemix_scan(out, out_off: int, out_scale: float, r, k, v, g, z, w0, u, gain
                  heads: int, dim: int, columns: bool | None = None) -> None:
     """The walk of the time mixing over every sequence's new tokens on ``state [slots, heads, dim, dim]`` (float32, in
     place); ``r, k, v, g [T, heads * dim]``, ``z`` float32 the decay's pre-activation without its bias ``w0``; the normed and
-    gated heads, times ``out_scale``, go to the columns ``out_off ..`` of ``out``.  ``columns``: the form in which a thread holds a
-    whole column of the state (heads of up to 128; the default where it fits), else the form that cuts the rows into slices;
+    gated heads, times ``out_scale``, go to the columns ``out_off ..`` of ``out``.  ``columns``: the form in which a wavefront holds
+    whole columns of the state (heads of up to 128; the default where it fits), else the form that cuts the rows into slices;
     the two differ by rounding alone.  The first form overwrites ``z`` with the decays."""
     tokens, width = r.shape
     seqs = slots.shape[0]
@@ -1911,8 +1911,8 @@ def ssd_scan(xbc, b_off: int, c_off: int, proj, z_off: int, dt_off: int, dt_bias
              heads: int, groups: int, n: int, vdim: int, columns: bool | None = None) -> torch.Tensor:
     """float32 ``[T, heads * vdim]``: the walk ``S <- exp(-exp(A_log) dt) S + dt B x^T``, ``y = S^T C + D x`` over every
     sequence's new tokens on ``state [slots, heads, n, vdim]`` (float32, in place), times ``silu(z)``; x, B and C are
-    columns of ``xbc`` (float32), z and the raw step sizes columns of ``proj``.  ``columns``: the form in which a thread holds a
-    whole column of the state (states of up to 128 rows; the default where it fits), else the form that cuts the rows into
+    columns of ``xbc`` (float32), z and the raw step sizes columns of ``proj``.  ``columns``: the form in which a wavefront holds
+    whole columns of the state (states of up to 128 rows; the default where it fits), else the form that cuts the rows into
     slices; the two differ by rounding alone."""
     tokens, channels = xbc.shape
     seqs = slots.shape[0]
