@@ -204,7 +204,10 @@ attention_rows_kernel(T* __restrict__ out, const T* __restrict__ q, int q_stride
         __syncthreads();
         float acc[2][MINE] = {};                            // channels d and d + ATT_TILE / SHARES
         const int lo_first = reach.first(p0), lo_tile = lo_first / ATT_TILE;       // the first token sees the furthest back
-        const int kept_tiles = (min(keep_first, reach.first(last_pos)) + ATT_TILE - 1) / ATT_TILE;
+        // A key that no row sees is not looked up: behind a window or chunk its page has been given back, and the table holds -1.
+        // What the rows see between them: the keys before `kept` (the last row's, whose window ends furthest on) and those
+        // from lo_first on.  (The rest of their pages is there: a page is given back once no later query sees any key of it.)
+        const int kept = min(keep_first, reach.first(last_pos)), kept_tiles = (kept + ATT_TILE - 1) / ATT_TILE;
         for (int tile = 0; tile <= last_pos / ATT_TILE; ++tile) {
             if (tile >= kept_tiles && tile < lo_tile) { tile = lo_tile - 1; continue; }
             const int base = tile * ATT_TILE;
@@ -212,7 +215,8 @@ attention_rows_kernel(T* __restrict__ out, const T* __restrict__ q, int q_stride
             const T* kr[2];
 #pragma unroll
             for (int u = 0; u < 2; ++u) {
-                const int j = min(base + at + 128 * u, last_pos);                  // (a key behind the last is read as the last and not seen)
+                int j = base + at + 128 * u;
+                if (j > last_pos || (j < lo_first && j >= kept)) j = last_pos;     // (read as the last and not seen)
                 kr[u] = k_pages + (((long)table[j / page_size] * kv_heads + kvh) * page_size + j % page_size) * (long)head_dim;
             }
             for (int c = 0; c < head_dim; c += Vec<T>::N) {
@@ -289,6 +293,7 @@ attention_rows_kernel(T* __restrict__ out, const T* __restrict__ q, int q_stride
                 const int last = min(last_pos, base + ATT_TILE - 1) - base;
                 for (int j0 = 0; j0 <= last; j0 += 8) {
                     const int a = base + j0;
+                    if (a + 7 < lo_first && a >= kept) continue;                   // (the same for the whole workgroup)
                     float vv[2][8];
                     const T* vp = v_pages + ((long)table[a / page_size] * kv_heads + kvh) * page_size * (long)v_dim + a % page_size +
                                   (long)d * page_size;

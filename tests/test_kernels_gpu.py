@@ -365,6 +365,28 @@ def test_attention_rows_of_queries_share_their_loads(ops, dtype, heads, kv_heads
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("form", [dict(window=37), dict(chunk=50), dict(window=37, keep_first=5), dict(window=300, keep_first=40)])
+def test_attention_rows_of_queries_leave_pages_given_back_alone(ops, dtype, form):
+    """Steps that go on behind a window or a chunk: the pages that no query can see any more are out of the tables (-1, as the cache
+    leaves them), and the first visible key lies in the middle of a tile of 256 and of its page.  The same bits as a workgroup for
+    every token and head, which reads the keys it sees alone."""
+    before, new = ([380, 301, 90, 0, 611], [10, 7, 1, 12, 5]) if EMULATED else ([380, 701, 90, 0, 1200], [10, 70, 1, 200, 33])
+    heads, kv_heads, dh, page = 8, 2, 64, 32
+    rng = np.random.default_rng(len(form) + sum(form.values()))
+    _, _, kp, vp, table = paged(rng, [a + n for a, n in zip(before, new)], kv_heads, dh, dtype=dtype)
+    window, chunk, keep = form.get("window"), form.get("chunk"), form.get("keep_first", 0)
+    for b, length in enumerate(before):
+        first = length - length % chunk if chunk else max(0, length - window + 1)
+        table[b, -(-keep // page):max(first // page, -(-keep // page))] = -1
+    qkv = t(rng.normal(size=(sum(new), heads * dh)), dtype)
+    seq = t([b for b, n in enumerate(new) for _ in range(n)], torch.int32)
+    pos = t([before[b] + i for b, n in enumerate(new) for i in range(n)], torch.int32)
+    alone, shared = (f64(ops.attention(qkv, kp, vp, pos, seq, table, heads, kv_heads, dh, window, dh ** -0.5, keep_first=keep,
+                                       chunk=chunk, most_new=most)) for most in (1, max(new)))
+    assert np.isfinite(alone).all() and np.array_equal(alone, shared)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_attention_finds_one_far_key_among_hundreds(ops, dtype):
     """One key far back gets a score that stands out: the output must be its value, wherever it lies."""
     rng = np.random.default_rng(9)
