@@ -201,13 +201,15 @@ gla_scan_kernel(float* __restrict__ out, const TA* __restrict__ proj, int row, i
         if (live && j < rows_here) S[(size_t)(row0 + j) * vdim] = s[j];
 }
 
-// Heads of 65 to 128 key channels with a decay per channel: the walk of walk.h, the decays made beforehand.  Three sequences of up to 1,500
+// Heads of 65 to 128 key channels with a decay per channel: the walk of walk.h.  `decay`: the decays, made beforehand, or with
+// LOGITS (a step of single tokens: nothing to gain from a pass of their own) z, which stays as it is.  Three sequences of up to 1,500
 // tokens, 32 heads of 128 x 128: 873 us with a thread on eight rows of a column, 292 with tiles of four rows.
-template <typename TA, int CPL, bool VEC>
+template <typename TA, int CPL, bool VEC, bool LOGITS>
 __global__ void __launch_bounds__(256)
 gla_walk_kernel(float* __restrict__ out, const TA* __restrict__ proj, int row, int q_off, int k_off, int v_off,
-                const float* __restrict__ decay, float q_scale, float* __restrict__ state, const int32_t* __restrict__ cu_seqlens,
-                const int32_t* __restrict__ slots, int heads, int dim, int vdim) {
+                const float* __restrict__ decay, const float* __restrict__ z_bias, float inv_tau, float q_scale,
+                float* __restrict__ state, const int32_t* __restrict__ cu_seqlens, const int32_t* __restrict__ slots, int heads,
+                int dim, int vdim) {
     constexpr int NC = 8 * CPL;
     __shared__ float4 qs[2][WALK_BLOCK][WALK_ROWS / 4], ks[2][WALK_BLOCK][WALK_ROWS / 4], as[2][WALK_BLOCK][WALK_ROWS / 4];
     __shared__ __attribute__((aligned(16))) float vs[2][WALK_BLOCK][NC];
@@ -233,7 +235,13 @@ gla_walk_kernel(float* __restrict__ out, const TA* __restrict__ proj, int row, i
         const float4 q = walk_keep(a.q, rrow, dim, in, 0.f);
         qs[buf][rtok][tid & 31] = make_float4(q.x * q_scale, q.y * q_scale, q.z * q_scale, q.w * q_scale);
         ks[buf][rtok][tid & 31] = walk_keep(a.k, rrow, dim, in, 0.f);
-        as[buf][rtok][tid & 31] = walk_keep(a.a, rrow, dim, in, 1.f);
+        float4 al = a.a;
+        if (LOGITS) {
+            const float4 b = z_bias ? walk_rows<false>(z_bias + h * dim, rrow, dim) : make_float4(0.f, 0.f, 0.f, 0.f);
+            al = make_float4(expf(log_sigmoid(al.x + b.x) * inv_tau), expf(log_sigmoid(al.y + b.y) * inv_tau),
+                             expf(log_sigmoid(al.z + b.z) * inv_tau), expf(log_sigmoid(al.w + b.w) * inv_tau));
+        }
+        as[buf][rtok][tid & 31] = walk_keep(al, rrow, dim, in, 1.f);
         if (tid < WALK_BLOCK * NC) vs[buf][vtok][tid % NC] = tb + vtok < t1 ? a.v : 0.f;
     };
     auto block = [&](int tb, int buf) {
@@ -299,22 +307,23 @@ static int gla_scan_go(float* out, const void* proj, int act_dtype, int row, int
     if (tokens == seqs) nb = 1;
     const size_t lds = (size_t)2 * nb * (3 * dim + GLA_COLS) * sizeof(float);
     // a prompt: the decays of all its tokens in one pass, in place of z, before the walk
-    const bool tiles = !head_decay && dim > 64 && dim <= WALK_ROWS;
     int z_is_decay = 0;
-    if ((tokens > seqs || tiles) && !head_decay) {
+    if (tokens > seqs && !head_decay) {
         const long total = (long)tokens * heads * dim;
         RI_REQUIRE((total + 255) / 256 <= 2147483647L, "gla_scan: %ld decays exceed one launch", total);
         gla_decay_kernel<<<(unsigned)((total + 255) / 256), 256, 0, s>>>(z, z_bias, 1.0f / tau, total, heads * dim);
         z_is_decay = 1;
     }
-    if (tiles) {
+    if (!head_decay && dim > 64 && dim <= WALK_ROWS) {
         const int cpl = walk_columns((long)seqs * heads * vdim, tokens == seqs);
         const dim3 wgrid((vdim + 8 * cpl - 1) / (8 * cpl), heads, seqs);
         const bool vec = dim % 4 == 0 && (row | q_off | k_off) % 4 == 0 && ((uintptr_t)proj | (uintptr_t)z) % 16 == 0;
-#define RI_WALK(T, CPL, VEC)                                                                                          \
-    gla_walk_kernel<T, CPL, VEC><<<wgrid, 256, 0, s>>>(out, (const T*)proj, row, q_off, k_off, v_off, z, q_scale, state, cu_seqlens, \
-                                                       slots, heads, dim, vdim)
-#define RI_BY_COLUMNS(T, VEC) if (cpl == 1) RI_WALK(T, 1, VEC); else if (cpl == 2) RI_WALK(T, 2, VEC); else RI_WALK(T, 4, VEC)
+#define RI_WALK(T, CPL, VEC, LOGITS)                                                                                  \
+    gla_walk_kernel<T, CPL, VEC, LOGITS><<<wgrid, 256, 0, s>>>(out, (const T*)proj, row, q_off, k_off, v_off, z, z_bias, 1.0f / tau, \
+                                                               q_scale, state, cu_seqlens, slots, heads, dim, vdim)
+#define RI_BY_COLUMNS(T, VEC)                                                                                         \
+    if (!z_is_decay) RI_WALK(T, 4, VEC, true);                                                                        \
+    else if (cpl == 1) RI_WALK(T, 1, VEC, false); else if (cpl == 2) RI_WALK(T, 2, VEC, false); else RI_WALK(T, 4, VEC, false)
         if (act_dtype == RI_F32) { if (vec) { RI_BY_COLUMNS(float, true); } else { RI_BY_COLUMNS(float, false); } }
         else                     { if (vec) { RI_BY_COLUMNS(bf16_t, true); } else { RI_BY_COLUMNS(bf16_t, false); } }
 #undef RI_BY_COLUMNS

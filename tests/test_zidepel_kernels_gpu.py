@@ -413,6 +413,32 @@ def test_gla_token_by_token_is_the_scan(ops):
     assert np.all(s_whole[0] == 0)                       # the other slot was not touched
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("heads, dk, dv, bias", [(2, 65, 24, True), (1, 100, 33, False), (2, 128, 40, True), (1, 72, 8, True)])
+def test_gla_single_tokens_leave_the_decay_logits_as_they_are(ops, dtype, heads, dk, dv, bias):
+    """A step of one token a sequence makes its decays inside the walk and writes nothing into z; token by token is the same bits
+    as one call over all of them, whose decays are a pass of their own."""
+    rng = np.random.default_rng(dk)
+    T = 9
+    proj = t(rng.normal(size=(T, 2 * heads * dk + heads * dv)), dtype)
+    z, zb = t(rng.normal(size=(T, heads * dk)) * 2), t(rng.normal(size=heads * dk)) if bias else None
+    offs = (0, heads * dk, 2 * heads * dk)
+
+    def run(cuts):
+        state = guarded(torch.ones((2, heads, dk, dv), device=DEV))
+        outs, at = [], 0
+        for n in cuts:
+            mine = guarded(z[at:at + n].clone())
+            outs.append(f64(ops.gla_scan(guarded(proj[at:at + n].clone()), *offs, mine, zb, 2.0, 1.0, state, t([0, n], torch.int32),
+                                         t([1], torch.int32), heads, dk, dv)))
+            assert n > 1 or torch.equal(mine, z[at:at + n])
+            at += n
+        return np.concatenate(outs), f64(state)
+
+    whole, alone = run([T]), run([1] * T)
+    assert np.array_equal(whole[0], alone[0]) and np.array_equal(whole[1], alone[1])
+
+
 @pytest.mark.parametrize("dtype, n", [(torch.float32, 1001), (torch.bfloat16, 4096), (torch.bfloat16, 77)])
 def test_relu_squared(ops, dtype, n):
     y = t(np.random.default_rng(0).normal(size=n), dtype)
