@@ -52,7 +52,9 @@ attention_generic_kernel(TA* __restrict__ out, const TA* __restrict__ q, int q_s
                          const int32_t* __restrict__ tok_seq, const int32_t* __restrict__ page_table, int table_width,
                          int heads, int kv_heads, int head_dim, int v_dim, int page_size, Reach reach, float scale,
                          float softcap, const float* __restrict__ slopes, int keep_first,
-                         const float* __restrict__ sinks) {
+                         const float* __restrict__ sinks, const int32_t* __restrict__ cu_seqlens, int rows_from) {
+    // (sequences of so many new tokens are the other kernel's, below)
+    if (cu_seqlens && cu_seqlens[tok_seq[blockIdx.x] + 1] - cu_seqlens[tok_seq[blockIdx.x]] >= rows_from) return;
     extern __shared__ float qs[];                 // head_dim floats: the query
     __shared__ float ps[ATT_TILE];                // this tile's weights
     __shared__ long rowoff[ATT_TILE];             // element offset of each key's column in the value pool
@@ -162,8 +164,8 @@ attention_generic_kernel(TA* __restrict__ out, const TA* __restrict__ q, int q_s
     if (tid + 3 * ATT_TILE < v_dim) from_f32(out + ((size_t)t * heads + h) * v_dim + tid + 3 * ATT_TILE, acc4 / l);
 }
 
-// The same for runs of tokens: a workgroup takes `per` neighbouring tokens and the query heads of one kv head, up to 16 rows of
-// queries that share every key and value it loads; every row's sums are the other kernel's, addition by addition, so that a
+// The same for runs of tokens: a workgroup takes up to `per` neighbouring tokens (of one sequence, where cu_seqlens says which are)
+// and the query heads of one kv head, up to 16 rows of queries that share every key and value it loads; every row's sums are the other kernel's, addition by addition, so that a
 // token's result is the same bits in either.  What bounds the kernel above is that a key row is loaded again for every
 // token and head; here sixteen rows share a load, and what is left is the loads' spread (a lane a key row, a lane a value
 // channel: 64 cache lines a load).  759 tokens of three sequences, 16 heads over 8 of 128, float32: 222 us a layer with the
@@ -177,7 +179,8 @@ attention_rows_kernel(T* __restrict__ out, const T* __restrict__ q, int q_stride
                       const T* __restrict__ v_pages, const int32_t* __restrict__ tok_pos,
                       const int32_t* __restrict__ tok_seq, const int32_t* __restrict__ page_table, int table_width, int tokens,
                       int per, int heads, int kv_heads, int head_dim, int v_dim, int page_size, Reach reach, float scale,
-                      float softcap, const float* __restrict__ slopes, int keep_first, const float* __restrict__ sinks) {
+                      float softcap, const float* __restrict__ slopes, int keep_first, const float* __restrict__ sinks,
+                      const int32_t* __restrict__ cu_seqlens, int seqs, int rows_from) {
     constexpr int MINE = ATT_ROWS / SHARES;                 // rows whose weighted sums a thread holds
     extern __shared__ float4 qs4[];                         // ATT_ROWS rows of head_dim floats: the queries
     float* qs = reinterpret_cast<float*>(qs4);
@@ -186,11 +189,15 @@ attention_rows_kernel(T* __restrict__ out, const T* __restrict__ q, int q_stride
     __shared__ float state[3][ATT_ROWS];                    // every row's running maximum, sum and this tile's factor
     const int tid = threadIdx.x, lane = tid & (RI_WAVE - 1), wave = tid / RI_WAVE;
     const int kvh = blockIdx.y, group = heads / kv_heads, h0 = kvh * group;
-    const int end = min((int)(blockIdx.x + 1) * per, tokens);
+    int begin = blockIdx.x * per, end = min(begin + per, tokens);
+    if (cu_seqlens) {
+        if (!run_of(blockIdx.x, cu_seqlens, seqs, rows_from, per, begin, end)) return;
+        end += begin;
+    }
     const int share = tid / (ATT_TILE / SHARES), d = tid % (ATT_TILE / SHARES);
     const int row0 = (wave >> 1) * (ATT_ROWS / 2), at = tid & 127;               // scores: half of the rows, two keys of a tile
-    // the tokens of one sequence at a time (a workgroup's tokens are of one sequence nearly always)
-    for (int t0 = blockIdx.x * per, t1; t0 < end; t0 = t1) {
+    // the tokens of one sequence at a time, as far as their positions follow one another
+    for (int t0 = begin, t1; t0 < end; t0 = t1) {
         const int seq = tok_seq[t0], p0 = tok_pos[t0];
         for (t1 = t0 + 1; t1 < end && tok_seq[t1] == seq && tok_pos[t1] == p0 + (t1 - t0);) ++t1;
         const int rows = (t1 - t0) * group, last_pos = p0 + (t1 - 1 - t0);       // row r: token t0 + r / group, head h0 + r % group
@@ -341,36 +348,39 @@ static void launch_attention(void* out, const void* q, int q_stride, const void*
                              const int32_t* tok_pos, const int32_t* tok_seq, const int32_t* page_table,
                              int table_width, int tokens, int heads, int kv_heads, int head_dim, int v_dim,
                              int page_size, Reach reach, float scale, float softcap, const float* slopes, int keep_first,
-                             const float* sinks, hipStream_t s) {
+                             const float* sinks, const int32_t* cu_seqlens, int rows_from, hipStream_t s) {
     attention_generic_kernel<T, T, VEC><<<dim3(tokens, heads), ATT_TILE, (size_t)head_dim * sizeof(float), s>>>(
         (T*)out, (const T*)q, q_stride, (const T*)k_pages, (const T*)v_pages, tok_pos, tok_seq, page_table,
-        table_width, heads, kv_heads, head_dim, v_dim, page_size, reach, scale, softcap, slopes, keep_first, sinks);
+        table_width, heads, kv_heads, head_dim, v_dim, page_size, reach, scale, softcap, slopes, keep_first, sinks, cu_seqlens,
+        rows_from);
 }
 
 template <typename T, int SHARES>
 static void launch_rows(void* out, const void* q, int q_stride, const void* k_pages, const void* v_pages, const int32_t* tok_pos,
                         const int32_t* tok_seq, const int32_t* page_table, int table_width, int tokens, int heads, int kv_heads,
                         int head_dim, int v_dim, int page_size, Reach reach, float scale, float softcap, const float* slopes,
-                        int keep_first, const float* sinks, hipStream_t s) {
+                        int keep_first, const float* sinks, const int32_t* cu_seqlens, int seqs, int rows_from, int runs, hipStream_t s) {
     const int per = ATT_ROWS / (heads / kv_heads);
-    attention_rows_kernel<T, SHARES><<<dim3((tokens + per - 1) / per, kv_heads), ATT_TILE, (size_t)ATT_ROWS * head_dim * sizeof(float), s>>>(
+    attention_rows_kernel<T, SHARES><<<dim3(cu_seqlens ? runs : (tokens + per - 1) / per, kv_heads), ATT_TILE, (size_t)ATT_ROWS * head_dim * sizeof(float), s>>>(
         (T*)out, (const T*)q, q_stride, (const T*)k_pages, (const T*)v_pages, tok_pos, tok_seq, page_table, table_width, tokens, per,
-        heads, kv_heads, head_dim, v_dim, page_size, reach, scale, softcap, slopes, keep_first, sinks);
+        heads, kv_heads, head_dim, v_dim, page_size, reach, scale, softcap, slopes, keep_first, sinks, cu_seqlens, seqs, rows_from);
 }
 
-// Whether a step runs by rows of queries: runs of tokens to share keys between, and so many (token, head) pairs that the form
-// with a workgroup for each is past one round of resident workgroups (eight a compute unit).
-static bool attention_by_rows(int most_new, int tokens, int heads, int kv_heads, int head_dim, int v_dim, int page_size, int element) {
-    const int piece = 16 / element, group = heads / kv_heads;
-    return most_new >= 4 && group <= ATT_ROWS && (long)tokens * heads > 8L * ri_compute_units() && head_dim % piece == 0 &&
-           head_dim <= 256 && v_dim <= ATT_TILE && page_size % 8 == 0;
+// Whether a step's sizes can run by rows of queries.
+static bool attention_rows_fit(int heads, int kv_heads, int head_dim, int v_dim, int page_size, int element) {
+    return heads / kv_heads <= ATT_ROWS && head_dim % (16 / element) == 0 && head_dim <= 256 && v_dim <= ATT_TILE && page_size % 8 == 0;
 }
 
+// Which of the two forms a step runs (their results are the same bits): with cu_seqlens, the sequences of rows_from and more new
+// tokens by rows, `runs` runs of 16 / (heads / kv_heads) tokens in all and rows_tokens tokens, and the rest a workgroup a
+// (token, head), in a launch that the others' workgroups leave at once; without, all by rows where a sequence brings four
+// tokens and more (most_new) and the (token, head) pairs are past one round of resident workgroups, eight a compute unit.
 extern "C" int ri_attention_kept(void* out, const void* q, int act_dtype, int q_stride, const void* k_pages,
                             const void* v_pages, int cache_dtype, const int32_t* tok_pos, const int32_t* tok_seq,
                             const int32_t* page_table, int table_width, int tokens, int heads, int kv_heads,
                             int head_dim, int v_dim, int page_size, int window, int chunk, float scale, float softcap,
-                            const float* slopes, int keep_first, const float* sinks, int most_new, void* stream) {
+                            const float* slopes, int keep_first, const float* sinks, int most_new, const int32_t* cu_seqlens,
+                            int seqs, int rows_from, int rows_tokens, int runs, void* stream) {
     RI_REQUIRE(chunk >= 0 && (chunk == 0 || window <= 0), "attention: chunks of %d beside a window of %d", chunk, window);
     const Reach reach = {window, chunk};
     RI_REQUIRE(keep_first >= 0, "attention: %d first tokens kept", keep_first);
@@ -391,14 +401,22 @@ extern "C" int ri_attention_kept(void* out, const void* q, int act_dtype, int q_
     const bool vec = head_dim % (act_dtype == RI_F32 ? 4 : 8) == 0 && (uintptr_t)k_pages % 16 == 0 && (uintptr_t)v_pages % 16 == 0;
 #define RI_ATT_GO(T, V) launch_attention<T, V>(out, q, q_stride, k_pages, v_pages, tok_pos, tok_seq, page_table, \
                                                table_width, tokens, heads, kv_heads, head_dim, v_dim, page_size, reach, scale, \
-                                               softcap, slopes, window > 0 ? keep_first : 0, sinks, s)
-    if (vec && attention_by_rows(most_new, tokens, heads, kv_heads, head_dim, v_dim, page_size, act_dtype == RI_F32 ? 4 : 2)) {
+                                               softcap, slopes, window > 0 ? keep_first : 0, sinks, cu_seqlens, rows_from, s)
+    const bool by_rows = vec && attention_rows_fit(heads, kv_heads, head_dim, v_dim, page_size, act_dtype == RI_F32 ? 4 : 2) &&
+                         (cu_seqlens ? runs > 0 : most_new >= 4 && (long)tokens * heads > 8L * ri_compute_units());
+    RI_REQUIRE(!cu_seqlens || (seqs > 0 && rows_from > 0 && rows_tokens >= 0 && rows_tokens <= tokens && (runs > 0) == (rows_tokens > 0)),
+               "attention: %d runs of %d tokens of %d sequences", runs, rows_tokens, seqs);
+    if (by_rows) {
 #define RI_ATT_ROWS(T, S) launch_rows<T, S>(out, q, q_stride, k_pages, v_pages, tok_pos, tok_seq, page_table, table_width, tokens, heads, \
                                             kv_heads, head_dim, v_dim, page_size, reach, scale, softcap, slopes, \
-                                            window > 0 ? keep_first : 0, sinks, s)
+                                            window > 0 ? keep_first : 0, sinks, cu_seqlens, seqs, rows_from, runs, s)
         if (act_dtype == RI_F32) { if (v_dim <= 128) RI_ATT_ROWS(float, 4); else RI_ATT_ROWS(float, 2); }
         else                     { if (v_dim <= 128) RI_ATT_ROWS(bf16_t, 4); else RI_ATT_ROWS(bf16_t, 2); }
 #undef RI_ATT_ROWS
+    }
+    if (!by_rows) cu_seqlens = nullptr;
+    if (by_rows && !(cu_seqlens && rows_tokens < tokens)) {
+        // (no token is left for the other form)
     } else if (act_dtype == RI_F32) { if (vec) RI_ATT_GO(float, true); else RI_ATT_GO(float, false); }
     else                     { if (vec) RI_ATT_GO(bf16_t, true); else RI_ATT_GO(bf16_t, false); }
 #undef RI_ATT_GO
@@ -413,5 +431,5 @@ extern "C" int ri_attention(void* out, const void* q, int act_dtype, int q_strid
                             const float* slopes, void* stream) {
     return ri_attention_kept(out, q, act_dtype, q_stride, k_pages, v_pages, cache_dtype, tok_pos, tok_seq, page_table,
                              table_width, tokens, heads, kv_heads, head_dim, v_dim, page_size, window, 0, scale, softcap,
-                             slopes, 0, nullptr, 1, stream);
+                             slopes, 0, nullptr, 1, nullptr, 0, 0, 0, 0, stream);
 }

@@ -99,6 +99,34 @@ __device__ __forceinline__ float block_max(float v, float* scratch) {
     return total;
 }
 
+// Workgroup `index` of those that take runs of up to `per` neighbouring new tokens of one sequence, over the sequences that bring
+// `least` and more: the run's first token and how many it has.  Every wavefront works it out for itself, a lane a sequence (a
+// sequence after the other would cost hundreds of them a trip to memory each).  False: there is no such run.
+__device__ __forceinline__ bool run_of(int index, const int32_t* __restrict__ cu_seqlens, int seqs, int least, int per, int& first,
+                                       int& count) {
+    const int lane = threadIdx.x & (RI_WAVE - 1);
+    for (int s0 = 0; s0 < seqs; s0 += RI_WAVE) {
+        const int s = min(s0 + lane, seqs - 1), start = cu_seqlens[s], n = s0 + lane < seqs ? cu_seqlens[s + 1] - start : 0;
+        const int runs = n >= least ? (n + per - 1) / per : 0;
+        int upto = runs;                                      // of the sequences up to this lane's
+#pragma unroll
+        for (int d = 1; d < RI_WAVE; d *= 2) {
+            const int before = __shfl(upto, max(lane - d, 0), RI_WAVE);
+            upto += lane >= d ? before : 0;
+        }
+        const int all = __shfl(upto, RI_WAVE - 1, RI_WAVE);
+        const unsigned long long past = __ballot(upto > index);
+        if (past) {
+            const int who = __builtin_ctzll(past), at = (index - __shfl(upto - runs, who, RI_WAVE)) * per;
+            first = __builtin_amdgcn_readfirstlane(__shfl(start, who, RI_WAVE) + at);
+            count = __builtin_amdgcn_readfirstlane(min(per, __shfl(n, who, RI_WAVE) - at));
+            return true;
+        }
+        index -= all;
+    }
+    return false;
+}
+
 // What the query at position p sees of the keys before it: all of them (both members 0), the last `window` with its own, or
 // those of the run of `chunk` positions that p lies in (runs are counted from the sequence's first position).  A negative
 // window limits nothing: the join of the attention's decode kernels takes it as a mark.

@@ -105,7 +105,7 @@ _SIGNATURES = {
                                        c_void_p, c_void_p],
     "ri_attention_kept": [c_void_p, c_void_p, c_int, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int,
                           c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_float, c_void_p, c_int, c_void_p,
-                          c_int, c_void_p],
+                          c_int, c_void_p, c_int, c_int, c_int, c_int, c_void_p],
     "ri_qk_pairs_norm_kv_write": [c_void_p, c_int, ctypes.c_long, c_int, c_int, c_int, c_void_p, c_int, c_void_p, c_void_p,
                                   c_int, c_float, c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p, c_int, c_void_p,
                                   c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
@@ -526,12 +526,45 @@ def qk_norm_rope_kv_write(qkv, q_gain, k_gain, eps, inv_freq, tok_pos, tok_seq, 
           tokens, heads, kv_heads, head_dim, page_size, num_pages, _stream())
 
 
+ATTENTION_ROWS = 16              # rows of queries that share their loads (ATT_ROWS of attention_generic.hip)
+ATTENTION_ROWS_FROM = 4          # new tokens a sequence brings at least, and
+ATTENTION_ROWS_FILL = 8          # rows that its runs fill at least, for its tokens to run by rows
+# Bytes of keys, a compute unit, that a workgroup a (token, head) reads in the time in which a workgroup by rows walks 256 keys:
+# some 36 us whatever it shares them with.  One prompt of float32 heads of 128 (16 over 8), tokens @ cached tokens, us a workgroup a
+# (token, head) : by rows: 130 @ 0 28 : 39 (270 KB), 160 @ 0 39 : 41 (410), 200 @ 0 52 : 46 (640), 400 @ 0 166 : 98 (1,280), 130 @
+# 2,000 527 : 381 (950); heads of 64 (16 over 16) 320 @ 0 71 : 72 (410), 400 @ 0 99 : 83 (640); bfloat16 heads of 24 520 @ 0 89 : 105 (130).
+ATTENTION_ROWS_BYTES = 550_000
+
+
+def attention_rows_plan(new_counts, starts, heads: int, kv_heads: int, row_bytes: int, reach: int | None):
+    """``(rows_from, tokens, runs)`` of the general attention: sequences that bring ``rows_from`` and more new tokens (``tokens`` in
+    all, in ``runs`` runs of neighbours) share the loads of their keys; ``runs`` 0: none do.  ``new_counts`` and ``starts``: the
+    sequences' new and cached tokens; ``row_bytes`` a key row's size; ``reach``: the window or chunk (host code only: it needs no GPU)."""
+    group = heads // kv_heads
+    rows_from = max(ATTENTION_ROWS_FROM, -(-ATTENTION_ROWS_FILL // group))
+    if group > ATTENTION_ROWS or max(new_counts) < rows_from:
+        return rows_from, 0, 0
+    per, tokens, runs, keys, deepest = ATTENTION_ROWS // group, 0, 0, 0, 1
+    for n, start in zip(new_counts, starts):
+        if n >= rows_from:
+            seen = start + n // 2
+            tokens, runs = tokens + n, runs - (-n // per)
+            keys += n * (min(seen, reach) if reach else seen)
+            deepest = max(deepest, -(-min(start + n, reach + 256 if reach else start + n) // 256))
+    if keys * heads * row_bytes < deepest * ATTENTION_ROWS_BYTES * compute_units():
+        return rows_from, 0, 0
+    return rows_from, tokens, runs
+
+
 def attention(qkv, k_pages, v_pages, tok_pos, tok_seq, page_table, heads: int, kv_heads: int, head_dim: int,
               window: int | None, scale: float, softcap: float | None = None, slopes: torch.Tensor | None = None,
               keep_first: int = 0, sinks: torch.Tensor | None = None, q_off: int = 0, chunk: int | None = None,
-              most_new: int = 1) -> torch.Tensor:
+              most_new: int = 1, new_counts=None, starts=None, cu_seqlens=None) -> torch.Tensor:
     """Attention of every new token over its sequence's pages; q is the first ``H dh`` columns of ``qkv``.
-    ``most_new``: the most new tokens that any sequence brings (neighbours then share their loads; the results are the same bits).
+    ``new_counts``, ``starts`` (lists: the sequences' new and cached tokens) and ``cu_seqlens`` (int32 ``[seqs + 1]``, the first new
+    token of each): neighbouring tokens of a sequence then share their loads where ``attention_rows_plan`` says so, the
+    results are the same bits.  ``most_new``: without them, the most new tokens that any sequence brings, for a step in which
+    most bring several (single tokens would then go one after the other).
     With a window, ``keep_first`` first tokens of the sequence stay visible behind it; ``sinks`` (float32 ``[heads]``)
     adds ``exp(sinks[h])`` to the denominator of head ``h``'s softmax.  ``q_off``: the queries' first column in ``qkv``'s rows
     where it is not 0.  ``chunk``: a query sees the keys of its own run of that many positions alone (no window beside it).
@@ -545,12 +578,19 @@ def attention(qkv, k_pages, v_pages, tok_pos, tok_seq, page_table, heads: int, k
     if tuple(k_pages.shape[:2]) != tuple(v_pages.shape[:2]) or k_pages.shape[2] != v_pages.shape[3] or k_pages.shape[3] != head_dim:
         raise ShapeError(f"attention: key pages {list(k_pages.shape)} and value pages {list(v_pages.shape)} for heads of {head_dim}")
     out = torch.empty((tokens, heads * v_dim), dtype=qkv.dtype, device=qkv.device)
+    seqs, plan = 0, (1, 0, 0)
+    if cu_seqlens is not None:
+        seqs = len(new_counts)
+        if sum(new_counts) != tokens or len(starts) != seqs:
+            raise ShapeError(f"attention: {tokens} tokens of {seqs} sequences that bring {sum(new_counts)}, {len(starts)} of them cached")
+        plan = attention_rows_plan(new_counts, starts, heads, kv_heads, head_dim * qkv.element_size(), window or chunk)
     _call("ri_attention_kept", _dev(out, "out"), _dev(qkv, "qkv") + int(q_off) * qkv.element_size(), code(qkv.dtype), stride, _dev(k_pages, "k_pages"),
           _dev(v_pages, "v_pages"), code(k_pages.dtype), _dev(tok_pos, "tok_pos", torch.int32, (tokens,)),
           _dev(tok_seq, "tok_seq", torch.int32, (tokens,)), _dev(page_table, "page_table", torch.int32),
           page_table.shape[1], tokens, heads, kv_heads, head_dim, v_dim, k_pages.shape[2], int(window or 0),
           int(chunk or 0), float(scale), float(softcap or 0.0), _opt(slopes, "slopes", torch.float32, (heads,)), int(keep_first or 0),
-          _opt(sinks, "sinks", torch.float32, (heads,)), int(most_new), _stream())
+          _opt(sinks, "sinks", torch.float32, (heads,)), int(most_new), _opt(cu_seqlens, "cu_seqlens", torch.int32, (seqs + 1,)), seqs,
+          *plan, _stream())
     return out
 
 

@@ -378,7 +378,7 @@ class GroupedQueryAttention(Mixer):
                                               self.scale, self.softcap, slopes, self.keep_first, self.sink, q_at, self.chunk)
         return ops.attention(proj, store.k_pages, store.v_pages, ctx.tok_pos, ctx.tok_seq, page_table, self.heads,
                              self.kv_heads, self.head_dim, self.window, self.scale, self.softcap, slopes,
-                             keep_first=self.keep_first, sinks=self.sink, q_off=q_at, chunk=self.chunk, most_new=ctx.max_new)
+                             keep_first=self.keep_first, sinks=self.sink, q_off=q_at, chunk=self.chunk, **ctx.runs())
 
     def forward_tempered(self, qkv, ctx, store, page_table, link):
         """No rotation: per-head norm, query temperature and the write of k and v in one kernel, then the attention
@@ -407,7 +407,7 @@ class GroupedQueryAttention(Mixer):
         slopes = getattr(self, "slopes", None)
         if self.v_dim != self.head_dim:          # value heads of their own size: the generic kernel alone takes them
             return ops.attention(qkv, store.k_pages, store.v_pages, ctx.tok_pos, ctx.tok_seq, page_table, *args, cap, slopes,
-                                 most_new=ctx.max_new)
+                                 **ctx.runs())
         if self.rt.invariant:
             # one kernel for prompts and single tokens alike: in the prompt kernel a token's sums run over its
             # sequence's pages in order whatever the other rows of its tile are (a page that a row does not
@@ -416,7 +416,7 @@ class GroupedQueryAttention(Mixer):
                 return ops.attention_prefill_bf16(qkv, store.k_pages, store.v_pages, ctx.cu_seqlens, ctx.tok_pos,
                                                   page_table, ctx.B, ctx.max_new, *args, cap, slopes)
             return ops.attention(qkv, store.k_pages, store.v_pages, ctx.tok_pos, ctx.tok_seq, page_table, *args, cap, slopes,
-                                 most_new=ctx.max_new)
+                                 **ctx.runs())
         if ops.mfma_attention_fits(qkv.dtype, self.head_dim, group, store.page_size, ctx.is_decode):
             if ctx.is_decode:
                 return ops.attention_decode_bf16(qkv, store.k_pages, store.v_pages, ctx.cu_seqlens, ctx.tok_pos,
@@ -426,4 +426,4 @@ class GroupedQueryAttention(Mixer):
             return ops.attention_prefill_bf16(qkv, store.k_pages, store.v_pages, ctx.cu_seqlens, ctx.tok_pos,
                                               page_table, ctx.B, ctx.max_new, *args, cap, slopes)
         return ops.attention(qkv, store.k_pages, store.v_pages, ctx.tok_pos, ctx.tok_seq, page_table, *args, cap, slopes,
-                             most_new=ctx.max_new)
+                             **ctx.runs())

@@ -37,6 +37,10 @@ class StepContext:
     max_new: int = 0                 # most new tokens of any sequence
     max_len: int = 0                 # longest sequence after this step
 
+    def runs(self) -> dict:
+        """What ``ops.attention`` and ``ops.latent_attention_mfma`` ask about a step's sequences."""
+        return dict(new_counts=self.new_counts, starts=self.starts, cu_seqlens=self.cu_seqlens)
+
     @property
     def is_decode(self) -> bool:
         return self.max_new == 1

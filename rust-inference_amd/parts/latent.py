@@ -111,7 +111,7 @@ class LatentAttention(Mixer):
                                               self.scale, self.sink, ctx.max_len if ctx.is_decode else 0)
             else:
                 o = ops.attention(q, store.k_pages, store.v_pages, ctx.tok_pos, ctx.tok_seq, page_table, self.heads, 1,
-                                  self.rank + self.rot, None, self.scale, sinks=self.sink, most_new=ctx.max_new)
+                                  self.rank + self.rot, None, self.scale, sinks=self.sink, **ctx.runs())
             if batched and o.dtype == torch.bfloat16:
                 heads = ops.head_products_batched(o, 0, self.rank, self.w_uv, self.heads, self.rank, self.vdim,
                                                   gates=proj if self.gate else None, g_off=kv_at + self.rank + self.rot)

@@ -366,7 +366,7 @@ def test_attention_rows_of_queries_share_their_loads(ops, dtype, heads, kv_heads
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("form", [dict(window=37), dict(chunk=50), dict(window=37, keep_first=5), dict(window=300, keep_first=40)])
-def test_attention_rows_of_queries_leave_pages_given_back_alone(ops, dtype, form):
+def test_attention_rows_of_queries_leave_pages_given_back_alone(ops, dtype, form, monkeypatch):
     """Steps that go on behind a window or a chunk: the pages that no query can see any more are out of the tables (-1, as the cache
     leaves them), and the first visible key lies in the middle of a tile of 256 and of its page.  The same bits as a workgroup for
     every token and head, which reads the keys it sees alone."""
@@ -381,9 +381,45 @@ def test_attention_rows_of_queries_leave_pages_given_back_alone(ops, dtype, form
     qkv = t(rng.normal(size=(sum(new), heads * dh)), dtype)
     seq = t([b for b, n in enumerate(new) for _ in range(n)], torch.int32)
     pos = t([before[b] + i for b, n in enumerate(new) for i in range(n)], torch.int32)
-    alone, shared = (f64(ops.attention(qkv, kp, vp, pos, seq, table, heads, kv_heads, dh, window, dh ** -0.5, keep_first=keep,
-                                       chunk=chunk, most_new=most)) for most in (1, max(new)))
-    assert np.isfinite(alone).all() and np.array_equal(alone, shared)
+    monkeypatch.setattr(ops, "ATTENTION_ROWS_BYTES", 0)
+    runs = dict(new_counts=new, starts=before, cu_seqlens=t(np.concatenate([[0], np.cumsum(new)]), torch.int32))
+    alone, shared, runs = (f64(ops.attention(qkv, kp, vp, pos, seq, table, heads, kv_heads, dh, window, dh ** -0.5, keep_first=keep,
+                                             chunk=chunk, **how)) for how in ({}, dict(most_new=max(new)), runs))
+    assert np.isfinite(alone).all() and np.array_equal(alone, shared) and np.array_equal(alone, runs)
+
+
+@pytest.mark.parametrize("heads, kv_heads, dh, vd", [(4, 4, 16, 24), (8, 2, 32, 160), (16, 1, 16, 16)])
+def test_attention_rows_of_queries_beside_single_tokens(ops, heads, kv_heads, dh, vd, monkeypatch):
+    """A step of single tokens, short pieces and prompts, more sequences than a wavefront has lanes: the prompts' runs share their
+    loads, every other token keeps a workgroup a head.  The same bits as without the sequences' bounds."""
+    new = [1] * 5 + [40, 3, 1, 4, 17] + [1] * 57 + [9, 1, 16, 2]
+    rng = np.random.default_rng(heads)
+    before = [int(n) for n in rng.integers(0, 40 if EMULATED else 700, len(new))]
+    _, _, kp, _, table = paged(rng, [a + n for a, n in zip(before, new)], kv_heads, dh)
+    vp = t(rng.normal(size=(kp.shape[0], kv_heads, vd, 32)))
+    qkv = t(rng.normal(size=(sum(new), heads * dh)))
+    seq = t([b for b, n in enumerate(new) for _ in range(n)], torch.int32)
+    pos = t([before[b] + i for b, n in enumerate(new) for i in range(n)], torch.int32)
+    cu = t(np.concatenate([[0], np.cumsum(new)]), torch.int32)
+    monkeypatch.setattr(ops, "ATTENTION_ROWS_BYTES", 0)
+    least, tokens, runs = ops.attention_rows_plan(new, before, heads, kv_heads, 4 * dh, None)
+    per = 16 // (heads // kv_heads)
+    many = [n for n in new if n >= least]
+    assert least == max(4, 8 * kv_heads // heads) and tokens == sum(many) < sum(new) and runs == sum(-(-n // per) for n in many)
+    got = ops.attention(qkv, kp, vp, pos, seq, table, heads, kv_heads, dh, None, 0.3, new_counts=new, starts=before, cu_seqlens=cu)
+    want = ops.attention(qkv, kp, vp, pos, seq, table, heads, kv_heads, dh, None, 0.3)
+    assert torch.isfinite(want).all() and torch.equal(got, want)
+
+
+def test_attention_shares_loads_where_that_is_less_to_wait_for(ops, monkeypatch):
+    """Prompts enough to fill the machine do; one of 130 tokens, many of four and steps of single tokens do not, nor do single tokens
+    that stand beside a prompt."""
+    monkeypatch.setattr(ops, "compute_units", lambda: 256)
+    plan = lambda new, starts, heads=16, kv_heads=8, reach=None: ops.attention_rows_plan(new, starts, heads, kv_heads, 512, reach)[1:]
+    assert plan([326, 33, 400], [0] * 3) == (759, 41 + 5 + 50) and plan([2000], [0]) == (2000, 250)
+    assert plan([1] * 64 + [300], [2000] * 64 + [0]) == (300, 38) and plan([130], [2000]) == (130, 17)
+    assert plan([130], [0]) == plan([4] * 200, [0] * 200) == plan([1] * 300, [1000] * 300) == plan([1] * 300 + [4], [1000] * 301) == (0, 0)
+    assert plan([200], [3000], reach=512) == (200, 25) and plan([2000], [0], 32, 1) == (0, 0)      # (32 heads a kv head: too many rows)
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
