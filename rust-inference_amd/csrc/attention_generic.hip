@@ -191,8 +191,10 @@ attention_rows_kernel(T* __restrict__ out, const T* __restrict__ q, int q_stride
     const int kvh = blockIdx.y, group = heads / kv_heads, h0 = kvh * group;
     int begin = blockIdx.x * per, end = min(begin + per, tokens);
     if (cu_seqlens) {
-        if (!run_of(blockIdx.x, cu_seqlens, seqs, rows_from, per, begin, end)) return;
-        end += begin;
+        Run run;
+        if (!run_of(blockIdx.x, cu_seqlens, seqs, rows_from, per, 1, run)) return;
+        begin = run.start + run.first;
+        end = begin + run.count;
     }
     const int share = tid / (ATT_TILE / SHARES), d = tid % (ATT_TILE / SHARES);
     const int row0 = (wave >> 1) * (ATT_ROWS / 2), at = tid & 127;               // scores: half of the rows, two keys of a tile

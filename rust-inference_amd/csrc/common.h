@@ -99,15 +99,20 @@ __device__ __forceinline__ float block_max(float v, float* scratch) {
     return total;
 }
 
-// Workgroup `index` of those that take runs of up to `per` neighbouring new tokens of one sequence, over the sequences that bring
-// `least` and more: the run's first token and how many it has.  Every wavefront works it out for itself, a lane a sequence (a
-// sequence after the other would cost hundreds of them a trip to memory each).  False: there is no such run.
-__device__ __forceinline__ bool run_of(int index, const int32_t* __restrict__ cu_seqlens, int seqs, int least, int per, int& first,
-                                       int& count) {
+// A run of up to `per` neighbouring pieces of one sequence's new tokens, `each` pieces a token: the sequence's first new token and
+// how many it brings, the run's first piece and how many it has.
+struct Run {
+    int start, tokens, first, count;
+};
+
+// Run `index` of the sequences that bring `least` new tokens and more.  Every wavefront works it out for itself, a lane a sequence
+// (a sequence after the other would cost hundreds of them a trip to memory each).  False: there is no such run.
+__device__ __forceinline__ bool run_of(int index, const int32_t* __restrict__ cu_seqlens, int seqs, int least, int per, int each,
+                                       Run& run) {
     const int lane = threadIdx.x & (RI_WAVE - 1);
     for (int s0 = 0; s0 < seqs; s0 += RI_WAVE) {
         const int s = min(s0 + lane, seqs - 1), start = cu_seqlens[s], n = s0 + lane < seqs ? cu_seqlens[s + 1] - start : 0;
-        const int runs = n >= least ? (n + per - 1) / per : 0;
+        const int runs = n >= least ? (n * each + per - 1) / per : 0;
         int upto = runs;                                      // of the sequences up to this lane's
 #pragma unroll
         for (int d = 1; d < RI_WAVE; d *= 2) {
@@ -118,8 +123,10 @@ __device__ __forceinline__ bool run_of(int index, const int32_t* __restrict__ cu
         const unsigned long long past = __ballot(upto > index);
         if (past) {
             const int who = __builtin_ctzll(past), at = (index - __shfl(upto - runs, who, RI_WAVE)) * per;
-            first = __builtin_amdgcn_readfirstlane(__shfl(start, who, RI_WAVE) + at);
-            count = __builtin_amdgcn_readfirstlane(min(per, __shfl(n, who, RI_WAVE) - at));
+            run.start = __builtin_amdgcn_readfirstlane(__shfl(start, who, RI_WAVE));
+            run.tokens = __builtin_amdgcn_readfirstlane(__shfl(n, who, RI_WAVE));
+            run.first = __builtin_amdgcn_readfirstlane(at);
+            run.count = min(per, run.tokens * each - run.first);
             return true;
         }
         index -= all;

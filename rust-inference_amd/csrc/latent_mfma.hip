@@ -131,8 +131,8 @@ latent_attention_mfma_kernel(bf16_t* __restrict__ out, const bf16_t* __restrict_
     }
 }
 
-// Prompts: a workgroup of eight wavefronts takes eight (token, tile of 16 heads) pairs of neighbouring tokens, which walk the same
-// pages, and brings every page into LDS once for all of them.  What bounds the kernel above on a prompt is the caches: every wavefront
+// Prompts: a workgroup of eight wavefronts takes eight (token, tile of 16 heads) pairs of neighbouring tokens (of one sequence, where
+// cu_seqlens says which are), which walk the same pages, and brings every page into LDS once for all of them.  What bounds the kernel above on a prompt is the caches: every wavefront
 // fetches every page for itself, 69 KB for 68 MFMAs.  Here a page crosses once for eight wavefronts, and what is left is
 // reading the fragments from LDS, two cycles of it for every one of the matrix cores.  A page's key and value halves take turns: while
 // the scores are made from the keys the values are on their way into registers, and the other way round, so that two barriers a
@@ -145,24 +145,24 @@ latent_attention_shared_kernel(bf16_t* __restrict__ out, const bf16_t* __restric
                                const bf16_t* __restrict__ k_pages, const bf16_t* __restrict__ v_pages,
                                const int32_t* __restrict__ tok_pos, const int32_t* __restrict__ tok_seq,
                                const int32_t* __restrict__ page_table, int table_width, int tokens, int heads, int tiles,
-                               float scale_log2, const float* __restrict__ sinks) {
+                               float scale_log2, const float* __restrict__ sinks, const int32_t* __restrict__ cu_seqlens, int seqs) {
     constexpr int DK = 32 * KS, RANK = 16 * VT, THREADS = 64 * LP_WAVES;
     constexpr int KP = DK / 8, KPIECES = LM_PAGE * KP;        // 16-byte pieces of a key row and of a page's keys
     constexpr int VP = LM_PAGE / 8, VPIECES = RANK * VP;      // ... of a value channel's row and of a page's values
     constexpr int KN = (KPIECES + THREADS - 1) / THREADS, VN = (VPIECES + THREADS - 1) / THREADS;
     __shared__ uint4 ks_[KPIECES], vs_[VPIECES];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, col = lane & 15, g = lane >> 4;
-    const long pairs = (long)tokens * tiles;
     // (long prompts first: the workgroups launched last are the short ones; pairs count back from the last token's)
-    const long pair = (long)blockIdx.x * LP_WAVES + wave;
-    const bool there = pair < pairs;
-    const long mine = there ? pair : pairs - 1;
-    const int t = tokens - 1 - (int)(mine / tiles), tile = (int)(mine % tiles);
+    Run run = {0, tokens, (int)blockIdx.x * LP_WAVES, 0};
+    run.count = min(LP_WAVES, tokens * tiles - run.first);
+    if (cu_seqlens && !run_of(blockIdx.x, cu_seqlens, seqs, 1, LP_WAVES, tiles, run)) return;
+    const bool there = wave < run.count;
+    const int mine = run.first + min(wave, run.count - 1), last = run.start + run.tokens - 1;
+    const int t = last - mine / tiles, tile = mine % tiles;
     const int head = tile * 16 + col, hq = head < heads ? head : heads - 1;
     const int qpos = tok_pos[t], seq = tok_seq[t];
-    // the tokens of a workgroup are of one sequence nearly always; where they are not, the sequences go one after the other
-    const int t_last = tokens - 1 - (int)((long)blockIdx.x * LP_WAVES / tiles);
-    const int t_first = tokens - 1 - (int)(min((long)blockIdx.x * LP_WAVES + LP_WAVES, pairs) - 1) / tiles;
+    // where the tokens of a workgroup are of several sequences, these go one after the other
+    const int t_last = last - run.first / tiles, t_first = last - (run.first + run.count - 1) / tiles;
 
     LmFrag qf[KS];
 #pragma unroll
@@ -319,11 +319,14 @@ extern "C" int ri_latent_attention_mfma_fits(int key_dim, int rank, int page_siz
 
 // out [tokens, heads * rank] bfloat16: causal attention of every new token's heads (q [tokens, >= heads * key_dim], the
 // heads side by side) over its sequence's one key/value head of key rows of key_dim and value rows of rank.
-// shared_pages: neighbouring tokens are of one sequence for the most part, and share the pages they fetch (the results are the same bits).
+// shared_pages: neighbouring tokens share the pages they fetch (the results are the same bits): in as many workgroups of eight
+// (token, tile of 16 heads) pairs as it says, each of one sequence, where cu_seqlens [seqs + 1] is given; else 1, a workgroup's tokens
+// the step's neighbours, of one sequence for the most part.
 extern "C" int ri_latent_attention_mfma(void* out, const void* q, int q_stride, const void* k_pages, const void* v_pages,
                                         const int32_t* tok_pos, const int32_t* tok_seq, const int32_t* page_table,
                                         int table_width, int tokens, int heads, int key_dim, int rank, int page_size, float scale,
-                                        const float* sinks, float* partial, int chunks, int chunk_pages, int shared_pages, void* stream) {
+                                        const float* sinks, float* partial, int chunks, int chunk_pages, int shared_pages,
+                                        const int32_t* cu_seqlens, int seqs, void* stream) {
     RI_REQUIRE(tokens > 0 && heads > 0 && ri_latent_attention_mfma_fits(key_dim, rank, page_size),
                "latent_attention_mfma: %d tokens, %d heads, keys of %d, values of %d, pages of %d", tokens, heads, key_dim, rank, page_size);
     RI_REQUIRE(q_stride >= heads * key_dim && q_stride % 8 == 0 && (uintptr_t)q % 16 == 0 && (uintptr_t)k_pages % 16 == 0 &&
@@ -345,12 +348,13 @@ extern "C" int ri_latent_attention_mfma(void* out, const void* q, int q_stride, 
                                                                           heads, tiles, scale_log2, sinks, partial, chunks, \
                                                                           chunk_pages)
     if (shared_pages && chunks == 1) {
-        const unsigned groups = (unsigned)((pairs + LP_WAVES - 1) / LP_WAVES);
+        RI_REQUIRE(pairs <= 2147483647L - LP_WAVES && (!cu_seqlens || seqs > 0), "latent_attention_mfma: %ld pairs of %d sequences", pairs, seqs);
+        const unsigned groups = cu_seqlens ? (unsigned)shared_pages : (unsigned)((pairs + LP_WAVES - 1) / LP_WAVES);
 #define RI_SHARED(KS, VT)                                                                                               \
     latent_attention_shared_kernel<KS, VT><<<groups, 64 * LP_WAVES, 0, s>>>((bf16_t*)out, (const bf16_t*)q, q_stride,   \
                                                                             (const bf16_t*)k_pages, (const bf16_t*)v_pages, tok_pos, \
                                                                             tok_seq, page_table, table_width, tokens, heads, tiles, \
-                                                                            scale_log2, sinks)
+                                                                            scale_log2, sinks, cu_seqlens, seqs)
         if (key_dim == 576) RI_SHARED(18, 32); else if (key_dim == 288) RI_SHARED(9, 16); else RI_SHARED(5, 8);
 #undef RI_SHARED
     } else if (key_dim == 576) RI_GO(18, 32); else if (key_dim == 288) RI_GO(9, 16); else RI_GO(5, 8);

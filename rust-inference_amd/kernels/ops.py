@@ -167,7 +167,7 @@ _SIGNATURES = {
                           c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
     "ri_latent_attention_mfma_fits": [c_int, c_int, c_int],
     "ri_latent_attention_mfma": [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int,
-                                 c_int, c_int, c_int, c_float, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p],
+                                 c_int, c_int, c_int, c_float, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_int, c_void_p],
     "ri_head_products": [c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_int, c_void_p,
                          c_int, c_int, c_float, c_int, c_int, c_int, c_int, c_int, c_void_p],
     "ri_whole_norm_kv_write": [c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_float, c_void_p, c_void_p, c_void_p,
@@ -1696,16 +1696,39 @@ def latent_attention_mfma_fits(dtype, key_dim: int, rank: int, page_size: int) -
     return dtype == torch.bfloat16 and bool(_get("ri_latent_attention_mfma_fits")(key_dim, rank, page_size))
 
 
-LATENT_SHARED_FROM = 16          # new tokens a sequence brings on average from which neighbours share the pages they fetch: where a
-                                 # workgroup's tokens are of different sequences they go one sequence after the other
+LATENT_SHARED_FROM = 16          # new tokens a sequence brings on average from which neighbours share the pages they fetch, where the
+                                 # sequences' bounds are not given: there a workgroup's sequences go one after the other
+# Where they are given: by the size of a key row, the wavefronts ((token, tile of 16 heads) pairs) a compute unit, or the keys of the
+# longest sequence, from which a page is shared.  One prompt, tokens @ cached tokens, us a wavefront for itself : shared.  576: the caches
+# are slower than the walk as soon as the pages are many, or the machine is full: 32 heads 128 @ 0 39 : 43, 512 @ 0 161 : 127, 16 @
+# 500 132 : 124, 16 @ 2,000 725 : 447; 128 heads 128 @ 0 53 : 45.  288: with room on the machine its two barriers a page cost more
+# than the pages: 32 heads 512 @ 2,000 163 : 256, 1,024 @ 0 103 : 111, 2,048 @ 0 286 : 231; 128 heads 256 @ 0 35 : 37, 512 @ 0 89 : 75.
+# 160: 32 heads 512 @ 0 27 : 34, 512 @ 2,000 110 : 110, 16 @ 8,000 552 : 355, 2,048 @ 0 175 : 106; 128 heads 256 @ 0 21 : 29, 512 @ 0 52 : 44.
+LATENT_SHARED = {576: (4, 512), 288: (9, None), 160: (9, 4096)}
+LATENT_SHARED_WAVES = 8          # wavefronts of a workgroup (LP_WAVES of latent_mfma.hip)
+
+
+def latent_attention_shared(new_counts, starts, heads: int, key_dim: int) -> int:
+    """The workgroups in which a step's tokens share the pages they fetch, each of one sequence, or 0 where every wavefront fetches
+    for itself (host code only: it needs no GPU)."""
+    tiles = -(-heads // 16)
+    waves, keys = LATENT_SHARED[key_dim]
+    # (a sequence of few tokens fills no workgroup; where pages are many and large that is still the faster form)
+    if keys is not None and max(s + n for s, n in zip(starts, new_counts)) >= keys:
+        pass
+    elif sum(new_counts) * tiles < waves * compute_units() or min(new_counts) * tiles < LATENT_SHARED_WAVES:
+        return 0
+    return sum(-(-n * tiles // LATENT_SHARED_WAVES) for n in new_counts)
 
 
 def latent_attention_mfma(q, k_pages, v_pages, tok_pos, tok_seq, page_table, heads: int, scale: float, sinks,
-                          max_len: int = 0) -> torch.Tensor:
+                          max_len: int = 0, new_counts=None, starts=None, cu_seqlens=None) -> torch.Tensor:
     """bfloat16 ``[T, heads * rank]``: causal attention on the matrix cores of every new token's ``heads`` query rows (``q [T,
     heads * key_dim]``) over its sequence's single key/value head (``k_pages [pages, 1, 32, key_dim]``, ``v_pages [pages, 1, rank,
     32]``), with a sink per head in the softmax's denominator (or None).  ``max_len``: a bound on the sequences' lengths; given, a
-    step of few tokens cuts every token's pages into chunks that run side by side and are joined by a second launch."""
+    step of few tokens cuts every token's pages into chunks that run side by side and are joined by a second launch.
+    ``new_counts``, ``starts`` (lists: the sequences' new and cached tokens) and ``cu_seqlens`` (int32 ``[seqs + 1]``): for prompts, whose
+    neighbouring tokens then share the pages they fetch where ``latent_attention_shared`` says so (the results are the same bits)."""
     tokens = q.shape[0]
     key_dim, rank, page = k_pages.shape[3], v_pages.shape[2], k_pages.shape[2]
     if k_pages.shape[1] != 1 or v_pages.shape[1] != 1 or v_pages.shape[3] != page or q.shape[1] != heads * key_dim:
@@ -1720,12 +1743,21 @@ def latent_attention_mfma(q, k_pages, v_pages, tok_pos, tok_seq, page_table, hea
         chunks = -(-pages // chunk_pages)
         if chunks > 1:
             partial = torch.empty((tokens, heads, chunks, rank + 2), dtype=torch.float32, device=q.device)
+    seqs = 0 if cu_seqlens is None else len(new_counts)
+    if seqs and (sum(new_counts) != tokens or len(starts) != seqs):
+        raise ShapeError(f"latent_attention_mfma: {tokens} tokens of {seqs} sequences that bring {sum(new_counts)}, {len(starts)} of them cached")
+    if max_len:
+        shared = 0
+    elif seqs:
+        shared = latent_attention_shared(new_counts, starts, heads, key_dim)
+    else:
+        shared = int(tokens >= LATENT_SHARED_FROM * page_table.shape[0])
     _call("ri_latent_attention_mfma", _dev(out, "out"), _dev(q, "q", torch.bfloat16), q.shape[1],
           _dev(k_pages, "k_pages", torch.bfloat16), _dev(v_pages, "v_pages", torch.bfloat16),
           _dev(tok_pos, "tok_pos", torch.int32, (tokens,)), _dev(tok_seq, "tok_seq", torch.int32, (tokens,)),
           _dev(page_table, "page_table", torch.int32), page_table.shape[1], tokens, heads, key_dim, rank, page, float(scale),
-          _opt(sinks, "sinks", torch.float32, (heads,)), _opt(partial, "partial"), chunks, chunk_pages,
-          int(not max_len and tokens >= LATENT_SHARED_FROM * page_table.shape[0]), _stream())
+          _opt(sinks, "sinks", torch.float32, (heads,)), _opt(partial, "partial"), chunks, chunk_pages, shared,
+          _opt(cu_seqlens, "cu_seqlens", torch.int32, (seqs + 1,)), seqs, _stream())
     return out
 
 

@@ -108,7 +108,7 @@ class LatentAttention(Mixer):
                 # tokens cuts the pages into chunks side by side (one walk of 1,024 keys by the two wavefronts a sequence has
                 # takes 319 us, the general kernel 106)
                 o = ops.latent_attention_mfma(q, store.k_pages, store.v_pages, ctx.tok_pos, ctx.tok_seq, page_table, self.heads,
-                                              self.scale, self.sink, ctx.max_len if ctx.is_decode else 0)
+                                              self.scale, self.sink, ctx.max_len if ctx.is_decode else 0, **ctx.runs())
             else:
                 o = ops.attention(q, store.k_pages, store.v_pages, ctx.tok_pos, ctx.tok_seq, page_table, self.heads, 1,
                                   self.rank + self.rot, None, self.scale, sinks=self.sink, **ctx.runs())

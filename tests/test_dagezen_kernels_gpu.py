@@ -398,6 +398,41 @@ def test_latent_attention_with_shared_pages_gives_the_same_bits(ops, heads, dk, 
     assert np.isfinite(got[0]).all() and np.array_equal(*got)
 
 
+@pytest.mark.parametrize("heads, dk, rank", [(20, 160, 128), (130, 160, 128), (40, 288, 256), (16, 576, 512)])
+def test_latent_attention_with_shared_pages_a_sequence_a_workgroup(ops, heads, dk, rank, monkeypatch):
+    """The sequences' bounds given: workgroups of one sequence alone, more sequences than a wavefront has lanes, single tokens among
+    them; the same bits as a wavefront that fetches its pages itself."""
+    rng = np.random.default_rng(heads)
+    new = [1] * 30 + [9, 2, 1, 5] + [1] * 33 + [3] if dk == 160 and heads == 20 else [9, 1, 1, 5]
+    before = [int(n) for n in rng.integers(0, 60, len(new))]
+    width = -(-max(a + n for a, n in zip(before, new)) // PAGE)
+    pages = sum(-(-(a + n) // PAGE) for a, n in zip(before, new)) + 2
+    k_pages = guarded((torch.randn((pages, 1, PAGE, dk), device=DEV) * 0.5).to(torch.bfloat16))
+    v_pages = guarded(k_pages[:, :, :, :rank].transpose(2, 3).contiguous())
+    order = iter(rng.permutation(pages))
+    table = t([[next(order) if i < -(-(a + n) // PAGE) else -1 for i in range(width)] for a, n in zip(before, new)], torch.int32)
+    tok_seq = t([s for s, n in enumerate(new) for _ in range(n)], torch.int32)
+    tok_pos = t([before[s] + i for s, n in enumerate(new) for i in range(n)], torch.int32)
+    q = guarded((torch.randn((sum(new), heads * dk), device=DEV) * 0.5).to(torch.bfloat16))
+    cu, sinks, got = t(np.concatenate([[0], np.cumsum(new)]), torch.int32), t(rng.standard_normal(heads)), []
+    for keys in (1, 1 << 30):                                 # shared from one key on, and apart
+        monkeypatch.setattr(ops, "LATENT_SHARED", {dk: (1 << 20, keys)})
+        assert (ops.latent_attention_shared(new, before, heads, dk) > 0) == (keys == 1)
+        got.append(f64(ops.latent_attention_mfma(q, k_pages, v_pages, tok_pos, tok_seq, table, heads, 0.11, sinks, new_counts=new,
+                                                 starts=before, cu_seqlens=cu)))
+    assert np.isfinite(got[0]).all() and np.array_equal(*got)
+
+
+def test_latent_attention_shares_pages_where_that_is_less_to_wait_for(ops, monkeypatch):
+    """Small prompts fetch for themselves; long ones and steps that fill the machine share, in workgroups of one sequence each."""
+    monkeypatch.setattr(ops, "compute_units", lambda: 256)
+    plan = ops.latent_attention_shared
+    assert plan([2048], [0], 32, 576) == 512 and plan([16], [2000], 32, 576) == 4 and plan([20] * 32, [0] * 32, 32, 576) == 160
+    assert plan([2048] + [1] * 64, [0] + [4000] * 64, 32, 576) == 512 + 64
+    assert plan([128], [0], 32, 576) == plan([17] * 10, [0] * 10, 32, 576) == plan([512], [8000], 32, 288) == plan([300], [0], 20, 160) == 0
+    assert plan([2048], [0], 32, 288) == 512 and plan([2048] + [1] * 64, [0] + [2000] * 64, 32, 288) == 0 and plan([16], [8000], 32, 160) == 4
+
+
 @pytest.mark.parametrize("heads, kv_heads, dim, window", [(8, 2, 32, 40), (16, 16, 32, None), (8, 1, 64, 33)])
 def test_talking_attention_on_the_matrix_cores_is_the_general_kernel(ops, heads, kv_heads, dim, window):
     """bfloat16: two sequences whose pages lie in shuffled order, one that goes on from 37 cached tokens with 21 new ones
