@@ -190,11 +190,11 @@ latent_attention_shared_kernel(bf16_t* __restrict__ out, const bf16_t* __restric
 
     for (int from = t_last; from >= t_first;) {               // (uniform: the tokens' sequences and positions are memory's)
         const int s_now = tok_seq[from];
-        int to = from;
-        while (to > t_first && tok_seq[to - 1] == s_now) --to;
+        int to = from, far = tok_pos[from];                   // (the tokens of a sequence may come in any order)
+        while (to > t_first && tok_seq[to - 1] == s_now) far = max(far, tok_pos[--to]);
         const bool active = there && t <= from && t >= to;
         const int32_t* table = page_table + (size_t)s_now * table_width;
-        const int pages = tok_pos[from] / LM_PAGE + 1;        // (positions grow with the tokens of a sequence)
+        const int pages = far / LM_PAGE + 1;
         fetch_keys(table[0]);
         for (int page = 0; page < pages; ++page) {
             const long phys = table[page], next = table[min(page + 1, pages - 1)];

@@ -423,6 +423,23 @@ def test_latent_attention_with_shared_pages_a_sequence_a_workgroup(ops, heads, d
     assert np.isfinite(got[0]).all() and np.array_equal(*got)
 
 
+@pytest.mark.parametrize("order", [[3, 0, 2, 1, 4], [4, 3, 2, 1, 0]])
+def test_latent_attention_with_shared_pages_takes_the_tokens_in_any_order(ops, order, monkeypatch):
+    """The tokens of a sequence need not come by their positions: every one sees its own keys, the same bits as by position."""
+    torch.manual_seed(1)
+    heads, dk, rank, before, n = 16, 160, 128, 61, 5
+    pages = -(-(before + n) // PAGE)
+    k_pages = guarded((torch.randn((pages, 1, PAGE, dk), device=DEV) * 0.5).to(torch.bfloat16))
+    v_pages = guarded(k_pages[:, :, :, :rank].transpose(2, 3).contiguous())
+    table, seq = t([list(range(pages))], torch.int32), t([0] * n, torch.int32)
+    q = (torch.randn((n, heads * dk), device=DEV) * 0.5).to(torch.bfloat16)
+    monkeypatch.setattr(ops, "LATENT_SHARED_FROM", 0)
+    want = f64(ops.latent_attention_mfma(guarded(q), k_pages, v_pages, t(before + np.arange(n), torch.int32), seq, table, heads, 0.11, None))
+    got = f64(ops.latent_attention_mfma(guarded(q[order].contiguous()), k_pages, v_pages, t(before + np.array(order), torch.int32), seq, table,
+                                        heads, 0.11, None))
+    assert np.isfinite(want).all() and np.array_equal(got, want[order])
+
+
 def test_latent_attention_shares_pages_where_that_is_less_to_wait_for(ops, monkeypatch):
     """Small prompts fetch for themselves; long ones and steps that fill the machine share, in workgroups of one sequence each."""
     monkeypatch.setattr(ops, "compute_units", lambda: 256)
