@@ -1866,13 +1866,30 @@ def talking_attention_mfma_fits(dtype, heads: int, kv_heads: int, dim: int, page
     return dtype == torch.bfloat16 and bool(_get("ri_talking_attention_mfma_fits")(heads, kv_heads, dim, page_size))
 
 
-TALKING_MAX_SHARES = 4           # parts of a tile's pages: past this the adding of the parts costs what the walk gains
+# Parts of a tile's pages.  32 heads of 128, a window of 1,024, us at 1 / 2 / 4 / 8 shares: 16 tokens (a page) 40.6 / 42.4 / 43.1 / 44.1, 64
+# (two) 59.0 / 43.4 / 44.8 / 47.6, 256 173 / 107 / 75 / 62, 1,024 671 / 391 / 257; 32 prompts of 17 tokens 49.8 / 60.7 / 63.5.
+TALKING_MAX_SHARES = 4
+# Up to this window a table of its distances is made: 32 heads, windows of 1,024 and 16,384 alike: 16 tokens 43 us with the table (44 with a
+# logarithm a score), 2,048 tokens under a window of 16,384 894 (2,104).
+TALKING_TABLE_WINDOW = 16384
+
+
+def talking_attention_mfma_shares(tiles: int, longest: int | None, window: int | None) -> int:
+    """Into how many shares the second walk of a step of ``tiles`` tiles cuts a tile's pages: as many as leave no compute unit idle, but
+    a page a share at least.  ``longest``: the longest sequence's keys (host code only: it needs no GPU)."""
+    shares = min(TALKING_MAX_SHARES, compute_units() // tiles)
+    if longest is not None:
+        shares = min(shares, -(-min(longest, window + 16 if window else longest) // 32))
+    return max(1, shares)
 
 
 def talking_attention_mfma(proj, q_off: int, k_pages, v_pages, tok_pos, cu_seqlens, new_counts, page_table, heads: int,
-                           kv_heads: int, dim: int, window: int | None, scale: float, r1, r2, talk) -> torch.Tensor:
+                           kv_heads: int, dim: int, window: int | None, scale: float, r1, r2, talk,
+                           longest: int | None = None) -> torch.Tensor:
     """The same attention on the matrix cores, for prompts in bfloat16: ``[T, heads * dim]``.  ``new_counts``: every
-    sequence's number of new tokens (the host's list), by which the launch counts its tiles of 16 tokens."""
+    sequence's number of new tokens (the host's list), by which the launch counts its tiles of 16 tokens; ``longest``: the most keys
+    of any sequence.  In how many shares a token's sums run (``talking_attention_mfma_shares``) depends on both, and with it the
+    rounding of its float32 sums."""
     tokens = proj.shape[0]
     seqs = len(new_counts)
     tiles = sum(-(-int(n) // 16) for n in new_counts)
@@ -1881,8 +1898,10 @@ def talking_attention_mfma(proj, q_off: int, k_pages, v_pages, tok_pos, cu_seqle
         return out
     stats = torch.empty((tokens, heads, 2), dtype=torch.float32, device=proj.device)
     # (a table of the biases a distance for windows it is small for; shares of the pages where the tiles leave compute units idle)
-    bias = torch.empty((heads, window + 16), dtype=torch.float32, device=proj.device) if window and window <= 16384 and r1 is not None else None
-    shares = max(1, min(TALKING_MAX_SHARES, compute_units() // tiles))
+    bias = None
+    if window and window <= TALKING_TABLE_WINDOW and r1 is not None:
+        bias = torch.empty((heads, window + 16), dtype=torch.float32, device=proj.device)
+    shares = talking_attention_mfma_shares(tiles, longest, window)
     parts = torch.empty((shares, tokens, heads * dim), dtype=torch.float32, device=proj.device) if shares > 1 else None
     _call("ri_talking_attention_mfma", _dev(out, "out"), _dev(stats, "stats"), _dev(proj, "proj", torch.bfloat16), proj.shape[1],
           int(q_off), _dev(k_pages, "k_pages", torch.bfloat16), _dev(v_pages, "v_pages", torch.bfloat16),

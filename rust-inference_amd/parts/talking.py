@@ -93,7 +93,7 @@ class TalkingAttention(Mixer):
                 # prompts at the sizes the matrix cores take: tiles of 16 tokens, both walks on them
                 o = ops.talking_attention_mfma(proj, 0, store.k_pages, store.v_pages, ctx.tok_pos, ctx.cu_seqlens, ctx.new_counts,
                                                page_table, self.heads, self.kv_heads, self.dim, self.window, self.scale, self.r1,
-                                               self.r2, self.mix)
+                                               self.r2, self.mix, ctx.max_len)
             else:
                 o = ops.talking_attention(proj, 0, store.k_pages, store.v_pages, ctx.tok_pos, ctx.tok_seq, page_table, self.heads,
                                           self.kv_heads, self.dim, self.window, self.scale, self.r1, self.r2, self.mix, shares)

@@ -474,6 +474,15 @@ def test_talking_attention_on_the_matrix_cores_is_the_general_kernel(ops, heads,
         close(got, f64(want), 1.5e-2, "matrix cores against the general kernels")
 
 
+def test_talking_attention_cuts_no_page_between_shares(ops, monkeypatch):
+    """As many shares as leave no compute unit idle, none of them without a page: prompts of a page or two are walked whole or in two."""
+    monkeypatch.setattr(ops, "compute_units", lambda: 256)
+    shares = ops.talking_attention_mfma_shares
+    assert [shares(1, n, 1024) for n in (16, 32, 33, 100, 2016)] == [1, 1, 2, 4, 4]
+    assert shares(64, 17, 1024) == 1 and shares(128, 2048, 1024) == 2 and shares(128, 2048, None) == 2 and shares(129, 2064, 1024) == 1
+    assert shares(1, 5000, 16) == 1 and shares(1, 5000, 17) == 2 and shares(1, None, 1024) == 4
+
+
 # ---------------------------------------------------------------- the walks over states of 65 to 128 rows
 @pytest.mark.parametrize("kind", ["ssd", "timemix", "gla"])
 @pytest.mark.parametrize("rows, cols, heads, many", [(65, 65, 2, False), (100, 33, 2, False), (128, 40, 1, False), (128, 128, 33, True)])
