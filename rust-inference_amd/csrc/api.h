@@ -488,6 +488,7 @@ int ri_timemix_scan_cols(void* out, int out_stride, int out_off, float out_scale
 
 // ---- the state-space mixer (ssd.hip)
 // update_tails 0: the convolution; 1: the tails move on by the step's tokens (call it after the convolution).
+int ri_causal_conv_blocks(int tokens, int seqs, int channels);
 int ri_causal_conv_silu(float* out, const void* proj, int act_dtype, int stride, int col0, const float* taps_w,
                         const float* bias, float* tails, int taps, const int32_t* tok_seq, const int32_t* cu_seqlens,
                         const int32_t* slots, int tokens, int seqs, int channels, int update_tails, void* stream);

@@ -118,6 +118,15 @@ conv_tails_kernel(float* __restrict__ tails, const TA* __restrict__ proj, int st
     for (int idx = 0; idx < taps - 1; ++idx) tail[(size_t)idx * channels + ch] = keep[idx];
 }
 
+// Whether a step takes the block form: from as many results on as fill the machine with 32 a thread; below, its chain of eight tokens is
+// what a launch takes (us with the tails' launch, an element a thread : blocks; 1,536 channels of 256 / 512 / 1,024 tokens 6.4 : 7.9, 8.8 :
+// 8.4, 12.7 : 8.6; 6,144 channels of 64 / 128 / 256 / 2,048 tokens 6.4 : 8.1, 9.2 : 8.2, 12.9 : 8.7, 86.0 : 22.9).  Where sequences bring
+// fewer than two tokens on average most rows take their tails, four loads a row in a pass of their own: four times as many
+// results (6,144 channels of 128 / 256 / 512 sequences of one token 11.1 : 15.9, 18.3 : 21.4, 34.2 : 26.9; of two tokens 20.3 : 15.8 at 128).
+extern "C" int ri_causal_conv_blocks(int tokens, int seqs, int channels) {
+    return (long)tokens * channels >= (tokens >= 2L * seqs ? 1 : 4) * CONV_BLOCK_FROM;
+}
+
 extern "C" int ri_causal_conv_silu(float* out, const void* proj, int act_dtype, int stride, int col0, const float* taps_w,
                                    const float* bias, float* tails, int taps, const int32_t* tok_seq, const int32_t* cu_seqlens,
                                    const int32_t* slots, int tokens, int seqs, int channels, int update_tails, void* stream) {
@@ -128,11 +137,8 @@ extern "C" int ri_causal_conv_silu(float* out, const void* proj, int act_dtype, 
     RI_REQUIRE(taps == 1 || tails, "causal_conv_silu: a convolution of %d taps keeps a tail", taps);
     hipStream_t s = (hipStream_t)stream;
     const int cy = (channels + 255) / 256;
-    // The block form from as many results on as fill the machine with 32 a thread; below, its chain of eight tokens is what a launch
-    // takes (us with the tails' launch, an element a thread : blocks; 1,536 channels of 256 / 512 / 1,024 tokens 6.4 : 7.9, 8.8 : 8.4,
-    // 12.7 : 8.6; 6,144 channels of 64 / 128 / 256 / 2,048 tokens 6.4 : 8.1, 9.2 : 8.2, 12.9 : 8.7, 86.0 : 22.9).  A thread's four
-    // channels have to start on the boundary of their loads.
-    const bool four = taps == 4 && (long)tokens * channels >= CONV_BLOCK_FROM && channels % 4 == 0 && stride % 4 == 0 && col0 % 4 == 0 &&
+    // (a thread's four channels of the block form have to start on the boundary of their loads)
+    const bool four = taps == 4 && ri_causal_conv_blocks(tokens, seqs, channels) && channels % 4 == 0 && stride % 4 == 0 && col0 % 4 == 0 &&
                       (((uintptr_t)out | (uintptr_t)taps_w | (uintptr_t)bias | (uintptr_t)tails) & 15) == 0 &&
                       ((uintptr_t)proj & (act_dtype == RI_F32 ? 15 : 7)) == 0;
     if (!update_tails && four) {

@@ -190,6 +190,7 @@ _SIGNATURES = {
     "ri_timemix_scan_cols": [c_void_p, c_int, c_int, c_float, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p,
                              c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
                              c_void_p],
+    "ri_causal_conv_blocks": [c_int, c_int, c_int],
     "ri_causal_conv_silu": [c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p,
                             c_void_p, c_int, c_int, c_int, c_int, c_void_p],
     "ri_ssd_scan": [c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p,
@@ -1978,6 +1979,11 @@ def timemix_scan(out, out_off: int, out_scale: float, r, k, v, g, z, w0, u, gain
 
 # ---------------------------------------------------------------- the state-space mixer
 SSD_MAX_TAPS = 16
+
+
+def causal_conv_blocks(tokens: int, seqs: int, channels: int) -> bool:
+    """Whether ``causal_conv_silu`` of four taps runs by blocks of eight tokens and four channels (host code only: it needs no GPU)."""
+    return bool(_get("ri_causal_conv_blocks")(int(tokens), int(seqs), int(channels)))
 
 
 def causal_conv_silu(proj, col0: int, channels: int, taps_w, bias, tails, tok_seq, cu_seqlens, slots) -> torch.Tensor:

@@ -276,6 +276,7 @@ def test_convolution_of_four_taps_by_blocks_of_tokens(ops, lengths, channels, dt
     goes on where it stopped.  The sums are the same sums in the same order: the same bits."""
     rng = np.random.default_rng(channels)
     seqs, tokens = len(lengths), sum(lengths)
+    assert ops.causal_conv_blocks(tokens, seqs, channels) and not ops.causal_conv_blocks(100, 1, channels)
     proj = t(rng.standard_normal((tokens, channels + 8)), dtype)
     w, bias = t(rng.standard_normal((channels, 4)) / 2), t(rng.standard_normal(channels))
     tails = t(rng.standard_normal((seqs + 1, 3, channels)))
@@ -291,6 +292,13 @@ def test_convolution_of_four_taps_by_blocks_of_tokens(ops, lengths, channels, dt
                                         t([0, end - at], torch.int32), t([order[s]], torch.int32))
             assert torch.equal(got[at:end], want), f"sequence {s}, tokens {at}..{end}"
     assert torch.equal(kept, tails)
+
+
+def test_convolution_of_single_tokens_keeps_an_element_a_thread(ops):
+    """Steps whose rows mostly take their tails go by blocks from four times as many results on."""
+    blocks = lambda tokens, seqs, channels=6144: ops.causal_conv_blocks(tokens, seqs, channels)
+    assert blocks(128, 1) and blocks(128, 64) and blocks(512, 512) and blocks(600, 301)
+    assert not blocks(127, 1) and not blocks(128, 128) and not blocks(128, 65) and not blocks(256, 256) and not blocks(600, 600, 1536)
 
 
 @pytest.mark.parametrize("columns", [True, False])
