@@ -3,13 +3,16 @@
 // has, so a row's result does not depend on the other rows.
 //
 // bfloat16 weights (a checkpoint's usual form) run on the matrix cores without loss: a float32 has 24 bits, three
-// bfloat16 of eight each, x = a + b + c exactly (cut off, not rounded, so that nothing overflows).  Every product of a part
-// and a weight is exact in float32, and the sums of the three parts are float32 sums of their own, added at the end: what
-// is rounded is the additions alone, as in a chain of multiply-adds, and there are fewer of them.  Relative error against
+// bfloat16 of eight each (a published method: Henry, Tang and Heinecke, "Leveraging the bfloat16 Artificial Intelligence Datatype
+// For Higher-Precision Computations", 2019).  Here x = a + (b + c) 2^-16 exactly, for every float32: the parts are cut off, not
+// rounded, and b and c are kept 2^16 times as large, so that the last bit of the smallest float32, 2^-149, is still one of bfloat16's
+// (2^-133; the matrix cores take subnormal numbers as they are).  Every product of a part and a weight is exact in float32 above
+// the subnormal numbers, and the sums of the three parts are float32 sums of their own, added at the end: what is rounded is the
+// additions alone, as in a chain of multiply-adds, and there are fewer of them.  Relative error against
 // 64 bits (2-norm, normal x and weights): at K = 1,024 1.9e-7 where the chain of multiply-adds has 5.7e-7, at 3,072
 // 3.4e-7 : 9.9e-7.  The three products run at a third of the bfloat16 rate, ten times the vector units' multiply-adds.
-// An infinity or NaN has no such parts, but leaves an infinity or NaN in every sum it enters: such an output is computed
-// again by the chain.
+// An infinity, a NaN or a number past 2^119 has no such parts, but leaves an infinity or NaN in every sum it enters: such an
+// output is computed again by the chain.
 //
 // Other forms (float32 weights, rows that 16-byte loads do not divide): float32 multiply-adds on the vector units, every
 // output one sum over k = 0..K-1.
@@ -28,7 +31,9 @@ __device__ __forceinline__ uint32_t upper_halves(float a, float b) {
 }
 __device__ __forceinline__ float below_upper(float a) { return a - __uint_as_float(__float_as_uint(a) & 0xFFFF0000u); }
 
-// Eight floats as three times eight bfloat16 whose sum they are.
+#define F32_LOWER 65536.f     // the second and third part are so much larger than what they stand for
+
+// Eight floats as three times eight bfloat16 whose sum they are, the first and 1 / F32_LOWER of the others.
 __device__ __forceinline__ void split8(const float4 lo, const float4 hi, uint4& a, uint4& b, uint4& c) {
     float v[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
     uint32_t p[3][4];
@@ -37,7 +42,7 @@ __device__ __forceinline__ void split8(const float4 lo, const float4 hi, uint4& 
 #pragma unroll
         for (int i = 0; i < 4; ++i) p[part][i] = upper_halves(v[2 * i], v[2 * i + 1]);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] = below_upper(v[i]);
+        for (int i = 0; i < 8; ++i) v[i] = part == 0 ? below_upper(v[i]) * F32_LOWER : below_upper(v[i]);
     }
     a = make_uint4(p[0][0], p[0][1], p[0][2], p[0][3]);
     b = make_uint4(p[1][0], p[1][1], p[1][2], p[1][3]);
@@ -172,7 +177,7 @@ gemm_f32_tile_kernel(float* __restrict__ out, const float* __restrict__ x, const
             float sum[4];
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                sum[e] = acc[i][j][0][e] + (acc[i][j][1][e] + acc[i][j][2][e]);
+                sum[e] = acc[i][j][0][e] + (acc[i][j][1][e] + acc[i][j][2][e]) * (1.f / F32_LOWER);
                 bad |= !(fabsf(sum[e]) < INFINITY);
             }
             float* o = out + (size_t)m * N + n;

@@ -741,6 +741,19 @@ def test_gemm_f32_on_the_matrix_cores(ops, m, n, k):
     assert np.array_equal(got[m // 2:], f64(some)), "a row's sums depend on the other rows"
 
 
+@pytest.mark.parametrize("top", [-100, -112, -118, -126, -135])
+def test_gemm_f32_of_the_smallest_numbers(ops, top):
+    """x down to the smallest float32, subnormal numbers among them: no bit of it is lost.  The bound of the test above, and half the
+    smallest float32 for every one of the products and additions that may end among the subnormal numbers."""
+    rng = np.random.default_rng(-top)
+    m, n, k = 33, 40, 136
+    x = t(np.ldexp(rng.choice([-1.0, 1.0], (m, k)) * rng.uniform(1, 2, (m, k)), rng.integers(top - 8, top + 1, (m, k))))
+    w = t(rng.normal(size=(n, k)), torch.bfloat16)
+    got = f64(ops.gemm_f32(x, w))
+    bound = (k / 32 + 32) * 2.0 ** -24 * (np.abs(f64(x)) @ np.abs(f64(w)).T) + 3 * 2 * k * 2.0 ** -150
+    assert (np.abs(got - f64(x) @ f64(w).T) <= bound).all()
+
+
 def test_gemm_f32_infinities_and_nan(ops):
     """Numbers that have no parts: the row of x and the column of the weights they stand in become what multiply-adds make of them."""
     rng = np.random.default_rng(3)
