@@ -236,7 +236,7 @@ gla_walk_kernel(float* __restrict__ out, const TA* __restrict__ proj, int row, i
         qs[buf][rtok][tid & 31] = make_float4(q.x * q_scale, q.y * q_scale, q.z * q_scale, q.w * q_scale);
         ks[buf][rtok][tid & 31] = walk_keep(a.k, rrow, dim, in, 0.f);
         float4 al = a.a;
-        if (LOGITS) {
+        if (LOGITS && in) {                                   // (the wavefronts of tokens that are not there have nothing to wait for)
             const float4 b = z_bias ? walk_rows<false>(z_bias + h * dim, rrow, dim) : make_float4(0.f, 0.f, 0.f, 0.f);
             al = make_float4(expf(log_sigmoid(al.x + b.x) * inv_tau), expf(log_sigmoid(al.y + b.y) * inv_tau),
                              expf(log_sigmoid(al.z + b.z) * inv_tau), expf(log_sigmoid(al.w + b.w) * inv_tau));
