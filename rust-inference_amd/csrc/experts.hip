@@ -141,12 +141,12 @@ experts_activate_kernel(T* __restrict__ out, const T* __restrict__ gu, const flo
     }
 }
 
-// The same eight bfloat16 elements a thread (ff a multiple of 8), a workgroup a stretch of 2,048 elements: 32 tokens of eight experts of
-// 6,144 in 6 us, where a workgroup an expert and an element a load takes 16.
+// The same eight bfloat16 elements a thread (ff a multiple of 8), a workgroup a stretch of up to 2,048 elements: 32 tokens of eight
+// experts of 6,144 in 3.8 us, where a workgroup an expert and an element a load takes 8.2.
 __global__ void __launch_bounds__(256)
 experts_activate_pieces_kernel(bf16_t* __restrict__ out, const bf16_t* __restrict__ gu, const float* __restrict__ dense,
                                int dense_stride, int experts, int ff, float limit) {
-    const int t = blockIdx.x, e = blockIdx.y, i = (blockIdx.z * 256 + threadIdx.x) * 8;
+    const int t = blockIdx.x, e = blockIdx.y, i = (blockIdx.z * blockDim.x + threadIdx.x) * 8;
     if (i >= ff) return;
     const float w = dense ? dense[(size_t)t * dense_stride + e] : 1.f;
     const bf16_t* g = gu + ((size_t)t * experts + e) * 2 * ff + i;
@@ -434,6 +434,14 @@ extern "C" int ri_experts_route(int32_t* ids, float* weights, float* dense, cons
                                     ROUTE_SIGMOID, 1, 1, 1, 1, stream);
 }
 
+// Whether bfloat16 rows go in pieces of eight elements: where an expert's row takes a thread of the other form six turns and more, or the
+// step is bound by memory.  Else a thread's eight exponentials one after the other are what a launch takes.  Us an element a load :
+// in pieces, tokens x experts x ff: 2,048 x 8 x 40 5.5 : 7.7, 512 x 128 x 128 18.7 : 19.4, 64 x 64 x 768 5.0 : 5.4, 300 x 8 x 520 3.7 : 4.6; 128 x 64
+// x 768 7.5 : 7.3, 64 x 8 x 1,536 3.6 : 3.2, 1 x 8 x 2,048 3.7 : 2.6, 512 x 128 x 256 26.6 : 19.7, 4,000 x 8 x 520 19.4 : 14.8.
+extern "C" int ri_experts_activate_pieces(int tokens, int experts, int ff) {
+    return ff % 8 == 0 && (ff >= 1536 || (ff >= 256 && (long)tokens * experts * ff >= 6L << 20));
+}
+
 extern "C" int ri_experts_activate_strided(void* out, const void* gu, int dtype, const float* dense, int dense_stride,
                                            int tokens, int experts, int ff, float limit, void* stream) {
     RI_REQUIRE(!dense || dense_stride >= experts, "experts_activate: weight rows of %d for %d experts", dense_stride, experts);
@@ -444,9 +452,9 @@ extern "C" int ri_experts_activate_strided(void* out, const void* gu, int dtype,
     hipStream_t s = (hipStream_t)stream;
     if (dtype == RI_F32)
         experts_activate_kernel<float><<<grid, 256, 0, s>>>((float*)out, (const float*)gu, dense, dense_stride, experts, ff, limit);
-    else if (ff % 8 == 0 && (ff / 8 + 255) / 256 <= 65535 && ((uintptr_t)out | (uintptr_t)gu) % 16 == 0)
-        experts_activate_pieces_kernel<<<dim3(tokens, experts, (ff / 8 + 255) / 256), 256, 0, s>>>((bf16_t*)out, (const bf16_t*)gu, dense,
-                                                                                                  dense_stride, experts, ff, limit);
+    else if (ri_experts_activate_pieces(tokens, experts, ff) && (ff / 8 + 255) / 256 <= 65535 && ((uintptr_t)out | (uintptr_t)gu) % 16 == 0)
+        experts_activate_pieces_kernel<<<dim3(tokens, experts, (ff / 8 + 255) / 256), ff < 2048 ? (ff / 8 + 63) / 64 * 64 : 256, 0, s>>>(
+            (bf16_t*)out, (const bf16_t*)gu, dense, dense_stride, experts, ff, limit);
     else
         experts_activate_kernel<bf16_t><<<grid, 256, 0, s>>>((bf16_t*)out, (const bf16_t*)gu, dense, dense_stride, experts, ff, limit);
     RI_LAUNCH_CHECK("experts_activate");

@@ -155,6 +155,7 @@ _SIGNATURES = {
                          c_int, c_int, c_void_p],
     "ri_experts_route_general": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_int, c_int, c_int,
                                  c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
+    "ri_experts_activate_pieces": [c_int, c_int, c_int],
     "ri_experts_activate_strided": [c_void_p, c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_int, c_float, c_void_p],
     "ri_experts_finish": [c_void_p, c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_int, c_void_p, c_int, c_int,
                           c_void_p],
@@ -1134,6 +1135,11 @@ def experts_combine(y: torch.Tensor, dest: torch.Tensor, weights: torch.Tensor) 
     _call("ri_experts_combine", _dev(out, "out"), _dev(y, "y", torch.bfloat16, (tokens * top, dim)),
           _dev(dest, "dest", torch.int32, (tokens * top,)), _dev(weights, "weights", torch.float32), tokens, top, dim, _stream())
     return out
+
+
+def experts_activate_pieces(tokens: int, experts: int, ff: int) -> bool:
+    """Whether ``experts_activate`` takes bfloat16 rows in pieces of eight elements (host code only: it needs no GPU)."""
+    return bool(_get("ri_experts_activate_pieces")(int(tokens), int(experts), int(ff)))
 
 
 def experts_activate(gu: torch.Tensor, dense, ff: int, limit: float) -> torch.Tensor:

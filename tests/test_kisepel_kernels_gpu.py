@@ -484,7 +484,7 @@ def test_a_shared_expert_without_a_gate_is_added_as_it_is(ops):
         close(ops.experts_finish(t(routed), None, t(shared), None), routed.sum(0) + shared.sum(0), F32)
 
 
-@pytest.mark.parametrize("tokens, experts, ff, limit", [(1, 1, 8, 0.0), (3, 5, 40, 1.1), (2, 2, 2056, 0.0)])
+@pytest.mark.parametrize("tokens, experts, ff, limit", [(1, 1, 8, 0.0), (3, 5, 40, 1.1), (2, 2, 2056, 0.0), (2, 3, 1536, 1.1), (3, 1, 1544, 0.0)])
 def test_experts_activation_in_pieces_is_the_one_by_elements(ops, tokens, experts, ff, limit):
     """Rows of a multiple of eight elements against the same numbers as float32, rounded once; experts not chosen give zeros over NaN."""
     rng = np.random.default_rng(ff)
@@ -494,3 +494,10 @@ def test_experts_activation_in_pieces_is_the_one_by_elements(ops, tokens, expert
     chosen = (dense[:, :experts, None] != 0).expand(-1, -1, 2 * ff).reshape(tokens, -1)
     got = ops.experts_activate(guarded(torch.where(chosen, gu, torch.full_like(gu, float("nan")))), dense, ff, limit)
     assert torch.equal(got, want)
+
+
+def test_experts_activation_of_short_rows_takes_an_element_a_load(ops):
+    """Rows of fewer than 1,536 elements go in pieces where the step is bound by memory alone."""
+    assert ops.experts_activate_pieces(1, 8, 1536) and ops.experts_activate_pieces(128, 64, 768) and ops.experts_activate_pieces(4000, 8, 520)
+    assert not (ops.experts_activate_pieces(64, 64, 768) or ops.experts_activate_pieces(2048, 8, 40) or ops.experts_activate_pieces(512, 128, 128)
+                or ops.experts_activate_pieces(1, 8, 2052))
