@@ -493,6 +493,43 @@ def test_talking_attention_cuts_no_page_between_shares(ops, monkeypatch):
 
 # ---------------------------------------------------------------- the walks over states of 65 to 128 rows
 @pytest.mark.parametrize("kind", ["ssd", "timemix", "gla"])
+def test_walks_take_a_state_that_starts_anywhere(ops, kind):
+    """A state that is a part of a larger buffer, four bytes behind the boundary of 16-byte loads: the same bits, and nothing beside it
+    is touched."""
+    rng = np.random.default_rng(5)
+    heads, n, T = 2, 68, 3
+    start = rng.standard_normal(heads * n * n)
+    cu, slots = t([0, 1, 2, 3], torch.int32), t([0, 0, 0], torch.int32)[:1]
+    row = rng.standard_normal((T, 4 * heads * n))
+    zero = t(np.zeros(heads * n))
+
+    def run(offset):
+        whole = guarded(torch.full((offset + heads * n * n + 3,), 7.0, device=DEV))
+        state = whole[offset:offset + heads * n * n].view(1, heads, n, n)
+        state.copy_(torch.tensor(start, dtype=torch.float32).view(1, heads, n, n))
+        outs = []
+        for k in range(T):                                    # (single tokens: four columns a lane)
+            one, c1 = row[k:k + 1], t([0, 1], torch.int32)
+            a, b, v, z = (one[:, i * heads * n:(i + 1) * heads * n] for i in range(4))
+            if kind == "ssd":
+                proj = t(np.concatenate([z, one[:, :heads]], 1))
+                outs.append(ops.ssd_scan(t(np.concatenate([v, b, a], 1)), heads * n, 2 * heads * n, proj, 0, heads * n, None, t(np.zeros(heads)),
+                                         None, state, c1, slots, heads, heads, n, n))
+            elif kind == "timemix":
+                o = guarded(torch.zeros((1, heads * n), device=DEV))
+                ops.timemix_scan(o, 0, 1.0, t(a), t(b), t(v), t(z), t(z), zero, zero, t(np.ones(heads * n)), 1e-5, state, c1, slots, heads, n)
+                outs.append(o)
+            else:
+                outs.append(ops.gla_scan(t(np.concatenate([a, b, v], 1)), 0, heads * n, 2 * heads * n, t(z), None, 2.0, 1.0, state, c1, slots,
+                                         heads, n, n))
+        assert (whole[:offset] == 7).all() and (whole[offset + heads * n * n:] == 7).all()
+        return np.concatenate([f64(x) for x in outs]), f64(state)
+
+    at, off = run(0), run(1)
+    assert np.isfinite(at[0]).all() and np.array_equal(at[0], off[0]) and np.array_equal(at[1], off[1])
+
+
+@pytest.mark.parametrize("kind", ["ssd", "timemix", "gla"])
 @pytest.mark.parametrize("rows, cols, heads, many", [(65, 65, 2, False), (100, 33, 2, False), (128, 40, 1, False), (128, 128, 33, True)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_walks_in_tiles_of_four_rows(ops, kind, rows, cols, heads, many, dtype):
