@@ -45,10 +45,10 @@ __device__ __forceinline__ float4 walk_keep(const float4 v, int row, int n, bool
                        token && row + 3 < n ? v.w : fill);
 }
 
-// A lane's tile of the state, and back.
+// A lane's tile of the state, and back: 16 bytes of a row at a time where the state starts on the boundary of such loads.
 template <int CPL>
 __device__ __forceinline__ void walk_load(float (&st)[4][CPL], const float* sp, int row0, int n, int c0, int vdim) {
-    if (CPL == 4 && vdim % 4 == 0) {
+    if (CPL == 4 && vdim % 4 == 0 && (uintptr_t)sp % 16 == 0) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const float4 v = *reinterpret_cast<const float4*>(sp + (size_t)min(row0 + i, n - 1) * vdim + min(c0, vdim - 4));
@@ -68,11 +68,12 @@ __device__ __forceinline__ void walk_load(float (&st)[4][CPL], const float* sp, 
 }
 template <int CPL>
 __device__ __forceinline__ void walk_store(const float (&st)[4][CPL], float* sp, int row0, int n, int c0, int vdim) {
+    const bool four = CPL == 4 && vdim % 4 == 0 && (uintptr_t)sp % 16 == 0;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         if (row0 + i >= n) continue;
         float* to = sp + (size_t)(row0 + i) * vdim + c0;
-        if (CPL == 4 && vdim % 4 == 0) {
+        if (four) {
             if (c0 < vdim)
                 *reinterpret_cast<float4*>(to) = make_float4(st[i][0], st[i][CPL > 1 ? 1 : 0], st[i][CPL > 2 ? 2 : 0], st[i][CPL > 3 ? 3 : 0]);
         } else {
