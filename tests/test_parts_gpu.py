@@ -172,6 +172,36 @@ def test_prenorm_block_leaves_norms_to_the_products(rows):
     assert rel_to_max(f64(x), P.rms_norm(h1[-1:], w64["b"], eps)) < 1e-2
 
 
+@pytest.mark.parametrize("n, k", [(16384, 72), (16385, 264), (24576, 8), (16383, 72)])
+def test_plain_matrices_of_many_rows_take_the_wide_kernel_at_17_to_48_rows(n, k, monkeypatch):
+    """From four row tiles a compute unit on: edges of the row tiles, of the slices of K and of the rows that it is chosen for, bfloat16 and
+    float32 sums, against float64; below that size and past those rows the product is another kernel's, with the same result."""
+    from rust_inference_amd.kernels import ops
+    from rust_inference_amd.parts import runtime
+    rt = runtime.Runtime(DEV, torch.bfloat16)
+    monkeypatch.setattr(runtime, "MID_MAX_BYTES", 0)           # (matrices of these sizes are the packed kernel's otherwise)
+    rng = np.random.default_rng(k)
+    w = t(rng.normal(size=(n, k)) / np.sqrt(k), torch.bfloat16)
+    pw = runtime.PackedWeight(w, ops.pack_for_mfma(w), False)
+    taken, kernel = [], ops.gemm_wide_packed_bf16
+    monkeypatch.setattr(ops, "gemm_wide_packed_bf16", lambda *a, **kw: (taken.append(kw["waves"]), kernel(*a, **kw))[1])
+    for m in (17, 32, 33, 48, 49):
+        x = t(rng.normal(size=(m, k)), torch.bfloat16)
+        want = f64(x) @ f64(w).T
+        taken.clear()
+        assert rel_to_max(f64(rt.linear_packed(x, pw)), want) < 1e-2
+        assert rel_to_max(f64(rt.linear_packed(x, pw, out_dtype=torch.float32)), want) < 1e-5
+        if ops.compute_units() == 256:
+            assert taken == ([runtime._wide_whole_waves(n, m)] * 2 if n >= 16384 and m <= 48 else [])
+
+
+def test_wavefronts_of_a_whole_wide_product(monkeypatch):
+    """Three or four row tiles a workgroup, whichever has a compute unit fetch fewer rows over its rounds."""
+    from rust_inference_amd.parts import runtime
+    monkeypatch.setattr(runtime, "_compute_units", lambda: 256)
+    assert [runtime._wide_whole_waves(n, 32) for n in (16384, 24576, 65536, 98304)] == [4, 3, 4, 4]
+
+
 def test_tiled_rows_reach_every_kind_of_product():
     """Rows in the matrix cores' order may meet a product that has no packed kernel for them (a matrix
     without a packed copy, the one-row kernel, the library): it gets plain rows and gives the same result."""
