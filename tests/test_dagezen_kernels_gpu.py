@@ -482,6 +482,41 @@ def test_talking_attention_on_the_matrix_cores_is_the_general_kernel(ops, heads,
         close(got, f64(want), 1.5e-2, "matrix cores against the general kernels")
 
 
+@pytest.mark.parametrize("dim, window, table", [(32, 40, True), (64, 45, False), (128, None, False)])
+def test_talking_attention_whole_and_in_shares(ops, dim, window, table, monkeypatch):
+    """Tiles that are walked whole, whose result is bfloat16 at once, and in two, three and four shares of their pages, whose float32 sums
+    are added first, some of them without a page; the bias from the table of distances and as a logarithm a score.  Each against the
+    general kernel, and the shares against the whole: a sum of fewer than 128 weighted values (their magnitudes' sum is under 30) in another
+    order, then a rounding to bfloat16."""
+    torch.manual_seed(dim)
+    rng = np.random.default_rng(dim)
+    heads, kv_heads, counts, starts, lens = 8, 2, [33, 70], [21, 0], [54, 70]
+    k_pages = guarded((torch.randn((10, kv_heads, PAGE, dim), device=DEV) * 0.6).to(torch.bfloat16))
+    v_pages = guarded((torch.randn((10, kv_heads, dim, PAGE), device=DEV) * 0.6).to(torch.bfloat16))
+    pages = t([[5, 2, 9], [7, 1, 3]], torch.int32)
+    tok_seq = t([0] * 33 + [1] * 70, torch.int32)
+    tok_pos = t(list(range(21, 54)) + list(range(70)), torch.int32)
+    cu = t([0, 33, 103], torch.int32)
+    proj = guarded((torch.randn((103, heads * dim), device=DEV) * 0.6).to(torch.bfloat16))
+    r1, r2 = t(rng.random(heads)), t(rng.random(heads) * 3)
+    talk = t(np.eye(heads) + 0.3 * rng.standard_normal((heads, heads)))
+    want = f64(ops.talking_attention(proj, 0, k_pages, v_pages, tok_pos, tok_seq, pages, heads, kv_heads, dim, window, 0.2, r1, r2, talk))
+    monkeypatch.setattr(ops, "compute_units", lambda: 256)
+    monkeypatch.setattr(ops, "TALKING_TABLE_WINDOW", 16384 if table else 0)
+    whole = None
+    for shares in (1, 2, 3, 4):
+        monkeypatch.setattr(ops, "TALKING_MAX_SHARES", shares)
+        for longest in (max(lens), None):
+            assert ops.talking_attention_mfma_shares(8, longest, window) == (min(shares, 3) if longest and window is None else
+                                                                            min(shares, 2) if longest else shares)
+            got = ops.talking_attention_mfma(proj, 0, k_pages, v_pages, tok_pos, cu, counts, pages, heads, kv_heads, dim, window, 0.2,
+                                             r1, r2, talk, longest)
+            close(got, want, 1.5e-2, f"{shares} shares against the general kernel")
+            got = f64(got)
+            whole = got if whole is None else whole
+            assert (np.abs(got - whole) <= 2.0 ** -7 * np.abs(whole) + 128 * 2.0 ** -24 * 30).all(), f"{shares} shares against one"
+
+
 def test_talking_attention_cuts_no_page_between_shares(ops, monkeypatch):
     """As many shares as leave no compute unit idle, none of them without a page: prompts of a page or two are walked whole or in two."""
     monkeypatch.setattr(ops, "compute_units", lambda: 256)
