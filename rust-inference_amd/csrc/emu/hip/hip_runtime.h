@@ -169,6 +169,14 @@ static inline int emu_mov_dpp_quad(int v, int control) {
     return all[(lane & ~3) | ((control >> (2 * (lane & 3))) & 3)];
 }
 #define __builtin_amdgcn_mov_dpp(v, control, row_mask, bank_mask, bound_ctrl) emu_mov_dpp_quad((v), (control))
+// v_perm_b32: byte i of the result is the one that byte i of `sel` names, 0 .. 3 of b and 4 .. 7 of a.
+static inline uint32_t emu_perm(uint32_t a, uint32_t b, uint32_t sel) {
+    const uint64_t both = (uint64_t)a << 32 | b;
+    uint32_t r = 0;
+    for (int i = 0; i < 4; ++i) r |= (uint32_t)(both >> 8 * (sel >> 8 * i & 7) & 255) << 8 * i;
+    return r;
+}
+#define __builtin_amdgcn_perm(a, b, sel) emu_perm((a), (b), (sel))
 #define __builtin_amdgcn_readlane(v, l) emu_readlane((int)(v), (l))
 #define __builtin_amdgcn_readfirstlane(v) emu_readfirstlane((int)(v))
 // The lanes of a wavefront run in step on the GPU, so what one lane has written to LDS another lane reads

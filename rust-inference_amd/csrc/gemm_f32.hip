@@ -40,7 +40,9 @@ __device__ __forceinline__ void split8(const float4 lo, const float4 hi, uint4& 
 #pragma unroll
     for (int part = 0; part < 3; ++part) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) p[part][i] = upper_halves(v[2 * i], v[2 * i + 1]);
+        for (int i = 0; i < 4; ++i)                           // (the last part's cut off halves are not needed: one byte exchange for two)
+            p[part][i] = part < 2 ? upper_halves(v[2 * i], v[2 * i + 1])
+                                  : __builtin_amdgcn_perm(__float_as_uint(v[2 * i + 1]), __float_as_uint(v[2 * i]), 0x07060302u);
 #pragma unroll
         for (int i = 0; i < 8; ++i) v[i] = part == 0 ? below_upper(v[i]) * F32_LOWER : below_upper(v[i]);
     }
@@ -252,10 +254,11 @@ extern "C" int ri_gemm_f32(float* out, const float* x, const void* w, int w_dtyp
     else if (!aligned)
         gemm_f32_kernel<bf16_t><<<grid, 256, 0, s>>>(out, x, (const bf16_t*)w, m, n, k);
     else {
-        // The largest tile that still gives every compute unit a workgroup: a tile's time grows more slowly than its work.
-        // 759 rows, us for 32 x 32 / 32 x 64 / 64 x 128: 1,024 x 3,072 36 / 35 / 49, 4,096 x 1,024 43 / 33 / 31, 6,144 x 1,024
-        // 65 / 48 / 46 (the vector units' form: 363, 127, 176); 33 rows of 1,024 x 3,072 20 / 23 / 47, 2,048 rows 109 / 64 / 51.
-        // Up to 32 rows half of a tile of 64 would be padding: 151,936 x 1,024 at one row 67 / 55 / 68 (302).
+        // A tile's time grows more slowly than its work: tiles of 64 x 128 where they still give every compute unit a workgroup, else
+        // 32 x 64 as soon as 32 x 32 would need a second round of workgroups.
+        // 759 rows, us for 32 x 32 / 32 x 64 / 64 x 128: 1,024 x 3,072 37 / 34 / 48, 4,096 x 1,024 46 / 32 / 31, 6,144 x 1,024
+        // 64 / 45 / 46 (the vector units' form: 363, 127, 176); 33 rows of 1,024 x 3,072 19 / 23 / 46, 2,048 rows 110 / 64 / 55.
+        // Up to 32 rows half of a tile of 64 would be padding: 151,936 x 1,024 at one row 77 / 57 / 75 (302).
         const auto tiles = [&](int rows, int cols) { return (long)((m + rows - 1) / rows) * ((n + cols - 1) / cols); };
         const bf16_t* wb = (const bf16_t*)w;
         RI_REQUIRE(tiles(32, 32) + 8 * ((m + 31) / 32) < (1L << 31), "gemm_f32: %d x %d exceed one launch", m, n);
