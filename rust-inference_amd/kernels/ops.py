@@ -532,10 +532,13 @@ ATTENTION_ROWS = 16              # rows of queries that share their loads (ATT_R
 ATTENTION_ROWS_FROM = 4          # new tokens a sequence brings at least, and
 ATTENTION_ROWS_FILL = 8          # rows that its runs fill at least, for its tokens to run by rows
 # Bytes of keys, a compute unit, that a workgroup a (token, head) reads in the time in which a workgroup by rows walks 256 keys:
-# some 36 us whatever it shares them with.  One prompt of float32 heads of 128 (16 over 8), tokens @ cached tokens, us a workgroup a
-# (token, head) : by rows: 130 @ 0 28 : 39 (270 KB), 160 @ 0 39 : 41 (410), 200 @ 0 52 : 46 (640), 400 @ 0 166 : 98 (1,280), 130 @
-# 2,000 527 : 381 (950); heads of 64 (16 over 16) 320 @ 0 71 : 72 (410), 400 @ 0 99 : 83 (640); bfloat16 heads of 24 520 @ 0 89 : 105 (130).
-ATTENTION_ROWS_BYTES = 550_000
+# some 36 us whatever it shares them with.  A key costs that form 0.05 ns a byte and as much as 128 bytes beside them (33 ns of 512 bytes, 20 of
+# 256, 13 of 144, 9 of 48, over 256 compute units).  One prompt of float32 heads of 128 (16 over 8), tokens @ cached tokens, us a workgroup a
+# (token, head) : by rows (the sum's KB): 130 @ 0 27 : 38 (340), 160 @ 0 38 : 41 (510), 200 @ 0 51 : 45 (800), 400 @ 0 165 : 87 (1,600), 64 @ 2,000
+# 248 : 356 (580), 130 @ 2,000 528 : 363 (1,190); heads of 64 (16 over 16) 320 @ 0 72 : 68 (615), 400 @ 0 99 : 77 (960); bfloat16 heads of 24 520 @ 0
+# 90 : 85 (495), 1,000 @ 0 267 : 162 (1,375), of 72 700 @ 0 200 : 116 (1,390).
+ATTENTION_ROWS_BYTES = 600_000
+ATTENTION_KEY_BYTES = 128
 
 
 def attention_rows_plan(new_counts, starts, heads: int, kv_heads: int, row_bytes: int, reach: int | None):
@@ -553,7 +556,7 @@ def attention_rows_plan(new_counts, starts, heads: int, kv_heads: int, row_bytes
             tokens, runs = tokens + n, runs - (-n // per)
             keys += n * (min(seen, reach) if reach else seen)
             deepest = max(deepest, -(-min(start + n, reach + 256 if reach else start + n) // 256))
-    if keys * heads * row_bytes < deepest * ATTENTION_ROWS_BYTES * compute_units():
+    if keys * heads * (row_bytes + ATTENTION_KEY_BYTES) < deepest * ATTENTION_ROWS_BYTES * compute_units():
         return rows_from, 0, 0
     return rows_from, tokens, runs
 

@@ -420,6 +420,7 @@ def test_attention_shares_loads_where_that_is_less_to_wait_for(ops, monkeypatch)
     assert plan([1] * 64 + [300], [2000] * 64 + [0]) == (300, 38) and plan([130], [2000]) == (130, 17)
     assert plan([130], [0]) == plan([4] * 200, [0] * 200) == plan([1] * 300, [1000] * 300) == plan([1] * 300 + [4], [1000] * 301) == (0, 0)
     assert plan([200], [3000], reach=512) == (200, 25) and plan([2000], [0], 32, 1) == (0, 0)      # (32 heads a kv head: too many rows)
+    assert ops.attention_rows_plan([1000], [0], 16, 8, 48, None)[1:] == (1000, 125)               # (small rows: what a key costs beside its bytes)
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
