@@ -234,6 +234,7 @@ int ri_attention_prefill_bf16(void* out, const void* qkv, int q_stride, const vo
 // sequence after this step), pieces = ri_attention_decode_pieces(seqs, kv_heads, heads, max_chunks); at most 16
 // query heads per kv head.
 int ri_attention_decode_chunks(int max_len);
+int ri_attention_decode_ranks(int seqs, int kv_heads, int max_chunks);
 int ri_attention_decode_pieces(int seqs, int kv_heads, int heads, int max_chunks);
 // Whether ri_attention_decode_bf16 takes a step of this size with its streaming kernel (a workgroup walks a
 // whole run of a sequence's pages; no join when a sequence is one run): the number of runs per sequence, or

@@ -944,20 +944,16 @@ __device__ __forceinline__ void finish_head(bf16_t* dst_lds, const HeadLoads<DH>
 // Which (sequence, kv head) a workgroup takes, and the sequence's position, where sequences run whole and two workgroups and
 // more share a compute unit: a unit takes as long as its walks together, and in the launch's own order (64 sequences of 8 kv
 // heads on 256 units) they are of one sequence, the longest with itself.  The sequences are ranked by their lengths (every
-// workgroup for itself), the longest go out first, and every second round of workgroups runs the other way, so that the
+// wavefront for itself), the longest go out first, and every second round of workgroups runs the other way, so that the
 // longest meets the shortest.  Eight sequences go out side by side and then their next heads: an XCD then has whole sequences.
-// Lengths within a sixteenth of the first's stay in the launch's order: there the ranking only costs (200 sequences of 800 keys:
-// 134.5 us a layer, 136.0 with the look at them, ranked too 144.8).  64 sequences of 1,100 to 2,040 keys at 32 heads of 128:
-// 80.0 us in the launch's order, 72.3 ranked; of 30 to 4,000: 133.9, 100.6; 200 of 30 to 2,000: 194.0, 167.8.
+// Lengths within a sixteenth of the first's stay in the launch's order: there the ranking only costs.
 #define STREAM_BALANCE_MOST 256  // sequences
-template <int W>
 __device__ __forceinline__ int stream_balance(int& b, int& kvh, const int32_t* __restrict__ tok_pos, int kv_heads, int units,
-                                              const Reach& reach, int32_t* __restrict__ len) {
-    __shared__ int chosen[2];  // (len is the workgroup's LDS for its sums, which nothing has written yet)
+                                              const Reach& reach, int most_keys) {
     constexpr int HELD = STREAM_BALANCE_MOST / 64;
-    const int n = gridDim.x, tid = threadIdx.x, lane = tid & 63;
+    const int n = gridDim.x, lane = threadIdx.x & 63;
     const int own = tok_pos[b], first = tok_pos[0];
-    int pos[HELD], far = 0;
+    int pos[HELD], len[HELD], far = 0;
 #pragma unroll
     for (int i = 0; i < HELD; ++i) pos[i] = tok_pos[min(64 * i + lane, n - 1)];
     __builtin_amdgcn_sched_barrier(0);  // (one trip to memory for all of them)
@@ -965,41 +961,55 @@ __device__ __forceinline__ int stream_balance(int& b, int& kvh, const int32_t* _
     const int first_len = first + 1 - reach.first(first);
 #pragma unroll
     for (int i = 0; i < HELD; ++i) {
-        const int more = pos[i] + 1 - reach.first(pos[i]) - first_len;
+        len[i] = pos[i] + 1 - reach.first(pos[i]);
+        const int more = len[i] - first_len;
         far |= 16 * max(more, -more) > first_len;
+        if (64 * i + lane >= n) len[i] = -1;
     }
     if (!__any(far)) return own;
-    const int padded = (n + 15) & ~15;
-    if (tid < 64)
-#pragma unroll
-        for (int i = 0; i < HELD; ++i) len[64 * i + lane] = 64 * i + lane < n ? pos[i] + 1 - reach.first(pos[i]) : -1;
-    __syncthreads();
     const int at = blockIdx.x + n * blockIdx.y, round = at / units, place = at - round * units;
     const int unit = round * units + ((round & 1) ? min(units, n * kv_heads - round * units) - 1 - place : place);
     const int set = unit / (8 * kv_heads), in_set = unit - set * 8 * kv_heads, wide = min(8, n - 8 * set);
-    const int rank = 8 * set + in_set % wide;
-    for (int i = tid; i < n; i += W * 64) {
-        const int mine = len[i];
-        int before = 0;
-        for (int k = 0; k < padded; k += 16)
+    // The length that `before` sequences exceed, a bit at a time from the top (a comparison of all by every workgroup took 256
+    // sequences of 10 to 256 keys from 39 to 61 us), then the right one of those that have it.
+    int rank = 8 * set + in_set % wide, mine = 0;
+    for (int bit = 31 - __builtin_clz(most_keys); bit >= 0; --bit) {
+        int count = 0;
 #pragma unroll
-            for (int d = 0; d < 16; d++) before += len[k + d] > mine || (len[k + d] == mine && k + d < i);
-        if (before == rank) {
-            chosen[0] = i;
-            chosen[1] = tok_pos[i];
-        }
+        for (int i = 0; i < HELD; ++i) count += __builtin_popcountll(__ballot(len[i] >= (mine | 1 << bit)));
+        if (count > rank) mine |= 1 << bit;
     }
-    __syncthreads();
-    b = __builtin_amdgcn_readfirstlane(chosen[0]);
+    unsigned long long same[HELD];
+#pragma unroll
+    for (int i = 0; i < HELD; ++i) {
+        rank -= __builtin_popcountll(__ballot(len[i] > mine));
+        same[i] = __ballot(len[i] == mine);
+    }
+    int qpos = own;
+#pragma unroll
+    for (int i = 0; i < HELD; ++i) {
+        const int count = __builtin_popcountll(same[i]);
+        if (rank >= 0 && rank < count) {
+            const unsigned long long me = __ballot((same[i] >> lane & 1) && __builtin_popcountll(same[i] & ((1ull << lane) - 1)) == rank);
+            const int who = __builtin_ctzll(me);
+            b = 64 * i + who;
+            qpos = __builtin_amdgcn_readlane(pos[i], who);
+        }
+        rank -= count;
+    }
     kvh = in_set / wide;
-    return __builtin_amdgcn_readfirstlane(chosen[1]);
+    return qpos;
 }
 
-// The compute units for stream_balance, or 0 where the order makes no difference: one round of workgroups, runs, or more
-// sequences than it ranks.
-static int stream_balances(int seqs, int kv_heads, int splits) {
+// The compute units for stream_balance, or 0 where the order makes no difference (one round of workgroups, runs), where there are
+// more sequences than it ranks, and where the bound on the lengths is one chunk: walks so short end within the look at the others'
+// lengths of one another (us a layer without : with, 32 heads of 128 over 8: 256 sequences of 250 keys 46.8 : 49.5, of 10 to 256 39.1 : 41.0, 128
+// of 250 24.4 : 25.8).  Else equal lengths pay half a microsecond a launch for the look (64 of 300 15.9 : 16.5, of 800 34.6 : 35.2, 256 of
+// 500 85.1 : 85.8, of 1,000 164.7 : 165.0, 200 of 800 108.2 : 108.6) and unequal ones gain: 64 of 30 to 300 14.1 : 13.3, of 1,100 to 2,040
+// 75.8 : 67.8, of 30 to 4,000 136.2 : 110.3; 128 of 100 to 500 36.9 : 32.7; 200 of 30 to 2,000 159.8 : 131.4; 256 of 200 to 1,000 131.2 : 107.6.
+static int stream_balances(int seqs, int kv_heads, int splits, int max_chunks) {
     const int cus = ri_compute_units();
-    return splits == 1 && seqs > 1 && seqs <= STREAM_BALANCE_MOST && (long)seqs * kv_heads > cus ? cus : 0;
+    return splits == 1 && max_chunks > 1 && seqs > 1 && seqs <= STREAM_BALANCE_MOST && (long)seqs * kv_heads > cus ? cus : 0;
 }
 
 // FUSED: qkv is the raw projection; the kernel norms and rotates the group's queries for itself, and the
@@ -1026,7 +1036,7 @@ attn_decode_stream_kernel(bf16_t* __restrict__ out, float* __restrict__ ws, cons
     const int split = blockIdx.z;
     const int group = heads / kv_heads;
     // (token b is sequence b's one new token)
-    const int qpos = balance > 0 ? stream_balance<W>(b, kvh, tok_pos, kv_heads, balance, reach, reinterpret_cast<int32_t*>(o_lds)) : tok_pos[b];
+    const int qpos = balance > 0 ? stream_balance(b, kvh, tok_pos, kv_heads, balance, reach, table_width * PAGE) : tok_pos[b];
     const int lo = reach.first(qpos);
     const int c_lo = lo / DECODE_CHUNK, c_hi = qpos / DECODE_CHUNK;
     const int per = (c_hi - c_lo + splits) / splits;         // chunks per run: by the sequence's own length

@@ -95,6 +95,11 @@ extern "C" int ri_attention_prefill_bf16(void* out, const void* qkv, int q_strid
                                           0, nullptr, stream);
 }
 
+// Whether the streaming kernel ranks the step's sequences by their lengths (host code only).
+extern "C" int ri_attention_decode_ranks(int seqs, int kv_heads, int max_chunks) {
+    return !stream_wide(seqs, kv_heads, max_chunks) && stream_balances(seqs, kv_heads, stream_splits(seqs, kv_heads, max_chunks), max_chunks) > 0;
+}
+
 extern "C" int ri_attention_decode_chunks(int max_len) { return (max_len + DECODE_CHUNK - 1) / DECODE_CHUNK; }
 
 // The workspace of a decode attention call has room for max_chunks times this many results a sequence and head.
@@ -143,7 +148,7 @@ extern "C" int ri_attention_decode_kept_bf16(void* out, float* workspace, const 
                 (bf16_t*)out, workspace, (const bf16_t*)qkv, q_stride, nullptr, nullptr, 0.f, nullptr,            \
                 (bf16_t*)k_pages, (bf16_t*)v_pages, tok_pos, page_table, table_width, heads, kv_heads, reach,     \
                 scale_log2, splits, tiled_out, cap_pre, cap_post, slopes, 1.f / scale, sinks, DH, DH,             \
-                stream_balances(seqs, kv_heads, splits));                                                         \
+                stream_balances(seqs, kv_heads, splits, max_chunks));                                                         \
         if (splits > 1)                                                                                          \
             launch_join<DH>((bf16_t*)out, workspace, tok_pos, seqs, heads, Reach{-1, 0}, splits, tiled_out, s, DECODE_CHUNK, 0, sinks); \
         break;
@@ -231,7 +236,7 @@ extern "C" int ri_attention_decode_fused_bf16(void* out, float* workspace, const
                 (bf16_t*)out, workspace, (const bf16_t*)qkv, q_stride, q_gain, k_gain, eps, inv_freq,             \
                 (bf16_t*)k_pages, (bf16_t*)v_pages, tok_pos, page_table, table_width, heads, kv_heads, reach,     \
                 scale_log2, splits, tiled_out, 0.f, 0.f, nullptr, 0.f, nullptr, DH, DH,                           \
-                stream_balances(seqs, kv_heads, splits));                                                         \
+                stream_balances(seqs, kv_heads, splits, max_chunks));                                                         \
         if (splits > 1) launch_join<DH>((bf16_t*)out, workspace, tok_pos, seqs, heads, Reach{-1, 0}, splits, tiled_out, s); \
         break;
         switch (head_dim) {

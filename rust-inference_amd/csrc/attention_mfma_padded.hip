@@ -106,7 +106,7 @@ extern "C" int ri_attention_decode_padded_bf16(void* out, float* workspace, cons
         (bf16_t*)out, workspace, (const bf16_t*)qkv, q_stride, nullptr, nullptr, 0.f, nullptr, (bf16_t*)k_pages,  \
         (bf16_t*)v_pages, tok_pos, page_table, table_width, heads, kv_heads, reach, scale_log2, splits,          \
         tiled_out, cap_pre, cap_post, slopes, 1.f / scale, sinks, dim, vdim,                          \
-        stream_balances(seqs, kv_heads, splits))
+        stream_balances(seqs, kv_heads, splits, max_chunks))
 #define RI_CASE(DH, DV)                                                                                           \
     case DH * 512 + DV:                                                                                           \
         if (wide) RI_STREAM(DH, 8, DV);                                                                           \

@@ -87,6 +87,7 @@ _SIGNATURES = {
     "ri_gemm_wide_stretch_plan": [c_int, c_int, c_int, c_void_p, c_void_p],
     "ri_compute_units": [],
     "ri_sum_parts": [c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p],
+    "ri_attention_decode_ranks": [c_int, c_int, c_int],
     "ri_attention_decode_chunks": [c_int],
     "ri_attention_decode_streams": [c_int, c_int, c_int],
     "ri_attention_decode_pieces": [c_int, c_int, c_int, c_int],
@@ -1295,6 +1296,11 @@ def decode_attention_runs(seqs: int, kv_heads: int, max_len: int) -> int:
     where it takes one workgroup per chunk of 256 keys instead (host code only: it needs no GPU)."""
     chunks = _get("ri_attention_decode_chunks")(int(max_len))
     return _get("ri_attention_decode_streams")(int(seqs), int(kv_heads), chunks)
+
+
+def decode_attention_ranks(seqs: int, kv_heads: int, max_len: int) -> bool:
+    """Whether the streaming kernel ranks the sequences of a step of this size by their lengths (host code only: it needs no GPU)."""
+    return bool(_get("ri_attention_decode_ranks")(int(seqs), int(kv_heads), _get("ri_attention_decode_chunks")(int(max_len))))
 
 
 def decode_attention_streams(seqs: int, kv_heads: int, max_len: int) -> bool:

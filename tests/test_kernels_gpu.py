@@ -656,6 +656,29 @@ def test_streams_that_share_a_compute_unit_take_every_sequence_once(ops, seqs, k
     close(out, want, BF16_OUT, f"{seqs} sequences of {kv_heads} heads")
 
 
+@pytest.mark.parametrize("window", [None, 40])
+def test_streams_that_share_a_compute_unit_and_their_ranks(ops, window):
+    """Lengths that all differ, that are one for a half of the sequences and the rest longer or shorter, and that a window makes one; more
+    sequences than a wavefront has lanes, the last length of all the longest."""
+    if ops.compute_units() not in (256, 1):
+        pytest.skip("the sizes are for the machine's")
+    seqs, kv_heads = 130, 4
+    assert ops.decode_attention_ranks(seqs, kv_heads, 400)
+    for lens in ([1 + (37 * i) % 131 for i in range(seqs - 1)] + [200], [64] * 65 + [63] * 32 + [65] * 33, [48 + i % 2 for i in range(seqs)]):
+        out, want = attention_case(ops, np.random.default_rng(1), lens, [1] * seqs, kv_heads, kv_heads, 32, torch.bfloat16, window,
+                                   kernel="decode")
+        close(out, want, BF16_OUT, f"{lens[:4]} ...")
+
+
+def test_streams_are_ranked_where_their_walks_are_longer_than_the_look(ops):
+    """Several streams a compute unit whose bound is more than one chunk of keys, up to 256 of them."""
+    if ops.compute_units() != 256:
+        pytest.skip("the sizes are for the machine's")
+    ranks = ops.decode_attention_ranks
+    assert ranks(64, 8, 257) and ranks(256, 8, 2000) and ranks(100, 8, 2000)
+    assert not (ranks(256, 8, 256) or ranks(64, 8, 100) or ranks(32, 8, 2000) or ranks(257, 8, 2000) or ranks(1, 8, 100000))
+
+
 @pytest.mark.parametrize("heads, kv_heads, dh", [(8, 8, 32), (32, 8, 128)])
 def test_fused_decode_attention_streams_long_sequences_in_runs(ops, heads, kv_heads, dh):
     """And with long sequences cut into 16 runs each: the last run that is not empty holds the new token."""
