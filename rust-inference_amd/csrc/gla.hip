@@ -354,7 +354,7 @@ static int gla_scan_go(float* out, const void* proj, int act_dtype, int row, int
 #define RI_GLA_ROWS(T)                                                                                               \
     switch (fixed) {                                                                                                 \
         case 4: RI_GLA_STAGE(T, 4) break;                                                                            \
-        case 8: RI_GLA_STAGE(T, 8) break;                                                                            \
+        case 8: if (few) { RI_GLA_GO(T, 8, 4, true); } else { RI_GLA_GO(T, 8, 16, true); } break;     /* (of one decay a head) */ \
         case 16: RI_GLA_STAGE(T, 16) break;                                                                          \
         case 32: RI_GLA_STAGE(T, 32) break;                                                                          \
         default: RI_GLA_STAGE(T, 0) break;                                                                           \

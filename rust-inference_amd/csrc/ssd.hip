@@ -271,15 +271,15 @@ extern "C" int ri_ssd_scan(float* out, const float* xbc, int channels, int b_off
 #define SSD_BLOCK 8
 #define SSD_WAVES 4          // wavefronts of a workgroup: they share the staged tokens, each on columns of its own
 
-template <typename TA, int RPL, int SL>                       // RPL: rows a lane holds, a multiple of 4; SL: slices of rows, 4
+template <typename TA, int RPL>                               // RPL: rows a lane holds, a multiple of 4
 __global__ void __launch_bounds__(64 * SSD_WAVES)
 ssd_scan_cols_kernel(float* __restrict__ out, const float* __restrict__ xbc, int channels, int b_off, int c_off,
                      const TA* __restrict__ proj, int stride, int z_off, int dt_off, const float* __restrict__ dt_bias,
                      const float* __restrict__ a_log, const float* __restrict__ d_skip, float* __restrict__ state,
                      const int32_t* __restrict__ cu_seqlens, const int32_t* __restrict__ slots, int heads, int groups, int n,
                      int vdim) {
-    // COLS: columns of a wavefront; NC: of the workgroup; TPP: tokens whose x and z one pass of the workgroup's threads fetches
-    constexpr int ROWS = SL * RPL, COLS = 64 / SL, NC = COLS * SSD_WAVES, THREADS = 64 * SSD_WAVES, TPP = THREADS / NC,
+    // SL: slices of rows; COLS: columns of a wavefront; NC: of the workgroup; TPP: tokens whose x and z one pass of the workgroup's threads fetches
+    constexpr int SL = 4, ROWS = SL * RPL, COLS = 64 / SL, NC = COLS * SSD_WAVES, THREADS = 64 * SSD_WAVES, TPP = THREADS / NC,
                   PASSES = SSD_BLOCK / TPP;
     __shared__ __attribute__((aligned(16))) float bs[2][SSD_BLOCK][ROWS];
     __shared__ __attribute__((aligned(16))) float cs[2][SSD_BLOCK][ROWS];
@@ -524,12 +524,12 @@ extern "C" int ri_ssd_scan_cols(float* out, const float* xbc, int channels, int 
     const int cols = 16 * SSD_WAVES;
     const dim3 grid(seqs, heads, (vdim + cols - 1) / cols);
     RI_REQUIRE(grid.z <= 65535, "ssd_scan_cols: heads of %d channels", vdim);
-#define RI_GO(TA, RPL, SL)                                                                                              \
-    ssd_scan_cols_kernel<TA, RPL, SL><<<grid, 64 * SSD_WAVES, 0, s>>>(out, xbc, channels, b_off, c_off, (const TA*)proj, stride, z_off,  \
+#define RI_GO(TA, RPL)                                                                                                  \
+    ssd_scan_cols_kernel<TA, RPL><<<grid, 64 * SSD_WAVES, 0, s>>>(out, xbc, channels, b_off, c_off, (const TA*)proj, stride, z_off,  \
                                                       dt_off, dt_bias, a_log, d_skip, state, cu_seqlens, slots, heads,   \
                                                       groups, n, vdim)
 #define RI_BY_ROWS(TA)                                                                                                  \
-    if (n <= 16) RI_GO(TA, 4, 4); else if (n <= 32) RI_GO(TA, 8, 4); else RI_GO(TA, 16, 4)
+    if (n <= 16) RI_GO(TA, 4); else if (n <= 32) RI_GO(TA, 8); else RI_GO(TA, 16)
     if (act_dtype == RI_F32) { RI_BY_ROWS(float); } else { RI_BY_ROWS(bf16_t); }
 #undef RI_BY_ROWS
 #undef RI_GO

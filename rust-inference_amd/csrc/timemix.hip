@@ -200,14 +200,14 @@ extern "C" int ri_timemix_scan(void* out, int out_stride, int out_off, float out
 #define TM_BLOCK 8
 #define TM_WAVES 4           // wavefronts of a workgroup: they share the staged tokens, each on columns of its own
 
-template <typename TA, int RPL, int SL>                       // RPL: rows a lane holds, a multiple of 4; SL: slices of rows, 4
+template <typename TA, int RPL>                               // RPL: rows a lane holds, a multiple of 4
 __global__ void __launch_bounds__(64 * TM_WAVES)
 timemix_scan_cols_kernel(float* __restrict__ out, const TA* __restrict__ r, const TA* __restrict__ k, const TA* __restrict__ v,
                          const float* __restrict__ z, const float* __restrict__ u,
                          float* __restrict__ state, const int32_t* __restrict__ cu_seqlens, const int32_t* __restrict__ slots,
                          int heads, int dim) {
-    // COLS: columns of a wavefront; NC: of the workgroup; TPP: tokens whose v one pass of the workgroup's threads fetches
-    constexpr int ROWS = SL * RPL, COLS = 64 / SL, NC = COLS * TM_WAVES, THREADS = 64 * TM_WAVES, TPP = THREADS / NC,
+    // SL: slices of rows; COLS: columns of a wavefront; NC: of the workgroup; TPP: tokens whose v one pass of the workgroup's threads fetches
+    constexpr int SL = 4, ROWS = SL * RPL, COLS = 64 / SL, NC = COLS * TM_WAVES, THREADS = 64 * TM_WAVES, TPP = THREADS / NC,
                   PASSES = TM_BLOCK / TPP;
     __shared__ __attribute__((aligned(16))) float rs[2][TM_BLOCK][ROWS];
     __shared__ __attribute__((aligned(16))) float ks[2][TM_BLOCK][ROWS];
@@ -433,15 +433,15 @@ extern "C" int ri_timemix_scan_cols(void* out, int out_stride, int out_off, floa
     const long total = (long)tokens * heads * dim;
     RI_REQUIRE((total + 255) / 256 <= 2147483647L, "timemix_scan_cols: %ld decays exceed one launch", total);
     timemix_decay_kernel<<<(unsigned)((total + 255) / 256), 256, 0, s>>>(z, w0, total, heads * dim);
-#define RI_GO(TA, ROWS, SL)                                                                                             \
-    timemix_scan_cols_kernel<TA, ROWS, SL><<<grid, 64 * TM_WAVES, 0, s>>>(o, (const TA*)r, (const TA*)k, (const TA*)v, z, u, state,  \
+#define RI_GO(TA, ROWS)                                                                                                 \
+    timemix_scan_cols_kernel<TA, ROWS><<<grid, 64 * TM_WAVES, 0, s>>>(o, (const TA*)r, (const TA*)k, (const TA*)v, z, u, state,  \
                                                            cu_seqlens, slots, heads, dim)
 #define RI_WALK(TA, CPL, VEC)                                                                                           \
     timemix_walk_kernel<TA, CPL, VEC><<<grid, 256, 0, s>>>(o, (const TA*)r, (const TA*)k, (const TA*)v, z, u, state, cu_seqlens, \
                                                            slots, heads, dim)
 #define RI_BY_COLUMNS(TA, VEC) if (cpl == 1) RI_WALK(TA, 1, VEC); else if (cpl == 2) RI_WALK(TA, 2, VEC); else RI_WALK(TA, 4, VEC)
 #define RI_BY_ROWS(TA)                                                                                                  \
-    if (dim <= 16) RI_GO(TA, 4, 4); else if (dim <= 32) RI_GO(TA, 8, 4); else if (dim <= 64) RI_GO(TA, 16, 4);             \
+    if (dim <= 16) RI_GO(TA, 4); else if (dim <= 32) RI_GO(TA, 8); else if (dim <= 64) RI_GO(TA, 16);             \
     else if (vec) { RI_BY_COLUMNS(TA, true); } else { RI_BY_COLUMNS(TA, false); }
     if (act_dtype == RI_F32) {
         RI_BY_ROWS(float)

@@ -7,6 +7,10 @@
 // meet for eight tokens at once, two sums in one exchange and the rest by lane shifts that ride in the additions.  A block's
 // missing tokens are staged so that they change nothing: no branch stands between the tokens.
 // The order of every sum is fixed by the lanes' places, not by CPL: CPL is chosen by how many columns a launch has.
+// States of up to 64 rows keep the forms of their own in ssd.hip, timemix.hip and gla.hip: half of the lanes here would hold no row.  Their
+// single tokens and steps that fill the machine are faster so, their few long prompts would not be (32 heads of 64 x 64, us own form : this
+// one, state-space / time mixing / gated linear attention: 32 single tokens 11 : 17, 17 : 22, 36 : 20; 32 prompts of 256 194 : 257, 361 : 350,
+// 486 : 271; one of 2,048 911 : 241, 863 : 229, 455 : 231).
 #pragma once
 #include "common.h"
 
