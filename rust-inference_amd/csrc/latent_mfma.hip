@@ -133,11 +133,11 @@ latent_attention_mfma_kernel(bf16_t* __restrict__ out, const bf16_t* __restrict_
 
 // Prompts: a workgroup of eight wavefronts takes eight (token, tile of 16 heads) pairs of neighbouring tokens (of one sequence, where
 // cu_seqlens says which are), which walk the same pages, and brings every page into LDS once for all of them.  What bounds the kernel above on a prompt is the caches: every wavefront
-// fetches every page for itself, 69 KB for 68 MFMAs.  Here a page crosses once for eight wavefronts, and what is left is
-// reading the fragments from LDS, two cycles of it for every one of the matrix cores.  A page's key and value halves take turns: while
-// the scores are made from the keys the values are on their way into registers, and the other way round, so that two barriers a
-// page are all that is waited for.  Pieces of 16 bytes are exchanged by the row's number so that a fragment's sixteen rows meet every
-// bank equally.  A token's sums are the other kernel's.  2,048 tokens, 32 heads, keys of 576: 1,400 us with a page a wavefront, 616.
+// fetches every page for itself, 69 KB for 68 MFMAs.  Here a page crosses once for eight wavefronts, and what is left is the wait for
+// the next half page and for the two barriers a page (83% of the wavefronts' cycles; LDS is busy a fifth of the time, the matrix cores a
+// ninth).  A page's key and value halves take turns: while the scores are made from the keys the values are on their way into registers,
+// and the other way round.  Pieces of 16 bytes are exchanged by the row's number so that a fragment's sixteen rows meet every
+// bank equally.  A token's sums are the other kernel's.  2,048 tokens, 32 heads, keys of 576: 1,400 us with a page a wavefront, 525.
 #define LP_WAVES 8
 template <int KS, int VT>
 __global__ void __launch_bounds__(64 * LP_WAVES)

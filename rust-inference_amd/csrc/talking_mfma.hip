@@ -12,13 +12,14 @@
 // The key rows of a half page are permuted (row r of the first half is key 8 (r / 4) + r % 4, of the second that plus
 // 4), so that a lane's eight scores are eight neighbouring keys, which is how the value product wants its weights.
 // Scores, the logarithm, maxima, sums, the weights before and after the mix and the accumulators are float32.  A token's
-// sums run over its sequence's pages in order, whatever else the step holds, or over equal parts of them that are added.
+// sums run over its sequence's pages in order, or over equal parts of them that are added: into how many depends on the step's tiles
+// and its longest sequence, so that in bfloat16 the rest of a step may move a token's result by the rounding of its float32 sums.
 //
 // The distance bias of a windowed head is a number a distance: a table of window + 16 entries a head is made first, by the
 // same logarithm, and both walks read eight neighbouring entries of it for their eight keys (a logarithm a score was half
 // of what the walks took).  The second walk of a step with fewer tiles than compute units cuts every tile's pages into
 // shares, whose float32 results are added.  2,048 tokens, 32 heads of 128 over 8, a window of 1,024, us: first walk 283 ->
-// 133, second 950 -> 395 with the adding.
+// 136, second 950 -> 394 with the adding; it waits for loads and the two barriers a page for two thirds of its time.
 #include "api.h"
 #include "common.h"
 

@@ -47,7 +47,10 @@ WIDE_GATED_BYTES = 64_000_000    # pairs larger than this (smaller ones, up to 3
 # 17 to 48 rows against a plain matrix of many rows (all experts' gates and ups side by side: 4 row tiles a compute unit and
 # more): the wide kernel, K whole.  98,304 x 4,096 at 17 / 32 / 48 / 64 rows: 136 / 143 / 163 / 183 us against the library's 180 / 180 / 172 / 177;
 # 24,576 x 1,024: 13 / 15 / 17 / 20 against 32 / 32 / 18 / 18; 24,576 x 4,096 37 / 41 / 49 / 58 against 52 / 51 / 51 / 51; with fewer row
-# tiles level (12,288 x 4,096 at 32 rows 23 against 24).
+# tiles level (12,288 x 4,096 at 32 rows 23 against 24).  Weights not in the caches, at 17 / 32 / 48 rows, the wide kernel : the library: 16,384 x 1,024
+# 8.9 / 9.6 / 10.6 : 12.9 / 12.8 / 13.3, x 5,120 30 / 32 / 36 : 35 / 35 / 37; 32,768 x 4,096 50 / 53 / 55 : 66 / 66 / 67; 49,152 x 2,048 37 / 40 / 45 : 50 / 49 / 49;
+# 151,936 x 2,048 108 / 120 / 139 : 151 / 153 / 150.  At 48 rows some sizes are the library's: 20,480 x 4,096 33 / 37 / 43 : 41 / 40 / 41, 24,576 x 2,560
+# 25 / 28 / 32 : 28 / 27 / 29, 65,536 x 768 22 / 26 / 29 : 25 / 25 / 26 (no rule of tiles and K tells them from the others).
 WIDE_PLAIN_TILES = 4
 WIDE_PLAIN_ROWS = 48
 SPLIT_K = 4096                   # pieces of a long K (PACKED_LONG_K and more) whose sums the next norm adds
