@@ -349,6 +349,162 @@ attention_rows_kernel(T* __restrict__ out, const T* __restrict__ q, int q_stride
     }
 }
 
+// float32 heads of 64 and 128 run on the matrix cores' float32 products (16x16x4): every product and sum is a 32-bit one, the dot
+// product of a query and a key in two chains of head_dim / 2 (by blocks of sixteen channels), added at the end.  A workgroup takes
+// sixteen rows of queries (neighbouring tokens of one sequence times the query heads of one kv head); its four wavefronts take
+// the tiles of sixteen keys in turn, tile t the wavefront t % 4, each with its own running maximum, sum and weighted values, joined
+// in the wavefronts' order at the end: a row's result depends on its own position and the keys alone, never on the rows
+// beside it.  The scores are computed with the keys as rows and the queries as columns: lane (g, r) then holds keys 4 g ..+4 of query r,
+// which is what the second product reads from it as its operand, and both products read keys and values 16 bytes a lane
+// straight from their pages, whole 64-byte pieces of a row: nothing passes through LDS but the join.
+// What bounds it: the products, 2,048 cycles a tile of keys, and for short prompts the depth of the longest walk.  759 tokens of
+// three prompts (of 33 to 400), 16 heads over 8 of 128: 31 us a layer, by rows on the vector units 91; one prompt of 2,000 248 : 906,
+// 12 of 200 68 : 201, 64 single tokens at 500 keys 47 : 74, one at 2,000 60 : 105, one at 50 13 : 13 (heads of 64 alike).
+// Error against 64 bits over a whole model's logits 1.0e-6 : 1.1e-6.
+#define ATT_M_WAVES 4
+typedef __attribute__((__vector_size__(4 * sizeof(float)))) float att_floatx4;
+
+template <int D>
+__global__ void __launch_bounds__(64 * ATT_M_WAVES)
+attention_f32_matrix_kernel(float* __restrict__ out, const float* __restrict__ q, int q_stride, const float* __restrict__ k_pages,
+                            const float* __restrict__ v_pages, const int32_t* __restrict__ tok_pos,
+                            const int32_t* __restrict__ tok_seq, const int32_t* __restrict__ page_table, int table_width, int tokens,
+                            int per, int heads, int kv_heads, int page_size, Reach reach, float scale, float softcap,
+                            const float* __restrict__ slopes, int keep_first, const float* __restrict__ sinks,
+                            const int32_t* __restrict__ cu_seqlens, int seqs) {
+    constexpr int BLOCKS = D / 16, PITCH = D + 4;
+    __shared__ float sums[ATT_M_WAVES][ATT_ROWS][PITCH];
+    __shared__ float tops[ATT_M_WAVES][ATT_ROWS], totals[ATT_M_WAVES][ATT_ROWS];
+    const int tid = threadIdx.x, lane = tid & (RI_WAVE - 1), r = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / RI_WAVE);
+    // the longest walks first, a run's key heads side by side (as in the kernel above)
+    const int place = blockIdx.x + gridDim.x * blockIdx.y, at_run = gridDim.x - 1 - place / kv_heads;
+    const int kvh = place % kv_heads, group = heads / kv_heads, h0 = kvh * group;
+    int begin = at_run * per, end = min(begin + per, tokens);
+    if (cu_seqlens) {
+        Run run;
+        if (!run_of(at_run, cu_seqlens, seqs, 1, per, 1, run)) return;
+        begin = run.start + run.first;
+        end = begin + run.count;
+    }
+    // the tokens of one sequence at a time, as far as their positions follow one another
+    for (int t0 = begin, t1; t0 < end; t0 = t1) {
+        const int seq = tok_seq[t0], p0 = tok_pos[t0];
+        // (a lane a token: one after the other each would be a trip to memory)
+        const int ahead = min(t0 + 1 + lane, tokens - 1);
+        const bool follows = t0 + 1 + lane < end && tok_seq[ahead] == seq && tok_pos[ahead] == p0 + 1 + lane;
+        t1 = t0 + 1 + __builtin_ctzll(~__ballot(follows));   // (a run is shorter than a wavefront)
+        const int rows = (t1 - t0) * group, last_pos = p0 + (t1 - 1 - t0);       // row r: token t0 + r / group, head h0 + r % group
+        const int32_t* table = page_table + (size_t)seq * table_width;
+        const int mine = min(r, rows - 1), qpos = p0 + mine / group, head = h0 + mine % group;   // (rows past the last are it again)
+        const int lo = reach.first(qpos), kept = min(keep_first, lo);
+        const float slope = slopes ? slopes[head] : 0.f;
+        att_floatx4 qf[BLOCKS], acc[BLOCKS];
+        const float* qp = q + (size_t)(t0 + mine / group) * q_stride + (size_t)head * D + 4 * g;
+#pragma unroll
+        for (int b = 0; b < BLOCKS; ++b) {
+            qf[b] = att_floatx4{qp[16 * b], qp[16 * b + 1], qp[16 * b + 2], qp[16 * b + 3]};
+            acc[b] = att_floatx4{0.f, 0.f, 0.f, 0.f};
+        }
+        float m = -INFINITY, l = 0.f;                       // l: of this lane's keys
+        // the tiles that any row sees: those of the kept keys, and from the first token's first key on
+        const int first_tile = reach.first(p0) / 16, kept_tiles = (min(keep_first, reach.first(last_pos)) + 15) / 16;
+        const auto seen_from = [&](int tile) {              // this wavefront's first such tile from `tile` on
+            return tile >= kept_tiles && tile < first_tile ? tile + (first_tile - tile + ATT_M_WAVES - 1) / ATT_M_WAVES * ATT_M_WAVES : tile;
+        };
+        const auto page_of = [&](int tile) { return ((long)table[tile * 16 / page_size] * kv_heads + kvh) * page_size * D; };
+        const auto fetch_keys = [&](att_floatx4 (&kf)[BLOCKS], long page, int tile) {
+            const float* kp = k_pages + page + (long)(tile * 16 % page_size + r) * D + 4 * g;
+#pragma unroll
+            for (int b = 0; b < BLOCKS; ++b) kf[b] = *reinterpret_cast<const att_floatx4*>(kp + 16 * b);
+        };
+        const int last_tile = last_pos / 16;
+        att_floatx4 kf[BLOCKS], vf[BLOCKS];
+        long page = 0;
+        int tile = seen_from(wave);
+        if (tile <= last_tile) fetch_keys(kf, page = page_of(tile), tile);
+        // a tile's values are asked for before its scores are computed, the next tile's keys before the values are used
+        for (int next; tile <= last_tile; tile = next) {
+            const int base = tile * 16;
+            next = seen_from(tile + ATT_M_WAVES);
+            const long next_page = page_of(min(next, last_tile));
+            const float* vp = v_pages + page + (long)r * page_size + base % page_size + 4 * g;
+#pragma unroll
+            for (int b = 0; b < BLOCKS; ++b) vf[b] = *reinterpret_cast<const att_floatx4*>(vp + (long)(16 * b) * page_size);
+            __builtin_amdgcn_sched_barrier(0);
+            att_floatx4 dot[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+            for (int b = 0; b < BLOCKS; b += 2)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    dot[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[b][i], qf[b][i], dot[0], 0, 0, 0);
+                    dot[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[b + 1][i], qf[b + 1][i], dot[1], 0, 0, 0);
+                }
+            __builtin_amdgcn_sched_barrier(0);
+            fetch_keys(kf, page = next_page, min(next, last_tile));
+            __builtin_amdgcn_sched_barrier(0);
+            float s[4], top = -INFINITY;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int j = base + 4 * g + i;
+                s[i] = (dot[0][i] + dot[1][i]) * scale;
+                if (softcap > 0.f) s[i] = softcap * tanhf(s[i] / softcap);
+                if (slopes) s[i] -= slope * (float)(qpos - j);
+                if (!((j >= lo || j < kept) && j <= qpos)) s[i] = -INFINITY;
+                top = fmaxf(top, s[i]);
+            }
+            top = fmaxf(top, __shfl_xor(top, 16, RI_WAVE));
+            top = fmaxf(top, __shfl_xor(top, 32, RI_WAVE));
+            const float m_new = fmaxf(m, top), ref = m_new > -INFINITY ? m_new : 0.f;   // (nothing seen yet: any number will do)
+            const float corr = expf(m - ref);
+            float p[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) p[i] = expf(s[i] - ref);
+            l = l * corr + ((p[0] + p[1]) + (p[2] + p[3]));
+            m = m_new;
+            if (base + 15 > last_pos) {                     // keys that no row has yet: whatever their places hold does not count
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int b = 0; b < BLOCKS; ++b) vf[b][i] = base + 4 * g + i <= last_pos ? vf[b][i] : 0.f;
+            }
+#pragma unroll
+            for (int b = 0; b < BLOCKS; ++b) acc[b] *= corr;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int b = 0; b < BLOCKS; ++b) acc[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[b][i], p[i], acc[b], 0, 0, 0);
+        }
+        l += __shfl_xor(l, 16, RI_WAVE);
+        l += __shfl_xor(l, 32, RI_WAVE);
+        __syncthreads();                                    // the last run's sums have been read
+#pragma unroll
+        for (int b = 0; b < BLOCKS; ++b) *reinterpret_cast<att_floatx4*>(&sums[wave][r][16 * b + 4 * g]) = acc[b];
+        if (g == 0) { tops[wave][r] = m; totals[wave][r] = l; }
+        __syncthreads();
+        const int row = tid / 16, h = h0 + row % group;
+        if (row >= rows) continue;
+        float all = tops[0][row], total = 0.f, part[ATT_M_WAVES];
+#pragma unroll
+        for (int w = 1; w < ATT_M_WAVES; ++w) all = fmaxf(all, tops[w][row]);
+#pragma unroll
+        for (int w = 0; w < ATT_M_WAVES; ++w) {
+            part[w] = tops[w][row] > -INFINITY ? expf(tops[w][row] - all) : 0.f;
+            total += totals[w][row] * part[w];
+        }
+        if (sinks) total += expf(sinks[h] - all);           // the sink: a term of the denominator alone
+        float* o = out + ((size_t)(t0 + row / group) * heads + h) * D;
+#pragma unroll
+        for (int c = 4 * (tid % 16); c < D; c += 64) {
+            att_floatx4 sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int w = 0; w < ATT_M_WAVES; ++w) sum += *reinterpret_cast<const att_floatx4*>(&sums[w][row][c]) * part[w];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) o[c + i] = sum[i] / total;
+        }
+    }
+}
+
 template <typename T, bool VEC>
 static void launch_attention(void* out, const void* q, int q_stride, const void* k_pages, const void* v_pages,
                              const int32_t* tok_pos, const int32_t* tok_seq, const int32_t* page_table,
@@ -377,7 +533,13 @@ static bool attention_rows_fit(int heads, int kv_heads, int head_dim, int v_dim,
     return heads / kv_heads <= ATT_ROWS && head_dim % (16 / element) == 0 && head_dim <= 256 && v_dim <= ATT_TILE && page_size % 8 == 0;
 }
 
-// Which of the two forms a step runs (their results are the same bits): with cu_seqlens, the sequences of rows_from and more new
+// Whether a step's sizes run on the matrix cores: a rule on types and sizes alone, so that a sequence's tokens have the same bits
+// however they are cut into steps.
+static bool attention_matrix_fits(int dtype, int heads, int kv_heads, int head_dim, int v_dim, int page_size) {
+    return dtype == RI_F32 && heads / kv_heads <= ATT_ROWS && (head_dim == 64 || head_dim == 128) && v_dim == head_dim && page_size % 16 == 0;
+}
+
+// Which of the two other forms a step runs (their results are the same bits): with cu_seqlens, the sequences of rows_from and more new
 // tokens by rows, `runs` runs of 16 / (heads / kv_heads) tokens in all and rows_tokens tokens, and the rest a workgroup a
 // (token, head), in a launch that the others' workgroups leave at once; without, all by rows where a sequence brings four
 // tokens and more (most_new) and the (token, head) pairs are past one round of resident workgroups, eight a compute unit.
@@ -412,6 +574,20 @@ extern "C" int ri_attention_kept(void* out, const void* q, int act_dtype, int q_
                          (cu_seqlens ? runs > 0 : most_new >= 4 && (long)tokens * heads > 8L * ri_compute_units());
     RI_REQUIRE(!cu_seqlens || (seqs > 0 && rows_from > 0 && rows_tokens >= 0 && rows_tokens <= tokens && (runs > 0) == (rows_tokens > 0)),
                "attention: %d runs of %d tokens of %d sequences", runs, rows_tokens, seqs);
+    if (vec && attention_matrix_fits(act_dtype, heads, kv_heads, head_dim, v_dim, page_size)) {
+        // runs of neighbours of one sequence where all of them are known, else tokens as they lie, one by one where no sequence
+        // is said to bring several
+        const bool known = cu_seqlens && runs > 0 && rows_from == 1 && rows_tokens == tokens;
+        const int per = known || cu_seqlens || most_new >= 4 ? ATT_ROWS / (heads / kv_heads) : 1;
+        const dim3 matrix_grid(known ? runs : (tokens + per - 1) / per, kv_heads);
+#define RI_ATT_MATRIX(D) attention_f32_matrix_kernel<D><<<matrix_grid, 64 * ATT_M_WAVES, 0, s>>>( \
+            (float*)out, (const float*)q, q_stride, (const float*)k_pages, (const float*)v_pages, tok_pos, tok_seq, page_table, table_width, tokens, \
+            per, heads, kv_heads, page_size, reach, scale, softcap, slopes, window > 0 ? keep_first : 0, sinks, known ? cu_seqlens : nullptr, seqs)
+        if (head_dim == 64) RI_ATT_MATRIX(64); else RI_ATT_MATRIX(128);
+#undef RI_ATT_MATRIX
+        RI_LAUNCH_CHECK("attention");
+        return 0;
+    }
     if (by_rows) {
 #define RI_ATT_ROWS(T, S) launch_rows<T, S>(out, q, q_stride, k_pages, v_pages, tok_pos, tok_seq, page_table, table_width, tokens, heads, \
                                             kv_heads, head_dim, v_dim, page_size, reach, scale, softcap, slopes, \

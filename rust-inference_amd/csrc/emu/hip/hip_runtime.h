@@ -241,3 +241,17 @@ static inline V4 emu_mfma_16x16x32_bf16(V8 a, V8 b, V4 c) {
     return d;
 }
 #define __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, x, y, z) emu_mfma_16x16x32_bf16((a), (b), (c))
+
+// MFMA 16x16x4 float32: D[16 x 16] = A[16 x 4] . B[4 x 16] + C.  Lane l holds A[l % 16][l / 16], B[l / 16][l % 16] and
+// D[4 * (l / 16) + i][l % 16] for i = 0..3.
+template <class V4>
+static inline V4 emu_mfma_16x16x4_f32(float a, float b, V4 c) {
+    float mine[2] = {a, b}, all[64][2];
+    emu::wave_gather(mine, sizeof(mine), all);
+    const int lane = emu::self->lane, col = lane & 15, rows = 4 * (lane >> 4);
+    V4 d = c;
+    for (int i = 0; i < 4; ++i)
+        for (int k = 0; k < 4; ++k) d[i] = fmaf(all[rows + i + 16 * k][0], all[col + 16 * k][1], d[i]);
+    return d;
+}
+#define __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, x, y, z) emu_mfma_16x16x4_f32((a), (b), (c))

@@ -562,6 +562,13 @@ def attention_rows_plan(new_counts, starts, heads: int, kv_heads: int, row_bytes
     return rows_from, tokens, runs
 
 
+def attention_runs_on_matrix_cores(dtype, heads: int, kv_heads: int, head_dim: int, v_dim: int, page_size: int) -> bool:
+    """Whether the general attention takes these sizes with the float32 matrix products (``attention_matrix_fits`` of
+    attention_generic.hip): all of a step's sequences then come as runs of neighbours."""
+    return (dtype == torch.float32 and heads // kv_heads <= ATTENTION_ROWS and head_dim in (64, 128) and v_dim == head_dim
+            and page_size % 16 == 0)
+
+
 def attention(qkv, k_pages, v_pages, tok_pos, tok_seq, page_table, heads: int, kv_heads: int, head_dim: int,
               window: int | None, scale: float, softcap: float | None = None, slopes: torch.Tensor | None = None,
               keep_first: int = 0, sinks: torch.Tensor | None = None, q_off: int = 0, chunk: int | None = None,
@@ -589,7 +596,11 @@ def attention(qkv, k_pages, v_pages, tok_pos, tok_seq, page_table, heads: int, k
         seqs = len(new_counts)
         if sum(new_counts) != tokens or len(starts) != seqs:
             raise ShapeError(f"attention: {tokens} tokens of {seqs} sequences that bring {sum(new_counts)}, {len(starts)} of them cached")
-        plan = attention_rows_plan(new_counts, starts, heads, kv_heads, head_dim * qkv.element_size(), window or chunk)
+        if attention_runs_on_matrix_cores(qkv.dtype, heads, kv_heads, head_dim, v_dim, k_pages.shape[2]):
+            per = ATTENTION_ROWS // (heads // kv_heads)
+            plan = 1, tokens, sum(-(-n // per) for n in new_counts)
+        else:
+            plan = attention_rows_plan(new_counts, starts, heads, kv_heads, head_dim * qkv.element_size(), window or chunk)
     _call("ri_attention_kept", _dev(out, "out"), _dev(qkv, "qkv") + int(q_off) * qkv.element_size(), code(qkv.dtype), stride, _dev(k_pages, "k_pages"),
           _dev(v_pages, "v_pages"), code(k_pages.dtype), _dev(tok_pos, "tok_pos", torch.int32, (tokens,)),
           _dev(tok_seq, "tok_seq", torch.int32, (tokens,)), _dev(page_table, "page_table", torch.int32),

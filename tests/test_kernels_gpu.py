@@ -411,6 +411,55 @@ def test_attention_rows_of_queries_beside_single_tokens(ops, heads, kv_heads, dh
     assert torch.isfinite(want).all() and torch.equal(got, want)
 
 
+@pytest.mark.parametrize("heads, kv_heads, dh, form", [(4, 2, 64, dict(softcap=15.0)), (3, 1, 128, dict(window=20, keep_first=5)),
+                                                       (16, 1, 64, dict(chunk=24)), (2, 2, 128, dict())])
+def test_attention_float32_on_the_matrix_cores(ops, heads, kv_heads, dh, form):
+    """Tiles of sixteen keys and sixteen rows and their remainders, every mask, with sinks and slopes, against 64 bits; whatever lies
+    behind a sequence's last key does not count; the same bits in runs, as tokens lie and one by one, and in pieces."""
+    before, new = [0, 0, 0, 15, 16, 63, 40, 0], [1, 15, 33, 1, 17, 2, 30, 16]
+    rng = np.random.default_rng(dh + heads)
+    k, v, kp, vp, table = paged(rng, [a + n for a, n in zip(before, new)], kv_heads, dh)
+    for b, (a, n) in enumerate(zip(before, new)):
+        if (a + n) % 32:
+            page = table[b, (a + n) // 32].item()
+            kp[page, :, (a + n) % 32:], vp[page, :, :, (a + n) % 32:] = float("nan"), float("nan")
+    q = rng.normal(size=(sum(new), heads * dh)).astype(np.float32)
+    slopes, sinks = (rng.uniform(0.01, 0.1, heads).astype(np.float32), rng.normal(size=heads).astype(np.float32))
+    window, chunk, keep, cap = (form.get(n) for n in ("window", "chunk", "keep_first", "softcap"))
+    more = dict(softcap=cap, slopes=t(slopes), keep_first=keep or 0, sinks=t(sinks), chunk=chunk)
+
+    def run(pieces, **how):
+        """Every sequence's new tokens from its piece of them on."""
+        rows = [sum(new[:b]) + i for b, (lo, hi) in enumerate(pieces) for i in range(lo, hi)]
+        pos = t([before[b] + i for b, (lo, hi) in enumerate(pieces) for i in range(lo, hi)], torch.int32)
+        seq = t([b for b, (lo, hi) in enumerate(pieces) for _ in range(lo, hi)], torch.int32)
+        if how.pop("runs", False):
+            n = [hi - lo for lo, hi in pieces]
+            how = dict(new_counts=n, starts=[a + lo for a, (lo, hi) in zip(before, pieces)], cu_seqlens=t(np.concatenate([[0], np.cumsum(n)]), torch.int32))
+        return rows, f64(ops.attention(t(q[rows]), kp, vp, pos, seq, table, heads, kv_heads, dh, window, dh ** -0.5, **how, **more))
+
+    whole = [(0, n) for n in new]
+    got = run(whole, runs=True)[1]
+    assert np.array_equal(got, run(whole)[1]) and np.array_equal(got, run(whole, most_new=max(new))[1])
+    for pieces in ([(0, n // 2) for n in new], [(n // 2, n) for n in new]):
+        rows, part = run(pieces, runs=True)
+        assert np.array_equal(part, got[rows])
+    row = 0
+    for b, (a, n) in enumerate(zip(before, new)):
+        kb = np.stack([f64(kp[table[b, j // 32].item(), :, j % 32]) for j in range(a + n)])
+        vb = np.stack([f64(vp[table[b, j // 32].item(), :, :, j % 32]) for j in range(a + n)])
+        for i in range(n):
+            at, j = a + i, np.arange(a + i + 1)
+            lo = at - at % chunk if chunk else max(0, at - window + 1) if window else 0
+            for h in range(heads):
+                s = kb[:at + 1, h * kv_heads // heads] @ q[row, h * dh:(h + 1) * dh].astype(np.float64) * dh ** -0.5
+                s = (cap * np.tanh(s / cap) if cap else s) - slopes[h].astype(np.float64) * (at - j)
+                p = np.where((j >= lo) | (j < (keep or 0)), np.exp(s), 0.0)
+                want = p @ vb[:at + 1, h * kv_heads // heads] / (p.sum() + np.exp(np.float64(sinks[h])))
+                close(t(got[row, h * dh:(h + 1) * dh]), want, 3e-6, f"sequence {b}, token {i}, head {h}")
+            row += 1
+
+
 def test_attention_shares_loads_where_that_is_less_to_wait_for(ops, monkeypatch):
     """Prompts enough to fill the machine do; one of 130 tokens, many of four and steps of single tokens do not, nor do single tokens
     that stand beside a prompt."""
