@@ -1,5 +1,5 @@
 // What the kernels that make queries, keys and values ready for the cache share: eight neighbours at once, and a
-// prompt's values into their pages a page at a time.
+// prompt's values into their pages, eight positions or a page at a time.
 #pragma once
 #include "common.h"
 
@@ -30,9 +30,74 @@ template <> struct Eight<bf16_t> {
     }
 };
 
-// Values into their pages, a page at a time: one workgroup per (32 positions touched by this step, sequence, kv
-// head) reads the new tokens' value heads as rows, turns them through LDS and writes channel rows.
+// Values into their pages, turned in registers: a thread takes 16 bytes of channels of eight neighbouring positions (those that
+// start at a multiple of eight), eight loads all asked for together, and writes channel rows of eight positions, 16 bytes each
+// (two in float32); neighbouring threads take the four such groups of 32 positions, so that a store covers whole lines.  What bounded
+// the form through LDS below is the wait for its loads, a barrier and its few workgroups at work (three prompts of 500 to 1,500 tokens,
+// 8 heads of 128, bfloat16: 13.8 us, 9.1 so).  A workgroup of 256 threads is number `part` of the values_turn_parts of one sequence's
+// `piece`-th 32 positions that this step may touch.
 #define QT_TOKENS 32
+template <typename T>
+static inline int values_turn_parts(int kv_heads, int vdim) { return (kv_heads * (vdim / (16 / (int)sizeof(T))) * 4 + 255) / 256; }
+static inline int values_turn_pieces(int max_new) { return (max_new + QT_TOKENS - 2) / QT_TOKENS + 1; }
+
+template <typename T>
+__device__ __forceinline__ void values_turn(const T* __restrict__ rows, size_t row_len, size_t v_off, const int32_t* __restrict__ cu_seqlens,
+                                            const int32_t* __restrict__ tok_pos, const int32_t* __restrict__ page_table, int table_width,
+                                            T* __restrict__ v_pages, int kv_heads, int vdim, int page_size,
+                                            const float* __restrict__ bias, int piece, int seq, int part) {
+    constexpr int E = 16 / (int)sizeof(T);                   // channels a thread takes
+    const int t_begin = cu_seqlens[seq], n = cu_seqlens[seq + 1] - t_begin;
+    if (n <= 0) return;
+    const int start = tok_pos[t_begin];                      // the sequence's new tokens sit at start .. start + n - 1
+    const int item = part * 256 + threadIdx.x, of_head = vdim / E, rest = item >> 2, kvh = rest / of_head, d = rest % of_head * E;
+    const int first = (start / QT_TOKENS + piece) * QT_TOKENS + (item & 3) * 8;
+    if (kvh >= kv_heads || first + 7 < start || first >= start + n) return;
+    const T* from = rows + v_off + (size_t)kvh * vdim + d;
+    uint4 in[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j)                              // (positions that are not the step's: read as its first or last, not written)
+        in[j] = *reinterpret_cast<const uint4*>(from + (size_t)(t_begin + min(max(first + j - start, 0), n - 1)) * row_len);
+    const bool whole = first >= start && first + 8 <= start + n;
+    const int page = page_table[(size_t)seq * table_width + first / page_size];
+    T* to = v_pages + (((size_t)page * kv_heads + kvh) * vdim + d) * page_size + first % page_size;
+#pragma unroll
+    for (int c = 0; c < E; ++c, to += page_size) {
+        T y[8];
+        const float b = bias ? bias[(size_t)kvh * vdim + d + c] : 0.f;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const uint32_t w[4] = {in[j].x, in[j].y, in[j].z, in[j].w};
+            if constexpr (sizeof(T) == 4) y[j] = __uint_as_float(w[c]) + (bias ? b : 0.f);
+            else {
+                y[j] = (T)(w[c / 2] >> (c & 1) * 16);
+                if (bias) from_f32(&y[j], to_f32(y[j]) + b);
+            }
+        }
+        if (whole) {
+            if constexpr (sizeof(T) == 4) Eight<T>::store(to, y);
+            else
+                *reinterpret_cast<uint4*>(to) = make_uint4(y[0] | (uint32_t)y[1] << 16, y[2] | (uint32_t)y[3] << 16, y[4] | (uint32_t)y[5] << 16,
+                                                           y[6] | (uint32_t)y[7] << 16);
+        } else {
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                if (first + j >= start && first + j < start + n) to[j] = y[j];
+        }
+    }
+}
+
+template <typename T>
+__global__ void __launch_bounds__(256)
+values_turn_kernel(const T* __restrict__ rows, size_t row_len, size_t v_off, const int32_t* __restrict__ cu_seqlens,
+                   const int32_t* __restrict__ tok_pos, const int32_t* __restrict__ page_table, int table_width,
+                   T* __restrict__ v_pages, int kv_heads, int vdim, int page_size, const float* __restrict__ bias) {
+    values_turn<T>(rows, row_len, v_off, cu_seqlens, tok_pos, page_table, table_width, v_pages, kv_heads, vdim, page_size, bias, blockIdx.x,
+                   blockIdx.y, blockIdx.z);
+}
+
+// Through LDS, where 16-byte pieces do not divide the value heads or their rows, a page at a time: one workgroup per (32 positions touched by this step, sequence, kv
+// head) reads the new tokens' value heads as rows, turns them through LDS and writes channel rows.
 template <typename TA, typename TC>
 __global__ void __launch_bounds__(256)
 values_to_pages_kernel(const TA* __restrict__ qkv, size_t row_len, size_t v_off, const int32_t* __restrict__ cu_seqlens,
@@ -83,4 +148,19 @@ values_to_pages_kernel(const TA* __restrict__ qkv, size_t row_len, size_t v_off,
             if (first + tt >= lo && first + tt <= hi) from_f32(base + (size_t)d * page_size + tt, tile[tt * stride + d] + (add ? add[d] : 0.f));
         }
     }
+}
+
+// A prompt's values into their pages (which hold a multiple of 32 positions).
+template <typename T>
+static void launch_values_to_pages(const T* rows, size_t row_len, size_t v_off, const int32_t* cu_seqlens, const int32_t* tok_pos,
+                                   const int32_t* page_table, int table_width, T* v_pages, int seqs, int max_new, int kv_heads, int vdim,
+                                   int page_size, const float* bias, hipStream_t s) {
+    constexpr int E = 16 / (int)sizeof(T);
+    const int parts = vdim % E == 0 ? values_turn_parts<T>(kv_heads, vdim) : 0;
+    if (parts > 0 && parts <= 65535 && row_len % E == 0 && v_off % E == 0 && ((uintptr_t)rows | (uintptr_t)v_pages) % 16 == 0)
+        values_turn_kernel<T><<<dim3(values_turn_pieces(max_new), seqs, parts), 256, 0, s>>>(
+            rows, row_len, v_off, cu_seqlens, tok_pos, page_table, table_width, v_pages, kv_heads, vdim, page_size, bias);
+    else
+        values_to_pages_kernel<T, T><<<dim3(values_turn_pieces(max_new), seqs, kv_heads), 256, QT_TOKENS * (vdim + 1) * sizeof(float), s>>>(
+            rows, row_len, v_off, cu_seqlens, tok_pos, page_table, table_width, v_pages, kv_heads, vdim, page_size, bias);
 }

@@ -82,7 +82,7 @@ qk_half_bias_kv_write_kernel(T* __restrict__ proj, size_t row_len, int q_off, in
 // A prompt whose halves and head sizes 16-byte pieces divide: a workgroup a token.  The token's sines and cosines are
 // made once, in LDS; with gains a head's norm meets over the lanes that hold its pieces, where they are a power of two (`lanes`),
 // and else in a pass of its own ahead (a wavefront a head, lanes 0); a thread takes a piece of eight from each half of a head (or one of the part that passes), every
-// load and store 16 bytes (32 for float32).  The values go a page at a time (values_to_pages_kernel).
+// load and store 16 bytes (32 for float32).  The values go eight positions at a time (launch_values_to_pages).
 template <typename T>
 __global__ void __launch_bounds__(512)
 qk_half_bias_k_write_vec_kernel(T* __restrict__ proj, size_t row_len, int q_off, int k_off, const float* __restrict__ q_bias,
@@ -209,9 +209,8 @@ static void launch_qk_half(T* proj, size_t row_len, int q_off, int k_off, int v_
             table_width, k_pages, v_pages, tokens, heads, kv_heads, dim, vdim, page_size, !paged_values);
     }
     if (paged_values) {
-        dim3 grid((max_new + QT_TOKENS - 2) / QT_TOKENS + 1, seqs, kv_heads);      // the 32-position pieces a sequence may touch
-        values_to_pages_kernel<T, T><<<grid, 256, QT_TOKENS * (vdim + 1) * sizeof(float), s>>>(
-            proj, row_len, (size_t)v_off, cu_seqlens, tok_pos, page_table, table_width, v_pages, kv_heads, vdim, page_size, v_bias);
+        launch_values_to_pages<T>(proj, row_len, (size_t)v_off, cu_seqlens, tok_pos, page_table, table_width, v_pages, seqs, max_new, kv_heads,
+                                  vdim, page_size, v_bias, s);
     }
 }
 

@@ -7,6 +7,7 @@
 // element is normed and rotated in float32 and rounded once.
 #include "api.h"
 #include "common.h"
+#include "kv_pages.h"
 
 #define QK_MAX_PAIRS 4   // pairs per lane: head_dim / 2 <= 64 * QK_MAX_PAIRS
 #define QK_MAX_TAIL 8    // elements per lane behind the rotated part: head_dim <= 64 * QK_MAX_TAIL
@@ -103,42 +104,23 @@ __global__ void qk_norm_rope_kv_write_kernel(
 // For head sizes whose half is 8 lanes' worth of eight elements or a power-of-two fraction of it
 // (head_dim 16, 32, 64, 128, 256, 512 ...): a lane takes eight consecutive pairs (d, d + half) of one
 // head, so head_dim / 16 lanes make a head and a wavefront works on 1024 / head_dim heads at once, every
-// load and store 16 bytes (32 for float32).  Values are not written here but by the page-wise kernel
-// below, which transposes whole pages through LDS instead of scattering single elements.
-template <typename T> struct Vec8;
-template <> struct Vec8<float> {
-    __device__ static void load(const float* p, float* o) {
-        const float4 a = *reinterpret_cast<const float4*>(p), b = *reinterpret_cast<const float4*>(p + 4);
-        o[0] = a.x; o[1] = a.y; o[2] = a.z; o[3] = a.w; o[4] = b.x; o[5] = b.y; o[6] = b.z; o[7] = b.w;
-    }
-    __device__ static void store(float* p, const float* v) {
-        *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
-        *reinterpret_cast<float4*>(p + 4) = make_float4(v[4], v[5], v[6], v[7]);
-    }
-};
-template <> struct Vec8<bf16_t> {
-    __device__ static void load(const bf16_t* p, float* o) {
-        const uint4 v = *reinterpret_cast<const uint4*>(p);
-        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            o[2 * i] = __uint_as_float(w[i] << 16);
-            o[2 * i + 1] = __uint_as_float(w[i] & 0xFFFF0000u);
-        }
-    }
-    __device__ static void store(bf16_t* p, const float* v) {
-        *reinterpret_cast<uint4*>(p) = make_uint4(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]),
-                                                  pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7]));
-    }
-};
-
+// load and store 16 bytes (32 for float32).  The workgroups past the tokens write the values (values_turn), so that neither
+// kind waits for the other.  16 prompts of 16 to 1,024 tokens, 16 heads over 8 of 128: 32 us, in two launches (the values through LDS)
+// 20.8 + 17.4; three prompts of 33 to 400 in float32 8.6 : 6.7 + 10.3.  Bound by memory: 125 MB, 3.9 TB/s.
 template <typename TA, typename TC>
 __global__ void __launch_bounds__(256)
 qk_norm_rope_k_write_vec_kernel(
     TA* __restrict__ qkv, const float* __restrict__ q_gain, const float* __restrict__ k_gain, float eps,
     const float* __restrict__ inv_freq, const int32_t* __restrict__ tok_pos, const int32_t* __restrict__ tok_seq,
     const int32_t* __restrict__ page_table, int table_width, TC* __restrict__ k_pages, int heads, int kv_heads,
-    int head_dim, int page_size) {
+    int head_dim, int page_size, int tokens, const int32_t* __restrict__ cu_seqlens, int pieces, int parts, TC* __restrict__ v_pages) {
+    if ((int)blockIdx.x >= tokens) {
+        const int at = blockIdx.x - tokens, of_seq = at / parts;
+        values_turn<TC>((const TC*)qkv, (size_t)(heads + 2 * kv_heads) * head_dim, (size_t)(heads + kv_heads) * head_dim, cu_seqlens, tok_pos,
+                        page_table, table_width, v_pages, kv_heads, head_dim, page_size, nullptr, of_seq % pieces, of_seq / pieces,
+                        at % parts);
+        return;
+    }
     extern __shared__ float cs_sn[];                         // cos[half] then sin[half] of this token
     const int lane = threadIdx.x & (RI_WAVE - 1), wave = threadIdx.x / RI_WAVE;
     const int t = blockIdx.x;
@@ -158,8 +140,8 @@ qk_norm_rope_k_write_vec_kernel(
         if (hh >= qk_heads) continue;                        // lanes of a head stay together: shuffles below are safe
         TA* x = row + (size_t)hh * head_dim + piece * 8;
         float a[8], b[8];
-        Vec8<TA>::load(x, a);
-        Vec8<TA>::load(x + half, b);
+        Eight<TA>::load(x, a);
+        Eight<TA>::load(x + half, b);
         const float* gain = hh < heads ? q_gain : k_gain;
         if (gain) {
             float ss = 0.f;
@@ -168,8 +150,8 @@ qk_norm_rope_k_write_vec_kernel(
             for (int m = lanes_per_head / 2; m > 0; m >>= 1) ss += __shfl_xor(ss, m, RI_WAVE);
             const float inv = 1.0f / sqrtf(ss / (float)head_dim + eps);
             float ga[8], gb[8];
-            Vec8<float>::load(gain + piece * 8, ga);
-            Vec8<float>::load(gain + half + piece * 8, gb);
+            Eight<float>::load(gain + piece * 8, ga);
+            Eight<float>::load(gain + half + piece * 8, gb);
 #pragma unroll
             for (int e = 0; e < 8; ++e) { a[e] = a[e] * inv * ga[e]; b[e] = b[e] * inv * gb[e]; }
         }
@@ -182,75 +164,14 @@ qk_norm_rope_k_write_vec_kernel(
             }
         }
         if (hh < heads) {
-            Vec8<TA>::store(x, a);
-            Vec8<TA>::store(x + half, b);
+            Eight<TA>::store(x, a);
+            Eight<TA>::store(x + half, b);
         } else {
             TC* dst = k_pages + (((size_t)page * kv_heads + (hh - heads)) * page_size + pos % page_size) * head_dim
                       + piece * 8;
-            Vec8<TC>::store(dst, a);
-            Vec8<TC>::store(dst + half, b);
+            Eight<TC>::store(dst, a);
+            Eight<TC>::store(dst + half, b);
         }
-    }
-}
-
-// Values into their pages, a page at a time: one workgroup per (page touched by this step, sequence,
-// kv head) reads the page's new tokens as rows, turns them through LDS and writes channel rows.
-#define VW_TOKENS 32      // tokens of a page handled at once (pages of other sizes are walked in such pieces)
-template <typename TA, typename TC>
-__global__ void __launch_bounds__(256)
-v_write_pages_kernel(const TA* __restrict__ qkv, const int32_t* __restrict__ cu_seqlens,
-                     const int32_t* __restrict__ tok_pos, const int32_t* __restrict__ page_table, int table_width,
-                     TC* __restrict__ v_pages, int heads, int kv_heads, int head_dim, int page_size) {
-    extern __shared__ float tile[];                          // [VW_TOKENS][head_dim + 1]
-    const int b = blockIdx.y, kvh = blockIdx.z;
-    const int t_begin = cu_seqlens[b], n = cu_seqlens[b + 1] - t_begin;
-    const int start = tok_pos[t_begin];                      // the sequence's new tokens sit at start .. start + n - 1
-    const int first = (start / VW_TOKENS + blockIdx.x) * VW_TOKENS;      // this workgroup's 32 positions
-    const int lo = max(first, start), hi = min(first + VW_TOKENS - 1, start + n - 1);
-    if (lo > hi) return;
-    const int stride = head_dim + 1;
-    const size_t v_off = (size_t)(heads + kv_heads + kvh) * head_dim;
-    const size_t row_len = (size_t)(heads + 2 * kv_heads) * head_dim;
-    if constexpr (sizeof(TA) == 2 && sizeof(TC) == 2) {
-        // 32 new tokens of 16-bit values with a head of whole 16-byte pieces: 16 bytes a thread each way (a
-        // prompt's full pages; the same bits as below, a third of the time)
-        if (lo == first && hi == first + VW_TOKENS - 1 && head_dim % 8 == 0 && page_size % 8 == 0) {
-            const int pieces = head_dim / 8;
-            for (int e = threadIdx.x; e < VW_TOKENS * pieces; e += blockDim.x) {
-                const int tt = e / pieces, d = (e - tt * pieces) * 8;
-                const uint4 v = *reinterpret_cast<const uint4*>(qkv + (size_t)(t_begin + first - start + tt) * row_len + v_off + d);
-                const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    tile[tt * stride + d + 2 * j] = __uint_as_float(w[j] << 16);
-                    tile[tt * stride + d + 2 * j + 1] = __uint_as_float(w[j] & 0xFFFF0000u);
-                }
-            }
-            __syncthreads();
-            const int page = page_table[(size_t)b * table_width + first / page_size];
-            TC* base = v_pages + ((size_t)page * kv_heads + kvh) * page_size * head_dim + first % page_size;
-            for (int e = threadIdx.x; e < head_dim * (VW_TOKENS / 8); e += blockDim.x) {
-                const int d = e / (VW_TOKENS / 8), t8 = (e - d * (VW_TOKENS / 8)) * 8;
-                uint32_t w[4];
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    w[j] = (__float_as_uint(tile[(t8 + 2 * j) * stride + d]) >> 16) |
-                           (__float_as_uint(tile[(t8 + 2 * j + 1) * stride + d]) & 0xFFFF0000u);
-                *reinterpret_cast<uint4*>(base + (size_t)d * page_size + t8) = make_uint4(w[0], w[1], w[2], w[3]);
-            }
-            return;
-        }
-    }
-    for (int e = threadIdx.x; e < (hi - lo + 1) * head_dim; e += blockDim.x) {
-        const int tt = e / head_dim, d = e - tt * head_dim;
-        tile[(lo - first + tt) * stride + d] = to_f32(qkv[(size_t)(t_begin + lo - start + tt) * row_len + v_off + d]);
-    }
-    __syncthreads();
-    const int page = page_table[(size_t)b * table_width + first / page_size];
-    TC* base = v_pages + ((size_t)page * kv_heads + kvh) * page_size * head_dim + first % page_size;
-    for (int e = threadIdx.x; e < head_dim * VW_TOKENS; e += blockDim.x) {
-        const int d = e / VW_TOKENS, tt = e - d * VW_TOKENS;
-        if (first + tt >= lo && first + tt <= hi) from_f32(base + (size_t)d * page_size + tt, tile[tt * stride + d]);
     }
 }
 
@@ -258,9 +179,7 @@ static bool vec_path_fits(int head_dim, int page_size) {
     const int half = head_dim / 2;
     if (half % 8) return false;
     const int lph = half / 8;
-    // (the page-wise value writer holds 32 tokens of a head in LDS: 64 KB at most without asking for more)
-    return lph <= 64 && (lph & (lph - 1)) == 0 && page_size % VW_TOKENS == 0 &&
-           (size_t)VW_TOKENS * (head_dim + 1) * sizeof(float) <= 65536;
+    return lph <= 64 && (lph & (lph - 1)) == 0 && page_size % QT_TOKENS == 0;
 }
 
 template <typename TA, typename TC>
@@ -273,14 +192,16 @@ static void launch_qk(void* qkv, const float* q_gain, const float* k_gain, float
     // than two
     const bool whole = head_dim % 2 == 0 && (!inv_freq || rot_dim == head_dim);      // what the 16-byte kernels rotate
     if (cu_seqlens && max_new > 1 && whole && k_pages && vec_path_fits(head_dim, page_size)) {
-        qk_norm_rope_k_write_vec_kernel<TA, TC><<<tokens, 256, head_dim * sizeof(float), s>>>(
+        const int pieces = values_turn_pieces(max_new), parts = values_turn_parts<TC>(kv_heads, head_dim);
+        const long turns = (long)pieces * seqs * parts;
+        const bool together = tokens + turns < 1 << 23;       // (what one launch holds by far)
+        qk_norm_rope_k_write_vec_kernel<TA, TC><<<tokens + (together ? (int)turns : 0), 256, head_dim * sizeof(float), s>>>(
             (TA*)qkv, q_gain, k_gain, eps, inv_freq, tok_pos, tok_seq, page_table, table_width, (TC*)k_pages, heads,
-            kv_heads, head_dim, page_size);
-        // a sequence's max_new tokens touch at most this many 32-token pieces
-        dim3 grid((max_new + VW_TOKENS - 2) / VW_TOKENS + 1, seqs, kv_heads);
-        v_write_pages_kernel<TA, TC><<<grid, 256, VW_TOKENS * (head_dim + 1) * sizeof(float), s>>>(
-            (const TA*)qkv, cu_seqlens, tok_pos, page_table, table_width, (TC*)v_pages, heads, kv_heads, head_dim,
-            page_size);
+            kv_heads, head_dim, page_size, tokens, cu_seqlens, pieces, parts, (TC*)v_pages);
+        if (!together)
+            launch_values_to_pages<TC>((const TC*)qkv, (size_t)(heads + 2 * kv_heads) * head_dim, (size_t)(heads + kv_heads) * head_dim,
+                                       cu_seqlens, tok_pos, page_table, table_width, (TC*)v_pages, seqs, max_new, kv_heads, head_dim, page_size,
+                                       nullptr, s);
         return;
     }
     const long items = (long)tokens * (heads + 2 * kv_heads);

@@ -130,10 +130,8 @@ static void launch_qk_temper(void* qkv, const float* q_gain, const float* k_gain
         qk_norm_temper_k_write_vec_kernel<TA, TC><<<tokens, 256, 0, s>>>(
             (TA*)qkv, q_gain, k_gain, eps, temp_coef, temp_every, tok_pos, tok_seq, page_table, table_width, (TC*)k_pages,
             heads, kv_heads, dim, vdim, page_size);
-        dim3 grid((max_new + QT_TOKENS - 2) / QT_TOKENS + 1, seqs, kv_heads);      // the 32-position pieces a sequence may touch
-        values_to_pages_kernel<TA, TC><<<grid, 256, QT_TOKENS * (vdim + 1) * sizeof(float), s>>>(
-            (const TA*)qkv, row_len, (size_t)(heads + kv_heads) * dim, cu_seqlens, tok_pos, page_table, table_width,
-            (TC*)v_pages, kv_heads, vdim, page_size, nullptr);
+        launch_values_to_pages<TC>((const TC*)qkv, row_len, (size_t)(heads + kv_heads) * dim, cu_seqlens, tok_pos, page_table, table_width,
+                                   (TC*)v_pages, seqs, max_new, kv_heads, vdim, page_size, nullptr, s);
         return;
     }
     const long items = (long)tokens * (heads + 2 * kv_heads);
@@ -180,7 +178,7 @@ extern "C" int ri_qk_norm_temper_kv_write(void* qkv, int act_dtype, const float*
 // `dim`, or without one: unit_norm), from a projection row that may hold more than this mixer's columns: q heads
 // at q_off, k heads at k_off, v heads at v_off of rows of row_len elements.  q in place, k and v into their pages.
 // Angle, sine and cosine, and the norm are float32; an element is rounded once.  One wavefront per (token, head),
-// a lane on pairs of neighbours; a prompt's values go a page at a time (values_to_pages_kernel).
+// a lane on pairs of neighbours; a prompt's values go eight positions at a time (launch_values_to_pages).
 #define QP_PAIRS_PER_LANE 4     // head sizes up to 64 * 2 * 4
 
 // HPW: heads a wavefront takes one after the other (all of one token, so that the angles' sines and cosines are made
@@ -268,7 +266,7 @@ __global__ void qk_pairs_norm_kv_write_kernel(
 // A prompt with head sizes that 16-byte pieces divide (8 times a power of two, up to 512): a workgroup a token, a lane
 // on eight neighbours (four pairs) of a head, so that a wavefront takes 512 / dim heads at once; the four angles'
 // sines and cosines are made once a lane and serve every head of the token.  q in place, k into its page; the values
-// go a page at a time (values_to_pages_kernel).
+// go eight positions at a time (launch_values_to_pages).
 template <typename TA, typename TC>
 __global__ void __launch_bounds__(256)
 qk_pairs_norm_k_write_vec_kernel(TA* __restrict__ proj, size_t row_len, int q_off, int k_off,
@@ -355,10 +353,8 @@ extern "C" int ri_qk_pairs_norm_kv_write(void* proj, int act_dtype, long row_len
     qk_pairs_norm_k_write_vec_kernel<T, T><<<tokens, 256, 0, s>>>(                                                        \
         (T*)proj, (size_t)row_len, q_off, k_off, inv_freq, rot_dims, q_gain, k_gain, norm, eps, tok_pos, tok_seq,         \
         page_table, table_width, (T*)k_pages, heads, kv_heads, dim, page_size);                                          \
-    values_to_pages_kernel<T, T><<<dim3((max_new + QT_TOKENS - 2) / QT_TOKENS + 1, seqs, kv_heads), 256,                   \
-                                   QT_TOKENS * (vdim + 1) * sizeof(float), s>>>(                                          \
-        (const T*)proj, (size_t)row_len, (size_t)v_off, cu_seqlens, tok_pos, page_table, table_width, (T*)v_pages,        \
-        kv_heads, vdim, page_size, nullptr)
+    launch_values_to_pages<T>((const T*)proj, (size_t)row_len, (size_t)v_off, cu_seqlens, tok_pos, page_table, table_width, (T*)v_pages, seqs, \
+                              max_new, kv_heads, vdim, page_size, nullptr, s)
         if (act_dtype == RI_F32) { RI_VEC(float); } else { RI_VEC(bf16_t); }
 #undef RI_VEC
         RI_LAUNCH_CHECK("qk_pairs_norm_kv_write");
@@ -375,12 +371,9 @@ extern "C" int ri_qk_pairs_norm_kv_write(void* proj, int act_dtype, long row_len
         page_table, table_width, (T*)k_pages, (T*)v_pages, tokens, heads, kv_heads, dim, vdim, page_size, !paged_values)
 #define RI_GO(T)                                                                                                        \
     if (four) RI_PAIRS(T, 4); else RI_PAIRS(T, 1);                                                                       \
-    if (paged_values) {                                                                                                 \
-        dim3 grid((max_new + QT_TOKENS - 2) / QT_TOKENS + 1, seqs, kv_heads);                                            \
-        values_to_pages_kernel<T, T><<<grid, 256, QT_TOKENS * (vdim + 1) * sizeof(float), s>>>(                           \
-            (const T*)proj, (size_t)row_len, (size_t)v_off, cu_seqlens, tok_pos, page_table, table_width, (T*)v_pages,    \
-            kv_heads, vdim, page_size, nullptr);                                                                        \
-    }
+    if (paged_values)                                                                                                   \
+        launch_values_to_pages<T>((const T*)proj, (size_t)row_len, (size_t)v_off, cu_seqlens, tok_pos, page_table, table_width, (T*)v_pages, \
+                                  seqs, max_new, kv_heads, vdim, page_size, nullptr, s);
     if (act_dtype == RI_F32) { RI_GO(float) } else { RI_GO(bf16_t) }
 #undef RI_GO
 #undef RI_PAIRS

@@ -259,6 +259,23 @@ def test_qk_norm_rope_kv_write(ops, dtype, rel, heads, kv_heads, dh, paged_value
     assert np.array_equal(f64(qkv2), qkv)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("heads, kv_heads, dh", [(2, 1, 16), (3, 3, 128), (6, 2, 256)])
+def test_values_turned_by_groups_of_eight_positions(ops, dtype, heads, kv_heads, dh):
+    """Steps that begin and end on and beside a group's and a page's edge: the values as they are, and no other place touched."""
+    before, new = [0, 8, 7, 9, 24, 31, 0, 33, 40], [32, 8, 1, 6, 8, 2, 9, 31, 64]
+    rng = np.random.default_rng(dh)
+    _, _, kp, vp, table = paged(rng, [a + n for a, n in zip(before, new)], kv_heads, dh, dtype=dtype)
+    want = f64(vp).copy()
+    qkv = t(rng.normal(size=(sum(new), (heads + 2 * kv_heads) * dh)), dtype)
+    seq, pos = [b for b, n in enumerate(new) for _ in range(n)], [before[b] + i for b, n in enumerate(new) for i in range(n)]
+    for i, (b, p) in enumerate(zip(seq, pos)):
+        want[table[b, p // 32].item(), :, :, p % 32] = f64(qkv[i, (heads + kv_heads) * dh:]).reshape(kv_heads, dh)
+    ops.qk_norm_rope_kv_write(qkv, None, None, 1e-5, None, t(pos, torch.int32), t(seq, torch.int32), table, kp, vp, heads, kv_heads, dh,
+                              cu_seqlens=t(np.concatenate([[0], np.cumsum(new)]), torch.int32), max_new=max(new))
+    assert np.array_equal(f64(vp), want)
+
+
 @pytest.mark.parametrize("dtype, rel", [(torch.float32, 3e-6), (torch.bfloat16, BF16_OUT)])
 @pytest.mark.parametrize("dh, rot", [(64, 16), (48, 24), (40, 8), (7, 4), (9, 0), (130, 128), (512, 64)])
 def test_rotation_over_part_of_the_head(ops, dtype, rel, dh, rot):
