@@ -469,6 +469,14 @@ int ri_talking_attention_mfma(void* out, float* stats, const void* q, int q_stri
                               int page_size, int window, float scale, const float* r1, const float* r2, const float* talk,
                               float* bias, float* parts, int shares, int tokens, void* stream);
 
+// The same for single tokens in bfloat16 (talking_decode.hip): pages of 32, heads of 32, 64 or 128, up to 64 of them in groups of a
+// power of two; pages: as many as any token sees; out float32 [shares][tokens][heads * dim], partial sums for the caller to add.
+int ri_talking_decode_fits(int heads, int kv_heads, int dim, int page_size);
+int ri_talking_decode(float* out, int shares, float* scores, float* sums, int pages, const void* q, int q_stride, int q_off,
+                      const void* k_pages, const void* v_pages, const int32_t* tok_pos, const int32_t* tok_seq,
+                      const int32_t* page_table, int table_width, int tokens, int heads, int kv_heads, int dim, int page_size,
+                      int window, float scale, const float* r1, const float* r2, const float* talk, void* stream);
+
 // ---- time mixing (timemix.hip)
 int ri_shift_mix(void* out, int out_dtype, const float* x, const float* kept, const float* mu, int n_mix,
                  const int32_t* tok_seq, const int32_t* cu_seqlens, const int32_t* slots, int tokens, int width, void* stream);

@@ -410,7 +410,16 @@ __global__ void sum_parts_kernel(TO* __restrict__ out, const float* __restrict__
     const int m = (int)(e / width), i = (int)(e - (long)m * width);
     const float* p = parts + (long)m * (swiglu ? 2 * width : width) + i;
     float g = 0.f, u = 0.f;
-    for (int q = 0; q < n_parts; ++q) {
+    int q = 0;
+    if (!swiglu)
+        for (; q + 8 <= n_parts; q += 8) {                    // eight parts asked for together, added in order
+            float v[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[i] = p[(q + i) * part_stride];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) g += v[i];
+        }
+    for (; q < n_parts; ++q) {
         g += p[q * part_stride];
         if (swiglu) u += p[q * part_stride + width];
     }

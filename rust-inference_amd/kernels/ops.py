@@ -182,6 +182,9 @@ _SIGNATURES = {
     "ri_talking_attention_mfma": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_int,
                                   c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_void_p, c_void_p, c_void_p,
                                   c_void_p, c_void_p, c_int, c_int, c_void_p],
+    "ri_talking_decode_fits": [c_int, c_int, c_int, c_int],
+    "ri_talking_decode": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p,
+                          c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_void_p, c_void_p, c_void_p, c_void_p],
     "ri_shift_mix": [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p],
     "ri_shift_keep": [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p],
     "ri_timemix_max_dim": [],
@@ -1938,6 +1941,43 @@ def talking_attention_mfma(proj, q_off: int, k_pages, v_pages, tok_pos, cu_seqle
           _opt(talk, "talk", torch.float32, (heads, heads)), _opt(bias, "bias", torch.float32), _opt(parts, "parts", torch.float32), shares,
           tokens, _stream())
     return sum_parts(parts) if parts is not None else out
+
+
+# Bytes of scores that a step of single tokens may keep between its two launches.
+TALKING_DECODE_SCORES = 1 << 28
+# Workgroups that its second launch is to have at least (a page a workgroup at most).  32 heads of 128, us at 256 / 512 / 1,024: 8 tokens at
+# 1,400 keys 29.9 / 27.5 / 27.4, 40 at 1,500 66.7 / 59.0 / 60.6, 300 at 1,500 422 / 325 / 338, 4 at 8,000 without a window 66.6 / 62.9 / 73.6.
+TALKING_DECODE_FILL = 512
+
+
+def talking_decode_pages(longest: int, window: int | None) -> int:
+    """The most pages of 32 keys that one token sees of ``longest`` keys."""
+    pages = -(-longest // 32)
+    return min(pages, (window + 30) // 32 + 1) if window else pages
+
+
+def talking_decode_fits(dtype, tokens: int, longest: int, window: int | None, heads: int, kv_heads: int, dim: int, page_size: int) -> bool:
+    """Whether a step of single tokens runs ``talking_decode``: sizes that the matrix cores take, and scores that fit a workspace."""
+    return (dtype == torch.bfloat16 and tokens <= 65535 and bool(_get("ri_talking_decode_fits")(heads, kv_heads, dim, page_size))
+            and tokens * talking_decode_pages(longest, window) * heads * 128 <= TALKING_DECODE_SCORES)
+
+
+def talking_decode(proj, q_off: int, k_pages, v_pages, tok_pos, tok_seq, page_table, heads: int, kv_heads: int, dim: int,
+                   window: int | None, scale: float, r1, r2, talk, longest: int) -> torch.Tensor:
+    """The same attention for single tokens in bfloat16, of sequences of up to ``longest`` keys: float32 ``[T, heads * dim]``."""
+    tokens, pages = proj.shape[0], talking_decode_pages(longest, window)
+    blocks = -(-kv_heads * dim // 1024)
+    shares = max(1, min(pages, -(-TALKING_DECODE_FILL // (tokens * blocks))))
+    new = lambda *shape: torch.empty(shape, dtype=torch.float32, device=proj.device)
+    out, scores, sums = new(shares, tokens, heads * dim), new(tokens, pages, heads, 32), new(tokens, pages, heads, 2)
+    _call("ri_talking_decode", _dev(out, "out"), shares, _dev(scores, "scores"), _dev(sums, "sums"), pages,
+          _dev(proj, "proj", torch.bfloat16), proj.shape[1], int(q_off), _dev(k_pages, "k_pages", torch.bfloat16),
+          _dev(v_pages, "v_pages", torch.bfloat16, (k_pages.shape[0], kv_heads, dim, k_pages.shape[2])),
+          _dev(tok_pos, "tok_pos", torch.int32, (tokens,)), _dev(tok_seq, "tok_seq", torch.int32, (tokens,)),
+          _dev(page_table, "page_table", torch.int32), page_table.shape[1], tokens, heads, kv_heads, dim, k_pages.shape[2], int(window or 0),
+          float(scale), _opt(r1, "r1", torch.float32, (heads,)), _opt(r2, "r2", torch.float32, (heads,)),
+          _opt(talk, "talk", torch.float32, (heads, heads)), _stream())
+    return out[0] if shares == 1 else sum_parts(out, torch.float32)
 
 
 # ---------------------------------------------------------------- time mixing

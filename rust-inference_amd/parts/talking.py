@@ -94,6 +94,12 @@ class TalkingAttention(Mixer):
                 o = ops.talking_attention_mfma(proj, 0, store.k_pages, store.v_pages, ctx.tok_pos, ctx.cu_seqlens, ctx.new_counts,
                                                page_table, self.heads, self.kv_heads, self.dim, self.window, self.scale, self.r1,
                                                self.r2, self.mix, ctx.max_len)
+            elif (ctx.is_decode and not rt.invariant and proj.shape[1] % 8 == 0
+                    and ops.talking_decode_fits(proj.dtype, proj.shape[0], ctx.max_len, self.window, self.heads, self.kv_heads, self.dim,
+                                                store.page_size)):
+                # single tokens: the scores of every page side by side, then the mix and the values of a few pages a workgroup
+                o = ops.talking_decode(proj, 0, store.k_pages, store.v_pages, ctx.tok_pos, ctx.tok_seq, page_table, self.heads,
+                                       self.kv_heads, self.dim, self.window, self.scale, self.r1, self.r2, self.mix, ctx.max_len)
             else:
                 o = ops.talking_attention(proj, 0, store.k_pages, store.v_pages, ctx.tok_pos, ctx.tok_seq, page_table, self.heads,
                                           self.kv_heads, self.dim, self.window, self.scale, self.r1, self.r2, self.mix, shares)

@@ -482,6 +482,37 @@ def test_talking_attention_on_the_matrix_cores_is_the_general_kernel(ops, heads,
         close(got, f64(want), 1.5e-2, "matrix cores against the general kernels")
 
 
+@pytest.mark.parametrize("heads, kv_heads, dim, window", [(8, 2, 32, 40), (16, 16, 32, None), (4, 2, 128, 33), (16, 1, 64, 32), (24, 12, 128, 1),
+                                                          (64, 8, 32, None)])
+def test_single_tokens_of_talking_heads_are_the_general_kernel(ops, heads, kv_heads, dim, window, monkeypatch):
+    """bfloat16: sequences that end at the first and last key of a page, pages behind the window given back (-1 in the table), bounds on
+    the length above the real one; a page a workgroup, several and all of them; with the distance bias and the mixing matrix and
+    without; against the general kernels on the same pages in float32."""
+    rng = np.random.default_rng(heads)
+    pages, ends = 12, [0, 31, 32, 95, 65]
+    k_pages = guarded((torch.randn((pages, kv_heads, PAGE, dim), device=DEV) * 0.6).to(torch.bfloat16))
+    v_pages = guarded((torch.randn((pages, kv_heads, dim, PAGE), device=DEV) * 0.6).to(torch.bfloat16))
+    table = np.full((5, 4), -1, dtype=np.int32)
+    free = iter(rng.permutation(pages))
+    for b, end in enumerate(ends):
+        for page in range(max(0, end - window + 1) // 32 if window else 0, end // 32 + 1):
+            table[b, page] = next(free)
+    table, pos, seq = t(table, torch.int32), t(ends, torch.int32), t(range(5), torch.int32)
+    proj = guarded((torch.randn((5, heads * dim + 16), device=DEV) * 0.6).to(torch.bfloat16))
+    r1, r2 = t(rng.random(heads)), t(rng.random(heads) * 3)
+    talk = t(np.eye(heads) + 0.3 * rng.standard_normal((heads, heads)))
+    assert ops.talking_decode_fits(torch.bfloat16, 5, 128, window, heads, kv_heads, dim, PAGE)
+    for fill, longest in ((512, 128), (5 * -(-kv_heads * dim // 1024) * 2, 96), (1, 4096)):
+        monkeypatch.setattr(ops, "TALKING_DECODE_FILL", fill)
+        for a, b, c in ((r1, r2, talk), (None, None, None)):
+            want = [ops.talking_attention(proj[i:i + 1].float(), 8, k_pages.float(), v_pages.float(), pos[i:i + 1], seq[i:i + 1], table,
+                                          heads, kv_heads, dim, window, 0.2, a, b, c) for i in range(5)] if heads * dim <= 3072 else \
+                   [ops.talking_attention(proj[i:i + 1], 8, k_pages, v_pages, pos[i:i + 1], seq[i:i + 1], table, heads, kv_heads, dim, window,
+                                          0.2, a, b, c, 2) for i in range(5)]
+            got = ops.talking_decode(proj, 8, k_pages, v_pages, pos, seq, table, heads, kv_heads, dim, window, 0.2, a, b, c, longest)
+            close(got, np.concatenate([f64(w) for w in want]), F32, f"{fill} workgroups")
+
+
 @pytest.mark.parametrize("dim, window, table", [(32, 40, True), (64, 45, False), (128, None, False)])
 def test_talking_attention_whole_and_in_shares(ops, dim, window, table, monkeypatch):
     """Tiles that are walked whole, whose result is bfloat16 at once, and in two, three and four shares of their pages, whose float32 sums
