@@ -445,7 +445,7 @@ int ri_latent_attention_mfma(void* out, const void* q, int q_stride, const void*
                              const int32_t* tok_pos, const int32_t* tok_seq, const int32_t* page_table, int table_width,
                              int tokens, int heads, int key_dim, int rank, int page_size, float scale, const float* sinks,
                              float* partial, int chunks, int chunk_pages, int shared_pages, const int32_t* cu_seqlens, int seqs,
-                             void* stream);
+                             int quarters, void* stream);
 
 // ---- windowed attention whose heads talk (talking_attention.hip)
 int ri_whole_norm_kv_write(void* proj, int act_dtype, int stride, int q_off, int k_off, const float* q_gain,

@@ -153,6 +153,86 @@ head_products_kernel(TO* __restrict__ out, int out_stride, int out_off, int out_
     }
 }
 
+// bfloat16 matrices whose rows 16-byte pieces divide: tiles of 16 tokens by 128 columns, the eight wavefronts of a workgroup on a slice of K
+// each, on the matrix cores' float32 product (16x16x4; the matrix elements are widened, so every product and sum is a 32-bit one).  Lane
+// (g, r) reads eight neighbouring columns of row k + g at once, one of each of eight products, up to sixteen such loads asked for
+// together; the slices meet through LDS in order, so a result's sum depends on K alone.  What bounds it is two trips to memory and
+// the sum; the kernel above made sixteen, two bytes a lane.  32 heads, us the kernel above : this: 512 x 128, one token
+// 16.7 : 9.8, 32 19.3 : 11.8, 120 42 : 18; 128 x 512 6.3 : 5.6, 9.2 : 7.0, 28 : 24 (with cold caches, as in a model's step, 8 tokens
+// 37 : 12.7 and 12.0 : 7.0).
+#define HM_TOKENS 16
+#define HM_COLS 128
+#define HM_WAVES 8
+#define HM_DEEP 16           // loads of a wavefront that are under way together
+typedef __attribute__((__vector_size__(4 * sizeof(float)))) float hm_floatx4;
+
+template <typename TX, typename TO>
+__global__ void __launch_bounds__(64 * HM_WAVES)
+head_products_matrix_kernel(TO* __restrict__ out, int out_stride, int out_off, int out_head, const TX* __restrict__ x, int x_stride,
+                            int x_off, int x_head, const bf16_t* __restrict__ w, const TX* __restrict__ gates, int g_stride, int g_off,
+                            float scale, int tokens, int k, int n, int extra) {
+    extern __shared__ float4 lds4[];
+    float* xs = reinterpret_cast<float*>(lds4);               // [HM_TOKENS][k + 4], then the slices' sums [HM_WAVES][HM_TOKENS][HM_COLS]
+    const int h = blockIdx.y, t0 = blockIdx.x * HM_TOKENS, tid = threadIdx.x, lane = tid & 63, r = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), c0 = blockIdx.z * HM_COLS, pitch = k + 4;
+    const int steps = (k / 4 + HM_WAVES - 1) / HM_WAVES, s0 = min(wave * steps, k / 4), s1 = min(s0 + steps, k / 4);
+    const bf16_t* wp = w + (size_t)h * k * n + min(c0 + 8 * r, n - 8);
+    uint4 wv[HM_DEEP];
+    auto fetch = [&](int from) {
+#pragma unroll
+        for (int i = 0; i < HM_DEEP; ++i) wv[i] = *reinterpret_cast<const uint4*>(wp + (size_t)(4 * min(from + i, k / 4 - 1) + g) * n);
+    };
+    fetch(s0);
+    for (int e = tid; e < HM_TOKENS * k; e += 64 * HM_WAVES) {
+        const int tt = e / k, col = e % k, t = t0 + tt;
+        xs[tt * pitch + col] = t < tokens ? to_f32(x[(size_t)t * x_stride + x_off + (size_t)h * x_head + col]) : 0.f;
+    }
+    __syncthreads();
+    hm_floatx4 acc[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) acc[j] = hm_floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int s = s0; s < s1; s += HM_DEEP) {
+#pragma unroll
+        for (int i = 0; i < HM_DEEP; ++i) {
+            if (s + i >= s1) break;                           // (the same for the whole wavefront)
+            const float xv = xs[r * pitch + 4 * (s + i) + g];
+            const uint32_t p[4] = {wv[i].x, wv[i].y, wv[i].z, wv[i].w};
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                acc[2 * j] = __builtin_amdgcn_mfma_f32_16x16x4f32(xv, __uint_as_float(p[j] << 16), acc[2 * j], 0, 0, 0);
+                acc[2 * j + 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(xv, __uint_as_float(p[j] & 0xFFFF0000u), acc[2 * j + 1], 0, 0, 0);
+            }
+        }
+        if (s + HM_DEEP < s1) fetch(s + HM_DEEP);
+    }
+    __syncthreads();                                          // the rows have been read
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {                             // token 4 g + i, columns 8 r ..+8
+        float4* to = lds4 + ((wave * HM_TOKENS + 4 * g + i) * HM_COLS + 8 * r) / 4;
+        to[0] = make_float4(acc[0][i], acc[1][i], acc[2][i], acc[3][i]);
+        to[1] = make_float4(acc[4][i], acc[5][i], acc[6][i], acc[7][i]);
+    }
+    __syncthreads();
+    for (int e = tid; e < HM_TOKENS * HM_COLS; e += 64 * HM_WAVES) {
+        const int tt = e / HM_COLS, c = c0 + e % HM_COLS, t = t0 + tt;
+        if (t >= tokens || c >= n) continue;
+        float v = xs[e];
+        for (int s = 1; s < HM_WAVES; ++s) v += xs[s * HM_TOKENS * HM_COLS + e];
+        float f = scale;
+        if (gates) f *= 1.f / (1.f + expf(-to_f32(gates[(size_t)t * g_stride + g_off + h])));
+        from_f32(out + (size_t)t * out_stride + out_off + (size_t)h * out_head + c, v * f);
+    }
+    if (blockIdx.z == 0)
+        for (int e = tid; e < HM_TOKENS * extra; e += 64 * HM_WAVES) {
+            const int c = e % extra, t = t0 + e / extra;
+            if (t >= tokens) break;
+            float f = scale;
+            if (gates) f *= 1.f / (1.f + expf(-to_f32(gates[(size_t)t * g_stride + g_off + h])));
+            from_f32(out + (size_t)t * out_stride + out_off + (size_t)h * out_head + n + c,
+                     to_f32(x[(size_t)t * x_stride + x_off + (size_t)h * x_head + k + c]) * f);
+        }
+}
+
 extern "C" int ri_head_products(void* out, int out_dtype, int out_stride, int out_off, int out_head, const void* x, int x_dtype,
                                 int x_stride, int x_off, int x_head, const void* w, int w_dtype, const void* gates, int g_stride,
                                 int g_off, float scale, int tokens, int heads, int k, int n, int extra, void* stream) {
@@ -171,6 +251,23 @@ extern "C" int ri_head_products(void* out, int out_dtype, int out_stride, int ou
     hipStream_t s = (hipStream_t)stream;
     const dim3 grid((tokens + HP_TOKENS - 1) / HP_TOKENS, heads, (n + extra + HP_COLS - 1) / HP_COLS);
     RI_REQUIRE(grid.z <= 65535, "head_products: results of %d", n + extra);
+    // Sizes and alignment alone decide, so that a token's result does not depend on the step.  Fewer than 128 rows are too few for eight
+    // slices (16 heads of 64 x 128, us the other : this: 8 tokens 4.8 : 5.1, 64 5.0 : 5.5); up to 1,020 fit the kernel's LDS.
+    const size_t sums = sizeof(float) * HM_WAVES * HM_TOKENS * HM_COLS, rows = sizeof(float) * HM_TOKENS * ((size_t)k + 4);
+    if (k >= 128 && w_dtype == RI_BF16 && k % 4 == 0 && n % 8 == 0 && rows <= 64 * 1024 && (uintptr_t)w % 16 == 0 &&
+        !(x_dtype == RI_F32 && out_dtype != RI_F32)) {
+        const dim3 tiles((tokens + HM_TOKENS - 1) / HM_TOKENS, heads, (n + HM_COLS - 1) / HM_COLS);
+#define RI_MATRIX(TX, TO)                                                                                               \
+    head_products_matrix_kernel<TX, TO><<<tiles, 64 * HM_WAVES, rows > sums ? rows : sums, s>>>(                        \
+        (TO*)out, out_stride, out_off, out_head, (const TX*)x, x_stride, x_off, x_head, (const bf16_t*)w, (const TX*)gates, g_stride, g_off, \
+        scale, tokens, k, n, extra)
+        if (x_dtype == RI_F32) RI_MATRIX(float, float);
+        else if (out_dtype == RI_F32) RI_MATRIX(bf16_t, float);
+        else RI_MATRIX(bf16_t, bf16_t);
+#undef RI_MATRIX
+        RI_LAUNCH_CHECK("head_products");
+        return 0;
+    }
 #define RI_GO(TX, TW, TO)                                                                                               \
     head_products_kernel<TX, TW, TO><<<grid, HP_COLS * HP_SLICES, lds, s>>>((TO*)out, out_stride, out_off, out_head, (const TX*)x, x_stride, \
                                                             x_off, x_head, (const TW*)w, (const TX*)gates, g_stride, g_off, \

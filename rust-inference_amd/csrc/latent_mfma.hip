@@ -9,7 +9,7 @@
 // how the value product wants its weights: no exchange between lanes.  A sink per head joins the sum once at the end.
 // Scores, maxima, sums and the accumulators are float32; the weights are rounded to bfloat16 for the value product, as
 // in this library's other matrix-core attention.  A token's sums run over its pages in order, whatever else the step holds.
-// A step of few tokens cuts a token's pages into chunks that wavefronts walk side by side; each leaves its maximum, its sum
+// A step of few single tokens cuts a token's pages into chunks that workgroups walk side by side; each leaves its maximum, its sum
 // and its sums of values, and a second kernel joins them in the chunks' order.
 #include "api.h"
 #include "common.h"
@@ -33,13 +33,11 @@ latent_attention_mfma_kernel(bf16_t* __restrict__ out, const bf16_t* __restrict_
                              const bf16_t* __restrict__ k_pages, const bf16_t* __restrict__ v_pages,
                              const int32_t* __restrict__ tok_pos, const int32_t* __restrict__ tok_seq,
                              const int32_t* __restrict__ page_table, int table_width, int tokens, int heads, int tiles,
-                             float scale_log2, const float* __restrict__ sinks, float* __restrict__ partial, int chunks,
-                             int chunk_pages) {
+                             float scale_log2, const float* __restrict__ sinks) {
     constexpr int DK = 32 * KS, RANK = 16 * VT;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int unit = blockIdx.x * LM_WAVES + wave;            // (token, tile of 16 heads, chunk of pages)
-    if (unit >= tokens * tiles * chunks) return;
-    const int pair = unit / chunks, chunk = unit % chunks;
+    const int pair = blockIdx.x * LM_WAVES + wave;            // (token, tile of 16 heads)
+    if (pair >= tokens * tiles) return;
     // (long prompts first: the workgroups launched last are the short ones)
     const int t = tokens - 1 - pair / tiles, tile = pair % tiles;
     const int col = lane & 15, g = lane >> 4;
@@ -58,8 +56,7 @@ latent_attention_mfma_kernel(bf16_t* __restrict__ out, const bf16_t* __restrict_
     float m = -INFINITY, l = 0.f;
     const int key_row = 8 * (col >> 2) + (col & 3);           // the key this lane's operand row holds in the first half page
 
-    const int page_end = chunks > 1 ? min(qpos / LM_PAGE + 1, (chunk + 1) * chunk_pages) : qpos / LM_PAGE + 1;
-    for (int page = chunks > 1 ? chunk * chunk_pages : 0; page < page_end; ++page) {
+    for (int page = 0; page <= qpos / LM_PAGE; ++page) {
         const long phys = table[page];
         const bf16_t* kp = k_pages + phys * LM_PAGE * (long)DK + (long)key_row * DK + 8 * g;
         lm_floatx4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
@@ -105,18 +102,6 @@ latent_attention_mfma_kernel(bf16_t* __restrict__ out, const bf16_t* __restrict_
     }
     l += __shfl_xor(l, 16, RI_WAVE);                          // a column's sum over its four lanes
     l += __shfl_xor(l, 32, RI_WAVE);
-    if (chunks > 1) {
-        // a chunk's share: its maximum, its sum and its sums of values as they are, for the join (a chunk without pages: -inf, 0, 0)
-        if (head < heads) {
-            float* pp = partial + (((size_t)t * heads + head) * chunks + chunk) * (RANK + 2);
-            if (g == 0) { pp[0] = m; pp[1] = l; }
-#pragma unroll
-            for (int vt = 0; vt < VT; ++vt)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) pp[2 + vt * 16 + 4 * g + i] = o[vt][i];
-        }
-        return;
-    }
     if (sinks) l += exp2f(sinks[hq] * 1.4426950408889634f - m);
     const float inv = 1.0f / l;
     if (head < heads) {
@@ -128,6 +113,128 @@ latent_attention_mfma_kernel(bf16_t* __restrict__ out, const bf16_t* __restrict_
             w.y = pack_bf16x2(o[vt][2] * inv, o[vt][3] * inv);
             *reinterpret_cast<uint2*>(op + vt * 16) = w;
         }
+    }
+}
+
+// Single tokens: the four wavefronts of a workgroup share a (token, tile of 16 heads, chunk of pages).  Each makes the scores' products
+// over its quarter of the key rows' elements, the quarters meet lane by lane in LDS (one barrier a page: two buffers take turns), and
+// each goes on with all scores and a quarter of the value rows.  What bounds the kernel above on a step of few tokens is a wavefront's
+// wait for the 68 loads a page that its registers cannot hold at once; a quarter's 18 are all asked for together, the next page's
+// keys before the values are used.  32 heads, keys of 576, us with the join, a wavefront a chunk : this: one token at 1,000 keys 21.5 :
+// 11.9, 8 at 1,400 42.4 : 16.6, 40 at 1,500 165 : 47, 128 at 1,000 571 : 81, 300 at 1,000 590 : 216; 16 heads, keys of 160: 8.2 : 7.4,
+// 11.5 : 8.7, 21.9 : 16.4, 27.8 : 19.1.
+template <int KS, int VT>
+__global__ void __launch_bounds__(64 * LM_WAVES)
+latent_attention_quarters_kernel(bf16_t* __restrict__ out, const bf16_t* __restrict__ q, int q_stride,
+                                 const bf16_t* __restrict__ k_pages, const bf16_t* __restrict__ v_pages,
+                                 const int32_t* __restrict__ tok_pos, const int32_t* __restrict__ tok_seq,
+                                 const int32_t* __restrict__ page_table, int table_width, int tokens, int heads, int tiles,
+                                 float scale_log2, const float* __restrict__ sinks, float* __restrict__ partial, int chunks,
+                                 int chunk_pages) {
+    constexpr int DK = 32 * KS, RANK = 16 * VT, KW = (KS + LM_WAVES - 1) / LM_WAVES, VW = VT / LM_WAVES;
+    __shared__ lm_floatx4 scores[2][LM_WAVES][2][RI_WAVE];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), unit = blockIdx.x;
+    const int pair = unit / chunks, chunk = unit % chunks;
+    const int t = tokens - 1 - pair / tiles, tile = pair % tiles;
+    const int col = lane & 15, g = lane >> 4;
+    const int head = tile * 16 + col;
+    const int hq = head < heads ? head : heads - 1;
+    const int qpos = tok_pos[t];
+    const int32_t* table = page_table + (size_t)tok_seq[t] * table_width;
+    const int k0 = KS * wave / LM_WAVES, k1 = KS * (wave + 1) / LM_WAVES;        // this wavefront's steps over the key rows
+
+    LmFrag qf[KW], kf[KW][2], vf[VW];
+#pragma unroll
+    for (int i = 0; i < KW; ++i)
+        qf[i].u = *reinterpret_cast<const uint4*>(q + (size_t)t * q_stride + (size_t)hq * DK + min(k0 + i, KS - 1) * 32 + 8 * g);
+    lm_floatx4 o[VW];
+#pragma unroll
+    for (int vt = 0; vt < VW; ++vt) o[vt] = lm_floatx4{0.f, 0.f, 0.f, 0.f};
+    float m = -INFINITY, l = 0.f;
+    const int key_row = 8 * (col >> 2) + (col & 3);           // (the kernel above's order of keys)
+    const int page_end = chunks > 1 ? min(qpos / LM_PAGE + 1, (chunk + 1) * chunk_pages) : qpos / LM_PAGE + 1;
+    const int page_begin = chunks > 1 ? chunk * chunk_pages : 0;
+    auto fetch_keys = [&](long phys) {
+        const bf16_t* kp = k_pages + phys * LM_PAGE * (long)DK + (long)key_row * DK + 8 * g;
+#pragma unroll
+        for (int i = 0; i < KW; ++i) {
+            kf[i][0].u = *reinterpret_cast<const uint4*>(kp + min(k0 + i, KS - 1) * 32);
+            kf[i][1].u = *reinterpret_cast<const uint4*>(kp + 4 * DK + min(k0 + i, KS - 1) * 32);
+        }
+    };
+    long phys = 0;
+    if (page_begin < page_end) fetch_keys(phys = table[page_begin]);
+    for (int page = page_begin, buf = 0; page < page_end; ++page, buf ^= 1) {    // (the same for the whole workgroup)
+        const bf16_t* vp = v_pages + phys * (long)RANK * LM_PAGE + (long)(wave * VW * 16 + col) * LM_PAGE + 8 * g;
+        phys = table[min(page + 1, page_end - 1)];
+#pragma unroll
+        for (int vt = 0; vt < VW; ++vt) vf[vt].u = *reinterpret_cast<const uint4*>(vp + (long)vt * 16 * LM_PAGE);
+        lm_floatx4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < KW; ++i)
+            if (k0 + i < k1) {                                // (the same for the whole wavefront)
+                s0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[i][0].v, qf[i].v, s0, 0, 0, 0);
+                s1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[i][1].v, qf[i].v, s1, 0, 0, 0);
+            }
+        fetch_keys(phys);
+        scores[buf][wave][0][lane] = s0;
+        scores[buf][wave][1][lane] = s1;
+        __syncthreads();
+        s0 = scores[buf][0][0][lane];
+        s1 = scores[buf][0][1][lane];
+#pragma unroll
+        for (int w = 1; w < LM_WAVES; ++w) {
+            s0 += scores[buf][w][0][lane];
+            s1 += scores[buf][w][1][lane];
+        }
+        float s[8] = {s0[0], s0[1], s0[2], s0[3], s1[0], s1[1], s1[2], s1[3]};
+        const int key0 = page * LM_PAGE + 8 * g;
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+            if (key0 + e > qpos) s[e] = -INFINITY;
+        float mx = fmaxf(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3])), fmaxf(fmaxf(s[4], s[5]), fmaxf(s[6], s[7])));
+        mx = fmaxf(mx, __shfl_xor(mx, 16, RI_WAVE));
+        mx = fmaxf(mx, __shfl_xor(mx, 32, RI_WAVE));
+        const float m_new = fmaxf(m, mx * scale_log2);        // the scale is positive; every page of the walk has a key that is seen
+        LmFrag p;
+        float sum = 0.f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float a = exp2f(fmaf(s[2 * e], scale_log2, -m_new));
+            const float b = exp2f(fmaf(s[2 * e + 1], scale_log2, -m_new));
+            p.w[e] = pack_bf16x2(a, b);
+            sum += a + b;
+        }
+        const float corr = exp2f(m - m_new);
+        l = l * corr + sum;
+        m = m_new;
+#pragma unroll
+        for (int vt = 0; vt < VW; ++vt) {
+            o[vt] *= corr;
+            o[vt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[vt].v, p.v, o[vt], 0, 0, 0);
+        }
+    }
+    l += __shfl_xor(l, 16, RI_WAVE);
+    l += __shfl_xor(l, 32, RI_WAVE);
+    if (head >= heads) return;
+    if (chunks > 1) {
+        float* pp = partial + (((size_t)t * heads + head) * chunks + chunk) * (RANK + 2);
+        if (g == 0 && wave == 0) { pp[0] = m; pp[1] = l; }
+#pragma unroll
+        for (int vt = 0; vt < VW; ++vt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) pp[2 + (wave * VW + vt) * 16 + 4 * g + i] = o[vt][i];
+        return;
+    }
+    if (sinks) l += exp2f(sinks[hq] * 1.4426950408889634f - m);
+    const float inv = 1.0f / l;
+    bf16_t* op = out + ((size_t)t * heads + head) * RANK + wave * VW * 16 + 4 * g;
+#pragma unroll
+    for (int vt = 0; vt < VW; ++vt) {
+        uint2 w;
+        w.x = pack_bf16x2(o[vt][0] * inv, o[vt][1] * inv);
+        w.y = pack_bf16x2(o[vt][2] * inv, o[vt][3] * inv);
+        *reinterpret_cast<uint2*>(op + vt * 16) = w;
     }
 }
 
@@ -321,19 +428,19 @@ extern "C" int ri_latent_attention_mfma_fits(int key_dim, int rank, int page_siz
 // heads side by side) over its sequence's one key/value head of key rows of key_dim and value rows of rank.
 // shared_pages: neighbouring tokens share the pages they fetch (the results are the same bits): in as many workgroups of eight
 // (token, tile of 16 heads) pairs as it says, each of one sequence, where cu_seqlens [seqs + 1] is given; else 1, a workgroup's tokens
-// the step's neighbours, of one sequence for the most part.
+// the step's neighbours, of one sequence for the most part.  quarters: for single tokens, a workgroup a (token, tile, chunk).
 extern "C" int ri_latent_attention_mfma(void* out, const void* q, int q_stride, const void* k_pages, const void* v_pages,
                                         const int32_t* tok_pos, const int32_t* tok_seq, const int32_t* page_table,
                                         int table_width, int tokens, int heads, int key_dim, int rank, int page_size, float scale,
                                         const float* sinks, float* partial, int chunks, int chunk_pages, int shared_pages,
-                                        const int32_t* cu_seqlens, int seqs, void* stream) {
+                                        const int32_t* cu_seqlens, int seqs, int quarters, void* stream) {
     RI_REQUIRE(tokens > 0 && heads > 0 && ri_latent_attention_mfma_fits(key_dim, rank, page_size),
                "latent_attention_mfma: %d tokens, %d heads, keys of %d, values of %d, pages of %d", tokens, heads, key_dim, rank, page_size);
     RI_REQUIRE(q_stride >= heads * key_dim && q_stride % 8 == 0 && (uintptr_t)q % 16 == 0 && (uintptr_t)k_pages % 16 == 0 &&
                (uintptr_t)v_pages % 16 == 0 && (uintptr_t)out % 8 == 0, "latent_attention_mfma: rows of %d for %d heads of %d, or a buffer that is not aligned",
                q_stride, heads, key_dim);
     RI_REQUIRE(scale > 0.f && table_width > 0, "latent_attention_mfma: scale %g", (double)scale);
-    RI_REQUIRE(chunks >= 1 && chunks <= LM_MAX_CHUNKS && (chunks == 1 || (partial && chunk_pages >= 1)) && heads <= 65535,
+    RI_REQUIRE(chunks >= 1 && chunks <= LM_MAX_CHUNKS && (chunks == 1 || (quarters && partial && chunk_pages >= 1)) && heads <= 65535,
                "latent_attention_mfma: %d chunks of %d pages", chunks, chunk_pages);
     const int tiles = (heads + 15) / 16;
     const long pairs = (long)tokens * tiles * chunks;
@@ -345,9 +452,16 @@ extern "C" int ri_latent_attention_mfma(void* out, const void* q, int q_stride, 
     latent_attention_mfma_kernel<KS, VT><<<blocks, 64 * LM_WAVES, 0, s>>>((bf16_t*)out, (const bf16_t*)q, q_stride,     \
                                                                           (const bf16_t*)k_pages, (const bf16_t*)v_pages, \
                                                                           tok_pos, tok_seq, page_table, table_width, tokens, \
-                                                                          heads, tiles, scale_log2, sinks, partial, chunks, \
-                                                                          chunk_pages)
-    if (shared_pages && chunks == 1) {
+                                                                          heads, tiles, scale_log2, sinks)
+    if (quarters) {
+        RI_REQUIRE(pairs <= 2147483647L, "latent_attention_mfma: %ld tiles exceed one launch", pairs);
+#define RI_QUARTERS(KS, VT)                                                                                             \
+    latent_attention_quarters_kernel<KS, VT><<<(unsigned)pairs, 64 * LM_WAVES, 0, s>>>(                                 \
+        (bf16_t*)out, (const bf16_t*)q, q_stride, (const bf16_t*)k_pages, (const bf16_t*)v_pages, tok_pos, tok_seq, page_table, table_width, \
+        tokens, heads, tiles, scale_log2, sinks, partial, chunks, chunk_pages)
+        if (key_dim == 576) RI_QUARTERS(18, 32); else if (key_dim == 288) RI_QUARTERS(9, 16); else RI_QUARTERS(5, 8);
+#undef RI_QUARTERS
+    } else if (shared_pages) {
         RI_REQUIRE(pairs <= 2147483647L - LP_WAVES && (!cu_seqlens || seqs > 0), "latent_attention_mfma: %ld pairs of %d sequences", pairs, seqs);
         const unsigned groups = cu_seqlens ? (unsigned)shared_pages : (unsigned)((pairs + LP_WAVES - 1) / LP_WAVES);
 #define RI_SHARED(KS, VT)                                                                                               \

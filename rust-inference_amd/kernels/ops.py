@@ -169,7 +169,7 @@ _SIGNATURES = {
                           c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
     "ri_latent_attention_mfma_fits": [c_int, c_int, c_int],
     "ri_latent_attention_mfma": [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int,
-                                 c_int, c_int, c_int, c_float, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_int, c_void_p],
+                                 c_int, c_int, c_int, c_float, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_int, c_int, c_void_p],
     "ri_head_products": [c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_int, c_void_p,
                          c_int, c_int, c_float, c_int, c_int, c_int, c_int, c_int, c_void_p],
     "ri_whole_norm_kv_write": [c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_float, c_void_p, c_void_p, c_void_p,
@@ -1751,6 +1751,12 @@ def latent_attention_shared(new_counts, starts, heads: int, key_dim: int) -> int
     return sum(-(-n * tiles // LATENT_SHARED_WAVES) for n in new_counts)
 
 
+# Workgroups that a step of single tokens has at most when it cuts its sequences' pages into chunks.  32 heads, keys of 576, us at 256 / 512 /
+# 1,024: 8 tokens at 200 keys 12.8 / 20.0 / 20.0, at 1,400 16.6 / 21.5 / 30.5, 40 at 1,500 47 / 56 / 57, 128 at 1,000 81 / 94 / 102 (more chunks are more
+# for the join to add); 16 heads, keys of 160, 40 at 1,500 16.4 / 13.6 / 16.9.
+LATENT_DECODE_FILL = 256
+
+
 def latent_attention_mfma(q, k_pages, v_pages, tok_pos, tok_seq, page_table, heads: int, scale: float, sinks,
                           max_len: int = 0, new_counts=None, starts=None, cu_seqlens=None) -> torch.Tensor:
     """bfloat16 ``[T, heads * rank]``: causal attention on the matrix cores of every new token's ``heads`` query rows (``q [T,
@@ -1766,9 +1772,9 @@ def latent_attention_mfma(q, k_pages, v_pages, tok_pos, tok_seq, page_table, hea
     out = torch.empty((tokens, heads * rank), dtype=torch.bfloat16, device=q.device)
     chunks, chunk_pages, partial = 1, 0, None
     units = tokens * -(-heads // 16)
-    if max_len and units < 256:                      # fewer wavefronts than half the machine's SIMDs: chunks of pages side by side
+    if max_len and units < LATENT_DECODE_FILL:       # fewer workgroups than fill the machine: chunks of pages side by side
         pages = -(-int(max_len) // page)
-        chunks = max(1, min(pages, 512 // units, 64))
+        chunks = max(1, min(pages, LATENT_DECODE_FILL // units, 64))
         chunk_pages = -(-pages // chunks)
         chunks = -(-pages // chunk_pages)
         if chunks > 1:
@@ -1787,7 +1793,7 @@ def latent_attention_mfma(q, k_pages, v_pages, tok_pos, tok_seq, page_table, hea
           _dev(tok_pos, "tok_pos", torch.int32, (tokens,)), _dev(tok_seq, "tok_seq", torch.int32, (tokens,)),
           _dev(page_table, "page_table", torch.int32), page_table.shape[1], tokens, heads, key_dim, rank, page, float(scale),
           _opt(sinks, "sinks", torch.float32, (heads,)), _opt(partial, "partial"), chunks, chunk_pages, shared,
-          _opt(cu_seqlens, "cu_seqlens", torch.int32, (seqs + 1,)), seqs, _stream())
+          _opt(cu_seqlens, "cu_seqlens", torch.int32, (seqs + 1,)), seqs, int(bool(max_len)), _stream())
     return out
 
 

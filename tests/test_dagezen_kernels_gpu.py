@@ -362,6 +362,24 @@ def test_batched_head_products_are_the_products_per_head(ops, heads, k, n, extra
     close(alone, want, 6e-3, "products per head")
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("tokens, k, n, extra", [(1, 128, 8, 0), (17, 132, 136, 5), (16, 516, 128, 0), (3, 1020, 8, 2), (33, 160, 264, 64)])
+def test_products_per_head_with_bfloat16_matrices(ops, dtype, tokens, k, n, extra):
+    """Tiles of 16 tokens and 128 columns, slices of the rows that leave wavefronts without one, and their remainders, in float32."""
+    rng = np.random.default_rng(k)
+    heads, x_off = 2, 3
+    x = t(rng.standard_normal((tokens, x_off + heads * (k + extra) + heads)), dtype)
+    w = t(rng.standard_normal((heads, k, n)), torch.bfloat16)
+    gated = k > 140
+    got = ops.head_products(x, x_off, k + extra, w, heads, k, n, extra=extra, gates=x if gated else None, g_off=x_off + heads * (k + extra),
+                            scale=0.5, out_dtype=torch.float32)
+    xs = f64(x)[:, x_off:x_off + heads * (k + extra)].reshape(tokens, heads, k + extra)
+    want = 0.5 * np.concatenate([np.einsum("thk,hkn->thn", xs[:, :, :k], f64(w)), xs[:, :, k:]], 2)
+    if gated:
+        want *= (1 / (1 + np.exp(-f64(x)[:, -heads:])))[:, :, None]
+    close(got, want.reshape(tokens, -1), F32, "products per head")
+
+
 # ---------------------------------------------------------------- the latent attention on the matrix cores
 @pytest.mark.parametrize("heads", [3, 20])
 def test_latent_attention_on_the_matrix_cores_is_the_general_kernel(ops, heads):
@@ -382,6 +400,25 @@ def test_latent_attention_on_the_matrix_cores_is_the_general_kernel(ops, heads):
         for bound in (101, 128, 1024):                    # chunks of one page, of one page with more room than pages, of eight
             got = ops.latent_attention_mfma(q, k_pages, v_pages, tok_pos, tok_seq, table, heads, 0.11, sink, bound)
             close(got, f64(want), 1.2e-2, f"in chunks, sequences of up to {bound}")
+
+
+@pytest.mark.parametrize("heads, dk, rank", [(3, 160, 128), (20, 288, 256), (16, 576, 512)])
+def test_latent_attention_of_single_tokens_in_quarters(ops, heads, dk, rank, monkeypatch):
+    """A workgroup's wavefronts on a quarter of the key rows and of the value rows each: whole walks, chunks of a page and of several, more
+    chunks than pages; against a wavefront that walks all of them, up to the order of float32 sums and their rounding to bfloat16."""
+    pages, ends = 9, [0, 31, 32, 100, 69]
+    k_pages = guarded((torch.randn((pages, 1, PAGE, dk), device=DEV) * 0.3).to(torch.bfloat16))
+    v_pages = guarded(k_pages[:, :, :, :rank].transpose(2, 3).contiguous())
+    table = t([[8, -1, -1, -1], [0, -1, -1, -1], [3, 1, -1, -1], [7, 5, 2, 4], [6, 3, 0, -1]], torch.int32)
+    pos, seq = t(ends, torch.int32), t(range(5), torch.int32)
+    q = guarded((torch.randn((5, heads * dk), device=DEV) * 0.3).to(torch.bfloat16))
+    sinks = t(np.linspace(-1, 1, heads))
+    want = f64(ops.latent_attention_mfma(q, k_pages, v_pages, pos, seq, table, heads, 0.11, sinks))
+    for fill in (1, 5 * -(-heads // 16) * 2, 512):
+        monkeypatch.setattr(ops, "LATENT_DECODE_FILL", fill)
+        for bound in (101, 2048):
+            got = ops.latent_attention_mfma(q, k_pages, v_pages, pos, seq, table, heads, 0.11, sinks, bound)
+            close(got, want, 8e-3, f"{fill} workgroups, sequences of up to {bound}")
 
 
 @pytest.mark.parametrize("heads, dk, rank", [(3, 160, 128), (20, 288, 256), (40, 160, 128), (130, 160, 128), (16, 576, 512)])
