@@ -451,7 +451,8 @@ int ri_latent_attention_mfma(void* out, const void* q, int q_stride, const void*
 int ri_whole_norm_kv_write(void* proj, int act_dtype, int stride, int q_off, int k_off, const float* q_gain,
                            const float* k_gain, float eps, const int32_t* tok_pos, const int32_t* tok_seq,
                            const int32_t* page_table, int table_width, void* k_pages, void* v_pages, int cache_dtype,
-                           int page_size, int tokens, int heads, int kv_heads, int dim, void* stream);
+                           int page_size, int tokens, int heads, int kv_heads, int dim, const int32_t* cu_seqlens, int seqs, int max_new,
+                           void* stream);
 // shares > 1: out is float32 [shares][tokens][out_stride] partial sums for the caller to add; stats: float32 workspace
 // [tokens][heads][2].
 int ri_talking_attention_shares(int tokens, int longest);

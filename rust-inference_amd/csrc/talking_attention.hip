@@ -15,6 +15,7 @@
 // and the accumulators are float32.
 #include "api.h"
 #include "common.h"
+#include "kv_pages.h"
 
 #define TK_TILE 32
 #define TK_ACCS 16           // results a thread accumulates: heads * vdim <= 256 * TK_ACCS
@@ -53,10 +54,95 @@ whole_norm_kv_write_kernel(TA* __restrict__ proj, int stride, int q_off, int k_o
     }
 }
 
+// The same in 16-byte pieces that a thread keeps from the sums to the stores: a workgroup a token, all of its loads asked for together (the
+// form above reads every element twice, 2 bytes a lane, and waits for 16 of them one after the other).  A prompt's values go eight
+// positions at a time by the workgroups past the tokens (values_turn); a single token's go element by element.  32 heads over 8 of 128,
+// us the form above : this: 8 single tokens 8.4 : 4.5 (with cold caches, as in a model's step, 14 : 5), 300 15.0 : 8.1, a prompt of
+// 2,048 26 : 11.5; 16 heads 6.5 : 4.3, 11.4 : 7.7, 21.5 : 10.1.
+#define WN_Q 4               // pieces of the queries a thread holds at most, and
+#define WN_K 2               // of the keys
+template <typename T>
+__global__ void __launch_bounds__(256)
+whole_norm_kv_write_vec_kernel(T* __restrict__ proj, int stride, int q_off, int k_off, const float* __restrict__ q_gain,
+                               const float* __restrict__ k_gain, float eps, const int32_t* __restrict__ tok_pos,
+                               const int32_t* __restrict__ tok_seq, const int32_t* __restrict__ page_table, int table_width,
+                               T* __restrict__ k_pages, T* __restrict__ v_pages, int page_size, int heads, int kv_heads, int dim, int tokens,
+                               const int32_t* __restrict__ cu_seqlens, int pieces, int parts) {
+    if ((int)blockIdx.x >= tokens) {
+        const int at = blockIdx.x - tokens, of_seq = at / parts;
+        values_turn<T>(proj, (size_t)stride, (size_t)k_off, cu_seqlens, tok_pos, page_table, table_width, v_pages, kv_heads, dim, page_size,
+                       nullptr, of_seq % pieces, of_seq / pieces, at % parts);
+        return;
+    }
+    __shared__ float sums[2][4];
+    constexpr int E = 16 / (int)sizeof(T);
+    const int t = blockIdx.x, tid = threadIdx.x, qn = heads * dim / E, kn = kv_heads * dim / E;
+    T* row = proj + (size_t)t * stride;
+    uint4 qv[WN_Q], kv[WN_K];
+#pragma unroll
+    for (int i = 0; i < WN_Q; ++i) qv[i] = *reinterpret_cast<const uint4*>(row + q_off + (size_t)min(tid + 256 * i, qn - 1) * E);
+#pragma unroll
+    for (int i = 0; i < WN_K; ++i) kv[i] = *reinterpret_cast<const uint4*>(row + k_off + (size_t)min(tid + 256 * i, kn - 1) * E);
+    const int pos = tok_pos[t], slot = pos % page_size;
+    const long page = page_table[(size_t)tok_seq[t] * table_width + pos / page_size];
+    const auto element = [](const uint4 v, int e) {
+        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+        if constexpr (sizeof(T) == 4) return __uint_as_float(w[e]);
+        else return __uint_as_float(e & 1 ? w[e / 2] & 0xFFFF0000u : w[e / 2] << 16);
+    };
+    float qs = 0.f, ks = 0.f;
+#pragma unroll
+    for (int i = 0; i < WN_Q; ++i)
+#pragma unroll
+        for (int e = 0; e < E; ++e) qs += tid + 256 * i < qn ? element(qv[i], e) * element(qv[i], e) : 0.f;
+#pragma unroll
+    for (int i = 0; i < WN_K; ++i)
+#pragma unroll
+        for (int e = 0; e < E; ++e) ks += tid + 256 * i < kn ? element(kv[i], e) * element(kv[i], e) : 0.f;
+    qs = wave_sum(qs);
+    ks = wave_sum(ks);
+    if (tid % RI_WAVE == 0) { sums[0][tid / RI_WAVE] = qs; sums[1][tid / RI_WAVE] = ks; }
+    __syncthreads();
+    const float q_inv = 1.0f / sqrtf((sums[0][0] + sums[0][1] + sums[0][2] + sums[0][3]) / (float)(heads * dim) + eps);
+    const float k_inv = 1.0f / sqrtf((sums[1][0] + sums[1][1] + sums[1][2] + sums[1][3]) / (float)(kv_heads * dim) + eps);
+    const auto store = [&](T* to, const uint4 v, float inv, const float* gain) {
+        T y[E];
+#pragma unroll
+        for (int e = 0; e < E; e += 4) {
+            const float4 g = *reinterpret_cast<const float4*>(gain + e);
+            from_f32(&y[e], element(v, e) * inv * g.x);
+            from_f32(&y[e + 1], element(v, e + 1) * inv * g.y);
+            from_f32(&y[e + 2], element(v, e + 2) * inv * g.z);
+            from_f32(&y[e + 3], element(v, e + 3) * inv * g.w);
+        }
+        if constexpr (sizeof(T) == 4) *reinterpret_cast<float4*>(to) = make_float4(y[0], y[1], y[2], y[3]);
+        else
+            *reinterpret_cast<uint4*>(to) = make_uint4(y[0] | (uint32_t)y[1] << 16, y[2] | (uint32_t)y[3] << 16, y[4] | (uint32_t)y[5] << 16,
+                                                       y[6] | (uint32_t)y[7] << 16);
+    };
+#pragma unroll
+    for (int i = 0; i < WN_Q; ++i) {
+        const int e = (tid + 256 * i) * E;
+        if (tid + 256 * i < qn) store(row + q_off + e, qv[i], q_inv, q_gain + e);
+    }
+#pragma unroll
+    for (int i = 0; i < WN_K; ++i) {
+        if (tid + 256 * i >= kn) continue;
+        const int e = (tid + 256 * i) * E, g = e / dim, c = e % dim;
+        store(k_pages + ((page * kv_heads + g) * page_size + slot) * (long)dim + c, kv[i], k_inv, k_gain + e);
+        if (pieces == 0) {
+            T* to = v_pages + ((page * kv_heads + g) * (long)dim + c) * page_size + slot;
+#pragma unroll
+            for (int j = 0; j < E; ++j) from_f32(to + (long)j * page_size, element(kv[i], j));      // (as it lies: it is rounded already)
+        }
+    }
+}
+
 extern "C" int ri_whole_norm_kv_write(void* proj, int act_dtype, int stride, int q_off, int k_off, const float* q_gain,
                                       const float* k_gain, float eps, const int32_t* tok_pos, const int32_t* tok_seq,
                                       const int32_t* page_table, int table_width, void* k_pages, void* v_pages, int cache_dtype,
-                                      int page_size, int tokens, int heads, int kv_heads, int dim, void* stream) {
+                                      int page_size, int tokens, int heads, int kv_heads, int dim, const int32_t* cu_seqlens, int seqs,
+                                      int max_new, void* stream) {
     RI_REQUIRE(tokens > 0 && heads > 0 && kv_heads > 0 && dim > 0, "whole_norm_kv_write: %d tokens, %d and %d heads of %d", tokens,
                heads, kv_heads, dim);
     RI_REQUIRE(q_off >= 0 && k_off >= 0 && q_off + heads * dim <= stride && k_off + kv_heads * dim <= stride,
@@ -64,7 +150,28 @@ extern "C" int ri_whole_norm_kv_write(void* proj, int act_dtype, int stride, int
     RI_REQUIRE(act_dtype == cache_dtype && (act_dtype == RI_F32 || act_dtype == RI_BF16), "whole_norm_kv_write: dtypes %d and %d",
                act_dtype, cache_dtype);
     RI_REQUIRE(page_size > 0 && table_width > 0 && q_gain && k_gain, "whole_norm_kv_write: page geometry and gains");
+    RI_REQUIRE(!cu_seqlens || (seqs > 0 && max_new > 0), "whole_norm_kv_write: seqs %d, max_new %d", seqs, max_new);
     hipStream_t s = (hipStream_t)stream;
+    const int unit = act_dtype == RI_F32 ? 4 : 8;
+    // Sizes and alignment alone decide which form norms: a token's bits do not depend on the step.  Where the queries are no piece a
+    // thread the other form's loads are few (8 heads over 2 of 64, us: 8 single tokens 4.0 : 3.9, prompts of 17 4.1 : 4.6, 2,048 6.8 : 7.7).
+    if (dim % unit == 0 && heads * dim >= 256 * unit && (stride | q_off | k_off) % unit == 0 && heads * dim <= 256 * WN_Q * unit && kv_heads * dim <= 256 * WN_K * unit &&
+        (((uintptr_t)proj | (uintptr_t)k_pages | (uintptr_t)v_pages | (uintptr_t)q_gain | (uintptr_t)k_gain) & 15) == 0) {
+        int pieces = 0, parts = 1;
+        if (cu_seqlens && max_new > 1 && page_size % QT_TOKENS == 0) {
+            pieces = values_turn_pieces(max_new);
+            parts = act_dtype == RI_F32 ? values_turn_parts<float>(kv_heads, dim) : values_turn_parts<bf16_t>(kv_heads, dim);
+            if (tokens + (long)pieces * seqs * parts >= 1 << 23) pieces = 0;       // (more than a launch is to hold: element by element)
+        }
+        const int blocks = tokens + pieces * seqs * parts;
+#define RI_WHOLE(T)                                                                                                     \
+        whole_norm_kv_write_vec_kernel<T><<<blocks, 256, 0, s>>>((T*)proj, stride, q_off, k_off, q_gain, k_gain, eps, tok_pos, tok_seq, \
+            page_table, table_width, (T*)k_pages, (T*)v_pages, page_size, heads, kv_heads, dim, tokens, cu_seqlens, pieces, parts)
+        if (act_dtype == RI_F32) RI_WHOLE(float); else RI_WHOLE(bf16_t);
+#undef RI_WHOLE
+        RI_LAUNCH_CHECK("whole_norm_kv_write");
+        return 0;
+    }
     if (act_dtype == RI_F32)
         whole_norm_kv_write_kernel<float, float><<<tokens, 256, 0, s>>>((float*)proj, stride, q_off, k_off, q_gain, k_gain, eps,
                                                                        tok_pos, tok_seq, page_table, table_width, (float*)k_pages,

@@ -173,7 +173,7 @@ _SIGNATURES = {
     "ri_head_products": [c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_int, c_void_p,
                          c_int, c_int, c_float, c_int, c_int, c_int, c_int, c_int, c_void_p],
     "ri_whole_norm_kv_write": [c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_float, c_void_p, c_void_p, c_void_p,
-                               c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
+                               c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p, c_int, c_int, c_void_p],
     "ri_talking_attention_shares": [c_int, c_int],
     "ri_talking_attention": [c_void_p, c_int, c_int, c_int, c_float, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p,
                              c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int,
@@ -1859,10 +1859,11 @@ def head_products_batched(x, x_off: int, x_head: int, w, heads: int, k: int, n: 
 
 # ---------------------------------------------------------------- windowed attention whose heads talk
 def whole_norm_kv_write(proj, q_off: int, k_off: int, q_gain, k_gain, eps: float, tok_pos, tok_seq, page_table, k_pages,
-                        v_pages, heads: int, kv_heads: int, dim: int) -> None:
+                        v_pages, heads: int, kv_heads: int, dim: int, cu_seqlens=None, max_new: int = 0) -> None:
     """q (``heads * dim`` columns from ``q_off``) and k (``kv_heads * dim`` from ``k_off``) of every row are RMS-normed over
     the whole projection with a gain an element; q stays in place, the normed k goes to the key pages and k as projected
-    to the value pages."""
+    to the value pages.  ``cu_seqlens`` (int32 ``[seqs + 1]``) and ``max_new``: the sequences' new tokens, whose values then go eight
+    positions at a time."""
     tokens, stride = proj.shape
     if tuple(k_pages.shape[1:]) != (kv_heads, v_pages.shape[3], dim) or tuple(v_pages.shape[1:3]) != (kv_heads, dim):
         raise ShapeError(f"whole_norm_kv_write: key pages {list(k_pages.shape)}, value pages {list(v_pages.shape)}")
@@ -1870,7 +1871,8 @@ def whole_norm_kv_write(proj, q_off: int, k_off: int, q_gain, k_gain, eps: float
           _dev(q_gain, "q_gain", torch.float32, (heads * dim,)), _dev(k_gain, "k_gain", torch.float32, (kv_heads * dim,)),
           float(eps), _dev(tok_pos, "tok_pos", torch.int32, (tokens,)), _dev(tok_seq, "tok_seq", torch.int32, (tokens,)),
           _dev(page_table, "page_table", torch.int32), page_table.shape[1], _dev(k_pages, "k_pages"), _dev(v_pages, "v_pages"),
-          code(k_pages.dtype), k_pages.shape[2], tokens, heads, kv_heads, dim, _stream())
+          code(k_pages.dtype), k_pages.shape[2], tokens, heads, kv_heads, dim, _opt(cu_seqlens, "cu_seqlens", torch.int32),
+          0 if cu_seqlens is None else cu_seqlens.shape[0] - 1, int(max_new), _stream())
 
 
 def talking_attention_shares(tokens: int, longest: int) -> int:

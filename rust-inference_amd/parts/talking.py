@@ -83,7 +83,8 @@ class TalkingAttention(Mixer):
             proj = ops.as_rows(rt.linear_packed(x, self.w_in))             # [T, q | k | g]
         with profiler.section(profiler.QK_NORM_ROPE_APPEND):
             ops.whole_norm_kv_write(proj, 0, self.q_width, self.q_gain, self.k_gain, self.eps, ctx.tok_pos, ctx.tok_seq,
-                                    page_table, store.k_pages, store.v_pages, self.heads, self.kv_heads, self.dim)
+                                    page_table, store.k_pages, store.v_pages, self.heads, self.kv_heads, self.dim, ctx.cu_seqlens,
+                                    ctx.max_new)
         with profiler.section(profiler.ATTENTION):
             # a step of few tokens cuts its walk over the keys into shares that run side by side
             longest = min(ctx.max_len, self.window) if self.window else ctx.max_len

@@ -211,6 +211,38 @@ def test_talking_attention_through_every_cut(ops, heads, kv_heads, dim, window, 
         close(got[:, 3:], 0.5 * np.concatenate(want), 2e-5, f"talking attention, step {counts}")
 
 
+@pytest.mark.parametrize("dtype, rel", [(torch.float32, F32), (torch.bfloat16, 8e-3)])
+@pytest.mark.parametrize("heads, kv_heads, dim, stray", [(18, 9, 128, 0), (9, 3, 8, 0), (32, 16, 32, 0), (16, 4, 256, 0), (3, 1, 40, 4), (2, 1, 6, 0)])
+def test_whole_norm_and_both_writes(ops, dtype, rel, heads, kv_heads, dim, stray):
+    """Pieces of sixteen bytes and single elements (rows that they do not divide), prompts and single tokens, pages begun and left inside:
+    keys normed over the row, values the keys as projected, the columns beside them and the pages' other places as they were."""
+    rng = np.random.default_rng(heads)
+    before, new = [0, 5, 31, 40, 24], [33, 1, 2, 24, 9]
+    seq, pos = [b for b, n in enumerate(new) for _ in range(n)], [before[b] + i for b, n in enumerate(new) for i in range(n)]
+    tokens, qw, kw, gap = len(seq), heads * dim, kv_heads * dim, 8 + stray
+    rows = t(rng.standard_normal((tokens, gap + qw + kw + 8 + stray)), dtype)
+    q_gain, k_gain = 1 + 0.1 * rng.standard_normal(qw), 1 + 0.1 * rng.standard_normal(kw)
+    table = rng.permutation(10).reshape(5, 2)
+    x = f64(rows)
+    q, k = x[:, gap:gap + qw], x[:, gap + qw:gap + qw + kw]
+    norm = lambda v, g: v / np.sqrt((v * v).mean(1, keepdims=True) + 1e-5) * g
+    for bounds in ({}, dict(cu_seqlens=t(np.concatenate([[0], np.cumsum(new)]), torch.int32), max_new=max(new))):
+        k_pages, v_pages = (t(np.full((10, kv_heads) + shape, 7.0), dtype) for shape in ((PAGE, dim), (dim, PAGE)))
+        proj = guarded(rows.clone())
+        ops.whole_norm_kv_write(proj, gap, gap + qw, t(q_gain), t(k_gain), 1e-5, t(pos, torch.int32), t(seq, torch.int32), t(table, torch.int32),
+                                k_pages, v_pages, heads, kv_heads, dim, **bounds)
+        got = f64(proj)
+        close(t(got[:, gap:gap + qw]), norm(q, q_gain), rel, "queries")
+        got[:, gap:gap + qw] = q
+        assert np.array_equal(got, x)
+        want_k, want_v, kn = np.full(k_pages.shape, 7.0), np.full(v_pages.shape, 7.0), norm(k, k_gain)
+        for i, (b, p) in enumerate(zip(seq, pos)):
+            want_k[table[b, p // PAGE], :, p % PAGE] = kn[i].reshape(kv_heads, dim)
+            want_v[table[b, p // PAGE], :, :, p % PAGE] = k[i].reshape(kv_heads, dim)
+        close(k_pages, want_k, rel, "keys")
+        assert np.array_equal(f64(v_pages), want_v)
+
+
 def test_a_key_at_the_windows_edge_counts_and_the_next_one_does_not(ops):
     """One loud key: at distance window - 1 it takes the softmax, at distance window it is not seen."""
     heads, dim, window, n = 2, 8, 37, 80
