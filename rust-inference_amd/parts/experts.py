@@ -171,6 +171,7 @@ class RoutedExperts(FeedForward):
             routed = (rt.dtype == torch.bfloat16 and not rt.invariant and self.top < self.experts
                       and self.hidden % 8 == 0 and self.inter % 8 == 0)
             own = self.identity > 0                   # whether the identity experts' share is still to be added
+            shared = None
             if routed and tokens * self.top < self.experts:
                 if self.gated:
                     y, own = ops.experts_few_tokens(rt.normed_now(x), self.w_gate_up.w, self.w_down.w, ids, weights, self.inter,
@@ -180,7 +181,10 @@ class RoutedExperts(FeedForward):
                                                      self.activation)
             elif (routed and tokens >= self.SORTED_MIN_TOKENS and not ctx.is_decode
                     and not torch.cuda.is_current_stream_capturing()):
-                y, own = self.forward_sorted(rt.normed_now(x), ids, weights), False
+                rows = self.sort(rt.normed_now(x), ids)
+                # (ahead of the host's wait for the experts' row counts: the GPU has work while the host asks for theirs)
+                shared = self.shared_product(x)
+                y, own = self.forward_sorted(*rows, weights), False
             else:
                 gu = ops.as_rows(rt.linear_packed(x, self.w_gate_up))
                 a = (ops.experts_activate(gu, dense, self.inter, self.limit) if self.gated
@@ -189,24 +193,36 @@ class RoutedExperts(FeedForward):
                 y = rt.linear_packed(a, self.w_down, out_dtype=torch.float32, parts_ok=True)
             if not own and self.shared is None:
                 return y
-            shared = None
-            if self.shared is not None:
-                act = rt.linear_packed(x, self.w_shared_in)
-                shared = rt.linear_packed(act, self.w_shared_down, out_dtype=torch.float32, parts_ok=True)
+            if shared is None:
+                shared = self.shared_product(x)
             if separate and not own and not self.shared_gate:
                 return [y, shared]
             # (without a gate the shared expert is added as it is)
             return ops.experts_finish(y, rt.normed_now(x) if own else None, shared, extra if own or self.shared_gate else None)
 
-    def forward_sorted(self, x, ids, weights):
+    def shared_product(self, x):
+        if self.shared is None:
+            return None
+        act = self.rt.linear_packed(x, self.w_shared_in)
+        return self.rt.linear_packed(act, self.w_shared_down, out_dtype=torch.float32, parts_ok=True)
+
+    def sort(self, x, ids):
+        """A prompt's assignments as rows side by side, expert after expert; where each expert's begin is on its way to the host."""
+        dest, offsets = ops.experts_sort(ids, self.outs)
+        starts = torch.empty(offsets.shape, dtype=offsets.dtype, pin_memory=True)
+        starts.copy_(offsets, non_blocking=True)
+        there = torch.cuda.Event()
+        there.record()
+        return ops.experts_gather(x, dest, self.top), dest, starts, there
+
+    def forward_sorted(self, rows, dest, starts, there, weights):
         """A prompt: every expert's tokens as rows side by side, two library products an expert, the weighted sum in
         float32.  The host reads how many rows every expert has (one wait a layer), which a captured step could not."""
         ff = self.inter
         rows_each = 2 * ff if self.gated else ff
-        dest, offsets = ops.experts_sort(ids, self.outs)
-        rows = ops.experts_gather(x, dest, self.top)
         y = torch.empty_like(rows)
-        starts = offsets.tolist()
+        there.synchronize()
+        starts = starts.tolist()
         for e in range(self.experts):
             a, b = starts[e], starts[e + 1]
             if b > a:
