@@ -7,8 +7,9 @@
 // For Higher-Precision Computations", 2019).  Here x = a + (b + c) 2^-16 exactly, for every float32: the parts are cut off, not
 // rounded, and b and c are kept 2^16 times as large, so that the last bit of the smallest float32, 2^-149, is still one of bfloat16's
 // (2^-133; the matrix cores take subnormal numbers as they are).  Every product of a part and a weight is exact in float32 above
-// the subnormal numbers, and the sums of the three parts are float32 sums of their own, added at the end: what is rounded is the
-// additions alone, as in a chain of multiply-adds, and there are fewer of them.  Relative error against
+// the subnormal numbers; the first part's sum and that of the two lower ones, whose last bits lie far below what the first rounds away, are
+// float32 sums of their own, added at the end: what is rounded is the additions alone, as in a chain of multiply-adds, and there
+// are fewer of them.  Relative error against
 // 64 bits (2-norm, normal x and weights): at K = 1,024 1.9e-7 where the chain of multiply-adds has 5.7e-7, at 3,072
 // 3.4e-7 : 9.9e-7.  The three products run at a third of the bfloat16 rate, ten times the vector units' multiply-adds.
 // An infinity, a NaN or a number past 2^119 has no such parts, but leaves an infinity or NaN in every sum it enters: such an
@@ -64,42 +65,42 @@ __device__ __forceinline__ void chain_again(float* out, const float* x, const bf
     }
 }
 
-// Tiles of 32 MT rows of x and 32 NT rows of weights a workgroup of four wavefronts, K in stages of 64 through two LDS buffers;
-// x is split once, on its way into LDS.  A row of a stage is 128 bytes, its 16-byte pieces exchanged by the row's number so
+// Tiles of 16 MT rows of x and 16 NT rows of weights a wavefront, WM by WN wavefronts a workgroup, K in stages of 64 through two LDS
+// buffers; x is split once, on its way into LDS.  A row of a stage is 128 bytes, its 16-byte pieces exchanged by the row's number so
 // that reads of a fragment's sixteen rows meet every bank equally.  What bounds a tile is its chain of stages, each the
-// split (as many cycles of the vector units as the matrix cores take for it), LDS both ways and a barrier: 0.4 us for
-// 32 x 32, 0.7 for 64 x 64, 0.95 for 64 x 128.
+// split (half as many cycles of the vector units as the matrix cores take for it), LDS both ways and a barrier: 0.4 us for 32 x 32, 0.8 for
+// 64 x 128 with eight wavefronts (0.95 with four), 1.65 for 128 x 192.
 #define FT_BK 64
-// A thread's share of a stage on its way through registers: 16 bytes of bfloat16 (8 k) of rows row + 32 i.
-template <int MT, int NT>
+// A thread's share of a stage on its way through registers: 16 bytes of bfloat16 (8 k) of rows row + THREADS / 8 i.
+template <int XN, int WR, int THREADS>
 struct TileStage {
-    float4 lo[MT], hi[MT];
-    uint4 w[NT];
-    __device__ __forceinline__ void fetch(const float* const (&xp)[MT], const bf16_t* const (&wp)[NT], int k) {
+    float4 lo[XN], hi[XN];
+    uint4 w[WR];
+    __device__ __forceinline__ void fetch(const float* const (&xp)[XN], const bf16_t* const (&wp)[WR], int k) {
 #pragma unroll
-        for (int i = 0; i < MT; ++i) {
+        for (int i = 0; i < XN; ++i) {
             lo[i] = *reinterpret_cast<const float4*>(xp[i] + k);
             hi[i] = *reinterpret_cast<const float4*>(xp[i] + k + 4);
         }
 #pragma unroll
-        for (int i = 0; i < NT; ++i) w[i] = *reinterpret_cast<const uint4*>(wp[i] + k);
+        for (int i = 0; i < WR; ++i) w[i] = *reinterpret_cast<const uint4*>(wp[i] + k);
     }
     __device__ __forceinline__ void store(uint4* xs, uint4* ws, int slot, int plane, uint32_t keep) const {
 #pragma unroll
-        for (int i = 0; i < MT; ++i) {
+        for (int i = 0; i < XN; ++i) {
             uint4 a, b, c;
             split8(lo[i], hi[i], a, b, c);
-            xs[slot + 256 * i] = make_uint4(a.x & keep, a.y & keep, a.z & keep, a.w & keep);
-            xs[plane + slot + 256 * i] = make_uint4(b.x & keep, b.y & keep, b.z & keep, b.w & keep);
-            xs[2 * plane + slot + 256 * i] = make_uint4(c.x & keep, c.y & keep, c.z & keep, c.w & keep);
+            xs[slot + THREADS * i] = make_uint4(a.x & keep, a.y & keep, a.z & keep, a.w & keep);
+            xs[plane + slot + THREADS * i] = make_uint4(b.x & keep, b.y & keep, b.z & keep, b.w & keep);
+            xs[2 * plane + slot + THREADS * i] = make_uint4(c.x & keep, c.y & keep, c.z & keep, c.w & keep);
         }
 #pragma unroll
-        for (int i = 0; i < NT; ++i) ws[slot + 256 * i] = w[i];
+        for (int i = 0; i < WR; ++i) ws[slot + THREADS * i] = w[i];
     }
 };
 
 template <int MT, int NT>
-__device__ __forceinline__ void multiply_stage(f32_floatx4 (&acc)[MT][NT][3], const uint4* xs, const uint4* ws, int plane, int wm,
+__device__ __forceinline__ void multiply_stage(f32_floatx4 (&acc)[MT][NT][2], const uint4* xs, const uint4* ws, int plane, int wm,
                                                int wn, int r, int g) {
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
@@ -112,20 +113,20 @@ __device__ __forceinline__ void multiply_stage(f32_floatx4 (&acc)[MT][NT][3], co
 #pragma unroll
             for (int q = 0; q < 3; ++q) xf[i][q] = as_bf16x8(xs[q * plane + (wm + 16 * i + r) * 8 + at]);
 #pragma unroll
-        for (int i = 0; i < MT; ++i)
+        for (int q = 2; q >= 0; --q)
 #pragma unroll
-            for (int q = 0; q < 3; ++q)
+            for (int i = 0; i < MT; ++i)
 #pragma unroll
                 for (int j = 0; j < NT; ++j)
-                    acc[i][j][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j], xf[i][q], acc[i][j][q], 0, 0, 0);
+                    acc[i][j][q > 0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j], xf[i][q], acc[i][j][q > 0], 0, 0, 0);
     }
 }
 
-template <int MT, int NT, bool FULL>
-__global__ void __launch_bounds__(256)
+template <int MT, int NT, int WM, int WN, int DEEP, bool FULL>
+__global__ void __launch_bounds__(64 * WM * WN, 2)
 gemm_f32_tile_kernel(float* __restrict__ out, const float* __restrict__ x, const bf16_t* __restrict__ w, int M, int N, int K,
                      int m_tiles, int n_tiles) {
-    constexpr int BM = 32 * MT, BN = 32 * NT;
+    constexpr int BM = 16 * MT * WM, BN = 16 * NT * WN, THREADS = 64 * WM * WN, XN = BM * 8 / THREADS, WR = BN * 8 / THREADS, STEP = THREADS / 8;
     __shared__ uint4 xs[2][3 * BM * 8];
     __shared__ uint4 ws[2][BN * 8];
     // workgroups that read the same weights are a multiple of eight apart, so that they meet in one L2 cache
@@ -133,40 +134,39 @@ gemm_f32_tile_kernel(float* __restrict__ out, const float* __restrict__ x, const
     const int nt = group * 8 + within % 8, m0 = within / 8 * BM, n0 = nt * BN;
     if (nt >= n_tiles) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 15, g = lane >> 4;
-    const int wm = (wave & 1) * 16 * MT, wn = (wave >> 1) * 16 * NT;
-    const int piece = tid & 7, row = tid >> 3;              // of a stage: 16 bytes of bfloat16 (8 k) of rows row + 32 i
-    const float* xp[MT];
-    const bf16_t* wp[NT];
+    const int wm = wave % WM * 16 * MT, wn = wave / WM * 16 * NT;
+    const int piece = tid & 7, row = tid >> 3;              // of a stage: 16 bytes of bfloat16 (8 k) of rows row + STEP i
+    const float* xp[XN];
+    const bf16_t* wp[WR];
 #pragma unroll
-    for (int i = 0; i < MT; ++i) xp[i] = x + (size_t)min(m0 + row + 32 * i, M - 1) * K;
+    for (int i = 0; i < XN; ++i) xp[i] = x + (size_t)min(m0 + row + STEP * i, M - 1) * K;
 #pragma unroll
-    for (int i = 0; i < NT; ++i) wp[i] = w + (size_t)min(n0 + row + 32 * i, N - 1) * K;
-    const int slot = row * 8 + (piece ^ (row & 7));         // (32 rows on, the exchange is the same)
-    f32_floatx4 acc[MT][NT][3];
+    for (int i = 0; i < WR; ++i) wp[i] = w + (size_t)min(n0 + row + STEP * i, N - 1) * K;
+    const int slot = row * 8 + (piece ^ (row & 7));         // (STEP rows on, a multiple of eight, the exchange is the same)
+    f32_floatx4 acc[MT][NT][2];
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
         for (int j = 0; j < NT; ++j)
 #pragma unroll
-            for (int p = 0; p < 3; ++p) acc[i][j][p] = f32_floatx4{0.f, 0.f, 0.f, 0.f};
-    // Two stages are under way in registers while a third is multiplied (one is not enough: a stage of a small tile is multiplied
-    // in a third of the time that its loads take).
-    TileStage<MT, NT> even, odd;
+            for (int p = 0; p < 2; ++p) acc[i][j][p] = f32_floatx4{0.f, 0.f, 0.f, 0.f};
+    // DEEP stages are under way in registers while another is multiplied: a stage of a small tile is multiplied in a fraction of the
+    // time that its loads take.
+    TileStage<XN, WR, THREADS> ahead[DEEP];
     const int stages = (K + FT_BK - 1) / FT_BK;
-    even.fetch(xp, wp, min(8 * piece, K - 8));
-    odd.fetch(xp, wp, min(FT_BK + 8 * piece, K - 8));
-    even.store(xs[0], ws[0], slot, BM * 8, FULL || 8 * piece < K ? ~0u : 0u);
+#pragma unroll
+    for (int d = 0; d < DEEP; ++d) ahead[d].fetch(xp, wp, min(d * FT_BK + 8 * piece, K - 8));
+    ahead[0].store(xs[0], ws[0], slot, BM * 8, FULL || 8 * piece < K ? ~0u : 0u);
     __syncthreads();
-    for (int s = 0; s < stages; s += 2) {
+    for (int s = 0; s < stages; s += DEEP) {
         const int k = s * FT_BK + 8 * piece;                // (beyond K: x counts as zeros where it is stored)
-        even.fetch(xp, wp, min(k + 2 * FT_BK, K - 8));
-        multiply_stage<MT, NT>(acc, xs[0], ws[0], BM * 8, wm, wn, r, g);
-        odd.store(xs[1], ws[1], slot, BM * 8, FULL || k + FT_BK < K ? ~0u : 0u);
-        __syncthreads();
-        odd.fetch(xp, wp, min(k + 3 * FT_BK, K - 8));
-        multiply_stage<MT, NT>(acc, xs[1], ws[1], BM * 8, wm, wn, r, g);
-        even.store(xs[0], ws[0], slot, BM * 8, FULL || k + 2 * FT_BK < K ? ~0u : 0u);
-        __syncthreads();
+#pragma unroll
+        for (int d = 0; d < DEEP; ++d) {
+            ahead[d].fetch(xp, wp, min(k + (d + DEEP) * FT_BK, K - 8));
+            multiply_stage<MT, NT>(acc, xs[d & 1], ws[d & 1], BM * 8, wm, wn, r, g);
+            ahead[(d + 1) % DEEP].store(xs[(d + 1) & 1], ws[(d + 1) & 1], slot, BM * 8, FULL || k + (d + 1) * FT_BK < K ? ~0u : 0u);
+            __syncthreads();
+        }
     }
     const bool four = N % 4 == 0;
     bool bad = false;
@@ -179,7 +179,7 @@ gemm_f32_tile_kernel(float* __restrict__ out, const float* __restrict__ x, const
             float sum[4];
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                sum[e] = acc[i][j][0][e] + (acc[i][j][1][e] + acc[i][j][2][e]) * (1.f / F32_LOWER);
+                sum[e] = acc[i][j][0][e] + acc[i][j][1][e] * (1.f / F32_LOWER);
                 bad |= !(fabsf(sum[e]) < INFINITY);
             }
             float* o = out + (size_t)m * N + n;
@@ -192,12 +192,13 @@ gemm_f32_tile_kernel(float* __restrict__ out, const float* __restrict__ x, const
     if (bad) chain_again<MT, NT>(out, x, w, m0 + wm + r, n0 + wn + 4 * g, M, N, K);
 }
 
-template <int MT, int NT>
+template <int MT, int NT, int WM, int WN, int DEEP>
 static void launch_tiles(float* out, const float* x, const bf16_t* w, int m, int n, int k, hipStream_t s) {
-    const int m_tiles = (m + 32 * MT - 1) / (32 * MT), n_tiles = (n + 32 * NT - 1) / (32 * NT);
+    constexpr int BM = 16 * MT * WM, BN = 16 * NT * WN;
+    const int m_tiles = (m + BM - 1) / BM, n_tiles = (n + BN - 1) / BN;
     const int grid = (n_tiles + 7) / 8 * 8 * m_tiles;
-    if (k % (2 * FT_BK) == 0) gemm_f32_tile_kernel<MT, NT, true><<<grid, 256, 0, s>>>(out, x, w, m, n, k, m_tiles, n_tiles);
-    else gemm_f32_tile_kernel<MT, NT, false><<<grid, 256, 0, s>>>(out, x, w, m, n, k, m_tiles, n_tiles);
+    if (k % (DEEP * FT_BK) == 0) gemm_f32_tile_kernel<MT, NT, WM, WN, DEEP, true><<<grid, 64 * WM * WN, 0, s>>>(out, x, w, m, n, k, m_tiles, n_tiles);
+    else gemm_f32_tile_kernel<MT, NT, WM, WN, DEEP, false><<<grid, 64 * WM * WN, 0, s>>>(out, x, w, m, n, k, m_tiles, n_tiles);
 }
 
 #define GT_M 64
@@ -254,17 +255,21 @@ extern "C" int ri_gemm_f32(float* out, const float* x, const void* w, int w_dtyp
     else if (!aligned)
         gemm_f32_kernel<bf16_t><<<grid, 256, 0, s>>>(out, x, (const bf16_t*)w, m, n, k);
     else {
-        // A tile's time grows more slowly than its work: tiles of 64 x 128 where they still give every compute unit a workgroup, else
-        // 32 x 64 as soon as 32 x 32 would need a second round of workgroups.
-        // 759 rows, us for 32 x 32 / 32 x 64 / 64 x 128: 1,024 x 3,072 37 / 34 / 48, 4,096 x 1,024 46 / 32 / 31, 6,144 x 1,024
-        // 64 / 45 / 46 (the vector units' form: 363, 127, 176); 33 rows of 1,024 x 3,072 19 / 23 / 46, 2,048 rows 110 / 64 / 55.
-        // Up to 32 rows half of a tile of 64 would be padding: 151,936 x 1,024 at one row 77 / 57 / 75 (302).
+        // The order of a row's sums is the same in every tile.  The largest tiles, 128 x 192, where their last round of workgroups (one a
+        // compute unit) leaves little of the machine idle; 64 x 128 from three quarters of the machine on, else 32 x 64 as soon as 32 x 32
+        // would need a second round.  us for 32 x 32 / 32 x 64 / 64 x 128 / 128 x 192 (rows; columns x K): 759; 6,144 x 1,024 60 / 44 / 46 /
+        // 38, 4,096 x 1,024 43 / 32 / 31 / 36, 1,024 x 3,072 33 / 30 / 39 / 83; 1,200; 4,096 x 1,024 65 / 54 / 53 / 43, 6,144 x 1,024 102 / 73 / 60 / 77;
+        // 400; 4,096 x 1,024 27 / 22 / 18 / 35, 6,144 x 1,024 37 / 28 / 30 / 37; 200; 4,096 x 1,024 17 / 14 / 17 / 34; 2,400; 6,144 x 1,024 252 / 149 /
+        // 121 / 117; 33; 1,024 x 3,072 20 / 22 / 38 / 80, 4,096 x 1,024 8.8 / 9.6 / 16 / 30 (the vector units' form: 759; 1,024 x 3,072 363).
+        // Up to 32 rows half of a tile of 64 would be padding: 151,936 x 1,024 at one row 77 / 57 / 75.
         const auto tiles = [&](int rows, int cols) { return (long)((m + rows - 1) / rows) * ((n + cols - 1) / cols); };
         const bf16_t* wb = (const bf16_t*)w;
         RI_REQUIRE(tiles(32, 32) + 8 * ((m + 31) / 32) < (1L << 31), "gemm_f32: %d x %d exceed one launch", m, n);
-        if (m > 32 && tiles(64, 128) >= ri_compute_units()) launch_tiles<2, 4>(out, x, wb, m, n, k, s);
-        else if (tiles(32, 32) > ri_compute_units()) launch_tiles<1, 2>(out, x, wb, m, n, k, s);
-        else launch_tiles<1, 1>(out, x, wb, m, n, k, s);
+        const long units = ri_compute_units(), largest = tiles(128, 192), rounds = (largest + units - 1) / units;
+        if (m > 64 && 10 * largest >= 7 * rounds * units) launch_tiles<2, 6, 4, 2, 2>(out, x, wb, m, n, k, s);
+        else if (m > 32 && 4 * tiles(64, 128) >= 3 * units) launch_tiles<2, 2, 2, 4, 2>(out, x, wb, m, n, k, s);
+        else if (tiles(32, 32) > units) launch_tiles<1, 2, 2, 2, 2>(out, x, wb, m, n, k, s);
+        else launch_tiles<1, 1, 2, 2, 4>(out, x, wb, m, n, k, s);
     }
     RI_LAUNCH_CHECK("gemm_f32");
     return 0;

@@ -831,6 +831,18 @@ def test_gemm_f32_on_the_matrix_cores(ops, m, n, k):
     assert np.array_equal(got[m // 2:], f64(some)), "a row's sums depend on the other rows"
 
 
+@pytest.mark.parametrize("m,n,k", [(385, 4096, 200), (1153, 4096, 64), (1200, 4096, 392), (31, 4096, 328)])
+def test_gemm_f32_tiles_of_a_full_machine(ops, m, n, k):
+    """The tiles that a whole machine chooses, 64 x 128 and 128 x 192, their edges and stages that are not whole, and the smallest ones'
+    four stages; the bound of the test above."""
+    rng = np.random.default_rng(m + n + k)
+    x, w = t(rng.normal(size=(m, k))), t(rng.normal(size=(n, k)), torch.bfloat16)
+    got = f64(ops.gemm_f32(x, w))
+    bound = (k / 32 + 32) * 2.0 ** -24 * (np.abs(f64(x)) @ np.abs(f64(w)).T)
+    assert (np.abs(got - f64(x) @ f64(w).T) <= bound).all()
+    assert np.array_equal(got[m - 30:], f64(ops.gemm_f32(x[m - 30:].contiguous(), w))), "a row's sums depend on the other rows"
+
+
 @pytest.mark.parametrize("top", [-100, -112, -118, -126, -135])
 def test_gemm_f32_of_the_smallest_numbers(ops, top):
     """x down to the smallest float32, subnormal numbers among them: no bit of it is lost.  The bound of the test above, and half the
