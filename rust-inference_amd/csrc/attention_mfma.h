@@ -414,12 +414,12 @@ attn_prefill_mfma_kernel(bf16_t* __restrict__ out, const bf16_t* __restrict__ qk
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     // The kv head is the fastest grid index: consecutive workgroups go to consecutive XCDs, so the
     // workgroups that walk the same keys and values (one kv head of one sequence) meet in one XCD's L2.
-    const int kvh = blockIdx.x, b = blockIdx.z;
+    const int kvh = blockIdx.x, b = blockIdx.y;
     const int group = heads / kv_heads;
     const int tile_tokens = (16 * NT) / group;               // tokens per wavefront
     const int t_end = cu_seqlens[b + 1];
-    // the last tokens of a sequence see the most keys: their workgroups are launched first
-    const int t_wg = cu_seqlens[b] + (int)(gridDim.y - 1 - blockIdx.y) * 4 * tile_tokens;
+    // the last tokens of a sequence see the most keys: the workgroups of all sequences' last tokens are launched first
+    const int t_wg = cu_seqlens[b] + (int)(gridDim.z - 1 - blockIdx.z) * 4 * tile_tokens;
     if (t_wg >= t_end) return;                               // the whole workgroup leaves
     const int t0 = t_wg + wave * tile_tokens;
     const int nt = max(0, min(tile_tokens, t_end - t0));     // a wavefront without tokens still helps to fetch

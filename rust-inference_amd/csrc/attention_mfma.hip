@@ -60,7 +60,7 @@ extern "C" int ri_attention_prefill_kept_bf16(void* out, const void* qkv, int q_
     const int tile_tokens = (16 * nt_tiles) / group;
     const int tiles = (max_new + 4 * tile_tokens - 1) / (4 * tile_tokens);
     RI_REQUIRE(tiles <= 65535, "attention_prefill_bf16: %d tiles of tokens exceed one launch", tiles);
-    dim3 grid(kv_heads, tiles, seqs);
+    dim3 grid(kv_heads, seqs, tiles);
     const float scale_log2 = scale * 1.4426950408889634f;
     hipStream_t s = (hipStream_t)stream;
 #define RI_PREFILL_CASE(DH, NT)                                                                                  \
