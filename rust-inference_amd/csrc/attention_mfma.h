@@ -144,6 +144,7 @@ struct Columns {
     // column's slope over the scale, so that it too acts on the raw products; all 0 (biased false): none
     float bias[NT];
     bool biased;
+    bool capped;                  // (the cap is known to be there: no look at cap_pre)
 };
 
 // tanh through one exponential: 1 - 2 / (e^(2x) + 1), exact at both ends (e^(2x) = inf or 0).
@@ -253,7 +254,7 @@ __device__ __forceinline__ void init_columns(Columns<DH, NT, DV>& c) {
         c.keep = 0;
         c.cap_pre = c.cap_post = 0.f;
         c.bias[j] = 0.f;
-        c.biased = false;
+        c.biased = c.capped = false;
 #pragma unroll
         for (int ks = 0; ks < DH / 32; ++ks) c.q[j][ks].u = make_uint4(0, 0, 0, 0);
 #pragma unroll
@@ -279,7 +280,7 @@ __device__ __forceinline__ void scores_of(const Columns<DH, NT, DV>& c, const Fr
             s[j][e] = s0[e];
             s[j][4 + e] = s1[e];
         }
-        if (c.cap_pre != 0.f) cap_scores(s[j], c.cap_pre, c.cap_post);
+        if (c.capped || c.cap_pre != 0.f) cap_scores(s[j], c.cap_pre, c.cap_post);
         if (c.biased) bias_scores(s[j], c.bias[j], c.qpos[j], page * PAGE + (lane >> 4) * 8);
     }
 }
@@ -396,7 +397,12 @@ __device__ __forceinline__ void value_frags_from_lds(Frag (&vf)[DV / 16], const 
         vf[dt].u = *reinterpret_cast<const uint4*>(v_lds + (dt * 16 + i) * LdsPage<DV>::VS + jg * 8);
 }
 
-template <int DH, int NT, int DV = DH, bool PAD = false>
+// FORM says which changes of a score the launch has, so that a turn without them has no branch in it and is scheduled whole: none
+// (PREFILL_PLAIN), the cap alone, or whatever the arguments say.
+#define PREFILL_PLAIN 0
+#define PREFILL_CAPPED 1
+#define PREFILL_ANY 2
+template <int DH, int NT, int DV = DH, bool PAD = false, int FORM = PREFILL_ANY>
 __global__ void __launch_bounds__(256, 2)
 attn_prefill_mfma_kernel(bf16_t* __restrict__ out, const bf16_t* __restrict__ qkv, int q_stride,
                          const bf16_t* __restrict__ k_pages, const bf16_t* __restrict__ v_pages,
@@ -426,9 +432,10 @@ attn_prefill_mfma_kernel(bf16_t* __restrict__ out, const bf16_t* __restrict__ qk
 
     Columns<DH, NT, DV> c;
     init_columns<DH, NT, DV>(c);
-    c.cap_pre = cap_pre;
+    c.cap_pre = FORM == PREFILL_PLAIN ? 0.f : cap_pre;
     c.cap_post = cap_post;
-    c.biased = slopes != nullptr;
+    c.biased = FORM == PREFILL_ANY && slopes != nullptr;
+    c.capped = FORM == PREFILL_CAPPED;
     c.keep = reach.window > 0 ? keep_first : 0;
     const int jg = lane >> 4;
     float sink[NT];                                          // the column's sink in the exponents' units; -inf: none
@@ -436,7 +443,7 @@ attn_prefill_mfma_kernel(bf16_t* __restrict__ out, const bf16_t* __restrict__ qk
     for (int j = 0; j < NT; ++j) {
         const int col = j * 16 + (lane & 15);
         const int tl = col / group, g = col - tl * group;
-        if (slopes) c.bias[j] = slopes[kvh * group + g] * inv_scale;
+        if (FORM == PREFILL_ANY && slopes) c.bias[j] = slopes[kvh * group + g] * inv_scale;
         sink[j] = sinks ? sinks[kvh * group + g] * 1.4426950408889634f : -INFINITY;
         if (tl < nt) {
             const int tok = t0 + tl;
@@ -471,7 +478,7 @@ attn_prefill_mfma_kernel(bf16_t* __restrict__ out, const bf16_t* __restrict__ qk
     constexpr bool TWO = LdsPage<DH>::PER_THREAD > 1;
     constexpr int VN = LdsPage<DH, DV>::V_PER_THREAD;
     const int c0 = threadIdx.x;
-    const bool has0 = c0 < LdsPage<DH>::CHUNKS;
+    const bool has0 = LdsPage<DH>::CHUNKS >= 256 || c0 < LdsPage<DH>::CHUNKS;
     uint4 sk0 = make_uint4(0, 0, 0, 0), sk1 = sk0, sv0 = sk0, sv1 = sk0, sv2 = sk0, sv3 = sk0;
     // a piece of the key page: row c / (DH / 8), columns 8 (c % (DH / 8)) ..+8 (with PAD those behind dim stay zero)
     auto key_piece = [&](int c) -> int { return PAD ? (c / (DH / 8)) * dim + (c % (DH / 8)) * 8 : c * 8; };
@@ -501,9 +508,14 @@ attn_prefill_mfma_kernel(bf16_t* __restrict__ out, const bf16_t* __restrict__ qk
     // Every wavefront takes every page of the workgroup (those outside its own tokens' sight are masked
     // whole and add nothing), and the page numbers of the loads are clamped: no branch in a turn but the mask
     // and the move of the reference point, so that each half of a turn is one stretch of code to schedule.
+    // A turn's keys come from the page looked up in the turn before, its values from the turn's before that one: no load waits
+    // for a look into the table.
+    int page_v = table[RI_PG(0)], page_k = table[RI_PG(min(1, w_last))];
 #define RI_TURN_LOADS(W)                                                                             \
-    RI_STAGE_LOAD_K(table[RI_PG(min((W) + 2, w_last))]);                                             \
-    RI_STAGE_LOAD_V(table[RI_PG(min((W) + 1, w_last))]);
+    RI_STAGE_LOAD_K(page_k);                                                                         \
+    RI_STAGE_LOAD_V(page_v);                                                                         \
+    page_v = page_k;                                                                                 \
+    page_k = table[RI_PG(min((W) + 3, w_last))];
 #define RI_TURN_STORES(I)                                                                            \
     {                                                                                                \
         if (has0) stage_store_key<DH>(k_lds[((I) & 1) ^ 1], c0, sk0);                                \
@@ -515,7 +527,7 @@ attn_prefill_mfma_kernel(bf16_t* __restrict__ out, const bf16_t* __restrict__ qk
         __syncthreads();                /* what arrived is in place; what was read may be overwritten */ \
     }
 #define RI_PAGE_OPEN(W) ((W) >= nk && RI_PG(W) * PAGE + PAGE - 1 <= min_qpos && RI_PG(W) * PAGE >= max_lo)
-    RI_STAGE_LOAD_K(table[RI_PG(0)]);
+    RI_STAGE_LOAD_K(page_v);
     {
         if (has0) stage_store_key<DH>(k_lds[0], c0, sk0);
         if (TWO) stage_store_key<DH>(k_lds[0], c0 + 256, sk1);

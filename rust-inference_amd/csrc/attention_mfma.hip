@@ -63,12 +63,17 @@ extern "C" int ri_attention_prefill_kept_bf16(void* out, const void* qkv, int q_
     dim3 grid(kv_heads, seqs, tiles);
     const float scale_log2 = scale * 1.4426950408889634f;
     hipStream_t s = (hipStream_t)stream;
+    const int form = slopes ? PREFILL_ANY : cap_pre != 0.f ? PREFILL_CAPPED : PREFILL_PLAIN;
+#define RI_PREFILL_GO(DH, NT, FORM)                                                                              \
+    attn_prefill_mfma_kernel<DH, NT, DH, false, FORM><<<grid, 256, 0, s>>>(                                      \
+        (bf16_t*)out, (const bf16_t*)qkv, q_stride, (const bf16_t*)k_pages, (const bf16_t*)v_pages,              \
+        cu_seqlens, tok_pos, page_table, table_width, heads, kv_heads, reach, scale_log2, cap_pre,              \
+        cap_post, slopes, 1.f / scale, keep_first, sinks)
 #define RI_PREFILL_CASE(DH, NT)                                                                                  \
     case DH * 8 + NT:                                                                                            \
-        attn_prefill_mfma_kernel<DH, NT><<<grid, 256, 0, s>>>(                                                   \
-            (bf16_t*)out, (const bf16_t*)qkv, q_stride, (const bf16_t*)k_pages, (const bf16_t*)v_pages,          \
-            cu_seqlens, tok_pos, page_table, table_width, heads, kv_heads, reach, scale_log2, cap_pre,          \
-            cap_post, slopes, 1.f / scale, keep_first, sinks);                                                   \
+        if (form == PREFILL_PLAIN) RI_PREFILL_GO(DH, NT, PREFILL_PLAIN);                                         \
+        else if (form == PREFILL_CAPPED) RI_PREFILL_GO(DH, NT, PREFILL_CAPPED);                                  \
+        else RI_PREFILL_GO(DH, NT, PREFILL_ANY);                                                                 \
         break;
     switch (head_dim * 8 + nt_tiles) {
         RI_PREFILL_CASE(32, 4)
@@ -81,6 +86,7 @@ extern "C" int ri_attention_prefill_kept_bf16(void* out, const void* qkv, int q_
         RI_PREFILL_CASE(128, 1)
     }
 #undef RI_PREFILL_CASE
+#undef RI_PREFILL_GO
     RI_LAUNCH_CHECK("attention_prefill_bf16");
     return 0;
 }
