@@ -124,7 +124,12 @@ int ri_decay_step(float* out, const void* proj, int act_dtype, int row, int q_of
 // chunk, every chunk's outputs), where ri_decay_chunks_fit says the head sizes are taken (multiples of 4 up to 128;
 // the offsets and the row multiples of 4 too).  max_new: the most new tokens of a sequence; workspace: float32 of at
 // least ri_decay_chunks_workspace(...) floats.  The results differ from ri_decay_scan's by rounding alone.
+// ri_ssd_scan_chunked: the same of the state-space mixer's walk (ssd.hip), with the same sizes and workspace.
 int ri_decay_chunks_fit(int dim, int vdim);
+int ri_ssd_scan_chunked(float* out, const float* xbc, int channels, int b_off, int c_off, const void* proj, int act_dtype, int stride,
+                        int z_off, int dt_off, const float* dt_bias, const float* a_log, const float* d_skip, float* state,
+                        const int32_t* cu_seqlens, const int32_t* slots, int seqs, int tokens, int max_new, int heads, int groups, int n,
+                        int vdim, float* workspace, long workspace_floats, void* stream);
 long ri_decay_chunks_workspace(int seqs, int tokens, int heads, int dim, int vdim);
 int ri_decay_scan_chunked(float* out, const void* proj, int act_dtype, int row, int q_off, int k_off, int v_off,
                           const float* head_decay, float q_scale, float* state, const int32_t* cu_seqlens,

@@ -1,25 +1,31 @@
-// Linear attention with one fixed decay per head over prompts, in chunks of 64 tokens instead of token by token:
-//     S_t = d S_(t-1) + k_t v_t^T,   o_t = S_t^T q_t,   q = silu(.) * q_scale, k = silu(.), v = silu(.).
-// With a decay that is a constant the tokens of a chunk need not wait for one another.  For a chunk of n tokens that
-// starts from the state S0,
-//     o_i   = sum_{j <= i} d^(i - j) (q_i . k_j) v_j  +  d^(i + 1) S0^T q_i,
-//     S_end = d^n S0 + sum_j d^(n - 1 - j) k_j v_j^T,
-// so a step is three launches: every chunk's own sum U = sum_j d^(n - 1 - j) k_j v_j^T (all chunks side by side), the
-// walk from chunk to chunk, S0 of the next = d^n S0 + U, which leaves every chunk's S0 where its U was and the last
+// Recurrences whose decay is one number a head and token over prompts, in chunks of 64 tokens instead of token by token:
+//     S_t = d_t S_(t-1) + k_t v_t^T,   o_t = S_t^T q_t,
+// linear attention with a fixed decay (d_t = d_h; q = silu(.) * q_scale, k = silu(.), v = silu(.)) and the state-space mixer
+// (ssd.hip: d_t = exp(-exp(A_log_h) dt_t), q = C, k = B, v = dt x; y = o + D x, times silu(z)).
+// The tokens of a chunk need not wait for one another.  With D(i, j) = d_(j+1) ... d_i, for a chunk of n tokens from the state S0,
+//     o_i   = sum_{j <= i} D(i, j) (q_i . k_j) v_j  +  D(i, -1) S0^T q_i,
+//     S_end = D(n - 1, -1) S0 + sum_j D(n - 1, j) k_j v_j^T,
+// so a step is three launches: every chunk's own sum U = sum_j D(n - 1, j) k_j v_j^T (all chunks side by side), the
+// walk from chunk to chunk, S0 of the next = D S0 + U, which leaves every chunk's S0 where its U was and the last
 // state in the sequence's slot (a few loads and stores an element), and every chunk's outputs (all chunks side by side).
-// Only powers d^m with m >= 0 appear, so no decay is too small or too large for it.  Everything is float32: the
-// activations after silu, the powers, the scores q . k, the state and all sums; a sum runs over its tokens or channels
-// in their order.  A workgroup of 512 threads takes one (chunk, sequence, head); a thread keeps tiles of 4 x 4 results
-// and reads its operands from LDS 16 bytes at a time.  Head sizes: multiples of 4 up to 128.
+// Only products of decays from an earlier token to a later one appear, never their inverses: the powers d^m, m >= 0, of a fixed decay, and
+// exp of a difference of sums of -exp(A_log) dt, which are added up in 64 bits so that the difference keeps every bit
+// of a float32.  Everything else is float32: the activations, the scores q . k, the state and all sums; the products run on the matrix
+// cores' float32 product (16x16x4), whose products and sums are 32-bit ones.  A workgroup of eight wavefronts takes one (chunk,
+// sequence, head), a wavefront sixteen columns of the results (sixteen rows of a chunk's own sum): what only its columns need comes straight
+// from memory, once, and what all need (q and k, the scores, v) passes through LDS.  What bounds it: the products, some 230 of 32
+// cycles a wavefront and chunk, and two trips to memory.  Fixed decay, 32 heads of 128 x 128, four prompts of 300 to
+// 1,800 tokens, us on the vector units : so: sums 136 : 101, outputs 357 : 163 (the carry 65 : 70).
+// Head sizes: multiples of 4 up to 128.
 #include "api.h"
 #include "common.h"
 
 #define DC_TOK 64                // tokens of a chunk
 #define DC_MAX 128               // largest key or value head
-#define DC_SLAB 32               // rows of S0 staged at a time
+#define DC_STRIDE (DC_MAX + 4)   // of the rows of q and k, and of v, in LDS
 #define DC_ASTRIDE (DC_TOK + 4)
-#define DC_THREADS 512           // of the workgroups that work on a chunk: two wavefronts a SIMD, one behind the other's loads
-#define DC_STAGED (DC_TOK * DC_MAX / 4 / DC_THREADS)    // most 16-byte pieces a thread stages of one operand
+#define DC_THREADS 512           // of the workgroups that work on a chunk: a wavefront for sixteen of 128 columns
+typedef __attribute__((__vector_size__(4 * sizeof(float)))) float dc_floatx4;
 
 __device__ __forceinline__ float dc_silu(float v) { return v / (1.0f + expf(-v)); }
 
@@ -34,115 +40,166 @@ __device__ __forceinline__ float4 dc_ld4(const bf16_t* p) {
 // meet, since a sequence of len tokens has at most len / 64 + 1 chunks.
 __device__ __forceinline__ size_t dc_entry(int t0, int b, int c) { return (size_t)(t0 / DC_TOK + b + c); }
 
-// Rows of `width` activations of tokens first .. first + n - 1 (columns col0 .. of proj's rows) through silu into LDS
-// rows of `stride` floats, times factor * d^(n - 1 - j) with pw (pw == nullptr: times factor alone); rows n .. 63 zero.
-// Loads are issued whatever the indices are, from a token pulled back inside the chunk.
+// Where a head's q, k and v come from, and its decays.  `made` is the workgroup's: the powers of a fixed decay, or the sums of the
+// exponents and the step sizes.
+struct DcMade {
+    double sums[DC_TOK];
+    float powers[DC_TOK + 1], dt[DC_TOK];
+};
+
 template <typename TA>
-__device__ __forceinline__ void dc_stage(float* dst, int stride, const TA* __restrict__ proj, int row, int col0, int first,
-                                         int n, int width, float factor, const float* pw) {
-    const int per = width / 4, total = DC_TOK * per;
-    float4 x[DC_STAGED];
-    int tok[DC_STAGED], at[DC_STAGED];
-    // all of a thread's loads are asked for before the first is used
-#pragma unroll
-    for (int it = 0; it < DC_STAGED; ++it) {
-        const int e = min((int)threadIdx.x + it * DC_THREADS, total - 1);
-        tok[it] = e / per;
-        at[it] = (e - tok[it] * per) * 4;
-        x[it] = dc_ld4(proj + (size_t)(first + min(tok[it], n - 1)) * row + col0 + at[it]);
+struct DcFixed {
+    const TA* proj;
+    int row, q_off, k_off, v_off;
+    const float* head_decay;
+    float q_scale;
+    __device__ __forceinline__ float4 q4(int t, int h, int dim, int k) const {
+        const float4 v = dc_ld4(proj + (size_t)t * row + q_off + h * dim + k);
+        return make_float4(dc_silu(v.x) * q_scale, dc_silu(v.y) * q_scale, dc_silu(v.z) * q_scale, dc_silu(v.w) * q_scale);
     }
-#pragma unroll
-    for (int it = 0; it < DC_STAGED; ++it) {
-        if ((int)threadIdx.x + it * DC_THREADS < total) {
-            const int j = tok[it];
-            const float f = j < n ? factor * (pw ? pw[n - 1 - j] : 1.0f) : 0.f;
-            float4 y;
-            y.x = j < n ? dc_silu(x[it].x) * f : 0.f;
-            y.y = j < n ? dc_silu(x[it].y) * f : 0.f;
-            y.z = j < n ? dc_silu(x[it].z) * f : 0.f;
-            y.w = j < n ? dc_silu(x[it].w) * f : 0.f;
-            *reinterpret_cast<float4*>(dst + j * stride + at[it]) = y;
+    __device__ __forceinline__ float4 k4(int t, int h, int dim, int k) const {
+        const float4 v = dc_ld4(proj + (size_t)t * row + k_off + h * dim + k);
+        return make_float4(dc_silu(v.x), dc_silu(v.y), dc_silu(v.z), dc_silu(v.w));
+    }
+    __device__ __forceinline__ float4 v4(int t, int, int h, int vdim, int c, const DcMade&) const {
+        const float4 v = dc_ld4(proj + (size_t)t * row + v_off + h * vdim + c);
+        return make_float4(dc_silu(v.x), dc_silu(v.y), dc_silu(v.z), dc_silu(v.w));
+    }
+    __device__ __forceinline__ float k1(int t, int h, int dim, int k) const { return dc_silu(to_f32(proj[(size_t)t * row + k_off + h * dim + k])); }
+    __device__ __forceinline__ float v1(int t, int, int h, int vdim, int c, const DcMade&) const {
+        return dc_silu(to_f32(proj[(size_t)t * row + v_off + h * vdim + c]));
+    }
+    __device__ __forceinline__ void make(DcMade& made, int, int, int h) const {
+        const int m = threadIdx.x;                           // (d^0 = 1 also for d = 0)
+        if (m <= DC_TOK) made.powers[m] = m == 0 ? 1.0f : powf(head_decay[h], (float)m);
+        __syncthreads();
+    }
+    __device__ __forceinline__ float between(const DcMade& made, int i, int j) const { return made.powers[i - j]; }
+    __device__ __forceinline__ float from_start(const DcMade& made, int i) const { return made.powers[i + 1]; }
+    __device__ __forceinline__ float finish(float o, int, int, int, int) const { return o; }
+};
+
+template <typename TA>
+struct DcSteps {
+    const float* xbc;
+    int channels, b_off, c_off;
+    const TA* proj;
+    int stride, z_off, dt_off;
+    const float *dt_bias, *a_log, *d_skip;
+    int share;                                               // heads that read one B and C
+    __device__ __forceinline__ float4 q4(int t, int h, int dim, int k) const {
+        return dc_ld4(xbc + (size_t)t * channels + c_off + h / share * dim + k);
+    }
+    __device__ __forceinline__ float4 k4(int t, int h, int dim, int k) const {
+        return dc_ld4(xbc + (size_t)t * channels + b_off + h / share * dim + k);
+    }
+    __device__ __forceinline__ float4 v4(int t, int j, int h, int vdim, int c, const DcMade& made) const {
+        const float4 v = dc_ld4(xbc + (size_t)t * channels + h * vdim + c);
+        const float dt = made.dt[j];
+        return make_float4(dt * v.x, dt * v.y, dt * v.z, dt * v.w);
+    }
+    __device__ __forceinline__ float k1(int t, int h, int dim, int k) const { return xbc[(size_t)t * channels + b_off + h / share * dim + k]; }
+    __device__ __forceinline__ float v1(int t, int j, int h, int vdim, int c, const DcMade& made) const {
+        return made.dt[j] * xbc[(size_t)t * channels + h * vdim + c];
+    }
+    __device__ __forceinline__ void make(DcMade& made, int first, int n, int h) const {
+        const int i = threadIdx.x;
+        if (i < DC_TOK) {
+            const float raw = to_f32(proj[(size_t)(first + min(i, n - 1)) * stride + dt_off + h]) + (dt_bias ? dt_bias[h] : 0.f);
+            made.dt[i] = raw > 20.f ? raw : log1pf(expf(raw));           // softplus: beyond 20 it is its argument to the last bit
         }
+        __syncthreads();
+        if (i < DC_TOK) {
+            const float neg_a = -expf(a_log[h]);
+            double sum = 0.0;
+            for (int j = 0; j <= i; ++j) sum += (double)(neg_a * made.dt[j]);
+            made.sums[i] = sum;
+        }
+        __syncthreads();
     }
-}
+    __device__ __forceinline__ float between(const DcMade& made, int i, int j) const {
+        return i == j ? 1.0f : expf((float)(made.sums[i] - made.sums[j]));
+    }
+    __device__ __forceinline__ float from_start(const DcMade& made, int i) const { return expf((float)made.sums[i]); }
+    __device__ __forceinline__ float finish(float o, int t, int h, int vdim, int c) const {
+        if (d_skip) o += d_skip[h] * xbc[(size_t)t * channels + h * vdim + c];
+        const float z = to_f32(proj[(size_t)t * stride + z_off + h * vdim + c]);
+        return o * (z / (1.f + expf(-z)));
+    }
+};
 
-// pw[m] = d^m for m = 0 .. 64 (d^0 = 1 also for d = 0).
-__device__ __forceinline__ void dc_powers(float* pw, float d) {
-    if (threadIdx.x <= DC_TOK) pw[threadIdx.x] = threadIdx.x == 0 ? 1.0f : powf(d, (float)threadIdx.x);
-}
-
-// U[entry, h] = sum_j d^(n - 1 - j) k_j v_j^T   [dim, vdim]
-template <typename TA>
+// U[entry, h] = sum_j D(n - 1, j) k_j v_j^T   [dim, vdim]; wholes[entry, h] = D(n - 1, -1)
+template <typename SRC>
 __global__ void __launch_bounds__(DC_THREADS)
-decay_chunk_sums_kernel(float* __restrict__ U, const TA* __restrict__ proj, int row, int k_off, int v_off,
-                        const int32_t* __restrict__ cu_seqlens, const float* __restrict__ head_decay, int heads, int dim,
-                        int vdim) {
-    extern __shared__ __align__(16) float lds[];           // read 16 bytes at a time: it must start on a multiple of 16,
-    __shared__ __align__(16) float pw[DC_TOK + 4];         // so what stands before it is a multiple of 16 bytes too
-    const int c = blockIdx.x, b = blockIdx.y, h = blockIdx.z;
+decay_chunk_sums_kernel(float* __restrict__ U, float* __restrict__ wholes, SRC src, const int32_t* __restrict__ cu_seqlens, int heads,
+                        int dim, int vdim) {
+    __shared__ __align__(16) float Vs[DC_TOK * DC_STRIDE];
+    __shared__ DcMade made;
+    const int c = blockIdx.x, b = blockIdx.y, h = blockIdx.z, tid = threadIdx.x;
+    const int lane = tid & 63, r = lane & 15, g = lane >> 4, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int t0 = cu_seqlens[b], t1 = cu_seqlens[b + 1];
     const int first = t0 + c * DC_TOK;
     if (first >= t1) return;
     const int n = min(DC_TOK, t1 - first);
-    float* Ks = lds;                       // [64][dim], already times d^(n - 1 - j)
-    float* Vs = lds + DC_TOK * dim;        // [64][vdim]
-    dc_powers(pw, head_decay[h]);
-    __syncthreads();
-    dc_stage(Ks, dim, proj, row, k_off + h * dim, first, n, dim, 1.0f, pw);
-    dc_stage(Vs, vdim, proj, row, v_off + h * vdim, first, n, vdim, 1.0f, (const float*)nullptr);
-    __syncthreads();
-    float* Uc = U + (dc_entry(t0, b, c) * heads + h) * dim * vdim;
-    const int tcs = vdim / 4, tiles = (dim / 4) * tcs;
-    for (int tile = threadIdx.x; tile < tiles; tile += DC_THREADS) {
-        const int tr = tile / tcs, tc = tile - tr * tcs;
-        float acc[4][4] = {};
-        for (int j0 = 0; j0 < n; j0 += 4) {                  // (the rows from n on are zeros)
-            float4 k4[4], v4[4];
+    const int k = 16 * wave + r, kk = min(k, dim - 1);       // this lane's row of the result
+    float kv[4][4];                                          // its keys of tokens 16 b + 4 g + e
 #pragma unroll
-            for (int m = 0; m < 4; ++m) {
-                k4[m] = *reinterpret_cast<const float4*>(Ks + (j0 + m) * dim + 4 * tr);
-                v4[m] = *reinterpret_cast<const float4*>(Vs + (j0 + m) * vdim + 4 * tc);
-            }
+    for (int q = 0; q < 4; ++q)
 #pragma unroll
-            for (int m = 0; m < 4; ++m) {
-                const float kk[4] = {k4[m].x, k4[m].y, k4[m].z, k4[m].w};
+        for (int e = 0; e < 4; ++e) kv[q][e] = src.k1(first + min(16 * q + 4 * g + e, n - 1), h, dim, kk);
+    src.make(made, first, n, h);
+    const int wide = (vdim + 15) / 16 * 16;
+    for (int e = tid; e < DC_TOK * wide / 4; e += DC_THREADS) {
+        const int j = e / (wide / 4), at = e % (wide / 4) * 4;
+        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (j < n && at < vdim) v = src.v4(first + j, j, h, vdim, at, made);
+        *reinterpret_cast<float4*>(Vs + j * DC_STRIDE + at) = v;
+    }
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    acc[r][0] += kk[r] * v4[m].x;
-                    acc[r][1] += kk[r] * v4[m].y;
-                    acc[r][2] += kk[r] * v4[m].z;
-                    acc[r][3] += kk[r] * v4[m].w;
-                }
-            }
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int j = 16 * q + 4 * g + e;
+            kv[q][e] = j < n && k < dim ? kv[q][e] * src.between(made, n - 1, min(j, n - 1)) : 0.f;
         }
+    const size_t entry = dc_entry(t0, b, c) * heads + h;
+    if (tid == 0) wholes[entry] = src.from_start(made, n - 1);
+    __syncthreads();
+    if (16 * wave >= dim) return;
+    float* Uc = U + entry * dim * vdim;
+    for (int ct = 0; ct < wide / 16; ++ct) {
+        dc_floatx4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-            *reinterpret_cast<float4*>(Uc + (size_t)(4 * tr + r) * vdim + 4 * tc) = make_float4(acc[r][0], acc[r][1], acc[r][2], acc[r][3]);
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[q][e], Vs[(16 * q + 4 * g + e) * DC_STRIDE + 16 * ct + r], acc, 0, 0, 0);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (16 * wave + 4 * g + e < dim && 16 * ct + r < vdim) Uc[(size_t)(16 * wave + 4 * g + e) * vdim + 16 * ct + r] = acc[e];
     }
 }
 
 // From chunk to chunk: every chunk's entry gets the state it starts from, the slot the state after the last token.
 __global__ void __launch_bounds__(256)
-decay_chunk_carry_kernel(float* __restrict__ U, float* __restrict__ state, const int32_t* __restrict__ cu_seqlens,
-                         const int32_t* __restrict__ slots, const float* __restrict__ head_decay, int heads, int dim,
-                         int vdim) {
+decay_chunk_carry_kernel(float* __restrict__ U, const float* __restrict__ wholes, float* __restrict__ state,
+                         const int32_t* __restrict__ cu_seqlens, const int32_t* __restrict__ slots, int heads, int dim, int vdim) {
     const int b = blockIdx.y, h = blockIdx.z;
     const int e = (blockIdx.x * 256 + threadIdx.x) * 4, size = dim * vdim;
     const int t0 = cu_seqlens[b], len = cu_seqlens[b + 1] - t0;
     if (e >= size || len <= 0) return;
-    const float d = head_decay[h], whole = powf(d, (float)DC_TOK);
     float* Sp = state + ((size_t)slots[b] * heads + h) * size + e;
     float4 s = *reinterpret_cast<const float4*>(Sp);
     const int chunks = (len + DC_TOK - 1) / DC_TOK;
-    float* Up = U + (dc_entry(t0, b, 0) * heads + h) * size + e;
+    const size_t entry = dc_entry(t0, b, 0) * heads + h;
+    float* Up = U + entry * size + e;
     const size_t step = (size_t)heads * size;
     float4 u = *reinterpret_cast<const float4*>(Up);
     for (int c = 0; c < chunks; ++c) {
         // the next chunk's sum is asked for before this one's place is written (the last chunk asks for its own again)
         const float4 next = *reinterpret_cast<const float4*>(Up + (size_t)min(c + 1, chunks - 1) * step);
         *reinterpret_cast<float4*>(Up + (size_t)c * step) = s;
-        const int n = min(DC_TOK, len - c * DC_TOK);
-        const float f = n == DC_TOK ? whole : powf(d, (float)n);
+        const float f = wholes[entry + (size_t)c * heads];
         s.x = f * s.x + u.x;
         s.y = f * s.y + u.y;
         s.z = f * s.z + u.z;
@@ -152,134 +209,115 @@ decay_chunk_carry_kernel(float* __restrict__ U, float* __restrict__ state, const
     *reinterpret_cast<float4*>(Sp) = s;
 }
 
-// o_i = sum_{j <= i} d^(i - j) (q_i . k_j) v_j + d^(i + 1) S0^T q_i for the tokens of one chunk.
-template <typename TA>
+// o_i = sum_{j <= i} D(i, j) (q_i . k_j) v_j + D(i, -1) S0^T q_i for the tokens of one chunk.
+template <typename SRC>
 __global__ void __launch_bounds__(DC_THREADS)
-decay_chunk_out_kernel(float* __restrict__ out, const float* __restrict__ U, const TA* __restrict__ proj, int row, int q_off,
-                       int k_off, int v_off, const int32_t* __restrict__ cu_seqlens, const float* __restrict__ head_decay,
-                       float q_scale, int heads, int dim, int vdim) {
-    extern __shared__ __align__(16) float lds[];           // read 16 bytes at a time: it must start on a multiple of 16,
-    __shared__ __align__(16) float pw[DC_TOK + 4];         // so what stands before it is a multiple of 16 bytes too
+decay_chunk_out_kernel(float* __restrict__ out, const float* __restrict__ U, SRC src, const int32_t* __restrict__ cu_seqlens, int heads,
+                       int dim, int vdim) {
+    __shared__ __align__(16) float Qs[DC_TOK * DC_STRIDE];
+    __shared__ __align__(16) float Ks[DC_TOK * DC_STRIDE];   // the keys, later the scores times the decays [64][DC_ASTRIDE]
+    __shared__ DcMade made;
+    float* As = Ks;
     const int c = blockIdx.x, b = blockIdx.y, h = blockIdx.z, tid = threadIdx.x;
+    const int lane = tid & 63, r = lane & 15, g = lane >> 4, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int t0 = cu_seqlens[b], t1 = cu_seqlens[b + 1];
     const int first = t0 + c * DC_TOK;
     if (first >= t1) return;
-    const int n = min(DC_TOK, t1 - first);
-    const int qs = dim + 4;                                  // row stride of Q and K
-    float* Qs = lds;                                         // [64][dim + 4]
-    float* KV = Qs + DC_TOK * qs;                            // K [64][dim + 4], later V [64][vdim]
-    float* As = KV + DC_TOK * max(qs, vdim);                 // [64][68]: the scores times the decay's powers
-    float* Ss = As + DC_TOK * DC_ASTRIDE;                    // [32][vdim]: a slab of S0's rows
-    dc_powers(pw, head_decay[h]);
-    dc_stage(Qs, qs, proj, row, q_off + h * dim, first, n, dim, q_scale, (const float*)nullptr);
-    dc_stage(KV, qs, proj, row, k_off + h * dim, first, n, dim, 1.0f, (const float*)nullptr);
-    __syncthreads();
-    {   // scores: thread (ti, tj) takes queries 4 ti .. 4 ti + 3 and keys tj and tj + 32
-        const int ti = tid / 32, tj = tid % 32;
-        float acc[4][2] = {};
-        for (int k = 0; k < dim; k += 4) {
-            float4 q4[4], k4[2];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) q4[r] = *reinterpret_cast<const float4*>(Qs + (4 * ti + r) * qs + k);
-#pragma unroll
-            for (int s = 0; s < 2; ++s) k4[s] = *reinterpret_cast<const float4*>(KV + (tj + 32 * s) * qs + k);
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-#pragma unroll
-                for (int s = 0; s < 2; ++s)
-                    acc[r][s] += q4[r].x * k4[s].x + q4[r].y * k4[s].y + q4[r].z * k4[s].z + q4[r].w * k4[s].w;
+    const int n = min(DC_TOK, t1 - first), wide = (dim + 15) / 16 * 16;
+    for (int e = tid; e < DC_TOK * wide / 4; e += DC_THREADS) {
+        const int j = e / (wide / 4), at = e % (wide / 4) * 4;
+        float4 qv = make_float4(0.f, 0.f, 0.f, 0.f), kv = qv;
+        if (j < n && at < dim) {
+            qv = src.q4(first + j, h, dim, at);
+            kv = src.k4(first + j, h, dim, at);
         }
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-#pragma unroll
-            for (int s = 0; s < 2; ++s) {
-                const int i = 4 * ti + r, j = tj + 32 * s;
-                As[i * DC_ASTRIDE + j] = (j <= i && i < n) ? acc[r][s] * pw[i - min(j, i)] : 0.f;
-            }
+        *reinterpret_cast<float4*>(Qs + j * DC_STRIDE + at) = qv;
+        *reinterpret_cast<float4*>(Ks + j * DC_STRIDE + at) = kv;
     }
-    __syncthreads();                                         // the keys have been read: the values take their place
-    dc_stage(KV, vdim, proj, row, v_off + h * vdim, first, n, vdim, 1.0f, (const float*)nullptr);
+    src.make(made, first, n, h);
     __syncthreads();
-    // results: tiles of 4 tokens x 4 columns, at most one a thread
-    const int tcs = vdim / 4, tiles = (DC_TOK / 4) * tcs;
-    float acc[1][4][4] = {}, from_state[1][4][4] = {};
-#pragma unroll
-    for (int w = 0; w < 1; ++w) {
-        const int tile = tid + w * DC_THREADS;
-        if (tile < tiles) {
-            const int ti = tile / tcs, tc = tile - ti * tcs;
-            for (int j = 0; j < DC_TOK; j += 4) {
-                float4 a4[4], v4[4];
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    a4[r] = *reinterpret_cast<const float4*>(As + (4 * ti + r) * DC_ASTRIDE + j);
-                    v4[r] = *reinterpret_cast<const float4*>(KV + (j + r) * vdim + 4 * tc);
-                }
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const float a[4] = {a4[r].x, a4[r].y, a4[r].z, a4[r].w};
-#pragma unroll
-                    for (int m = 0; m < 4; ++m) {
-                        acc[w][r][0] += a[m] * v4[m].x;
-                        acc[w][r][1] += a[m] * v4[m].y;
-                        acc[w][r][2] += a[m] * v4[m].z;
-                        acc[w][r][3] += a[m] * v4[m].w;
-                    }
-                }
-            }
-        }
-    }
+    // this wavefront's columns of the values and of the state, on their way while the scores are made
+    const int col = 16 * wave + r, cc = min(col, vdim - 1);
     const float* S0 = U + (dc_entry(t0, b, c) * heads + h) * dim * vdim;
-    for (int k0 = 0; k0 < dim; k0 += DC_SLAB) {
-        const int rows = min(DC_SLAB, dim - k0);             // a multiple of 4
-        __syncthreads();                                     // the slab before has been read
-        for (int e = tid; e < rows * tcs; e += DC_THREADS)
-            *reinterpret_cast<float4*>(Ss + e * 4) = *reinterpret_cast<const float4*>(S0 + (size_t)k0 * vdim + e * 4);
-        __syncthreads();
+    float v[4][4], sv[DC_MAX / 16][4];
 #pragma unroll
-        for (int w = 0; w < 1; ++w) {
-            const int tile = tid + w * DC_THREADS;
-            if (tile < tiles) {
-                const int ti = tile / tcs, tc = tile - ti * tcs;
-                for (int k = 0; k < rows; k += 4) {
-                    float4 q4[4], s4[4];
+    for (int q = 0; q < 4; ++q)
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        q4[r] = *reinterpret_cast<const float4*>(Qs + (4 * ti + r) * qs + k0 + k);
-                        s4[r] = *reinterpret_cast<const float4*>(Ss + (k + r) * vdim + 4 * tc);
-                    }
+        for (int e = 0; e < 4; ++e) {
+            const int j = 16 * q + 4 * g + e;
+            const float x = src.v1(first + min(j, n - 1), min(j, n - 1), h, vdim, cc, made);
+            v[q][e] = j < n ? x : 0.f;
+        }
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const float q[4] = {q4[r].x, q4[r].y, q4[r].z, q4[r].w};
+    for (int q = 0; q < DC_MAX / 16; ++q)
 #pragma unroll
-                        for (int m = 0; m < 4; ++m) {
-                            from_state[w][r][0] += q[m] * s4[m].x;
-                            from_state[w][r][1] += q[m] * s4[m].y;
-                            from_state[w][r][2] += q[m] * s4[m].z;
-                            from_state[w][r][3] += q[m] * s4[m].w;
-                        }
-                    }
-                }
-            }
+        for (int e = 0; e < 4; ++e) {
+            const int k = 16 * q + 4 * g + e;
+            const float x = S0[(size_t)min(k, dim - 1) * vdim + cc];
+            sv[q][e] = k < dim ? x : 0.f;
+        }
+    // scores: the ten tiles of 16 x 16 on and below the diagonal
+    dc_floatx4 score[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const int tile = wave + 8 * u, ti = tile < 1 ? 0 : tile < 3 ? 1 : tile < 6 ? 2 : 3, tj = tile - ti * (ti + 1) / 2;
+        if (tile >= 10) break;
+        for (int k = 0; k < wide; k += 16) {
+            const dc_floatx4 qa = *reinterpret_cast<const dc_floatx4*>(Qs + (16 * ti + r) * DC_STRIDE + k + 4 * g);
+            const dc_floatx4 kb = *reinterpret_cast<const dc_floatx4*>(Ks + (16 * tj + r) * DC_STRIDE + k + 4 * g);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) score[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(qa[e], kb[e], score[u], 0, 0, 0);
         }
     }
+    __syncthreads();                                         // the keys have been read: the scores take their place
 #pragma unroll
-    for (int w = 0; w < 1; ++w) {
-        const int tile = tid + w * DC_THREADS;
-        if (tile < tiles) {
-            const int ti = tile / tcs, tc = tile - ti * tcs;
+    for (int u = 0; u < 2; ++u) {
+        const int tile = wave + 8 * u, ti = tile < 1 ? 0 : tile < 3 ? 1 : tile < 6 ? 2 : 3, tj = tile - ti * (ti + 1) / 2;
+        if (tile >= 10) break;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int i = 4 * ti + r;
-                if (i < n) {
-                    const float f = pw[i + 1];
-                    *reinterpret_cast<float4*>(out + (size_t)(first + i) * heads * vdim + h * vdim + 4 * tc) =
-                        make_float4(acc[w][r][0] + f * from_state[w][r][0], acc[w][r][1] + f * from_state[w][r][1],
-                                    acc[w][r][2] + f * from_state[w][r][2], acc[w][r][3] + f * from_state[w][r][3]);
-                }
-            }
+        for (int e = 0; e < 4; ++e) {
+            const int i = 16 * ti + 4 * g + e, j = 16 * tj + r;
+            As[i * DC_ASTRIDE + j] = j <= i && i < n ? score[u][e] * src.between(made, i, min(j, i)) : 0.f;
         }
     }
+    __syncthreads();
+    if (16 * wave >= vdim) return;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        dc_floatx4 sum = {0.f, 0.f, 0.f, 0.f}, from_state = sum;
+        if (16 * t >= n) break;                              // (the same for the whole workgroup)
+#pragma unroll
+        for (int q = 0; q < DC_MAX / 16; ++q) {
+            if (16 * q >= wide) break;
+            const dc_floatx4 qa = *reinterpret_cast<const dc_floatx4*>(Qs + (16 * t + r) * DC_STRIDE + 16 * q + 4 * g);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) from_state = __builtin_amdgcn_mfma_f32_16x16x4f32(qa[e], sv[q][e], from_state, 0, 0, 0);
+        }
+#pragma unroll
+        for (int q = 0; q <= t; ++q) {
+            const dc_floatx4 a = *reinterpret_cast<const dc_floatx4*>(As + (16 * t + r) * DC_ASTRIDE + 16 * q + 4 * g);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) sum = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], v[q][e], sum, 0, 0, 0);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int i = 16 * t + 4 * g + e;
+            if (i < n && col < vdim)
+                out[(size_t)(first + i) * heads * vdim + h * vdim + col] =
+                    src.finish(sum[e] + src.from_start(made, i) * from_state[e], first + i, h, vdim, col);
+        }
+    }
+}
+
+template <typename SRC>
+static void launch_chunks(float* out, float* workspace, const SRC& src, float* state, const int32_t* cu_seqlens, const int32_t* slots,
+                          int seqs, int tokens, int max_new, int heads, int dim, int vdim, hipStream_t s) {
+    const dim3 grid((max_new + DC_TOK - 1) / DC_TOK, seqs, heads);
+    float* wholes = workspace + ((size_t)tokens / DC_TOK + seqs) * heads * dim * vdim;
+    decay_chunk_sums_kernel<SRC><<<grid, DC_THREADS, 0, s>>>(workspace, wholes, src, cu_seqlens, heads, dim, vdim);
+    decay_chunk_carry_kernel<<<dim3((dim * vdim / 4 + 255) / 256, seqs, heads), 256, 0, s>>>(workspace, wholes, state, cu_seqlens, slots,
+                                                                                             heads, dim, vdim);
+    decay_chunk_out_kernel<SRC><<<grid, DC_THREADS, 0, s>>>(out, workspace, src, cu_seqlens, heads, dim, vdim);
 }
 
 extern "C" int ri_decay_chunks_fit(int dim, int vdim) {
@@ -288,7 +326,7 @@ extern "C" int ri_decay_chunks_fit(int dim, int vdim) {
 
 // How many floats of workspace a step of `tokens` tokens in `seqs` sequences needs.
 extern "C" long ri_decay_chunks_workspace(int seqs, int tokens, int heads, int dim, int vdim) {
-    return ((long)tokens / DC_TOK + seqs) * heads * dim * vdim;
+    return ((long)tokens / DC_TOK + seqs) * heads * (dim * vdim + 1L);
 }
 
 extern "C" int ri_decay_scan_chunked(float* out, const void* proj, int act_dtype, int row, int q_off, int k_off, int v_off,
@@ -306,32 +344,39 @@ extern "C" int ri_decay_scan_chunked(float* out, const void* proj, int act_dtype
     RI_REQUIRE(workspace_floats >= ri_decay_chunks_workspace(seqs, tokens, heads, dim, vdim),
                "decay_scan_chunked: a workspace of %ld floats", workspace_floats);
     hipStream_t s = (hipStream_t)stream;
-    const int chunks = (max_new + DC_TOK - 1) / DC_TOK;
-    const dim3 grid(chunks, seqs, heads);
-    const size_t lds_sums = (size_t)DC_TOK * (dim + vdim) * sizeof(float);
-    const size_t lds_out = ((size_t)DC_TOK * (dim + 4) + (size_t)DC_TOK * (dim + 4 > vdim ? dim + 4 : vdim) +
-                            (size_t)DC_TOK * DC_ASTRIDE + (size_t)DC_SLAB * vdim) * sizeof(float);
 #define RI_DC_GO(T)                                                                                                  \
-    {                                                                                                                \
-        static bool asked = false;                                                                                   \
-        if (!asked) {                                                                                                \
-            hipError_t e_ = hipFuncSetAttribute((const void*)decay_chunk_sums_kernel<T>,                             \
-                                                hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024);             \
-            RI_REQUIRE(e_ == hipSuccess, "decay_scan_chunked: %s", hipGetErrorString(e_));                           \
-            e_ = hipFuncSetAttribute((const void*)decay_chunk_out_kernel<T>, hipFuncAttributeMaxDynamicSharedMemorySize, \
-                                     128 * 1024);                                                                    \
-            RI_REQUIRE(e_ == hipSuccess, "decay_scan_chunked: %s", hipGetErrorString(e_));                           \
-            asked = true;                                                                                            \
-        }                                                                                                            \
-        decay_chunk_sums_kernel<T><<<grid, DC_THREADS, lds_sums, s>>>(workspace, (const T*)proj, row, k_off, v_off, cu_seqlens, \
-                                                               head_decay, heads, dim, vdim);                        \
-        decay_chunk_carry_kernel<<<dim3((dim * vdim / 4 + 255) / 256, seqs, heads), 256, 0, s>>>(                    \
-            workspace, state, cu_seqlens, slots, head_decay, heads, dim, vdim);                                      \
-        decay_chunk_out_kernel<T><<<grid, DC_THREADS, lds_out, s>>>(out, workspace, (const T*)proj, row, q_off, k_off, v_off, \
-                                                             cu_seqlens, head_decay, q_scale, heads, dim, vdim);     \
-    }
-    if (act_dtype == RI_F32) RI_DC_GO(float) else RI_DC_GO(bf16_t)
+    launch_chunks(out, workspace, DcFixed<T>{(const T*)proj, row, q_off, k_off, v_off, head_decay, q_scale}, state, cu_seqlens, slots, seqs, \
+                  tokens, max_new, heads, dim, vdim, s)
+    if (act_dtype == RI_F32) RI_DC_GO(float); else RI_DC_GO(bf16_t);
 #undef RI_DC_GO
     RI_LAUNCH_CHECK("decay_scan_chunked");
+    return 0;
+}
+
+extern "C" int ri_ssd_scan_chunked(float* out, const float* xbc, int channels, int b_off, int c_off, const void* proj, int act_dtype,
+                                   int stride, int z_off, int dt_off, const float* dt_bias, const float* a_log, const float* d_skip,
+                                   float* state, const int32_t* cu_seqlens, const int32_t* slots, int seqs, int tokens, int max_new,
+                                   int heads, int groups, int n, int vdim, float* workspace, long workspace_floats, void* stream) {
+    RI_REQUIRE(out && xbc && proj && a_log && state && cu_seqlens && slots && workspace, "ssd_scan_chunked: a null pointer");
+    RI_REQUIRE(act_dtype == RI_F32 || act_dtype == RI_BF16, "ssd_scan_chunked: dtype %d", act_dtype);
+    RI_REQUIRE(ri_decay_chunks_fit(n, vdim), "ssd_scan_chunked: states of %d x %d (multiples of 4 up to %d)", n, vdim, DC_MAX);
+    RI_REQUIRE(seqs >= 1 && tokens >= seqs && heads >= 1 && heads <= 65535 && seqs <= 65535 && max_new >= 1 && max_new <= tokens &&
+               groups >= 1 && heads % groups == 0, "ssd_scan_chunked: %d tokens in %d sequences of at most %d, %d heads in %d groups", tokens,
+               seqs, max_new, heads, groups);
+    RI_REQUIRE(channels % 4 == 0 && b_off % 4 == 0 && c_off % 4 == 0 && b_off >= 0 && c_off >= 0 && b_off + groups * n <= channels &&
+               c_off + groups * n <= channels && heads * vdim <= channels && (uintptr_t)xbc % 16 == 0 && (uintptr_t)state % 16 == 0 &&
+               (uintptr_t)workspace % 16 == 0, "ssd_scan_chunked: columns %d and %d of %d channels, or a buffer that is not aligned", b_off,
+               c_off, channels);
+    RI_REQUIRE(z_off >= 0 && dt_off >= 0 && z_off + heads * vdim <= stride && dt_off + heads <= stride,
+               "ssd_scan_chunked: columns %d and %d of rows of %d", z_off, dt_off, stride);
+    RI_REQUIRE(workspace_floats >= ri_decay_chunks_workspace(seqs, tokens, heads, n, vdim), "ssd_scan_chunked: a workspace of %ld floats",
+               workspace_floats);
+    hipStream_t s = (hipStream_t)stream;
+#define RI_DC_GO(T)                                                                                                  \
+    launch_chunks(out, workspace, DcSteps<T>{xbc, channels, b_off, c_off, (const T*)proj, stride, z_off, dt_off, dt_bias, a_log, d_skip, \
+                                             heads / groups}, state, cu_seqlens, slots, seqs, tokens, max_new, heads, n, vdim, s)
+    if (act_dtype == RI_F32) RI_DC_GO(float); else RI_DC_GO(bf16_t);
+#undef RI_DC_GO
+    RI_LAUNCH_CHECK("ssd_scan_chunked");
     return 0;
 }

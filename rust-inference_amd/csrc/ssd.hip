@@ -14,7 +14,8 @@
 // The step size with its softplus, the decay with both exponentials, the state, every sum of the recurrence, the gate and
 // the norm are float32.  A workgroup of ssd_scan owns one (sequence, head): a thread holds some rows of one column of
 // the state in registers and the slices of rows meet through LDS in a fixed order, so a token's sums do not depend on
-// how the tokens were cut into steps.  The same kernels walk a prompt and take a single step.
+// how the tokens were cut into steps.  The same kernels walk a prompt and take a single step; prompts whose walk is a chain of many
+// tokens with little beside it go in chunks instead (decay_chunks.hip), whose sums differ from the walk's by rounding.
 #include "api.h"
 #include "common.h"
 #include "walk.h"

@@ -203,6 +203,8 @@ _SIGNATURES = {
     "ri_ssd_scan_cols_fits": [c_int, c_int],
     "ri_ssd_scan_cols": [c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p,
                          c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
+    "ri_ssd_scan_chunked": [c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p,
+                            c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p, ctypes.c_long, c_void_p],
     "ri_group_rms_norm": [c_void_p, c_int, c_void_p, c_void_p, c_float, c_int, c_int, c_int, c_void_p],
 }
 
@@ -794,6 +796,10 @@ def decay_chunks_fit(dim: int, vdim: int, row: int, offsets: tuple) -> bool:
     return bool(_get("ri_decay_chunks_fit")(int(dim), int(vdim))) and row % 4 == 0 and all(o % 4 == 0 for o in offsets)
 
 
+def _decay_chunks_workspace(seqs: int, tokens: int, heads: int, dim: int, vdim: int) -> int:
+    return (tokens // 64 + seqs) * heads * (dim * vdim + 1)
+
+
 def decay_scan_chunked(proj, q_off: int, k_off: int, v_off: int, head_decay, q_scale: float, state, cu_seqlens, slots,
                        heads: int, dim: int, vdim: int, max_new: int) -> torch.Tensor:
     """``decay_scan`` for prompts, in chunks of 64 tokens: with a constant decay a chunk's tokens do not wait for one
@@ -803,7 +809,7 @@ def decay_scan_chunked(proj, q_off: int, k_off: int, v_off: int, head_decay, q_s
     tokens, row = proj.shape
     seqs = slots.shape[0]
     out = torch.empty((tokens, heads * vdim), dtype=torch.float32, device=proj.device)
-    need = (tokens // 64 + seqs) * heads * dim * vdim
+    need = _decay_chunks_workspace(seqs, tokens, heads, dim, vdim)
     work = torch.empty((need,), dtype=torch.float32, device=proj.device)
     _call("ri_decay_scan_chunked", _dev(out, "out"), _dev(proj, "proj"), code(proj.dtype), row, int(q_off), int(k_off),
           int(v_off), _dev(head_decay, "head_decay", torch.float32, (heads,)), float(q_scale),
@@ -2097,6 +2103,49 @@ def ssd_scan(xbc, b_off: int, c_off: int, proj, z_off: int, dt_off: int, dt_bias
           _dev(a_log, "a_log", torch.float32, (heads,)), _opt(d_skip, "d_skip", torch.float32, (heads,)),
           _dev(state, "state", torch.float32), _dev(cu_seqlens, "cu_seqlens", torch.int32, (seqs + 1,)),
           _dev(slots, "slots", torch.int32), *((tokens,) if columns else ()), seqs, heads, groups, n, vdim, _stream())
+    return out
+
+
+SSD_CHUNKS_WORKSPACE = 1 << 28   # floats of workspace at most: a gigabyte, beyond which a step keeps to the walk
+
+
+def ssd_chunks_pay(new_counts, heads: int, n: int, vdim: int) -> bool:
+    """Whether ``ssd_scan_chunked`` is expected to take less time than ``ssd_scan`` (host arithmetic only).  The walk takes a token's latency
+    times the longest sequence, 0.145, 0.17 and 0.27 us with one, two and four columns a lane (``walk_columns`` of walk.h; 0.44 us for states
+    of up to 64 rows), or what the machine does at most, 2 ns a token and head of 128 x 128 (0.7 of 64 x 64); the chunks 25 us and 0.13
+    (0.07) us a chunk and head.  256 compute units, us walk : chunks; 32 heads of 128 x 128, one prompt of 256 43 : 48, 512 82 : 57, 2,048 296 :
+    130, four of 300 to 1,800 484 : 359, eight of 500 255 : 268, 32 of 1,000 1,941 : 2,170, 40 single tokens beside a prompt of 200 92 : 324;
+    32 heads of 64 x 64, one of 64 33 : 29, 2,048 910 : 82, eight of 500 223 : 134, 32 of 128 98 : 135."""
+    units, longest, size = compute_units(), max(new_counts), n * vdim / 16384
+    if _decay_chunks_workspace(len(new_counts), sum(new_counts), heads, n, vdim) > SSD_CHUNKS_WORKSPACE:
+        return False
+    columns, waves = len(new_counts) * heads * vdim, 8 * units
+    a_token = 0.44 if n <= 64 else 0.145 if columns <= 2 * waves else 0.17 if columns <= 4 * waves else 0.27
+    walk = max(longest * a_token, sum(new_counts) * heads * (0.0003 + 0.0017 * size) * 256 / units)
+    return 25 + sum(-(-k // 64) for k in new_counts) * heads * (0.05 + 0.08 * size) * 256 / units < 0.9 * walk
+
+
+def ssd_chunks_fit(n: int, vdim: int, channels: int, offsets: tuple) -> bool:
+    """Whether ``ssd_scan_chunked`` takes these sizes (host code only)."""
+    return bool(_get("ri_decay_chunks_fit")(int(n), int(vdim))) and channels % 4 == 0 and all(o % 4 == 0 for o in offsets)
+
+
+def ssd_scan_chunked(xbc, b_off: int, c_off: int, proj, z_off: int, dt_off: int, dt_bias, a_log, d_skip, state, cu_seqlens, slots,
+                     heads: int, groups: int, n: int, vdim: int, max_new: int) -> torch.Tensor:
+    """``ssd_scan`` for prompts, in chunks of 64 tokens as in ``decay_scan_chunked``: a chunk's decays are known before its walk.  float32
+    throughout; differs from ``ssd_scan`` by rounding alone.  ``max_new``: the most new tokens of a sequence."""
+    tokens, channels = xbc.shape
+    seqs = slots.shape[0]
+    if tuple(state.shape[1:]) != (heads, n, vdim) or proj.shape[0] != tokens:
+        raise ShapeError(f"ssd_scan_chunked: state {list(state.shape)} for {heads} heads of {n} x {vdim}")
+    out = torch.empty((tokens, heads * vdim), dtype=torch.float32, device=xbc.device)
+    need = _decay_chunks_workspace(seqs, tokens, heads, n, vdim)
+    work = torch.empty((need,), dtype=torch.float32, device=xbc.device)
+    _call("ri_ssd_scan_chunked", _dev(out, "out"), _dev(xbc, "xbc", torch.float32), channels, int(b_off), int(c_off), _dev(proj, "proj"),
+          code(proj.dtype), proj.shape[1], int(z_off), int(dt_off), _opt(dt_bias, "dt_bias", torch.float32, (heads,)),
+          _dev(a_log, "a_log", torch.float32, (heads,)), _opt(d_skip, "d_skip", torch.float32, (heads,)),
+          _dev(state, "state", torch.float32), _dev(cu_seqlens, "cu_seqlens", torch.int32, (seqs + 1,)),
+          _dev(slots, "slots", torch.int32, (seqs,)), seqs, tokens, int(max_new), heads, groups, n, vdim, _dev(work, "workspace"), need, _stream())
     return out
 
 

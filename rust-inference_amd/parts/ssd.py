@@ -74,8 +74,15 @@ class StateSpaceMixer(Mixer):
             xbc = ops.causal_conv_silu(proj, self.inner, self.channels, self.conv_w, self.conv_b, tails, ctx.tok_seq,
                                        ctx.cu_seqlens, ctx.slots)
             gn = self.groups * self.state
-            y = ops.ssd_scan(xbc, self.inner, self.inner + gn, proj, 0, self.inner + self.channels, self.dt_bias, self.a_log,
-                             self.d_skip, state, ctx.cu_seqlens, ctx.slots, self.heads, self.groups, self.state, self.vdim)
+            args = (xbc, self.inner, self.inner + gn, proj, 0, self.inner + self.channels, self.dt_bias, self.a_log, self.d_skip, state,
+                    ctx.cu_seqlens, ctx.slots, self.heads, self.groups, self.state, self.vdim)
+            if (proj.dtype != torch.float32 and not rt.invariant and ctx.max_new > 1
+                    and ops.ssd_chunks_pay(ctx.new_counts, self.heads, self.state, self.vdim)
+                    and ops.ssd_chunks_fit(self.state, self.vdim, self.channels, (self.inner, self.inner + gn))):
+                # prompts: chunks of 64 tokens side by side (float32 and the invariant mode keep the one form of the walk)
+                y = ops.ssd_scan_chunked(*args, ctx.max_new)
+            else:
+                y = ops.ssd_scan(*args)
             y = ops.group_rms_norm(y, self.gain, self.eps, self.norm_groups, rt.dtype)
         with profiler.section(profiler.OUT_PROJECTION):
             return rt.linear_packed(y, self.w_o, out_dtype=torch.float32, parts_ok=True)

@@ -367,6 +367,53 @@ def test_state_space_mixer_through_every_cut(ops, heads, vdim, n, groups, taps, 
         close(got, np.concatenate(want), 3e-5, f"state-space mixer, step {counts}")
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("heads, groups, n, vdim, lens", [(2, 1, 64, 32, (200,)), (3, 3, 12, 20, (64, 1, 130)), (2, 1, 128, 128, (65, 63)),
+                                                          (4, 2, 100, 36, (2, 191, 128)), (2, 2, 4, 8, (129,))])
+def test_state_space_walk_in_chunks(ops, dtype, heads, groups, n, vdim, lens):
+    """States that are not zero, at slots in another order, lengths on and beside a chunk's edge, steps that hardly decay and such that
+    forget all within a few tokens; against the recurrence in 64 bits, whose distance is no larger than the walk's, and against the walk."""
+    rng = np.random.default_rng(heads * 17 + n)
+    T, inner = sum(lens), heads * vdim
+    channels, b_off, c_off = inner + 2 * groups * n + 4, inner + 4, inner + 4 + groups * n
+    xbc, proj = t(rng.normal(size=(T, channels))), t(rng.normal(size=(T, 3 + inner + heads)), dtype)
+    dt_bias, a_log, skip = t(rng.normal(size=heads) * 2), t(np.linspace(-6, 3, heads)), t(rng.normal(size=heads))
+    slots = [2, 0, 3][:len(lens)]
+    start = t(rng.normal(size=(4, heads, n, vdim)))
+    x, p, want_state = f64(xbc), f64(proj), f64(start).copy()
+    want = np.zeros((T, inner))
+    cu = np.concatenate([[0], np.cumsum(lens)])
+    for s, slot in enumerate(slots):
+        for i in range(cu[s], cu[s + 1]):
+            for h in range(heads):
+                raw = p[i, 3 + inner + h] + f64(dt_bias)[h]
+                dt = raw if raw > 20 else np.log1p(np.exp(raw))
+                B, C = (x[i, o + h * groups // heads * n:][:n] for o in (b_off, c_off))
+                xv, z = x[i, h * vdim:(h + 1) * vdim], p[i, 3 + h * vdim:3 + (h + 1) * vdim]
+                S = want_state[slot, h]
+                S[:] = np.exp(-np.exp(f64(a_log)[h]) * dt) * S + dt * np.outer(B, xv)
+                want[i, h * vdim:(h + 1) * vdim] = (S.T @ C + f64(skip)[h] * xv) * z / (1 + np.exp(-z))
+    args = (xbc, b_off, c_off, proj, 3, 3 + inner, dt_bias, a_log, skip)
+    more = (t(cu, torch.int32), t(slots, torch.int32), heads, groups, n, vdim)
+    assert ops.ssd_chunks_fit(n, vdim, channels, (b_off, c_off))
+    chunked, walked = guarded(start.clone()), guarded(start.clone())
+    got, walk = ops.ssd_scan_chunked(*args, chunked, *more, max(lens)), ops.ssd_scan(*args, walked, *more)
+    close(got, want, 1e-5, "outputs")
+    close(chunked, want_state, 1e-5, "state")
+    assert np.array_equal(f64(chunked[1]), f64(start[1]))     # a slot that no sequence of the step has
+    close(got, f64(walk), 1e-5, "chunks against the walk")
+    error = lambda y: np.linalg.norm(f64(y) - want) / np.linalg.norm(want)
+    assert error(got) <= 1.5 * error(walk) + 1e-7
+
+
+def test_state_space_chunks_where_the_walk_waits_for_its_tokens(ops, monkeypatch):
+    monkeypatch.setattr(ops, "compute_units", lambda: 256)
+    pay = ops.ssd_chunks_pay
+    assert pay([2048], 32, 128, 128) and pay([512], 32, 128, 128) and pay([300, 1800, 1500, 1300], 32, 128, 128) and pay([500] * 8, 32, 64, 64)
+    assert not pay([256], 32, 128, 128) and not pay([500] * 8, 32, 128, 128) and not pay([1000] * 32, 32, 128, 128)
+    assert not pay([1] * 40 + [200], 32, 128, 128) and not pay([128] * 32, 32, 64, 64) and not pay([64], 32, 64, 64)
+
+
 # ---------------------------------------------------------------- the products per head through the library
 @pytest.mark.parametrize("heads, k, n, extra, gated", [(3, 24, 40, 6, False), (5, 40, 12, 0, True), (2, 16, 16, 10, True)])
 def test_batched_head_products_are_the_products_per_head(ops, heads, k, n, extra, gated):
