@@ -64,22 +64,26 @@ talking_bias_kernel(float* __restrict__ table, const float* __restrict__ r1, con
 
 struct __attribute__((packed, aligned(4))) TmEight { float v[8]; };
 
-// The eight scores of a lane (column = token, keys key0 .. key0 + 7) of head h for one page: raw products times the scale,
-// minus the distance bias, minus infinity where the token does not see the key.
-// TABLE: `bias` is the head's row of the table of distances, its entry for a gap of 0.
-template <int KS, bool TABLE>
-__device__ __forceinline__ void talking_scores(float (&s)[8], const TmFrag (&qf)[KS], const bf16_t* __restrict__ kp, int dim,
-                                               float scale, float b1, float b2, bool biased, int qpos, int lo, int key0,
-                                               const float* __restrict__ bias, int window) {
-    TmEight by_gap;                                            // of the gaps from the last of the eight keys up to the first's
-    TmFrag k0[KS], k1[KS];
+// A lane's fragments of a page's keys (both half pages).
+template <int KS>
+__device__ __forceinline__ void talking_keys(TmFrag (&k0)[KS], TmFrag (&k1)[KS], const bf16_t* __restrict__ kp) {
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
         k0[ks].u = *reinterpret_cast<const uint4*>(kp + ks * 32);
-        k1[ks].u = *reinterpret_cast<const uint4*>(kp + 4 * dim + ks * 32);
+        k1[ks].u = *reinterpret_cast<const uint4*>(kp + 4 * 32 * KS + ks * 32);
     }
-    if (TABLE) by_gap = *reinterpret_cast<const TmEight*>(bias + min(max(qpos - key0 - 7, -8), window));
-    __builtin_amdgcn_sched_barrier(0);                         // every load is asked for before the first is waited for
+}
+// The biases of the gaps from the last of the lane's eight keys up to the first's; `bias` is the head's row of the table of distances, its
+// entry for a gap of 0.
+__device__ __forceinline__ TmEight talking_gaps(const float* __restrict__ bias, int qpos, int key0, int window) {
+    return *reinterpret_cast<const TmEight*>(bias + min(max(qpos - key0 - 7, -8), window));
+}
+
+// The eight scores of a lane (column = token, keys key0 .. key0 + 7) of a head for one page: raw products times the scale,
+// minus the distance bias, minus infinity where the token does not see the key.
+template <int KS, bool TABLE>
+__device__ __forceinline__ void talking_scores(float (&s)[8], const TmFrag (&qf)[KS], const TmFrag (&k0)[KS], const TmFrag (&k1)[KS],
+                                               const TmEight& by_gap, float scale, float b1, float b2, bool biased, int qpos, int lo, int key0) {
     tm_floatx4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
@@ -97,7 +101,10 @@ __device__ __forceinline__ void talking_scores(float (&s)[8], const TmFrag (&qf)
     }
 }
 
-template <int KS, bool TABLE>
+// HG: query heads of one key head that a wavefront takes: a page's keys are loaded once for all of them, the next page's while
+// these are weighed.  A wavefront a head is bound by the caches (every key row 32 times over): 2,048 tokens, 32 heads over 8 of 128, a
+// window of 1,024 133 us, 101 with four heads.
+template <int KS, int HG, bool TABLE>
 __global__ void __launch_bounds__(64)
 talking_stats_mfma_kernel(float* __restrict__ stats, const bf16_t* __restrict__ q, int q_stride, int q_off,
                           const bf16_t* __restrict__ k_pages, const int32_t* __restrict__ tok_pos,
@@ -107,48 +114,76 @@ talking_stats_mfma_kernel(float* __restrict__ stats, const bf16_t* __restrict__ 
     constexpr int DIM = 32 * KS;
     int seq, first, count;
     if (!tile_of(blockIdx.x, cu_seqlens, seqs, seq, first, count)) return;
-    const int h = blockIdx.y, lane = threadIdx.x;
+    const int h0 = blockIdx.y * HG, lane = threadIdx.x;
     const int col = lane & 15, g = lane >> 4;
     const int t = first + min(col, count - 1);                 // a column pulled back inside the tile: loads are issued anyway
     const int qpos = tok_pos[t];
     const int lo = window > 0 ? max(0, qpos - window + 1) : 0;
-    const int kvh = h / (heads / kv_heads);
+    const int kvh = h0 / (heads / kv_heads);
     const int32_t* table = page_table + (size_t)seq * table_width;
-    TmFrag qf[KS];
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks)
-        qf[ks].u = *reinterpret_cast<const uint4*>(q + (size_t)t * q_stride + q_off + (size_t)h * DIM + ks * 32 + 8 * g);
     const bool biased = r1 != nullptr;
-    const float b1 = biased ? r1[h] : 0.f, b2 = biased ? r2[h] : 0.f;
-    const float* hb = TABLE ? bias + (size_t)h * (window + 16) + 8 : nullptr;
+    TmFrag qf[HG][KS], k0[KS], k1[KS];
+    float b1[HG], b2[HG], m[HG], l[HG];
+#pragma unroll
+    for (int i = 0; i < HG; ++i) {
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks)
+            qf[i][ks].u = *reinterpret_cast<const uint4*>(q + (size_t)t * q_stride + q_off + (size_t)(h0 + i) * DIM + ks * 32 + 8 * g);
+        b1[i] = biased ? r1[h0 + i] : 0.f;
+        b2[i] = biased ? r2[h0 + i] : 0.f;
+        m[i] = -INFINITY;
+        l[i] = 0.f;
+    }
     const int pos_first = tok_pos[first], pos_last = pos_first + count - 1;
     const int lo_first = window > 0 ? max(0, pos_first - window + 1) : 0;
     const int key_row = 8 * (col >> 2) + (col & 3);
-    float m = -INFINITY, l = 0.f;
-    for (int page = lo_first / TM_PAGE; page <= pos_last / TM_PAGE; ++page) {
-        const bf16_t* kp = k_pages + (((long)table[page] * kv_heads + kvh) * TM_PAGE + key_row) * (long)DIM + 8 * g;
-        float s[8];
-        talking_scores<KS, TABLE>(s, qf, kp, DIM, scale, b1, b2, biased, qpos, lo, page * TM_PAGE + 8 * g, hb, window);
-        float mx = fmaxf(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3])), fmaxf(fmaxf(s[4], s[5]), fmaxf(s[6], s[7])));
-        mx = fmaxf(mx, __shfl_xor(mx, 16, RI_WAVE));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, RI_WAVE));
-        const float m_new = fmaxf(m, mx);
-        const float m_safe = m_new == -INFINITY ? 0.f : m_new;  // a column that has seen no key yet
-        float sum = 0.f;
+    const auto keys_of = [&](int page) { return k_pages + (((long)table[page] * kv_heads + kvh) * TM_PAGE + key_row) * (long)DIM + 8 * g; };
+    const int page_last = pos_last / TM_PAGE;
+    talking_keys<KS>(k0, k1, keys_of(lo_first / TM_PAGE));
+    for (int page = lo_first / TM_PAGE; page <= page_last; ++page) {
+        const int key0 = page * TM_PAGE + 8 * g;
+        const bf16_t* next = keys_of(min(page + 1, page_last));
+        TmEight gaps[HG];
+        float s[HG][8];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) sum += expf(s[e] - m_safe);
-        l = l * expf(m - m_safe) + sum;                          // the factor is 0 while m is -inf
-        m = m_new;
+        for (int i = 0; i < HG; ++i)
+            if (TABLE) gaps[i] = talking_gaps(bias + (size_t)(h0 + i) * (window + 16) + 8, qpos, key0, window);
+#pragma unroll
+        for (int i = 0; i < HG; ++i) talking_scores<KS, TABLE>(s[i], qf[i], k0, k1, gaps[i], scale, b1[i], b2[i], biased, qpos, lo, key0);
+        __builtin_amdgcn_sched_barrier(0);
+        talking_keys<KS>(k0, k1, next);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < HG; ++i) {
+            float mx = fmaxf(fmaxf(fmaxf(s[i][0], s[i][1]), fmaxf(s[i][2], s[i][3])), fmaxf(fmaxf(s[i][4], s[i][5]), fmaxf(s[i][6], s[i][7])));
+            mx = fmaxf(mx, __shfl_xor(mx, 16, RI_WAVE));
+            mx = fmaxf(mx, __shfl_xor(mx, 32, RI_WAVE));
+            const float m_new = fmaxf(m[i], mx);
+            const float m_safe = m_new == -INFINITY ? 0.f : m_new;  // a column that has seen no key yet
+            float sum = 0.f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) sum += expf(s[i][e] - m_safe);
+            l[i] = l[i] * expf(m[i] - m_safe) + sum;                 // the factor is 0 while m is -inf
+            m[i] = m_new;
+        }
     }
-    l += __shfl_xor(l, 16, RI_WAVE);
-    l += __shfl_xor(l, 32, RI_WAVE);
-    if (g == 0 && col < count) {
-        stats[((size_t)t * heads + h) * 2] = m;
-        stats[((size_t)t * heads + h) * 2 + 1] = l;
+#pragma unroll
+    for (int i = 0; i < HG; ++i) {
+        l[i] += __shfl_xor(l[i], 16, RI_WAVE);
+        l[i] += __shfl_xor(l[i], 32, RI_WAVE);
+        if (g == 0 && col < count) {
+            stats[((size_t)t * heads + h0 + i) * 2] = m[i];
+            stats[((size_t)t * heads + h0 + i) * 2 + 1] = l[i];
+        }
     }
 }
 
-template <int KS, int HPW, bool TABLE>
+#define TM_ROW (TM_PAGE + 4)  // of a token's weights in LDS: sixteen tokens' pieces meet every bank equally
+// ONE: a wavefront's heads read one key head, whose keys and values a page it then loads once instead of once a head.  What bounds a page
+// is a chain of trips to memory (keys, queries a head, values) and the mix between them, two wavefronts a SIMD.  Both walks, 32 heads over 8
+// of 128, a window of 1,024, us keys and values a head and tokens' rows of 32 in LDS : this: 2,048 tokens 511 : 327 (this walk 370 : 221 in a
+// model's step), 1,024 259 : 195, 256 76 : 59, 17 40 : 33; 16 heads 223 : 166, 119 : 97, 41 : 33, 22 : 18.
+template <int KS, int HPW, bool TABLE, bool ONE>
 __global__ void __launch_bounds__(64 * TM_WAVES)
 talking_mix_mfma_kernel(bf16_t* __restrict__ out, float* __restrict__ parts, size_t part_stride, const float* __restrict__ stats, const bf16_t* __restrict__ q, int q_stride,
                         int q_off, const bf16_t* __restrict__ k_pages, const bf16_t* __restrict__ v_pages,
@@ -158,8 +193,8 @@ talking_mix_mfma_kernel(bf16_t* __restrict__ out, float* __restrict__ parts, siz
                         const float* __restrict__ bias) {
     constexpr int DIM = 32 * KS, VT = DIM / 16, HEADS = HPW * TM_WAVES;
     extern __shared__ float lds[];
-    float* ps = lds;                                           // [HEADS][TM_TILE][TM_PAGE] the heads' weights of a page
-    float* tk = ps + HEADS * TM_TILE * TM_PAGE;                // [HEADS][HEADS] the mixing matrix, transposed
+    float* ps = lds;                                           // [HEADS][TM_TILE][TM_ROW] the heads' weights of a page
+    float* tk = ps + HEADS * TM_TILE * TM_ROW;                 // [HEADS][HEADS] the mixing matrix, transposed
     int seq, first, count;
     if (!tile_of(blockIdx.x, cu_seqlens, seqs, seq, first, count)) return;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -195,27 +230,47 @@ talking_mix_mfma_kernel(bf16_t* __restrict__ out, float* __restrict__ parts, siz
     for (int page = page_first; page < page_end; ++page) {
         const long phys = table[page];
         // this wavefront's heads: their weights of the page, into LDS
+        // (queries are fetched again a page, a head ahead where the sums leave registers for it)
+        constexpr bool AHEAD = HPW * VT < 32;
+        TmFrag k0[KS], k1[KS], qf[AHEAD ? 2 : 1][KS];
+        TmEight gaps[AHEAD ? 2 : 1];
+        const auto fetch = [&](int i) {
+            const int h = wave * HPW + i;
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks)
+                qf[AHEAD ? i & 1 : 0][ks].u = *reinterpret_cast<const uint4*>(q + (size_t)t * q_stride + q_off + (size_t)h * DIM + ks * 32 + 8 * g);
+            if (TABLE) gaps[AHEAD ? i & 1 : 0] = talking_gaps(bias + (size_t)h * (window + 16) + 8, qpos, page * TM_PAGE + 8 * g, window);
+        };
+        const auto keys_of = [&](int h) { return k_pages + ((phys * kv_heads + h / share) * TM_PAGE + key_row) * (long)DIM + 8 * g; };
+        if (ONE) talking_keys<KS>(k0, k1, keys_of(wave * HPW));
+        if (AHEAD) fetch(0);
 #pragma unroll
         for (int i = 0; i < HPW; ++i) {
             const int h = wave * HPW + i;
-            const bf16_t* kp = k_pages + ((phys * kv_heads + h / share) * TM_PAGE + key_row) * (long)DIM + 8 * g;
-            TmFrag qf[KS];                                     // (fetched again a page: the caches hold them, the registers are the sums')
-#pragma unroll
-            for (int ks = 0; ks < KS; ++ks)
-                qf[ks].u = *reinterpret_cast<const uint4*>(q + (size_t)t * q_stride + q_off + (size_t)h * DIM + ks * 32 + 8 * g);
+            if (!ONE) talking_keys<KS>(k0, k1, keys_of(h));
+            if (!AHEAD) fetch(i);
+            else if (i + 1 < HPW) fetch(i + 1);
+            __builtin_amdgcn_sched_barrier(0);
             float s[8];
-            talking_scores<KS, TABLE>(s, qf, kp, DIM, scale, b1[i], b2[i], biased, qpos, lo, page * TM_PAGE + 8 * g,
-                                      TABLE ? bias + (size_t)h * (window + 16) + 8 : nullptr, window);
+            talking_scores<KS, TABLE>(s, qf[AHEAD ? i & 1 : 0], k0, k1, gaps[AHEAD ? i & 1 : 0], scale, b1[i], b2[i], biased, qpos, lo, page * TM_PAGE + 8 * g);
             float4 lo4, hi4;
             lo4.x = expf(s[0] - ms[i]) * inv_l[i]; lo4.y = expf(s[1] - ms[i]) * inv_l[i];
             lo4.z = expf(s[2] - ms[i]) * inv_l[i]; lo4.w = expf(s[3] - ms[i]) * inv_l[i];
             hi4.x = expf(s[4] - ms[i]) * inv_l[i]; hi4.y = expf(s[5] - ms[i]) * inv_l[i];
             hi4.z = expf(s[6] - ms[i]) * inv_l[i]; hi4.w = expf(s[7] - ms[i]) * inv_l[i];
-            float* pp = ps + ((size_t)h * TM_TILE + col) * TM_PAGE + 8 * g;
+            float* pp = ps + (h * TM_TILE + col) * TM_ROW + 8 * g;
             *reinterpret_cast<float4*>(pp) = lo4;
             *reinterpret_cast<float4*>(pp + 4) = hi4;
             __builtin_amdgcn_sched_barrier(0);                 // (a head at a time: the registers are the sums')
         }
+        const auto values_of = [&](TmFrag (&vf)[VT], int h) {
+            const bf16_t* vp = v_pages + ((phys * kv_heads + h / share) * (long)DIM + col) * TM_PAGE + 8 * g;
+#pragma unroll
+            for (int vt = 0; vt < VT; ++vt) vf[vt].u = *reinterpret_cast<const uint4*>(vp + (long)vt * 16 * TM_PAGE);
+        };
+        TmFrag vf[VT];
+        if (ONE && AHEAD) values_of(vf, wave * HPW);
+        __builtin_amdgcn_sched_barrier(0);
         __syncthreads();
         // the mix for this wavefront's heads, then their value products; a head's values are asked for together (left to itself
         // the compiler waits for every single load)
@@ -226,7 +281,7 @@ talking_mix_mfma_kernel(bf16_t* __restrict__ out, float* __restrict__ parts, siz
 #pragma unroll
             for (int e = 0; e < 8; ++e) mixed[i][e] = 0.f;
         for (int gh = 0; gh < HEADS; ++gh) {
-            const float* pp = ps + ((size_t)gh * TM_TILE + col) * TM_PAGE + 8 * g;
+            const float* pp = ps + (gh * TM_TILE + col) * TM_ROW + 8 * g;
             const float4 a = *reinterpret_cast<const float4*>(pp), b = *reinterpret_cast<const float4*>(pp + 4);
             const float w8[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
 #pragma unroll
@@ -242,10 +297,7 @@ talking_mix_mfma_kernel(bf16_t* __restrict__ out, float* __restrict__ parts, siz
             for (int e = 0; e < 4; ++e) p[i].w[e] = pack_bf16x2(mixed[i][2 * e], mixed[i][2 * e + 1]);
 #pragma unroll
         for (int i = 0; i < HPW; ++i) {
-            const bf16_t* vp = v_pages + ((phys * kv_heads + (wave * HPW + i) / share) * (long)DIM + col) * TM_PAGE + 8 * g;
-            TmFrag vf[VT];
-#pragma unroll
-            for (int vt = 0; vt < VT; ++vt) vf[vt].u = *reinterpret_cast<const uint4*>(vp + (long)vt * 16 * TM_PAGE);
+            if (!ONE || (!AHEAD && i == 0)) values_of(vf, wave * HPW + i);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int vt = 0; vt < VT; ++vt)
@@ -297,8 +349,8 @@ extern "C" int ri_talking_attention_mfma(void* out, float* stats, const void* q,
                (uintptr_t)k_pages % 16 == 0 && (uintptr_t)v_pages % 16 == 0 && (uintptr_t)out % 8 == 0,
                "talking_attention_mfma: column %d of rows of %d, or a buffer that is not aligned", q_off, q_stride);
     RI_REQUIRE((r1 == nullptr) == (r2 == nullptr) && window >= 0 && table_width > 0 && stats, "talking_attention_mfma: arguments");
-    const size_t lds = ((size_t)heads * TM_TILE * TM_PAGE + (size_t)heads * heads) * sizeof(float);
-    RI_REQUIRE(lds <= 64 * 1024 + 4096, "talking_attention_mfma: %d heads need %zu bytes of LDS", heads, lds);
+    const size_t lds = ((size_t)heads * TM_TILE * TM_ROW + (size_t)heads * heads) * sizeof(float);
+    RI_REQUIRE(lds <= 80 * 1024, "talking_attention_mfma: %d heads need %zu bytes of LDS", heads, lds);
     hipStream_t s = (hipStream_t)stream;
     const int hpw = heads / TM_WAVES;
     const bool table = bias && r1 && window > 0;
@@ -307,27 +359,32 @@ extern "C" int ri_talking_attention_mfma(void* out, float* stats, const void* q,
         talking_bias_kernel<<<(heads * (window + 16) + 255) / 256, 256, 0, s>>>(bias, r1, r2, heads, window);
     }
     if (shares == 1) parts = nullptr;
-#define RI_STATS(KS, T)                                                                                                 \
-    talking_stats_mfma_kernel<KS, T><<<dim3(tiles, heads), 64, 0, s>>>(stats, (const bf16_t*)q, q_stride, q_off,       \
+    // (four heads a wavefront from as many wavefronts on as half of the machine's SIMDs; a wavefront's heads read one key head)
+    const int of_kv = heads / kv_heads;
+    const bool four = of_kv % 4 == 0 && (long)tiles * heads / 4 >= 2L * ri_compute_units();
+#define RI_STATS(KS, HG, T)                                                                                             \
+    talking_stats_mfma_kernel<KS, HG, T><<<dim3(tiles, heads / HG), 64, 0, s>>>(stats, (const bf16_t*)q, q_stride, q_off, \
                                                                      (const bf16_t*)k_pages, tok_pos, cu_seqlens, seqs, \
                                                                      page_table, table_width, heads, kv_heads, window, scale, r1, r2, bias)
-#define RI_MIX(KS, HPW, T)                                                                                              \
+#define RI_MIX(KS, HPW, T, ONE)                                                                                         \
     do {                                                                                                                \
         if (lds > 64 * 1024)                                                                                            \
-            hipFuncSetAttribute((const void*)talking_mix_mfma_kernel<KS, HPW, T>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); \
-        talking_mix_mfma_kernel<KS, HPW, T><<<dim3(tiles, shares), 64 * TM_WAVES, lds, s>>>(                            \
+            hipFuncSetAttribute((const void*)talking_mix_mfma_kernel<KS, HPW, T, ONE>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); \
+        talking_mix_mfma_kernel<KS, HPW, T, ONE><<<dim3(tiles, shares), 64 * TM_WAVES, lds, s>>>(                       \
             (bf16_t*)out, parts, (size_t)tokens * heads * dim, stats, (const bf16_t*)q, q_stride, q_off, (const bf16_t*)k_pages, \
             (const bf16_t*)v_pages, tok_pos, cu_seqlens, seqs, page_table, table_width, kv_heads, window, scale, r1, r2, talk, bias); \
     } while (0)
+#define RI_MIX_OF(KS, HPW, T) do { if (of_kv % HPW == 0) RI_MIX(KS, HPW, T, true); else RI_MIX(KS, HPW, T, false); } while (0)
 #define RI_BY_TABLE(KS, T)                                                                                              \
     do {                                                                                                                \
-        RI_STATS(KS, T);                                                                                                \
-        if (hpw == 1) RI_MIX(KS, 1, T); else if (hpw == 2) RI_MIX(KS, 2, T); else if (hpw == 3) RI_MIX(KS, 3, T); else RI_MIX(KS, 4, T); \
+        if (four) RI_STATS(KS, 4, T); else RI_STATS(KS, 1, T);                                                          \
+        if (hpw == 1) RI_MIX(KS, 1, T, true); else if (hpw == 2) RI_MIX_OF(KS, 2, T); else if (hpw == 3) RI_MIX_OF(KS, 3, T); else RI_MIX_OF(KS, 4, T); \
     } while (0)
 #define RI_BY_HEADS(KS) do { if (table) RI_BY_TABLE(KS, true); else RI_BY_TABLE(KS, false); } while (0)
     if (dim == 32) RI_BY_HEADS(1); else if (dim == 64) RI_BY_HEADS(2); else RI_BY_HEADS(4);
 #undef RI_BY_HEADS
 #undef RI_BY_TABLE
+#undef RI_MIX_OF
 #undef RI_MIX
 #undef RI_STATS
     RI_LAUNCH_CHECK("talking_attention_mfma");

@@ -177,6 +177,26 @@ def test_latent_attention_through_every_cut(ops, heads, dim, rot, vdim, rank):
 
 
 # ---------------------------------------------------------------- the windowed attention whose heads talk
+@pytest.mark.skipif(EMULATED, reason="a thousand tokens; on an emulated machine of one unit the small tests take this form")
+@pytest.mark.parametrize("heads, kv_heads, window", [(32, 8, 100), (16, 2, None), (24, 8, 64)])
+def test_talking_attention_of_a_full_machine(ops, heads, kv_heads, window):
+    """Enough tiles that a wavefront of the first walk takes four heads (and groups of three, which it cannot); against the general kernel."""
+    counts, dim = [1000, 45, 3], 32
+    rng = np.random.default_rng(heads)
+    pages = 32 + 2 + 1
+    k_pages, v_pages = ((torch.randn(shape, device=DEV) * 0.6).to(torch.bfloat16) for shape in
+                        ((pages, kv_heads, PAGE, dim), (pages, kv_heads, dim, PAGE)))
+    table = np.zeros((3, 32), dtype=np.int32)
+    table[0], table[1, :2], table[2, 0] = np.arange(32), [32, 33], 34
+    seq, pos = t([s for s, n in enumerate(counts) for _ in range(n)], torch.int32), t([i for n in counts for i in range(n)], torch.int32)
+    proj = (torch.randn((sum(counts), heads * dim), device=DEV) * 0.6).to(torch.bfloat16)
+    args = (heads, kv_heads, dim, window, 0.2, t(rng.random(heads)), t(rng.random(heads) * 3), t(np.eye(heads) + 0.2 * rng.standard_normal((heads, heads))))
+    want = ops.talking_attention(proj, 0, k_pages, v_pages, pos, seq, t(table, torch.int32), *args)
+    got = ops.talking_attention_mfma(proj, 0, k_pages, v_pages, pos, t(np.concatenate([[0], np.cumsum(counts)]), torch.int32), counts,
+                                     t(table, torch.int32), *args, 1000)
+    close(got, f64(want), 1.5e-2, "matrix cores against the general kernels")
+
+
 @pytest.mark.parametrize("heads, kv_heads, dim, window, shares", [(4, 2, 12, 9, 1), (3, 3, 20, 33, 2), (6, 1, 8, 70, 1), (20, 2, 16, None, 3)])
 def test_talking_attention_through_every_cut(ops, heads, kv_heads, dim, window, shares):
     rng = np.random.default_rng(4)
