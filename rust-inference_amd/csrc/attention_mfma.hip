@@ -28,13 +28,21 @@ static int check_common(const char* name, int heads, int kv_heads, int head_dim,
 // 256 of them: a prompt of 3,072 tokens at Qwen3-8B sizes takes 105 us with two tiles a wavefront in 768
 // workgroups, 126 us with one tile in 1,536; at 2,048 tokens one tile in 1,024 workgroups takes 57 us, two in
 // 512 take 67).
+// Heads of 128: the workgroups are counted by the step's tokens, and two tiles a wavefront also want sequences of twelve workgroups' tokens
+// and more on average.  Below, most of what a workgroup of twice the tokens does is its start and the pages on the diagonal, which it
+// walks whole.  us with one : two tiles a wavefront (heads of 128 over 8; the workgroups that two tiles make): prompts of 500, 1,500 and 900, 32
+// heads (728) 60 : 82; 12 of 200 to 1,024, 16 heads (896) 44 : 53; 16 of 16 to 1,024 (1,016) 65 : 68, 32 (2,408) 127 : 133; eight of 500, 32 heads
+// (1,024) 41 : 41; four of 300 to 1,800 (1,240) 150 : 141; one of 2,048 (512) 64 : 73, 3,072 (768) 140 : 122, 8,192 of 16 heads (1,024) 387 : 342.
 #define PREFILL_MIN_WGS_PER_CU 3
-static int prefill_tiles(int head_dim, int group, int max_new, int seqs, int kv_heads) {
+#define PREFILL_MIN_WGS_PER_SEQ 12
+static int prefill_tiles(int head_dim, int group, int max_new, int seqs, int kv_heads, int tokens) {
     int nt = head_dim <= 64 ? 4 : 2;
     while (nt > 1 && group <= 16 * (nt / 2)) {
-        const int tile_tokens = (16 * nt) / group;
-        const long wgs = (long)((max_new + 4 * tile_tokens - 1) / (4 * tile_tokens)) * seqs * kv_heads;
-        if (wgs >= (long)PREFILL_MIN_WGS_PER_CU * ri_compute_units()) break;
+        const int of_wg = 4 * ((16 * nt) / group);
+        const long wgs = head_dim <= 64 ? (long)((max_new + of_wg - 1) / of_wg) * seqs * kv_heads
+                                        : (tokens + (long)seqs * of_wg / 2) / of_wg * kv_heads;
+        if (wgs >= (long)PREFILL_MIN_WGS_PER_CU * ri_compute_units() &&
+            (head_dim <= 64 || tokens >= (long)PREFILL_MIN_WGS_PER_SEQ * of_wg * seqs)) break;
         nt /= 2;
     }
     return nt;
@@ -45,7 +53,7 @@ extern "C" int ri_attention_prefill_kept_bf16(void* out, const void* qkv, int q_
                                               const int32_t* page_table, int table_width, int seqs, int max_new,
                                               int heads, int kv_heads, int head_dim, int page_size, int window, int chunk,
                                               float scale, float softcap, const float* slopes, int keep_first,
-                                              const float* sinks, void* stream) {
+                                              const float* sinks, int tokens, void* stream) {
     RI_REQUIRE(chunk >= 0 && (chunk == 0 || window <= 0), "attention_prefill: chunks of %d beside a window of %d", chunk, window);
     const Reach reach = {window, chunk};
     RI_REQUIRE(keep_first >= 0, "attention_prefill_bf16: %d first tokens kept", keep_first);
@@ -54,7 +62,7 @@ extern "C" int ri_attention_prefill_kept_bf16(void* out, const void* qkv, int q_
     if (check_common("attention_prefill_bf16", heads, kv_heads, head_dim, page_size, q_stride, table_width)) return 1;
     const int group = heads / kv_heads;
     RI_REQUIRE(seqs > 0 && seqs <= 65535 && max_new > 0, "attention_prefill_bf16: seqs %d, max_new %d", seqs, max_new);
-    const int nt_tiles = prefill_tiles(head_dim, group, max_new, seqs, kv_heads);
+    const int nt_tiles = prefill_tiles(head_dim, group, max_new, seqs, kv_heads, tokens);
     RI_REQUIRE(group <= 16 * nt_tiles, "attention_prefill_bf16: %d query heads per kv head (at most %d)", group,
                16 * nt_tiles);
     const int tile_tokens = (16 * nt_tiles) / group;
@@ -98,7 +106,7 @@ extern "C" int ri_attention_prefill_bf16(void* out, const void* qkv, int q_strid
                                          float scale, float softcap, const float* slopes, void* stream) {
     return ri_attention_prefill_kept_bf16(out, qkv, q_stride, k_pages, v_pages, cu_seqlens, tok_pos, page_table, table_width,
                                           seqs, max_new, heads, kv_heads, head_dim, page_size, window, 0, scale, softcap, slopes,
-                                          0, nullptr, stream);
+                                          0, nullptr, (int)(max_new * (long)seqs < 1 << 30 ? max_new * (long)seqs : 1 << 30), stream);
 }
 
 // Whether the streaming kernel ranks the step's sequences by their lengths (host code only).

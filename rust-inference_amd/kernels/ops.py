@@ -103,7 +103,7 @@ _SIGNATURES = {
     "ri_argmax": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p],
     "ri_attention_prefill_kept_bf16": [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int,
                                        c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_float, c_void_p, c_int,
-                                       c_void_p, c_void_p],
+                                       c_void_p, c_int, c_void_p],
     "ri_attention_kept": [c_void_p, c_void_p, c_int, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int,
                           c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_float, c_void_p, c_int, c_void_p,
                           c_int, c_void_p, c_int, c_int, c_int, c_int, c_void_p],
@@ -1251,7 +1251,7 @@ def attention_prefill_bf16(qkv, k_pages, v_pages, cu_seqlens, tok_pos, page_tabl
           _dev(page_table, "page_table", torch.int32), page_table.shape[1], seqs, max_new, heads, kv_heads, head_dim,
           k_pages.shape[2], int(window or 0), int(chunk or 0), float(scale), float(softcap or 0.0),
           _opt(slopes, "slopes", torch.float32, (heads,)), int(keep_first or 0), _opt(sinks, "sinks", torch.float32, (heads,)),
-          _stream())
+          tokens, _stream())
     return out
 
 

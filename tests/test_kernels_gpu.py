@@ -526,6 +526,27 @@ def test_mfma_prefill_attention(ops, heads, kv_heads, dh):
     close(out, want, BF16_OUT, "prefill attention on the matrix cores")
 
 
+@pytest.mark.parametrize("heads", [20, 32])
+def test_mfma_prefill_attention_with_two_tiles_a_wavefront(ops, heads):
+    """More query heads a key head than one tile of sixteen columns holds: two tiles whatever the step's size."""
+    out, want = attention_case(ops, np.random.default_rng(heads), [33, 100, 1], [33, 5, 1], heads, 1, 128, torch.bfloat16, kernel="prefill")
+    close(out, want, BF16_OUT, "prefill attention, two tiles a wavefront")
+
+
+@pytest.mark.skipif(EMULATED, reason="eight thousand tokens")
+@pytest.mark.parametrize("cap", [None, 20.0])
+def test_mfma_prefill_attention_of_a_long_prompt_is_its_pieces(ops, cap):
+    """A prompt long enough for two tiles a wavefront, and its last tokens in a step of their own, with one: the same bits."""
+    rng = np.random.default_rng(3)
+    n, last, heads, kv_heads, dh = 8000, 75, 16, 8, 128
+    kp, vp = (torch.randn(shape, device=DEV).to(torch.bfloat16) for shape in ((250, kv_heads, 32, dh), (250, kv_heads, dh, 32)))
+    table = t(rng.permutation(250)[None], torch.int32)
+    qkv = torch.randn((n, heads * dh), device=DEV).to(torch.bfloat16)
+    run = lambda first: ops.attention_prefill_bf16(qkv[first:], kp, vp, t([0, n - first], torch.int32), t(np.arange(first, n), torch.int32), table,
+                                                   1, n - first, heads, kv_heads, dh, None, dh ** -0.5, cap)
+    assert torch.equal(run(0)[n - last:], run(n - last))
+
+
 @pytest.mark.parametrize("heads, kv_heads, dh", MFMA_SHAPES)
 def test_mfma_decode_attention(ops, heads, kv_heads, dh):
     rng = np.random.default_rng(heads * 11 + dh)
