@@ -1,5 +1,6 @@
 // Causal grouped-query attention over the paged cache for any number of new tokens per sequence:
-// the form every other attention kernel here is checked against, and the one the float32 path runs.
+// the form every other attention kernel here is checked against, and the one the float32 path runs (heads of 64 and 128 in a form of
+// their own on the matrix cores, at the end).
 // One workgroup per (token, query head); keys in tiles of 256 that start at multiples of 256, so the
 // order of every sum depends on the key's position alone, never on how tokens were cut into steps.
 //
@@ -169,7 +170,7 @@ attention_generic_kernel(TA* __restrict__ out, const TA* __restrict__ q, int q_s
 // token's result is the same bits in either.  What bounds the kernel above is that a key row is loaded again for every
 // token and head; here sixteen rows share a load, and what is left is the loads' spread (a lane a key row, a lane a value
 // channel: 64 cache lines a load).  759 tokens of three sequences, 16 heads over 8 of 128, float32: 222 us a layer with the
-// kernel above, 133 with this one, 94 with the longest walks first.
+// kernel above, 133 with this one, 94 with the longest walks first (before such heads went to the matrix cores, below).
 // head_dim and the value rows in 16-byte pieces, v_dim <= 512 / SHARES: the rows' weighted sums go to SHARES groups of threads,
 // two channels a thread, so that a weight read from LDS serves two of them; a query read from LDS serves two keys likewise.
 #define ATT_ROWS 16

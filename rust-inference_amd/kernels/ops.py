@@ -542,7 +542,8 @@ ATTENTION_ROWS_FILL = 8          # rows that its runs fill at least, for its tok
 # 256, 13 of 144, 9 of 48, over 256 compute units).  One prompt of float32 heads of 128 (16 over 8), tokens @ cached tokens, us a workgroup a
 # (token, head) : by rows (the sum's KB): 130 @ 0 27 : 38 (340), 160 @ 0 38 : 41 (510), 200 @ 0 51 : 45 (800), 400 @ 0 165 : 87 (1,600), 64 @ 2,000
 # 248 : 356 (580), 130 @ 2,000 528 : 363 (1,190); heads of 64 (16 over 16) 320 @ 0 72 : 68 (615), 400 @ 0 99 : 77 (960); bfloat16 heads of 24 520 @ 0
-# 90 : 85 (495), 1,000 @ 0 267 : 162 (1,375), of 72 700 @ 0 200 : 116 (1,390).
+# 90 : 85 (495), 1,000 @ 0 267 : 162 (1,375), of 72 700 @ 0 200 : 116 (1,390).  (float32 heads of 64 and 128 were measured before they went to the
+# matrix cores; the rule stands for the sizes that are left.)
 ATTENTION_ROWS_BYTES = 600_000
 ATTENTION_KEY_BYTES = 128
 
