@@ -527,7 +527,7 @@ def test_mfma_prefill_attention(ops, heads, kv_heads, dh):
 
 
 @pytest.mark.parametrize("heads", [20, 32])
-def test_mfma_prefill_attention_with_two_tiles_a_wavefront(ops, heads):
+def test_prompt_attention_with_two_tiles_a_wavefront(ops, heads):
     """More query heads a key head than one tile of sixteen columns holds: two tiles whatever the step's size."""
     out, want = attention_case(ops, np.random.default_rng(heads), [33, 100, 1], [33, 5, 1], heads, 1, 128, torch.bfloat16, kernel="prefill")
     close(out, want, BF16_OUT, "prefill attention, two tiles a wavefront")
@@ -535,7 +535,7 @@ def test_mfma_prefill_attention_with_two_tiles_a_wavefront(ops, heads):
 
 @pytest.mark.skipif(EMULATED, reason="eight thousand tokens")
 @pytest.mark.parametrize("cap", [None, 20.0])
-def test_mfma_prefill_attention_of_a_long_prompt_is_its_pieces(ops, cap):
+def test_prompt_attention_of_a_long_prompt_is_its_pieces(ops, cap):
     """A prompt long enough for two tiles a wavefront, and its last tokens in a step of their own, with one: the same bits."""
     rng = np.random.default_rng(3)
     n, last, heads, kv_heads, dh = 8000, 75, 16, 8, 128
