@@ -9,8 +9,9 @@
 // walk from chunk to chunk, S0 of the next = D S0 + U, which leaves every chunk's S0 where its U was and the last
 // state in the sequence's slot (a few loads and stores an element), and every chunk's outputs (all chunks side by side).
 // Only products of decays from an earlier token to a later one appear, never their inverses: the powers d^m, m >= 0, of a fixed decay, and
-// exp of a difference of sums of -exp(A_log) dt, which are added up in 64 bits so that the difference keeps every bit
-// of a float32.  Everything else is float32: the activations, the scores q . k, the state and all sums; the products run on the matrix
+// exp of the sum of -exp(A_log) dt over the tokens from j + 1 to i.  That sum is made of those tokens' terms alone, all of one sign (in 64
+// bits, rounded once): a difference of two sums from the chunk's start would lose a small decay behind a large one, and is NaN where a decay
+// is 0.  Everything else is float32: the activations, the scores q . k, the state and all sums; the products run on the matrix
 // cores' float32 product (16x16x4), whose products and sums are 32-bit ones.  A workgroup of eight wavefronts takes one (chunk,
 // sequence, head), a wavefront sixteen columns of the results (sixteen rows of a chunk's own sum): what only its columns need comes straight
 // from memory, once, and what all need (q and k, the scores, v) passes through LDS.  What bounds it: the products, some 230 of 32
@@ -40,15 +41,12 @@ __device__ __forceinline__ float4 dc_ld4(const bf16_t* p) {
 // meet, since a sequence of len tokens has at most len / 64 + 1 chunks.
 __device__ __forceinline__ size_t dc_entry(int t0, int b, int c) { return (size_t)(t0 / DC_TOK + b + c); }
 
-// Where a head's q, k and v come from, and its decays.  `made` is the workgroup's: the powers of a fixed decay, or the sums of the
-// exponents and the step sizes.
-struct DcMade {
-    double sums[DC_TOK];
-    float powers[DC_TOK + 1], dt[DC_TOK];
-};
-
+// Where a head's q, k and v come from, and its decays.  `Made` is the workgroup's, in LDS: what its decays are read from.
 template <typename TA>
 struct DcFixed {
+    struct Made {
+        float powers[DC_TOK + 1];
+    };
     const TA* proj;
     int row, q_off, k_off, v_off;
     const float* head_decay;
@@ -61,26 +59,32 @@ struct DcFixed {
         const float4 v = dc_ld4(proj + (size_t)t * row + k_off + h * dim + k);
         return make_float4(dc_silu(v.x), dc_silu(v.y), dc_silu(v.z), dc_silu(v.w));
     }
-    __device__ __forceinline__ float4 v4(int t, int, int h, int vdim, int c, const DcMade&) const {
+    __device__ __forceinline__ float4 v4(int t, int, int h, int vdim, int c, const Made&) const {
         const float4 v = dc_ld4(proj + (size_t)t * row + v_off + h * vdim + c);
         return make_float4(dc_silu(v.x), dc_silu(v.y), dc_silu(v.z), dc_silu(v.w));
     }
     __device__ __forceinline__ float k1(int t, int h, int dim, int k) const { return dc_silu(to_f32(proj[(size_t)t * row + k_off + h * dim + k])); }
-    __device__ __forceinline__ float v1(int t, int, int h, int vdim, int c, const DcMade&) const {
+    __device__ __forceinline__ float v1(int t, int, int h, int vdim, int c, const Made&) const {
         return dc_silu(to_f32(proj[(size_t)t * row + v_off + h * vdim + c]));
     }
-    __device__ __forceinline__ void make(DcMade& made, int, int, int h) const {
+    __device__ __forceinline__ void make(Made& made, int, int, int h) const {
         const int m = threadIdx.x;                           // (d^0 = 1 also for d = 0)
         if (m <= DC_TOK) made.powers[m] = m == 0 ? 1.0f : powf(head_decay[h], (float)m);
         __syncthreads();
     }
-    __device__ __forceinline__ float between(const DcMade& made, int i, int j) const { return made.powers[i - j]; }
-    __device__ __forceinline__ float from_start(const DcMade& made, int i) const { return made.powers[i + 1]; }
+    __device__ __forceinline__ float between(const Made& made, int i, int j) const { return made.powers[i - j]; }
+    __device__ __forceinline__ float from_start(const Made& made, int i) const { return made.powers[i + 1]; }
     __device__ __forceinline__ float finish(float o, int, int, int, int) const { return o; }
 };
 
 template <typename TA>
 struct DcSteps {
+    // Sums of exponents by blocks of sixteen tokens: near[j][i % 16] from j + 1 to i of j's block, behind[j] from j + 1 to its block's end,
+    // upto[i] from its block's start to i, of whole blocks, and from the chunk's start to i.
+    struct Made {
+        double behind[DC_TOK], upto[DC_TOK], blocks[DC_TOK / 16];
+        float near[DC_TOK][16], start[DC_TOK], dt[DC_TOK];
+    };
     const float* xbc;
     int channels, b_off, c_off;
     const TA* proj;
@@ -93,34 +97,55 @@ struct DcSteps {
     __device__ __forceinline__ float4 k4(int t, int h, int dim, int k) const {
         return dc_ld4(xbc + (size_t)t * channels + b_off + h / share * dim + k);
     }
-    __device__ __forceinline__ float4 v4(int t, int j, int h, int vdim, int c, const DcMade& made) const {
+    __device__ __forceinline__ float4 v4(int t, int j, int h, int vdim, int c, const Made& made) const {
         const float4 v = dc_ld4(xbc + (size_t)t * channels + h * vdim + c);
         const float dt = made.dt[j];
         return make_float4(dt * v.x, dt * v.y, dt * v.z, dt * v.w);
     }
     __device__ __forceinline__ float k1(int t, int h, int dim, int k) const { return xbc[(size_t)t * channels + b_off + h / share * dim + k]; }
-    __device__ __forceinline__ float v1(int t, int j, int h, int vdim, int c, const DcMade& made) const {
+    __device__ __forceinline__ float v1(int t, int j, int h, int vdim, int c, const Made& made) const {
         return made.dt[j] * xbc[(size_t)t * channels + h * vdim + c];
     }
-    __device__ __forceinline__ void make(DcMade& made, int first, int n, int h) const {
+    __device__ __forceinline__ void make(Made& made, int first, int n, int h) const {
         const int i = threadIdx.x;
         if (i < DC_TOK) {
             const float raw = to_f32(proj[(size_t)(first + min(i, n - 1)) * stride + dt_off + h]) + (dt_bias ? dt_bias[h] : 0.f);
             made.dt[i] = raw > 20.f ? raw : log1pf(expf(raw));           // softplus: beyond 20 it is its argument to the last bit
         }
         __syncthreads();
+        const int first_of = i / 16 * 16;
         if (i < DC_TOK) {
             const float neg_a = -expf(a_log[h]);
-            double sum = 0.0;
-            for (int j = 0; j <= i; ++j) sum += (double)(neg_a * made.dt[j]);
-            made.sums[i] = sum;
+            float x[16];
+#pragma unroll
+            for (int m = 0; m < 16; ++m) x[m] = neg_a * made.dt[first_of + m];
+            double upto = 0.0, behind = 0.0;
+#pragma unroll
+            for (int m = 0; m < 16; ++m) {
+                if (first_of + m <= i) upto += (double)x[m];
+                else behind += (double)x[m];
+                made.near[i][m] = (float)behind;
+            }
+            made.upto[i] = upto;
+            made.behind[i] = behind;
+            if (i % 16 == 15) made.blocks[i / 16] = upto;
+        }
+        __syncthreads();
+        if (i < DC_TOK) {
+            double sum = made.upto[i];
+            for (int b = 0; b < i / 16; ++b) sum += made.blocks[b];
+            made.start[i] = (float)sum;
         }
         __syncthreads();
     }
-    __device__ __forceinline__ float between(const DcMade& made, int i, int j) const {
-        return i == j ? 1.0f : expf((float)(made.sums[i] - made.sums[j]));
+    // from token j to token i, j <= i
+    __device__ __forceinline__ float between(const Made& made, int i, int j) const {
+        if (i / 16 == j / 16) return expf(made.near[j][i % 16]);
+        double sum = made.behind[j] + made.upto[i];
+        for (int b = j / 16 + 1; b < i / 16; ++b) sum += made.blocks[b];
+        return expf((float)sum);
     }
-    __device__ __forceinline__ float from_start(const DcMade& made, int i) const { return expf((float)made.sums[i]); }
+    __device__ __forceinline__ float from_start(const Made& made, int i) const { return expf(made.start[i]); }
     __device__ __forceinline__ float finish(float o, int t, int h, int vdim, int c) const {
         if (d_skip) o += d_skip[h] * xbc[(size_t)t * channels + h * vdim + c];
         const float z = to_f32(proj[(size_t)t * stride + z_off + h * vdim + c]);
@@ -134,7 +159,7 @@ __global__ void __launch_bounds__(DC_THREADS)
 decay_chunk_sums_kernel(float* __restrict__ U, float* __restrict__ wholes, SRC src, const int32_t* __restrict__ cu_seqlens, int heads,
                         int dim, int vdim) {
     __shared__ __align__(16) float Vs[DC_TOK * DC_STRIDE];
-    __shared__ DcMade made;
+    __shared__ typename SRC::Made made;
     const int c = blockIdx.x, b = blockIdx.y, h = blockIdx.z, tid = threadIdx.x;
     const int lane = tid & 63, r = lane & 15, g = lane >> 4, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int t0 = cu_seqlens[b], t1 = cu_seqlens[b + 1];
@@ -216,7 +241,7 @@ decay_chunk_out_kernel(float* __restrict__ out, const float* __restrict__ U, SRC
                        int dim, int vdim) {
     __shared__ __align__(16) float Qs[DC_TOK * DC_STRIDE];
     __shared__ __align__(16) float Ks[DC_TOK * DC_STRIDE];   // the keys, later the scores times the decays [64][DC_ASTRIDE]
-    __shared__ DcMade made;
+    __shared__ typename SRC::Made made;
     float* As = Ks;
     const int c = blockIdx.x, b = blockIdx.y, h = blockIdx.z, tid = threadIdx.x;
     const int lane = tid & 63, r = lane & 15, g = lane >> 4, wave = __builtin_amdgcn_readfirstlane(tid >> 6);

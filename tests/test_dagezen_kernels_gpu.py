@@ -426,6 +426,40 @@ def test_state_space_walk_in_chunks(ops, dtype, heads, groups, n, vdim, lens):
     assert error(got) <= 1.5 * error(walk) + 1e-7
 
 
+@pytest.mark.parametrize("lens", [(70,), (33, 1, 130)])
+def test_state_space_chunks_of_decays_of_every_size(ops, lens):
+    """Heads whose exponents are moderate on some tokens and beyond every sum of moderate ones on the others (A = e^25, e^30, e^35), and heads
+    that forget all with every token (A past float32, and infinite): the bounds of the test above."""
+    rng = np.random.default_rng(len(lens))
+    a_logs, n, vdim, T = [25.0, 30.0, 35.0, 89.0, np.inf], 8, 12, sum(lens)
+    heads, groups = len(a_logs), 1
+    inner = heads * vdim
+    channels, b_off, c_off = inner + 2 * n, inner, inner + n
+    raw = np.stack([(rng.normal(size=T) - (a * (rng.random(T) < 0.8) if a < 80 else 0)) for a in a_logs], 1)
+    xbc, proj = t(rng.normal(size=(T, channels))), t(np.concatenate([rng.normal(size=(T, inner)), raw], 1))
+    a_log, start = t(a_logs), t(rng.normal(size=(4, heads, n, vdim)))
+    slots, cu = [2, 0, 3][:len(lens)], np.concatenate([[0], np.cumsum(lens)])
+    x, p, want_state, want = f64(xbc), f64(proj), f64(start).copy(), np.zeros((T, inner))
+    with np.errstate(over="ignore"):
+        A = np.exp(np.array(a_logs, dtype=np.float32)).astype(np.float64)          # (float32's range: past it a decay is 0)
+    for s, slot in enumerate(slots):
+        for i in range(cu[s], cu[s + 1]):
+            for h in range(heads):
+                dt, xv, z = np.log1p(np.exp(p[i, inner + h])), x[i, h * vdim:(h + 1) * vdim], p[i, h * vdim:(h + 1) * vdim]
+                S = want_state[slot, h]
+                S[:] = np.exp(-A[h] * dt) * S + dt * np.outer(x[i, b_off:b_off + n], xv)
+                want[i, h * vdim:(h + 1) * vdim] = S.T @ x[i, c_off:] * z / (1 + np.exp(-z))
+    args = (xbc, b_off, c_off, proj, 0, inner, None, a_log, None)
+    more = (t(cu, torch.int32), t(slots, torch.int32), heads, groups, n, vdim)
+    chunked, walked = guarded(start.clone()), guarded(start.clone())
+    got, walk = ops.ssd_scan_chunked(*args, chunked, *more, max(lens)), ops.ssd_scan(*args, walked, *more)
+    for h in range(heads):                                    # (a head by itself: steps differ by many powers of ten)
+        of = slice(h * vdim, (h + 1) * vdim)
+        close(got[:, of], want[:, of], 1e-5, f"outputs, A = e^{a_logs[h]}")
+        close(chunked[:, h], want_state[:, h], 1e-5, f"state, A = e^{a_logs[h]}")
+        close(got[:, of], f64(walk[:, of]), 1e-5, f"chunks against the walk, A = e^{a_logs[h]}")
+
+
 def test_state_space_chunks_where_the_walk_waits_for_its_tokens(ops, monkeypatch):
     monkeypatch.setattr(ops, "compute_units", lambda: 256)
     pay = ops.ssd_chunks_pay
