@@ -9,14 +9,18 @@
 // walk from chunk to chunk, S0 of the next = D S0 + U, which leaves every chunk's S0 where its U was and the last
 // state in the sequence's slot (a few loads and stores an element), and every chunk's outputs (all chunks side by side).
 // Only products of decays from an earlier token to a later one appear, never their inverses: the powers d^m, m >= 0, of a fixed decay, and
-// exp of the sum of -exp(A_log) dt over the tokens from j + 1 to i.  That sum is made of those tokens' terms alone, all of one sign (in 64
-// bits, rounded once): a difference of two sums from the chunk's start would lose a small decay behind a large one, and is NaN where a decay
-// is 0.  Everything else is float32: the activations, the scores q . k, the state and all sums; the products run on the matrix
-// cores' float32 product (16x16x4), whose products and sums are 32-bit ones.  A workgroup of eight wavefronts takes one (chunk,
-// sequence, head), a wavefront sixteen columns of the results (sixteen rows of a chunk's own sum): what only its columns need comes straight
-// from memory, once, and what all need (q and k, the scores, v) passes through LDS.  What bounds it: the products, some 230 of 32
-// cycles a wavefront and chunk, and two trips to memory.  Fixed decay, 32 heads of 128 x 128, four prompts of 300 to
-// 1,800 tokens, us on the vector units : so: sums 136 : 101, outputs 357 : 163 (the carry 65 : 70).
+// those tokens' own decays multiplied in 64 bits and rounded once (a difference of exponents summed from the chunk's start would lose a
+// small one behind a large one, and is NaN where a decay is 0).  Everything else is float32: the activations, the scores q . k, the state
+// and all sums; the products run on the matrix cores' float32 product (16x16x4), whose products and sums are 32-bit ones.  A sum goes by
+// blocks of sixteen steps, the blocks two by two, a score's four products at a time two by two: one chain of 128 steps errs twice as much as
+// the walk's sums over its lanes.  Relative error against 64 bits, 2-norm, x 1e-8, outputs and states: state-space mixer, 32 heads, steps
+// that forget fast and slowly, 128 x 128: the walk 10.5 5.2, 11.1 6.7, in one chain 21.7 4.9, 20.9 6.6, so 10.5 4.9, 11.0 6.7; 64 x 64 10.0
+// 4.9, 10.4 7.2 : 16.0 4.8, 14.9 7.2 : 10.1 4.8, 10.3 7.1; fixed decay, 128 x 128 11.8 41 : 17.0 12.4 : 9.1 11.3.
+// A workgroup of eight wavefronts takes one (chunk, sequence, head), a wavefront sixteen columns of the results (sixteen rows of a
+// chunk's own sum): what only its columns need comes straight from memory, once, and what all need (q and k, the scores, v) passes
+// through LDS.  What bounds it: the products, some 230 of 32 cycles a wavefront and chunk, and two trips to memory.  32 heads
+// of 128 x 128, us the walk : in chunks: one prompt of 2,048 tokens 671 : 131 (fixed decay; 182 on the vector units, 124 with one chain a
+// sum), 287 : 134 (state-space mixer); eight of 500 620 : 248, 257 : 277; four of 300 to 1,800 490 : 372 (state-space mixer).
 // Head sizes: multiples of 4 up to 128.
 #include "api.h"
 #include "common.h"
@@ -79,8 +83,8 @@ struct DcFixed {
 
 template <typename TA>
 struct DcSteps {
-    // Sums of exponents by blocks of sixteen tokens: near[j][i % 16] from j + 1 to i of j's block, behind[j] from j + 1 to its block's end,
-    // upto[i] from its block's start to i, of whole blocks, and from the chunk's start to i.
+    // Products of decays, of 64 bits until they are whole, by blocks of sixteen tokens: near[j][i % 16] from j + 1 to i of j's block,
+    // behind[j] from j + 1 to its block's end, upto[i] from its block's start to i, of whole blocks, and from the chunk's start to i.
     struct Made {
         double behind[DC_TOK], upto[DC_TOK], blocks[DC_TOK / 16];
         float near[DC_TOK][16], start[DC_TOK], dt[DC_TOK];
@@ -107,45 +111,46 @@ struct DcSteps {
         return made.dt[j] * xbc[(size_t)t * channels + h * vdim + c];
     }
     __device__ __forceinline__ void make(Made& made, int first, int n, int h) const {
-        const int i = threadIdx.x;
+        const int i = threadIdx.x, first_of = i / 16 * 16;
         if (i < DC_TOK) {
             const float raw = to_f32(proj[(size_t)(first + min(i, n - 1)) * stride + dt_off + h]) + (dt_bias ? dt_bias[h] : 0.f);
             made.dt[i] = raw > 20.f ? raw : log1pf(expf(raw));           // softplus: beyond 20 it is its argument to the last bit
+            made.upto[i] = exp((double)-expf(a_log[h]) * (double)made.dt[i]);
         }
         __syncthreads();
-        const int first_of = i / 16 * 16;
+        double upto = 1.0, behind = 1.0;
         if (i < DC_TOK) {
-            const float neg_a = -expf(a_log[h]);
-            float x[16];
+            double d[16];
 #pragma unroll
-            for (int m = 0; m < 16; ++m) x[m] = neg_a * made.dt[first_of + m];
-            double upto = 0.0, behind = 0.0;
+            for (int m = 0; m < 16; ++m) d[m] = made.upto[first_of + m];
 #pragma unroll
             for (int m = 0; m < 16; ++m) {
-                if (first_of + m <= i) upto += (double)x[m];
-                else behind += (double)x[m];
+                if (first_of + m <= i) upto *= d[m];
+                else behind *= d[m];
                 made.near[i][m] = (float)behind;
             }
+        }
+        __syncthreads();                                     // the tokens' own decays have been read
+        if (i < DC_TOK) {
             made.upto[i] = upto;
             made.behind[i] = behind;
             if (i % 16 == 15) made.blocks[i / 16] = upto;
         }
         __syncthreads();
         if (i < DC_TOK) {
-            double sum = made.upto[i];
-            for (int b = 0; b < i / 16; ++b) sum += made.blocks[b];
-            made.start[i] = (float)sum;
+            for (int b = 0; b < i / 16; ++b) upto *= made.blocks[b];
+            made.start[i] = (float)upto;
         }
         __syncthreads();
     }
     // from token j to token i, j <= i
     __device__ __forceinline__ float between(const Made& made, int i, int j) const {
-        if (i / 16 == j / 16) return expf(made.near[j][i % 16]);
-        double sum = made.behind[j] + made.upto[i];
-        for (int b = j / 16 + 1; b < i / 16; ++b) sum += made.blocks[b];
-        return expf((float)sum);
+        if (i / 16 == j / 16) return made.near[j][i % 16];
+        double d = made.behind[j] * made.upto[i];
+        for (int b = j / 16 + 1; b < i / 16; ++b) d *= made.blocks[b];
+        return (float)d;
     }
-    __device__ __forceinline__ float from_start(const Made& made, int i) const { return expf(made.start[i]); }
+    __device__ __forceinline__ float from_start(const Made& made, int i) const { return made.start[i]; }
     __device__ __forceinline__ float finish(float o, int t, int h, int vdim, int c) const {
         if (d_skip) o += d_skip[h] * xbc[(size_t)t * channels + h * vdim + c];
         const float z = to_f32(proj[(size_t)t * stride + z_off + h * vdim + c]);
@@ -153,9 +158,30 @@ struct DcSteps {
     }
 };
 
+// The products of sixteen steps of a sum, four a matrix instruction: one after the other, or each added to nothing and the four results
+// two by two (APART).
+template <bool APART, typename A, typename B>
+__device__ __forceinline__ dc_floatx4 dc_block(const A& a, const B& b) {
+    const dc_floatx4 zero = {0.f, 0.f, 0.f, 0.f};
+    dc_floatx4 x[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) x[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b[e], APART || e == 0 ? zero : x[e - 1], 0, 0, 0);
+    return APART ? (x[0] + x[1]) + (x[2] + x[3]) : x[3];
+}
+
+// The sum of up to N such blocks (a power of two; `block(q)` of those there are), two by two.
+template <int N, typename F>
+__device__ __forceinline__ dc_floatx4 dc_tree(int from, int count, const F& block) {
+    if constexpr (N == 1) return from < count ? block(from) : dc_floatx4{0.f, 0.f, 0.f, 0.f};
+    else {
+        const dc_floatx4 first = dc_tree<N / 2>(from, count, block);
+        return first + dc_tree<N / 2>(from + N / 2, count, block);
+    }
+}
+
 // U[entry, h] = sum_j D(n - 1, j) k_j v_j^T   [dim, vdim]; wholes[entry, h] = D(n - 1, -1)
 template <typename SRC>
-__global__ void __launch_bounds__(DC_THREADS)
+__global__ void __launch_bounds__(DC_THREADS, 6)
 decay_chunk_sums_kernel(float* __restrict__ U, float* __restrict__ wholes, SRC src, const int32_t* __restrict__ cu_seqlens, int heads,
                         int dim, int vdim) {
     __shared__ __align__(16) float Vs[DC_TOK * DC_STRIDE];
@@ -193,12 +219,12 @@ decay_chunk_sums_kernel(float* __restrict__ U, float* __restrict__ wholes, SRC s
     if (16 * wave >= dim) return;
     float* Uc = U + entry * dim * vdim;
     for (int ct = 0; ct < wide / 16; ++ct) {
-        dc_floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+        const dc_floatx4 acc = dc_tree<4>(0, 4, [&](int q) {
+            float v[4];
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[q][e], Vs[(16 * q + 4 * g + e) * DC_STRIDE + 16 * ct + r], acc, 0, 0, 0);
+            for (int e = 0; e < 4; ++e) v[e] = Vs[(16 * q + 4 * g + e) * DC_STRIDE + 16 * ct + r];
+            return dc_block<false>(kv[q], v);
+        });
 #pragma unroll
         for (int e = 0; e < 4; ++e)
             if (16 * wave + 4 * g + e < dim && 16 * ct + r < vdim) Uc[(size_t)(16 * wave + 4 * g + e) * vdim + 16 * ct + r] = acc[e];
@@ -236,7 +262,7 @@ decay_chunk_carry_kernel(float* __restrict__ U, const float* __restrict__ wholes
 
 // o_i = sum_{j <= i} D(i, j) (q_i . k_j) v_j + D(i, -1) S0^T q_i for the tokens of one chunk.
 template <typename SRC>
-__global__ void __launch_bounds__(DC_THREADS)
+__global__ void __launch_bounds__(DC_THREADS, 4)
 decay_chunk_out_kernel(float* __restrict__ out, const float* __restrict__ U, SRC src, const int32_t* __restrict__ cu_seqlens, int heads,
                        int dim, int vdim) {
     __shared__ __align__(16) float Qs[DC_TOK * DC_STRIDE];
@@ -281,18 +307,17 @@ decay_chunk_out_kernel(float* __restrict__ out, const float* __restrict__ U, SRC
             const float x = S0[(size_t)min(k, dim - 1) * vdim + cc];
             sv[q][e] = k < dim ? x : 0.f;
         }
-    // scores: the ten tiles of 16 x 16 on and below the diagonal
+    // scores: the tiles of 16 x 16 on and below the diagonal, ten of a whole chunk
     dc_floatx4 score[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
         const int tile = wave + 8 * u, ti = tile < 1 ? 0 : tile < 3 ? 1 : tile < 6 ? 2 : 3, tj = tile - ti * (ti + 1) / 2;
         if (tile >= 10) break;
-        for (int k = 0; k < wide; k += 16) {
-            const dc_floatx4 qa = *reinterpret_cast<const dc_floatx4*>(Qs + (16 * ti + r) * DC_STRIDE + k + 4 * g);
-            const dc_floatx4 kb = *reinterpret_cast<const dc_floatx4*>(Ks + (16 * tj + r) * DC_STRIDE + k + 4 * g);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) score[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(qa[e], kb[e], score[u], 0, 0, 0);
-        }
+        score[u] = dc_tree<DC_MAX / 16>(0, 16 * ti < n ? wide / 16 : 0, [&](int q) {
+            const dc_floatx4 qa = *reinterpret_cast<const dc_floatx4*>(Qs + (16 * ti + r) * DC_STRIDE + 16 * q + 4 * g);
+            const dc_floatx4 kb = *reinterpret_cast<const dc_floatx4*>(Ks + (16 * tj + r) * DC_STRIDE + 16 * q + 4 * g);
+            return dc_block<true>(qa, kb);
+        });
     }
     __syncthreads();                                         // the keys have been read: the scores take their place
 #pragma unroll
@@ -307,23 +332,15 @@ decay_chunk_out_kernel(float* __restrict__ out, const float* __restrict__ U, SRC
     }
     __syncthreads();
     if (16 * wave >= vdim) return;
-#pragma unroll
+#pragma unroll 1
     for (int t = 0; t < 4; ++t) {
-        dc_floatx4 sum = {0.f, 0.f, 0.f, 0.f}, from_state = sum;
         if (16 * t >= n) break;                              // (the same for the whole workgroup)
-#pragma unroll
-        for (int q = 0; q < DC_MAX / 16; ++q) {
-            if (16 * q >= wide) break;
-            const dc_floatx4 qa = *reinterpret_cast<const dc_floatx4*>(Qs + (16 * t + r) * DC_STRIDE + 16 * q + 4 * g);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) from_state = __builtin_amdgcn_mfma_f32_16x16x4f32(qa[e], sv[q][e], from_state, 0, 0, 0);
-        }
-#pragma unroll
-        for (int q = 0; q <= t; ++q) {
-            const dc_floatx4 a = *reinterpret_cast<const dc_floatx4*>(As + (16 * t + r) * DC_ASTRIDE + 16 * q + 4 * g);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) sum = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], v[q][e], sum, 0, 0, 0);
-        }
+        const dc_floatx4 from_state = dc_tree<DC_MAX / 16>(0, wide / 16, [&](int q) {
+            return dc_block<false>(*reinterpret_cast<const dc_floatx4*>(Qs + (16 * t + r) * DC_STRIDE + 16 * q + 4 * g), sv[q]);
+        });
+        const dc_floatx4 sum = dc_tree<4>(0, t + 1, [&](int q) {
+            return dc_block<false>(*reinterpret_cast<const dc_floatx4*>(As + (16 * t + r) * DC_ASTRIDE + 16 * q + 4 * g), v[q]);
+        });
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             const int i = 16 * t + 4 * g + e;

@@ -782,11 +782,11 @@ DECAY_CHUNKS_FORCED = None    # True or False: every step of two tokens and more
 
 def decay_chunks_pay(seqs: int, tokens: int, max_new: int, heads: int, dim: int, vdim: int) -> bool:
     """Whether ``decay_scan_chunked`` is expected to take less time than ``decay_scan`` for this step (host arithmetic
-    only).  Measured on 256 compute units with heads of 64 x 32 to 128 x 128, 1 to 32 sequences and 128 to 8,192
-    tokens: the walk takes a token's latency (0.2 to 0.33 us) times the longest sequence, the chunks a workgroup's time
-    (25 to 45 us in all three launches) for as many (chunk, head) pairs as the machine holds at once; they are even at
-    128 tokens and the chunks ahead from there on, for one prompt (2,048 tokens: 67 against 672 us) and for batches of
-    prompts (32 of 1,024: 0.74 against 1.32 ms)."""
+    only).  The walk takes a token's latency (0.2 to 0.5 us) times the longest sequence, the chunks some 20 us in all
+    three launches and 0.13 us a (chunk, head) of 128 x 128 at 256 compute units.  us walk : chunks: one prompt of 128 tokens, heads of 128 x 128
+    50 : 39, 64 x 64 33 : 24, 64 x 32 33 : 22, 16 x 16 64 : 18; one of 2,048 671 : 131, 435 : 72, 434 : 42, 949 : 27; 100 of 130 (32 heads; 16 of
+    64 x 32) 2,106 : 1,107, 833 : 443, 214 : 184.  (A step of many single tokens beside a prompt loses: 40 and one of 200, 32 heads of 128 x
+    128, 171 : 315.)"""
     if DECAY_CHUNKS_FORCED is not None:
         return bool(DECAY_CHUNKS_FORCED) and max_new >= 2
     return max_new >= DECAY_CHUNKS_FROM
@@ -2113,17 +2113,17 @@ SSD_CHUNKS_WORKSPACE = 1 << 28   # floats of workspace at most: a gigabyte, beyo
 def ssd_chunks_pay(new_counts, heads: int, n: int, vdim: int) -> bool:
     """Whether ``ssd_scan_chunked`` is expected to take less time than ``ssd_scan`` (host arithmetic only).  The walk takes a token's latency
     times the longest sequence, 0.145, 0.17 and 0.27 us with one, two and four columns a lane (``walk_columns`` of walk.h; 0.44 us for states
-    of up to 64 rows), or what the machine does at most, 2 ns a token and head of 128 x 128 (0.7 of 64 x 64); the chunks 25 us and 0.13
-    (0.07) us a chunk and head.  256 compute units, us walk : chunks; 32 heads of 128 x 128, one prompt of 256 43 : 48, 512 82 : 57, 2,048 296 :
-    130, four of 300 to 1,800 484 : 359, eight of 500 255 : 268, 32 of 1,000 1,941 : 2,170, 40 single tokens beside a prompt of 200 92 : 324;
-    32 heads of 64 x 64, one of 64 33 : 29, 2,048 910 : 82, eight of 500 223 : 134, 32 of 128 98 : 135."""
+    of up to 64 rows), or what the machine does at most, 2 ns a token and head of 128 x 128 (0.7 of 64 x 64); the chunks 25 us and 0.135
+    (0.07) us a chunk and head.  256 compute units, us walk : chunks; 32 heads of 128 x 128, one prompt of 256 43 : 48, 512 82 : 58, 2,048 287 :
+    134, four of 300 to 1,800 490 : 372, eight of 500 257 : 277, 32 of 1,000 1,906 : 2,204, 40 single tokens beside a prompt of 200 92 : 324;
+    32 heads of 64 x 64, one of 64 33 : 28, 2,048 908 : 85, eight of 500 224 : 135, 32 of 128 98 : 138."""
     units, longest, size = compute_units(), max(new_counts), n * vdim / 16384
     if _decay_chunks_workspace(len(new_counts), sum(new_counts), heads, n, vdim) > SSD_CHUNKS_WORKSPACE:
         return False
     columns, waves = len(new_counts) * heads * vdim, 8 * units
     a_token = 0.44 if n <= 64 else 0.145 if columns <= 2 * waves else 0.17 if columns <= 4 * waves else 0.27
     walk = max(longest * a_token, sum(new_counts) * heads * (0.0003 + 0.0017 * size) * 256 / units)
-    return 25 + sum(-(-k // 64) for k in new_counts) * heads * (0.05 + 0.08 * size) * 256 / units < 0.9 * walk
+    return 25 + sum(-(-k // 64) for k in new_counts) * heads * (0.05 + 0.085 * size) * 256 / units < 0.9 * walk
 
 
 def ssd_chunks_fit(n: int, vdim: int, channels: int, offsets: tuple) -> bool:

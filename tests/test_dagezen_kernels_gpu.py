@@ -460,6 +460,30 @@ def test_state_space_chunks_of_decays_of_every_size(ops, lens):
         close(got[:, of], f64(walk[:, of]), 1e-5, f"chunks against the walk, A = e^{a_logs[h]}")
 
 
+@pytest.mark.parametrize("n, vdim, bias", [(128, 64, 1.0), (128, 32, -3.0), (64, 64, -3.0)])
+def test_state_space_chunks_err_no_more_than_the_walk(ops, n, vdim, bias):
+    """Distance from 64 bits (2-norm), for steps that forget fast and slowly: of the outputs and the states that of the walk, up to a tenth
+    for what differs by chance (a sum over 128 rows in one chain has twice as much)."""
+    rng = np.random.default_rng(n + vdim)
+    heads, groups, T = 8, 2, 200
+    inner, gn = heads * vdim, groups * n
+    xbc, proj = t(rng.normal(size=(T, inner + 2 * gn))), t(rng.normal(size=(T, inner + heads)), torch.bfloat16)
+    dt_bias, a_log, start = t(rng.normal(size=heads) + bias), t(np.log(rng.uniform(1, 16, heads))), t(rng.normal(size=(1, heads, n, vdim)))
+    x, p = f64(xbc), f64(proj)
+    dt = np.log1p(np.exp(p[:, inner:] + f64(dt_bias)))
+    B, C = (np.repeat(x[:, o:o + gn].reshape(T, groups, n), heads // groups, 1) for o in (inner, inner + gn))
+    decay, xv, S, want = np.exp(-np.exp(f64(a_log)) * dt), x[:, :inner].reshape(T, heads, vdim), f64(start)[0].copy(), []
+    for i in range(T):
+        S = decay[i][:, None, None] * S + (dt[i][:, None] * B[i])[:, :, None] * xv[i][:, None, :]
+        want.append(np.einsum("hn,hnv->hv", C[i], S).reshape(-1) * p[i, :inner] / (1 + np.exp(-p[i, :inner])))
+    args = (xbc, inner, inner + gn, proj, 0, inner, dt_bias, a_log, None)
+    more = (t([0, T], torch.int32), t([0], torch.int32), heads, groups, n, vdim)
+    chunked, walked = guarded(start.clone()), guarded(start.clone())
+    got, walk = ops.ssd_scan_chunked(*args, chunked, *more, T), ops.ssd_scan(*args, walked, *more)
+    error = lambda y, w: np.linalg.norm(f64(y) - w) / np.linalg.norm(w)
+    assert error(got, np.stack(want)) <= 1.1 * error(walk, np.stack(want)) and error(chunked[0], S) <= 1.1 * error(walked[0], S)
+
+
 def test_state_space_chunks_where_the_walk_waits_for_its_tokens(ops, monkeypatch):
     monkeypatch.setattr(ops, "compute_units", lambda: 256)
     pay = ops.ssd_chunks_pay
