@@ -7,9 +7,9 @@
 // For Higher-Precision Computations", 2019).  Here x = a + (b + c) 2^-16 exactly, for every float32: the parts are cut off, not
 // rounded, and b and c are kept 2^16 times as large, so that the last bit of the smallest float32, 2^-149, is still one of bfloat16's
 // (2^-133; the matrix cores take subnormal numbers as they are).  Every product of a part and a weight is exact in float32 above
-// the subnormal numbers; the first part's sum and that of the two lower ones, whose last bits lie far below what the first rounds away, are
-// float32 sums of their own, added at the end: what is rounded is the additions alone, as in a chain of multiply-adds, and there
-// are fewer of them.  Relative error against
+// the subnormal numbers, and the sums of the three parts are float32 sums of their own, added at the end: what is rounded is the
+// additions alone, as in a chain of multiply-adds, and there are fewer of them.  (The lower two in one sum would be twice as many
+// additions at the size of the second part's: where the first parts cancel, K = 1,024, 2.65e-7 instead of 1.75e-7.)  Relative error against
 // 64 bits (2-norm, normal x and weights): at K = 1,024 1.9e-7 where the chain of multiply-adds has 5.7e-7, at 3,072
 // 3.4e-7 : 9.9e-7.  The three products run at a third of the bfloat16 rate, ten times the vector units' multiply-adds.
 // An infinity, a NaN or a number past 2^119 has no such parts, but leaves an infinity or NaN in every sum it enters: such an
@@ -69,7 +69,7 @@ __device__ __forceinline__ void chain_again(float* out, const float* x, const bf
 // buffers; x is split once, on its way into LDS.  A row of a stage is 128 bytes, its 16-byte pieces exchanged by the row's number so
 // that reads of a fragment's sixteen rows meet every bank equally.  What bounds a tile is its chain of stages, each the
 // split (half as many cycles of the vector units as the matrix cores take for it), LDS both ways and a barrier: 0.4 us for 32 x 32, 0.8 for
-// 64 x 128 with eight wavefronts (0.95 with four), 1.65 for 128 x 192.
+// 64 x 128 with eight wavefronts (0.95 with four).
 #define FT_BK 64
 // A thread's share of a stage on its way through registers: 16 bytes of bfloat16 (8 k) of rows row + THREADS / 8 i.
 template <int XN, int WR, int THREADS>
@@ -100,7 +100,7 @@ struct TileStage {
 };
 
 template <int MT, int NT>
-__device__ __forceinline__ void multiply_stage(f32_floatx4 (&acc)[MT][NT][2], const uint4* xs, const uint4* ws, int plane, int wm,
+__device__ __forceinline__ void multiply_stage(f32_floatx4 (&acc)[MT][NT][3], const uint4* xs, const uint4* ws, int plane, int wm,
                                                int wn, int r, int g) {
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
@@ -118,7 +118,7 @@ __device__ __forceinline__ void multiply_stage(f32_floatx4 (&acc)[MT][NT][2], co
             for (int i = 0; i < MT; ++i)
 #pragma unroll
                 for (int j = 0; j < NT; ++j)
-                    acc[i][j][q > 0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j], xf[i][q], acc[i][j][q > 0], 0, 0, 0);
+                    acc[i][j][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j], xf[i][q], acc[i][j][q], 0, 0, 0);
     }
 }
 
@@ -143,13 +143,13 @@ gemm_f32_tile_kernel(float* __restrict__ out, const float* __restrict__ x, const
 #pragma unroll
     for (int i = 0; i < WR; ++i) wp[i] = w + (size_t)min(n0 + row + STEP * i, N - 1) * K;
     const int slot = row * 8 + (piece ^ (row & 7));         // (STEP rows on, a multiple of eight, the exchange is the same)
-    f32_floatx4 acc[MT][NT][2];
+    f32_floatx4 acc[MT][NT][3];
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
         for (int j = 0; j < NT; ++j)
 #pragma unroll
-            for (int p = 0; p < 2; ++p) acc[i][j][p] = f32_floatx4{0.f, 0.f, 0.f, 0.f};
+            for (int p = 0; p < 3; ++p) acc[i][j][p] = f32_floatx4{0.f, 0.f, 0.f, 0.f};
     // DEEP stages are under way in registers while another is multiplied: a stage of a small tile is multiplied in a fraction of the
     // time that its loads take.
     TileStage<XN, WR, THREADS> ahead[DEEP];
@@ -179,7 +179,7 @@ gemm_f32_tile_kernel(float* __restrict__ out, const float* __restrict__ x, const
             float sum[4];
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                sum[e] = acc[i][j][0][e] + acc[i][j][1][e] * (1.f / F32_LOWER);
+                sum[e] = acc[i][j][0][e] + (acc[i][j][1][e] + acc[i][j][2][e]) * (1.f / F32_LOWER);
                 bad |= !(fabsf(sum[e]) < INFINITY);
             }
             float* o = out + (size_t)m * N + n;
@@ -255,19 +255,18 @@ extern "C" int ri_gemm_f32(float* out, const float* x, const void* w, int w_dtyp
     else if (!aligned)
         gemm_f32_kernel<bf16_t><<<grid, 256, 0, s>>>(out, x, (const bf16_t*)w, m, n, k);
     else {
-        // The order of a row's sums is the same in every tile.  The largest tiles, 128 x 192, where their last round of workgroups (one a
-        // compute unit) leaves little of the machine idle; 64 x 128 from three quarters of the machine on, else 32 x 64 as soon as 32 x 32
-        // would need a second round.  us for 32 x 32 / 32 x 64 / 64 x 128 / 128 x 192 (rows; columns x K): 759; 6,144 x 1,024 60 / 44 / 46 /
-        // 38, 4,096 x 1,024 43 / 32 / 31 / 36, 1,024 x 3,072 33 / 30 / 39 / 83; 1,200; 4,096 x 1,024 65 / 54 / 53 / 43, 6,144 x 1,024 102 / 73 / 60 / 77;
-        // 400; 4,096 x 1,024 27 / 22 / 18 / 35, 6,144 x 1,024 37 / 28 / 30 / 37; 200; 4,096 x 1,024 17 / 14 / 17 / 34; 2,400; 6,144 x 1,024 252 / 149 /
-        // 121 / 117; 33; 1,024 x 3,072 20 / 22 / 38 / 80, 4,096 x 1,024 8.8 / 9.6 / 16 / 30 (the vector units' form: 759; 1,024 x 3,072 363).
+        // The order of a row's sums is the same in every tile.  64 x 128 from three quarters of the machine on (one workgroup a compute unit), else
+        // 32 x 64 as soon as 32 x 32 would need a second round.  us for 32 x 32 / 32 x 64 / 64 x 128 (rows; columns x K): 759; 6,144 x
+        // 1,024 60 / 44 / 49, 4,096 x 1,024 43 / 32 / 33, 1,024 x 3,072 33 / 30 / 39; 1,200; 4,096 x 1,024 65 / 54 / 47, 6,144 x 1,024 102 / 73 / 65;
+        // 400; 4,096 x 1,024 27 / 22 / 20, 6,144 x 1,024 37 / 28 / 32; 200; 4,096 x 1,024 17 / 14 / 17; 2,400; 6,144 x 1,024 252 / 149 / 128; 33;
+        // 1,024 x 3,072 20 / 22 / 38, 4,096 x 1,024 8.8 / 9.6 / 16 (the vector units' form: 759; 1,024 x 3,072 363).  (128 x 192 has no registers
+        // for three sums a result: with a stage less under way 48 and 46 us at 759; 6,144 and 1,200; 4,096, 136 at 2,400; 6,144.)
         // Up to 32 rows half of a tile of 64 would be padding: 151,936 x 1,024 at one row 77 / 57 / 75.
         const auto tiles = [&](int rows, int cols) { return (long)((m + rows - 1) / rows) * ((n + cols - 1) / cols); };
         const bf16_t* wb = (const bf16_t*)w;
         RI_REQUIRE(tiles(32, 32) + 8 * ((m + 31) / 32) < (1L << 31), "gemm_f32: %d x %d exceed one launch", m, n);
-        const long units = ri_compute_units(), largest = tiles(128, 192), rounds = (largest + units - 1) / units;
-        if (m > 64 && 10 * largest >= 7 * rounds * units) launch_tiles<2, 6, 4, 2, 2>(out, x, wb, m, n, k, s);
-        else if (m > 32 && 4 * tiles(64, 128) >= 3 * units) launch_tiles<2, 2, 2, 4, 2>(out, x, wb, m, n, k, s);
+        const long units = ri_compute_units();
+        if (m > 32 && 4 * tiles(64, 128) >= 3 * units) launch_tiles<2, 2, 2, 4, 2>(out, x, wb, m, n, k, s);
         else if (tiles(32, 32) > units) launch_tiles<1, 2, 2, 2, 2>(out, x, wb, m, n, k, s);
         else launch_tiles<1, 1, 2, 2, 4>(out, x, wb, m, n, k, s);
     }

@@ -854,14 +854,31 @@ def test_gemm_f32_on_the_matrix_cores(ops, m, n, k):
 
 @pytest.mark.parametrize("m,n,k", [(385, 4096, 200), (1153, 4096, 64), (1200, 4096, 392), (31, 4096, 328)])
 def test_gemm_f32_tiles_of_a_full_machine(ops, m, n, k):
-    """The tiles that a whole machine chooses, 64 x 128 and 128 x 192, their edges and stages that are not whole, and the smallest ones'
-    four stages; the bound of the test above."""
+    """The tiles of 64 x 128 that a whole machine chooses, their edges and stages that are not whole, and the smallest ones' four stages;
+    the bound of the test above."""
     rng = np.random.default_rng(m + n + k)
     x, w = t(rng.normal(size=(m, k))), t(rng.normal(size=(n, k)), torch.bfloat16)
     got = f64(ops.gemm_f32(x, w))
     bound = (k / 32 + 32) * 2.0 ** -24 * (np.abs(f64(x)) @ np.abs(f64(w)).T)
     assert (np.abs(got - f64(x) @ f64(w).T) <= bound).all()
     assert np.array_equal(got[m - 30:], f64(ops.gemm_f32(x[m - 30:].contiguous(), w))), "a row's sums depend on the other rows"
+
+
+@pytest.mark.parametrize("m, n", [(5, 48), (70, 72)])
+def test_gemm_f32_where_the_first_parts_cancel(ops, m, n):
+    """Pairs of k with opposite weights and x that agree in their first eight bits: what is left are the lower parts' products, whose sum is
+    rounded once for each of the S = K / 32 steps of the second part.  A rounding errs by some 2.5e-8 of the partial sum, which after s steps is
+    sqrt(s / S) of the result (2-norm): sqrt(S / 2) 2.5e-8 = 1.0e-7 at K = 1,024, and more within the steps (1.75e-7 measured); the third
+    part's additions in the same sum make it sqrt(2) as much (2.65e-7 measured)."""
+    rng = np.random.default_rng(m)
+    k = 1024
+    top = rng.normal(size=(m, k // 2)).astype(np.float32).view(np.uint32) & np.uint32(0xFFFF0000)
+    x = np.repeat(top, 2, 1) | rng.integers(0, 1 << 16, (m, k), dtype=np.uint32)
+    w = np.repeat(rng.normal(size=(n, k // 2)), 2, 1) * np.where(np.arange(k) % 2, -1.0, 1.0)
+    x, w = t(x.view(np.float32)), t(w, torch.bfloat16)
+    want = f64(x) @ f64(w).T
+    error = np.linalg.norm(f64(ops.gemm_f32(x, w)) - want) / np.linalg.norm(want)
+    assert error <= 2.2e-7, error
 
 
 @pytest.mark.parametrize("top", [-100, -112, -118, -126, -135])
