@@ -33,19 +33,29 @@ static int check_common(const char* name, int heads, int kv_heads, int head_dim,
 // walks whole.  us with one : two tiles a wavefront (heads of 128 over 8; the workgroups that two tiles make): prompts of 500, 1,500 and 900, 32
 // heads (728) 60 : 82; 12 of 200 to 1,024, 16 heads (896) 44 : 53; 16 of 16 to 1,024 (1,016) 65 : 68, 32 (2,408) 127 : 133; eight of 500, 32 heads
 // (1,024) 41 : 41; four of 300 to 1,800 (1,240) 150 : 141; one of 2,048 (512) 64 : 73, 3,072 (768) 140 : 122, 8,192 of 16 heads (1,024) 387 : 342.
+// Single tokens beside prompts bring the average down and take longer themselves with two tiles: such a step wants a hundred workgroups' tokens
+// of the sequence that a token is of on average (`weighted`, the sum of squares over the sum).  With single tokens at 1,000 keys: one of 8,192 and
+// 40 (16 heads) 403 : 365, two of 4,096 and 100 (32) 475 : 446, one of 3,000 and 63 157 : 192, one of 2,048 and 256 251 : 319, eight of 1,024 and
+// eight (16) 90 : 103.
 #define PREFILL_MIN_WGS_PER_CU 3
 #define PREFILL_MIN_WGS_PER_SEQ 12
-static int prefill_tiles(int head_dim, int group, int max_new, int seqs, int kv_heads, int tokens) {
+#define PREFILL_MIN_WGS_WEIGHTED 100
+static int prefill_tiles(int head_dim, int group, int max_new, int seqs, int kv_heads, int tokens, int weighted) {
     int nt = head_dim <= 64 ? 4 : 2;
     while (nt > 1 && group <= 16 * (nt / 2)) {
         const int of_wg = 4 * ((16 * nt) / group);
         const long wgs = head_dim <= 64 ? (long)((max_new + of_wg - 1) / of_wg) * seqs * kv_heads
                                         : (tokens + (long)seqs * of_wg / 2) / of_wg * kv_heads;
         if (wgs >= (long)PREFILL_MIN_WGS_PER_CU * ri_compute_units() &&
-            (head_dim <= 64 || tokens >= (long)PREFILL_MIN_WGS_PER_SEQ * of_wg * seqs)) break;
+            (head_dim <= 64 || tokens >= (long)PREFILL_MIN_WGS_PER_SEQ * of_wg * seqs || weighted >= PREFILL_MIN_WGS_WEIGHTED * of_wg)) break;
         nt /= 2;
     }
     return nt;
+}
+
+// The column tiles a wavefront takes of a step (host code only).
+extern "C" int ri_attention_prefill_tiles(int head_dim, int group, int max_new, int seqs, int kv_heads, int tokens, int weighted) {
+    return prefill_tiles(head_dim, group, max_new, seqs, kv_heads, tokens, weighted);
 }
 
 extern "C" int ri_attention_prefill_kept_bf16(void* out, const void* qkv, int q_stride, const void* k_pages,
@@ -53,7 +63,7 @@ extern "C" int ri_attention_prefill_kept_bf16(void* out, const void* qkv, int q_
                                               const int32_t* page_table, int table_width, int seqs, int max_new,
                                               int heads, int kv_heads, int head_dim, int page_size, int window, int chunk,
                                               float scale, float softcap, const float* slopes, int keep_first,
-                                              const float* sinks, int tokens, void* stream) {
+                                              const float* sinks, int tokens, int weighted, void* stream) {
     RI_REQUIRE(chunk >= 0 && (chunk == 0 || window <= 0), "attention_prefill: chunks of %d beside a window of %d", chunk, window);
     const Reach reach = {window, chunk};
     RI_REQUIRE(keep_first >= 0, "attention_prefill_bf16: %d first tokens kept", keep_first);
@@ -62,7 +72,7 @@ extern "C" int ri_attention_prefill_kept_bf16(void* out, const void* qkv, int q_
     if (check_common("attention_prefill_bf16", heads, kv_heads, head_dim, page_size, q_stride, table_width)) return 1;
     const int group = heads / kv_heads;
     RI_REQUIRE(seqs > 0 && seqs <= 65535 && max_new > 0, "attention_prefill_bf16: seqs %d, max_new %d", seqs, max_new);
-    const int nt_tiles = prefill_tiles(head_dim, group, max_new, seqs, kv_heads, tokens);
+    const int nt_tiles = prefill_tiles(head_dim, group, max_new, seqs, kv_heads, tokens, weighted);
     RI_REQUIRE(group <= 16 * nt_tiles, "attention_prefill_bf16: %d query heads per kv head (at most %d)", group,
                16 * nt_tiles);
     const int tile_tokens = (16 * nt_tiles) / group;
@@ -106,7 +116,7 @@ extern "C" int ri_attention_prefill_bf16(void* out, const void* qkv, int q_strid
                                          float scale, float softcap, const float* slopes, void* stream) {
     return ri_attention_prefill_kept_bf16(out, qkv, q_stride, k_pages, v_pages, cu_seqlens, tok_pos, page_table, table_width,
                                           seqs, max_new, heads, kv_heads, head_dim, page_size, window, 0, scale, softcap, slopes,
-                                          0, nullptr, (int)(max_new * (long)seqs < 1 << 30 ? max_new * (long)seqs : 1 << 30), stream);
+                                          0, nullptr, (int)(max_new * (long)seqs < 1 << 30 ? max_new * (long)seqs : 1 << 30), max_new, stream);
 }
 
 // Whether the streaming kernel ranks the step's sequences by their lengths (host code only).

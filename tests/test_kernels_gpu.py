@@ -533,6 +533,19 @@ def test_prompt_attention_with_two_tiles_a_wavefront(ops, heads):
     close(out, want, BF16_OUT, "prefill attention, two tiles a wavefront")
 
 
+def test_prompt_attention_tiles_follow_the_tokens_of_the_long_prompts(ops):
+    """Heads of 128 on 256 compute units, as measured beside the rule: two tiles a wavefront for long prompts, for very long ones also
+    where single tokens stand beside them; one for short prompts and for steps that two would not fill."""
+    if not EMULATED and torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("measured on 256 compute units")
+    tiles = ops.attention_prefill_tiles
+    ragged = [200 + i * 824 // 11 for i in range(12)]
+    assert tiles([8192], 16, 8, 128) == 2 and tiles([8192] + [1] * 40, 16, 8, 128) == 2 and tiles([4096, 4096] + [1] * 200, 32, 8, 128) == 2
+    assert tiles([3072], 32, 8, 128) == 2 and tiles([300, 900, 1500, 1800], 32, 8, 128) == 2
+    assert tiles([500, 1500, 900], 32, 8, 128) == 1 and tiles(ragged, 16, 8, 128) == 1 and tiles([2048], 32, 8, 128) == 1
+    assert tiles([3000] + [1] * 63, 32, 8, 128) == 1 and tiles([1024] * 8 + [1] * 8, 16, 8, 128) == 1 and tiles([1] * 1000, 16, 8, 128) == 1
+
+
 @pytest.mark.skipif(EMULATED, reason="eight thousand tokens")
 @pytest.mark.parametrize("cap", [None, 20.0])
 def test_prompt_attention_of_a_long_prompt_is_its_pieces(ops, cap):
