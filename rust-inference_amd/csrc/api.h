@@ -530,7 +530,7 @@ int ri_attention_prefill_padded_bf16(void* out, const void* qkv, int q_stride, c
                                      const int32_t* cu_seqlens, const int32_t* tok_pos, const int32_t* page_table,
                                      int table_width, int seqs, int max_new, int heads, int kv_heads, int dim, int vdim,
                                      int page_size, int window, int chunk, float scale, float softcap, const float* slopes,
-                                     int keep_first, const float* sinks, void* stream);
+                                     int keep_first, const float* sinks, int tokens, void* stream);
 int ri_attention_decode_padded_bf16(void* out, float* workspace, const void* qkv, int q_stride, const void* k_pages,
                                     const void* v_pages, const int32_t* tok_pos, const int32_t* page_table, int table_width,
                                     int seqs, int max_chunks, int heads, int kv_heads, int dim, int vdim, int page_size,

@@ -78,7 +78,8 @@ extern "C" int ri_attention_prefill_kept_bf16(void* out, const void* qkv, int q_
     const int tile_tokens = (16 * nt_tiles) / group;
     const int tiles = (max_new + 4 * tile_tokens - 1) / (4 * tile_tokens);
     RI_REQUIRE(tiles <= 65535, "attention_prefill_bf16: %d tiles of tokens exceed one launch", tiles);
-    dim3 grid(kv_heads, seqs, tiles);
+    int long_runs;
+    const dim3 grid = prefill_grid(kv_heads, seqs, tiles, 4 * tile_tokens, tokens, long_runs);
     const float scale_log2 = scale * 1.4426950408889634f;
     hipStream_t s = (hipStream_t)stream;
     const int form = slopes ? PREFILL_ANY : cap_pre != 0.f ? PREFILL_CAPPED : PREFILL_PLAIN;
@@ -86,7 +87,7 @@ extern "C" int ri_attention_prefill_kept_bf16(void* out, const void* qkv, int q_
     attn_prefill_mfma_kernel<DH, NT, DH, false, FORM><<<grid, 256, 0, s>>>(                                      \
         (bf16_t*)out, (const bf16_t*)qkv, q_stride, (const bf16_t*)k_pages, (const bf16_t*)v_pages,              \
         cu_seqlens, tok_pos, page_table, table_width, heads, kv_heads, reach, scale_log2, cap_pre,              \
-        cap_post, slopes, 1.f / scale, keep_first, sinks)
+        cap_post, slopes, 1.f / scale, keep_first, sinks, seqs, long_runs)
 #define RI_PREFILL_CASE(DH, NT)                                                                                  \
     case DH * 8 + NT:                                                                                            \
         if (form == PREFILL_PLAIN) RI_PREFILL_GO(DH, NT, PREFILL_PLAIN);                                         \

@@ -35,7 +35,7 @@ extern "C" int ri_attention_prefill_padded_bf16(void* out, const void* qkv, int 
                                                 const int32_t* page_table, int table_width, int seqs, int max_new,
                                                 int heads, int kv_heads, int dim, int vdim, int page_size, int window, int chunk,
                                                 float scale, float softcap, const float* slopes, int keep_first,
-                                                const float* sinks, void* stream) {
+                                                const float* sinks, int tokens, void* stream) {
     RI_REQUIRE(chunk >= 0 && (chunk == 0 || window <= 0), "attention_prefill_padded: chunks of %d beside a window of %d", chunk, window);
     const Reach reach = {window, chunk};
     RI_REQUIRE(keep_first >= 0, "attention_prefill_padded: %d first tokens kept", keep_first);
@@ -53,7 +53,8 @@ extern "C" int ri_attention_prefill_padded_bf16(void* out, const void* qkv, int 
     const int tile_tokens = (16 * nt_tiles) / group;
     const int tiles = (max_new + 4 * tile_tokens - 1) / (4 * tile_tokens);
     RI_REQUIRE(tiles <= 65535, "attention_prefill_padded: %d tiles of tokens exceed one launch", tiles);
-    dim3 grid(kv_heads, seqs, tiles);
+    int long_runs;
+    const dim3 grid = prefill_grid(kv_heads, seqs, tiles, 4 * tile_tokens, tokens, long_runs);
     const float scale_log2 = scale * 1.4426950408889634f;
     hipStream_t s = (hipStream_t)stream;
 #define RI_CASE(DH, NT, DV)                                                                                       \
@@ -61,7 +62,7 @@ extern "C" int ri_attention_prefill_padded_bf16(void* out, const void* qkv, int 
         attn_prefill_mfma_kernel<DH, NT, DV, true><<<grid, 256, 0, s>>>(                                           \
             (bf16_t*)out, (const bf16_t*)qkv, q_stride, (const bf16_t*)k_pages, (const bf16_t*)v_pages,          \
             cu_seqlens, tok_pos, page_table, table_width, heads, kv_heads, reach, scale_log2, cap_pre,          \
-            cap_post, slopes, 1.f / scale, keep_first, sinks, dim, vdim);                                         \
+            cap_post, slopes, 1.f / scale, keep_first, sinks, seqs, long_runs, dim, vdim);                        \
         break;
 #define RI_CASES(DH)                                                                                              \
     RI_CASE(DH, 2, 64) RI_CASE(DH, 1, 64) RI_CASE(DH, 2, 96) RI_CASE(DH, 1, 96) RI_CASE(DH, 2, 128) RI_CASE(DH, 1, 128) \

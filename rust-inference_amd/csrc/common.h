@@ -102,17 +102,17 @@ __device__ __forceinline__ float block_max(float v, float* scratch) {
 // A run of up to `per` neighbouring pieces of one sequence's new tokens, `each` pieces a token: the sequence's first new token and
 // how many it brings, the run's first piece and how many it has.
 struct Run {
-    int start, tokens, first, count;
+    int seq, start, tokens, first, count;
 };
 
-// Run `index` of the sequences that bring `least` new tokens and more.  Every wavefront works it out for itself, a lane a sequence
+// Run `index` of the sequences that bring `least` to `most` new tokens.  Every wavefront works it out for itself, a lane a sequence
 // (a sequence after the other would cost hundreds of them a trip to memory each).  False: there is no such run.
 __device__ __forceinline__ bool run_of(int index, const int32_t* __restrict__ cu_seqlens, int seqs, int least, int per, int each,
-                                       Run& run) {
+                                       Run& run, int most = 0x7fffffff) {
     const int lane = threadIdx.x & (RI_WAVE - 1);
     for (int s0 = 0; s0 < seqs; s0 += RI_WAVE) {
         const int s = min(s0 + lane, seqs - 1), start = cu_seqlens[s], n = s0 + lane < seqs ? cu_seqlens[s + 1] - start : 0;
-        const int runs = n >= least ? (n * each + per - 1) / per : 0;
+        const int runs = n >= least && n <= most ? (n * each + per - 1) / per : 0;
         int upto = runs;                                      // of the sequences up to this lane's
 #pragma unroll
         for (int d = 1; d < RI_WAVE; d *= 2) {
@@ -123,6 +123,7 @@ __device__ __forceinline__ bool run_of(int index, const int32_t* __restrict__ cu
         const unsigned long long past = __ballot(upto > index);
         if (past) {
             const int who = __builtin_ctzll(past), at = (index - __shfl(upto - runs, who, RI_WAVE)) * per;
+            run.seq = s0 + who;
             run.start = __builtin_amdgcn_readfirstlane(__shfl(start, who, RI_WAVE));
             run.tokens = __builtin_amdgcn_readfirstlane(__shfl(n, who, RI_WAVE));
             run.first = __builtin_amdgcn_readfirstlane(at);

@@ -123,7 +123,7 @@ _SIGNATURES = {
     "ri_attention_padded_fits": [c_int, c_int, c_int, c_int],
     "ri_attention_prefill_padded_bf16": [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int,
                                          c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_float, c_void_p, c_int,
-                                         c_void_p, c_void_p],
+                                         c_void_p, c_int, c_void_p],
     "ri_attention_decode_padded_bf16": [c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_int,
                                         c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_float, c_void_p, c_int,
                                         c_int, c_void_p, c_void_p],
@@ -1299,7 +1299,7 @@ def attention_prefill_padded(qkv, k_pages, v_pages, cu_seqlens, tok_pos, page_ta
           _dev(cu_seqlens, "cu_seqlens", torch.int32, (seqs + 1,)), _dev(tok_pos, "tok_pos", torch.int32, (tokens,)),
           _dev(page_table, "page_table", torch.int32), page_table.shape[1], seqs, max_new, heads, kv_heads, dim, vdim, page_size,
           int(window or 0), int(chunk or 0), float(scale), float(softcap or 0.0), _opt(slopes, "slopes", torch.float32, (heads,)),
-          int(keep_first or 0), _opt(sinks, "sinks", torch.float32, (heads,)), _stream())
+          int(keep_first or 0), _opt(sinks, "sinks", torch.float32, (heads,)), tokens, _stream())
     return out
 
 

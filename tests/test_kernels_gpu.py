@@ -546,6 +546,35 @@ def test_prompt_attention_tiles_follow_the_tokens_of_the_long_prompts(ops):
     assert tiles([3000] + [1] * 63, 32, 8, 128) == 1 and tiles([1024] * 8 + [1] * 8, 16, 8, 128) == 1 and tiles([1] * 1000, 16, 8, 128) == 1
 
 
+@pytest.mark.parametrize("heads, kv_heads, dh, vdim", [(16, 1, 128, 128), (32, 2, 64, 64), (15, 1, 32, 32), (16, 1, 24, 40)])
+def test_prompt_attention_of_a_prompt_among_single_tokens(ops, heads, kv_heads, dh, vdim):
+    """Steps whose grid would be empty for the most part go run by run: prompts of one workgroup's tokens, one more and many, first, last
+    and between single tokens; the same bits as every sequence by itself."""
+    rng = np.random.default_rng(dh)
+    new = [1] * 5 + [33] + [1] * 2 + [4, 5] + [1] * 4 + [17]
+    before = [int(x) for x in rng.integers(0, 70, len(new))]
+    pages = [-(-(a + n) // 32) for a, n in zip(before, new)]
+    table = np.full((len(new), max(pages)), -1, dtype=np.int32)
+    order = iter(rng.permutation(sum(pages)))
+    for b, n in enumerate(pages):
+        table[b, :n] = [next(order) for _ in range(n)]
+    kp, vp = (t(rng.normal(size=(sum(pages), kv_heads) + shape), torch.bfloat16) for shape in ((32, dh), (vdim, 32)))
+    qkv, at = t(rng.normal(size=(sum(new), heads * dh)), torch.bfloat16), np.concatenate([[0], np.cumsum(new)])
+    pos = [a + i for a, n in zip(before, new) for i in range(n)]
+
+    def run(seqs):
+        n, rows = [new[b] for b in seqs], [i for b in seqs for i in range(at[b], at[b + 1])]
+        args = (t(f64(qkv)[rows], torch.bfloat16), kp, vp, t(np.concatenate([[0], np.cumsum(n)]), torch.int32), t([pos[i] for i in rows], torch.int32),
+                t(table[seqs], torch.int32), len(n), max(n), heads, kv_heads)
+        if dh == vdim:
+            return f64(ops.attention_prefill_bf16(*args, dh, None, dh ** -0.5, new_counts=n))
+        return f64(ops.attention_prefill_padded(*args, None, dh ** -0.5))
+
+    together = run(list(range(len(new))))
+    for b in range(len(new)):
+        assert np.array_equal(together[at[b]:at[b + 1]], run([b])), f"sequence {b} of {new[b]} tokens"
+
+
 @pytest.mark.skipif(EMULATED, reason="eight thousand tokens")
 @pytest.mark.parametrize("cap", [None, 20.0])
 def test_prompt_attention_of_a_long_prompt_is_its_pieces(ops, cap):
