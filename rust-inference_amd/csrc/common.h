@@ -100,9 +100,9 @@ __device__ __forceinline__ float block_max(float v, float* scratch) {
 }
 
 // A run of up to `per` neighbouring pieces of one sequence's new tokens, `each` pieces a token: the sequence's first new token and
-// how many it brings, the run's first piece and how many it has.
+// how many it brings, the run's first piece and how many it has, and the sequence (last: the members before it are set by place elsewhere).
 struct Run {
-    int seq, start, tokens, first, count;
+    int start, tokens, first, count, seq;
 };
 
 // Run `index` of the sequences that bring `least` to `most` new tokens.  Every wavefront works it out for itself, a lane a sequence
