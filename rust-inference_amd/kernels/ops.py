@@ -1972,8 +1972,13 @@ def talking_attention_mfma(proj, q_off: int, k_pages, v_pages, tok_pos, cu_seqle
     return sum_parts(parts) if parts is not None else out
 
 
-# Bytes of scores that a step of single tokens may keep between its two launches.
-TALKING_DECODE_SCORES = 1 << 28
+# Bytes of scores and sums that a step of single tokens keeps between its two launches: tokens past them go in further pairs of launches over the
+# same workspace.  A captured step holds it for as long as its graph lives, and an engine keeps up to 96 graphs, 6 GB at the most.  32 heads over 8 of
+# 128, us in all tokens at once : 128 : 64 : 32 MB (the general kernels): 64 tokens at 16,000 keys without a window 941 : 1,020 : 1,130 : 1,269
+# (3,507), 300 in a window of 1,024 305 : 309 : 310 : 341 (1,774); 16 heads over 8 of 64, 64 tokens at 32,000 1,314 : 1,428 : 1,536 : 1,690 (2,520).
+# TALKING_DECODE_TOKEN: of a single token at most (32 heads: two million keys); beyond, a step keeps to the general kernels.
+TALKING_DECODE_SCORES = 1 << 26
+TALKING_DECODE_TOKEN = 1 << 28
 # Workgroups that its second launch is to have at least (a page a workgroup at most).  32 heads of 128, us at 256 / 512 / 1,024: 8 tokens at
 # 1,400 keys 29.9 / 27.5 / 27.4, 40 at 1,500 66.7 / 59.0 / 60.6, 300 at 1,500 422 / 325 / 338, 4 at 8,000 without a window 66.6 / 62.9 / 73.6.
 TALKING_DECODE_FILL = 512
@@ -1986,27 +1991,39 @@ def talking_decode_pages(longest: int, window: int | None) -> int:
 
 
 def talking_decode_fits(dtype, tokens: int, longest: int, window: int | None, heads: int, kv_heads: int, dim: int, page_size: int) -> bool:
-    """Whether a step of single tokens runs ``talking_decode``: sizes that the matrix cores take, and scores that fit a workspace."""
+    """Whether a step of single tokens runs ``talking_decode``: sizes that the matrix cores take, and a token's scores that fit a workspace."""
     return (dtype == torch.bfloat16 and tokens <= 65535 and bool(_get("ri_talking_decode_fits")(heads, kv_heads, dim, page_size))
-            and tokens * talking_decode_pages(longest, window) * heads * 128 <= TALKING_DECODE_SCORES)
+            and talking_decode_pages(longest, window) * heads * 136 <= TALKING_DECODE_TOKEN)
+
+
+def talking_decode_piece(tokens: int, pages: int, heads: int) -> int:
+    """How many of a step's tokens a pair of launches takes: as many as the workspace holds, one at least, in pieces of one size."""
+    most = min(tokens, max(1, TALKING_DECODE_SCORES // (pages * heads * 136)))
+    return -(-tokens // -(-tokens // most))
 
 
 def talking_decode(proj, q_off: int, k_pages, v_pages, tok_pos, tok_seq, page_table, heads: int, kv_heads: int, dim: int,
                    window: int | None, scale: float, r1, r2, talk, longest: int) -> torch.Tensor:
     """The same attention for single tokens in bfloat16, of sequences of up to ``longest`` keys: float32 ``[T, heads * dim]``."""
     tokens, pages = proj.shape[0], talking_decode_pages(longest, window)
-    blocks = -(-kv_heads * dim // 1024)
-    shares = max(1, min(pages, -(-TALKING_DECODE_FILL // (tokens * blocks))))
+    blocks, piece = -(-kv_heads * dim // 1024), talking_decode_piece(tokens, pages, heads)
+    shares = max(1, min(pages, -(-TALKING_DECODE_FILL // (piece * blocks))))
     new = lambda *shape: torch.empty(shape, dtype=torch.float32, device=proj.device)
-    out, scores, sums = new(shares, tokens, heads * dim), new(tokens, pages, heads, 32), new(tokens, pages, heads, 2)
-    _call("ri_talking_decode", _dev(out, "out"), shares, _dev(scores, "scores"), _dev(sums, "sums"), pages,
-          _dev(proj, "proj", torch.bfloat16), proj.shape[1], int(q_off), _dev(k_pages, "k_pages", torch.bfloat16),
-          _dev(v_pages, "v_pages", torch.bfloat16, (k_pages.shape[0], kv_heads, dim, k_pages.shape[2])),
-          _dev(tok_pos, "tok_pos", torch.int32, (tokens,)), _dev(tok_seq, "tok_seq", torch.int32, (tokens,)),
-          _dev(page_table, "page_table", torch.int32), page_table.shape[1], tokens, heads, kv_heads, dim, k_pages.shape[2], int(window or 0),
-          float(scale), _opt(r1, "r1", torch.float32, (heads,)), _opt(r2, "r2", torch.float32, (heads,)),
-          _opt(talk, "talk", torch.float32, (heads, heads)), _stream())
-    return out[0] if shares == 1 else sum_parts(out, torch.float32)
+    scores, sums, out = new(piece, pages, heads, 32), new(piece, pages, heads, 2), new(tokens, heads * dim)
+    parts = out if shares == 1 else new(shares, piece, heads * dim)
+    row = proj.shape[1]
+    for at in range(0, tokens, piece):
+        n, to = min(piece, tokens - at), _dev(out, "out") + at * heads * dim * 4
+        _call("ri_talking_decode", to if shares == 1 else _dev(parts, "parts"), shares, _dev(scores, "scores"), _dev(sums, "sums"), pages,
+              _dev(proj, "proj", torch.bfloat16) + at * row * 2, row, int(q_off), _dev(k_pages, "k_pages", torch.bfloat16),
+              _dev(v_pages, "v_pages", torch.bfloat16, (k_pages.shape[0], kv_heads, dim, k_pages.shape[2])),
+              _dev(tok_pos, "tok_pos", torch.int32, (tokens,)) + at * 4, _dev(tok_seq, "tok_seq", torch.int32, (tokens,)) + at * 4,
+              _dev(page_table, "page_table", torch.int32), page_table.shape[1], n, heads, kv_heads, dim, k_pages.shape[2], int(window or 0),
+              float(scale), _opt(r1, "r1", torch.float32, (heads,)), _opt(r2, "r2", torch.float32, (heads,)),
+              _opt(talk, "talk", torch.float32, (heads, heads)), _stream())
+        if shares > 1:
+            _call("ri_sum_parts", to, code(torch.float32), _dev(parts, "parts"), shares, n, heads * dim, 0, 0, _stream())
+    return out
 
 
 # ---------------------------------------------------------------- time mixing

@@ -707,6 +707,26 @@ def test_single_tokens_of_talking_heads_are_the_general_kernel(ops, heads, kv_he
             close(got, np.concatenate([f64(w) for w in want]), F32, f"{fill} workgroups")
 
 
+@pytest.mark.parametrize("fill", [1, 1 << 20])
+def test_single_tokens_of_talking_heads_in_a_bounded_workspace(ops, fill, monkeypatch):
+    """What a step keeps between its launches is bounded however many tokens and keys it has; a token, two and several a pair of launches,
+    whole and in shares of the pages: the same bits as all tokens in one."""
+    for tokens, pages, heads in ((64, 512, 32), (512, 64, 64), (1, 4, 8), (40, 8000, 32)):
+        assert ops.talking_decode_piece(tokens, pages, heads) * pages * heads * 34 * 4 <= max(1 << 26, pages * heads * 136)
+    assert ops.talking_decode_piece(64, 32, 32) == 64 and ops.talking_decode_fits(torch.bfloat16, 64, 65536, None, 32, 8, 128, PAGE)
+    monkeypatch.setattr(ops, "TALKING_DECODE_FILL", fill)
+    heads, kv_heads, dim, n = 8, 4, 32, 5
+    k_pages, v_pages = (guarded((torch.randn(shape, device=DEV) * 0.6).to(torch.bfloat16)) for shape in
+                        ((12, kv_heads, PAGE, dim), (12, kv_heads, dim, PAGE)))
+    table, pos, seq = t(np.arange(15).reshape(5, 3) % 12, torch.int32), t([0, 31, 32, 95, 65], torch.int32), t(range(n), torch.int32)
+    proj = guarded((torch.randn((n, heads * dim + 16), device=DEV) * 0.6).to(torch.bfloat16))
+    args = (heads, kv_heads, dim, None, 0.2, t(np.arange(heads) / 9.0), t(np.arange(heads) / 4.0), t(np.eye(heads) + 0.1), 96)
+    whole = f64(ops.talking_decode(proj, 8, k_pages, v_pages, pos, seq, table, *args))
+    for piece in (1, 2, 3):
+        monkeypatch.setattr(ops, "TALKING_DECODE_SCORES", piece * 3 * heads * 136)
+        assert np.array_equal(f64(ops.talking_decode(proj, 8, k_pages, v_pages, pos, seq, table, *args)), whole), f"{piece} tokens at a time"
+
+
 @pytest.mark.parametrize("dim, window, table", [(32, 40, True), (64, 45, False), (128, None, False)])
 def test_talking_attention_whole_and_in_shares(ops, dim, window, table, monkeypatch):
     """Tiles that are walked whole, whose result is bfloat16 at once, and in two, three and four shares of their pages, whose float32 sums
