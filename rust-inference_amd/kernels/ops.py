@@ -2157,9 +2157,11 @@ def ssd_chunks_pay(new_counts, heads: int, n: int, vdim: int) -> bool:
     return 25 + sum(-(-k // 64) for k in new_counts) * heads * (0.05 + 0.085 * size) * 256 / units < 0.9 * walk
 
 
-def ssd_chunks_fit(n: int, vdim: int, channels: int, offsets: tuple) -> bool:
-    """Whether ``ssd_scan_chunked`` takes these sizes (host code only)."""
-    return bool(_get("ri_decay_chunks_fit")(int(n), int(vdim))) and channels % 4 == 0 and all(o % 4 == 0 for o in offsets)
+def ssd_chunks_fit(n: int, vdim: int, channels: int, offsets: tuple, state=None) -> bool:
+    """Whether ``ssd_scan_chunked`` takes these sizes and this state, which it reads 16 bytes at a time (host code only; ``ssd_scan`` takes
+    a state that starts anywhere)."""
+    return (bool(_get("ri_decay_chunks_fit")(int(n), int(vdim))) and channels % 4 == 0 and all(o % 4 == 0 for o in offsets)
+            and (state is None or state.data_ptr() % 16 == 0))
 
 
 def ssd_scan_chunked(xbc, b_off: int, c_off: int, proj, z_off: int, dt_off: int, dt_bias, a_log, d_skip, state, cu_seqlens, slots,

@@ -78,7 +78,7 @@ class StateSpaceMixer(Mixer):
                     ctx.cu_seqlens, ctx.slots, self.heads, self.groups, self.state, self.vdim)
             if (proj.dtype != torch.float32 and not rt.invariant and ctx.max_new > 1
                     and ops.ssd_chunks_pay(ctx.new_counts, self.heads, self.state, self.vdim)
-                    and ops.ssd_chunks_fit(self.state, self.vdim, self.channels, (self.inner, self.inner + gn))):
+                    and ops.ssd_chunks_fit(self.state, self.vdim, self.channels, (self.inner, self.inner + gn), state)):
                 # prompts: chunks of 64 tokens side by side (float32 and the invariant mode keep the one form of the walk)
                 y = ops.ssd_scan_chunked(*args, ctx.max_new)
             else:

@@ -484,6 +484,12 @@ def test_state_space_chunks_err_no_more_than_the_walk(ops, n, vdim, bias):
     assert error(got, np.stack(want)) <= 1.1 * error(walk, np.stack(want)) and error(chunked[0], S) <= 1.1 * error(walked[0], S)
 
 
+def test_state_space_chunks_leave_a_state_off_their_loads_boundary_to_the_walk(ops):
+    whole = guarded(torch.zeros(1 + 2 * 8 * 12, device=DEV))
+    fit = lambda state: ops.ssd_chunks_fit(8, 12, 40, (24, 32), state)
+    assert fit(whole[:-1].view(1, 2, 8, 12)) and not fit(whole[1:].view(1, 2, 8, 12))
+
+
 def test_state_space_chunks_where_the_walk_waits_for_its_tokens(ops, monkeypatch):
     monkeypatch.setattr(ops, "compute_units", lambda: 256)
     pay = ops.ssd_chunks_pay
