@@ -178,22 +178,25 @@ def test_latent_attention_through_every_cut(ops, heads, dim, rot, vdim, rank):
 
 # ---------------------------------------------------------------- the windowed attention whose heads talk
 @pytest.mark.skipif(EMULATED, reason="a thousand tokens; on an emulated machine of one unit the small tests take this form")
-@pytest.mark.parametrize("heads, kv_heads, window", [(32, 8, 100), (16, 2, None), (24, 8, 64)])
-def test_talking_attention_of_a_full_machine(ops, heads, kv_heads, window):
-    """Enough tiles that a wavefront of the first walk takes four heads (and groups of three, which it cannot); against the general kernel."""
-    counts, dim = [1000, 45, 3], 32
+@pytest.mark.parametrize("heads, kv_heads, dim, window, first", [(32, 8, 32, 100, 1000), (16, 2, 32, None, 2000), (24, 8, 32, 64, 1000),
+                                                                 (32, 8, 64, None, 1000), (32, 8, 128, 100, 1000), (32, 8, 128, None, 1000)])
+def test_talking_attention_of_a_full_machine(ops, heads, kv_heads, dim, window, first):
+    """Enough tiles that a wavefront of the first walk takes four heads, 512 wavefronts and more (and groups of three, which it cannot), with the
+    table of distances and with a logarithm a score; against the general kernel."""
+    counts = [first, 45, 3]
+    assert heads % (4 * kv_heads) or sum(-(-n // 16) for n in counts) * heads // 4 >= 2 * 256
     rng = np.random.default_rng(heads)
-    pages = 32 + 2 + 1
+    pages = -(-first // 32)
     k_pages, v_pages = ((torch.randn(shape, device=DEV) * 0.6).to(torch.bfloat16) for shape in
-                        ((pages, kv_heads, PAGE, dim), (pages, kv_heads, dim, PAGE)))
-    table = np.zeros((3, 32), dtype=np.int32)
-    table[0], table[1, :2], table[2, 0] = np.arange(32), [32, 33], 34
+                        ((pages + 3, kv_heads, PAGE, dim), (pages + 3, kv_heads, dim, PAGE)))
+    table = np.zeros((3, pages), dtype=np.int32)
+    table[0], table[1, :2], table[2, 0] = np.arange(pages), [pages, pages + 1], pages + 2
     seq, pos = t([s for s, n in enumerate(counts) for _ in range(n)], torch.int32), t([i for n in counts for i in range(n)], torch.int32)
     proj = (torch.randn((sum(counts), heads * dim), device=DEV) * 0.6).to(torch.bfloat16)
     args = (heads, kv_heads, dim, window, 0.2, t(rng.random(heads)), t(rng.random(heads) * 3), t(np.eye(heads) + 0.2 * rng.standard_normal((heads, heads))))
     want = ops.talking_attention(proj, 0, k_pages, v_pages, pos, seq, t(table, torch.int32), *args)
     got = ops.talking_attention_mfma(proj, 0, k_pages, v_pages, pos, t(np.concatenate([[0], np.cumsum(counts)]), torch.int32), counts,
-                                     t(table, torch.int32), *args, 1000)
+                                     t(table, torch.int32), *args, first)
     close(got, f64(want), 1.5e-2, "matrix cores against the general kernels")
 
 
@@ -658,7 +661,7 @@ def test_latent_attention_shares_pages_where_that_is_less_to_wait_for(ops, monke
     assert plan([2048], [0], 32, 288) == 512 and plan([2048] + [1] * 64, [0] + [2000] * 64, 32, 288) == 0 and plan([16], [8000], 32, 160) == 4
 
 
-@pytest.mark.parametrize("heads, kv_heads, dim, window", [(8, 2, 32, 40), (16, 16, 32, None), (8, 1, 64, 33)])
+@pytest.mark.parametrize("heads, kv_heads, dim, window", [(8, 2, 32, 40), (16, 16, 32, None), (8, 1, 64, 33), (32, 8, 128, 40), (8, 2, 64, None)])
 def test_talking_attention_on_the_matrix_cores_is_the_general_kernel(ops, heads, kv_heads, dim, window):
     """bfloat16: two sequences whose pages lie in shuffled order, one that goes on from 37 cached tokens with 21 new ones
     (two tiles, the second partial) and one that starts with 50; with the distance bias and the mixing matrix, and without;

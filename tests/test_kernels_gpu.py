@@ -276,6 +276,24 @@ def test_values_turned_by_groups_of_eight_positions(ops, dtype, heads, kv_heads,
     assert np.array_equal(f64(vp), want)
 
 
+@pytest.mark.skipif(EMULATED, reason="eight million workgroups, almost all of them empty")
+def test_values_in_a_launch_of_their_own_past_what_one_holds(ops):
+    """A bound on the new tokens far above the real ones, whose workgroups are more than the launch with the queries is to hold."""
+    rng = np.random.default_rng(5)
+    heads, kv_heads, dh, new = 16, 2, 128, [37, 3]
+    qkv, out = t(rng.normal(size=(40, (heads + 2 * kv_heads) * dh)), torch.bfloat16), []
+    pos, seq, cu = t(list(range(37)) + [0, 1, 2], torch.int32), t([0] * 37 + [1] * 3, torch.int32), t([0, 37, 40], torch.int32)
+    for most in (37, 1 << 27):
+        _, _, kp, vp, table = paged(np.random.default_rng(6), new, kv_heads, dh, dtype=torch.bfloat16)
+        rows = qkv.clone()
+        ops.qk_norm_rope_kv_write(rows, None, None, 1e-5, None, pos, seq, table, kp, vp, heads, kv_heads, dh, cu_seqlens=cu, max_new=most)
+        whole, wk, wv = qkv[:, :(heads + kv_heads) * dh].contiguous(), kp.clone(), vp.clone()
+        ops.whole_norm_kv_write(whole, 0, heads * dh, t(np.ones(heads * dh)), t(np.ones(kv_heads * dh)), 1e-5, pos, seq, table, wk, wv, heads, kv_heads, dh,
+                                cu_seqlens=cu, max_new=most)
+        out.append([f64(x) for x in (rows, kp, vp, whole, wk, wv)])
+    assert all(np.array_equal(a, b) for a, b in zip(*out)) and (out[0][2] != 0).any()
+
+
 @pytest.mark.parametrize("dtype, rel", [(torch.float32, 3e-6), (torch.bfloat16, BF16_OUT)])
 @pytest.mark.parametrize("dh, rot", [(64, 16), (48, 24), (40, 8), (7, 4), (9, 0), (130, 128), (512, 64)])
 def test_rotation_over_part_of_the_head(ops, dtype, rel, dh, rot):
@@ -383,12 +401,13 @@ def test_attention_rows_of_queries_share_their_loads(ops, dtype, heads, kv_heads
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("form", [dict(window=37), dict(chunk=50), dict(window=37, keep_first=5), dict(window=300, keep_first=40)])
-def test_attention_rows_of_queries_leave_pages_given_back_alone(ops, dtype, form, monkeypatch):
+@pytest.mark.parametrize("dh", [64, 48])
+def test_attention_rows_of_queries_leave_pages_given_back_alone(ops, dtype, form, dh, monkeypatch):
     """Steps that go on behind a window or a chunk: the pages that no query can see any more are out of the tables (-1, as the cache
     leaves them), and the first visible key lies in the middle of a tile of 256 and of its page.  The same bits as a workgroup for
-    every token and head, which reads the keys it sees alone."""
+    every token and head, which reads the keys it sees alone.  (float32 heads of 64 take the matrix cores each time.)"""
     before, new = ([380, 301, 90, 0, 611], [10, 7, 1, 12, 5]) if EMULATED else ([380, 701, 90, 0, 1200], [10, 70, 1, 200, 33])
-    heads, kv_heads, dh, page = 8, 2, 64, 32
+    heads, kv_heads, page = 8, 2, 32
     rng = np.random.default_rng(len(form) + sum(form.values()))
     _, _, kp, vp, table = paged(rng, [a + n for a, n in zip(before, new)], kv_heads, dh, dtype=dtype)
     window, chunk, keep = form.get("window"), form.get("chunk"), form.get("keep_first", 0)
@@ -477,6 +496,36 @@ def test_attention_float32_on_the_matrix_cores(ops, heads, kv_heads, dh, form):
             row += 1
 
 
+@pytest.mark.parametrize("dh, form", [(64, dict(window=37)), (128, dict(chunk=50)), (64, dict(window=37, keep_first=5)), (128, dict(window=100, keep_first=40))])
+def test_attention_float32_on_the_matrix_cores_leaves_pages_given_back_alone(ops, dh, form):
+    """Behind a window or a chunk a table holds -1; in runs, as tokens lie and one by one, against the general kernel, which takes the same
+    pages where they start off a 16-byte boundary.  float32 sums in another order."""
+    before, new = [180, 101, 90, 0, 211], [10, 7, 1, 12, 5]
+    heads, kv_heads, page = 8, 2, 32
+    rng = np.random.default_rng(dh + sum(form.values()))
+    _, _, kp, vp, table = paged(rng, [a + n for a, n in zip(before, new)], kv_heads, dh)
+    window, chunk, keep = form.get("window"), form.get("chunk"), form.get("keep_first", 0)
+    for b, length in enumerate(before):
+        first = length - length % chunk if chunk else max(0, length - window + 1)
+        table[b, -(-keep // page):max(first // page, -(-keep // page))] = -1
+    assert (table[:, :3] == -1).any()
+    qkv = t(rng.normal(size=(sum(new), heads * dh)))
+    seq, pos = t([b for b, n in enumerate(new) for _ in range(n)], torch.int32), t([before[b] + i for b, n in enumerate(new) for i in range(n)], torch.int32)
+    runs = dict(new_counts=new, starts=before, cu_seqlens=t(np.concatenate([[0], np.cumsum(new)]), torch.int32))
+
+    def off(x):
+        """The same numbers four bytes behind a boundary."""
+        whole = t(np.zeros(x.numel() + 1))
+        whole[1:] = x.reshape(-1)
+        return whole[1:].view(x.shape)
+
+    run = lambda k, v, how: f64(ops.attention(qkv, k, v, pos, seq, table, heads, kv_heads, dh, window, dh ** -0.5, keep_first=keep, chunk=chunk, **how))
+    want = run(off(kp), off(vp), {})
+    assert np.array_equal(want, run(off(kp), off(vp), runs)) and np.isfinite(want).all()
+    for how in ({}, dict(most_new=max(new)), runs):
+        close(t(run(kp, vp, how)), want, 3e-6, str(list(how)))
+
+
 def test_attention_shares_loads_where_that_is_less_to_wait_for(ops, monkeypatch):
     """Prompts enough to fill the machine do; one of 130 tokens, many of four and steps of single tokens do not, nor do single tokens
     that stand beside a prompt."""
@@ -531,6 +580,16 @@ def test_prompt_attention_with_two_tiles_a_wavefront(ops, heads):
     """More query heads a key head than one tile of sixteen columns holds: two tiles whatever the step's size."""
     out, want = attention_case(ops, np.random.default_rng(heads), [33, 100, 1], [33, 5, 1], heads, 1, 128, torch.bfloat16, kernel="prefill")
     close(out, want, BF16_OUT, "prefill attention, two tiles a wavefront")
+
+
+@pytest.mark.parametrize("heads, window", [(16, None), (13, 50), (16, 20)])
+def test_prompt_attention_with_two_tiles_on_a_small_machine(ops, heads, window):
+    """Heads of 128 whose queries one tile would hold: two where a machine of one unit is filled (on a larger one, one)."""
+    if ops.compute_units() == 1:
+        assert ops.attention_prefill_tiles([110], heads, 1, 128) == 2 and ops.attention_prefill_tiles([110, 97], heads, 1, 128) == 2
+    for lens, new in (([130], [110]), ([110, 160], [110, 97])):
+        out, want = attention_case(ops, np.random.default_rng(heads), lens, new, heads, 1, 128, torch.bfloat16, window=window, kernel="prefill")
+        close(out, want, BF16_OUT, "prefill attention, two tiles a wavefront")
 
 
 def test_prompt_attention_tiles_follow_the_tokens_of_the_long_prompts(ops):
@@ -878,10 +937,11 @@ def test_gemm_f32_rows_do_not_depend_on_the_batch(ops):
     assert torch.equal(whole[60:], ops.gemm_f32(x[60:].contiguous(), w))
 
 
-@pytest.mark.parametrize("m,n,k", [(1, 37, 72), (33, 129, 192), (65, 130, 64), (65, 16500, 72), (33, 4100, 136)])
+@pytest.mark.parametrize("m,n,k", [(1, 37, 72), (33, 129, 192), (65, 130, 64), (65, 16500, 72), (33, 4100, 136),
+                                   (33, 129, 256), (65, 130, 128), (70, 40, 512), (33, 4100, 256)])
 def test_gemm_f32_on_the_matrix_cores(ops, m, n, k):
-    """bfloat16 weights: edges of the tiles of 32 and 64 rows, 32 to 128 columns and stages of 64 k, values over many orders of
-    magnitude.  An additions' chain of k / 32 steps and 32 products a step: (k / 32 + 32) half units of 2^-24 of the sum of
+    """bfloat16 weights: edges of the tiles of 32 and 64 rows, 32 to 128 columns and stages of 64 k, whole turns of stages among them (no part
+    of one is masked then), values over many orders of magnitude.  An additions' chain of k / 32 steps and 32 products a step: (k / 32 + 32) half units of 2^-24 of the sum of
     magnitudes at most."""
     if EMULATED and n > 1000:
         pytest.skip("the larger tiles run on the emulated machine of one unit, at small sizes")
@@ -894,9 +954,10 @@ def test_gemm_f32_on_the_matrix_cores(ops, m, n, k):
     assert np.array_equal(got[m // 2:], f64(some)), "a row's sums depend on the other rows"
 
 
-@pytest.mark.parametrize("m,n,k", [(385, 4096, 200), (1153, 4096, 64), (1200, 4096, 392), (31, 4096, 328)])
+@pytest.mark.parametrize("m,n,k", [(385, 4096, 200), (1153, 4096, 64), (1200, 4096, 392), (31, 4096, 328), (385, 4096, 256), (1153, 4096, 1024),
+                                   (31, 4096, 512)])
 def test_gemm_f32_tiles_of_a_full_machine(ops, m, n, k):
-    """The tiles of 64 x 128 that a whole machine chooses, their edges and stages that are not whole, and the smallest ones' four stages;
+    """The tiles of 64 x 128 that a whole machine chooses, their edges and stages, whole and not, and the smallest ones' four stages;
     the bound of the test above."""
     rng = np.random.default_rng(m + n + k)
     x, w = t(rng.normal(size=(m, k))), t(rng.normal(size=(n, k)), torch.bfloat16)
