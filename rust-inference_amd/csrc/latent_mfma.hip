@@ -8,7 +8,7 @@
 // 8 (r / 4) + r % 4, of the second that plus 4), so that a lane's eight scores are eight neighbouring keys, which is
 // how the value product wants its weights: no exchange between lanes.  A sink per head joins the sum once at the end.
 // Scores, maxima, sums and the accumulators are float32; the weights are rounded to bfloat16 for the value product, as
-// in this library's other matrix-core attention.  A token's sums run over its pages in order, whatever else the step holds.
+// in this library's other matrix-core attention (of single tokens what that leaves of them is a second product's).  A token's sums run over its pages in order, whatever else the step holds.
 // A step of few single tokens cuts a token's pages into chunks that workgroups walk side by side; each leaves its maximum, its sum
 // and its sums of values, and a second kernel joins them in the chunks' order.
 #include "api.h"
@@ -120,7 +120,10 @@ latent_attention_mfma_kernel(bf16_t* __restrict__ out, const bf16_t* __restrict_
 // over its quarter of the key rows' elements, the quarters meet lane by lane in LDS (one barrier a page: two buffers take turns), and
 // each goes on with all scores and a quarter of the value rows.  What bounds the kernel above on a step of few tokens is a wavefront's
 // wait for the 68 loads a page that its registers cannot hold at once; a quarter's 18 are all asked for together, the next page's
-// keys before the values are used.  32 heads, keys of 576, us with the join, a wavefront a chunk : this: one token at 1,000 keys 21.5 :
+// keys before the values are used.  With fewer, longer chunks fewer weights are the 1 of a chunk's largest score, which bfloat16 holds
+// whole: what the rounding leaves of the weights goes through the matrix cores as well.  Error (2-norm) against 64 bits, 32 heads, keys of
+// 576 / 16 heads, keys of 288, a wavefront a chunk 1.93e-3 / 1.90e-3, in quarters with the weights rounded 1.96e-3 / 1.91e-3, so 1.66e-3 / 1.66e-3
+// (the result's own rounding); 48.8 : 50.3 us for 40 tokens at 1,500 keys.  32 heads, keys of 576, us with the join, a wavefront a chunk : this: one token at 1,000 keys 21.5 :
 // 11.9, 8 at 1,400 42.4 : 16.6, 40 at 1,500 165 : 47, 128 at 1,000 571 : 81, 300 at 1,000 590 : 216; 16 heads, keys of 160: 8.2 : 7.4,
 // 11.5 : 8.7, 21.9 : 16.4, 27.8 : 19.1.
 template <int KS, int VT>
@@ -196,13 +199,14 @@ latent_attention_quarters_kernel(bf16_t* __restrict__ out, const bf16_t* __restr
         mx = fmaxf(mx, __shfl_xor(mx, 16, RI_WAVE));
         mx = fmaxf(mx, __shfl_xor(mx, 32, RI_WAVE));
         const float m_new = fmaxf(m, mx * scale_log2);        // the scale is positive; every page of the walk has a key that is seen
-        LmFrag p;
+        LmFrag p, rest;                                       // the weights in bfloat16, and what that leaves of them
         float sum = 0.f;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             const float a = exp2f(fmaf(s[2 * e], scale_log2, -m_new));
             const float b = exp2f(fmaf(s[2 * e + 1], scale_log2, -m_new));
             p.w[e] = pack_bf16x2(a, b);
+            rest.w[e] = pack_bf16x2(a - __uint_as_float(p.w[e] << 16), b - __uint_as_float(p.w[e] & 0xFFFF0000u));
             sum += a + b;
         }
         const float corr = exp2f(m - m_new);
@@ -212,6 +216,7 @@ latent_attention_quarters_kernel(bf16_t* __restrict__ out, const bf16_t* __restr
         for (int vt = 0; vt < VW; ++vt) {
             o[vt] *= corr;
             o[vt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[vt].v, p.v, o[vt], 0, 0, 0);
+            o[vt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[vt].v, rest.v, o[vt], 0, 0, 0);
         }
     }
     l += __shfl_xor(l, 16, RI_WAVE);
