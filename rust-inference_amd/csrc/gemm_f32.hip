@@ -257,9 +257,9 @@ extern "C" int ri_gemm_f32(float* out, const float* x, const void* w, int w_dtyp
     else {
         // The order of a row's sums is the same in every tile.  64 x 128 from three quarters of the machine on (one workgroup a compute unit), else
         // 32 x 64 as soon as 32 x 32 would need a second round.  us for 32 x 32 / 32 x 64 / 64 x 128 (rows; columns x K): 759; 6,144 x
-        // 1,024 60 / 44 / 49, 4,096 x 1,024 43 / 32 / 33, 1,024 x 3,072 33 / 30 / 39; 1,200; 4,096 x 1,024 65 / 54 / 47, 6,144 x 1,024 102 / 73 / 65;
-        // 400; 4,096 x 1,024 27 / 22 / 20, 6,144 x 1,024 37 / 28 / 32; 200; 4,096 x 1,024 17 / 14 / 17; 2,400; 6,144 x 1,024 252 / 149 / 128; 33;
-        // 1,024 x 3,072 20 / 22 / 38, 4,096 x 1,024 8.8 / 9.6 / 16 (the vector units' form: 759; 1,024 x 3,072 363).  (128 x 192 has no registers
+        // 1,024 60 / 49 / 49, 4,096 x 1,024 43 / 38 / 32, 1,024 x 3,072 33 / 35 / 39; 1,200; 4,096 x 1,024 65 / 51 / 47, 6,144 x 1,024 102 / 78 / 62;
+        // 400; 4,096 x 1,024 27 / 23 / 20, 6,144 x 1,024 37 / 29 / 32; 200; 4,096 x 1,024 17 / 14 / 17; 2,400; 6,144 x 1,024 252 / 151 / 124; 1,000;
+        // 12,288 x 4,096 64 x 128 325, 32 x 64 455; 33; 1,024 x 3,072 20 / 22 / 38, 4,096 x 1,024 8.8 / 9.6 / 16 (the vector units' form: 759; 1,024 x 3,072 363).  (128 x 192 has no registers
         // for three sums a result: with a stage less under way 48 and 46 us at 759; 6,144 and 1,200; 4,096, 136 at 2,400; 6,144.)
         // Up to 32 rows half of a tile of 64 would be padding: 151,936 x 1,024 at one row 77 / 57 / 75.
         const auto tiles = [&](int rows, int cols) { return (long)((m + rows - 1) / rows) * ((n + cols - 1) / cols); };

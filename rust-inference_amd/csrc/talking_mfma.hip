@@ -2,7 +2,7 @@
 //
 // The mixing of the heads' weights needs every head's finished softmax, so the keys are walked twice, as in the general
 // kernels (talking_attention.hip), with tiles of 16 tokens of a sequence as the 16 columns of the matrix cores' tiles:
-//   talking_stats_mfma:  a wavefront per (tile of tokens, head): S^T = K Q^T page by page, the distance bias, the window's
+//   talking_stats_mfma:  a wavefront per (tile of tokens, head, or four heads of a key head): S^T = K Q^T page by page, the distance bias, the window's
 //                        mask, and each column's running maximum and sum;
 //   talking_mix_mfma:    a workgroup of eight wavefronts per tile of tokens, each wavefront on an eighth of the heads:
 //                        for a page it makes its heads' weights exp(s - m) / l from the first walk's numbers and leaves
