@@ -339,6 +339,15 @@ int ri_gemm_wide_packed_bf16(void* out, int out_dtype, const void* x, const void
 int ri_sum_parts(void* out, int out_dtype, const float* parts, int n_parts, int rows, int width, int swiglu, int tiled,
                  void* stream);
 
+// A product of a prompt's many rows in tiles: out[m, n] (rows of ldo elements) = x[m, k] (rows of ldx) . w[n, k]^T (rows of ldw), bfloat16
+// with float32 sums; out float32 or bfloat16.  act (on the sums; bfloat16 out): 0 none; 1 silu(gate) * up and 2 g sigmoid(1.702 g) (u + 1)
+// with g = min(gate + b_gate, limit), u = clamp(up + b_up, -limit, limit) (either bias may be NULL), both with w = [gate; up], 2 n rows;
+// 3 max(v, 0)^2.  k is a multiple of 64 from 192 on, n and the strides multiples of 8, the pointers of 16 bytes.  tile: rows of x by rows of w a
+// workgroup; 256 x 128 not with a gate.  The sums do not depend on it.
+enum { RI_TILE_256_256 = 0, RI_TILE_128_256 = 1, RI_TILE_256_128 = 2 };
+int ri_gemm_tiles_bf16(void* out, int out_dtype, int ldo, const void* x, int ldx, const void* w, int ldw, int m, int n, int k, int act,
+                       const float* b_gate, const float* b_up, float limit, int tile, void* stream);
+
 // x[t, i] += bias[i] in place (bias float32 [dim], x of dtype [rows, dim]).
 int ri_add_bias(void* x, int dtype, const float* bias, int rows, int dim, void* stream);
 

@@ -171,6 +171,16 @@ static inline int emu_mov_dpp_quad(int v, int control) {
     return all[(lane & ~3) | ((control >> (2 * (lane & 3))) & 3)];
 }
 #define __builtin_amdgcn_mov_dpp(v, control, row_mask, bank_mask, bound_ctrl) emu_mov_dpp_quad((v), (control))
+// The same with lanes that keep their old value: bank_mask's bit b is for lanes 4 b to 4 b + 3 of every sixteen; 0x128: turned by eight
+// inside every sixteen.
+static inline int emu_update_dpp(int old, int v, int control, int bank_mask) {
+    int all[64];
+    emu::wave_gather(&v, sizeof(int), all);
+    const int lane = emu::self->lane;
+    if (control != 0x128) abort();
+    return bank_mask >> ((lane & 15) >> 2) & 1 ? all[lane ^ 8] : old;
+}
+#define __builtin_amdgcn_update_dpp(old, v, control, row_mask, bank_mask, bound_ctrl) emu_update_dpp((old), (v), (control), (bank_mask))
 // v_perm_b32: byte i of the result is the one that byte i of `sel` names, 0 .. 3 of b and 4 .. 7 of a.
 static inline uint32_t emu_perm(uint32_t a, uint32_t b, uint32_t sel) {
     const uint64_t both = (uint64_t)a << 32 | b;

@@ -83,6 +83,8 @@ _SIGNATURES = {
     "ri_gemm_mid_packed_bf16": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p],
     "ri_gemm_wide_packed_bf16": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int,
                                  c_int, c_void_p],
+    "ri_gemm_tiles_bf16": [c_void_p, c_int, c_int, c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p,
+                           c_float, c_int, c_void_p],
     "ri_gemm_wide_packed_bf16_plan": [c_int, c_int, c_int, c_void_p, c_void_p],
     "ri_gemm_wide_stretch_plan": [c_int, c_int, c_int, c_void_p, c_void_p],
     "ri_compute_units": [],
@@ -1598,6 +1600,30 @@ def gemm_wide_packed_bf16(x, wpacked: torch.Tensor, n: int, out_dtype=torch.bflo
           _dev(x.data if x_tiled else x, "x", torch.bfloat16), _dev(wpacked, "wpacked", torch.bfloat16), m, n, k,
           int(swiglu), int(parts), (TILED_X if x_tiled else 0) | (TILED_OUT if tiled_out else 0), int(depth),
           int(waves), _stream())
+    return out
+
+
+TILES = ((256, 256), (128, 256), (256, 128))     # rows of x by rows of w a workgroup of gemm_tiles_bf16
+TILES_MIN_K = 192
+TILES_ACTIVATIONS = {None: 0, "silu_gate": 1, "clamped_gate": 2, "relu2": 3}
+
+
+def gemm_tiles_bf16(x: torch.Tensor, w: torch.Tensor, tile: int, out_dtype=torch.bfloat16, activation: str | None = None,
+                    b_gate=None, b_up=None, limit: float = 0.0, out: torch.Tensor | None = None) -> torch.Tensor:
+    """``x @ w.T`` for a prompt's many bfloat16 rows in tiles (``tile``: an index of ``TILES``, which the sums do not depend on;
+    256 x 128 not with a gate), float32 sums, the result in ``out_dtype`` or in ``out``.  ``activation`` on the sums (bfloat16 out):
+    ``"relu2"``; with ``w`` the rows ``[gate; up]``: ``"silu_gate"`` (``silu(gate) * up``) and ``"clamped_gate"`` (as
+    ``glu_clamped_bias``, with its biases and limit).  Rows of ``w`` may be a slice of longer ones."""
+    m, k = x.shape
+    gated = activation in ("silu_gate", "clamped_gate")
+    n = w.shape[0] // 2 if gated else w.shape[0]
+    if w.shape[1] != k or (gated and w.shape[0] % 2):
+        raise ShapeError(f"a product of {list(x.shape)} with {list(w.shape)}")
+    if out is None:
+        out = torch.empty((m, n), dtype=out_dtype, device=x.device)
+    _call("ri_gemm_tiles_bf16", _dev(out, "out", None, (m, n)), code(out.dtype), n, _dev(x, "x", torch.bfloat16), k,
+          _dev(w[0], "a row of w", torch.bfloat16), w.stride(0), m, n, k, TILES_ACTIVATIONS[activation], _opt(b_gate, "b_gate", torch.float32, (n,)), _opt(b_up, "b_up", torch.float32, (n,)),
+          float(limit), int(tile), _stream())
     return out
 
 

@@ -145,7 +145,7 @@ class RoutedExperts(FeedForward):
     # A step with fewer assignments (tokens x top) than experts reads only the rows of the experts its tokens chose
     # (one wavefront an output row: every assignment streams its expert's matrices once, so with as many assignments
     # as experts it would read what all experts hold); from SORTED_MIN_TOKENS tokens on a prompt's assignments are
-    # sorted by expert and every expert is two library products over its own rows; between them, and in float32, all
+    # sorted by expert and every expert is two products over its own rows; between them, and in float32, all
     # experts are computed for all tokens as two products, with zeros where a token did not choose.
     SORTED_MIN_TOKENS = 256
 
@@ -216,9 +216,9 @@ class RoutedExperts(FeedForward):
         return ops.experts_gather(x, dest, self.top), dest, starts, there
 
     def forward_sorted(self, rows, dest, starts, there, weights):
-        """A prompt: every expert's tokens as rows side by side, two library products an expert, the weighted sum in
+        """A prompt: every expert's tokens as rows side by side, two products an expert, the weighted sum in
         float32.  The host reads how many rows every expert has (one wait a layer), which a captured step could not."""
-        ff = self.inter
+        ff, rt = self.inter, self.rt
         rows_each = 2 * ff if self.gated else ff
         y = torch.empty_like(rows)
         there.synchronize()
@@ -226,10 +226,15 @@ class RoutedExperts(FeedForward):
         for e in range(self.experts):
             a, b = starts[e], starts[e + 1]
             if b > a:
-                gu = torch.mm(rows[a:b], self.w_gate_up.w[e * rows_each:(e + 1) * rows_each].t())
-                act = (ops.experts_activate(gu, None, ff, self.limit) if self.gated
-                       else ops.experts_activate_plain(gu, None, ff, self.activation))
-                torch.mm(act, self.w_down.w[:, e * ff:(e + 1) * ff].t(), out=y[a:b])
+                w = self.w_gate_up.w[e * rows_each:(e + 1) * rows_each]
+                if self.gated:
+                    act = rt.rows_activated(rows[a:b], w, "clamped_gate" if self.limit > 0 else "silu_gate",
+                                            lambda gu: ops.experts_activate(gu, None, ff, self.limit), limit=max(self.limit, 0.0))
+                elif self.activation == "relu2":
+                    act = rt.rows_activated(rows[a:b], w, "relu2", lambda u: ops.experts_activate_plain(u, None, ff, "relu2"))
+                else:
+                    act = ops.experts_activate_plain(torch.mm(rows[a:b], w.t()), None, ff, self.activation)
+                rt.rows_into(y[a:b], act, self.w_down.w[:, e * ff:(e + 1) * ff])
         if self.identity and starts[self.outs] > starts[self.experts]:
             y[starts[self.experts]:] = rows[starts[self.experts]:]        # identity experts: the token's own row
         return ops.experts_combine(y, dest, weights)

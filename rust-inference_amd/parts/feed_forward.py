@@ -88,7 +88,9 @@ class DenseFF(FeedForward):
     def forward(self, x, ctx):
         rt = self.rt
         with profiler.section(profiler.MLP):
-            a = ops.ACTIVATIONS[self.activation](ops.as_rows(rt.linear_packed(x, self.w_up)))
+            act = ops.ACTIVATIONS[self.activation]
+            a = (rt.linear_activated(x, self.w_up, "relu2", act) if self.activation == "relu2"
+                 else act(ops.as_rows(rt.linear_packed(x, self.w_up))))
             # float32 into the residual (or in parts that the stream's next read adds): the sum is never rounded to 16 bits
             return rt.linear_packed(a, self.w_down, out_dtype=torch.float32, parts_ok=True)
 
@@ -130,8 +132,9 @@ class ClampedGatedFF(FeedForward):
     def forward(self, x, ctx):
         rt = self.rt
         with profiler.section(profiler.MLP):
-            gu = ops.as_rows(rt.linear_packed(x, self.w_gate_up))
-            a = ops.glu_clamped_bias(gu, self.b_gate, self.b_up, self.limit)
+            a = rt.linear_activated(x, self.w_gate_up, "clamped_gate",
+                                    lambda gu: ops.glu_clamped_bias(gu, self.b_gate, self.b_up, self.limit),
+                                    self.b_gate, self.b_up, self.limit)
             # float32 into the residual (or in parts that the stream's next read adds); the last bias rides as out_bias
             return rt.linear_packed(a, self.w_down, out_dtype=torch.float32, parts_ok=True)
 

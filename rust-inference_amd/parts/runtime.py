@@ -26,7 +26,9 @@ def _wide_plan(n: int, k: int, swiglu: bool, rows: int = 64) -> tuple[int, int]:
 #              and up to 32 rows of tiled x; else the library.
 #   65-128     the wide kernel with two row tiles a wavefront for matrices of long rows whose reader adds stretches
 #              of K (`down`; up to 256 rows for the longest), and for the largest gate|up pairs; else the library.
-#   more       the vendor library (the reference hands every product to one: src/cuda/mod.rs:186-232).
+#   512 and more  the product in tiles (ops.gemm_tiles_bf16) where its tiles fill the machine or the activation rides in it
+#              (the rule is _tiles_plan below).
+#   else       the vendor library (the reference hands every product to one: src/cuda/mod.rs:186-232).
 GEMV_MAX_ROWS = 1
 SKINNY_MAX_ROWS = 16
 MID_MAX_ROWS = 64
@@ -81,6 +83,49 @@ def _packed_pays(n: int, k: int) -> bool:
     cus = _compute_units()
     last_round = tiles % cus
     return n * k * 2 <= PACKED_MAX_BYTES and not (tiles > cus and 0 < last_round < cus // 2)
+
+
+# Which tile of the product in tiles, if any.  Its time goes in rounds of tiles (one a compute unit), 256 x 256 at 1.35 PFLOP/s, the smaller
+# ones 0.87 of that; the library's product into bfloat16 makes 1.4 where its own rounds are full, into float32 1.22 (its epilogue), and 0.9 to 1.05
+# where half a round is left after two or more.  So, by the share of the rounds that is filled (us, tiles : library; rows; columns x K):
+#   one round of the smaller tiles from 0.88 on, either result: 2,048; 4,096 x 4,096 56 : 62, x 12,288 168 : 188; 7,640; 1,024 x 2,048 29 : 33, x 3,072
+#     41 : 46; 1,536; 5,120 x 5,120 69 : 79 (at 0.83 level, at 0.62 to 0.66 47 : 50 and 111 : 107);
+#   three and more rounds of 256 x 256, 0.8 to 0.93: 8,192; 5,120 x 8,192 499 : 667, x 25,600 1,606 : 2,088; 5,120; 8,192 x 4,096 265 : 367; 6,144; 12,288 x 4,096 458 : 582
+#     (at 0.75 253 : 239); float32 results also above, and in any number of rounds: 4,096; 8,192 x 4,096 210 : 227, 8,192; 12,288 x 4,096 604 : 656, 1,280 105 : 115
+#     (bfloat16 195 : 186, 582 : 562, 99 : 100);
+#   with the activation in it, which saves a kernel that reads and writes the results again: 2,048; 24,576 x 4,096 288 : 284 + 29, 7,640; 6,144 x 1,024 74 : 79 + 25,
+#     8,192; 51,200 x 5,120 3,072 : 3,119 + 212; from 0.62 on (the smaller tiles' share counted 0.87; 759; 24,576 x 4,096, 0.64: 159 : 147 + 13, 300, 0.59: 87 : 70 + 8),
+#     rows of up to 2,048 from 0.45 (759; 6,144 x 1,024: 14 : 15 + 5).  Without a gate less is saved: 0.1 more.
+TILES_MIN_ROWS = 512
+TILES_ONE_ROUND, TILES_FULL, TILES_MOST = 0.88, 0.93, 0.80
+TILES_FUSED, TILES_FUSED_SHORT, TILES_SHORT_K, TILES_SMALLER = 0.62, 0.45, 2048, 0.87
+
+
+@functools.lru_cache(maxsize=4096)
+def _tiles_plan(m: int, n: int, k: int, wide_out: bool, activation: str | None) -> int | None:
+    """The tile (of ``ops.TILES``) with which ``m`` rows go through a matrix of ``n`` rows of ``k``; None: not in tiles.  ``wide_out``: float32
+    results; ``activation``: what may ride in the product."""
+    gated = activation in ("silu_gate", "clamped_gate")
+    if m < TILES_MIN_ROWS or k < ops.TILES_MIN_K or k % 64 or n % (16 if gated else 8):
+        return None
+    cus = _compute_units()
+
+    def rounds_and_fill(tile):
+        rows, cols = ops.TILES[tile]
+        rounds = -(-(-(-m // rows) * -(-n // cols)) // cus)
+        return rounds, m * n / (rounds * cus * rows * cols)
+    rounds, fill = rounds_and_fill(0)
+    smaller = max((1,) if gated else (2, 1), key=lambda tile: rounds_and_fill(tile)[1])
+    small_rounds, small_fill = rounds_and_fill(smaller)
+    if activation is not None:
+        worth = max(fill, TILES_SMALLER * small_fill)
+        least = (TILES_FUSED_SHORT if k <= TILES_SHORT_K else TILES_FUSED) + (0.0 if gated else 0.1)
+        return None if worth < least else 0 if fill >= TILES_SMALLER * small_fill else smaller
+    if small_rounds == 1 and small_fill >= TILES_ONE_ROUND:
+        return smaller
+    if (rounds >= 3 and TILES_MOST <= fill < TILES_FULL) or (wide_out and fill >= TILES_FULL):
+        return 0
+    return None
 
 
 class PackedWeight:
@@ -153,6 +198,9 @@ class Runtime:
             if isinstance(x, ops.NormedLater):
                 return ops.linked_product(x, w, w.shape[0], False, out_dtype)
             return ops.gemv_bf16(ops.as_rows(x), w, out_dtype)
+        tile = self._tile(x, w, out_dtype)
+        if tile is not None:
+            return ops.gemm_tiles_bf16(self.normed_now(x), w, tile, out_dtype)
         return self._library_mm(self.normed_now(x), w, out_dtype)
 
     @staticmethod
@@ -315,8 +363,45 @@ class Runtime:
                     and pw.n >= 16 * WIDE_PLAIN_TILES * _compute_units()):
                 x = self.normed_now(x) if later else x
                 return ops.gemm_wide_packed_bf16(x, pw.packed, pw.n, out_dtype, depth=1, waves=_wide_whole_waves(pw.n, m))
-        y = self.linear(x, pw.w, None if pw.swiglu else out_dtype)
-        return ops.swiglu(y, tiled_out=tiled_out) if pw.swiglu else y
+        if pw.swiglu:
+            tile = self._tile(x, pw.w, self.dtype, "silu_gate")
+            if tile is not None:
+                return ops.gemm_tiles_bf16(self.normed_now(x), pw.w, tile, self.dtype, "silu_gate")
+            return ops.swiglu(self.linear(x, pw.w), tiled_out=tiled_out)
+        return self.linear(x, pw.w, out_dtype)
+
+    def linear_activated(self, x, pw: PackedWeight, activation: str, after, b_gate=None, b_up=None, limit: float = 0.0):
+        """``after(x @ w.T)``, with the activation (of ``ops.TILES_ACTIVATIONS``; ``after`` does the same) in the product where that goes in
+        tiles; the result in the compute dtype."""
+        tile = self._tile(x, pw.w, self.dtype, activation)
+        if tile is None:
+            return after(ops.as_rows(self.linear_packed(x, pw)))
+        return ops.gemm_tiles_bf16(self.normed_now(x), pw.w, tile, self.dtype, activation, b_gate, b_up, limit)
+
+    def rows_activated(self, x, w: torch.Tensor, activation: str, after, limit: float = 0.0):
+        """``linear_activated`` for rows and a stretch of a larger matrix (an expert's), without biases."""
+        tile = self._tile(x, w, self.dtype, activation)
+        if tile is None:
+            return after(torch.mm(x, w.t()))
+        return ops.gemm_tiles_bf16(x, w, tile, self.dtype, activation, limit=limit)
+
+    def rows_into(self, out, x, w: torch.Tensor) -> None:
+        """``out <- x @ w.T`` for rows and a stretch of a larger matrix, its rows or its columns."""
+        tile = self._tile(x, w, out.dtype) if out.data_ptr() % 16 == 0 else None
+        if tile is None:
+            torch.mm(x, w.t(), out=out)
+        else:
+            ops.gemm_tiles_bf16(x, w, tile, out=out)
+
+    def _tile(self, x, w: torch.Tensor, out_dtype, activation=None) -> int | None:
+        if self.dtype != torch.bfloat16 or self.invariant or x.shape[0] < TILES_MIN_ROWS:
+            return None
+        tile = _tiles_plan(x.shape[0], w.shape[0], w.shape[1], out_dtype == torch.float32, activation)
+        if tile is None or w.stride(1) != 1 or w.stride(0) % 8 or w.data_ptr() % 16:
+            return None
+        if isinstance(x, torch.Tensor) and not (x.is_contiguous() and x.data_ptr() % 16 == 0):
+            return None                                          # the library's product takes any strides
+        return tile
 
     def _library_mm(self, x, w, out_dtype):
         # The reference hands every product to a vendor library (src/cuda/mod.rs:186-232);

@@ -21,7 +21,7 @@ HERE = os.path.join(ROOT, "tests")
 # smaller sizes of the same tests or, where the form is chosen by the machine's size, on a machine made small (below).
 SELECT = ("not 4096 and not 12288 and not 5120 and not 5000 and not very_long and not more_pages_than and not thousands "
           "and not (many_sequences and not (16-8-32-100 or 16-8-32-40)) and not (in_runs and not 8-8-32) "
-          "and not (wide_packed and 1000 and not (1000-1024-33 or 1000-1024-64)) and not eight_wavefronts")
+          "and not (wide_packed and 1000 and not (1000-1024-33 or 1000-1024-64)) and not eight_wavefronts and not over_rounds")
 
 
 def _env(extra=None):
@@ -89,6 +89,7 @@ def runs():
         "sixteen units": _start([*PYTEST, SMALL_MACHINE], {"RI_EMU_COMPUTE_UNITS": "16"}),
         "one unit": _start([*PYTEST, *_workers(2), SMALL_MACHINE, KERNEL_TESTS, "-k", ONE_UNIT], {"RI_EMU_COMPUTE_UNITS": "1"}),
         "one unit, rows": _start([*PYTEST, *_workers(2), KERNEL_TESTS, "-k", ONE_UNIT_ROWS], {"RI_EMU_COMPUTE_UNITS": "1"}),
+        "one unit, tiles": _start([*PYTEST, KERNEL_TESTS, "-k", "over_rounds"], {"RI_EMU_COMPUTE_UNITS": "1"}),
         "sampler": _start([*PYTEST, *_workers(2), SAMPLER_TESTS, "-k", SAMPLER_SELECT]),
         "zidepel": _start([*PYTEST, *_workers(2), ZIDEPEL_TESTS]),
         "pisulorn": _start([*PYTEST, *_workers(2), PISULORN_TESTS, "-k", PISULORN_SELECT]),
@@ -128,6 +129,10 @@ def _passed(run, tests=None):
 
 def test_the_kernel_tests_pass_on_the_cpu_build_between_guard_pages(runs):
     _passed(runs["kernel tests"])
+
+
+def test_products_in_tiles_over_several_rounds_on_a_machine_made_small(runs):
+    _passed(runs["one unit, tiles"], 3)
 
 
 def test_the_sampler_tests_pass_on_the_cpu_build_between_guard_pages(runs):

@@ -1431,3 +1431,59 @@ def test_kernels_agree_with_their_plain_cpp_twins(ops):
     want = N.attention(qkv_t.cpu().numpy()[:, :heads * dh].reshape(tokens, heads, dh), kp.cpu().numpy(), vp.cpu().numpy(),
                        tok_pos, tok_seq, table.cpu().numpy(), None, 1 / np.sqrt(dh))
     close(got.reshape(tokens, heads, dh), want, 3e-6, "attention over the pages the kernel wrote")
+
+
+@pytest.mark.parametrize("act", [None, "float32", "relu2", "silu_gate", "clamped_gate"])
+@pytest.mark.parametrize("m, n, k", [(1, 8, 192), (129, 264, 256), (257, 128, 320), (300, 520, 192), (70, 1032, 448)])
+def test_product_in_tiles(ops, act, m, n, k):
+    """Products of prompts in tiles: edges of a tile in rows and columns, the fewest stages of K, stages of either number; every
+    activation on the sums; matrices that are a slice of longer rows; the same bits from every tile and from any number of rows."""
+    rng = np.random.default_rng(m + n + k)
+    gated = act in ("silu_gate", "clamped_gate")
+    x = t(rng.normal(size=(m, k)), torch.bfloat16)
+    wide = t(rng.normal(size=((2 if gated else 1) * n, k + 64)) * (3.0 / np.sqrt(k)), torch.bfloat16)
+    w = wide[:, 64:] if m % 2 else wide[:, :k].contiguous()
+    y = f64(x) @ f64(w).T
+    g, u = y[:, :n], y[:, n:]
+    bg, bu, limit = rng.normal(size=n), rng.normal(size=n), 2.5
+    kw, want = {}, y
+    if act == "relu2":
+        want = np.maximum(y, 0) ** 2
+    if act == "silu_gate":
+        want = P.silu(g) * u
+    if act == "clamped_gate":
+        kw = dict(b_gate=t(bg), b_up=t(bu), limit=limit)
+        g, u = np.minimum(g + np.float32(bg), limit), np.clip(u + np.float32(bu), -limit, limit)
+        want = g / (1 + np.exp(-1.702 * g)) * (u + 1)
+    out_dtype, name = (torch.float32, None) if act == "float32" else (torch.bfloat16, act)
+    got = ops.gemm_tiles_bf16(x, w, 0, out_dtype, name, **kw)
+    # bfloat16 results: half a unit in their last place, 2^-9 at the most; float32: sums of k products of eight bits each
+    close(got, want, 3e-6 if act == "float32" else 4e-3, f"tiles, {act}")
+    for tile in (1,) if gated else (1, 2):
+        assert torch.equal(ops.gemm_tiles_bf16(x, w, tile, out_dtype, name, **kw), got)
+    assert torch.equal(ops.gemm_tiles_bf16(x[m - 1:].contiguous(), w, 1, out_dtype, name, **kw), got[m - 1:])
+    taller = torch.full((m + 2, n), 7.0, dtype=out_dtype, device=x.device)
+    ops.gemm_tiles_bf16(x, w, 1, out_dtype, name, out=taller[1:m + 1], **kw)         # nothing beside its own rows
+    assert torch.equal(taller[1:m + 1], got) and bool((taller[0] == 7).all()) and bool((taller[m + 1] == 7).all())
+    with pytest.raises(Exception, match="gemm_tiles_bf16"):
+        ops.gemm_tiles_bf16(x[:, :128].contiguous(), w[:, :128].contiguous(), 0, out_dtype, name, **kw)
+    if gated:
+        with pytest.raises(Exception, match="tile"):
+            ops.gemm_tiles_bf16(x, w, 2, out_dtype, name, **kw)
+
+
+@pytest.mark.parametrize("act", [None, "float32", "silu_gate"])
+def test_product_in_tiles_over_rounds(ops, act):
+    """Workgroups that take one tile after another, the last round partly filled: what runs ahead into the next tile is that tile's."""
+    rng = np.random.default_rng(5)
+    room = max(8, ops.compute_units() // 8 * 8)
+    m, n, k = 256 * (room * 5 // 8) - 126, 272, 192          # 1.25 rounds of 256 x 256 and more, edges in rows and columns
+    x = t(rng.normal(size=(m, k)), torch.bfloat16)
+    w = t(rng.normal(size=(n, k)) * (3.0 / np.sqrt(k)), torch.bfloat16)
+    out_dtype, name = (torch.float32, None) if act == "float32" else (torch.bfloat16, act)
+    y = x.float() @ w.float().t()
+    want = torch.nn.functional.silu(y[:, :n // 2]) * y[:, n // 2:] if act == "silu_gate" else y
+    for tile in ((0, 1) if act == "silu_gate" else (0, 1, 2)):
+        got = ops.gemm_tiles_bf16(x, w, tile, out_dtype, name)
+        error = (got.float() - want).abs().amax(1) / want.abs().amax()
+        assert float(error.max()) < (1e-5 if act == "float32" else 8e-3), (tile, int(error.argmax()))
