@@ -348,6 +348,19 @@ enum { RI_TILE_256_256 = 0, RI_TILE_128_256 = 1, RI_TILE_256_128 = 2 };
 int ri_gemm_tiles_bf16(void* out, int out_dtype, int ldo, const void* x, int ldx, const void* w, int ldw, int m, int n, int k, int act,
                        const float* b_gate, const float* b_up, float limit, int tile, void* stream);
 
+// Attention over a cached latent for prompts (one key/value head, key rows [latent | turned part] in pages of 32).  ri_latent_gather: the
+// sequences' pages side by side, rows [pages * 32][key_dim], sequence after sequence, each from a multiple of 32 rows on, zeros behind its
+// len_after[s] keys.  ri_latent_prompt: causal attention of `tokens` queries (heads of dim + rot elements in rows of q_stride) over keys
+// [heads * dim] (rows of key_stride) beside turned [row] (rows of turned_stride, all heads') and values [heads * vdim] (rows of value_stride, a column a
+// key), rows as the gather leaves them; sinks [heads] join the denominators, gates (rows of q_stride, one a head) multiply by their
+// sigmoid, either may be NULL; out [tokens][heads * vdim].  ri_latent_prompt_fits: the sizes it takes.
+int ri_latent_gather(void* rows, const void* k_pages, const int32_t* len_after, const int32_t* page_table, int table_width, int seqs,
+                     int pages, int key_dim, int page_size, void* stream);
+int ri_latent_prompt_fits(int dim, int rot, int vdim);
+int ri_latent_prompt(void* out, const void* q, int q_stride, const void* keys, int key_stride, const void* turned, int turned_stride,
+                     const void* values, long value_stride, const void* gates, const float* sinks, const int32_t* cu_seqlens, const int32_t* tok_pos,
+                     const int32_t* len_after, int seqs, int tokens, int heads, int dim, int rot, int vdim, float scale, void* stream);
+
 // x[t, i] += bias[i] in place (bias float32 [dim], x of dtype [rows, dim]).
 int ri_add_bias(void* x, int dtype, const float* bias, int rows, int dim, void* stream);
 

@@ -83,6 +83,10 @@ _SIGNATURES = {
     "ri_gemm_mid_packed_bf16": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p],
     "ri_gemm_wide_packed_bf16": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int,
                                  c_int, c_void_p],
+    "ri_latent_gather": [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p],
+    "ri_latent_prompt_fits": [c_int, c_int, c_int],
+    "ri_latent_prompt": [c_void_p, c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_void_p, ctypes.c_long, c_void_p, c_void_p, c_void_p,
+                         c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_void_p],
     "ri_gemm_tiles_bf16": [c_void_p, c_int, c_int, c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p,
                            c_float, c_int, c_void_p],
     "ri_gemm_wide_packed_bf16_plan": [c_int, c_int, c_int, c_void_p, c_void_p],
@@ -1613,7 +1617,7 @@ def gemm_tiles_bf16(x: torch.Tensor, w: torch.Tensor, tile: int, out_dtype=torch
     """``x @ w.T`` for a prompt's many bfloat16 rows in tiles (``tile``: an index of ``TILES``, which the sums do not depend on;
     256 x 128 not with a gate), float32 sums, the result in ``out_dtype`` or in ``out``.  ``activation`` on the sums (bfloat16 out):
     ``"relu2"``; with ``w`` the rows ``[gate; up]``: ``"silu_gate"`` (``silu(gate) * up``) and ``"clamped_gate"`` (as
-    ``glu_clamped_bias``, with its biases and limit).  Rows of ``w`` may be a slice of longer ones."""
+    ``glu_clamped_bias``, with its biases and limit).  Rows of ``x``, ``w`` and ``out`` may be slices of longer ones."""
     m, k = x.shape
     gated = activation in ("silu_gate", "clamped_gate")
     n = w.shape[0] // 2 if gated else w.shape[0]
@@ -1621,8 +1625,10 @@ def gemm_tiles_bf16(x: torch.Tensor, w: torch.Tensor, tile: int, out_dtype=torch
         raise ShapeError(f"a product of {list(x.shape)} with {list(w.shape)}")
     if out is None:
         out = torch.empty((m, n), dtype=out_dtype, device=x.device)
-    _call("ri_gemm_tiles_bf16", _dev(out, "out", None, (m, n)), code(out.dtype), n, _dev(x, "x", torch.bfloat16), k,
-          _dev(w[0], "a row of w", torch.bfloat16), w.stride(0), m, n, k, TILES_ACTIVATIONS[activation], _opt(b_gate, "b_gate", torch.float32, (n,)), _opt(b_up, "b_up", torch.float32, (n,)),
+    elif out.shape != (m, n):
+        raise ShapeError(f"a product of {list(x.shape)} with {list(w.shape)} into {list(out.shape)}")
+    _call("ri_gemm_tiles_bf16", _dev(out[0], "a row of out", None, (n,)), code(out.dtype), out.stride(0), _dev(x[0], "a row of x", torch.bfloat16),
+          x.stride(0), _dev(w[0], "a row of w", torch.bfloat16), w.stride(0), m, n, k, TILES_ACTIVATIONS[activation], _opt(b_gate, "b_gate", torch.float32, (n,)), _opt(b_up, "b_up", torch.float32, (n,)),
           float(limit), int(tile), _stream())
     return out
 
@@ -1841,6 +1847,45 @@ def latent_attention_mfma(q, k_pages, v_pages, tok_pos, tok_seq, page_table, hea
           _dev(page_table, "page_table", torch.int32), page_table.shape[1], tokens, heads, key_dim, rank, page, float(scale),
           _opt(sinks, "sinks", torch.float32, (heads,)), _opt(partial, "partial"), chunks, chunk_pages, shared,
           _opt(cu_seqlens, "cu_seqlens", torch.int32, (seqs + 1,)), seqs, int(bool(max_len)), _stream())
+    return out
+
+
+def latent_prompt_fits(dtype, dim: int, rot: int, vdim: int, page_size: int) -> bool:
+    return dtype == torch.bfloat16 and page_size == 32 and bool(_get("ri_latent_prompt_fits")(dim, rot, vdim))
+
+
+def latent_gather(k_pages, len_after, page_table, pages: int) -> torch.Tensor:
+    """The key rows of a step's sequences side by side, ``[pages * 32, key_dim]``: sequence after sequence, each from a multiple of
+    32 rows on, zeros behind its ``len_after`` keys (``pages``: all of theirs)."""
+    seqs, page, key_dim = len_after.shape[0], k_pages.shape[2], k_pages.shape[3]
+    if k_pages.shape[1] != 1 or page_table.shape[0] != seqs:
+        raise ShapeError(f"latent_gather: key pages {list(k_pages.shape)}, {seqs} sequences, a table of {list(page_table.shape)}")
+    rows = torch.empty((pages * page, key_dim), dtype=torch.bfloat16, device=k_pages.device)
+    _call("ri_latent_gather", _dev(rows, "rows"), _dev(k_pages, "k_pages", torch.bfloat16), _dev(len_after, "len_after", torch.int32),
+          _dev(page_table, "page_table", torch.int32), page_table.shape[1], seqs, pages, key_dim, page, _stream())
+    return rows
+
+
+def latent_prompt(q, heads: int, dim: int, rot: int, vdim: int, keys, rows, values, scale: float, sinks, g_off, cu_seqlens, tok_pos,
+                  len_after) -> torch.Tensor:
+    """bfloat16 ``[T, heads * vdim]``: causal attention of every new token's heads (``q [T, ...]``: ``dim + rot`` elements a head from
+    column 0) over keys ``[keys [R, heads * dim] | the last rot columns of rows [R, .]]`` and values ``values [heads * vdim, R]``, all as
+    ``latent_gather`` lays the sequences' rows; ``sinks`` a head in the denominators or None; ``g_off``: the column of ``q`` from which on
+    every head's gate lies (its sigmoid multiplies the result), or None."""
+    tokens, total = q.shape[0], rows.shape[0]
+    if tuple(keys.shape) != (total, heads * dim) or tuple(values.shape) != (heads * vdim, total) or q.shape[1] < heads * (dim + rot):
+        raise ShapeError(f"latent_prompt: q {list(q.shape)}, keys {list(keys.shape)}, values {list(values.shape)}, rows {list(rows.shape)}")
+    if g_off is not None and not 0 <= g_off <= q.shape[1] - heads:
+        raise ShapeError(f"latent_prompt: gates at column {g_off} of rows of {q.shape[1]}")
+    out = torch.empty((tokens, heads * vdim), dtype=torch.bfloat16, device=q.device)
+    at = _dev(q, "q", torch.bfloat16)
+    _call("ri_latent_prompt", _dev(out, "out"), at, q.shape[1], _dev(keys[0], "a row of keys", torch.bfloat16), keys.stride(0),
+          _dev(rows, "rows", torch.bfloat16) + 2 * (rows.shape[1] - rot), rows.shape[1], _dev(values[0], "a row of values", torch.bfloat16),
+          values.stride(0),
+          None if g_off is None else at + 2 * g_off, _opt(sinks, "sinks", torch.float32, (heads,)),
+          _dev(cu_seqlens, "cu_seqlens", torch.int32), _dev(tok_pos, "tok_pos", torch.int32, (tokens,)),
+          _dev(len_after, "len_after", torch.int32, (cu_seqlens.shape[0] - 1,)), len_after.shape[0], tokens, heads, dim, rot, vdim,
+          float(scale), _stream())
     return out
 
 

@@ -26,7 +26,8 @@ class LatentAttention(Mixer):
     Only ``c`` and the rotated key part are cached, and the attention runs on them as they are: ``q_u . (U_h c) = (U_h^T q_u) .
     c`` and ``sum_j w_j V_h c_j = V_h sum_j w_j c_j``, so the cache entry is one key/value head with key rows ``[c | k_r]`` and
     value rows ``c``, the queries become ``[U_h^T q_u | q_r]`` (``ops.head_products``) and the heads' results go through
-    ``V_h`` afterwards (the same kernel, with the gate).  Names: ``<prefix>q, dkv, dkv.norm, uk, uv, sink, g, o``."""
+    ``V_h`` afterwards (the same kernel, with the gate).  Prompts make the keys and values of all heads instead, once a cached token
+    (``ops.latent_prompt``).  Names: ``<prefix>q, dkv, dkv.norm, uk, uv, sink, g, o``."""
 
     def __init__(self, hidden: int, heads: int, dim: int, rot_dim: int, vdim: int, kv_rank: int, scale: float, prefix: str,
                  eps: float = 1e-6, position: PartSpec | None = None, sinks: bool = True, gate: bool = True,
@@ -68,6 +69,9 @@ class LatentAttention(Mixer):
         # per head: U_h^T as [dim, rank] (the rows of W_uk as they lie) and V_h^T as [rank, vdim]
         self.w_uk = rt.place_matrix(weights[n["uk"]]).view(self.heads, self.dim, self.rank).contiguous() if self.dim else None
         self.w_uv = rt.place_matrix(weights[n["uv"]]).view(self.heads, self.vdim, self.rank).transpose(1, 2).contiguous()
+        self.w_uv_rows = None                                # [heads * vdim, rank], for the prompts' values
+        if self.dim and ops.latent_prompt_fits(rt.dtype, self.dim, self.rot, self.vdim, 32) and not rt.invariant:
+            self.w_uv_rows = rt.place_matrix(weights[n["uv"]])
         self.sink = rt.place_gain(weights[n["sink"]]) if self.sinks else None
         self.w_o = rt.pack(rt.place_matrix(weights[n["o"]]), parts_ok=True)
         self.position.bind(weights, rt)
@@ -80,6 +84,30 @@ class LatentAttention(Mixer):
                 full[:table.shape[0]] = table
             table = full
         self.inv_freq = table if self.rot else None
+
+    def _expanded(self, proj, ctx, store, page_table, g_off):
+        """A prompt's heads ``[T, heads * vdim]`` with the keys and values of all heads made once a cached token."""
+        rt = self.rt
+        pages = sum(-(-(s + n) // 32) for s, n in zip(ctx.starts, ctx.new_counts))
+        rows = ops.latent_gather(store.k_pages, ctx.len_after, page_table, pages)
+        latents = rows[:, :self.rank]
+        keys = torch.empty((rows.shape[0], self.heads * self.dim), dtype=rt.dtype, device=rows.device)
+        values = torch.empty((self.heads * self.vdim, rows.shape[0]), dtype=rt.dtype, device=rows.device)
+        rt.rows_into(keys, latents, self.w_uk.view(self.heads * self.dim, self.rank))
+        rt.rows_into(values, self.w_uv_rows, latents)
+        return ops.latent_prompt(proj, self.heads, self.dim, self.rot, self.vdim, keys, rows, values, self.scale, self.sink,
+                                 g_off if self.gate else None, ctx.cu_seqlens, ctx.tok_pos, ctx.len_after)
+
+    # Keys and values of all heads from EXPAND_TOKENS new tokens on, EXPAND_EACH of them a sequence on average and EXPAND_KEYS cached
+    # tokens for one new one at the most, up to EXPAND_BYTES of them.  (On the latents : so, us, 32 heads, 512 + 64: 128 tokens 65 : 29, eight
+    # of 32 after 1,000 keys 282 : 200; a token's scores gain on the latents what thirty keys' products cost.)
+    EXPAND_TOKENS, EXPAND_EACH, EXPAND_KEYS, EXPAND_BYTES = 128, 32, 32, 2 << 30
+
+    def _expand_pays(self, ctx, proj, store) -> bool:
+        if self.w_uv_rows is None or ctx.T < max(self.EXPAND_TOKENS, self.EXPAND_EACH * ctx.B) or store.page_size != 32 or proj.shape[1] % 8:
+            return False
+        keys = sum(ctx.starts) + ctx.T
+        return keys <= self.EXPAND_KEYS * ctx.T and keys * self.heads * (self.dim + self.vdim) * 2 <= self.EXPAND_BYTES
 
     def cache_need(self):
         return KVNeed(1, self.rank + self.rot, None, self.rank)
@@ -95,7 +123,10 @@ class LatentAttention(Mixer):
             # steps of many bfloat16 tokens: the products per head as one batched product of the library
             batched = (not rt.invariant and proj.dtype == torch.bfloat16 and self.w_uv.dtype == torch.bfloat16
                        and proj.shape[0] >= ops.BATCHED_HEAD_PRODUCTS_FROM)
-            if self.dim and batched:
+            expanded = batched and self._expand_pays(ctx, proj, store)
+            if expanded:
+                q = None
+            elif self.dim and batched:
                 q = ops.head_products_batched(proj, 0, self.dim + self.rot, self.w_uk, self.heads, self.dim, self.rank,
                                               extra=self.rot)
             elif self.dim:
@@ -103,7 +134,9 @@ class LatentAttention(Mixer):
             else:
                 raise ConfigError("a latent attention without unrotated elements has no kernel")
         with profiler.section(profiler.ATTENTION):
-            if not rt.invariant and ops.latent_attention_mfma_fits(q.dtype, self.rank + self.rot, self.rank, store.page_size):
+            if expanded:
+                heads = self._expanded(proj, ctx, store, page_table, kv_at + self.rank + self.rot)
+            elif not rt.invariant and ops.latent_attention_mfma_fits(q.dtype, self.rank + self.rot, self.rank, store.page_size):
                 # the sizes the matrix cores take: a wavefront on 16 heads of a token walks the token's pages; a step of few
                 # tokens cuts the pages into chunks side by side (one walk of 1,024 keys by the two wavefronts a sequence has
                 # takes 319 us, the general kernel 106)
@@ -112,7 +145,9 @@ class LatentAttention(Mixer):
             else:
                 o = ops.attention(q, store.k_pages, store.v_pages, ctx.tok_pos, ctx.tok_seq, page_table, self.heads, 1,
                                   self.rank + self.rot, None, self.scale, sinks=self.sink, **ctx.runs())
-            if batched and o.dtype == torch.bfloat16:
+            if expanded:
+                pass
+            elif batched and o.dtype == torch.bfloat16:
                 heads = ops.head_products_batched(o, 0, self.rank, self.w_uv, self.heads, self.rank, self.vdim,
                                                   gates=proj if self.gate else None, g_off=kv_at + self.rank + self.rot)
             else:

@@ -386,8 +386,8 @@ class Runtime:
         return ops.gemm_tiles_bf16(x, w, tile, self.dtype, activation, limit=limit)
 
     def rows_into(self, out, x, w: torch.Tensor) -> None:
-        """``out <- x @ w.T`` for rows and a stretch of a larger matrix, its rows or its columns."""
-        tile = self._tile(x, w, out.dtype) if out.data_ptr() % 16 == 0 else None
+        """``out <- x @ w.T``; rows of any of the three may be stretches of longer ones."""
+        tile = self._tile(x, w, out.dtype) if out.data_ptr() % 16 == 0 and out.stride(0) % 8 == 0 else None
         if tile is None:
             torch.mm(x, w.t(), out=out)
         else:
@@ -399,7 +399,7 @@ class Runtime:
         tile = _tiles_plan(x.shape[0], w.shape[0], w.shape[1], out_dtype == torch.float32, activation)
         if tile is None or w.stride(1) != 1 or w.stride(0) % 8 or w.data_ptr() % 16:
             return None
-        if isinstance(x, torch.Tensor) and not (x.is_contiguous() and x.data_ptr() % 16 == 0):
+        if isinstance(x, torch.Tensor) and (x.stride(1) != 1 or x.stride(0) % 8 or x.stride(0) < x.shape[1] or x.data_ptr() % 16):
             return None                                          # the library's product takes any strides
         return tile
 

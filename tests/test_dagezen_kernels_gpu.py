@@ -942,3 +942,53 @@ def test_walks_in_tiles_of_four_rows(ops, kind, rows, cols, heads, many, dtype):
     assert np.abs(whole - want).max() <= bound * np.abs(want).max()
     cut, cut_state = run(3)
     assert np.array_equal(cut, whole) and np.array_equal(cut_state, state)
+
+
+# ---------------------------------------------------------------- the latent attention of prompts, keys and values of all heads made
+@pytest.mark.parametrize("dim, rot, vdim, rank, heads, counts, starts", [
+    (64, 64, 64, 128, 3, [1, 129, 40, 33], [0, 0, 31, 64]), (64, 64, 64, 64, 2, [5, 1, 130], [100, 63, 7]),
+    (128, 64, 128, 512, 2, [70, 3], [0, 33]), (128, 64, 128, 64, 1, [32, 256], [32, 0])])
+def test_latent_attention_of_prompts_with_every_heads_keys(ops, dim, rot, vdim, rank, heads, counts, starts):
+    """Pages in shuffled order laid side by side; sequences of a token, of a run of 128 and one more, in the middle of a page, at its
+    border, with keys before them; sinks and gates, and without; against 64 bits on the same keys and values.  The weights are rounded to
+    bfloat16 (2^-9 of each) and the result once more: 2^-8 of the largest."""
+    rng = np.random.default_rng(dim + len(counts))
+    seqs, key_dim, ends = len(counts), rank + rot, [s + n for s, n in zip(starts, counts)]
+    held = [-(-e // PAGE) for e in ends]
+    order, width = rng.permutation(sum(held) + 2), max(held) + 1
+    table, at = np.zeros((seqs, width), np.int32), 0
+    for s, n in enumerate(held):
+        table[s, :n], at = order[at:at + n], at + n
+    k_pages = guarded((torch.randn((sum(held) + 2, 1, PAGE, key_dim), device=DEV) * 0.6).to(torch.bfloat16))
+    rows = ops.latent_gather(k_pages, t(ends, torch.int32), t(table, torch.int32), sum(held))
+    want_rows, pages = [], f64(k_pages)[:, 0]
+    for s, e in enumerate(ends):
+        own = np.concatenate([pages[table[s, j]] for j in range(held[s])])
+        own[e:] = 0
+        want_rows.append(own)
+    assert np.array_equal(f64(rows), np.concatenate(want_rows))
+    c = f64(rows)[:, :rank]
+    uk, uv = rng.normal(size=(heads * dim, rank)) / np.sqrt(rank), rng.normal(size=(heads * vdim, rank)) / np.sqrt(rank)
+    keys, values = t(c @ uk.T, torch.bfloat16), t(uv @ c.T, torch.bfloat16)
+    qw, tokens = heads * (dim + rot), sum(counts)
+    q = guarded((torch.randn((tokens, qw + 16 + (-heads) % 8 + heads), device=DEV) * 1.5).to(torch.bfloat16))
+    sinks, g_off, scale = rng.normal(size=heads), qw + 16, 0.3
+    cu = np.concatenate([[0], np.cumsum(counts)])
+    pos = t([p for s, n in enumerate(counts) for p in range(starts[s], starts[s] + n)], torch.int32)
+    k64, v64, q64 = f64(keys), f64(values), f64(q)
+    for sink, gate in ((True, True), (False, False)):
+        got = ops.latent_prompt(q, heads, dim, rot, vdim, keys, rows, values, scale, t(sinks) if sink else None, g_off if gate else None,
+                                t(cu, torch.int32), pos, t(ends, torch.int32))
+        want, first = np.zeros((tokens, heads, vdim)), 0
+        for s in range(seqs):
+            for h in range(heads):
+                k = np.concatenate([k64[first:first + ends[s], h * dim:(h + 1) * dim], f64(rows)[first:first + ends[s], rank:]], 1)
+                sc = scale * q64[cu[s]:cu[s + 1], h * (dim + rot):(h + 1) * (dim + rot)] @ k.T
+                sc[np.arange(ends[s])[None, :] > np.arange(starts[s], ends[s])[:, None]] = -np.inf
+                top = sc.max(1, keepdims=True)
+                w = np.exp(sc - top)
+                den = w.sum(1, keepdims=True) + (np.exp(np.float32(sinks[h]) - top) if sink else 0)
+                o = (w / den) @ v64[h * vdim:(h + 1) * vdim, first:first + ends[s]].T
+                want[cu[s]:cu[s + 1], h] = o / (1 + np.exp(-q64[cu[s]:cu[s + 1], g_off + h, None])) if gate else o
+            first += held[s] * PAGE
+        close(got, want.reshape(tokens, -1), 2.0 ** -8, f"latent prompt, sinks {sink}, gates {gate}")
