@@ -34,6 +34,7 @@
 
 #include "api.h"
 #include "common.h"
+#include "matrix_async.h"
 
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
@@ -620,6 +621,270 @@ attn_prefill_mfma_kernel(bf16_t* __restrict__ out, const bf16_t* __restrict__ qk
             w.y = (uint32_t)f32_to_bf16(c.o[j][dt][2] * inv) | ((uint32_t)f32_to_bf16(c.o[j][dt][3] * inv) << 16);
             *reinterpret_cast<uint2*>(op + dt * 16) = w;
         }
+    }
+}
+
+// How a page lies in LDS that copies past the registers fill, heads of DH elements: key rows [32][DH] in the order of the two products' rows, value
+// rows [DH][32], no padding; the 16-byte pieces of a row are exchanged by the row's number, so that the sixteen lanes LDS serves at once (of a
+// fragment's 0 to 3, 12 to 15 and 20 to 27, and so on) meet all its 64 banks: rows of 256 bytes by row % 16, of 128 by row % 8, of 64 by
+// -(row / 4) % 4.  Two wavefronts copy a page of keys, two one of values, a kilobyte each time.
+#define PAIR_SLOTS 2             // pairs of pages of keys, and of values, in LDS
+template <int DH>
+struct CopiedPage {
+    static constexpr int PIECES = DH / 8, MINE = DH / 32;    // of a key row; copies of a wavefront
+    __device__ static __forceinline__ int exchange(int row, int pieces) { return pieces == 4 ? -(row >> 2) & 3 : row & (pieces - 1); }
+    // where this lane's pieces lie in a page, bytes: of the key page for wavefronts 0 and 1, of the value page for 2 and 3
+    __device__ static __forceinline__ void offsets(uint32_t (&off)[MINE], int wave, int lane) {
+#pragma unroll
+        for (int i = 0; i < MINE; ++i) {
+            const int piece = ((wave & 1) * MINE + i) * 64 + lane, pieces = wave < 2 ? PIECES : 4, row = piece / pieces;
+            const int from = wave < 2 ? ((row & 15) >> 2) * 8 + (row >> 4) * 4 + (row & 3) : row;
+            off[i] = 16u * (uint32_t)(from * pieces + (piece % pieces ^ exchange(row, pieces)));
+        }
+    }
+    __device__ static __forceinline__ void copy(ma_lds_t to, const uint32_t (&off)[MINE], const bf16_t* page, int half) {
+#pragma unroll
+        for (int i = 0; i < MINE; ++i) ma_copy16(to + (half * MINE + i) * 1024, off[i], page);
+    }
+    template <int N>
+    __device__ static __forceinline__ void keys(Frag (&kf)[2][N], const bf16_t* page, int lane) {
+        const uint4* from = reinterpret_cast<const uint4*>(page);
+        const int i = lane & 15, jg = lane >> 4;
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+            for (int ks = 0; ks < N; ++ks) kf[kt][ks].u = from[(kt * 16 + i) * PIECES + ((4 * ks + jg) ^ exchange(i, PIECES))];
+    }
+    template <int N>
+    __device__ static __forceinline__ void values(Frag (&vf)[N], const bf16_t* page, int lane) {
+        const uint4* from = reinterpret_cast<const uint4*>(page);
+        const int i = lane & 15, jg = lane >> 4;
+#pragma unroll
+        for (int dt = 0; dt < N; ++dt) vf[dt].u = from[(dt * 16 + i) * 4 + (jg ^ exchange(i, 4))];
+    }
+};
+
+
+// The prompt kernel for long sequences, heads whose values have their size: the walk above, two pages a turn.  A turn is a chain (scores, their maximum
+// over a column's lanes, the reference point, weights, values) that two or three wavefronts a SIMD do not fill; with 64 keys there are half as many chains,
+// maxima and moves of the reference point.  Pages are paired by their numbers (2 u and 2 u + 1), so that a column's sums do not depend on its
+// tile; a page of a pair that the walk does not hold (before its first, behind its last, behind the kept ones) is another one's data under
+// the mask.  Pages go straight into LDS: keys of pair u + 2 and values of pair u + 1 while pair u is weighed; one place a turn where the wavefronts
+// meet.  Bound by the chain still: 1.7 us a turn of one wavefront, 1.0 PFLOP/s at 8,192 tokens of 64 heads.  us, a page a turn : so (heads of 128
+// over 8): 8,192 of 64 heads 1,216 : 1,081, 3,000 199 : 161, 8,192 of 16 345 : 288, 2,048 of 32 65 : 57, 512 15.3 : 13.2, 500 + 1,500 + 532 52 : 45, 16 of 16 to
+// 1,024 of 16 heads 55 : 53; heads of 64: 16 of 16 to 1,024 147 : 45, 6,000 252 : 204; of 32: 2,048 33 : 23.  With three single slots of keys and of
+// values and a meeting a page (three workgroups of one tile a compute unit instead of two) 27 : 30 us for 16 of 16 to 700, but 55 : 58 at 2,048 and
+// 52 : 45 at 500 + 1,500 + 532.
+template <int DH, int NT, int FORM>
+__global__ void __launch_bounds__(256, 2)
+attn_prefill_pairs_kernel(bf16_t* __restrict__ out, const bf16_t* __restrict__ qkv, int q_stride,
+                          const bf16_t* __restrict__ k_pages, const bf16_t* __restrict__ v_pages,
+                          const int32_t* __restrict__ cu_seqlens, const int32_t* __restrict__ tok_pos,
+                          const int32_t* __restrict__ page_table, int table_width, int heads, int kv_heads,
+                          Reach reach, float scale_log2, float cap_pre, float cap_post,
+                          const float* __restrict__ slopes, float inv_scale, int keep_first,
+                          const float* __restrict__ sinks, int seqs, int long_runs) {
+    typedef CopiedPage<DH> Copied;
+    __shared__ __attribute__((aligned(16))) bf16_t k_lds[PAIR_SLOTS][2][PAGE * DH];
+    __shared__ __attribute__((aligned(16))) bf16_t v_lds[PAIR_SLOTS][2][PAGE * DH];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int kvh = blockIdx.x;                              // (workgroups on the same keys meet in one XCD's L2)
+    const int group = heads / kv_heads;
+    const int tile_tokens = (16 * NT) / group;               // tokens per wavefront
+    const int of_wg = 4 * tile_tokens;
+    int b = blockIdx.y, t_end, t_wg;
+    if (long_runs > 0) {                                     // (prefill_grid) the runs of the sequences with several, then those with one
+        Run run;
+        if ((int)blockIdx.y < long_runs) {
+            if (!run_of(blockIdx.y, cu_seqlens, seqs, of_wg + 1, of_wg, 1, run)) return;
+            run.first = (run.tokens - 1) / of_wg * of_wg - run.first;
+        } else if (!run_of((int)blockIdx.y - long_runs, cu_seqlens, seqs, 1, of_wg, 1, run, of_wg)) return;
+        b = run.seq;
+        t_end = run.start + run.tokens;
+        t_wg = run.start + run.first;
+    } else {
+        // the last tokens of a sequence see the most keys: the workgroups of all sequences' last tokens are launched first
+        t_end = cu_seqlens[b + 1];
+        t_wg = cu_seqlens[b] + (int)(gridDim.z - 1 - blockIdx.z) * of_wg;
+        if (t_wg >= t_end) return;                           // the whole workgroup leaves
+    }
+    const int t0 = t_wg + wave * tile_tokens;
+    const int nt = max(0, min(tile_tokens, t_end - t0));     // a wavefront without tokens still helps to fetch
+
+    Columns<DH, NT> c;
+    init_columns<DH, NT, DH>(c);
+    c.cap_pre = FORM == PREFILL_PLAIN ? 0.f : cap_pre;
+    c.cap_post = cap_post;
+    c.biased = FORM == PREFILL_ANY && slopes != nullptr;
+    c.capped = FORM == PREFILL_CAPPED;
+    c.keep = reach.window > 0 ? keep_first : 0;
+    const int jg = lane >> 4;
+    float sink[NT];                                          // the column's sink in the exponents' units; -inf: none
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+        const int col = j * 16 + (lane & 15);
+        const int tl = col / group, g = col - tl * group;
+        if (FORM == PREFILL_ANY && slopes) c.bias[j] = slopes[kvh * group + g] * inv_scale;
+        sink[j] = sinks ? sinks[kvh * group + g] * 1.4426950408889634f : -INFINITY;
+        if (tl < nt) {
+            const int tok = t0 + tl;
+            c.qpos[j] = tok_pos[tok];
+            c.lo[j] = reach.first(c.qpos[j]);
+            const bf16_t* qp = qkv + (long)tok * q_stride + (kvh * group + g) * DH + jg * 8;
+#pragma unroll
+            for (int ks = 0; ks < DH / 32; ++ks) c.q[j][ks].u = *reinterpret_cast<const uint4*>(qp + ks * 32);
+        }
+    }
+    // pages the workgroup walks (every wavefront takes them all): those with kept first tokens, then from p_lo to p_hi
+    const int p_lo = reach.first(tok_pos[t_wg]) / PAGE, p_hi = tok_pos[min(t_end, t_wg + of_wg) - 1] / PAGE;
+    const int kept = (c.keep + PAGE - 1) / PAGE, kept_pairs = min((kept + 1) / 2, p_lo / 2), u_last = kept_pairs + p_hi / 2 - p_lo / 2;
+    // a pair is open to the whole wavefront when its last key is at or before the first token's position
+    // and its first key inside the last token's window; wavefronts with unused columns mask always
+    const bool full = nt * group == 16 * NT;
+    const int min_qpos = (nt > 0 && full) ? tok_pos[t0] : -1;
+    const int max_lo = nt > 0 ? reach.first(tok_pos[t0 + nt - 1]) : 0;
+    const int32_t* table = page_table + (long)b * table_width;
+    auto page_of = [&](int u) { return 2 * (u < kept_pairs ? u : p_lo / 2 + u - kept_pairs); };       // the first page of a pair
+    auto open = [&](int u) { const int at = page_of(u) * PAGE; return u >= kept_pairs && at + 2 * PAGE - 1 <= min_qpos && at >= max_lo; };
+    // where the data of a pair's pages lie; for a page that is not walked: of one that is
+    auto look = [&](int u, int h) -> int {
+        u = min(u, u_last);
+        const int page = page_of(u) + h;
+        return table[min(page < kept ? page : max(page, p_lo), p_hi)];
+    };
+    uint32_t off[Copied::MINE];
+    Copied::offsets(off, wave, lane);
+    auto fetch_keys = [&](int u, const int (&at)[2]) {       // (wavefronts 0 and 1)
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+            Copied::copy(ma_lds(k_lds[(unsigned)u % PAIR_SLOTS][h]), off, k_pages + ((long)at[h] * kv_heads + kvh) * (PAGE * DH), wave);
+    };
+    auto fetch_values = [&](int u, const int (&at)[2]) {     // (wavefronts 2 and 3)
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+            Copied::copy(ma_lds(v_lds[(unsigned)u % PAIR_SLOTS][h]), off, v_pages + ((long)at[h] * kv_heads + kvh) * (PAGE * DH), wave - 2);
+    };
+    auto fetch = [&](int u, const int (&k)[2], const int (&v)[2]) {       // keys of pair u, values of pair u - 1
+        if (wave < 2) fetch_keys(u, k);
+        else fetch_values(u - 1, v);
+    };
+    auto scores = [&](float (&s)[NT][2][8], int u) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            Frag kf[2][DH / 32];
+            Copied::keys(kf, k_lds[(unsigned)u % PAIR_SLOTS][h], lane);
+            float one[NT][8];
+            scores_of<DH, NT, DH>(c, kf, one, page_of(u) + h, lane);
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) s[j][h][e] = one[j][e];
+        }
+    };
+    auto mask = [&](float (&s)[NT][2][8], int u) {
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int key0 = (page_of(u) + h) * PAGE + jg * 8;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const int key = key0 + e;
+                    if (key > c.qpos[j] || (key < c.lo[j] && key >= c.keep)) s[j][h][e] = -INFINITY;
+                }
+            }
+    };
+    auto maxima = [&](const float (&s)[NT][2][8], float (&m_new)[NT]) {
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+            float mx = s[j][0][0];
+#pragma unroll
+            for (int e = 1; e < 16; ++e) mx = fmaxf(mx, s[j][e / 8][e % 8]);
+            m_new[j] = fmaxf(c.m[j], column_max<(NT >= 2 || DH < 128)>(mx) * scale_log2);
+        }
+    };
+    float s_cur[NT][2][8], ref[NT], m_new[NT];
+    int now[2], next[2];                                     // where the pages of pairs u + 1 and u + 2 lie
+    {
+        const int first[2] = {look(0, 0), look(0, 1)};
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            now[h] = look(1, h);
+            next[h] = look(2, h);
+        }
+        if (wave < 2) fetch_keys(0, first);
+        fetch(1, now, first);
+    }
+    ma_wait_copies<2 * Copied::MINE>();
+    ma_meet();
+    scores(s_cur, 0);
+    if (!open(0)) mask(s_cur, 0);
+    maxima(s_cur, m_new);
+    move_reference<DH, NT, DH>(c, m_new, ref);
+    auto weights = [&](Frag (&w)[NT], int h) {
+        float one[NT][8];
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) one[j][e] = s_cur[j][h][e];
+        weights_of<DH, NT, DH>(c, one, ref, w, scale_log2);
+    };
+    auto values = [&](const Frag (&w)[NT], int u, int h) {
+        Frag vf[DH / 16];
+        Copied::values(vf, v_lds[(unsigned)u % PAIR_SLOTS][h], lane);
+        weighted_values<DH, NT, DH>(c, vf, w);
+    };
+    auto turn = [&](int u, auto masked) {                    // u: the pair whose weights are due
+        ma_wait_copies<0>();                                  // the keys of pair u + 1 and the values of pair u are there,
+        ma_wait_lds();                                        // the keys of pair u and the values of pair u - 1 read
+        ma_meet();
+        fetch(u + 2, next, now);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            now[h] = next[h];
+            next[h] = look(u + 3, h);
+        }
+        Frag w[2][NT];
+        float s_next[NT][2][8];
+        scores(s_next, u + 1);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) weights(w[h], h);
+        if (decltype(masked)::value) mask(s_next, u + 1);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) values(w[h], u, h);
+        maxima(s_next, m_new);
+        move_reference<DH, NT, DH>(c, m_new, ref);
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) s_cur[j][e / 8][e % 8] = s_next[j][e / 8][e % 8];
+    };
+    int u = 0;
+    for (; u < u_last && !open(u + 1); ++u) turn(u, std::true_type());
+    for (; u < u_last && open(u + 1); ++u) turn(u, std::false_type());
+    for (; u < u_last; ++u) turn(u, std::true_type());
+    ma_wait_copies<0>();                                      // (also what was copied for nobody: it must not arrive in another workgroup's LDS)
+    ma_meet();
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {                            // the last pair's weights and value products
+        Frag w[NT];
+        weights(w, h);
+        values(w, u_last, h);
+    }
+    finish_columns<DH, NT, DH>(c);
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+        const int col = j * 16 + (lane & 15);
+        const int tl = col / group, g = col - tl * group;
+        if (tl >= nt) continue;
+        // the sink joins the denominator alone: exp(sink - maximum), in the exponents' units (exp2 of -inf is 0)
+        const float inv = 1.0f / (c.l[j] + __builtin_amdgcn_exp2f(sink[j] - c.m[j]));
+        bf16_t* op = out + ((long)(t0 + tl) * heads + kvh * group + g) * DH + jg * 4;
+#pragma unroll
+        for (int dt = 0; dt < DH / 16; ++dt)
+            *reinterpret_cast<uint2*>(op + dt * 16) = uint2{pack_bf16x2(c.o[j][dt][0] * inv, c.o[j][dt][1] * inv),
+                                                            pack_bf16x2(c.o[j][dt][2] * inv, c.o[j][dt][3] * inv)};
     }
 }
 

@@ -53,6 +53,20 @@ static int prefill_tiles(int head_dim, int group, int max_new, int seqs, int kv_
     return nt;
 }
 
+// Pairs of pages a turn (attn_prefill_pairs_kernel) where a sequence brings this many tokens on average: shorter ones are mostly the start and the
+// diagonal, which pairs make longer.  us, a page a turn : pairs (heads of 128 over 8): 40 of 64 (32 heads) 16.5 : 18.6, 16 of 200 (16) 15.9 : 17.2, 16 of 300
+// 24.1 : 25.8, 16 of 16 to 700 27 : 30, four of 300 (32) 15.3 : 14.0, eight of 500 40.4 : 39.8, 16 of 16 to 1,024 (16) 55 : 53, two of 1,000 (32) 39 : 35.
+// Two tiles a wavefront there (heads of 128) from three of their workgroups a compute unit on, for one sequence from two on, one : two tiles: 2,048 (512
+// workgroups) 58 : 56, 1,792 (448) 48 : 49, 2,816 (704) 94 : 80; two of 1,500 (752) 64 : 69, 500 + 1,500 + 532 (632) 45 : 67, eight of 500 (1,024) 42 : 39, 8,192 of 64 heads
+// 1,380 : 1,081.  Heads of 32 and 64: one, 2,048 of 32 heads of 64 32.5 : 38, 6,000 204 : 221 (4,096 99 : 95); more only where a key head's queries need them.
+#define PAIRS_MIN_TOKENS 400
+static int pair_tiles(int head_dim, int group, int seqs, int kv_heads, int tokens) {
+    const int of_wg = 4 * (32 / (group <= 32 ? group : 32));
+    const long wgs = (tokens + (long)seqs * of_wg / 2) / of_wg * kv_heads;
+    if (group > 16) return group > 32 ? 4 : 2;
+    return head_dim == 128 && wgs >= (seqs == 1 ? 2L : 3L) * ri_compute_units() ? 2 : 1;
+}
+
 // The column tiles a wavefront takes of a step (host code only).
 extern "C" int ri_attention_prefill_tiles(int head_dim, int group, int max_new, int seqs, int kv_heads, int tokens, int weighted) {
     return prefill_tiles(head_dim, group, max_new, seqs, kv_heads, tokens, weighted);
@@ -63,7 +77,7 @@ extern "C" int ri_attention_prefill_kept_bf16(void* out, const void* qkv, int q_
                                               const int32_t* page_table, int table_width, int seqs, int max_new,
                                               int heads, int kv_heads, int head_dim, int page_size, int window, int chunk,
                                               float scale, float softcap, const float* slopes, int keep_first,
-                                              const float* sinks, int tokens, int weighted, void* stream) {
+                                              const float* sinks, int tokens, int weighted, int pairs, void* stream) {
     RI_REQUIRE(chunk >= 0 && (chunk == 0 || window <= 0), "attention_prefill: chunks of %d beside a window of %d", chunk, window);
     const Reach reach = {window, chunk};
     RI_REQUIRE(keep_first >= 0, "attention_prefill_bf16: %d first tokens kept", keep_first);
@@ -72,7 +86,11 @@ extern "C" int ri_attention_prefill_kept_bf16(void* out, const void* qkv, int q_
     if (check_common("attention_prefill_bf16", heads, kv_heads, head_dim, page_size, q_stride, table_width)) return 1;
     const int group = heads / kv_heads;
     RI_REQUIRE(seqs > 0 && seqs <= 65535 && max_new > 0, "attention_prefill_bf16: seqs %d, max_new %d", seqs, max_new);
-    const int nt_tiles = prefill_tiles(head_dim, group, max_new, seqs, kv_heads, tokens, weighted);
+    RI_REQUIRE(pairs >= -1 && pairs <= 1, "attention_prefill_bf16: pairs %d", pairs);
+    RI_REQUIRE(group <= (head_dim <= 64 ? 64 : 32), "attention_prefill_bf16: %d query heads per kv head (at most %d)", group, head_dim <= 64 ? 64 : 32);
+    const bool paired = pairs == -1 ? tokens >= (long)PAIRS_MIN_TOKENS * seqs : pairs == 1;
+    const int nt_tiles = paired ? pair_tiles(head_dim, group, seqs, kv_heads, tokens)
+                                : prefill_tiles(head_dim, group, max_new, seqs, kv_heads, tokens, weighted);
     RI_REQUIRE(group <= 16 * nt_tiles, "attention_prefill_bf16: %d query heads per kv head (at most %d)", group,
                16 * nt_tiles);
     const int tile_tokens = (16 * nt_tiles) / group;
@@ -83,16 +101,18 @@ extern "C" int ri_attention_prefill_kept_bf16(void* out, const void* qkv, int q_
     const float scale_log2 = scale * 1.4426950408889634f;
     hipStream_t s = (hipStream_t)stream;
     const int form = slopes ? PREFILL_ANY : cap_pre != 0.f ? PREFILL_CAPPED : PREFILL_PLAIN;
+#define RI_PREFILL_ARGS                                                                                          \
+    (bf16_t*)out, (const bf16_t*)qkv, q_stride, (const bf16_t*)k_pages, (const bf16_t*)v_pages, cu_seqlens,      \
+        tok_pos, page_table, table_width, heads, kv_heads, reach, scale_log2, cap_pre, cap_post, slopes,         \
+        1.f / scale, keep_first, sinks, seqs, long_runs
 #define RI_PREFILL_GO(DH, NT, FORM)                                                                              \
-    attn_prefill_mfma_kernel<DH, NT, DH, false, FORM><<<grid, 256, 0, s>>>(                                      \
-        (bf16_t*)out, (const bf16_t*)qkv, q_stride, (const bf16_t*)k_pages, (const bf16_t*)v_pages,              \
-        cu_seqlens, tok_pos, page_table, table_width, heads, kv_heads, reach, scale_log2, cap_pre,              \
-        cap_post, slopes, 1.f / scale, keep_first, sinks, seqs, long_runs)
+    if (paired) attn_prefill_pairs_kernel<DH, NT, FORM><<<grid, 256, 0, s>>>(RI_PREFILL_ARGS);                   \
+    else attn_prefill_mfma_kernel<DH, NT, DH, false, FORM><<<grid, 256, 0, s>>>(RI_PREFILL_ARGS)
 #define RI_PREFILL_CASE(DH, NT)                                                                                  \
     case DH * 8 + NT:                                                                                            \
-        if (form == PREFILL_PLAIN) RI_PREFILL_GO(DH, NT, PREFILL_PLAIN);                                         \
-        else if (form == PREFILL_CAPPED) RI_PREFILL_GO(DH, NT, PREFILL_CAPPED);                                  \
-        else RI_PREFILL_GO(DH, NT, PREFILL_ANY);                                                                 \
+        if (form == PREFILL_PLAIN) { RI_PREFILL_GO(DH, NT, PREFILL_PLAIN); }                                     \
+        else if (form == PREFILL_CAPPED) { RI_PREFILL_GO(DH, NT, PREFILL_CAPPED); }                              \
+        else { RI_PREFILL_GO(DH, NT, PREFILL_ANY); }                                                             \
         break;
     switch (head_dim * 8 + nt_tiles) {
         RI_PREFILL_CASE(32, 4)
@@ -106,6 +126,7 @@ extern "C" int ri_attention_prefill_kept_bf16(void* out, const void* qkv, int q_
     }
 #undef RI_PREFILL_CASE
 #undef RI_PREFILL_GO
+#undef RI_PREFILL_ARGS
     RI_LAUNCH_CHECK("attention_prefill_bf16");
     return 0;
 }
@@ -117,7 +138,7 @@ extern "C" int ri_attention_prefill_bf16(void* out, const void* qkv, int q_strid
                                          float scale, float softcap, const float* slopes, void* stream) {
     return ri_attention_prefill_kept_bf16(out, qkv, q_stride, k_pages, v_pages, cu_seqlens, tok_pos, page_table, table_width,
                                           seqs, max_new, heads, kv_heads, head_dim, page_size, window, 0, scale, softcap, slopes,
-                                          0, nullptr, (int)(max_new * (long)seqs < 1 << 30 ? max_new * (long)seqs : 1 << 30), max_new, stream);
+                                          0, nullptr, (int)(max_new * (long)seqs < 1 << 30 ? max_new * (long)seqs : 1 << 30), max_new, -1, stream);
 }
 
 // Whether the streaming kernel ranks the step's sequences by their lengths (host code only).

@@ -32,6 +32,7 @@ __device__ __forceinline__ ma_lds_t ma_lds(void* p) { return (uint32_t)(uintptr_
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
 __device__ __forceinline__ void ma_copy16(ma_lds_t at, uint32_t off, const void* base) {
+    at = __builtin_amdgcn_readfirstlane(at);
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(at), "v"(off), "s"(base) : "memory", "m0");
 }
 #pragma clang diagnostic pop

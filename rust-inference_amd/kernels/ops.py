@@ -109,7 +109,7 @@ _SIGNATURES = {
     "ri_argmax": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p],
     "ri_attention_prefill_kept_bf16": [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int,
                                        c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_float, c_void_p, c_int,
-                                       c_void_p, c_int, c_int, c_void_p],
+                                       c_void_p, c_int, c_int, c_int, c_void_p],
     "ri_attention_prefill_tiles": [c_int, c_int, c_int, c_int, c_int, c_int, c_int],
     "ri_attention_kept": [c_void_p, c_void_p, c_int, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int,
                           c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_float, c_void_p, c_int, c_void_p,
@@ -1257,11 +1257,14 @@ def attention_prefill_tiles(new_counts, heads: int, kv_heads: int, head_dim: int
 def attention_prefill_bf16(qkv, k_pages, v_pages, cu_seqlens, tok_pos, page_table, seqs: int, max_new: int,
                            heads: int, kv_heads: int, head_dim: int, window: int | None, scale: float,
                            softcap: float | None = None, slopes: torch.Tensor | None = None, keep_first: int = 0,
-                           sinks: torch.Tensor | None = None, q_off: int = 0, chunk: int | None = None, new_counts=None) -> torch.Tensor:
+                           sinks: torch.Tensor | None = None, q_off: int = 0, chunk: int | None = None, new_counts=None,
+                           paired: bool | None = False) -> torch.Tensor:
     """Matrix-core attention for any number of new tokens per sequence (bfloat16, pages of 32).  With ``softcap`` a
     score ``s`` becomes ``softcap * tanh(s / softcap)`` before the softmax; with ``slopes`` (float32 ``[heads]``) head
     ``h``'s score at position ``p`` for the key at ``j`` then loses ``slopes[h] * (p - j)``.  ``keep_first``, ``sinks``,
-    ``q_off`` and ``chunk`` as in ``attention``.  ``new_counts``: every sequence's new tokens, where the caller knows them."""
+    ``q_off`` and ``chunk`` as in ``attention``.  ``new_counts``: every sequence's new tokens, where the caller knows them.
+    ``paired``: a sequence's pages two by two (True) or one by one (False), None: by what the sequences bring on average; a token's result
+    is the same bits with every step of either kind."""
     tokens, stride = qkv.shape
     if q_off < 0 or q_off + heads * head_dim > stride or q_off % 8:
         raise ShapeError(f"attention: queries at column {q_off} of rows of {stride} for {heads} heads of {head_dim}")
@@ -1272,7 +1275,7 @@ def attention_prefill_bf16(qkv, k_pages, v_pages, cu_seqlens, tok_pos, page_tabl
           _dev(page_table, "page_table", torch.int32), page_table.shape[1], seqs, max_new, heads, kv_heads, head_dim,
           k_pages.shape[2], int(window or 0), int(chunk or 0), float(scale), float(softcap or 0.0),
           _opt(slopes, "slopes", torch.float32, (heads,)), int(keep_first or 0), _opt(sinks, "sinks", torch.float32, (heads,)),
-          tokens, _weighted_length(new_counts, tokens, max_new), _stream())
+          tokens, _weighted_length(new_counts, tokens, max_new), -1 if paired is None else int(paired), _stream())
     return out
 
 

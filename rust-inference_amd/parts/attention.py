@@ -376,7 +376,7 @@ class GroupedQueryAttention(Mixer):
             return ops.attention_prefill_bf16(proj, store.k_pages, store.v_pages, ctx.cu_seqlens, ctx.tok_pos, page_table,
                                               ctx.B, ctx.max_new, self.heads, self.kv_heads, self.head_dim, self.window,
                                               self.scale, self.softcap, slopes, self.keep_first, self.sink, q_at, self.chunk,
-                                              ctx.new_counts)
+                                              ctx.new_counts, paired=False if self.rt.invariant else None)
         return ops.attention(proj, store.k_pages, store.v_pages, ctx.tok_pos, ctx.tok_seq, page_table, self.heads,
                              self.kv_heads, self.head_dim, self.window, self.scale, self.softcap, slopes,
                              keep_first=self.keep_first, sinks=self.sink, q_off=q_at, chunk=self.chunk, **ctx.runs())
@@ -425,6 +425,6 @@ class GroupedQueryAttention(Mixer):
                                                  tiled_out=self.rt.takes_tiled(self.w_o, ctx.B, self.b_o is None),
                                                  softcap=cap, slopes=slopes)
             return ops.attention_prefill_bf16(qkv, store.k_pages, store.v_pages, ctx.cu_seqlens, ctx.tok_pos,
-                                              page_table, ctx.B, ctx.max_new, *args, cap, slopes, new_counts=ctx.new_counts)
+                                              page_table, ctx.B, ctx.max_new, *args, cap, slopes, new_counts=ctx.new_counts, paired=None)
         return ops.attention(qkv, store.k_pages, store.v_pages, ctx.tok_pos, ctx.tok_seq, page_table, *args, cap, slopes,
                              **ctx.runs())

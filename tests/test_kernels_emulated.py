@@ -89,7 +89,7 @@ def runs():
         "sixteen units": _start([*PYTEST, SMALL_MACHINE], {"RI_EMU_COMPUTE_UNITS": "16"}),
         "one unit": _start([*PYTEST, *_workers(2), SMALL_MACHINE, KERNEL_TESTS, "-k", ONE_UNIT], {"RI_EMU_COMPUTE_UNITS": "1"}),
         "one unit, rows": _start([*PYTEST, *_workers(2), KERNEL_TESTS, "-k", ONE_UNIT_ROWS], {"RI_EMU_COMPUTE_UNITS": "1"}),
-        "one unit, tiles": _start([*PYTEST, KERNEL_TESTS, "-k", "over_rounds"], {"RI_EMU_COMPUTE_UNITS": "1"}),
+        "one unit, tiles": _start([*PYTEST, KERNEL_TESTS, "-k", "over_rounds or (in_pairs_of_pages and 16-1-128)"], {"RI_EMU_COMPUTE_UNITS": "1"}),
         "sampler": _start([*PYTEST, *_workers(2), SAMPLER_TESTS, "-k", SAMPLER_SELECT]),
         "zidepel": _start([*PYTEST, *_workers(2), ZIDEPEL_TESTS]),
         "pisulorn": _start([*PYTEST, *_workers(2), PISULORN_TESTS, "-k", PISULORN_SELECT]),
@@ -131,8 +131,8 @@ def test_the_kernel_tests_pass_on_the_cpu_build_between_guard_pages(runs):
     _passed(runs["kernel tests"])
 
 
-def test_products_in_tiles_over_several_rounds_on_a_machine_made_small(runs):
-    _passed(runs["one unit, tiles"], 3)
+def test_products_in_tiles_and_pairs_of_pages_on_a_machine_made_small(runs):
+    _passed(runs["one unit, tiles"], 12)
 
 
 def test_the_sampler_tests_pass_on_the_cpu_build_between_guard_pages(runs):

@@ -1487,3 +1487,59 @@ def test_product_in_tiles_over_rounds(ops, act):
         got = ops.gemm_tiles_bf16(x, w, tile, out_dtype, name)
         error = (got.float() - want).abs().amax(1) / want.abs().amax()
         assert float(error.max()) < (1e-5 if act == "float32" else 8e-3), (tile, int(error.argmax()))
+
+
+PAIR_FORMS = {"plain": {}, "window": {"window": 40}, "a page's window": {"window": 32}, "kept": {"window": 45, "keep_first": 37}, "kept pair": {"window": 70, "keep_first": 64},
+              "chunk": {"chunk": 96}, "cap": {"softcap": 3.0}, "slopes": {"slopes": 0.05}, "sinks": {"sinks": True}}
+
+
+@pytest.mark.parametrize("form", list(PAIR_FORMS))
+@pytest.mark.parametrize("heads, kv_heads, dh", [(16, 1, 128), (20, 1, 128), (5, 5, 64), (17, 1, 64), (6, 2, 32)])
+def test_prompt_attention_in_pairs_of_pages(ops, heads, kv_heads, dh, form):
+    """Two pages a turn against one: whole prompts and pieces, sequences that end in either page of a pair, windows and kept tokens whose first
+    and last pages are of either number, pages that nobody sees not mapped; one tile of columns and two.  The two are up to a rounding of the weights
+    (2^-9 of each) and of the result away from one another.  And the same bits alone, in one step with others and in pieces."""
+    rng = np.random.default_rng(heads + dh)
+    lens, new = [70, 300, 257, 1, 45, 131, 64], [70, 5, 1, 1, 45, 99, 64]
+    kw = dict(PAIR_FORMS[form])
+    reach = kw.get("window"), kw.get("chunk"), kw.get("keep_first", 0)
+    held = [-(-n // 32) for n in lens]
+    kp, vp = ((torch.randn(shape, device=DEV) * 0.8).to(torch.bfloat16) for shape in ((sum(held), kv_heads, 32, dh), (sum(held), kv_heads, dh, 32)))
+    if EMULATED:
+        kp, vp = (guarded(x) for x in (kp, vp))
+    order = rng.permutation(sum(held))
+    table, at = np.full((len(lens), max(held)), -1, np.int32), 0
+    for b, n in enumerate(held):
+        first = lens[b] - new[b]
+        first = first - first % reach[1] if reach[1] else max(0, first - reach[0] + 1) if reach[0] else 0
+        for p in range(n):
+            if p >= first // 32 or p * 32 < reach[2]:
+                table[b, p] = order[at + p]
+        at += n
+    if "slopes" in kw:
+        kw["slopes"] = t(np.linspace(0.01, kw["slopes"], heads))
+    if "sinks" in kw:
+        kw["sinks"] = t(rng.normal(size=heads))
+    window, cap = kw.pop("window", None), kw.pop("softcap", None)
+    qkv = (torch.randn((sum(new), heads * dh), device=DEV) * 0.8).to(torch.bfloat16)
+    pos = [p for b, n in enumerate(new) for p in range(lens[b] - n, lens[b])]
+
+    def run(first, seqs, paired):                            # sequences `seqs`, their tokens from `first` of them on
+        rows = [i for b in seqs for i in range(sum(new[:b]) + min(first, new[b] - 1), sum(new[:b + 1]))]
+        counts = [new[b] - min(first, new[b] - 1) for b in seqs]
+        index = torch.tensor(rows, device=qkv.device)
+        q = guarded(qkv[index].contiguous()) if EMULATED else qkv[index].contiguous()
+        return rows, f64(ops.attention_prefill_bf16(q, kp, vp, t(np.concatenate([[0], np.cumsum(counts)]), torch.int32),
+                                                    t([pos[i] for i in rows], torch.int32), t(table[seqs], torch.int32), len(seqs), max(counts), heads,
+                                                    kv_heads, dh, window, dh ** -0.5, cap, new_counts=counts, paired=paired, **kw))
+    every = list(range(len(lens)))
+    _, want = run(0, every, False)
+    _, got = run(0, every, True)
+    scale = np.abs(want).max()
+    assert np.isfinite(got).all() and np.abs(got - want).max() <= 2.0 ** -8 * scale, np.abs(got - want).max() / scale
+    for b in every:
+        rows, alone = run(0, [b], True)
+        assert np.array_equal(alone, got[rows])
+    for first in (1, 33, 64):
+        rows, pieces = run(first, every, True)
+        assert np.array_equal(pieces, got[rows])
