@@ -272,7 +272,7 @@ int ri_attention_decode_fused_bf16(void* out, float* workspace, const void* qkv,
                                    int window, float scale, int tiled_out, void* stream);
 
 // out[M, N] (float32) = x[M, K] (float32) . w[N, K]^T, w float32 or bfloat16; no input is rounded, the sums are float32.
-int ri_gemm_f32(float* out, const float* x, const void* w, int w_dtype, int m, int n, int k, void* stream);
+int ri_gemm_f32(float* out, const float* x, const void* w, int w_dtype, int m, int n, int k, int tile, void* stream);
 
 // out[M, N] (out_dtype) = x[M, K] . w[N, K]^T for bfloat16 x and w, float32 accumulation, M <= 8.
 // swiglu != 0: w is [2 * N, K] = gate rows then up rows and out[m, n] = silu(gate) * up.

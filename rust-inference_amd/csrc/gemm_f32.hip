@@ -19,7 +19,9 @@
 // output one sum over k = 0..K-1.
 #include "api.h"
 #include "common.h"
+#include "matrix_async.h"
 
+#include <type_traits>
 
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 f32_bf16x8;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32_floatx4;
@@ -201,6 +203,173 @@ static void launch_tiles(float* out, const float* x, const bf16_t* w, int m, int
     else gemm_f32_tile_kernel<MT, NT, WM, WN, DEEP, false><<<grid, 64 * WM * WN, 0, s>>>(out, x, w, m, n, k, m_tiles, n_tiles);
 }
 
+// ---- large tiles: x as it is into LDS, split where its fragments are read
+
+// Two floats' share of the split above, in steps of three or four instructions that fit between products.
+struct SplitPair {
+    float t0, t1;
+    __device__ __forceinline__ void step(int u, float& v0, float& v1, uint32_t& a, uint32_t& b, uint32_t& c) {
+        if (u == 0 || u == 2) {
+            (u == 0 ? a : b) = __builtin_amdgcn_perm(__float_as_uint(v1), __float_as_uint(v0), 0x07060302u);
+            t0 = __uint_as_float(__float_as_uint(v0) & 0xFFFF0000u);
+            t1 = __uint_as_float(__float_as_uint(v1) & 0xFFFF0000u);
+        } else if (u == 1) {
+            v0 = (v0 - t0) * F32_LOWER;
+            v1 = (v1 - t1) * F32_LOWER;
+        } else {
+            v0 -= t0;
+            v1 -= t1;
+            c = __builtin_amdgcn_perm(__float_as_uint(v1), __float_as_uint(v0), 0x07060302u);
+        }
+    }
+};
+
+// Tiles of 16 MT WAVES rows of x and 16 NT of w: a wavefront has 16 MT rows and all columns, so that no row is split twice and none of its parts
+// written.  K in stages of 64 through SLOTS buffers, filled by copies that do not pass through registers and go out one or two stages ahead.
+// The split, the reads and the copies stand between the products, three or four instructions each.  What bounds a large tile is then the matrix
+// cores at the clock that they leave (128 x 160: 1,920 cycles of products a stage, 1.19 us; 759 rows, 6,144 x 1,024: 48 -> 33 us; 128 x 128,
+// 4,096 x 1,024: 30 -> 23), the smallest the instructions it issues, half of them the split (64 x 64: 0.46 us a stage; 1,024 x 3,072: 31 -> 27).
+// The order of every sum is the one of the tiles above, to the bit.
+template <int MT, int NT, int WAVES, int SLOTS>
+__global__ void __launch_bounds__(64 * WAVES, WAVES / 4)
+gemm_f32_copied_kernel(float* __restrict__ out, const float* __restrict__ x, const bf16_t* __restrict__ w, int M, int N, int K,
+                       int m_tiles, int n_tiles) {
+    constexpr int BM = 16 * MT * WAVES, BN = 16 * NT, XC = 4 * MT, WC = 2 * NT / WAVES, FR = XC + WC, STAGE = BM * 16 + BN * 8;
+    constexpr int EACH = 3 * MT, P = EACH * NT, LAG = SLOTS > 4 ? 2 : 1, MEET = EACH * (3 - LAG) - 1, SPLITS = 16 * MT, READ0 = P <= 24 ? 0 : P / 3,
+                  GAP = (P - 1 - READ0) / FR;
+    static_assert(2 * NT % WAVES == 0 && GAP >= 1 && SLOTS > 2 && (SLOTS - 2) * FR <= 63, "a stage's copies go out within half a stage");
+    __shared__ uint4 lds[SLOTS * STAGE];
+    const int group = blockIdx.x / (8 * m_tiles), within = blockIdx.x % (8 * m_tiles);
+    const int nt = group * 8 + within % 8, m0 = within / 8 * BM, n0 = nt * BN;
+    if (nt >= n_tiles) return;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r = lane & 15, g = lane >> 4;
+    const int stages = K / 64;
+
+    // A copy of a wavefront fills four rows of x or eight of w.  Rows past the edge are the last row again.
+    uint32_t xo[XC], wo[WC];
+#pragma unroll
+    for (int j = 0; j < XC; ++j) {
+        const int row = 4 * j + (lane >> 4);
+        xo[j] = (uint32_t)min(wave * 16 * MT + row, M - 1 - m0) * (uint32_t)K * 4u + ((lane & 15) ^ (row & 15)) * 16;
+    }
+#pragma unroll
+    for (int j = 0; j < WC; ++j) {
+        const int row = lane >> 3;
+        wo[j] = (uint32_t)min(wave * 8 * WC + 8 * j + row, N - 1 - n0) * (uint32_t)K * 2u + ((lane & 7) ^ row) * 16;
+    }
+    const float* xa = x + (size_t)m0 * K;
+    const bf16_t* wa = w + (size_t)n0 * K;
+    const ma_lds_t x_at = ma_lds(lds + wave * 16 * MT * 16), w_at = ma_lds(lds + BM * 16 + wave * 64 * WC);
+    auto copy = [&](int e, int buf, size_t k) {
+        if (e < WC) ma_copy16(w_at + buf * STAGE * 16 + e * 1024, wo[e], wa + k);
+        else ma_copy16(x_at + buf * STAGE * 16 + (e - WC) * 1024, xo[e - WC], xa + k);
+    };
+#pragma unroll
+    for (int s = 0; s < SLOTS - LAG; ++s)
+#pragma unroll
+        for (int e = 0; e < FR; ++e) copy(e, s, (size_t)min(s, stages - 1) * 64);
+
+    ma_floatx4 acc[MT][NT][3];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int q = 0; q < 3; ++q) acc[i][j][q] = ma_floatx4{0.f, 0.f, 0.f, 0.f};
+    const float4* xr = reinterpret_cast<const float4*>(lds) + (wave * 16 * MT + r) * 16;
+    const uint4* wr = lds + BM * 16 + r * 8;
+    float raw[2][MT][8];
+    uint32_t xf[2][MT][3][4];
+    ma_bf16x8 wf[NT];
+    SplitPair pair;
+    auto read_x = [&](int to, int buf) {
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const float4 v = xr[buf * STAGE + i * 256 + ((to * 8 + 2 * g + h) ^ r)];
+                raw[to][i][4 * h] = v.x, raw[to][i][4 * h + 1] = v.y, raw[to][i][4 * h + 2] = v.z, raw[to][i][4 * h + 3] = v.w;
+            }
+    };
+    auto read_w = [&](int j, int to, int buf) { wf[j] = *reinterpret_cast<const ma_bf16x8*>(wr + buf * STAGE + j * 128 + ((to * 4 + g) ^ (r & 7))); };
+    auto split = [&](int t, int to) {
+        const int i = t / 16, at = t % 16 / 4;
+        pair.step(t % 4, raw[to][i][2 * at], raw[to][i][2 * at + 1], xf[to][i][0][at], xf[to][i][1][at], xf[to][i][2][at]);
+    };
+    ma_wait_copies<(SLOTS - LAG - 1) * FR>();
+    ma_meet();
+    read_x(0, 0);
+    read_x(1, 0);
+#pragma unroll
+    for (int j = 0; j < NT; ++j) read_w(j, 0, 0);
+#pragma unroll
+    for (int t = 0; t < SPLITS; ++t) split(t, 0);
+
+    // Products of half a stage; under them the next half's x is split in steps, that of the half after it read (a wavefront's own copies), and
+    // the next half's fragments of w, each where this half's has been used.
+    auto half = [&](auto which, int buf, int next, int free, size_t k) {
+        constexpr int H = decltype(which)::value, READ = H ? 0 : READ0;
+        ma_wait_written();
+#pragma unroll
+        for (int p = 0; p < P; ++p) {
+            const int j = p / EACH, i = p % EACH / 3, q = 2 - p % 3;
+            ma_product(acc[i][j][q], wf[j], *reinterpret_cast<const ma_bf16x8*>(xf[H][i][q]));
+            if (p == READ) {
+                if (!H) ma_wait_copies<(SLOTS - LAG - 2) * FR>();
+                read_x(H, next);
+            }
+            if (H && p == MEET) {
+                if (LAG == 1) ma_wait_lds();
+                ma_meet();
+#pragma unroll
+                for (int before = 0; before < j; ++before) read_w(before, 0, next);
+            }
+            if (p % EACH == EACH - 1 && (!H || p >= MEET)) read_w(j, 1 - H, H ? next : buf);
+            if (!H && p > READ && (p - READ) % GAP == 0 && (p - READ) / GAP <= FR) copy((p - READ) / GAP - 1, free, k);
+#pragma unroll
+            for (int c = 0; c < (SPLITS + P - 2) / (P - 1); ++c) {
+                const int t = p * SPLITS / (P - 1) + c;
+                if (p < P - 1 && t < (p + 1) * SPLITS / (P - 1)) split(t, 1 - H);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    int buf = 0, free = SLOTS - LAG;
+#pragma nounroll
+    for (int s = 0; s < stages; ++s) {
+        const int next = buf + 1 == SLOTS ? 0 : buf + 1;
+        half(std::integral_constant<int, 0>(), buf, next, free, (size_t)min(s - LAG + SLOTS, stages - 1) * 64);
+        half(std::integral_constant<int, 1>(), buf, next, free, 0);
+        buf = next;
+        free = free + 1 == SLOTS ? 0 : free + 1;
+    }
+    ma_wait_products();
+    bool bad = false;
+    const int m = m0 + wave * 16 * MT + r, n = n0 + 4 * g;
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+            float sum[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                sum[e] = ma_taken(acc[i][j][0][e]) + (ma_taken(acc[i][j][1][e]) + ma_taken(acc[i][j][2][e])) * (1.f / F32_LOWER);
+            if (m + 16 * i >= M || n + 16 * j >= N) continue;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) bad |= !(fabsf(sum[e]) < INFINITY);
+            *reinterpret_cast<float4*>(out + (size_t)(m + 16 * i) * N + n + 16 * j) = make_float4(sum[0], sum[1], sum[2], sum[3]);
+        }
+    ma_wait_copies<0>();
+    if (bad) chain_again<MT, NT>(out, x, w, m, n, M, N, K);
+}
+
+template <int MT, int NT, int WAVES, int SLOTS>
+static void launch_copied(float* out, const float* x, const bf16_t* w, int m, int n, int k, hipStream_t s) {
+    constexpr int BM = 16 * MT * WAVES;
+    const int m_tiles = (m + BM - 1) / BM, n_tiles = (n + 16 * NT - 1) / (16 * NT);
+    gemm_f32_copied_kernel<MT, NT, WAVES, SLOTS><<<(n_tiles + 7) / 8 * 8 * m_tiles, 64 * WAVES, 0, s>>>(out, x, w, m, n, k, m_tiles, n_tiles);
+}
+
 #define GT_M 64
 #define GT_N 64
 #define GT_K 16
@@ -243,7 +412,7 @@ gemm_f32_kernel(float* __restrict__ out, const float* __restrict__ x, const TW* 
         }
 }
 
-extern "C" int ri_gemm_f32(float* out, const float* x, const void* w, int w_dtype, int m, int n, int k, void* stream) {
+extern "C" int ri_gemm_f32(float* out, const float* x, const void* w, int w_dtype, int m, int n, int k, int tile, void* stream) {
     RI_REQUIRE(m > 0 && n > 0 && k > 0, "gemm_f32: m %d, n %d, k %d", m, n, k);
     RI_REQUIRE(w_dtype == RI_F32 || w_dtype == RI_BF16, "gemm_f32: weight dtype %d", w_dtype);
     dim3 grid((n + GT_N - 1) / GT_N, (m + GT_M - 1) / GT_M);
@@ -255,20 +424,47 @@ extern "C" int ri_gemm_f32(float* out, const float* x, const void* w, int w_dtyp
     else if (!aligned)
         gemm_f32_kernel<bf16_t><<<grid, 256, 0, s>>>(out, x, (const bf16_t*)w, m, n, k);
     else {
-        // The order of a row's sums is the same in every tile.  64 x 128 from three quarters of the machine on (one workgroup a compute unit), else
-        // 32 x 64 as soon as 32 x 32 would need a second round.  us for 32 x 32 / 32 x 64 / 64 x 128 (rows; columns x K): 759; 6,144 x
-        // 1,024 60 / 49 / 49, 4,096 x 1,024 43 / 38 / 32, 1,024 x 3,072 33 / 35 / 39; 1,200; 4,096 x 1,024 65 / 51 / 47, 6,144 x 1,024 102 / 78 / 62;
-        // 400; 4,096 x 1,024 27 / 23 / 20, 6,144 x 1,024 37 / 29 / 32; 200; 4,096 x 1,024 17 / 14 / 17; 2,400; 6,144 x 1,024 252 / 151 / 124; 1,000;
-        // 12,288 x 4,096 64 x 128 325, 32 x 64 455; 33; 1,024 x 3,072 20 / 22 / 38, 4,096 x 1,024 8.8 / 9.6 / 16 (the vector units' form: 759; 1,024 x 3,072 363).  (128 x 192 has no registers
-        // for three sums a result: with a stage less under way 48 and 46 us at 759; 6,144 and 1,200; 4,096, 136 at 2,400; 6,144.)
+        // The order of a row's sums is the same in every tile.  Without copies (K off a multiple of 64) 64 x 128 from three quarters of the
+        // machine on (one workgroup a compute unit), else 32 x 64 as soon as 32 x 32 would need a second round.  us for 32 x 32 / 32 x 64 /
+        // 64 x 128 (rows; columns x K): 759; 6,144 x 1,024 72 / 47 / 49, 4,096 x 1,024 47 / 31 / 30, 1,024 x 3,072 36 / 31 / 46; 1,200; 6,144 x
+        // 1,024 115 / 77 / 63; 400; 4,096 x 1,024 27 / 21 / 18; 200; 4,096 x 1,024 17 / 12.5 / 17; 1,000; 12,288 x 4,096 844 / 453 / 320; 33;
+        // 4,096 x 1,024 8.5 / 9.4 / 16 (the vector units' form: 759; 1,024 x 3,072 363).
         // Up to 32 rows half of a tile of 64 would be padding: 151,936 x 1,024 at one row 77 / 57 / 75.
         const auto tiles = [&](int rows, int cols) { return (long)((m + rows - 1) / rows) * ((n + cols - 1) / cols); };
         const bf16_t* wb = (const bf16_t*)w;
         RI_REQUIRE(tiles(32, 32) + 8 * ((m + 31) / 32) < (1L << 31), "gemm_f32: %d x %d exceed one launch", m, n);
+        const bool copied = k % 64 == 0 && n % 4 == 0 && k < (1 << 22);
+        RI_REQUIRE(tile >= -1 && tile <= (copied ? 6 : 2), "gemm_f32: tile %d for %d columns, K %d", tile, n, k);
         const long units = ri_compute_units();
-        if (m > 32 && 4 * tiles(64, 128) >= 3 * units) launch_tiles<2, 2, 2, 4, 2>(out, x, wb, m, n, k, s);
-        else if (tiles(32, 32) > units) launch_tiles<1, 2, 2, 2, 2>(out, x, wb, m, n, k, s);
-        else launch_tiles<1, 1, 2, 2, 4>(out, x, wb, m, n, k, s);
+        if (tile < 0) {
+            tile = m > 32 && 4 * tiles(64, 128) >= 3 * units ? 0 : tiles(32, 32) > units ? 1 : 2;
+            if (copied && m > 32) {
+                // With copies what a tile takes is its rounds times (a beginning and an end + its stages), in us; the smaller tiles above share
+                // a compute unit instead.  Measured, in the order 128 x 160 / 128 x 128 / 64 x 128 / 64 x 64 and the best of those above: 759; 6,144 x
+                // 1,024 33 / 43 / 42 / 51, 47; 759; 4,096 x 1,024 29 / 23 / 28 / 31, 30; 759; 1,024 x 3,072 63 / 49 / 34 / 27, 31; 1,200; 6,144 x
+                // 1,024 58 / 49 / 60 / 84, 62; 1,200; 1,024 x 3,072 63 / 48 / 34 / 51, 42; 400; 4,096 x 1,024 26 / 20 / 15 / 21, 18; 400; 1,024 x
+                // 3,072 63 / 48 / 33 / 26, 23; 100; 6,144 x 1,024 25 / 19 / 14 / 11.2, 13; 50; 6,144 x 1,024 25 / 18 / 13 / 10.5, 9.6; 1,000;
+                // 12,288 x 4,096 274 / 248 / 293 / 407, 312; 2,400; 6,144 x 1,024 91 / 100 / 119 / 153, 121.
+                static const struct { int rows, cols; double ends, stage; } form[4] = {{128, 160, 13, 1.19}, {128, 128, 9, 0.9}, {64, 128, 5, 0.61}, {64, 64, 4, 0.46}};
+                const double stages = k / 64, load = tiles(32, 64) / (double)units;
+                double best = tile == 2 ? 1.5 + 0.37 * stages : tile == 1 ? 2. + stages * (0.25 + 0.25 * (load > 0.8 ? load : 0.8)) : 1e30;
+                for (int i = 0; i < 4; ++i) {
+                    // (the eight L2 caches' columns are dealt out as the kernel does)
+                    const long own = (((n + form[i].cols - 1) / form[i].cols + 7) / 8) * (long)((m + form[i].rows - 1) / form[i].rows), room = units > 8 ? units / 8 : 1;
+                    const double takes = (own + room - 1) / room * (form[i].ends + form[i].stage * stages);
+                    if (takes < best) best = takes, tile = 3 + i;
+                }
+            }
+        }
+        switch (tile) {
+        case 0: launch_tiles<2, 2, 2, 4, 2>(out, x, wb, m, n, k, s); break;
+        case 1: launch_tiles<1, 2, 2, 2, 2>(out, x, wb, m, n, k, s); break;
+        case 2: launch_tiles<1, 1, 2, 2, 4>(out, x, wb, m, n, k, s); break;
+        case 3: launch_copied<2, 10, 4, 3>(out, x, wb, m, n, k, s); break;
+        case 4: launch_copied<1, 8, 8, 3>(out, x, wb, m, n, k, s); break;
+        case 5: launch_copied<1, 8, 4, 5>(out, x, wb, m, n, k, s); break;
+        case 6: launch_copied<1, 4, 4, 6>(out, x, wb, m, n, k, s); break;
+        }
     }
     RI_LAUNCH_CHECK("gemm_f32");
     return 0;

@@ -23,6 +23,7 @@ __device__ __forceinline__ float ma_taken(const float& a) { return a; }
 template <int N> __device__ __forceinline__ void ma_wait_copies() {}
 __device__ __forceinline__ void ma_wait_lds() {}
 __device__ __forceinline__ void ma_wait_products() {}
+__device__ __forceinline__ void ma_wait_written() {}
 __device__ __forceinline__ void ma_meet() { __syncthreads(); }
 #else
 typedef uint32_t ma_lds_t;                                    // an address within a workgroup's LDS
@@ -57,6 +58,8 @@ template <int N> __device__ __forceinline__ void ma_wait_copies() {
 __device__ __forceinline__ void ma_wait_lds() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 // Until the last product's sum may be read (more than the longest product takes).
 __device__ __forceinline__ void ma_wait_products() { asm volatile("s_nop 15\n\ts_nop 15" ::: "memory"); }
+// Until a product may read what the vector instruction before has written (the compiler does not know these products for what they are).
+__device__ __forceinline__ void ma_wait_written() { asm volatile("s_nop 3" ::: "memory"); }
 // The workgroup's wavefronts meet; what each has to have waited for before, it has waited for itself.
 __device__ __forceinline__ void ma_meet() {
     asm volatile("" ::: "memory");

@@ -72,7 +72,7 @@ _SIGNATURES = {
     "ri_attention_decode_fused_bf16": [c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_float,
                                        c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
                                        c_int, c_int, c_int, c_int, c_float, c_int, c_void_p],
-    "ri_gemm_f32": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p],
+    "ri_gemm_f32": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p],
     "ri_gemv_bf16": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p],
     "ri_sample": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_float, c_int, c_float, c_float,
                   c_void_p],
@@ -1412,13 +1412,14 @@ def attention_decode_fused_bf16(qkv, q_gain, k_gain, eps, inv_freq, k_pages, v_p
 
 
 # ---------------------------------------------------------------- products
-def gemm_f32(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """``x @ w.T`` with no input rounded and float32 sums; ``x`` float32 ``[M, K]``, ``w`` float32 or bfloat16 ``[N, K]``."""
+def gemm_f32(x: torch.Tensor, w: torch.Tensor, tile: int = -1) -> torch.Tensor:
+    """``x @ w.T`` with no input rounded and float32 sums; ``x`` float32 ``[M, K]``, ``w`` float32 or bfloat16 ``[N, K]``.
+    ``tile``: for bfloat16 weights one of the kernel's tiles (the same bits of each) instead of the rule's choice."""
     m, k = x.shape
     n = w.shape[0]
     out = torch.empty((m, n), dtype=torch.float32, device=x.device)
     _call("ri_gemm_f32", _dev(out, "out"), _dev(x, "x", torch.float32), _dev(w, "w", None, (n, k)), code(w.dtype),
-          m, n, k, _stream())
+          m, n, k, tile, _stream())
     return out
 
 

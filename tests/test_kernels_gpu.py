@@ -967,6 +967,17 @@ def test_gemm_f32_tiles_of_a_full_machine(ops, m, n, k):
     assert np.array_equal(got[m - 30:], f64(ops.gemm_f32(x[m - 30:].contiguous(), w))), "a row's sums depend on the other rows"
 
 
+@pytest.mark.parametrize("tile", range(3, 7))
+@pytest.mark.parametrize("m,n,k", [(1, 8, 64), (130, 164, 128), (67, 60, 192), (128, 160, 448)])
+def test_gemm_f32_in_tiles_copied_as_they_are(ops, m, n, k, tile):
+    """Edges of the tiles whose x is split out of LDS, fewer stages of 64 k than buffers and more: the bits of the smallest tile, also
+    where an infinity leaves the matrix cores' sums without a value.  (That tile against 64 bits: above.)"""
+    rng = np.random.default_rng(m + n + k)
+    x, w = t(rng.normal(size=(m, k)) * 10.0 ** rng.uniform(-6, 6, size=(m, k))), t(rng.normal(size=(n, k)), torch.bfloat16)
+    x[m // 2, k - 1] = float("inf")
+    assert np.array_equal(f64(ops.gemm_f32(x, w, tile)), f64(ops.gemm_f32(x, w, 2)), equal_nan=True)
+
+
 @pytest.mark.parametrize("m, n", [(5, 48), (70, 72)])
 def test_gemm_f32_where_the_first_parts_cancel(ops, m, n):
     """Pairs of k with opposite weights and x that agree in their first eight bits: what is left are the lower parts' products, whose sum is
