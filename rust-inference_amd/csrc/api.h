@@ -353,10 +353,10 @@ int ri_gemm_tiles_bf16(void* out, int out_dtype, int ldo, const void* x, int ldx
 // len_after[s] keys.  ri_latent_prompt: causal attention of `tokens` queries (heads of dim + rot elements in rows of q_stride) over keys
 // [heads * dim] (rows of key_stride) beside turned [row] (rows of turned_stride, all heads') and values [heads * vdim] (rows of value_stride, a column a
 // key), rows as the gather leaves them; sinks [heads] join the denominators, gates (rows of q_stride, one a head) multiply by their
-// sigmoid, either may be NULL; out [tokens][heads * vdim].  ri_latent_prompt_fits: the sizes it takes.
+// sigmoid, either may be NULL; out [tokens][heads * vdim].  ri_latent_prompt_fits: the sizes the two take, latents of `rank` elements.
 int ri_latent_gather(void* rows, const void* k_pages, const int32_t* len_after, const int32_t* page_table, int table_width, int seqs,
                      int pages, int key_dim, int page_size, void* stream);
-int ri_latent_prompt_fits(int dim, int rot, int vdim);
+int ri_latent_prompt_fits(int dim, int rot, int vdim, int rank);
 int ri_latent_prompt(void* out, const void* q, int q_stride, const void* keys, int key_stride, const void* turned, int turned_stride,
                      const void* values, long value_stride, const void* gates, const float* sinks, const int32_t* cu_seqlens, const int32_t* tok_pos,
                      const int32_t* len_after, int seqs, int tokens, int heads, int dim, int rot, int vdim, float scale, void* stream);

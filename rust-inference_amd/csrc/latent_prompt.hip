@@ -228,15 +228,20 @@ latent_prompt_kernel(const LatentPrompt a) {
     }
 }
 
-extern "C" int ri_latent_prompt_fits(int dim, int rot, int vdim) {
+static bool latent_prompt_heads(int dim, int rot, int vdim) {
     return (dim == 128 && rot == 64 && vdim == 128) || (dim == 64 && rot == 64 && vdim == 64);
+}
+
+// (a latent's rows are gathered, and the turned part behind `rank` elements is copied, sixteen bytes at a time)
+extern "C" int ri_latent_prompt_fits(int dim, int rot, int vdim, int rank) {
+    return latent_prompt_heads(dim, rot, vdim) && rank > 0 && rank % 8 == 0;
 }
 
 extern "C" int ri_latent_prompt(void* out, const void* q, int q_stride, const void* keys, int key_stride, const void* turned, int turned_stride,
                                 const void* values, long value_stride, const void* gates, const float* sinks, const int32_t* cu_seqlens,
                                 const int32_t* tok_pos, const int32_t* len_after, int seqs, int tokens, int heads, int dim, int rot, int vdim,
                                 float scale, void* stream) {
-    RI_REQUIRE(ri_latent_prompt_fits(dim, rot, vdim), "latent_prompt: heads of %d + %d and %d", dim, rot, vdim);
+    RI_REQUIRE(latent_prompt_heads(dim, rot, vdim), "latent_prompt: heads of %d + %d and %d", dim, rot, vdim);
     RI_REQUIRE(heads > 0 && seqs > 0 && tokens >= seqs && scale > 0.f, "latent_prompt: %d heads, %d tokens of %d sequences, scale %g", heads,
                tokens, seqs, (double)scale);
     RI_REQUIRE(q_stride >= heads * (dim + rot) && (q_stride | key_stride | turned_stride) % 8 == 0 && key_stride >= heads * dim && key_stride < (1 << 24) && turned_stride >= rot && value_stride % 8 == 0 && value_stride < (1 << 23) && turned_stride < (1 << 24),

@@ -84,7 +84,7 @@ _SIGNATURES = {
     "ri_gemm_wide_packed_bf16": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int,
                                  c_int, c_void_p],
     "ri_latent_gather": [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p],
-    "ri_latent_prompt_fits": [c_int, c_int, c_int],
+    "ri_latent_prompt_fits": [c_int, c_int, c_int, c_int],
     "ri_latent_prompt": [c_void_p, c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_void_p, ctypes.c_long, c_void_p, c_void_p, c_void_p,
                          c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_void_p],
     "ri_gemm_tiles_bf16": [c_void_p, c_int, c_int, c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p,
@@ -1854,8 +1854,9 @@ def latent_attention_mfma(q, k_pages, v_pages, tok_pos, tok_seq, page_table, hea
     return out
 
 
-def latent_prompt_fits(dtype, dim: int, rot: int, vdim: int, page_size: int) -> bool:
-    return dtype == torch.bfloat16 and page_size == 32 and bool(_get("ri_latent_prompt_fits")(dim, rot, vdim))
+def latent_prompt_fits(dtype, dim: int, rot: int, vdim: int, rank: int, page_size: int) -> bool:
+    """Whether ``latent_gather`` and ``latent_prompt`` take heads of ``dim + rot`` and ``vdim`` over latents of ``rank`` elements."""
+    return dtype == torch.bfloat16 and page_size == 32 and bool(_get("ri_latent_prompt_fits")(dim, rot, vdim, rank))
 
 
 def latent_gather(k_pages, len_after, page_table, pages: int) -> torch.Tensor:

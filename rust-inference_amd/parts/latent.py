@@ -70,7 +70,7 @@ class LatentAttention(Mixer):
         self.w_uk = rt.place_matrix(weights[n["uk"]]).view(self.heads, self.dim, self.rank).contiguous() if self.dim else None
         self.w_uv = rt.place_matrix(weights[n["uv"]]).view(self.heads, self.vdim, self.rank).transpose(1, 2).contiguous()
         self.w_uv_rows = None                                # [heads * vdim, rank], for the prompts' values
-        if self.dim and ops.latent_prompt_fits(rt.dtype, self.dim, self.rot, self.vdim, 32) and not rt.invariant:
+        if self.dim and ops.latent_prompt_fits(rt.dtype, self.dim, self.rot, self.vdim, self.rank, 32) and not rt.invariant:
             self.w_uv_rows = rt.place_matrix(weights[n["uv"]])
         self.sink = rt.place_gain(weights[n["sink"]]) if self.sinks else None
         self.w_o = rt.pack(rt.place_matrix(weights[n["o"]]), parts_ok=True)

@@ -59,6 +59,7 @@ ONE_UNIT = ("one_run or mfma_prefill_attention or two_tiles or (mfma_attention_w
 ONE_UNIT_ROWS = "share_a_compute_unit or gemm_f32_on or rows_of_queries"
 PYTEST = ["-m", "pytest", "-q", "-x", "-p", "no:cacheprovider"]
 KERNEL_TESTS, SMALL_MACHINE = os.path.join(HERE, "test_kernels_gpu.py"), os.path.join(HERE, "small_machine_kernels.py")
+ROUTE_TESTS = os.path.join(HERE, "test_prompt_routes_gpu.py")
 SAMPLER_TESTS = os.path.join(HERE, "test_sampling_gpu.py")
 ZIDEPEL_TESTS = os.path.join(HERE, "test_zidepel_kernels_gpu.py")
 PISULORN_TESTS = os.path.join(HERE, "test_pisulorn_kernels_gpu.py")
@@ -90,6 +91,7 @@ def runs():
         "one unit": _start([*PYTEST, *_workers(2), SMALL_MACHINE, KERNEL_TESTS, "-k", ONE_UNIT], {"RI_EMU_COMPUTE_UNITS": "1"}),
         "one unit, rows": _start([*PYTEST, *_workers(2), KERNEL_TESTS, "-k", ONE_UNIT_ROWS], {"RI_EMU_COMPUTE_UNITS": "1"}),
         "one unit, tiles": _start([*PYTEST, KERNEL_TESTS, "-k", "over_rounds or (in_pairs_of_pages and 16-1-128)"], {"RI_EMU_COMPUTE_UNITS": "1"}),
+        "routes": _start([*PYTEST, *_workers(2), ROUTE_TESTS]),
         "sampler": _start([*PYTEST, *_workers(2), SAMPLER_TESTS, "-k", SAMPLER_SELECT]),
         "zidepel": _start([*PYTEST, *_workers(2), ZIDEPEL_TESTS]),
         "pisulorn": _start([*PYTEST, *_workers(2), PISULORN_TESTS, "-k", PISULORN_SELECT]),
@@ -133,6 +135,11 @@ def test_the_kernel_tests_pass_on_the_cpu_build_between_guard_pages(runs):
 
 def test_products_in_tiles_and_pairs_of_pages_on_a_machine_made_small(runs):
     _passed(runs["one unit, tiles"], 12)
+
+
+def test_the_routes_of_prompts_pass_on_the_cpu_build(runs):
+    """tests/test_prompt_routes_gpu.py: what the parts choose for long prompts, against the plain functions."""
+    _passed(runs["routes"])
 
 
 def test_the_sampler_tests_pass_on_the_cpu_build_between_guard_pages(runs):

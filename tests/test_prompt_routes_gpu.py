@@ -1,0 +1,138 @@
+"""Which kernels a prompt's parts choose, and that what they choose agrees with the plain functions: parts alone, at sizes that
+reach the kernels of long prompts.
+
+Like tests/test_kernels_gpu.py these run without a GPU when the environment says RI_TEST_KERNELS=emulated
+(tests/test_kernels_emulated.py starts that run): the CPU build of the same sources."""
+import os
+
+import numpy as np
+import pytest
+import torch
+
+from helpers import rel_to_max
+from plain import dagezen_plain as P
+
+EMULATED = os.environ.get("RI_TEST_KERNELS") == "emulated"
+pytestmark = [] if EMULATED else pytest.mark.gpu
+DEV = "cpu" if EMULATED else "cuda:0"
+PAGE = 32
+
+
+@pytest.fixture(scope="module")
+def ops():
+    if EMULATED:
+        import emulated
+        return emulated.ops()
+    from rust_inference_amd.kernels import ops
+    return ops
+
+
+@pytest.fixture(scope="module")
+def rt(ops):
+    from rust_inference_amd.parts import Runtime
+    if not EMULATED:
+        return Runtime(DEV, torch.bfloat16)
+    made = Runtime.__new__(Runtime)                          # (a runtime refuses to be made for the CPU)
+    made.device, made.dtype, made.invariant, made._mm_out_dtype = torch.device(DEV), torch.bfloat16, False, None
+    return made
+
+
+def t(a, dtype=torch.float32):
+    return torch.tensor(np.asarray(a), dtype=dtype, device=DEV)
+
+
+def f64(x):
+    return x.detach().to("cpu", torch.float64).numpy()
+
+
+def calls_of(monkeypatch, ops, name):
+    """What is given to ``ops.<name>`` from now on, call by call."""
+    real, seen = getattr(ops, name), []
+
+    def recorded(*args, **kw):
+        seen.append((args, kw))
+        return real(*args, **kw)
+    monkeypatch.setattr(ops, name, recorded)
+    return seen
+
+
+def random_weights(part, rng, std=0.1):
+    return {name: torch.tensor(std * rng.normal(size=spec.shape) + (spec.kind == "gain")).to(torch.bfloat16)
+            for name, spec in part.tensors().items()}
+
+
+class Sequences:
+    """Sequences that take tokens step by step, their pages in shuffled order: a step's context and the store of one cache entry."""
+
+    def __init__(self, need, most, rng):
+        from rust_inference_amd.cache import KVView
+        held = -(-most // PAGE)
+        order = rng.permutation(held * 8)
+        self.table, self.done = order.reshape(8, held), [0] * 8
+        pages = (held * 8, need.kv_heads)
+        k, v = torch.zeros(pages + (PAGE, need.head_dim)), torch.zeros(pages + (need.value_dim, PAGE))
+        self.store = KVView(0, k.to(DEV, torch.bfloat16), v.to(DEV, torch.bfloat16), PAGE, None)
+
+    def step(self, counts):
+        """``counts[s]`` tokens of sequence ``s`` (0: none): the context, the page table, (sequence, first, last) of each."""
+        from rust_inference_amd.parts.context import StepContext
+        seqs = [s for s, n in enumerate(counts) if n]
+        new, starts = [counts[s] for s in seqs], [self.done[s] for s in seqs]
+        for s in seqs:
+            self.done[s] += counts[s]
+        i32 = lambda a: t(a, torch.int32)
+        pos = [p for n, at in zip(new, starts) for p in range(at, at + n)]
+        ctx = StepContext(T=sum(new), B=len(seqs), new_counts=new, slot_list=seqs, starts=starts, tokens=i32(np.zeros(sum(new))),
+                          tok_seq=i32(np.repeat(np.arange(len(seqs)), new)), tok_pos=i32(pos), slots=i32(seqs),
+                          cu_seqlens=i32(np.concatenate([[0], np.cumsum(new)])), len_after=i32([self.done[s] for s in seqs]),
+                          max_new=max(new), max_len=max(a + n for a, n in zip(starts, new)))
+        return ctx, i32(self.table[seqs]), [(s, a, a + n) for s, a, n in zip(seqs, starts, new)]
+
+
+# ---------------------------------------------------------------- latent attention
+LATENT_STEPS = [[37, 100, 3, 0, 64], [90, 1, 40, 33], [0, 130], [1, 1, 1, 1, 1]]
+
+
+@pytest.mark.parametrize("heads, dim, vdim, rank, extras, expanded", [
+    (8, 64, 64, 72, True, 3), (2, 128, 128, 64, False, 3),
+    (4, 64, 64, 100, True, 0),           # (rows of 164 elements: neither the rows side by side nor the turned part would be aligned)
+    (3, 64, 64, 72, True, 0)])           # (queries in rows of 523)
+def test_latent_attention_of_prompts(ops, rt, monkeypatch, heads, dim, vdim, rank, extras, expanded):
+    """Fresh prompts of unequal lengths, prompts that go on in the middle of a page and at its border beside a single token, a
+    sequence by itself, and single tokens: against 64 bits on the whole sequences, whether the heads' keys and values are made
+    first or the attention runs on the latents.  The bound is the one for parts in bfloat16: weights, latents and results of
+    eight bits."""
+    from rust_inference_amd.parts import PartSpec, build_part
+    rng = np.random.default_rng(heads + rank)
+    rot, hidden, scale, eps = 64, 96, 0.11, 1e-5
+    part = build_part("mixer", PartSpec("latent_attention", {
+        "hidden": hidden, "heads": heads, "dim": dim, "rot_dim": rot, "vdim": vdim, "kv_rank": rank, "scale": scale, "prefix": "a.",
+        "eps": eps, "sinks": extras, "gate": extras, "position": PartSpec("rotate_pairs", {"head_dim": rot, "dims": rot, "base": 1e4})}))
+    w = random_weights(part, rng)
+    part.bind(w, rt)
+    w64 = {name: f64(x) for name, x in w.items()}
+    if not extras:                                           # (the plain function has both: a gate of 1 and a sink of nothing)
+        w64["a.sink"], w64["a.g"] = np.full(heads, -np.inf), None
+    m = {"heads": heads, "dim": dim, "rot_dim": rot, "vdim": vdim, "kv_rank": rank, "scale": scale, "rot": {"dims": rot, "base": 1e4}}
+    seqs = Sequences(part.cache_need(), 240, rng)
+    x = {s: t(rng.normal(size=(240, hidden)), torch.bfloat16) for s in range(5)}
+    made = calls_of(monkeypatch, ops, "latent_prompt")
+    got = {s: [] for s in range(5)}
+    for counts in LATENT_STEPS:
+        ctx, table, own = seqs.step(counts)
+        out = part.forward(torch.cat([x[s][a:b] for s, a, b in own]), ctx, seqs.store, table)
+        rows = f64(ops.as_rows(out) if out.dim() == 2 else out.sum(0))
+        for s, a, b in own:
+            got[s].append(rows[:b - a])
+            rows = rows[b - a:]
+    assert len(made) == expanded
+    for s in range(5):
+        have = np.concatenate(got[s])
+        want = latent_mixer(f64(x[s][:len(have)]), w64, m, eps)
+        assert rel_to_max(have, want) < 2e-2, f"sequence {s}"
+
+
+def latent_mixer(h, w, m, eps):
+    if w["a.g"] is None:
+        w = dict(w, **{"a.g": np.zeros((m["heads"], h.shape[1])), "a.o": 2.0 * w["a.o"]})
+    return P.latent_mixer(h, w, "a.", m, eps, {})
