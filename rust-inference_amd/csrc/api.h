@@ -343,8 +343,10 @@ int ri_sum_parts(void* out, int out_dtype, const float* parts, int n_parts, int 
 // with float32 sums; out float32 or bfloat16.  act (on the sums; bfloat16 out): 0 none; 1 silu(gate) * up and 2 g sigmoid(1.702 g) (u + 1)
 // with g = min(gate + b_gate, limit), u = clamp(up + b_up, -limit, limit) (either bias may be NULL), both with w = [gate; up], 2 n rows;
 // 3 max(v, 0)^2.  k is a multiple of 64 from 192 on, n and the strides multiples of 8, the pointers of 16 bytes.  tile: rows of x by rows of w a
-// workgroup; 256 x 128 not with a gate.  The sums do not depend on it.
+// workgroup; 256 x 128 not with a gate.  The sums do not depend on it.  ri_gemm_tiles_bf16_fits: whether a product of this size is within
+// what the kernel can address (gated != 0: activations 1 and 2).
 enum { RI_TILE_256_256 = 0, RI_TILE_128_256 = 1, RI_TILE_256_128 = 2 };
+int ri_gemm_tiles_bf16_fits(int m, int n, int ldx, int ldw, int ldo, int gated);
 int ri_gemm_tiles_bf16(void* out, int out_dtype, int ldo, const void* x, int ldx, const void* w, int ldw, int m, int n, int k, int act,
                        const float* b_gate, const float* b_up, float limit, int tile, void* stream);
 

@@ -266,6 +266,11 @@ static void launch_tiles_form(int tile, const GtArgs& a, hipStream_t s) {
     launch_tiles_bf16<4, 8, ACT, TO>(a, s);
 }
 
+// (a tile's rows are reached by 32-bit offsets in bytes, those of up from those of its gate too)
+extern "C" int ri_gemm_tiles_bf16_fits(int m, int n, int ldx, int ldw, int ldo, int gated) {
+    return ldx < (1 << 22) && ldo < (1 << 22) && ((long)(gated ? n : 0) + 256) * ldw < (1L << 30) && (long)m * n < (1L << 46);
+}
+
 extern "C" int ri_gemm_tiles_bf16(void* out, int out_dtype, int ldo, const void* x, int ldx, const void* w, int ldw, int m, int n, int k,
                                   int act, const float* b_gate, const float* b_up, float limit, int tile, void* stream) {
     const bool gated = act == GT_SILU_GATE || act == GT_CLAMPED_GATE;
@@ -275,7 +280,7 @@ extern "C" int ri_gemm_tiles_bf16(void* out, int out_dtype, int ldo, const void*
     RI_REQUIRE(tile == RI_TILE_256_256 || tile == RI_TILE_128_256 || (tile == RI_TILE_256_128 && !gated), "gemm_tiles_bf16: tile %d", tile);
     RI_REQUIRE(ldx >= k && ldw >= k && ldo >= n && (ldx | ldw | ldo) % 8 == 0, "gemm_tiles_bf16: rows of %d, %d and %d", ldx, ldw, ldo);
     RI_REQUIRE(((uintptr_t)out | (uintptr_t)x | (uintptr_t)w) % 16 == 0, "gemm_tiles_bf16: an operand is off a multiple of 16 bytes");
-    RI_REQUIRE(ldx < (1 << 22) && ldo < (1 << 22) && ((long)(gated ? n : 0) + 256) * ldw < (1L << 30) && (long)m * n < (1L << 46),
+    RI_REQUIRE(ri_gemm_tiles_bf16_fits(m, n, ldx, ldw, ldo, gated),
                "gemm_tiles_bf16: %d rows of %d, %d rows of %d exceed one launch", m, ldx, n, ldw);
     const GtArgs a = {out, (const bf16_t*)x, (const bf16_t*)w, b_gate, b_up, limit, m, n, k, ldx, ldw, ldo, 0, 0, 0};
     hipStream_t s = (hipStream_t)stream;

@@ -87,6 +87,7 @@ _SIGNATURES = {
     "ri_latent_prompt_fits": [c_int, c_int, c_int, c_int],
     "ri_latent_prompt": [c_void_p, c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_void_p, ctypes.c_long, c_void_p, c_void_p, c_void_p,
                          c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_void_p],
+    "ri_gemm_tiles_bf16_fits": [c_int, c_int, c_int, c_int, c_int, c_int],
     "ri_gemm_tiles_bf16": [c_void_p, c_int, c_int, c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p,
                            c_float, c_int, c_void_p],
     "ri_gemm_wide_packed_bf16_plan": [c_int, c_int, c_int, c_void_p, c_void_p],
@@ -1614,6 +1615,11 @@ def gemm_wide_packed_bf16(x, wpacked: torch.Tensor, n: int, out_dtype=torch.bflo
 TILES = ((256, 256), (128, 256), (256, 128))     # rows of x by rows of w a workgroup of gemm_tiles_bf16
 TILES_MIN_K = 192
 TILES_ACTIVATIONS = {None: 0, "silu_gate": 1, "clamped_gate": 2, "relu2": 3}
+
+
+def gemm_tiles_fits(m: int, n: int, ldx: int, ldw: int, ldo: int, activation: str | None = None) -> bool:
+    """Whether ``gemm_tiles_bf16`` can address ``m`` rows (of ``ldx``) by ``n`` results (in rows of ``ldo``), the matrix in rows of ``ldw``."""
+    return bool(_get("ri_gemm_tiles_bf16_fits")(m, n, ldx, ldw, ldo, int(activation in ("silu_gate", "clamped_gate"))))
 
 
 def gemm_tiles_bf16(x: torch.Tensor, w: torch.Tensor, tile: int, out_dtype=torch.bfloat16, activation: str | None = None,

@@ -387,13 +387,14 @@ class Runtime:
 
     def rows_into(self, out, x, w: torch.Tensor) -> None:
         """``out <- x @ w.T``; rows of any of the three may be stretches of longer ones."""
-        tile = self._tile(x, w, out.dtype) if out.data_ptr() % 16 == 0 and out.stride(0) % 8 == 0 else None
+        tile = self._tile(x, w, out.dtype, ldo=out.stride(0)) if out.data_ptr() % 16 == 0 and out.stride(0) % 8 == 0 else None
         if tile is None:
             torch.mm(x, w.t(), out=out)
         else:
             ops.gemm_tiles_bf16(x, w, tile, out=out)
 
-    def _tile(self, x, w: torch.Tensor, out_dtype, activation=None) -> int | None:
+    def _tile(self, x, w: torch.Tensor, out_dtype, activation=None, ldo: int | None = None) -> int | None:
+        """The tile for ``x @ w.T`` as these operands lie (results in rows of ``ldo``, else side by side); None: the library's product."""
         if self.dtype != torch.bfloat16 or self.invariant or x.shape[0] < TILES_MIN_ROWS:
             return None
         tile = _tiles_plan(x.shape[0], w.shape[0], w.shape[1], out_dtype == torch.float32, activation)
@@ -401,7 +402,9 @@ class Runtime:
             return None
         if isinstance(x, torch.Tensor) and (x.stride(1) != 1 or x.stride(0) % 8 or x.stride(0) < x.shape[1] or x.data_ptr() % 16):
             return None                                          # the library's product takes any strides
-        return tile
+        n = w.shape[0] // 2 if activation in ("silu_gate", "clamped_gate") else w.shape[0]
+        ldx = x.stride(0) if isinstance(x, torch.Tensor) else x.shape[1]
+        return tile if ops.gemm_tiles_fits(x.shape[0], n, ldx, w.stride(0), ldo or n, activation) else None
 
     def _library_mm(self, x, w, out_dtype):
         # The reference hands every product to a vendor library (src/cuda/mod.rs:186-232);

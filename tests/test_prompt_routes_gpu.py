@@ -136,3 +136,24 @@ def latent_mixer(h, w, m, eps):
     if w["a.g"] is None:
         w = dict(w, **{"a.g": np.zeros((m["heads"], h.shape[1])), "a.o": 2.0 * w["a.o"]})
     return P.latent_mixer(h, w, "a.", m, eps, {})
+
+
+# ---------------------------------------------------------------- products in tiles
+def placeless(rows, columns, stride=None, dtype=torch.bfloat16):
+    """A matrix that is nowhere in memory, for rules that look at sizes alone."""
+    return torch.empty((rows, columns if stride is None else stride), dtype=dtype, device="meta")[:, :columns]
+
+
+def test_products_in_tiles_only_where_the_kernel_takes_them(ops, rt):
+    """Matrices and rows on both sides of what the kernel can address; what is beyond stays with the library's product."""
+    from rust_inference_amd.parts.runtime import Runtime
+    tile = lambda m, n, k, out=torch.bfloat16, act=None, x=None, w=None, ldo=None: Runtime._tile(
+        rt, placeless(m, k, x), placeless(n, k, w), out, act, **({} if ldo is None else {"ldo": ldo}))
+    for gate in ("silu_gate", "clamped_gate"):
+        assert tile(2048, 2 * 65536, 16384 - 64, act=gate) is not None          # (65,536 + 256 rows of w from a workgroup's first)
+        assert tile(2048, 2 * 65536, 16384, act=gate) is None
+        assert tile(2048, 2 * 65536, 8192, w=16384, act=gate) is None
+    assert tile(4096, 8192, 4096, torch.float32, x=(1 << 22) - 8) is not None and tile(4096, 8192, 4096, torch.float32, x=1 << 22) is None
+    assert tile(4096, 8192, 4096, torch.float32, w=(1 << 22) - 8) is not None and tile(4096, 8192, 4096, torch.float32, w=1 << 22) is None
+    assert tile(4096, (1 << 22) - 8, 4096, torch.float32) is not None and tile(4096, 1 << 22, 4096, torch.float32) is None
+    assert tile(4096, 8192, 4096, torch.float32, ldo=(1 << 22) - 8) is not None and tile(4096, 8192, 4096, torch.float32, ldo=1 << 22) is None
