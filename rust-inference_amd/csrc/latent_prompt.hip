@@ -244,7 +244,7 @@ extern "C" int ri_latent_prompt(void* out, const void* q, int q_stride, const vo
     RI_REQUIRE(latent_prompt_heads(dim, rot, vdim), "latent_prompt: heads of %d + %d and %d", dim, rot, vdim);
     RI_REQUIRE(heads > 0 && seqs > 0 && tokens >= seqs && scale > 0.f, "latent_prompt: %d heads, %d tokens of %d sequences, scale %g", heads,
                tokens, seqs, (double)scale);
-    RI_REQUIRE(q_stride >= heads * (dim + rot) && (q_stride | key_stride | turned_stride) % 8 == 0 && key_stride >= heads * dim && key_stride < (1 << 24) && turned_stride >= rot && value_stride % 8 == 0 && value_stride < (1 << 23) && turned_stride < (1 << 24),
+    RI_REQUIRE(q_stride >= heads * (dim + rot) && (q_stride | key_stride | turned_stride) % 8 == 0 && key_stride >= heads * dim && key_stride < (1 << 24) && turned_stride >= rot && value_stride % 8 == 0 && value_stride <= (1 << 23) && turned_stride < (1 << 24),
                "latent_prompt: rows of %d, %d, %d and %ld", q_stride, key_stride, turned_stride, value_stride);
     RI_REQUIRE(((uintptr_t)q | (uintptr_t)keys | (uintptr_t)turned | (uintptr_t)values | (uintptr_t)out) % 16 == 0,
                "latent_prompt: an operand is off a multiple of 16 bytes");

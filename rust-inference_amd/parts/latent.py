@@ -88,8 +88,7 @@ class LatentAttention(Mixer):
     def _expanded(self, proj, ctx, store, page_table, g_off):
         """A prompt's heads ``[T, heads * vdim]`` with the keys and values of all heads made once a cached token."""
         rt = self.rt
-        pages = sum(-(-(s + n) // 32) for s, n in zip(ctx.starts, ctx.new_counts))
-        rows = ops.latent_gather(store.k_pages, ctx.len_after, page_table, pages)
+        rows = ops.latent_gather(store.k_pages, ctx.len_after, page_table, self._pages(ctx))
         latents = rows[:, :self.rank]
         keys = torch.empty((rows.shape[0], self.heads * self.dim), dtype=rt.dtype, device=rows.device)
         values = torch.empty((self.heads * self.vdim, rows.shape[0]), dtype=rt.dtype, device=rows.device)
@@ -98,16 +97,23 @@ class LatentAttention(Mixer):
         return ops.latent_prompt(proj, self.heads, self.dim, self.rot, self.vdim, keys, rows, values, self.scale, self.sink,
                                  g_off if self.gate else None, ctx.cu_seqlens, ctx.tok_pos, ctx.len_after)
 
+    @staticmethod
+    def _pages(ctx) -> int:
+        """The pages that a step's sequences hold after it."""
+        return sum(-(-(s + n) // 32) for s, n in zip(ctx.starts, ctx.new_counts))
+
     # Keys and values of all heads from EXPAND_TOKENS new tokens on, EXPAND_EACH of them a sequence on average and EXPAND_KEYS cached
     # tokens for one new one at the most, up to EXPAND_BYTES of them.  (On the latents : so, us, 32 heads, 512 + 64: 128 tokens 65 : 29, eight
     # of 32 after 1,000 keys 282 : 200; a token's scores gain on the latents what thirty keys' products cost.)
-    EXPAND_TOKENS, EXPAND_EACH, EXPAND_KEYS, EXPAND_BYTES = 128, 32, 32, 2 << 30
+    EXPAND_TOKENS, EXPAND_EACH, EXPAND_KEYS, EXPAND_BYTES, EXPAND_RUNS = 128, 32, 32, 2 << 30, 65535
 
     def _expand_pays(self, ctx, proj, store) -> bool:
         if self.w_uv_rows is None or ctx.T < max(self.EXPAND_TOKENS, self.EXPAND_EACH * ctx.B) or store.page_size != 32 or proj.shape[1] % 8:
             return False
-        keys = sum(ctx.starts) + ctx.T
-        return keys <= self.EXPAND_KEYS * ctx.T and keys * self.heads * (self.dim + self.vdim) * 2 <= self.EXPAND_BYTES
+        # (the kernel's own limits: runs of tokens, which EXPAND_RUNS bounds, and value rows of 2^23, which EXPAND_BYTES does)
+        if sum(ctx.starts) + ctx.T > self.EXPAND_KEYS * ctx.T or (ctx.T - ctx.B) // 128 + ctx.B > self.EXPAND_RUNS:
+            return False
+        return self._pages(ctx) * 32 * self.heads * (self.dim + self.vdim) * 2 <= self.EXPAND_BYTES
 
     def cache_need(self):
         return KVNeed(1, self.rank + self.rot, None, self.rank)

@@ -157,3 +157,21 @@ def test_products_in_tiles_only_where_the_kernel_takes_them(ops, rt):
     assert tile(4096, 8192, 4096, torch.float32, w=(1 << 22) - 8) is not None and tile(4096, 8192, 4096, torch.float32, w=1 << 22) is None
     assert tile(4096, (1 << 22) - 8, 4096, torch.float32) is not None and tile(4096, 1 << 22, 4096, torch.float32) is None
     assert tile(4096, 8192, 4096, torch.float32, ldo=(1 << 22) - 8) is not None and tile(4096, 8192, 4096, torch.float32, ldo=1 << 22) is None
+
+
+def test_latent_prompts_only_where_the_kernel_takes_them(ops, rt):
+    """Steps on both sides of what one launch can hold: rows by their padded pages, runs of 128 tokens; beyond, the latents."""
+    from rust_inference_amd.parts import PartSpec, build_part
+    part = build_part("mixer", PartSpec("latent_attention", {"hidden": 64, "heads": 1, "dim": 64, "rot_dim": 64, "vdim": 64, "kv_rank": 64, "scale": 0.1,
+                                                             "prefix": "a.", "sinks": False, "gate": False}))
+    part.bind(random_weights(part, np.random.default_rng(0)), rt)
+
+    class Step:
+        def __init__(self, new, starts):
+            self.new_counts, self.starts, self.T, self.B = new, starts, sum(new), len(new)
+    pays = lambda new, starts: part._expand_pays(Step(new, starts), placeless(1, part.w_in.n), type("Store", (), {"page_size": PAGE}))
+    most = part.EXPAND_BYTES // (2 * (part.dim + part.vdim))          # rows that the keys and values of one head may have
+    assert pays([most // 2], [most // 2]) and not pays([most // 2], [most // 2 + 1])
+    assert pays([32] * 52758, [0] * 52758) and not pays([32] * 52759, [0] * 52759)           # 31 B / 128 + B of 65,535 and 65,536
+    part.EXPAND_BYTES >>= 7
+    assert pays([33] * (most >> 13), [0] * (most >> 13)) and not pays([33] * ((most >> 13) + 1), [0] * ((most >> 13) + 1))
