@@ -60,6 +60,7 @@ static int prefill_tiles(int head_dim, int group, int max_new, int seqs, int kv_
 // workgroups) 58 : 56, 1,792 (448) 48 : 49, 2,816 (704) 94 : 80; two of 1,500 (752) 64 : 69, 500 + 1,500 + 532 (632) 45 : 67, eight of 500 (1,024) 42 : 39, 8,192 of 64 heads
 // 1,380 : 1,081.  Heads of 32 and 64: one, 2,048 of 32 heads of 64 32.5 : 38, 6,000 204 : 221 (4,096 99 : 95); more only where a key head's queries need them.
 #define PAIRS_MIN_TOKENS 400
+#define PREFILL_MAX_LAUNCHES 65535
 static int pair_tiles(int head_dim, int group, int seqs, int kv_heads, int tokens) {
     const int of_wg = 4 * (32 / (group <= 32 ? group : 32));
     const long wgs = (tokens + (long)seqs * of_wg / 2) / of_wg * kv_heads;
@@ -67,7 +68,22 @@ static int pair_tiles(int head_dim, int group, int seqs, int kv_heads, int token
     return head_dim == 128 && wgs >= (seqs == 1 ? 2L : 3L) * ri_compute_units() ? 2 : 1;
 }
 
-// The column tiles a wavefront takes of a step (host code only).
+struct PrefillPlan { bool paired; int tiles, launches; };     // tiles of columns a wavefront, workgroups of the longest sequence's tokens a key head
+// pairs: 1 so, 0 not so, -1 where it pays and a launch holds it.
+static PrefillPlan prefill_plan(int head_dim, int group, int max_new, int seqs, int kv_heads, int tokens, int weighted, int pairs) {
+    const auto plan = [&](bool paired, int nt) { const int of_wg = 4 * (group < 16 * nt ? 16 * nt / group : 1); return PrefillPlan{paired, nt, (max_new + of_wg - 1) / of_wg}; };
+    const PrefillPlan two = plan(true, pair_tiles(head_dim, group, seqs, kv_heads, tokens));
+    if (pairs == 1 || (pairs == -1 && tokens >= (long)PAIRS_MIN_TOKENS * seqs && two.launches <= PREFILL_MAX_LAUNCHES)) return two;
+    return plan(false, prefill_tiles(head_dim, group, max_new, seqs, kv_heads, tokens, weighted));
+}
+
+// The tiles of columns a wavefront takes of a step that goes in pairs of pages, 0: a page a turn (host code only).
+extern "C" int ri_attention_prefill_pairs(int head_dim, int group, int max_new, int seqs, int kv_heads, int tokens, int weighted) {
+    const PrefillPlan plan = prefill_plan(head_dim, group, max_new, seqs, kv_heads, tokens, weighted, -1);
+    return plan.paired ? plan.tiles : 0;
+}
+
+// The column tiles a wavefront takes of a step with a page a turn (host code only).
 extern "C" int ri_attention_prefill_tiles(int head_dim, int group, int max_new, int seqs, int kv_heads, int tokens, int weighted) {
     return prefill_tiles(head_dim, group, max_new, seqs, kv_heads, tokens, weighted);
 }
@@ -88,16 +104,10 @@ extern "C" int ri_attention_prefill_kept_bf16(void* out, const void* qkv, int q_
     RI_REQUIRE(seqs > 0 && seqs <= 65535 && max_new > 0, "attention_prefill_bf16: seqs %d, max_new %d", seqs, max_new);
     RI_REQUIRE(pairs >= -1 && pairs <= 1, "attention_prefill_bf16: pairs %d", pairs);
     RI_REQUIRE(group <= (head_dim <= 64 ? 64 : 32), "attention_prefill_bf16: %d query heads per kv head (at most %d)", group, head_dim <= 64 ? 64 : 32);
-    const bool paired = pairs == -1 ? tokens >= (long)PAIRS_MIN_TOKENS * seqs : pairs == 1;
-    const int nt_tiles = paired ? pair_tiles(head_dim, group, seqs, kv_heads, tokens)
-                                : prefill_tiles(head_dim, group, max_new, seqs, kv_heads, tokens, weighted);
-    RI_REQUIRE(group <= 16 * nt_tiles, "attention_prefill_bf16: %d query heads per kv head (at most %d)", group,
-               16 * nt_tiles);
-    const int tile_tokens = (16 * nt_tiles) / group;
-    const int tiles = (max_new + 4 * tile_tokens - 1) / (4 * tile_tokens);
-    RI_REQUIRE(tiles <= 65535, "attention_prefill_bf16: %d tiles of tokens exceed one launch", tiles);
+    const PrefillPlan plan = prefill_plan(head_dim, group, max_new, seqs, kv_heads, tokens, weighted, pairs);
+    RI_REQUIRE(plan.launches <= PREFILL_MAX_LAUNCHES, "attention_prefill_bf16: %d tiles of tokens exceed one launch", plan.launches);
     int long_runs;
-    const dim3 grid = prefill_grid(kv_heads, seqs, tiles, 4 * tile_tokens, tokens, long_runs);
+    const dim3 grid = prefill_grid(kv_heads, seqs, plan.launches, 4 * (16 * plan.tiles / group), tokens, long_runs);
     const float scale_log2 = scale * 1.4426950408889634f;
     hipStream_t s = (hipStream_t)stream;
     const int form = slopes ? PREFILL_ANY : cap_pre != 0.f ? PREFILL_CAPPED : PREFILL_PLAIN;
@@ -106,7 +116,7 @@ extern "C" int ri_attention_prefill_kept_bf16(void* out, const void* qkv, int q_
         tok_pos, page_table, table_width, heads, kv_heads, reach, scale_log2, cap_pre, cap_post, slopes,         \
         1.f / scale, keep_first, sinks, seqs, long_runs
 #define RI_PREFILL_GO(DH, NT, FORM)                                                                              \
-    if (paired) attn_prefill_pairs_kernel<DH, NT, FORM><<<grid, 256, 0, s>>>(RI_PREFILL_ARGS);                   \
+    if (plan.paired) attn_prefill_pairs_kernel<DH, NT, FORM><<<grid, 256, 0, s>>>(RI_PREFILL_ARGS);                   \
     else attn_prefill_mfma_kernel<DH, NT, DH, false, FORM><<<grid, 256, 0, s>>>(RI_PREFILL_ARGS)
 #define RI_PREFILL_CASE(DH, NT)                                                                                  \
     case DH * 8 + NT:                                                                                            \
@@ -114,7 +124,7 @@ extern "C" int ri_attention_prefill_kept_bf16(void* out, const void* qkv, int q_
         else if (form == PREFILL_CAPPED) { RI_PREFILL_GO(DH, NT, PREFILL_CAPPED); }                              \
         else { RI_PREFILL_GO(DH, NT, PREFILL_ANY); }                                                             \
         break;
-    switch (head_dim * 8 + nt_tiles) {
+    switch (head_dim * 8 + plan.tiles) {
         RI_PREFILL_CASE(32, 4)
         RI_PREFILL_CASE(32, 2)
         RI_PREFILL_CASE(32, 1)

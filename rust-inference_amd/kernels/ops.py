@@ -111,6 +111,7 @@ _SIGNATURES = {
     "ri_attention_prefill_kept_bf16": [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int,
                                        c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_float, c_void_p, c_int,
                                        c_void_p, c_int, c_int, c_int, c_void_p],
+    "ri_attention_prefill_pairs": [c_int, c_int, c_int, c_int, c_int, c_int, c_int],
     "ri_attention_prefill_tiles": [c_int, c_int, c_int, c_int, c_int, c_int, c_int],
     "ri_attention_kept": [c_void_p, c_void_p, c_int, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int,
                           c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_float, c_void_p, c_int, c_void_p,
@@ -1252,6 +1253,13 @@ def attention_prefill_tiles(new_counts, heads: int, kv_heads: int, head_dim: int
     same bits)."""
     tokens, longest = sum(new_counts), max(new_counts)
     return _get("ri_attention_prefill_tiles")(head_dim, heads // kv_heads, longest, len(new_counts), kv_heads, tokens,
+                                              _weighted_length(new_counts, tokens, longest))
+
+
+def attention_prefill_pairs(new_counts, heads: int, kv_heads: int, head_dim: int) -> int:
+    """The same for a step that ``attention_prefill_bf16`` takes in pairs of pages where ``paired`` is None; 0: a page a turn."""
+    tokens, longest = sum(new_counts), max(new_counts)
+    return _get("ri_attention_prefill_pairs")(head_dim, heads // kv_heads, longest, len(new_counts), kv_heads, tokens,
                                               _weighted_length(new_counts, tokens, longest))
 
 

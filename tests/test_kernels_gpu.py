@@ -1554,3 +1554,21 @@ def test_prompt_attention_in_pairs_of_pages(ops, heads, kv_heads, dh, form):
     for first in (1, 33, 64):
         rows, pieces = run(first, every, True)
         assert np.array_equal(pieces, got[rows])
+
+
+def test_prompts_of_more_tokens_than_a_launch_of_pairs_holds(ops):
+    """A launch has 65,535 workgroups of a sequence's tokens: where pairs of pages take fewer tokens a workgroup than a page a turn, the
+    longest prompts go a page a turn."""
+    pairs = ops.attention_prefill_pairs
+    assert pairs([2048], 16, 8, 128) > 0 and pairs([4 * 65535], 16, 1, 64) == 1 and pairs([4 * 65535 + 1], 16, 1, 64) == 0
+    assert pairs([4 * 65535], 24, 1, 32) == 2 and pairs([4 * 65535 + 1], 24, 1, 32) == 0 and pairs([64 * 65535 + 1], 1, 1, 128) > 0
+    if EMULATED:                                             # (too many tokens for the CPU)
+        return
+    n, last, heads, dh, pages = 4 * 65535 + 1, 40, 16, 32, 8193
+    kp, vp = (torch.randn(shape, device=DEV).to(torch.bfloat16) for shape in ((pages, 1, 32, dh), (pages, 1, dh, 32)))
+    qkv, table = torch.randn((n, heads * dh), device=DEV).to(torch.bfloat16), t(np.arange(pages)[None], torch.int32)
+
+    def run(first, paired):
+        return ops.attention_prefill_bf16(qkv[first:], kp, vp, t([0, n - first], torch.int32), torch.arange(first, n, dtype=torch.int32, device=DEV),
+                                          table, 1, n - first, heads, 1, dh, None, dh ** -0.5, paired=paired)
+    assert torch.equal(run(0, None)[n - last:], run(n - last, False))
