@@ -233,8 +233,8 @@ int ri_attention_prefill_bf16(void* out, const void* qkv, int q_stride, const vo
                               int page_size, int window, float scale, float softcap, const float* slopes, void* stream);
 // How many column tiles a wavefront takes in a step of `tokens` new tokens whose sequences bring `weighted` on a token's average.
 int ri_attention_prefill_tiles(int head_dim, int group, int max_new, int seqs, int kv_heads, int tokens, int weighted);
-// The same where such a step goes in pairs of pages by itself; 0: it goes a page a turn.
-int ri_attention_prefill_pairs(int head_dim, int group, int max_new, int seqs, int kv_heads, int tokens, int weighted);
+// The same where such a step goes in pairs of pages by itself; 0: it goes a page a turn.  reach: its window or chunk, 0 where a token sees all keys.
+int ri_attention_prefill_pairs(int head_dim, int group, int max_new, int seqs, int kv_heads, int tokens, int weighted, int reach);
 // (softcap > 0, here and in the decode form: a score s becomes softcap * tanh(s / softcap) before the softmax)
 
 // Decode form: exactly one new token per sequence; keys in chunks of 256 (in a step of few workgroups each cut into

@@ -60,6 +60,11 @@ static int prefill_tiles(int head_dim, int group, int max_new, int seqs, int kv_
 // workgroups) 58 : 56, 1,792 (448) 48 : 49, 2,816 (704) 94 : 80; two of 1,500 (752) 64 : 69, 500 + 1,500 + 532 (632) 45 : 67, eight of 500 (1,024) 42 : 39, 8,192 of 64 heads
 // 1,380 : 1,081.  Heads of 32 and 64: one, 2,048 of 32 heads of 64 32.5 : 38, 6,000 204 : 221 (4,096 99 : 95); more only where a key head's queries need them.
 #define PAIRS_MIN_TOKENS 400
+// A window or a chunk of fewer keys than this (`reach`) leaves a turn's chain too few pages: a page a turn, unless its rule takes larger tiles.  us, a
+// page a turn : pairs (heads of 128 over 8; windows of 128 / 256 / 512): 8,192 of 32 heads 58 : 66 / 75 : 76 / 113 : 106, of 64 115 : 122 / 148 : 150 / 221 : 204,
+// six of 700 of 16 21 : 24 / 24 : 26 / 30 : 30, of 32 35 : 39 / 41 : 41 / 49 : 48; chunks of 128 / 512, six of 700 of 32 28 : 31 / 37 : 36.  Heads of 64, four
+// tiles against one: 8,192 of 32 heads 81 : 39 / 106 : 50 / 151 : 70; one against one: 2,048 11.6 : 12.5 / 15.2 : 15.8 / 21.6 : 20.0.
+#define PAIRS_MIN_REACH 512
 #define PREFILL_MAX_LAUNCHES 65535
 static int pair_tiles(int head_dim, int group, int seqs, int kv_heads, int tokens) {
     const int of_wg = 4 * (32 / (group <= 32 ? group : 32));
@@ -70,16 +75,19 @@ static int pair_tiles(int head_dim, int group, int seqs, int kv_heads, int token
 
 struct PrefillPlan { bool paired; int tiles, launches; };     // tiles of columns a wavefront, workgroups of the longest sequence's tokens a key head
 // pairs: 1 so, 0 not so, -1 where it pays and a launch holds it.
-static PrefillPlan prefill_plan(int head_dim, int group, int max_new, int seqs, int kv_heads, int tokens, int weighted, int pairs) {
+static PrefillPlan prefill_plan(int head_dim, int group, int max_new, int seqs, int kv_heads, int tokens, int weighted, int reach,
+                                int pairs) {
     const auto plan = [&](bool paired, int nt) { const int of_wg = 4 * (group < 16 * nt ? 16 * nt / group : 1); return PrefillPlan{paired, nt, (max_new + of_wg - 1) / of_wg}; };
+    const PrefillPlan one = plan(false, prefill_tiles(head_dim, group, max_new, seqs, kv_heads, tokens, weighted));
     const PrefillPlan two = plan(true, pair_tiles(head_dim, group, seqs, kv_heads, tokens));
-    if (pairs == 1 || (pairs == -1 && tokens >= (long)PAIRS_MIN_TOKENS * seqs && two.launches <= PREFILL_MAX_LAUNCHES)) return two;
-    return plan(false, prefill_tiles(head_dim, group, max_new, seqs, kv_heads, tokens, weighted));
+    if (pairs >= 0) return pairs ? two : one;
+    if (tokens < (long)PAIRS_MIN_TOKENS * seqs || two.launches > PREFILL_MAX_LAUNCHES) return one;
+    return reach > 0 && reach < PAIRS_MIN_REACH && one.tiles <= two.tiles ? one : two;
 }
 
 // The tiles of columns a wavefront takes of a step that goes in pairs of pages, 0: a page a turn (host code only).
-extern "C" int ri_attention_prefill_pairs(int head_dim, int group, int max_new, int seqs, int kv_heads, int tokens, int weighted) {
-    const PrefillPlan plan = prefill_plan(head_dim, group, max_new, seqs, kv_heads, tokens, weighted, -1);
+extern "C" int ri_attention_prefill_pairs(int head_dim, int group, int max_new, int seqs, int kv_heads, int tokens, int weighted, int reach) {
+    const PrefillPlan plan = prefill_plan(head_dim, group, max_new, seqs, kv_heads, tokens, weighted, reach, -1);
     return plan.paired ? plan.tiles : 0;
 }
 
@@ -104,7 +112,7 @@ extern "C" int ri_attention_prefill_kept_bf16(void* out, const void* qkv, int q_
     RI_REQUIRE(seqs > 0 && seqs <= 65535 && max_new > 0, "attention_prefill_bf16: seqs %d, max_new %d", seqs, max_new);
     RI_REQUIRE(pairs >= -1 && pairs <= 1, "attention_prefill_bf16: pairs %d", pairs);
     RI_REQUIRE(group <= (head_dim <= 64 ? 64 : 32), "attention_prefill_bf16: %d query heads per kv head (at most %d)", group, head_dim <= 64 ? 64 : 32);
-    const PrefillPlan plan = prefill_plan(head_dim, group, max_new, seqs, kv_heads, tokens, weighted, pairs);
+    const PrefillPlan plan = prefill_plan(head_dim, group, max_new, seqs, kv_heads, tokens, weighted, window > 0 ? window : chunk, pairs);
     RI_REQUIRE(plan.launches <= PREFILL_MAX_LAUNCHES, "attention_prefill_bf16: %d tiles of tokens exceed one launch", plan.launches);
     int long_runs;
     const dim3 grid = prefill_grid(kv_heads, seqs, plan.launches, 4 * (16 * plan.tiles / group), tokens, long_runs);

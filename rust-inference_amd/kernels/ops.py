@@ -111,7 +111,7 @@ _SIGNATURES = {
     "ri_attention_prefill_kept_bf16": [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int,
                                        c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_float, c_void_p, c_int,
                                        c_void_p, c_int, c_int, c_int, c_void_p],
-    "ri_attention_prefill_pairs": [c_int, c_int, c_int, c_int, c_int, c_int, c_int],
+    "ri_attention_prefill_pairs": [c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int],
     "ri_attention_prefill_tiles": [c_int, c_int, c_int, c_int, c_int, c_int, c_int],
     "ri_attention_kept": [c_void_p, c_void_p, c_int, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int,
                           c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_float, c_void_p, c_int, c_void_p,
@@ -1256,11 +1256,12 @@ def attention_prefill_tiles(new_counts, heads: int, kv_heads: int, head_dim: int
                                               _weighted_length(new_counts, tokens, longest))
 
 
-def attention_prefill_pairs(new_counts, heads: int, kv_heads: int, head_dim: int) -> int:
-    """The same for a step that ``attention_prefill_bf16`` takes in pairs of pages where ``paired`` is None; 0: a page a turn."""
+def attention_prefill_pairs(new_counts, heads: int, kv_heads: int, head_dim: int, reach: int = 0) -> int:
+    """The same for a step that ``attention_prefill_bf16`` takes in pairs of pages where ``paired`` is None; 0: a page a turn.  ``reach``: its
+    window or chunk."""
     tokens, longest = sum(new_counts), max(new_counts)
     return _get("ri_attention_prefill_pairs")(head_dim, heads // kv_heads, longest, len(new_counts), kv_heads, tokens,
-                                              _weighted_length(new_counts, tokens, longest))
+                                              _weighted_length(new_counts, tokens, longest), reach)
 
 
 def attention_prefill_bf16(qkv, k_pages, v_pages, cu_seqlens, tok_pos, page_table, seqs: int, max_new: int,

@@ -1572,3 +1572,17 @@ def test_prompts_of_more_tokens_than_a_launch_of_pairs_holds(ops):
         return ops.attention_prefill_bf16(qkv[first:], kp, vp, t([0, n - first], torch.int32), torch.arange(first, n, dtype=torch.int32, device=DEV),
                                           table, 1, n - first, heads, 1, dh, None, dh ** -0.5, paired=paired)
     assert torch.equal(run(0, None)[n - last:], run(n - last, False))
+
+
+def test_pairs_of_pages_where_they_pay(ops):
+    """On 256 compute units, as measured beside the rule: prompts of hundreds of tokens on average whose tokens see hundreds of keys; windows
+    and chunks shorter than that go a page a turn, unless that would take larger tiles."""
+    if not EMULATED and torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("measured on 256 compute units")
+    pairs = ops.attention_prefill_pairs
+    for heads in (16, 32, 64):
+        for new in ([2048], [8192], [700] * 6):
+            assert pairs(new, heads, 8, 128) > 0 and pairs(new, heads, 8, 128, 512) > 0
+            assert pairs(new, heads, 8, 128, 128) == 0 and pairs(new, heads, 8, 128, 511) == 0
+    assert pairs([300] * 16, 16, 8, 128) == 0 and pairs([8192] + [1] * 40, 16, 8, 128) == 0
+    assert pairs([8192], 32, 8, 64, 128) == 1 and ops.attention_prefill_tiles([8192], 32, 8, 64) == 4 and pairs([2048], 32, 8, 64, 128) == 0
