@@ -65,6 +65,12 @@ static int prefill_tiles(int head_dim, int group, int max_new, int seqs, int kv_
 // six of 700 of 16 21 : 24 / 24 : 26 / 30 : 30, of 32 35 : 39 / 41 : 41 / 49 : 48; chunks of 128 / 512, six of 700 of 32 28 : 31 / 37 : 36.  Heads of 64, four
 // tiles against one: 8,192 of 32 heads 81 : 39 / 106 : 50 / 151 : 70; one against one: 2,048 11.6 : 12.5 / 15.2 : 15.8 / 21.6 : 20.0.
 #define PAIRS_MIN_REACH 512
+// A key head's queries that fill pairs' tiles badly (9 and 10 one tile: 0.56 and 0.63 of its columns, 17 to 21 two tiles) beside tiles of twice the size that
+// they fill to 0.8 and more go a page a turn.  us, a page a turn : pairs, four key heads: 9 queries, eight of 500 35 : 39 (heads of 32), 41 : 48 (of 64), three of 1,500 92 : 97,
+// 102 : 121; 17, of 32, three of 1,500 193 : 216, 6,000 948 : 1,044.  Not four tiles against one (9 and 10 queries, 6,000: 455 : 449 and 530 : 446) nor four
+// of heads of 64 (17, 6,000: 1,630 : 1,138); 11 (0.69) three of 1,500 of 32 130 : 99, 22 (0.69) 283 : 217.  More than 32 queries take four tiles either way,
+// for heads of 64 with some of their registers in memory: 6,000, one key head of 64 queries of 64 867 : 552, of 40 1,273 : 936, of 40 of 32 714 : 647.
+#define PAIRS_MIN_FILL_TENTHS 7
 #define PREFILL_MAX_LAUNCHES 65535
 static int pair_tiles(int head_dim, int group, int seqs, int kv_heads, int tokens) {
     const int of_wg = 4 * (32 / (group <= 32 ? group : 32));
@@ -82,7 +88,10 @@ static PrefillPlan prefill_plan(int head_dim, int group, int max_new, int seqs, 
     const PrefillPlan two = plan(true, pair_tiles(head_dim, group, seqs, kv_heads, tokens));
     if (pairs >= 0) return pairs ? two : one;
     if (tokens < (long)PAIRS_MIN_TOKENS * seqs || two.launches > PREFILL_MAX_LAUNCHES) return one;
-    return reach > 0 && reach < PAIRS_MIN_REACH && one.tiles <= two.tiles ? one : two;
+    if (reach > 0 && reach < PAIRS_MIN_REACH && one.tiles <= two.tiles) return one;
+    const auto columns = [&](int nt) { return 16 * nt / group * group; };
+    const bool emptier = 10 * columns(two.tiles) * one.tiles < PAIRS_MIN_FILL_TENTHS * columns(one.tiles) * two.tiles;
+    return emptier && one.tiles == 2 * two.tiles && !(head_dim == 64 && one.tiles == 4) ? one : two;
 }
 
 // The tiles of columns a wavefront takes of a step that goes in pairs of pages, 0: a page a turn (host code only).

@@ -1584,5 +1584,9 @@ def test_pairs_of_pages_where_they_pay(ops):
         for new in ([2048], [8192], [700] * 6):
             assert pairs(new, heads, 8, 128) > 0 and pairs(new, heads, 8, 128, 512) > 0
             assert pairs(new, heads, 8, 128, 128) == 0 and pairs(new, heads, 8, 128, 511) == 0
+    for group in (9, 10, 17, 18, 21):                        # (pairs' tiles would leave almost half of their columns empty)
+        assert pairs([1500] * 3, 4 * group, 4, 32) == 0 and pairs([500] * 8, 4 * group, 4, 32) == 0
+        assert (pairs([1500] * 3, 4 * group, 4, 64) == 0) == (group < 16) and pairs([6000], 4 * group, 4, 64) > 0
+    assert pairs([1500] * 3, 12 * 4, 4, 32) > 0 and pairs([1500] * 3, 22 * 4, 4, 32) > 0 and pairs([2000], 20, 1, 32) > 0
     assert pairs([300] * 16, 16, 8, 128) == 0 and pairs([8192] + [1] * 40, 16, 8, 128) == 0
     assert pairs([8192], 32, 8, 64, 128) == 1 and ops.attention_prefill_tiles([8192], 32, 8, 64) == 4 and pairs([2048], 32, 8, 64, 128) == 0
