@@ -3,6 +3,7 @@ reach the kernels of long prompts.
 
 Like tests/test_kernels_gpu.py these run without a GPU when the environment says RI_TEST_KERNELS=emulated
 (tests/test_kernels_emulated.py starts that run): the CPU build of the same sources."""
+import math
 import os
 
 import numpy as np
@@ -175,3 +176,161 @@ def test_latent_prompts_only_where_the_kernel_takes_them(ops, rt):
     assert pays([32] * 52758, [0] * 52758) and not pays([32] * 52759, [0] * 52759)           # 31 B / 128 + B of 65,535 and 65,536
     part.EXPAND_BYTES >>= 7
     assert pays([33] * (most >> 13), [0] * (most >> 13)) and not pays([33] * ((most >> 13) + 1), [0] * ((most >> 13) + 1))
+
+
+@pytest.fixture
+def small_machine(ops, monkeypatch):
+    """The rule of the products in tiles on a machine of two compute units, from 128 rows on; the kernel runs on the real one."""
+    from rust_inference_amd.parts import runtime
+    runtime._tiles_plan.cache_clear()
+    monkeypatch.setattr(runtime, "_compute_units", lambda: 2)
+    monkeypatch.setattr(runtime, "TILES_MIN_ROWS", 128)
+    yield calls_of(monkeypatch, ops, "gemm_tiles_bf16")
+    runtime._tiles_plan.cache_clear()
+
+
+def activation_of(call):
+    args, kw = call
+    return args[4] if len(args) > 4 else kw.get("activation")
+
+
+def sigmoid(z):
+    return 1.0 / (1.0 + np.exp(-z))
+
+
+class Forms:
+    """The gated forms and the squared ReLU in 64 bits."""
+
+    @staticmethod
+    def clamped(g, u, limit):
+        g, u = np.minimum(g, limit), np.clip(u, -limit, limit)
+        return g * sigmoid(1.702 * g) * (u + 1.0)
+
+    silu = staticmethod(lambda g, u: g * sigmoid(g) * u)
+    relu2 = staticmethod(lambda z: np.maximum(z, 0.0) ** 2)
+
+
+@pytest.mark.parametrize("rows, tiles", [(250, True), (100, False)])
+@pytest.mark.parametrize("kind", ["swiglu", "relu2", "gelu_tanh", "clamped", "clamped with biases"])
+def test_feed_forward_of_prompts(ops, rt, monkeypatch, small_machine, kind, rows, tiles):
+    """A feed-forward whose products go in tiles, the activation in the first of them, and one of too few rows, where the activation
+    is a kernel of its own: both against 64 bits (gate and up exchanged, a bias or a clamp left out would be of order one)."""
+    from rust_inference_amd.parts import PartSpec, build_part
+    rng = np.random.default_rng(rows + len(kind))
+    hidden, inter, limit = 256, 192, 0.9
+    name, args = {"swiglu": ("swiglu", {}), "relu2": ("dense", {"activation": "relu2"}), "gelu_tanh": ("dense", {"activation": "gelu_tanh"}),
+                  "clamped": ("glu_clamped", {"limit": limit, "biases": False}), "clamped with biases": ("glu_clamped", {"limit": limit})}[kind]
+    part = build_part("feed_forward", PartSpec(name, {"hidden": hidden, "inter": inter, "prefix": "m.", **args}))
+    w = random_weights(part, rng)
+    part.bind(w, rt)
+    w = {key[2:].replace("_proj.weight", ""): f64(x) for key, x in w.items()}
+    x = t(rng.normal(size=(rows, hidden)), torch.bfloat16)
+    out = part.forward(x, None)
+    out = f64(out if out.dim() == 2 else out.sum(0))
+    if getattr(part, "out_bias", None) is not None:
+        out = out + f64(part.out_bias)
+    h = f64(x)
+    up = h @ w["up"].T + w.get("up.b", 0.0)
+    if "gate" in w:
+        gate = h @ w["gate"].T + w.get("gate.b", 0.0)
+        act = Forms.silu(gate, up) if kind == "swiglu" else Forms.clamped(gate, up, limit)
+    else:
+        act = Forms.relu2(up) if kind == "relu2" else 0.5 * up * (1.0 + np.tanh(np.sqrt(2 / np.pi) * (up + 0.044715 * up ** 3)))
+    assert rel_to_max(out, act @ w["down"].T + w.get("down.b", 0.0)) < 2e-2
+    fused = {"swiglu": "silu_gate", "relu2": "relu2", "gelu_tanh": None}.get(kind, "clamped_gate")
+    want = ([fused] if fused else []) + [None] if tiles else []
+    assert [activation_of(call) for call in small_machine] == want
+
+
+@pytest.mark.parametrize("kind", ["silu", "clamped", "relu2", "gelu_erf"])
+def test_experts_of_prompts(ops, rt, monkeypatch, small_machine, kind):
+    """Experts whose rows lie side by side, two of them with enough for tiles and one without: the activation in the product, and beside
+    it, against 64 bits; the stretches of the two matrices are an expert's own."""
+    from rust_inference_amd.parts import PartSpec, build_part
+    rng = np.random.default_rng(len(kind))
+    hidden, inter, vocab, tokens, limit = 256, 192, 40, 508, 0.8
+    args = {"silu": {"limit": None}, "clamped": {"limit": limit}}.get(kind, {"limit": None, "gated": False, "activation": kind})
+    part = build_part("feed_forward", PartSpec("routed_experts", {"hidden": hidden, "inter": inter, "experts": 3, "top": 1, "prefix": "m.", "scores": "table",
+                                                                  "vocab": vocab, "shared_gate": False, **args}))
+    w = random_weights(part, rng)
+    w["m.table"] = torch.tensor([[0 if i < 20 else 1 if i < 38 else 2] for i in range(vocab)], dtype=torch.int32)
+    part.bind(w, rt)
+    ids = np.concatenate([rng.integers(0, 20, 250), rng.integers(20, 38, 240), rng.integers(38, 40, 18)])
+    rng.shuffle(ids)
+    x = t(rng.normal(size=(tokens, hidden)), torch.bfloat16)
+    ctx = type("Step", (), {"tokens": t(ids, torch.int32), "T": tokens, "is_decode": False})
+    if EMULATED:                                             # (the host's wait for the row counts needs a GPU)
+        def sort(x, chosen):
+            dest, offsets = ops.experts_sort(chosen, part.outs)
+            return ops.experts_gather(x, dest, part.top), dest, offsets, type("There", (), {"synchronize": staticmethod(lambda: None)})
+        monkeypatch.setattr(part, "sort", sort)
+        monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    out = part.forward(x, ctx)
+    out = f64(out if out.dim() == 2 else out.sum(0))
+    h, want, w = f64(x), np.zeros((tokens, hidden)), {key[2:]: f64(v) for key, v in w.items()}
+    erf = np.vectorize(math.erf)
+    for e in range(3):
+        mine = w["table"][ids, 0] == e
+        up = h[mine] @ w[f"e{e}.up"].T
+        if kind in ("silu", "clamped"):
+            gate = h[mine] @ w[f"e{e}.gate"].T
+            act = Forms.silu(gate, up) if kind == "silu" else Forms.clamped(gate, up, limit)
+        else:
+            act = Forms.relu2(up) if kind == "relu2" else 0.5 * up * (1.0 + erf(up / np.sqrt(2.0)))
+        want[mine] = act @ w[f"e{e}.down"].T
+    assert rel_to_max(out, want) < 2e-2
+    fused = {"silu": ["silu_gate"], "clamped": ["clamped_gate"], "relu2": ["relu2"], "gelu_erf": []}[kind]
+    assert [activation_of(call) for call in small_machine] == (fused + [None]) * 2
+
+
+@pytest.mark.parametrize("lie", ["side by side", "rows of longer ones", "x off a line", "w off a line", "w transposed", "x transposed", "results off a line",
+                                 "results in rows of 252"])
+def test_rows_and_matrices_that_lie_as_the_tiles_want_them(ops, rt, small_machine, lie):
+    """Products into given rows: stretches of longer rows go in tiles; what lies off a multiple of sixteen bytes or across stays with the
+    library, with the same result."""
+    rng = np.random.default_rng(len(lie))
+    m, n, k = 256, 256, 192
+    put = lambda rows, columns, off=0, pad=0: torch.zeros(rows * (columns + pad) + off, dtype=torch.bfloat16, device=DEV)[off:].view(rows, columns + pad)[:, :columns]
+    x, w, out = put(m, k), put(n, k), put(m, n)
+    if lie == "rows of longer ones":
+        x, w, out = put(m, k, 8, 16), put(n, k, 16, 8), put(m, n, 8, 24)
+    elif lie == "x off a line":
+        x = put(m, k, 4)
+    elif lie == "w off a line":
+        w = put(n, k, 4)
+    elif lie == "w transposed":
+        w = put(k, n).t()
+    elif lie == "x transposed":
+        x = put(k, m).t()
+    elif lie == "results off a line":
+        out = put(m, n, 4)
+    elif lie == "results in rows of 252":
+        out = put(m + 4, 252)[4:].as_strided((m, n - 8), (252, 1))
+        w, n = put(n - 8, k), n - 8
+    x.copy_(t(rng.normal(size=(m, k))))
+    w.copy_(t(rng.normal(size=(n, k))))
+    rt.rows_into(out, x, w)
+    assert rel_to_max(f64(out), f64(x) @ f64(w).T) < 4e-3
+    assert len(small_machine) == (lie in ("side by side", "rows of longer ones"))
+
+
+def test_the_rule_of_the_products_in_tiles(monkeypatch):
+    """On 256 compute units, at sizes measured beside the rule: full rounds, an activation that rides along, and what is left to the library."""
+    from rust_inference_amd.parts import runtime
+    from rust_inference_amd.kernels.ops import TILES
+    monkeypatch.setattr(runtime, "_compute_units", lambda: 256)
+    runtime._tiles_plan.cache_clear()
+    plan = runtime._tiles_plan
+    large, wide, tall = TILES.index((256, 256)), TILES.index((128, 256)), TILES.index((256, 128))
+    assert plan(2048, 4096, 4096, False, None) in (wide, tall) and plan(1536, 5120, 5120, True, None) in (wide, tall)       # one round
+    assert plan(2048, 3400, 4096, False, None) is None                                  # (0.83 of one round)
+    assert plan(8192, 5120, 8192, False, None) == large and plan(5120, 8192, 4096, False, None) == large                    # three rounds, 0.8 to 0.93
+    assert plan(8192, 12288, 4096, False, None) is None and plan(8192, 12288, 4096, True, None) == large                    # full: float32 results alone
+    for act in ("silu_gate", "clamped_gate"):
+        assert plan(2048, 24576, 4096, False, act) == large and plan(759, 24576, 4096, False, act) is not None
+        assert plan(759, 6144, 1024, False, act) is not None and plan(759, 6144, 4096, False, act) is None                  # 0.45 for short rows, else 0.62
+        assert plan(2048, 24576 + 8, 4096, False, act) is None                          # (halves that are no multiple of 8)
+    assert plan(759, 6144, 1024, False, "relu2") is None and plan(2048, 18432, 4096, False, "relu2") == tall              # 0.1 more without a gate
+    for m, n, k in ((511, 4096, 4096), (2048, 4096, 4096 + 32), (2048, 4096, 128), (2048, 4096 + 4, 4096)):
+        assert plan(m, n, k, False, None) is None and plan(m, n, k, False, "relu2") is None
+    runtime._tiles_plan.cache_clear()
