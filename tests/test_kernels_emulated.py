@@ -21,7 +21,8 @@ HERE = os.path.join(ROOT, "tests")
 # smaller sizes of the same tests or, where the form is chosen by the machine's size, on a machine made small (below).
 SELECT = ("not 4096 and not 12288 and not 5120 and not 5000 and not very_long and not more_pages_than and not thousands "
           "and not (many_sequences and not (16-8-32-100 or 16-8-32-40)) and not (in_runs and not 8-8-32) "
-          "and not (wide_packed and 1000 and not (1000-1024-33 or 1000-1024-64)) and not eight_wavefronts and not over_rounds and not (copied_as_they_are and not (67-60 or 1-8-64))")
+          "and not (wide_packed and 1000 and not (1000-1024-33 or 1000-1024-64)) and not eight_wavefronts and not over_rounds and not (copied_as_they_are and not (67-60 or 1-8-64)) "
+          "and not (in_pairs_of_pages and (20-1-32 or 64-1-32 or 40-1-64) and (window or chunk or cap or sinks))")
 
 
 def _env(extra=None):

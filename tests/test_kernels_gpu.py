@@ -331,7 +331,7 @@ def test_rotation_over_part_of_the_head(ops, dtype, rel, dh, rot):
                                   t(tok_seq, torch.int32), table, kp, vp, heads, kv_heads, dh)
 
 
-def attention_case(ops, rng, lens, new, heads, kv_heads, dh, dtype, window=None, boost=None, kernel="generic"):
+def attention_case(ops, rng, lens, new, heads, kv_heads, dh, dtype, window=None, boost=None, kernel="generic", paired=False):
     k, v, kp, vp, table = paged(rng, lens, kv_heads, dh, dtype=dtype, spare=12)
     tokens = sum(new)
     width = (heads + 2 * kv_heads) * dh
@@ -349,7 +349,7 @@ def attention_case(ops, rng, lens, new, heads, kv_heads, dh, dtype, window=None,
         out = ops.attention(qkv_t, kp, vp, pos_t, seq_t, table, heads, kv_heads, dh, window, scale)
     elif kernel == "prefill":
         out = ops.attention_prefill_bf16(qkv_t, kp, vp, cu, pos_t, table, len(lens), max(new), heads, kv_heads, dh,
-                                         window, scale)
+                                         window, scale, **({} if paired is False else dict(new_counts=new, paired=paired)))
     else:
         assert all(n == 1 for n in new)
         # a bound on the length well above the real one: it sizes grid and workspace, never the result
@@ -1505,10 +1505,10 @@ PAIR_FORMS = {"plain": {}, "window": {"window": 40}, "a page's window": {"window
 
 
 @pytest.mark.parametrize("form", list(PAIR_FORMS))
-@pytest.mark.parametrize("heads, kv_heads, dh", [(16, 1, 128), (20, 1, 128), (5, 5, 64), (17, 1, 64), (6, 2, 32)])
+@pytest.mark.parametrize("heads, kv_heads, dh", [(16, 1, 128), (20, 1, 128), (5, 5, 64), (17, 1, 64), (6, 2, 32), (20, 1, 32), (64, 1, 32), (40, 1, 64)])
 def test_prompt_attention_in_pairs_of_pages(ops, heads, kv_heads, dh, form):
     """Two pages a turn against one: whole prompts and pieces, sequences that end in either page of a pair, windows and kept tokens whose first
-    and last pages are of either number, pages that nobody sees not mapped; one tile of columns and two.  The two are up to a rounding of the weights
+    and last pages are of either number, pages that nobody sees not mapped; one tile of columns, two and four.  The two are up to a rounding of the weights
     (2^-9 of each) and of the result away from one another.  And the same bits alone, in one step with others and in pieces."""
     rng = np.random.default_rng(heads + dh)
     lens, new = [70, 300, 257, 1, 45, 131, 64], [70, 5, 1, 1, 45, 99, 64]
@@ -1554,6 +1554,23 @@ def test_prompt_attention_in_pairs_of_pages(ops, heads, kv_heads, dh, form):
     for first in (1, 33, 64):
         rows, pieces = run(first, every, True)
         assert np.array_equal(pieces, got[rows])
+
+
+@pytest.mark.parametrize("window", [None, 50])
+@pytest.mark.parametrize("heads, kv_heads, dh", MFMA_SHAPES + [(20, 1, 32), (64, 1, 32), (40, 1, 64)])
+def test_mfma_prefill_attention_in_pairs(ops, heads, kv_heads, dh, window):
+    """Whole prompts and pieces of unequal lengths in pairs of pages against 64 bits, every number of tiles."""
+    out, want = attention_case(ops, np.random.default_rng(heads * 3 + dh), [70, 300, 257, 1, 45, 131], [70, 5, 1, 1, 45, 99], heads, kv_heads, dh,
+                               torch.bfloat16, window=window, kernel="prefill", paired=True)
+    close(out, want, BF16_OUT, "prefill attention in pairs of pages")
+
+
+def test_prompts_take_pairs_of_pages_by_themselves(ops):
+    """A step's rule: prompts that bring enough tokens go in pairs of pages, the same bits as when told so; shorter ones a page a turn."""
+    for lens, new in (([450, 460], [440, 460]), ([450, 90], [330, 90])):
+        both = [f64(attention_case(ops, np.random.default_rng(7), lens, new, 4, 2, 32, torch.bfloat16, kernel="prefill", paired=p)[0])
+                for p in (None, sum(new) >= 400 * len(new))]
+        assert (ops.attention_prefill_pairs(new, 4, 2, 32) > 0) == (sum(new) >= 400 * len(new)) and np.array_equal(*both)
 
 
 def test_prompts_of_more_tokens_than_a_launch_of_pairs_holds(ops):
