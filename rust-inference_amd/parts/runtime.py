@@ -128,6 +128,12 @@ def _tiles_plan(m: int, n: int, k: int, wide_out: bool, activation: str | None) 
     return None
 
 
+@functools.lru_cache(maxsize=4096)
+def _tiles_fit(m: int, n: int, ldx: int, ldw: int, ldo: int, activation: str | None) -> bool:
+    """``ops.gemm_tiles_fits``, asked once per size."""
+    return ops.gemm_tiles_fits(m, n, ldx, ldw, ldo, activation)
+
+
 class PackedWeight:
     """A bfloat16 weight as the library product wants it (row-major) and, for decode-size products,
     packed into MFMA tiles."""
@@ -404,7 +410,7 @@ class Runtime:
             return None                                          # the library's product takes any strides
         n = w.shape[0] // 2 if activation in ("silu_gate", "clamped_gate") else w.shape[0]
         ldx = x.stride(0) if isinstance(x, torch.Tensor) else x.shape[1]
-        return tile if ops.gemm_tiles_fits(x.shape[0], n, ldx, w.stride(0), ldo or n, activation) else None
+        return tile if _tiles_fit(x.shape[0], n, ldx, w.stride(0), ldo or n, activation) else None
 
     def _library_mm(self, x, w, out_dtype):
         # The reference hands every product to a vendor library (src/cuda/mod.rs:186-232);
