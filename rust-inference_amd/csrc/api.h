@@ -273,7 +273,9 @@ int ri_attention_decode_fused_bf16(void* out, float* workspace, const void* qkv,
                                    int seqs, int max_chunks, int heads, int kv_heads, int head_dim, int page_size,
                                    int window, float scale, int tiled_out, void* stream);
 
-// out[M, N] (float32) = x[M, K] (float32) . w[N, K]^T, w float32 or bfloat16; no input is rounded, the sums are float32.
+// out[M, N] (float32) = x[M, K] (float32) . w[N, K]^T, w float32 or bfloat16; no input is rounded, the sums are float32.  tile: -1, or for
+// bfloat16 w (K a multiple of 8, aligned rows) the form to take instead of the rule's, with the same bits: 0 to 2 tiles of 64 x 128, 32 x 64
+// and 32 x 32; 3 to 6 tiles of 128 x 160, 128 x 128, 64 x 128 and 64 x 64 with copies straight into LDS, only where K is a multiple of 64 and N of 4.
 int ri_gemm_f32(float* out, const float* x, const void* w, int w_dtype, int m, int n, int k, int tile, void* stream);
 
 // out[M, N] (out_dtype) = x[M, K] . w[N, K]^T for bfloat16 x and w, float32 accumulation, M <= 8.

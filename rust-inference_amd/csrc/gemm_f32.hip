@@ -225,7 +225,8 @@ struct SplitPair {
 };
 
 // Tiles of 16 MT WAVES rows of x and 16 NT of w: a wavefront has 16 MT rows and all columns, so that no row is split twice and none of its parts
-// written.  K in stages of 64 through SLOTS buffers, filled by copies that do not pass through registers and go out one or two stages ahead.
+// written.  K in stages of 64 through SLOTS buffers, filled by copies that do not pass through registers and go out SLOTS - LAG stages ahead: two
+// (three buffers), three (five) or four (six).
 // The split, the reads and the copies stand between the products, three or four instructions each.  What bounds a large tile is then the matrix
 // cores at the clock that they leave (128 x 160: 1,920 cycles of products a stage, 1.19 us; 759 rows, 6,144 x 1,024: 48 -> 33 us; 128 x 128,
 // 4,096 x 1,024: 30 -> 23), the smallest the instructions it issues, half of them the split (64 x 64: 0.46 us a stage; 1,024 x 3,072: 31 -> 27).

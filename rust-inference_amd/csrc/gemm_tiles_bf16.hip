@@ -8,7 +8,8 @@
 //  - the largest tile that four wavefronts can hold: 256 sums a lane, one wavefront a SIMD, which has to hide everything by itself;
 //  - so a stage's memory instructions stand between its products one by one (a run of them, some sixty cycles, is a gap of the matrix
 //    cores: 2,700 cycles a stage), the fragments of a half of K read while the other half is multiplied, and the buffer given back as soon
-//    as the second half's are read (at two of five of a stage, so that a copy has a stage and a half to arrive);
+//    as the second half's are read (at 0.28 of a stage, 0.25 in the smaller tiles), so that the copies, one every few products from there on,
+//    have 1.2 stages (the first) to 0.6 (the last) to arrive;
 //  - workgroups stay and take tile after tile, and the copies run ahead into the next tile, so that a tile begins with its operands there
 //    (a launch a tile: 3,800 cycles before the first product and 7,400 after the last, of 50,000 at K = 1,024);
 //  - the rows of w go into a fragment in an order that leaves a lane eight neighbouring bfloat16 results, and two lanes exchange halves, so

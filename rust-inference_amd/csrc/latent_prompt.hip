@@ -3,7 +3,7 @@
 // On the latents as they lie (latent_mfma.hip) a score costs key rows of rank + rot elements and a value product rows of rank: 1,088
 // multiply-adds a (token, key, head) at 576 and 512.  With U_h c and V_h c made once a key it costs dim + rot + vdim: 320.  The products that
 // make them are 2 rank (dim + vdim) operations a key and head, what about thirty tokens' scores cost more on the latents; so it pays for
-// prompts, and the single tokens keep the latents.  Three steps:
+// prompts, and steps of single tokens keep the latents (single tokens beside a prompt come along: below).  Three steps:
 //  - ri_latent_gather: the sequences' pages side by side, sequence after sequence (a sequence begins at a multiple of 32 rows): [c | k_r] rows,
 //    zeros behind a sequence's end;
 //  - two products of all rows (ri_gemm_tiles_bf16 or the library's): keys U c as rows [row][heads * dim], values V c transposed, [heads * vdim][row],
@@ -14,7 +14,9 @@
 // Bound by the chain of a turn, two wavefronts a SIMD (registers; four pages in LDS are half a compute unit's).  Pages come by copies straight into
 // LDS, three turns ahead: through registers, a turn ahead, a turn took the time of its loads (2,048 tokens, 32 heads of 128 + 64: 131 us; so 74).
 // us on the latents, with the two products per head there : these three steps; 32 heads, latents of 512 + 64: 2,048 tokens 619 : 104, 700 + 300 + 33
-// 239 : 66, 512 163 : 47, 128 65 : 29, eight of 64 69 : 35, 128 after 2,000 keys 499 : 116, eight of 32 after 1,000 282 : 200; error against 64 bits (2-norm)
+// 239 : 66, 512 163 : 47, 128 65 : 29, eight of 64 69 : 35, 128 after 2,000 keys 499 : 116, eight of 32 after 1,000 282 : 200; with single tokens
+// beside the prompt, whose sequences' keys are made for one query each (the whole mixer, us): 2,048 and eight at 1,000 keys 1,024 : 275, 512 and eight 311 : 233,
+// 1,024 and 16 at 2,000 599 : 519, 4,096 and 100 at 1,000 2,833 : 1,735, 1,024 and one at 30,000 6,510 : 1,124; error against 64 bits (2-norm)
 // 3.2e-3 : 2.7e-3 (queries and results per head are no longer rounded on their way through the latents).
 #include "attention_mfma.h"
 #include "matrix_async.h"

@@ -104,7 +104,10 @@ class LatentAttention(Mixer):
 
     # Keys and values of all heads from EXPAND_TOKENS new tokens on, EXPAND_EACH of them a sequence on average and EXPAND_KEYS cached
     # tokens for one new one at the most, up to EXPAND_BYTES of them.  (On the latents : so, us, 32 heads, 512 + 64: 128 tokens 65 : 29, eight
-    # of 32 after 1,000 keys 282 : 200; a token's scores gain on the latents what thirty keys' products cost.)
+    # of 32 after 1,000 keys 282 : 200; a token's scores gain on the latents what thirty keys' products cost.  Averages are enough: a prompt with single
+    # tokens beside it is ahead too, the figures at csrc/latent_prompt.hip.)  What EXPAND_BYTES bounds is there for the length of the layer's attention,
+    # with the rows side by side (rank + rot_dim numbers a cached token) beside it; on the latents the queries and results are (2 rank + rot_dim a head of
+    # every new token).
     EXPAND_TOKENS, EXPAND_EACH, EXPAND_KEYS, EXPAND_BYTES, EXPAND_RUNS = 128, 32, 32, 2 << 30, 65535
 
     def _expand_pays(self, ctx, proj, store) -> bool:
