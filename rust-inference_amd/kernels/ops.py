@@ -1273,8 +1273,8 @@ def attention_prefill_bf16(qkv, k_pages, v_pages, cu_seqlens, tok_pos, page_tabl
     score ``s`` becomes ``softcap * tanh(s / softcap)`` before the softmax; with ``slopes`` (float32 ``[heads]``) head
     ``h``'s score at position ``p`` for the key at ``j`` then loses ``slopes[h] * (p - j)``.  ``keep_first``, ``sinks``,
     ``q_off`` and ``chunk`` as in ``attention``.  ``new_counts``: every sequence's new tokens, where the caller knows them.
-    ``paired``: a sequence's pages two by two (True) or one by one (False), None: by what the sequences bring on average; a token's result
-    is the same bits with every step of either kind."""
+    ``paired``: a sequence's pages two by two (True) or one by one (False), None: whichever is faster (``attention_prefill_pairs``); a token's
+    result is the same bits with every step of either kind."""
     tokens, stride = qkv.shape
     if q_off < 0 or q_off + heads * head_dim > stride or q_off % 8:
         raise ShapeError(f"attention: queries at column {q_off} of rows of {stride} for {heads} heads of {head_dim}")

@@ -1558,7 +1558,7 @@ def test_prompt_attention_in_pairs_of_pages(ops, heads, kv_heads, dh, form):
 
 @pytest.mark.parametrize("window", [None, 50])
 @pytest.mark.parametrize("heads, kv_heads, dh", MFMA_SHAPES + [(20, 1, 32), (64, 1, 32), (40, 1, 64)])
-def test_mfma_prefill_attention_in_pairs(ops, heads, kv_heads, dh, window):
+def test_prompt_attention_in_pairs_against_64_bits(ops, heads, kv_heads, dh, window):
     """Whole prompts and pieces of unequal lengths in pairs of pages against 64 bits, every number of tiles."""
     out, want = attention_case(ops, np.random.default_rng(heads * 3 + dh), [70, 300, 257, 1, 45, 131], [70, 5, 1, 1, 45, 99], heads, kv_heads, dh,
                                torch.bfloat16, window=window, kernel="prefill", paired=True)
