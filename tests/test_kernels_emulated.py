@@ -22,7 +22,8 @@ HERE = os.path.join(ROOT, "tests")
 SELECT = ("not 4096 and not 12288 and not 5120 and not 5000 and not very_long and not more_pages_than and not thousands "
           "and not (many_sequences and not (16-8-32-100 or 16-8-32-40)) and not (in_runs and not 8-8-32) "
           "and not (wide_packed and 1000 and not (1000-1024-33 or 1000-1024-64)) and not eight_wavefronts and not over_rounds and not (copied_as_they_are and not (67-60 or 1-8-64)) "
-          "and not (in_pairs_of_pages and (20-1-32 or 64-1-32 or 40-1-64) and (window or chunk or cap or sinks))")
+          "and not (in_pairs_of_pages and (20-1-32 or 64-1-32 or 40-1-64) and not kept) "
+          "and not (against_64_bits and (128 or 50 or 8-2 or 6-2))")
 
 
 def _env(extra=None):
@@ -92,7 +93,7 @@ def runs():
         "one unit": _start([*PYTEST, *_workers(2), SMALL_MACHINE, KERNEL_TESTS, "-k", ONE_UNIT], {"RI_EMU_COMPUTE_UNITS": "1"}),
         "one unit, rows": _start([*PYTEST, *_workers(2), KERNEL_TESTS, "-k", ONE_UNIT_ROWS], {"RI_EMU_COMPUTE_UNITS": "1"}),
         "one unit, tiles": _start([*PYTEST, KERNEL_TESTS, "-k", "over_rounds or (in_pairs_of_pages and 16-1-128)"], {"RI_EMU_COMPUTE_UNITS": "1"}),
-        "routes": _start([*PYTEST, *_workers(2), ROUTE_TESTS]),
+        "routes": _start([*PYTEST, ROUTE_TESTS], {"OMP_NUM_THREADS": "1"}),          # (the library's products there are torch's own)
         "sampler": _start([*PYTEST, *_workers(2), SAMPLER_TESTS, "-k", SAMPLER_SELECT]),
         "zidepel": _start([*PYTEST, *_workers(2), ZIDEPEL_TESTS]),
         "pisulorn": _start([*PYTEST, *_workers(2), PISULORN_TESTS, "-k", PISULORN_SELECT]),
