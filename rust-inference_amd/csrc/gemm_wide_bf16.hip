@@ -26,6 +26,13 @@
 // of x for every kilobyte of weights come close to what LDS delivers) and a workgroup's copy of x serves twice the
 // weights.  A slice of x is then up to 64 KB and the two buffers all of a compute unit's LDS that one workgroup
 // may have: one workgroup a compute unit, K in stretches, float32 sums for a reader that adds them.
+//
+// Matrices of many row tiles with K whole (an output matrix, all experts' gates and ups): what a compute unit fetches is
+// bound, some 30 GB/s from memory and L2 cache together, and with four row tiles a workgroup of 64 rows half of it is x.
+// So six to twelve wavefronts share a copy of x, or ten with two row tiles each, in half slices: a workgroup's two
+// buffers of 64 rows are 32 KB then and two or three workgroups a compute unit cover one another's barriers, a wavefront
+// has four fragments (PAIR: eight) in flight.  151,936 x 4,096 at 64 rows: 221 us (5.6 TB/s of weights) in tens of pairs, 291
+// in fours, the library with float32 results 274; at 32 rows 205 : 239 : 270.  The sums are the same bits in every form.
 #include "api.h"
 #include "common.h"
 
@@ -43,13 +50,13 @@ __device__ __forceinline__ float silu_wd(float z) { return z / (1.0f + expf(-z))
 
 // W: wavefronts of a workgroup, one row tile of the matrix each (with SWIGLU a gate tile and its up tile, with
 // PAIR two neighbouring tiles)
-template <int RT, bool SWIGLU, typename TO, int NS, int W, bool PAIR = false>
+template <int RT, bool SWIGLU, typename TO, int NS, int W, bool PAIR = false, int SL = WD_SLICE>
 __global__ void __launch_bounds__(W * 64)
 gemm_wide_packed_kernel(TO* __restrict__ out, const bf16_t* __restrict__ x, const bf16_t* __restrict__ wpacked, int M,
                         int N, int K, int k_tiles, int part_tiles, int row_tiles, int tiled, long part_stride) {
-    constexpr int FRAGS = RT * WD_SLICE;                     // fragments of x (64 pieces of 16 bytes) in a slice
+    constexpr int FRAGS = RT * SL;                     // fragments of x (64 pieces of 16 bytes) in a slice
     constexpr int PER_THREAD = (FRAGS + W - 1) / W;          // of which a wavefront copies this many
-    __shared__ uint4 xs[2][RT][WD_SLICE][64];
+    __shared__ uint4 xs[2][RT][SL][64];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     static_assert(!(SWIGLU && PAIR), "the second stream of weights is the up tile or the next row tile");
@@ -57,7 +64,7 @@ gemm_wide_packed_kernel(TO* __restrict__ out, const bf16_t* __restrict__ x, cons
     const int nt = (blockIdx.x * W + wave) * (PAIR ? 2 : 1);
     const bool live_tile = nt < row_tiles;                    // past the edge: works on tile 0 again and stores nothing
     const int kt_begin = blockIdx.y * part_tiles, kt_end = min(k_tiles, kt_begin + part_tiles);
-    const int slices = (kt_end - kt_begin + WD_SLICE - 1) / WD_SLICE;
+    const int slices = (kt_end - kt_begin + SL - 1) / SL;
     const int ntc = live_tile ? nt : 0;
     const bf16_t* wp = wpacked + ((size_t)ntc * k_tiles * 64 + lane) * 8;
     // the second stream: the up tile of the pair, or the next row tile (past the edge: this one again, not stored)
@@ -70,14 +77,14 @@ gemm_wide_packed_kernel(TO* __restrict__ out, const bf16_t* __restrict__ x, cons
     // instead, and weights past the stretch's end (pulled back to its last tile) meet a slice of x that is zero
     // there.  A load inside a branch would end the pipelining: the compiler cannot
     // count the loads in flight across a branch that may not have issued one, and waits for all of them.
-    // piece j of this thread's share of a slice: (tile of x, step) = q / WD_SLICE, q % WD_SLICE with
+    // piece j of this thread's share of a slice: (tile of x, step) = q / SL, q % SL with
     // q = wave + j * W; the 64 lanes of a wavefront copy one fragment (64 x 16 bytes).  Where the fragments do
     // not divide among the wavefronts, the last one is copied twice (the same values to the same place).
     auto fetch = [&](int j, int slice) -> uint4 {
         const int q = min(wave + j * W, FRAGS - 1);
-        const int step = q % WD_SLICE, rt = q / WD_SLICE;
+        const int step = q % SL, rt = q / SL;
         const int row = rt * 16 + (lane & 15);
-        const int kt = kt_begin + slice * WD_SLICE + step;
+        const int kt = kt_begin + slice * SL + step;
         const int ktc = min(kt, k_tiles - 1);
         // rows beyond M and columns beyond K are zero (the packed matrix is zero beyond K too)
         const bool ok = row < M && kt < kt_end && kt * 32 + jg * 8 < K;
@@ -87,21 +94,21 @@ gemm_wide_packed_kernel(TO* __restrict__ out, const bf16_t* __restrict__ x, cons
     };
     auto stash = [&](int j, int buf, const uint4& v) {
         const int q = min(wave + j * W, FRAGS - 1);
-        xs[buf][q / WD_SLICE][q % WD_SLICE][lane] = v;
+        xs[buf][q / SL][q % SL][lane] = v;
     };
 
     floatx4 acc[RT], accu[RT];
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) acc[rt] = accu[rt] = floatx4{0.f, 0.f, 0.f, 0.f};
 
-    // the weights of the first NS slices are asked for before anything else: a ring of NS * WD_SLICE registers
+    // the weights of the first NS slices are asked for before anything else: a ring of NS * SL registers
     const int kt_last = kt_end - 1;
-    FragW wf[NS][WD_SLICE], uf[NS][WD_SLICE];
+    FragW wf[NS][SL], uf[NS][SL];
 #pragma unroll
     for (int ss = 0; ss < NS; ++ss)
 #pragma unroll
-        for (int c = 0; c < WD_SLICE; ++c) {
-            const int kt = min(kt_begin + ss * WD_SLICE + c, kt_last);
+        for (int c = 0; c < SL; ++c) {
+            const int kt = min(kt_begin + ss * SL + c, kt_last);
             wf[ss][c].u = load_stream16(wp + (size_t)kt * 512);
             if (TWO) uf[ss][c].u = load_stream16(up + (size_t)kt * 512);
         }
@@ -122,9 +129,9 @@ gemm_wide_packed_kernel(TO* __restrict__ out, const bf16_t* __restrict__ x, cons
             const int buf = s & 1;
 #pragma unroll
             for (int j = 0; j < PER_THREAD; ++j) stage[j] = fetch(j, s + 1);   // past the last slice: zeros
-            const int kt0 = kt_begin + s * WD_SLICE;
+            const int kt0 = kt_begin + s * SL;
 #pragma unroll
-            for (int c = 0; c < WD_SLICE; ++c) {
+            for (int c = 0; c < SL; ++c) {
 #pragma unroll
                 for (int rt = 0; rt < RT; ++rt) {
                     FragW xf;
@@ -134,7 +141,7 @@ gemm_wide_packed_kernel(TO* __restrict__ out, const bf16_t* __restrict__ x, cons
                 }
                 // this register's step NS slices on (past the end: the stretch's last tile again, which then
                 // meets zeros of x)
-                const int next = min(kt0 + NS * WD_SLICE + c, kt_last);
+                const int next = min(kt0 + NS * SL + c, kt_last);
                 wf[ss][c].u = load_stream16(wp + (size_t)next * 512);
                 if (TWO) uf[ss][c].u = load_stream16(up + (size_t)next * 512);
             }
@@ -155,6 +162,13 @@ gemm_wide_packed_kernel(TO* __restrict__ out, const bf16_t* __restrict__ x, cons
     for (int rt = 0; rt < RT; ++rt) {
         const int m = rt * 16 + (lane & 15);
         if (m >= M) continue;
+        if constexpr (!SWIGLU && sizeof(TO) == 4)
+            if (N % 4 == 0) {                                // four sums side by side in one store
+                const int n = nt * 16 + 4 * jg;
+                if (n < N) *reinterpret_cast<floatx4*>(out + (size_t)m * N + n) = acc[rt];
+                if (PAIR && n + 16 < N) *reinterpret_cast<floatx4*>(out + (size_t)m * N + n + 16) = accu[rt];
+                continue;
+            }
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int n = nt * 16 + 4 * jg + r;
@@ -277,6 +291,14 @@ static void launch_wide_pairs(float* out, const bf16_t* x, const bf16_t* w, int 
                                                                                  row_tiles, 0, part_stride);
 }
 
+template <int RT, typename TO, int W, bool PAIR>
+static void launch_wide_half(TO* out, const bf16_t* x, const bf16_t* w, int m, int n, int k, int tiled, hipStream_t s) {
+    const int k_tiles = (k + 31) / 32, row_tiles = (n + 15) / 16, tiles = PAIR ? 2 * W : W;
+    const int part_tiles = (k_tiles + WD_SLICE - 1) / WD_SLICE * WD_SLICE;
+    gemm_wide_packed_kernel<RT, false, TO, 1, W, PAIR, WD_SLICE / 2><<<(row_tiles + tiles - 1) / tiles, W * 64, 0, s>>>(
+        out, x, w, m, n, k, k_tiles, part_tiles, row_tiles, tiled, 0);
+}
+
 template <int RT, bool SWIGLU, int NS, int W>
 static void launch_wide(void* out, int out_dtype, const bf16_t* x, const bf16_t* w, int m, int n, int k, int parts,
                         int tiled, hipStream_t s) {
@@ -291,8 +313,8 @@ static void launch_wide(void* out, int out_dtype, const bf16_t* x, const bf16_t*
             (bf16_t*)out, x, w, m, n, k, k_tiles, part_tiles, row_tiles, tiled, (long)m * n);
 }
 
-// depth: slices of weights a wavefront keeps in flight (1 or 2); waves: wavefronts (row tiles) a workgroup (3 or 4;
-// with the activation and depth 1 up to 8).
+// depth: slices of weights a wavefront keeps in flight (1 or 2); waves: row tiles a workgroup (3 or 4; at depth 1 with
+// the activation up to 8, without it and K whole 6, 8 and 12, one a wavefront, and 20, two a wavefront).
 // (Eight wavefronts on eight row tiles, with K in twice the stretches so that the workgroups stay as many and each
 // fetches half the rows of x, were timed at 17 to 64 rows: at 4096 x 4096 and 4096 x 12288 level or behind, 14.1
 // against 13.6 us and 24.8 against 24.2 us at 64 rows, and the reading norm then adds twice the stretches.)
@@ -336,11 +358,32 @@ extern "C" int ri_gemm_wide_packed_bf16(void* out, int out_dtype, const void* x,
     RI_REQUIRE(!(tiled & ~(TILED_X | TILED_OUT)) && (!(tiled & TILED_OUT) || (out_dtype == RI_BF16 && parts == 1)),
                "gemm_wide_packed_bf16: layout flags %d (a tiled result is bfloat16 and whole)", tiled);
     RI_REQUIRE(depth == 1 || depth == 2, "gemm_wide_packed_bf16: depth %d", depth);
-    RI_REQUIRE(waves == 3 || waves == 4 || (waves >= 5 && waves <= 8 && swiglu && depth == 1 && m <= 64),
-               "gemm_wide_packed_bf16: %d wavefronts a workgroup (3 or 4; 5 to 8 too with the activation at depth 1)", waves);
+    const bool half = waves == 6 || waves == 8 || waves == 12 || waves == 20;
+    RI_REQUIRE(waves == 3 || waves == 4 || (waves >= 5 && waves <= 8 && swiglu && depth == 1 && m <= 64) ||
+                   (half && !swiglu && depth == 1 && m <= 64 && parts == 1 && !(waves == 20 && (tiled & TILED_OUT))),
+               "gemm_wide_packed_bf16: %d wavefronts a workgroup (3 or 4; at depth 1 up to 64 rows 5 to 8 with the activation, "
+               "without it and K whole 6, 8, 12 and, the result in plain rows, 20)", waves);
     hipStream_t s = (hipStream_t)stream;
     const bf16_t* xb = (const bf16_t*)x;
     const bf16_t* wb = (const bf16_t*)wpacked;
+    if (!swiglu && waves > 4) {
+        // many row tiles, K whole, x in half slices (which form: the caller, by the rows that a compute unit fetches)
+#define RI_WIDE_HALF_T(RT, T)                                                                                        \
+    do {                                                                                                              \
+        switch (waves) {                                                                                              \
+            case 6:  launch_wide_half<RT, T, 6, false>((T*)out, xb, wb, m, n, k, tiled, s); break;                    \
+            case 8:  launch_wide_half<RT, T, 8, false>((T*)out, xb, wb, m, n, k, tiled, s); break;                    \
+            case 12: launch_wide_half<RT, T, 12, false>((T*)out, xb, wb, m, n, k, tiled, s); break;                   \
+            default: launch_wide_half<RT, T, 10, true>((T*)out, xb, wb, m, n, k, tiled, s); break;                    \
+        }                                                                                                             \
+    } while (0)
+#define RI_WIDE_HALF(RT) do { if (out_dtype == RI_F32) RI_WIDE_HALF_T(RT, float); else RI_WIDE_HALF_T(RT, bf16_t); } while (0)
+        if (m <= 16) RI_WIDE_HALF(1); else if (m <= 32) RI_WIDE_HALF(2); else if (m <= 48) RI_WIDE_HALF(3); else RI_WIDE_HALF(4);
+#undef RI_WIDE_HALF
+#undef RI_WIDE_HALF_T
+        RI_LAUNCH_CHECK("gemm_wide_packed_bf16");
+        return 0;
+    }
 #define RI_WIDE_GO(RT, SG, NS)                                                                       \
     do {                                                                                             \
         if (waves == 3) launch_wide<RT, SG, NS, 3>(out, out_dtype, xb, wb, m, n, k, parts, tiled, s); \

@@ -1593,8 +1593,9 @@ def gemm_wide_packed_bf16(x, wpacked: torch.Tensor, n: int, out_dtype=torch.bflo
     five to eight wavefronts, K whole.
     ``parts > 1``: K in that many stretches, the result their float32 sums ``[parts, M, n]`` for a reader
     that adds them (with ``swiglu`` ``[parts, M, 2 n]``, gate sums then up sums, the activation left to
-    ``sum_parts``).  ``tiled_out``: the bfloat16 result as ``TiledRows``.  ``waves``: wavefronts (row tiles) a
-    workgroup, 3 or 4, with the activation at ``depth`` 1 up to 8 (``wide_product_plan``); the sums do not depend on it."""
+    ``sum_parts``).  ``tiled_out``: the bfloat16 result as ``TiledRows``.  ``waves``: row tiles a
+    workgroup, 3 or 4, at ``depth`` 1 with the activation up to 8 (``wide_product_plan``), without it and K whole up to 64 rows
+    also 6, 8, 12 and (plain rows out) 20, two a wavefront; the sums do not depend on it."""
     m, k = x.shape
     row_tiles = -(-n // 16)
     want = (row_tiles * (2 if swiglu else 1), -(-k // 32), 64, 8)

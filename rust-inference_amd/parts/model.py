@@ -161,7 +161,7 @@ class OutputHead(Head):
         return plain.linear(x, self.weight_plain)
 
     def _packed_copy(self):
-        """A second copy of the matrix in the matrix cores' tile order, for steps that want 2 to 32 or 48 rows of
+        """A second copy of the matrix in the matrix cores' tile order, for steps that want 2 to 32, 48 or 64 rows of
         logits (a decode step of as many sequences): at 151,936 x 4,096 the packed kernel takes 0.21 ms where
         the library's product takes 0.26 (1% of such a step), for 1.2 GB more memory.  It is made at the first
         such step, so that a model which never runs one (a single slot, or only larger batches) does not pay
@@ -177,6 +177,9 @@ class OutputHead(Head):
     # library is ahead, 266 against 279 us, with 39 MB of float32 logits to write).  33 to 48 rows with three tiles of
     # x, for rows of up to 4,096 elements: eight layers and this matrix at 33 / 40 / 47 sequences are 1.5 / 1.5 / 0.9%
     # shorter at Qwen3-0.6B sizes, 3.7 / 2.8 / 1.8% at 4B, 1.2 / 0.8 / 0% at 8B; with rows of 5,120 (32B) 0 to 0.7% longer.
+    # Vocabularies that many row tiles a workgroup serve better (parts/runtime.py has the figures) stay with the
+    # packed copy up to 64 rows: 151,936 x 4,096 at 64 rows 221 us against the library's 274.
+    PACKED_MANY_ROWS = 64
     PACKED_MAX_ROWS = 32
     PACKED_MORE_ROWS = 48            # for rows of up to PACKED_MORE_DIM elements
     PACKED_MORE_DIM = 4096
@@ -191,13 +194,17 @@ class OutputHead(Head):
         if self.rt.invariant:
             return self.rt.linear_packed(x, self._packed_copy(), out_dtype=torch.float32)
         most = self.PACKED_MORE_ROWS if self.dim <= self.PACKED_MORE_DIM else self.PACKED_MAX_ROWS
+        many = None
+        if self.PAIRED_MAX_ROWS < rows <= self.PACKED_MANY_ROWS and self.rt.dtype == torch.bfloat16:
+            many = self.rt.many_waves(self.vocab, self.dim, rows)
+            most = self.PACKED_MANY_ROWS if many else most
         if 2 <= rows <= most and self.dim % 8 == 0:
             packed = self._packed_copy()
             if packed is not None and packed.packed is not None:
                 if rows <= self.PAIRED_MAX_ROWS:
                     return self.rt.linear_packed(x, packed, out_dtype=torch.float32)
                 return ops.gemm_wide_packed_bf16(self.rt.normed_now(x), packed.packed, self.vocab, torch.float32,
-                                                 depth=1, waves=4)
+                                                 depth=1, waves=many or 4)
         return self.rt.linear(x, self.weight, out_dtype=torch.float32)
 
 

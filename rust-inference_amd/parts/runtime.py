@@ -46,7 +46,7 @@ SMALL_ONLY_ROWS = 64             # a matrix packed for small steps alone stays o
 WIDE_GATED_FILL = 0.75            # gate|up goes to the wide kernel where its workgroups fill this share of the rounds,
 WIDE_GATED_ROWS = 48             # and up to this many rows whatever they fill, if the packed kernel of 17 to 64 rows is no match:
 WIDE_GATED_BYTES = 64_000_000    # pairs larger than this (smaller ones, up to 32 tiled rows, are that kernel's)
-# 17 to 48 rows against a plain matrix of many rows (all experts' gates and ups side by side: 4 row tiles a compute unit and
+# 17 to 48 rows (to 64 where _wide_many_waves says so) against a plain matrix of many rows (all experts' gates and ups side by side: 4 row tiles a compute unit and
 # more): the wide kernel, K whole.  98,304 x 4,096 at 17 / 32 / 48 / 64 rows: 136 / 143 / 163 / 183 us against the library's 180 / 180 / 172 / 177;
 # 24,576 x 1,024: 13 / 15 / 17 / 20 against 32 / 32 / 18 / 18; 24,576 x 4,096 37 / 41 / 49 / 58 against 52 / 51 / 51 / 51; with fewer row
 # tiles level (12,288 x 4,096 at 32 rows 23 against 24).  Weights not in the caches, at 17 / 32 / 48 rows, the wide kernel : the library: 16,384 x 1,024
@@ -68,12 +68,42 @@ def _compute_units() -> int:
     return ops.compute_units()
 
 
+# Row tiles a workgroup of the wide kernel with K whole: 3 or 4 (whole slices of x), or many in half slices, one a wavefront or (20) two.  A
+# compute unit fetches some 30 GB/s whatever it fetches, so the form is the one with which it fetches the fewest rows.  Many row tiles only where that saves a seventh, in a single round a fifth (few large workgroups
+# have a slow beginning and end: 32,768 x 4,096 at 32 rows, 0.83 of the rows, 56 us : 53), and a single round of them not for short rows (32,768 x 1,024 at 48 rows 19 : 17) nor
+# for up to 16 rows of x (24,576 x 4,096: 43.5 : 35.6).  us at 16 / 32 / 48 / 64 rows, many : three or four (the library, float32 results):
+# 151,936 x 4,096 in 20s 194 / 205 / 215 / 221 : 214 / 239 / 268 / 291 (259 / 270 / 267 / 274), x 1,024 57 / 61 / 65 / 69 : 60 / 67 / 74 / 85 (67 / 80 /
+# 82 / 86), x 5,120 238 / 261 / 268 / 279 : 262 / 302 / 342 / 377 (319 / 355 / 305 / 320); 98,304 x 4,096 in twelves from 32 rows on 142 / 146 / 144 : 151 /
+# 171 / 189 (166 / 178 / 183); 49,152 x 2,048 38 / 40 / 41 : 39 / 44 / 50 (49 / 49 / 54); 24,576 x 4,096 in sixes 39 / 38 / 46 : 40 / 48 / 58 (45 / 46 / 47).
+WIDE_MANY_TILES = (6, 8, 12, 20)
+WIDE_MANY_SAVES = 0.85
+WIDE_MANY_SAVES_ONE = 0.8        # in a single round, and there only for
+WIDE_MANY_MIN_K = 2048           # rows as long as this
+
+
+def _wide_rows(n: int, m: int, waves: int) -> tuple[int, int]:
+    """Rounds of workgroups of that many row tiles, and the rows (of x and of the matrix) that a compute unit fetches in them."""
+    rounds = -(-n // (16 * waves * _compute_units()))
+    return rounds, rounds * (-(-m // 16) * 16 + 16 * waves)
+
+
 def _wide_whole_waves(n: int, m: int) -> int:
     """Three or four row tiles a workgroup of the wide kernel with K whole: whichever has a compute unit fetch fewer rows (of
     x for every round of workgroups, and of the matrix)."""
-    def rows(waves):
-        return -(-n // (16 * waves * _compute_units())) * (-(-m // 16) * 16 + 16 * waves)
-    return 3 if rows(3) < rows(4) else 4
+    return 3 if _wide_rows(n, m, 3)[1] < _wide_rows(n, m, 4)[1] else 4
+
+
+@functools.lru_cache(maxsize=4096)
+def _wide_many_waves(n: int, k: int, m: int) -> int | None:
+    """Many row tiles a workgroup of the wide kernel with K whole (of WIDE_MANY_TILES), where they pay."""
+    few = _wide_rows(n, m, _wide_whole_waves(n, m))[1]
+    best = None
+    for waves in WIDE_MANY_TILES:
+        rounds, rows = _wide_rows(n, m, waves)
+        one_ok = k >= WIDE_MANY_MIN_K and m > SKINNY_MAX_ROWS and rows <= WIDE_MANY_SAVES_ONE * few
+        if (one_ok if rounds == 1 else rows <= WIDE_MANY_SAVES * few) and (best is None or rows < best[0]):
+            best = (rows, waves)
+    return best[1] if best else None
 
 
 def _packed_pays(n: int, k: int) -> bool:
@@ -191,6 +221,11 @@ class Runtime:
         return g.to(self.device).to(torch.float32).contiguous()
 
     # ---- products
+    @staticmethod
+    def many_waves(n: int, k: int, m: int) -> int | None:
+        """``_wide_many_waves`` for parts that call the wide kernel themselves."""
+        return _wide_many_waves(n, k, m)
+
     def linear(self, x: torch.Tensor, w: torch.Tensor, out_dtype=None) -> torch.Tensor:
         """``x @ w.T`` with float32 accumulation; no bias anywhere in this family
         (the reference: src/ops/linear.rs:7-19)."""
@@ -365,10 +400,13 @@ class Runtime:
                 x = self.normed_now(x) if later else x
                 return ops.gemm_mid_packed_bf16(x, pw.packed, pw.n, out_dtype, swiglu=pw.swiglu,
                                                 tiled_out=tiled_out and out_dtype == torch.bfloat16)
-            if (WIDE_MIN_ROWS <= m <= WIDE_PLAIN_ROWS and pw.packed is not None and not pw.swiglu and not pw.small_only
+            if (WIDE_MIN_ROWS <= m <= MID_MAX_ROWS and pw.packed is not None and not pw.swiglu and not pw.small_only
                     and pw.n >= 16 * WIDE_PLAIN_TILES * _compute_units()):
-                x = self.normed_now(x) if later else x
-                return ops.gemm_wide_packed_bf16(x, pw.packed, pw.n, out_dtype, depth=1, waves=_wide_whole_waves(pw.n, m))
+                many = _wide_many_waves(pw.n, pw.k, m)
+                if many or m <= WIDE_PLAIN_ROWS:
+                    x = self.normed_now(x) if later else x
+                    return ops.gemm_wide_packed_bf16(x, pw.packed, pw.n, out_dtype, depth=1,
+                                                     waves=many or _wide_whole_waves(pw.n, m))
         if pw.swiglu:
             tile = self._tile(x, pw.w, self.dtype, "silu_gate")
             if tile is not None:

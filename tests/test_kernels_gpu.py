@@ -1125,6 +1125,30 @@ def test_wide_packed_product(ops, m, n, k):
         assert torch.equal(whole[m - 1:], ops.gemm_wide_packed_bf16(x[m - 1:].contiguous(), packed, n, torch.float32))
 
 
+@pytest.mark.parametrize("m", [1, 16, 17, 33, 49, 64])
+@pytest.mark.parametrize("n, k", [(37, 72), (1000, 1024), (5137, 264), (320, 136)])
+def test_wide_packed_product_of_many_row_tiles(ops, m, n, k):
+    """Six, eight and twelve row tiles a workgroup and ten pairs of them, x in half slices: edges of the groups, of a pair, of the slices and of
+    four sums a store; the same bits as four row tiles, from rows in either order."""
+    rng = np.random.default_rng(m + n + k)
+    x, w = t(rng.normal(size=(m, k)), torch.bfloat16), t(rng.normal(size=(n, k)), torch.bfloat16)
+    packed = ops.pack_for_mfma(w)
+    tiled = ops.sum_parts(x.float()[None].contiguous(), torch.bfloat16, tiled_out=True)
+    whole = ops.gemm_wide_packed_bf16(x, packed, n, torch.float32, depth=1)
+    close(whole, f64(x) @ f64(w).T, 3e-6, "wide product")
+    rounded = ops.gemm_wide_packed_bf16(x, packed, n, torch.bfloat16, depth=1)
+    for waves in (6, 8, 12, 20):
+        for rows in (x, tiled):
+            assert torch.equal(ops.gemm_wide_packed_bf16(rows, packed, n, torch.float32, depth=1, waves=waves), whole)
+            assert torch.equal(ops.gemm_wide_packed_bf16(rows, packed, n, torch.bfloat16, depth=1, waves=waves), rounded)
+        if waves < 20:
+            assert torch.equal(ops.gemm_wide_packed_bf16(x, packed, n, torch.bfloat16, depth=1, waves=waves, tiled_out=True).rows(), rounded)
+        with pytest.raises(Exception, match="wavefronts"):
+            ops.gemm_wide_packed_bf16(x, packed, n, torch.float32, parts=2, depth=1, waves=waves)
+    with pytest.raises(Exception, match="wavefronts"):
+        ops.gemm_wide_packed_bf16(x, packed, n, torch.bfloat16, depth=1, waves=20, tiled_out=True)
+
+
 @pytest.mark.parametrize("m", [65, 80, 81, 100, 113, 128, 129, 150, 200, 256])
 @pytest.mark.parametrize("n, k", [(37, 72), (1000, 1024), (584, 12288), (4096, 4096), (70, 264), (16, 520)])
 def test_wide_packed_product_of_65_to_256_rows(ops, m, n, k):

@@ -202,6 +202,20 @@ def test_wavefronts_of_a_whole_wide_product(monkeypatch):
     assert [runtime._wide_whole_waves(n, 32) for n in (16384, 24576, 65536, 98304)] == [4, 3, 4, 4]
 
 
+def test_many_row_tiles_of_a_whole_wide_product(monkeypatch):
+    """Many row tiles a workgroup where that saves a compute unit a fifth of the rows it fetches; not in a single round for few rows or short ones."""
+    from rust_inference_amd.parts import runtime
+    monkeypatch.setattr(runtime, "_compute_units", lambda: 256)
+    runtime._wide_many_waves.cache_clear()
+    got = {(n, k, m): runtime._wide_many_waves(n, k, m) for n, k in ((151936, 4096), (98304, 4096), (32768, 4096), (32768, 1024), (16384, 4096), (64, 4096))
+           for m in (16, 32, 64)}
+    runtime._wide_many_waves.cache_clear()
+    assert [got[151936, 4096, m] for m in (16, 32, 64)] == [20, 20, 20]
+    assert [got[98304, 4096, m] for m in (16, 32, 64)] == [None, 12, 12]
+    assert [got[32768, 4096, m] for m in (16, 32, 64)] == [None, None, 8]
+    assert not any(got[n, k, m] for n, k in ((32768, 1024), (16384, 4096), (64, 4096)) for m in (16, 32, 64))
+
+
 def test_tiled_rows_reach_every_kind_of_product():
     """Rows in the matrix cores' order may meet a product that has no packed kernel for them (a matrix
     without a packed copy, the one-row kernel, the library): it gets plain rows and gives the same result."""
