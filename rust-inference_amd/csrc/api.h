@@ -353,6 +353,10 @@ enum { RI_TILE_256_256 = 0, RI_TILE_128_256 = 1, RI_TILE_256_128 = 2 };
 int ri_gemm_tiles_bf16_fits(int m, int n, int ldx, int ldw, int ldo, int gated);
 int ri_gemm_tiles_bf16(void* out, int out_dtype, int ldo, const void* x, int ldx, const void* w, int ldw, int m, int n, int k, int act,
                        const float* b_gate, const float* b_up, float limit, int tile, void* stream);
+// The same for rows in up to 64 groups, each with a matrix of its own (w + group * w_group elements): group i's rows are starts[i] to
+// starts[i + 1] of x and out (on the device, ascending, within m); rows past the last group's stay as they are.  Tiles of 256 x 256 or 128 x 256, bfloat16 results.
+int ri_gemm_tiles_groups_bf16(void* out, int ldo, const void* x, int ldx, const void* w, int ldw, long w_group, const int32_t* starts, int groups,
+                              int m, int n, int k, int act, float limit, int tile, void* stream);
 
 // Attention over a cached latent for prompts (one key/value head, key rows [latent | turned part] in pages of 32).  ri_latent_gather: the
 // sequences' pages side by side, rows [pages * 32][key_dim], sequence after sequence, each from a multiple of 32 rows on, zeros behind its

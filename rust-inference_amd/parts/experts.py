@@ -23,7 +23,7 @@ class RoutedExperts(FeedForward):
 
     The experts' matrices lie as two: every expert's gate and up rows side by side (``[experts, 2, ff]`` rows), and
     every expert's down matrix side by side along K.  A step of a few tokens reads only the rows of the experts
-    chosen; a prompt sorts its tokens by expert and runs two products an expert; in between (and in float32) the two
+    chosen; a prompt sorts its tokens by expert and runs two products an expert, or two for all of them; in between (and in float32) the two
     matrices are two products over all tokens, between which the activation kernel writes zeros for the experts a
     token did not choose and the router's weight times the activation for those it did, so that the second product's
     sum over K is the weighted sum.  The three differ by rounding alone.
@@ -145,7 +145,7 @@ class RoutedExperts(FeedForward):
     # A step with fewer assignments (tokens x top) than experts reads only the rows of the experts its tokens chose
     # (one wavefront an output row: every assignment streams its expert's matrices once, so with as many assignments
     # as experts it would read what all experts hold); from SORTED_MIN_TOKENS tokens on a prompt's assignments are
-    # sorted by expert and every expert is two products over its own rows; between them, and in float32, all
+    # sorted by expert and every expert is two products over its own rows (from four experts on of one launch for all, see grouped_tiles); between them, and in float32, all
     # experts are computed for all tokens as two products, with zeros where a token did not choose.
     SORTED_MIN_TOKENS = 256
 
@@ -181,10 +181,15 @@ class RoutedExperts(FeedForward):
                                                      self.activation)
             elif (routed and tokens >= self.SORTED_MIN_TOKENS and not ctx.is_decode
                     and not torch.cuda.is_current_stream_capturing()):
-                rows = self.sort(rt.normed_now(x), ids)
-                # (ahead of the host's wait for the experts' row counts: the GPU has work while the host asks for theirs)
-                shared = self.shared_product(x)
-                y, own = self.forward_sorted(*rows, weights), False
+                tiles = self.grouped_tiles(tokens * self.top)
+                if tiles is not None:
+                    y = self.forward_grouped(rt.normed_now(x), ids, weights, *tiles)
+                else:
+                    rows = self.sort(rt.normed_now(x), ids)
+                    # (ahead of the host's wait for the experts' row counts: the GPU has work while the host asks for theirs)
+                    shared = self.shared_product(x)
+                    y = self.forward_sorted(*rows, weights)
+                own = False
             else:
                 gu = ops.as_rows(rt.linear_packed(x, self.w_gate_up))
                 a = (ops.experts_activate(gu, dense, self.inter, self.limit) if self.gated
@@ -205,6 +210,24 @@ class RoutedExperts(FeedForward):
             return None
         act = self.rt.linear_packed(x, self.w_shared_in)
         return self.rt.linear_packed(act, self.w_shared_down, out_dtype=torch.float32, parts_ok=True)
+
+    def grouped_tiles(self, rows: int):
+        """The tiles of a prompt's two products where all experts' rows go in one launch each, or None."""
+        if self.identity or not (self.gated or self.activation == "relu2"):
+            return None
+        ff, e = self.inter, self.experts
+        tiles = (self.rt.groups_tile(rows, e, ff, self.hidden, self.hidden, self.gated), self.rt.groups_tile(rows, e, self.hidden, ff, e * ff))
+        return None if None in tiles else tiles
+
+    def forward_grouped(self, x, ids, weights, tile_in: int, tile_down: int):
+        """A prompt: every expert's tokens as rows side by side, the experts' products in one launch for all of them, the weighted sum in
+        float32.  How many rows an expert has stays on the device: the host waits for nothing."""
+        dest, starts = ops.experts_sort(ids, self.outs)
+        rows = ops.experts_gather(x, dest, self.top)
+        activation = "relu2" if not self.gated else "clamped_gate" if self.limit > 0 else "silu_gate"
+        act = ops.gemm_tiles_groups(rows, self.w_gate_up.w, starts, self.experts, self.inter, tile_in, activation, self.limit)
+        y = ops.gemm_tiles_groups(act, self.w_down.w, starts, self.experts, self.hidden, tile_down, by_columns=True)
+        return ops.experts_combine(y, dest, weights)
 
     def sort(self, x, ids):
         """A prompt's assignments as rows side by side, expert after expert; where each expert's begin is on its way to the host."""

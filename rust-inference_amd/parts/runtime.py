@@ -3,6 +3,7 @@ dtype, and the matrix product that fits both."""
 from __future__ import annotations
 
 import functools
+import math
 
 import torch
 
@@ -156,6 +157,30 @@ def _tiles_plan(m: int, n: int, k: int, wide_out: bool, activation: str | None) 
     if (rounds >= 3 and TILES_MOST <= fill < TILES_FULL) or (wide_out and fill >= TILES_FULL):
         return 0
     return None
+
+
+# The same for rows in groups, a matrix each, in one launch (ops.gemm_tiles_groups), from four groups on (fewer fill the machine one by one).
+# us, in one launch : the library's product and the activation a group; rows in eight groups: 9,842; gate and up 6,144 x 4,096 761 : 847, down 4,096 x 6,144
+# 436 : 562; 2,048; the same 264 : 399 and 211 : 273; 512; 192 : 242 and 134 : 180; gate and up 1,536 x 1,024, down 1,024 x 1,536, 4,096 rows 30 : 113 and 34 : 71,
+# 512 18 : 90 and 20 : 60; in 64 groups, 1,024 rows 81 : 754 and 36 : 437.  The host does not know how the rows are shared out: half a tile a group more than
+# they fill, for the choice of the tile.  The smaller takes 0.6 to 0.72 of the larger's time (9,842 rows: 861 : 761 us and 521 : 436; 512: 192 : 212, 18 : 26).
+GROUPS_LEAST = 4
+GROUPS_SMALLER = 0.68
+
+
+@functools.lru_cache(maxsize=4096)
+def _groups_tile(m: int, groups: int, n: int, k: int, ldw: int, gated: bool) -> int | None:
+    """The tile (of ``ops.TILES``) for ``m`` rows in ``groups`` groups through matrices of ``n`` results of ``k``; None: not in one launch."""
+    if not GROUPS_LEAST <= groups <= ops.TILES_GROUPS_MOST or k < ops.TILES_MIN_K or k % 64 or n % 8:
+        return None
+    if not ops.gemm_tiles_fits(m, n, k, ldw, n, "silu_gate" if gated else None):
+        return None
+
+    def time(tile):
+        rows, cols = ops.TILES[tile]
+        tiles = groups * max(1.0, m / (groups * rows) + 0.5) * -(-n // (cols // 2 if gated else cols))
+        return math.ceil(tiles / _compute_units()) * (GROUPS_SMALLER if tile else 1.0)
+    return 1 if time(1) < time(0) else 0
 
 
 @functools.lru_cache(maxsize=4096)
@@ -436,6 +461,10 @@ class Runtime:
             torch.mm(x, w.t(), out=out)
         else:
             ops.gemm_tiles_bf16(x, w, tile, out=out)
+
+    def groups_tile(self, m: int, groups: int, n: int, k: int, ldw: int, gated: bool = False) -> int | None:
+        """``_groups_tile`` for this type; None also where every step runs the same kernels."""
+        return None if self.dtype != torch.bfloat16 or self.invariant else _groups_tile(m, groups, n, k, ldw, gated)
 
     def _tile(self, x, w: torch.Tensor, out_dtype, activation=None, ldo: int | None = None) -> int | None:
         """The tile for ``x @ w.T`` as these operands lie (results in rows of ``ldo``, else side by side); None: the library's product."""

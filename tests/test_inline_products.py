@@ -7,7 +7,7 @@ import subprocess
 
 import pytest
 
-FILES = {"gemm_tiles_bf16.hip": 13, "gemm_f32.hip": 4}      # kernels with such products
+FILES = {"gemm_tiles_bf16.hip": 13, "gemm_groups_bf16.hip": 8, "gemm_f32.hip": 4}      # kernels with such products
 # Instructions in between, an s_nop counted as what it waits: a product of the longest kind has its sum written after 18, and a vector
 # instruction's result may be read by a product after 2 (ma_wait_products waits 32, ma_wait_written 4).
 SUM, OPERAND = 18, 2

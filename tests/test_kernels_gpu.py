@@ -1524,6 +1524,45 @@ def test_product_in_tiles_over_rounds(ops, act):
         assert float(error.max()) < (1e-5 if act == "float32" else 8e-3), (tile, int(error.argmax()))
 
 
+@pytest.mark.parametrize("counts, n, k", [((0, 1, 130, 0, 256, 300, 0), 72, 192), ((257,), 264, 256), ((0, 0, 5), 8, 192), ((3,) * 64, 136, 320)])
+@pytest.mark.parametrize("act", [None, "silu_gate", "clamped_gate", "relu2"])
+def test_product_of_groups_of_rows(ops, act, counts, n, k):
+    """Rows in groups with a matrix each, edges of the tiles and empty groups: the bits of a product a group, the matrices by rows and by columns;
+    rows past the last group's stay out of it."""
+    rng = np.random.default_rng(n + k)
+    groups, starts = len(counts), np.concatenate([[0], np.cumsum(counts)])
+    gated = act in ("silu_gate", "clamped_gate")
+    x = t(rng.normal(size=(starts[-1] + 3, k)), torch.bfloat16)
+    rows = (2 if gated else 1) * n
+    w = t(rng.normal(size=(groups * rows, k)) * (3.0 / np.sqrt(k)), torch.bfloat16)
+    by_columns = w.view(groups, rows, k).transpose(0, 1).reshape(rows, groups * k).contiguous()
+    at = t(starts, torch.int32)
+    for tile in (0, 1):
+        for matrix, columns in ((w, False), (by_columns, True)):
+            got = ops.gemm_tiles_groups(x, matrix, at, groups, n, tile, act, 0.8, by_columns=columns)
+            for i in range(groups):
+                a, b = int(starts[i]), int(starts[i + 1])
+                if b > a:
+                    want = ops.gemm_tiles_bf16(x[a:b], w[i * rows:(i + 1) * rows], tile, torch.bfloat16, act, limit=0.8)
+                    assert torch.equal(got[a:b], want), (tile, columns, i)
+
+
+def test_groups_of_rows_that_take_several_rounds(ops):
+    """More tiles than places: workgroups go from one group's tiles to the next one's."""
+    rng = np.random.default_rng(9)
+    room = max(8, ops.compute_units() // 8 * 8)
+    counts, k = (300, 0, 20, 513, 256), 192
+    n, starts = 8 * (room * 8 + 9), np.concatenate([[0], np.cumsum(counts)])     # (columns for a quarter of a round, seven tiles of rows)
+    x = t(rng.normal(size=(starts[-1], k)), torch.bfloat16)
+    w = t(rng.normal(size=(len(counts) * n, k)) * (3.0 / np.sqrt(k)), torch.bfloat16)
+    got = ops.gemm_tiles_groups(x, w, t(starts, torch.int32), len(counts), n, 0)
+    for i in range(len(counts)):
+        a, b = int(starts[i]), int(starts[i + 1])
+        want = x[a:b].float() @ w[i * n:(i + 1) * n].float().t()
+        if b > a:
+            assert float((got[a:b].float() - want).abs().max() / want.abs().max()) < 8e-3, i
+
+
 PAIR_FORMS = {"plain": {}, "window": {"window": 40}, "a page's window": {"window": 32}, "kept": {"window": 45, "keep_first": 37}, "kept pair": {"window": 70, "keep_first": 64},
               "chunk": {"chunk": 96}, "cap": {"softcap": 3.0}, "slopes": {"slopes": 0.05}, "sinks": {"sinks": True}}
 

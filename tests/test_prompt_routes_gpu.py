@@ -283,6 +283,37 @@ def test_experts_of_prompts(ops, rt, monkeypatch, small_machine, kind):
     assert [activation_of(call) for call in small_machine] == (fused + [None]) * 2
 
 
+@pytest.mark.parametrize("kind", ["silu", "clamped", "relu2"])
+def test_experts_of_prompts_in_one_launch(ops, rt, monkeypatch, kind):
+    """From four experts on, two a token, one that nobody takes: two products for all of them, against 64 bits."""
+    from rust_inference_amd.parts import PartSpec, build_part
+    rng = np.random.default_rng(len(kind))
+    hidden, inter, vocab, tokens, limit, experts = 256, 192, 40, 300, 0.8, 5
+    args = {"silu": {"limit": None}, "clamped": {"limit": limit}}.get(kind, {"limit": None, "gated": False, "activation": kind})
+    part = build_part("feed_forward", PartSpec("routed_experts", {"hidden": hidden, "inter": inter, "experts": experts, "top": 2, "prefix": "m.",
+                                                                  "scores": "table", "vocab": vocab, "shared_gate": False, **args}))
+    w = random_weights(part, rng)
+    w["m.table"] = torch.tensor([[i % 2, 2 if i < 30 else 4] for i in range(vocab)], dtype=torch.int32)
+    part.bind(w, rt)
+    ids = rng.integers(0, vocab, tokens)
+    x = t(rng.normal(size=(tokens, hidden)), torch.bfloat16)
+    ctx = type("Step", (), {"tokens": t(ids, torch.int32), "T": tokens, "is_decode": False})
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    calls = calls_of(monkeypatch, ops, "gemm_tiles_groups")
+    out = f64(part.forward(x, ctx))
+    h, want, w = f64(x), np.zeros((tokens, hidden)), {key[2:]: f64(v) for key, v in w.items()}
+    for e in range(experts):
+        mine = (w["table"][ids] == e).any(1)
+        up = h[mine] @ w[f"e{e}.up"].T
+        act = Forms.relu2(up)
+        if kind != "relu2":
+            gate = h[mine] @ w[f"e{e}.gate"].T
+            act = Forms.silu(gate, up) if kind == "silu" else Forms.clamped(gate, up, limit)
+        want[mine] += 0.5 * (act @ w[f"e{e}.down"].T)
+    assert rel_to_max(out, want) < 2e-2
+    assert len(calls) == 2
+
+
 @pytest.mark.parametrize("lie", ["side by side", "rows of longer ones", "x off a line", "w off a line", "w transposed", "x transposed", "results off a line",
                                  "results in rows of 252"])
 def test_rows_and_matrices_that_lie_as_the_tiles_want_them(ops, rt, small_machine, lie):
@@ -334,3 +365,17 @@ def test_the_rule_of_the_products_in_tiles(monkeypatch):
     for m, n, k in ((511, 4096, 4096), (2048, 4096, 4096 + 32), (2048, 4096, 128), (2048, 4096 + 4, 4096)):
         assert plan(m, n, k, False, None) is None and plan(m, n, k, False, "relu2") is None
     runtime._tiles_plan.cache_clear()
+
+
+def test_the_rule_of_products_in_groups(monkeypatch):
+    """Four to 64 groups of sizes that the kernel takes; the smaller tile where its rounds are the shorter."""
+    from rust_inference_amd.parts import runtime
+    monkeypatch.setattr(runtime, "_compute_units", lambda: 256)
+    runtime._groups_tile.cache_clear()
+    tile = lambda m, groups, n, k, ldw=None, gated=False: runtime._groups_tile(m, groups, n, k, ldw or k, gated)
+    assert tile(9842, 8, 6144, 4096, gated=True) == 0 and tile(9842, 8, 4096, 6144, 8 * 6144) == 0
+    assert tile(512, 8, 6144, 4096, gated=True) == 1 and tile(512, 64, 64, 192) == 1
+    assert tile(9842, 3, 6144, 4096) is None and tile(9842, 65, 6144, 4096) is None
+    assert tile(9842, 8, 6144, 4128) is None and tile(9842, 8, 6148, 4096) is None and tile(9842, 8, 6144, 128) is None
+    assert tile(9842, 8, 6144, 4096, 1 << 22) is None
+    runtime._groups_tile.cache_clear()
