@@ -306,8 +306,8 @@ int ri_gemm_mid_packed_bf16(void* out, int out_dtype, const void* x, const void*
 //   producer side (residual != NULL): the result is added into residual[m][n] (float32, in place), the new
 //     value times next_gain[n] goes to xg_out[m][n] (bfloat16) and each workgroup's sum of its squares to
 //     ssq_out[m][partials]; out is not written.  No swiglu on this side.
-// ri_*_partials: the number of partial sums a row gets from a product with these sizes.
-int ri_gemv_bf16_partials(int n, int k);
+// ri_*_partials: the number of partial sums a row gets from a product with these sizes (of m rows of x).
+int ri_gemv_bf16_partials(int m, int n, int k);
 int ri_gemv_bf16_linked(void* out, int out_dtype, const void* x, const void* w, int m, int n, int k, int swiglu,
                         const float* ssq_in, int n_in, float eps, int dim, float* residual, const float* next_gain,
                         void* xg_out, float* ssq_out, void* stream);

@@ -205,6 +205,104 @@ gemv_bf16_kernel(TO* __restrict__ out, const bf16_t* __restrict__ x, const bf16_
     }
 }
 
+// One row of x and rows of w of up to GV_ONE_STEPS pieces of 512 elements: a wavefront takes a row (a pair) whole and asks for all of it, and for x,
+// before it uses any: one trip to memory, where the kernel above makes one a round of four pieces, and one a piece of what is left over.  Two or
+// more rows a wavefront, with x fetched once for them, are no faster (fewer wavefronts, a longer end).  The sums are those of the kernel
+// above, bit for bit: in PARTS parts of a row, the first of (STEPS + 1) / 2 pieces if there are two.
+// us, weights from memory, with the norm of x left to it where the model leaves it, before : now: gate and up 3,072 x 1,024 6.4 : 5.0, 6,144 x 2,048
+// 13.6 : 10.7, 9,728 x 2,560 19.0 : 17.9, 12,288 x 4,096 33.6 : 32.6, 25,600 x 5,120 81 : 78; plain 1,024 x 2,048 3.5 : 2.9, 1,024 x 3,072 4.2 : 3.3, 4,096 x 1,024
+// 4.8 : 4.3, 6,144 x 2,560 11.3 : 8.2, 4,096 x 4,096 7.9 : 7.7, 151,936 x 1,024 56 : 48 (6.5 TB/s).  Rows of 6,144 and more are level.
+// An empty launch takes 1.6 us of a chain: what bounds the small ones is that, a trip to memory, and the end of the launch.
+#define GV_ONE_STEPS 10
+
+template <int STEPS, bool SWIGLU, typename TO, int PARTS>
+__global__ void __launch_bounds__(GV_WAVES * RI_WAVE)
+gemv_one_kernel(TO* __restrict__ out, const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, int N, int K, NormLink link) {
+    constexpr int HALVES = SWIGLU ? 2 : 1, FIRST = PARTS == 2 ? (STEPS + 1) / 2 : STEPS;
+    constexpr int PRE = (STEPS + 1) / 2;                     // partial sums of squares a thread: four columns of x made each
+    __shared__ float scratch[16];
+    __shared__ float sq_lds[GV_WAVES];
+    const int lane = threadIdx.x & (RI_WAVE - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / RI_WAVE);
+    const int n = blockIdx.x * GV_WAVES + wave, row = min(n, N - 1);          // (past the edge: the last row again, not stored)
+    // a lane's eight elements of the last piece, if the row has them (else the row's last eight, times zero)
+    const int last = min(lane * 8 + (STEPS - 1) * 512, K - 8);
+    const bool whole = lane * 8 + (STEPS - 1) * 512 < K;
+    uint4 wq[HALVES][STEPS], xq[STEPS];
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s) xq[s] = *reinterpret_cast<const uint4*>(x + (s < STEPS - 1 ? lane * 8 + s * 512 : last));
+#pragma unroll
+    for (int h = 0; h < HALVES; ++h) {
+        const bf16_t* wr = w + ((size_t)(h * N) + row) * K;
+#pragma unroll
+        for (int s = 0; s < STEPS; ++s) wq[h][s] = load_stream16(wr + (s < STEPS - 1 ? lane * 8 + s * 512 : last));
+    }
+    float pre[PRE];
+    if (link.ssq_in) {
+#pragma unroll
+        for (int j = 0; j < PRE; ++j) {
+            const int p = threadIdx.x + j * GV_WAVES * RI_WAVE;
+            pre[j] = p < link.n_in ? link.ssq_in[p] : 0.f;
+        }
+    }
+    const bool writer = lane == 0 && n < N;
+    float gain = 0.f, res = 0.f;
+    if (link.residual && writer) {
+        gain = link.next_gain[n];
+        res = link.residual[n];
+    }
+    if (!whole) {
+        xq[STEPS - 1] = make_uint4(0, 0, 0, 0);
+#pragma unroll
+        for (int h = 0; h < HALVES; ++h) wq[h][STEPS - 1] = make_uint4(0, 0, 0, 0);
+    }
+    float sum[HALVES];
+#pragma unroll
+    for (int h = 0; h < HALVES; ++h) {
+        sum[h] = 0.f;
+#pragma unroll
+        for (int p = 0; p < PARTS; ++p) {
+            float acc = 0.f;
+#pragma unroll
+            for (int s = p ? FIRST : 0; s < (p ? STEPS : FIRST); ++s) {
+                float wv[8], xv[8];
+                unpack8(wq[h][s], wv);
+                unpack8(xq[s], xv);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) acc = fmaf(xv[e], wv[e], acc);
+            }
+            sum[h] += wave_sum(acc);
+        }
+    }
+    float inv = 1.0f;
+    if (link.ssq_in) {
+        float sq = 0.f;
+#pragma unroll
+        for (int j = 0; j < PRE; ++j) sq += pre[j];
+        for (int p = threadIdx.x + PRE * GV_WAVES * RI_WAVE; p < link.n_in; p += GV_WAVES * RI_WAVE) sq += link.ssq_in[p];
+        inv = 1.0f / sqrtf(block_sum(sq, scratch) / (float)link.dim + link.eps);
+    }
+    float v = SWIGLU ? silu_f(sum[0] * inv) * (sum[HALVES - 1] * inv) : sum[0] * inv;
+    if (writer) {
+        if (link.residual) {
+            v += res;
+            link.residual[n] = v;                            // this element belongs to this wavefront alone
+            link.xg_out[n] = f32_to_bf16(v * gain);
+        } else {
+            from_f32(out + n, v);
+        }
+    }
+    if (link.residual) {                                     // the workgroup's share of the row's sum of squares
+        if (lane == 0) sq_lds[wave] = n < N ? v * v : 0.f;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            float total = 0.f;
+            for (int wv = 0; wv < GV_WAVES; ++wv) total += sq_lds[wv];
+            link.ssq_out[blockIdx.x] = total;
+        }
+    }
+}
+
 // How many wavefronts share a row: measured on MI355X with one row of x (decode at batch 1).  A wavefront that
 // asks for four steps' loads at a time streams a row of 4,096 elements and more fastest alone (Qwen3-8B sizes,
 // tok/s at batch 1 with four, two and one wavefront on the rows of 12,288 elements: 308.5, 312.0, 313.4; with two
@@ -216,15 +314,39 @@ static int gemv_k_split(int n, int k) {
     return 1;
 }
 
-static unsigned gemv_grid(int n, int k) {
-    const int rows_per_wg = GV_WAVES / gemv_k_split(n, k);
+// Whether the kernel for one row of x takes it.
+static bool gemv_is_one(int m, int k) { return m == 1 && k <= GV_ONE_STEPS * 512; }
+
+static unsigned gemv_grid(int m, int n, int k) {
+    const int rows_per_wg = gemv_is_one(m, k) ? GV_WAVES : GV_WAVES / gemv_k_split(n, k);
     return (unsigned)((n + rows_per_wg - 1) / rows_per_wg);
+}
+
+template <int STEPS, bool SWIGLU, typename TO>
+static void launch_gemv_one(void* out, const void* x, const void* w, int n, int k, const NormLink& link, hipStream_t s) {
+    const unsigned grid = gemv_grid(1, n, k);
+    if constexpr (STEPS <= 8)
+        if (gemv_k_split(n, k) == 2) {
+            gemv_one_kernel<STEPS, SWIGLU, TO, 2><<<grid, GV_WAVES * RI_WAVE, 0, s>>>((TO*)out, (const bf16_t*)x, (const bf16_t*)w, n, k, link);
+            return;
+        }
+    gemv_one_kernel<STEPS, SWIGLU, TO, 1><<<grid, GV_WAVES * RI_WAVE, 0, s>>>((TO*)out, (const bf16_t*)x, (const bf16_t*)w, n, k, link);
+}
+
+template <bool SWIGLU, typename TO>
+static void launch_gemv_one_steps(void* out, const void* x, const void* w, int n, int k, const NormLink& link, hipStream_t s) {
+    switch ((k + 511) / 512) {
+#define RI_GEMV_STEPS(STEPS) case STEPS: launch_gemv_one<STEPS, SWIGLU, TO>(out, x, w, n, k, link, s); break;
+        RI_GEMV_STEPS(1) RI_GEMV_STEPS(2) RI_GEMV_STEPS(3) RI_GEMV_STEPS(4) RI_GEMV_STEPS(5)
+        RI_GEMV_STEPS(6) RI_GEMV_STEPS(7) RI_GEMV_STEPS(8) RI_GEMV_STEPS(9) RI_GEMV_STEPS(10)
+#undef RI_GEMV_STEPS
+    }
 }
 
 template <int MT, bool SWIGLU, int KS>
 static void launch_gemv_ks(void* out, int out_dtype, const void* x, const void* w, int m, int n, int k,
                            const NormLink& link, hipStream_t s) {
-    const unsigned grid = gemv_grid(n, k);
+    const unsigned grid = gemv_grid(m, n, k);
     // one row of x whose norm is still to finish, with more partial sums than four a thread cover
     const bool many = MT == 1 && link.ssq_in && link.n_in > GV_PRE_FEW * GV_WAVES * RI_WAVE;
     if (out_dtype == RI_F32) {
@@ -243,15 +365,22 @@ static void launch_gemv_ks(void* out, int out_dtype, const void* x, const void* 
 template <int MT, bool SWIGLU>
 static void launch_gemv(void* out, int out_dtype, const void* x, const void* w, int m, int n, int k,
                         const NormLink& link, hipStream_t s) {
-    switch (gemv_k_split(n, k)) {
-        case 4: launch_gemv_ks<MT, SWIGLU, 4>(out, out_dtype, x, w, m, n, k, link, s); break;
-        case 2: launch_gemv_ks<MT, SWIGLU, 2>(out, out_dtype, x, w, m, n, k, link, s); break;
-        default: launch_gemv_ks<MT, SWIGLU, 1>(out, out_dtype, x, w, m, n, k, link, s); break;
-    }
+    if constexpr (MT > 1)                                    // (one row of x comes here with long rows of w alone)
+        if (gemv_k_split(n, k) == 2) return launch_gemv_ks<MT, SWIGLU, 2>(out, out_dtype, x, w, m, n, k, link, s);
+    launch_gemv_ks<MT, SWIGLU, 1>(out, out_dtype, x, w, m, n, k, link, s);
 }
 
 static int gemv_run(void* out, int out_dtype, const void* x, const void* w, int m, int n, int k, int swiglu,
                     const NormLink& link, hipStream_t s) {
+    if (gemv_is_one(m, k)) {
+        if (out_dtype == RI_F32) {
+            if (swiglu) launch_gemv_one_steps<true, float>(out, x, w, n, k, link, s);
+            else        launch_gemv_one_steps<false, float>(out, x, w, n, k, link, s);
+        } else if (swiglu) launch_gemv_one_steps<true, bf16_t>(out, x, w, n, k, link, s);
+        else               launch_gemv_one_steps<false, bf16_t>(out, x, w, n, k, link, s);
+        RI_LAUNCH_CHECK("gemv_bf16");
+        return 0;
+    }
     const int mt = m <= 1 ? 1 : m <= 2 ? 2 : m <= 4 ? 4 : 8;
 #define RI_GEMV_CASE(MT)                                                             \
     case MT:                                                                         \
@@ -278,8 +407,8 @@ extern "C" int ri_gemv_bf16(void* out, int out_dtype, const void* x, const void*
     return gemv_run(out, out_dtype, x, w, m, n, k, swiglu, link, (hipStream_t)stream);
 }
 
-// Number of workgroups (and so of partial sums of squares per row) of a linked product with n output columns.
-extern "C" int ri_gemv_bf16_partials(int n, int k) { return (int)gemv_grid(n, k); }
+// Number of workgroups (and so of partial sums of squares per row) of a linked product of m rows with n output columns.
+extern "C" int ri_gemv_bf16_partials(int m, int n, int k) { return (int)gemv_grid(m, n, k); }
 
 extern "C" int ri_gemv_bf16_linked(void* out, int out_dtype, const void* x, const void* w, int m, int n, int k,
                                    int swiglu, const float* ssq_in, int n_in, float eps, int dim, float* residual,

@@ -100,7 +100,7 @@ _SIGNATURES = {
     "ri_attention_decode_chunks": [c_int],
     "ri_attention_decode_streams": [c_int, c_int, c_int],
     "ri_attention_decode_pieces": [c_int, c_int, c_int, c_int],
-    "ri_gemv_bf16_partials": [c_int, c_int],
+    "ri_gemv_bf16_partials": [c_int, c_int, c_int],
     "ri_gemm_skinny_packed_bf16_partials": [c_int],
     "ri_gemv_bf16_linked": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_int, c_float,
                             c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p],
@@ -1735,7 +1735,7 @@ def linked_product(x, w: torch.Tensor, n: int, packed: bool, out_dtype=torch.bfl
         return out
     if swiglu:
         raise ShapeError("a gate|up product does not feed the residual stream")
-    partials = _get("ri_gemm_skinny_packed_bf16_partials")(n) if packed else _get("ri_gemv_bf16_partials")(n, k)
+    partials = _get("ri_gemm_skinny_packed_bf16_partials")(n) if packed else _get("ri_gemv_bf16_partials")(m, n, k)
     xg = TiledRows.empty(m, n, xr.device) if tiled_out else torch.empty((m, n), dtype=torch.bfloat16, device=xr.device)
     ssq = torch.empty((m, partials), dtype=torch.float32, device=xr.device)
     _call(name + "_linked", None, code(torch.bfloat16), xd, wd, m, n, k, 0,

@@ -1030,6 +1030,43 @@ def test_gemm_f32_is_true_32_bit(ops):
     assert ops.gemm_f32(x, w).item() == 16.0 * (1.0 + 2.0 ** -12)
 
 
+@pytest.mark.parametrize("k", [8, 504, 512, 520, 1024, 1032, 1536, 2568, 3072, 3584, 4088, 4096, 4104, 4616, 5120, 5128])
+def test_gemv_of_one_row_whole(ops, k):
+    """One row of x and rows of w that a wavefront asks for whole, one to ten pieces of 512, and the first size past them: the bits of that row
+    beside another, rows past the edge, a weight that is no number behind the row's end left alone."""
+    rng = np.random.default_rng(k)
+    x = t(rng.normal(size=(2, k)), torch.bfloat16)
+    for n in (1, 4, 37):
+        w = t(rng.normal(size=(n, k)), torch.bfloat16)
+        for out_dtype in (torch.float32, torch.bfloat16):
+            got = ops.gemv_bf16(x[:1].contiguous(), w, out_dtype)
+            assert torch.equal(got, ops.gemv_bf16(x, w, out_dtype)[:1])
+        close(got, f64(x[:1]) @ f64(w).T, 5e-3, "one row")
+        pair = torch.cat([w, w.flip(0)])
+        assert torch.equal(ops.gemv_bf16(x[:1].contiguous(), pair, swiglu=True), ops.gemv_bf16(x, pair, swiglu=True)[:1])
+    w[-1, -1] = float("inf")
+    got = ops.gemv_bf16(x[:1].contiguous(), w, torch.float32)
+    assert torch.isfinite(got[0, :-1]).all() and torch.equal(got, ops.gemv_bf16(x, w, torch.float32)[:1])
+
+
+@pytest.mark.parametrize("k, n", [(1024, 37), (1024, 1032), (2560, 96), (4104, 40), (5120, 8)])
+@pytest.mark.parametrize("n_in", [1, 256, 300, 1281])
+def test_linked_product_of_one_row_whole(ops, k, n, n_in):
+    """The norm before it from any number of partial sums of squares, and the stream's sum and the next norm's preparation after it."""
+    rng = np.random.default_rng(n + n_in)
+    xg, ssq = t(rng.normal(size=(1, k)), torch.bfloat16), t(rng.uniform(0.5, 1.5, size=(1, n_in)) * k / n_in)
+    w, residual, gain = t(rng.normal(size=(n, k)) / np.sqrt(k), torch.bfloat16), t(rng.normal(size=(1, n))), t(rng.normal(size=(n,)))
+    y = f64(xg) @ f64(w).T / np.sqrt(f64(ssq).sum() / k + 1e-6)
+    later = ops.NormedLater(xg, ssq, 1e-6, k)
+    close(ops.linked_product(later, w, n, False, torch.float32), y, 2e-6, "normed")
+    total = residual.clone()
+    made = ops.linked_product(later, w, n, False, residual=total, next_gain=gain, next_eps=1e-6)
+    want = f64(residual) + y
+    close(total, want, 2e-6, "the stream")
+    close(made.xg, want * f64(gain), 5e-3, "the next rows")
+    close(made.ssq.sum(1), (want ** 2).sum(1), 1e-5, "sums of squares")
+
+
 @pytest.mark.parametrize("m", [1, 2, 3, 5, 8])
 @pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("k", [584, 2560, 1544, 2048, 9728])      # steps of 512: one and a bit, five, three and a bit, four, nineteen
@@ -1127,7 +1164,7 @@ def test_wide_packed_product(ops, m, n, k):
 
 @pytest.mark.parametrize("m", [1, 16, 17, 33, 49, 64])
 @pytest.mark.parametrize("n, k", [(37, 72), (1000, 1024), (5137, 264), (320, 136)])
-def test_wide_packed_product_of_many_row_tiles(ops, m, n, k):
+def test_product_with_many_row_tiles_a_workgroup(ops, m, n, k):
     """Six, eight and twelve row tiles a workgroup and ten pairs of them, x in half slices: edges of the groups, of a pair, of the slices and of
     four sums a store; the same bits as four row tiles, from rows in either order."""
     rng = np.random.default_rng(m + n + k)
