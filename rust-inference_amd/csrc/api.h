@@ -312,6 +312,8 @@ int ri_gemv_bf16_linked(void* out, int out_dtype, const void* x, const void* w, 
                         const float* ssq_in, int n_in, float eps, int dim, float* residual, const float* next_gain,
                         void* xg_out, float* ssq_out, void* stream);
 int ri_gemm_skinny_packed_bf16_partials(int n);
+// Several products of one size, without the activation, in one launch: x [batch, m, k], the packed matrices one after the other, out [batch, m, n].
+int ri_gemm_skinny_batch_bf16(void* out, int out_dtype, const void* x, const void* wpacked, int m, int n, int k, int batch, void* stream);
 int ri_gemm_skinny_packed_bf16_linked(void* out, int out_dtype, const void* x, const void* wpacked, int m, int n,
                                       int k, int swiglu, const float* ssq_in, int n_in, float eps, int dim,
                                       float* residual, const float* next_gain, void* xg_out, float* ssq_out,
@@ -518,8 +520,9 @@ int ri_talking_decode(float* out, int shares, float* scores, float* sums, int pa
                       int window, float scale, const float* r1, const float* r2, const float* talk, void* stream);
 
 // ---- time mixing (timemix.hip)
-int ri_shift_mix(void* out, int out_dtype, const float* x, const float* kept, const float* mu, int n_mix,
-                 const int32_t* tok_seq, const int32_t* cu_seqlens, const int32_t* slots, int tokens, int width, void* stream);
+// keep: every sequence brings one token, which becomes its kept row (else ri_shift_keep follows).
+int ri_shift_mix(void* out, int out_dtype, const float* x, float* kept, const float* mu, int n_mix, const int32_t* tok_seq,
+                 const int32_t* cu_seqlens, const int32_t* slots, int tokens, int width, int keep, void* stream);
 int ri_shift_keep(float* kept, const float* x, const int32_t* cu_seqlens, const int32_t* slots, int seqs, int width,
                   void* stream);
 int ri_timemix_max_dim();

@@ -5,7 +5,7 @@
 //                  the projections, one block of rows per s;
 //   tanh_rows:     tanh of float32 rows, written in the activations' format (between the decay's two products);
 //   shift_keep:    the last row of every sequence's step becomes its kept row (a launch of its own: the first token of a
-//                  step reads the kept row while the last would write it);
+//                  step reads the kept row while the last would write it; in a step of single tokens shift_mix keeps it);
 //   timemix_scan:  per head, with r, k, v of a token and its decay w = exp(-exp(z + w0)) per key channel,
 //                      o_t = (S_(t-1) + diag(u) k_t v_t^T)^T r_t,      S_t = diag(w_t) S_(t-1) + k_t v_t^T;
 //                  then o is divided by its root mean square over the head, multiplied by the gain of its place among
@@ -21,9 +21,9 @@
 
 template <typename TA>
 __global__ void __launch_bounds__(256)
-shift_mix_kernel(TA* __restrict__ out, const float* __restrict__ x, const float* __restrict__ kept,
+shift_mix_kernel(TA* __restrict__ out, const float* __restrict__ x, float* kept,
                  const float* __restrict__ mu, int n_mix, const int32_t* __restrict__ tok_seq,
-                 const int32_t* __restrict__ cu_seqlens, const int32_t* __restrict__ slots, int tokens, int width) {
+                 const int32_t* __restrict__ cu_seqlens, const int32_t* __restrict__ slots, int tokens, int width, int keep) {
     const int t = blockIdx.x;
     const int d = blockIdx.y * 256 + threadIdx.x;             // a thread an element: a single token is many short workgroups
     if (d >= width) return;
@@ -32,6 +32,8 @@ shift_mix_kernel(TA* __restrict__ out, const float* __restrict__ x, const float*
     const float h = x[(size_t)t * width + d], delta = before[d] - h;
     for (int s = 0; s < n_mix; ++s)
         from_f32(out + ((size_t)s * tokens + t) * width + d, h + delta * mu[(size_t)s * width + d]);
+    // (single tokens: the thread that has read the kept element is the only one to, and no other launch has to follow for it)
+    if (keep) kept[(size_t)slots[seq] * width + d] = h;
 }
 
 __global__ void __launch_bounds__(256)
@@ -43,16 +45,16 @@ shift_keep_kernel(float* __restrict__ kept, const float* __restrict__ x, const i
     for (int d = threadIdx.x; d < width; d += 256) kept[(size_t)slots[seq] * width + d] = x[(size_t)(end - 1) * width + d];
 }
 
-extern "C" int ri_shift_mix(void* out, int out_dtype, const float* x, const float* kept, const float* mu, int n_mix,
+extern "C" int ri_shift_mix(void* out, int out_dtype, const float* x, float* kept, const float* mu, int n_mix,
                             const int32_t* tok_seq, const int32_t* cu_seqlens, const int32_t* slots, int tokens, int width,
-                            void* stream) {
+                            int keep, void* stream) {
     RI_REQUIRE(tokens > 0 && width > 0 && width <= 65535 * 256 && n_mix >= 1, "shift_mix: %d tokens of %d, %d mixes", tokens, width, n_mix);
     RI_REQUIRE(out_dtype == RI_F32 || out_dtype == RI_BF16, "shift_mix: dtype %d", out_dtype);
     hipStream_t s = (hipStream_t)stream;
     if (out_dtype == RI_F32)
-        shift_mix_kernel<float><<<dim3(tokens, (width + 255) / 256), 256, 0, s>>>((float*)out, x, kept, mu, n_mix, tok_seq, cu_seqlens, slots, tokens, width);
+        shift_mix_kernel<float><<<dim3(tokens, (width + 255) / 256), 256, 0, s>>>((float*)out, x, kept, mu, n_mix, tok_seq, cu_seqlens, slots, tokens, width, keep);
     else
-        shift_mix_kernel<bf16_t><<<dim3(tokens, (width + 255) / 256), 256, 0, s>>>((bf16_t*)out, x, kept, mu, n_mix, tok_seq, cu_seqlens, slots, tokens, width);
+        shift_mix_kernel<bf16_t><<<dim3(tokens, (width + 255) / 256), 256, 0, s>>>((bf16_t*)out, x, kept, mu, n_mix, tok_seq, cu_seqlens, slots, tokens, width, keep);
     RI_LAUNCH_CHECK("shift_mix");
     return 0;
 }

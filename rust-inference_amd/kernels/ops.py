@@ -80,6 +80,7 @@ _SIGNATURES = {
     "ri_sample_split": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_float, c_int,
                         c_float, c_float, c_void_p],
     "ri_gemm_skinny_packed_bf16": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
+    "ri_gemm_skinny_batch_bf16": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p],
     "ri_gemm_mid_packed_bf16": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p],
     "ri_gemm_wide_packed_bf16": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int,
                                  c_int, c_void_p],
@@ -196,7 +197,7 @@ _SIGNATURES = {
     "ri_talking_decode_fits": [c_int, c_int, c_int, c_int],
     "ri_talking_decode": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p,
                           c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_void_p, c_void_p, c_void_p, c_void_p],
-    "ri_shift_mix": [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p],
+    "ri_shift_mix": [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p],
     "ri_shift_keep": [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p],
     "ri_timemix_max_dim": [],
     "ri_tanh_rows": [c_void_p, c_int, c_void_p, ctypes.c_long, c_void_p],
@@ -1522,6 +1523,19 @@ def gemm_skinny_packed_bf16(x, wpacked: torch.Tensor, n: int, out_dtype=torch.bf
     return out
 
 
+def gemm_skinny_batch(x: torch.Tensor, wpacked: torch.Tensor, n: int, out_dtype=torch.bfloat16) -> torch.Tensor:
+    """``x[i] @ w[i].T`` for up to 16 bfloat16 rows each, ``x [batch, M, k]`` and ``wpacked [batch, ...]`` of ``pack_for_mfma``, in one launch: the bits
+    of ``gemm_skinny_packed_bf16`` on each."""
+    batch, m, k = x.shape
+    want = (batch, -(-n // 16), -(-k // 32), 64, 8)
+    if tuple(wpacked.shape) != want:
+        raise ShapeError(f"packed weights are {list(wpacked.shape)}, {batch} products with n {n}, k {k} want {list(want)}")
+    out = torch.empty((batch, m, n), dtype=out_dtype, device=x.device)
+    _call("ri_gemm_skinny_batch_bf16", _dev(out, "out"), code(out_dtype), _dev(x, "x", torch.bfloat16), _dev(wpacked, "wpacked", torch.bfloat16),
+          m, n, k, batch, _stream())
+    return out
+
+
 class NormedLater:
     """Rows of a residual stream whose RMSNorm is left to the product that reads them:
     ``xg = bfloat16(r * gain)`` and partial sums of ``r^2`` per row, ``[M, partials]``; the
@@ -2147,15 +2161,18 @@ def timemix_max_dim() -> int:
     return _get("ri_timemix_max_dim")()
 
 
-def shift_mix(x32, kept, mu, tok_seq, cu_seqlens, slots, out_dtype) -> torch.Tensor:
+def shift_mix(x32, kept, mu, tok_seq, cu_seqlens, slots, out_dtype, keep: bool = False) -> torch.Tensor:
     """``[n, T, width]``: for every mixing vector ``mu[s]`` the rows ``h + (h' - h) * mu[s]``, ``h'`` the row before (the
-    sequence's kept row ``kept[slot]`` for the first token of the step)."""
+    sequence's kept row ``kept[slot]`` for the first token of the step).  ``keep``, where every sequence brings one token: it becomes the kept
+    row, as by ``shift_keep``."""
+    if keep and x32.shape[0] != slots.shape[0]:
+        raise ShapeError(f"{x32.shape[0]} tokens of {slots.shape[0]} sequences are not one each")
     tokens, width = x32.shape
     n = mu.shape[0]
     out = torch.empty((n, tokens, width), dtype=out_dtype, device=x32.device)
     _call("ri_shift_mix", _dev(out, "out"), code(out_dtype), _dev(x32, "x", torch.float32), _dev(kept, "kept", torch.float32),
           _dev(mu, "mu", torch.float32, (n, width)), n, _dev(tok_seq, "tok_seq", torch.int32, (tokens,)),
-          _dev(cu_seqlens, "cu_seqlens", torch.int32), _dev(slots, "slots", torch.int32), tokens, width, _stream())
+          _dev(cu_seqlens, "cu_seqlens", torch.int32), _dev(slots, "slots", torch.int32), tokens, width, int(keep), _stream())
     return out
 
 

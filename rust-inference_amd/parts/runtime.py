@@ -183,6 +183,26 @@ def _groups_tile(m: int, groups: int, n: int, k: int, ldw: int, gated: bool) -> 
     return 1 if time(1) < time(0) else 0
 
 
+# Products of one size that a part makes together (four of time mixing), all known: in one launch while the larger tile makes up to two rounds, after
+# which one product fills the machine by itself.  us, in one launch : the library's four; 512 / 1,000 / 2,048 / 4,096 / 8,192 rows; 1,024 x 4,096 44 / 47 / 61 / 101 /
+# 196 : 58 / 73 / 108 / 160 / 262; 512 x 1,024 16 / 17 / 18 / 22 / 34 : 33 / 35 / 38 / 44 / 56; 2,048 x 4,096 56 / 62 / 102 / 198 / 397 : 84 / 109 / 164 / 247 / 394.
+TOGETHER_ROUNDS = 2
+
+
+@functools.lru_cache(maxsize=4096)
+def _together_tile(count: int, m: int, n: int, k: int) -> int | None:
+    """The tile for ``count`` products of ``m`` rows with matrices of ``n`` rows of ``k`` in one launch; None: one after the other."""
+    if m < TILES_MIN_ROWS or _groups_tile(count * m, count, n, k, k, False) is None:
+        return None
+
+    def rounds(tile):
+        rows, cols = ops.TILES[tile]
+        return -(-count * -(-m // rows) * -(-n // cols) // _compute_units())
+    if rounds(0) > TOGETHER_ROUNDS:
+        return None
+    return 1 if rounds(1) * GROUPS_SMALLER < rounds(0) else 0
+
+
 @functools.lru_cache(maxsize=4096)
 def _tiles_fit(m: int, n: int, ldx: int, ldw: int, ldo: int, activation: str | None) -> bool:
     """``ops.gemm_tiles_fits``, asked once per size."""
@@ -203,6 +223,20 @@ class PackedWeight:
         # 2 to 16 rows into the residual stream go to the wide kernel (set by Runtime.pack: see there)
         self.small_wide = False
         self.small_only = False      # the packed copy was made for that alone: larger steps stay where they were
+
+
+class StackedWeights:
+    """Weights of one size whose products go together: row-major ``w [count, n, k]``, the packed copies likewise or None, and each as a
+    ``PackedWeight`` that shares the memory."""
+
+    def __init__(self, each: list[PackedWeight]):
+        self.each, self.n, self.k = each, each[0].n, each[0].k
+        self.w = torch.stack([pw.w for pw in each])
+        self.packed = torch.stack([pw.packed for pw in each]) if all(pw.packed is not None for pw in each) else None
+        for i, pw in enumerate(each):
+            pw.w = self.w[i]
+            if self.packed is not None:
+                pw.packed = self.packed[i]
 
 
 class Runtime:
@@ -438,6 +472,24 @@ class Runtime:
                 return ops.gemm_tiles_bf16(self.normed_now(x), pw.w, tile, self.dtype, "silu_gate")
             return ops.swiglu(self.linear(x, pw.w), tiled_out=tiled_out)
         return self.linear(x, pw.w, out_dtype)
+
+    def stack(self, weights: list[torch.Tensor]) -> StackedWeights:
+        """Placed weights of one size, for ``linear_each``."""
+        return StackedWeights([self.pack(w) for w in weights])
+
+    def linear_each(self, x: torch.Tensor, weights: StackedWeights) -> list[torch.Tensor]:
+        """``x[i] @ w[i].T`` of ``x [count, m, k]`` in the compute dtype: 2 to 16 rows in one launch of the packed kernel, prompts in one of the
+        product in tiles (_together_tile), else one after the other."""
+        count, m, k = x.shape
+        if self.dtype == torch.bfloat16 and not self.invariant:
+            if GEMV_MAX_ROWS < m <= SKINNY_MAX_ROWS and weights.packed is not None:
+                return list(ops.gemm_skinny_batch(x, weights.packed, weights.n).unbind(0))
+            tile = _together_tile(count, m, weights.n, k)
+            if tile is not None:
+                starts = torch.arange(0, count * m + 1, m, dtype=torch.int32, device=x.device)
+                out = ops.gemm_tiles_groups(x.view(count * m, k), weights.w.view(count * weights.n, k), starts, count, weights.n, tile)
+                return list(out.view(count, m, weights.n).unbind(0))
+        return [ops.as_rows(self.linear_packed(x[i], pw)) for i, pw in enumerate(weights.each)]
 
     def linear_activated(self, x, pw: PackedWeight, activation: str, after, b_gate=None, b_up=None, limit: float = 0.0):
         """``after(x @ w.T)``, with the activation (of ``ops.TILES_ACTIVATIONS``; ``after`` does the same) in the product where that goes in

@@ -60,7 +60,8 @@ class TimeMix(Mixer):
         if weights[n["w1"]].shape[0] != weights[n["w2"]].shape[1]:
             raise ConfigError(f"{n['w1']} has {weights[n['w1']].shape[0]} rows, {n['w2']} {weights[n['w2']].shape[1]} columns")
         self.mu = torch.stack([rt.place_gain(weights[n["mu_" + s]]) for s in self.MIXES], 0).contiguous()
-        self.w = {x: rt.pack(rt.place_matrix(weights[n[x]])) for x in ("r", "k", "v", "g", "w1", "w2")}
+        self.w_rkvg = rt.stack([rt.place_matrix(weights[n[x]]) for x in ("r", "k", "v", "g")])
+        self.w = {x: rt.pack(rt.place_matrix(weights[n[x]])) for x in ("w1", "w2")}
         self.w0, self.u = rt.place_gain(weights[n["w0"]]), rt.place_gain(weights[n["u"]]).reshape(-1).contiguous()
         self.gain = rt.place_gain(weights[n["norm"]])
         if alone:
@@ -76,9 +77,11 @@ class TimeMix(Mixer):
         state, kept = store
         x32 = residual if residual is not None else ops.as_rows(x).to(torch.float32)
         with profiler.section(profiler.QKV_PROJECTION):
-            mixes = ops.shift_mix(x32, kept, self.mu, ctx.tok_seq, ctx.cu_seqlens, ctx.slots, rt.dtype)
-            ops.shift_keep(kept, x32, ctx.cu_seqlens, ctx.slots)
-            r, k, v, g = (ops.as_rows(rt.linear_packed(mixes[i], self.w[s])) for i, s in enumerate(("r", "k", "v", "g")))
+            single = ctx.is_decode                        # one token a sequence: the mixes' kernel keeps it too
+            mixes = ops.shift_mix(x32, kept, self.mu, ctx.tok_seq, ctx.cu_seqlens, ctx.slots, rt.dtype, keep=single)
+            if not single:
+                ops.shift_keep(kept, x32, ctx.cu_seqlens, ctx.slots)
+            r, k, v, g = rt.linear_each(mixes[:4], self.w_rkvg)
             # the decay's pre-activation: tanh in float32 between its two products, the second one's sums float32
             mid = ops.tanh_rows(ops.as_rows(rt.linear_packed(mixes[4], self.w["w1"], out_dtype=torch.float32)), rt.dtype)
             z = ops.as_rows(rt.linear_packed(mid, self.w["w2"], out_dtype=torch.float32))

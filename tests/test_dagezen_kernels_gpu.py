@@ -283,6 +283,22 @@ def test_a_key_at_the_windows_edge_counts_and_the_next_one_does_not(ops):
 
 
 # ---------------------------------------------------------------- time mixing
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("seqs, width", [(1, 70), (5, 256), (9, 300)])
+def test_single_tokens_are_mixed_and_kept_in_one_launch(ops, seqs, width, dtype):
+    """The bits of the mixes and then the move, slots in any order, the others' rows left alone."""
+    rng = np.random.default_rng(seqs)
+    slots = t(rng.permutation(seqs + 2)[:seqs], torch.int32)
+    kept = t(rng.normal(size=(seqs + 2, width)))
+    x, mu = t(rng.normal(size=(seqs, width))), t(rng.uniform(size=(5, width)))
+    seq, cu = t(np.arange(seqs), torch.int32), t(np.arange(seqs + 1), torch.int32)
+    apart, together = kept.clone(), kept.clone()
+    want = ops.shift_mix(x, apart, mu, seq, cu, slots, dtype)
+    ops.shift_keep(apart, x, cu, slots)
+    assert torch.equal(ops.shift_mix(x, together, mu, seq, cu, slots, dtype, keep=True), want)
+    assert torch.equal(together, apart)
+
+
 @pytest.mark.parametrize("columns", [True, False])
 @pytest.mark.parametrize("heads, dim", [(3, 12), (2, 40), (1, 70), (1, 130)])
 def test_time_mixing_through_every_cut(ops, heads, dim, columns):

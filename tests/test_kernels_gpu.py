@@ -1107,6 +1107,19 @@ def test_gemm_skinny_packed_bf16(ops, m, n, k):
         close(got.sum(0), want, 3e-6, f"{parts} parts of K")
 
 
+@pytest.mark.parametrize("m", [1, 2, 8, 9, 16])
+@pytest.mark.parametrize("n, k", [(37, 72), (512, 1024), (1000, 264), (48, 8192)])
+def test_packed_products_of_one_size_in_one_launch(ops, m, n, k):
+    """The bits of a launch each, over both numbers of wavefronts, edges of the row tiles and of K."""
+    rng = np.random.default_rng(m + n)
+    x = t(rng.normal(size=(3, m, k)), torch.bfloat16)
+    packed = torch.stack([ops.pack_for_mfma(t(rng.normal(size=(n, k)), torch.bfloat16)) for _ in range(3)])
+    for out_dtype in (torch.float32, torch.bfloat16):
+        got = ops.gemm_skinny_batch(x, packed, n, out_dtype)
+        for i in range(3):
+            assert torch.equal(got[i], ops.gemm_skinny_packed_bf16(x[i], packed[i], n, out_dtype))
+
+
 @pytest.mark.parametrize("m", [1, 16, 17, 33, 40, 49, 64])
 @pytest.mark.parametrize("n, k", [(37, 72), (1000, 1024), (584, 12288), (4096, 4096), (70, 264)])
 def test_wide_packed_product(ops, m, n, k):

@@ -202,6 +202,28 @@ def test_wavefronts_of_a_whole_wide_product(monkeypatch):
     assert [runtime._wide_whole_waves(n, 32) for n in (16384, 24576, 65536, 98304)] == [4, 3, 4, 4]
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("m", [1, 2, 16, 17, 300, 600, 2048])
+def test_products_of_one_size_together(m, dtype, monkeypatch):
+    """Whatever takes them, each against float64; one launch for 2 to 16 rows and for prompts that fill it."""
+    from rust_inference_amd.kernels import ops
+    from rust_inference_amd.parts import runtime
+    rt = runtime.Runtime(DEV, dtype)
+    rng = np.random.default_rng(m)
+    n, k = 1024, 256
+    ws = [t(rng.normal(size=(n, k)) / np.sqrt(k), torch.bfloat16) for _ in range(4)]
+    stacked, x = rt.stack(ws), t(rng.normal(size=(4, m, k)), dtype)
+    taken = []
+    for name in ("gemm_skinny_batch", "gemm_tiles_groups"):
+        monkeypatch.setattr(ops, name, lambda *a, name=name, real=getattr(ops, name), **kw: (taken.append(name), real(*a, **kw))[1])
+    for got, one, w in zip(rt.linear_each(x, stacked), x, ws):
+        assert rel_to_max(f64(got), f64(one) @ f64(w).T) < (1e-2 if dtype == torch.bfloat16 else 1e-5)
+    if dtype == torch.float32 or m in (1, 17, 300):
+        assert not taken
+    elif m <= 16 or ops.compute_units() == 256:
+        assert taken == ["gemm_skinny_batch" if m <= 16 else "gemm_tiles_groups"]
+
+
 def test_many_row_tiles_of_a_whole_wide_product(monkeypatch):
     """Many row tiles a workgroup where that saves a compute unit a fifth of the rows it fetches; not in a single round for few rows or short ones."""
     from rust_inference_amd.parts import runtime
