@@ -43,7 +43,9 @@ __device__ __forceinline__ float silu_sk(float z) { return z / (1.0f + expf(-z))
 // do).  The fragment goes through the matrix cores with either step's weights: columns 0-7 of the first
 // product and columns 8-15 of the second are the rows' sums over the even and over the odd steps, the other
 // columns pair one step's weights with the other step's x and are dropped.  The same bits as without.
-template <int SK_WAVES, bool SWIGLU, typename TO, bool PAIRED>
+// BATCH: blockIdx.z is a product of its own (x, matrix and result one after the other; without the activation, parts of K, a link and tiles).
+// A form of its own: the forms of one product have no scalar registers left for the three offsets (with them they spilled one or two more).
+template <int SK_WAVES, bool SWIGLU, typename TO, bool PAIRED, bool BATCH = false>
 __global__ void __launch_bounds__(SK_WAVES * 64)
 gemm_skinny_packed_kernel(TO* __restrict__ out, const bf16_t* __restrict__ x, const bf16_t* __restrict__ wpacked,
                           int M, int N, int K, int k_tiles, int tiles_per_wave, int up_tile_offset, NormLink link, int tiled) {
@@ -59,10 +61,11 @@ gemm_skinny_packed_kernel(TO* __restrict__ out, const bf16_t* __restrict__ x, co
     const int part_tiles = (k_tiles + gridDim.y - 1) / gridDim.y;
     const int part_begin = blockIdx.y * part_tiles, part_end = min(k_tiles, part_begin + part_tiles);
     const int kt_begin = part_begin + wave * tiles_per_wave, kt_end = min(part_end, kt_begin + tiles_per_wave);
-    // blockIdx.z: a product of its own (x, matrix and result one after the other; without the activation, a link and tiles)
-    out += ((size_t)blockIdx.z * gridDim.y + blockIdx.y) * M * N;
-    x += (size_t)blockIdx.z * M * K;
-    wpacked += (size_t)blockIdx.z * gridDim.x * k_tiles * 512;
+    if constexpr (BATCH) {
+        out += (size_t)blockIdx.z * M * N;
+        x += (size_t)blockIdx.z * M * K;
+        wpacked += (size_t)blockIdx.z * gridDim.x * k_tiles * 512;
+    } else out += (size_t)blockIdx.y * M * N;
     const bf16_t* wp = wpacked + ((size_t)nt * k_tiles * 64 + lane) * 8;
     const bf16_t* up = SWIGLU ? wpacked + ((size_t)(up_tile_offset + nt) * k_tiles * 64 + lane) * 8 : nullptr;
     const bool x_tiled = tiled & TILED_X;
@@ -378,7 +381,7 @@ gemm_skinny_packed_kernel(TO* __restrict__ out, const bf16_t* __restrict__ x, co
 // bytes from the L2 cache like the ones from memory.)
 static int skinny_waves(int n, int k) { return k >= 8192 ? 8 : 4; }
 
-template <int WAVES, bool SWIGLU>
+template <int WAVES, bool SWIGLU, bool BATCH = false>
 static void launch_packed(void* out, int out_dtype, const bf16_t* x, const bf16_t* w, int m, int n, int k, int parts,
                           const NormLink& link, int tiled, hipStream_t s, int batch = 1) {
     const int k_tiles = (k + 31) / 32, row_tiles = (n + 15) / 16;
@@ -390,7 +393,7 @@ static void launch_packed(void* out, int out_dtype, const bf16_t* x, const bf16_
     const bool paired = m <= 8 && k % 32 == 0 && tiles_per_wave % 2 == 0 && part_tiles == tiles_per_wave * WAVES &&
                         k_tiles % part_tiles == 0;
 #define RI_SKINNY_GO(TO, PAIRED)                                                        \
-    gemm_skinny_packed_kernel<WAVES, SWIGLU, TO, PAIRED><<<grid, WAVES * 64, 0, s>>>(   \
+    gemm_skinny_packed_kernel<WAVES, SWIGLU, TO, PAIRED, BATCH><<<grid, WAVES * 64, 0, s>>>( \
         (TO*)out, x, w, m, n, k, k_tiles, tiles_per_wave, row_tiles, link, tiled)
     if (out_dtype == RI_F32) {
         if (paired) RI_SKINNY_GO(float, true); else RI_SKINNY_GO(float, false);
@@ -437,8 +440,8 @@ extern "C" int ri_gemm_skinny_batch_bf16(void* out, int out_dtype, const void* x
     RI_REQUIRE(n > 0 && k > 0 && k % 8 == 0 && batch > 0 && batch <= 65535, "gemm_skinny_batch_bf16: %d of n %d, k %d (k must be a multiple of 8)", batch, n, k);
     RI_REQUIRE(out_dtype == RI_F32 || out_dtype == RI_BF16, "gemm_skinny_batch_bf16: out dtype %d", out_dtype);
     const NormLink link = {};
-    if (skinny_waves(n, k) == 8) launch_packed<8, false>(out, out_dtype, (const bf16_t*)x, (const bf16_t*)wpacked, m, n, k, 1, link, 0, (hipStream_t)stream, batch);
-    else launch_packed<4, false>(out, out_dtype, (const bf16_t*)x, (const bf16_t*)wpacked, m, n, k, 1, link, 0, (hipStream_t)stream, batch);
+    if (skinny_waves(n, k) == 8) launch_packed<8, false, true>(out, out_dtype, (const bf16_t*)x, (const bf16_t*)wpacked, m, n, k, 1, link, 0, (hipStream_t)stream, batch);
+    else launch_packed<4, false, true>(out, out_dtype, (const bf16_t*)x, (const bf16_t*)wpacked, m, n, k, 1, link, 0, (hipStream_t)stream, batch);
     RI_LAUNCH_CHECK("gemm_skinny_batch_bf16");
     return 0;
 }
