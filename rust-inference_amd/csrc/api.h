@@ -356,7 +356,7 @@ int ri_gemm_tiles_bf16_fits(int m, int n, int ldx, int ldw, int ldo, int gated);
 int ri_gemm_tiles_bf16(void* out, int out_dtype, int ldo, const void* x, int ldx, const void* w, int ldw, int m, int n, int k, int act,
                        const float* b_gate, const float* b_up, float limit, int tile, void* stream);
 // The same for rows in up to 64 groups, each with a matrix of its own (w + group * w_group elements): group i's rows are starts[i] to
-// starts[i + 1] of x and out (on the device, ascending, within m); rows past the last group's stay as they are.  Tiles of 256 x 256 or 128 x 256, bfloat16 results.
+// starts[i + 1] of x and out (on the device, ascending, within m; what is not is held to both); rows past the last group's stay as they are.  Tiles of 256 x 256 or 128 x 256, bfloat16 results.
 int ri_gemm_tiles_groups_bf16(void* out, int ldo, const void* x, int ldx, const void* w, int ldw, long w_group, const int32_t* starts, int groups,
                               int m, int n, int k, int act, float limit, int tile, void* stream);
 

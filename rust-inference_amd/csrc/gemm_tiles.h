@@ -55,11 +55,17 @@ gemm_tiles_bf16_kernel(const GtArgs a) {
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r = lane & 15, g = lane >> 4;
     const int wm = wave & 1, wn = wave >> 1, nk = a.K / 64;
 
-    // The groups, a lane each: its rows, and the tiles of the groups up to it.
+    // The groups, a lane each: its rows, and the tiles of the groups up to it.  Where a group ends is the largest of the starts up to there
+    // within x, so whatever the starts hold, groups lie side by side inside x and out.
     int first_row = 0, its_rows = 0, its_tiles = 0, upto = 0, all_tiles = a.m_tiles * a.n_tiles;
     if (GROUPED) {
-        first_row = a.starts[min(lane, a.groups)];
-        its_rows = lane < a.groups ? a.starts[min(lane + 1, a.groups)] - first_row : 0;
+        const int begin = min(max(a.starts[0], 0), M);
+        int end = max(min(a.starts[min(lane + 1, a.groups)], M), begin);
+#pragma unroll
+        for (int d = 1; d < RI_WAVE; d *= 2) end = max(end, __shfl(end, max(lane - d, 0), RI_WAVE));
+        const int before_it = __shfl(end, max(lane - 1, 0), RI_WAVE);
+        first_row = lane ? before_it : begin;
+        its_rows = end - first_row;                           // (none past the last group)
         upto = its_tiles = (its_rows + BM - 1) / BM * a.n_tiles;
 #pragma unroll
         for (int d = 1; d < RI_WAVE; d *= 2) {

@@ -1673,10 +1673,10 @@ TILES_GROUPS_MOST = 64           # groups of rows that gemm_tiles_groups takes
 
 
 def gemm_tiles_groups(x: torch.Tensor, w: torch.Tensor, starts: torch.Tensor, groups: int, n: int, tile: int, activation: str | None = None,
-                      limit: float = 0.0, by_columns: bool = False) -> torch.Tensor:
+                      limit: float = 0.0, by_columns: bool = False, out: torch.Tensor | None = None) -> torch.Tensor:
     """``gemm_tiles_bf16`` for rows that lie in groups: group ``i``, the rows ``starts[i]`` to ``starts[i + 1]`` of ``x`` (int32 on the
     device, ascending), meets the ``i``-th stretch of ``w``, of ``n`` rows (``2 n``: gate and up) or, ``by_columns``, of as many columns as ``x`` has;
-    bfloat16 results, which rows past the last group's do not get.  ``tile``: 0 or 1 of ``TILES``."""
+    bfloat16 results (into ``out``, if given), which rows past the last group's do not get.  ``tile``: 0 or 1 of ``TILES``."""
     m, k = x.shape
     rows = 2 * n if activation in ("silu_gate", "clamped_gate") else n
     want = (rows, groups * k) if by_columns else (groups * rows, k)
@@ -1684,8 +1684,9 @@ def gemm_tiles_groups(x: torch.Tensor, w: torch.Tensor, starts: torch.Tensor, gr
         raise ShapeError(f"{groups} groups of rows of {k}: the matrices are {list(w.shape)}, not {list(want)} side by side")
     if starts.numel() < groups + 1:
         raise ShapeError(f"{groups} groups begin at {starts.numel()} places")
-    out = torch.empty((m, n), dtype=torch.bfloat16, device=x.device)
-    _call("ri_gemm_tiles_groups_bf16", _dev(out, "out"), n, _dev(x, "x", torch.bfloat16), k, _dev(w, "w", torch.bfloat16), w.stride(0),
+    if out is None:
+        out = torch.empty((m, n), dtype=torch.bfloat16, device=x.device)
+    _call("ri_gemm_tiles_groups_bf16", _dev(out, "out", torch.bfloat16, (m, n)), n, _dev(x, "x", torch.bfloat16), k, _dev(w, "w", torch.bfloat16), w.stride(0),
           k if by_columns else rows * k, _dev(starts, "starts", torch.int32), groups, m, n, k, TILES_ACTIVATIONS[activation], float(limit), int(tile),
           _stream())
     return out

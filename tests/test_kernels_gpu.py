@@ -1589,12 +1589,29 @@ def test_product_of_groups_of_rows(ops, act, counts, n, k):
     at = t(starts, torch.int32)
     for tile in (0, 1):
         for matrix, columns in ((w, False), (by_columns, True)):
-            got = ops.gemm_tiles_groups(x, matrix, at, groups, n, tile, act, 0.8, by_columns=columns)
+            got = ops.gemm_tiles_groups(x, matrix, at, groups, n, tile, act, 0.8, by_columns=columns,
+                                        out=t(np.full((len(x), n), 77.0), torch.bfloat16))
+            assert (got[int(starts[-1]):] == 77.0).all(), (tile, columns)
             for i in range(groups):
                 a, b = int(starts[i]), int(starts[i + 1])
                 if b > a:
                     want = ops.gemm_tiles_bf16(x[a:b], w[i * rows:(i + 1) * rows], tile, torch.bfloat16, act, limit=0.8)
                     assert torch.equal(got[a:b], want), (tile, columns, i)
+
+
+@pytest.mark.parametrize("given, held", [((0, 13, 50, 70), (0, 13, 30, 30)), ((0, 20, 5, 30), (0, 20, 20, 30)),
+                                         ((-5, 10, 2 ** 31 - 1, 0), (0, 10, 30, 30)), ((50, 2, 60, 3), (30, 30, 30, 30))])
+def test_groups_that_begin_outside_the_rows_are_held_to_them(ops, given, held):
+    """Starts past the rows, before them and that descend: no row outside is read or written, none twice."""
+    rng = np.random.default_rng(len(set(given)))
+    n, k, groups = 72, 192, 3
+    x, w = t(rng.normal(size=(30, k)), torch.bfloat16), t(rng.normal(size=(groups * n, k)) * (3.0 / np.sqrt(k)), torch.bfloat16)
+    got = ops.gemm_tiles_groups(x, w, t(given, torch.int32), groups, n, 1, out=t(np.full((30, n), 77.0), torch.bfloat16))
+    for i in range(groups):
+        a, b = held[i], held[i + 1]
+        if b > a:
+            close(got[a:b], f64(x[a:b]) @ f64(w[i * n:(i + 1) * n]).T, BF16_OUT, f"group {i}")
+    assert (got[:held[0]] == 77.0).all() and (got[held[-1]:] == 77.0).all()
 
 
 def test_groups_of_rows_that_take_several_rounds(ops):
