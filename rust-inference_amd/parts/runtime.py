@@ -226,17 +226,12 @@ class PackedWeight:
 
 
 class StackedWeights:
-    """Weights of one size whose products go together: row-major ``w [count, n, k]``, the packed copies likewise or None, and each as a
-    ``PackedWeight`` that shares the memory."""
+    """Weights of one size whose products go together, each as a ``PackedWeight``; where one launch may take them all, row-major
+    ``w [count, n, k]`` and the packed copies likewise, whose memory the single ones share (else None)."""
 
-    def __init__(self, each: list[PackedWeight]):
-        self.each, self.n, self.k = each, each[0].n, each[0].k
-        self.w = torch.stack([pw.w for pw in each])
-        self.packed = torch.stack([pw.packed for pw in each]) if all(pw.packed is not None for pw in each) else None
-        for i, pw in enumerate(each):
-            pw.w = self.w[i]
-            if self.packed is not None:
-                pw.packed = self.packed[i]
+    def __init__(self, each: list[PackedWeight], w: torch.Tensor | None = None, packed: torch.Tensor | None = None):
+        self.each, self.w, self.packed = each, w, packed
+        self.n, self.k = each[0].n, each[0].k
 
 
 class Runtime:
@@ -474,8 +469,24 @@ class Runtime:
         return self.linear(x, pw.w, out_dtype)
 
     def stack(self, weights: list[torch.Tensor]) -> StackedWeights:
-        """Placed weights of one size, for ``linear_each``."""
-        return StackedWeights([self.pack(w) for w in weights])
+        """Weights of one size, for ``linear_each``: side by side for bfloat16 compute (moved there one by one); where no launch takes them
+        together (float32, the invariant mode, rows of no multiple of 8) each as it is placed."""
+        if any(w.shape != weights[0].shape for w in weights):
+            raise ShapeError(f"weights of {[list(w.shape) for w in weights]} are not of one size")
+        if self.dtype != torch.bfloat16 or self.invariant or weights[0].shape[1] % 8:
+            return StackedWeights([self.pack(self.place_matrix(w)) for w in weights])
+        w = torch.empty((len(weights), *weights[0].shape), dtype=self.dtype, device=self.device)
+        each, packed = [], None
+        for i, one in enumerate(weights):
+            w[i].copy_(self.place_matrix(one))
+            pw = self.pack(w[i])
+            if pw.packed is not None:                    # (by size: all have one or none has)
+                if packed is None:
+                    packed = torch.empty((len(weights), *pw.packed.shape), dtype=pw.packed.dtype, device=pw.packed.device)
+                packed[i].copy_(pw.packed)
+                pw.packed = packed[i]
+            each.append(pw)
+        return StackedWeights(each, w, packed)
 
     def linear_each(self, x: torch.Tensor, weights: StackedWeights) -> list[torch.Tensor]:
         """``x[i] @ w[i].T`` of ``x [count, m, k]`` in the compute dtype: 2 to 16 rows in one launch of the packed kernel, prompts in one of the

@@ -60,7 +60,7 @@ class TimeMix(Mixer):
         if weights[n["w1"]].shape[0] != weights[n["w2"]].shape[1]:
             raise ConfigError(f"{n['w1']} has {weights[n['w1']].shape[0]} rows, {n['w2']} {weights[n['w2']].shape[1]} columns")
         self.mu = torch.stack([rt.place_gain(weights[n["mu_" + s]]) for s in self.MIXES], 0).contiguous()
-        self.w_rkvg = rt.stack([rt.place_matrix(weights[n[x]]) for x in ("r", "k", "v", "g")])
+        self.w_rkvg = rt.stack([weights[n[x]] for x in ("r", "k", "v", "g")])
         self.w = {x: rt.pack(rt.place_matrix(weights[n[x]])) for x in ("w1", "w2")}
         self.w0, self.u = rt.place_gain(weights[n["w0"]]), rt.place_gain(weights[n["u"]]).reshape(-1).contiguous()
         self.gain = rt.place_gain(weights[n["norm"]])

@@ -28,14 +28,18 @@ def ops():
     return ops
 
 
-@pytest.fixture(scope="module")
-def rt(ops):
+def runtime_of(dtype, invariant=False):
     from rust_inference_amd.parts import Runtime
     if not EMULATED:
-        return Runtime(DEV, torch.bfloat16)
+        return Runtime(DEV, dtype, invariant)
     made = Runtime.__new__(Runtime)                          # (a runtime refuses to be made for the CPU)
-    made.device, made.dtype, made.invariant, made._mm_out_dtype = torch.device(DEV), torch.bfloat16, False, None
+    made.device, made.dtype, made.invariant, made._mm_out_dtype = torch.device(DEV), dtype, invariant, None
     return made
+
+
+@pytest.fixture(scope="module")
+def rt(ops):
+    return runtime_of(torch.bfloat16)
 
 
 def t(a, dtype=torch.float32):
@@ -312,6 +316,31 @@ def test_experts_of_prompts_in_one_launch(ops, rt, monkeypatch, kind):
         want[mine] += 0.5 * (act @ w[f"e{e}.down"].T)
     assert rel_to_max(out, want) < 2e-2
     assert len(calls) == 2
+
+
+@pytest.mark.parametrize("m", [1, 3, 20])
+@pytest.mark.parametrize("mode", ["bfloat16", "invariant", "float32"])
+def test_weights_of_one_size_in_the_storage_they_come_in(ops, mode, m):
+    """Weights that go together, some stored in bfloat16 and some in float32: the bits of each alone; the float32 path keeps every one in
+    its own storage, bfloat16 has them side by side."""
+    rt = runtime_of(torch.float32 if mode == "float32" else torch.bfloat16, mode == "invariant")
+    rng = np.random.default_rng(m)
+    n, k, stored = 48, 264, (torch.bfloat16, torch.float32, torch.bfloat16, torch.float32)
+    ws = [t(rng.normal(size=(n, k)) / np.sqrt(k), kind) for kind in stored]
+    x = t(rng.normal(size=(4, m, k)), rt.dtype)
+    together = rt.stack(ws)
+    assert [pw.w.dtype for pw in together.each] == (list(stored) if mode == "float32" else [torch.bfloat16] * 4)
+    assert (together.w is not None) == (mode == "bfloat16") and (together.packed is None or mode == "bfloat16")
+    for got, one, w in zip(rt.linear_each(x, together), x, ws):
+        assert torch.equal(got, ops.as_rows(rt.linear_packed(one.contiguous(), rt.pack(rt.place_matrix(w)))))
+    from rust_inference_amd.errors import ShapeError
+    with pytest.raises(ShapeError):
+        rt.stack([ws[0], ws[1][:1]])
+    if mode != "invariant":                                  # (rows of no multiple of 8 are the library's, each matrix from an address of its own)
+        odd = [w[:, :13].contiguous() for w in ws]
+        assert rt.stack(odd).w is None
+        for got, one, w in zip(rt.linear_each(x[:, :, :13].contiguous(), rt.stack(odd)), x, odd):
+            assert rel_to_max(f64(got), f64(one)[:, :13] @ f64(w).T) < 1e-2
 
 
 @pytest.mark.parametrize("lie", ["side by side", "rows of longer ones", "x off a line", "w off a line", "w transposed", "x transposed", "results off a line",
