@@ -134,6 +134,7 @@ class OutputHead(Head):
     def bind(self, weights, rt):
         self.rt = rt
         self.weight = self.packed = None
+        self.no_room = False                        # the packed copy did not fit the memory
         if not self.tied and self.name in weights:
             self.weight = rt.place_matrix(weights[self.name])
 
@@ -165,9 +166,16 @@ class OutputHead(Head):
         logits (a decode step of as many sequences): at 151,936 x 4,096 the packed kernel takes 0.21 ms where
         the library's product takes 0.26 (1% of such a step), for 1.2 GB more memory.  It is made at the first
         such step, so that a model which never runs one (a single slot, or only larger batches) does not pay
-        for it; never while a graph is being captured (the engine runs every step once before it captures it)."""
-        if self.packed is None and not torch.cuda.is_current_stream_capturing():
-            self.packed = self.rt.pack(self.weight, always=True)
+        for it; never while a graph is being captured (the engine runs every step once before it captures it).
+        Where the cache has left no room for it the steps stay with the library's product, which needs none (the
+        invariant mode has no other product, and says so)."""
+        if self.packed is None and not self.no_room and not torch.cuda.is_current_stream_capturing():
+            try:
+                self.packed = self.rt.pack(self.weight, always=True)
+            except torch.OutOfMemoryError:
+                if self.rt.invariant:
+                    raise
+                self.no_room = True
         return self.packed
 
     # Rows of logits up to which the packed copy serves: 2 to 8 the packed kernel (one load of x serves two steps of

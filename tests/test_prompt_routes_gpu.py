@@ -1,5 +1,5 @@
 """Which kernels a prompt's parts choose, and that what they choose agrees with the plain functions: parts alone, at sizes that
-reach the kernels of long prompts.
+reach the kernels of long prompts; the same of products of a few rows with large matrices.
 
 Like tests/test_kernels_gpu.py these run without a GPU when the environment says RI_TEST_KERNELS=emulated
 (tests/test_kernels_emulated.py starts that run): the CPU build of the same sources."""
@@ -408,3 +408,42 @@ def test_the_rule_of_products_in_groups(monkeypatch):
     assert tile(9842, 8, 6144, 4128) is None and tile(9842, 8, 6148, 4096) is None and tile(9842, 8, 6144, 128) is None
     assert tile(9842, 8, 6144, 4096, 1 << 22) is None
     runtime._groups_tile.cache_clear()
+
+
+# ---------------------------------------------------------------- steps of a few rows
+# float32 sums of the library's product of bfloat16; on the CPU torch rounds them to bfloat16 first (half a unit in the eighth bit)
+LIBRARY_F32 = 2.0 ** -8 if EMULATED else 1e-5
+
+
+def output_head(rt, monkeypatch, vocab, dim, rng):
+    from rust_inference_amd.parts import PartSpec, build_part
+    head = build_part("head", PartSpec("linear", {"vocab": vocab, "dim": dim, "name": "head", "tied": False}))
+    w = torch.tensor(rng.normal(size=(vocab, dim)) / np.sqrt(dim)).to(torch.bfloat16)
+    head.bind({"head": w}, rt)
+    if EMULATED:
+        monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    return head, f64(w)
+
+
+@pytest.mark.parametrize("rows", [3, 20, 64])
+def test_output_matrix_without_room_for_a_second_copy(ops, monkeypatch, rows):
+    """The library's product then, and no second attempt; the invariant mode has no other product and says what is missing."""
+    rng = np.random.default_rng(rows)
+    x = t(rng.normal(size=(rows, 64)), torch.bfloat16)
+    for invariant in (False, True):
+        rt = runtime_of(torch.bfloat16, invariant)
+        head, w = output_head(rt, monkeypatch, 256 * 64, 64, rng)
+        monkeypatch.setattr(type(rt), "many_waves", staticmethod(lambda n, k, m: 8 if m > 16 else None))
+        tried = []
+
+        def full(*args, **kw):
+            tried.append(args)
+            raise torch.OutOfMemoryError("no room")
+        monkeypatch.setattr(rt, "pack", full)
+        if invariant:
+            with pytest.raises(torch.OutOfMemoryError):
+                head.forward(x)
+            continue
+        for _ in range(2):
+            assert rel_to_max(f64(head.forward(x)), f64(x) @ w.T) < LIBRARY_F32
+        assert len(tried) == 1
