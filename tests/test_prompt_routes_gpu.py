@@ -447,3 +447,39 @@ def test_output_matrix_without_room_for_a_second_copy(ops, monkeypatch, rows):
         for _ in range(2):
             assert rel_to_max(f64(head.forward(x)), f64(x) @ w.T) < LIBRARY_F32
         assert len(tried) == 1
+
+
+# results -> row tiles a workgroup on a machine of one compute unit, rows of 72: (9 and 16 rows of x, 17 to 48, 49 and 64); 0: not that kernel's choice
+MANY_TILES = {288: (0, 6, 6), 250: (0, 8, 8), 380: (0, 12, 12), 620: (20, 20, 20), 410: (0, 0, 0)}
+
+
+@pytest.mark.parametrize("rows", [9, 16, 17, 48, 49, 64, 65])
+@pytest.mark.parametrize("n", list(MANY_TILES))
+def test_products_of_many_row_tiles_are_sent_to_the_form_that_is_chosen(ops, rt, monkeypatch, n, rows):
+    """A plain matrix and an output matrix at the edges of the rows that each form takes: what the kernel is given, and float64.  Where the rule
+    has no form of many row tiles, a plain matrix has three or four from 17 to 48 rows, an output matrix four from 9 rows on, and others the rest."""
+    from rust_inference_amd.parts import runtime
+    runtime._wide_many_waves.cache_clear()
+    monkeypatch.setattr(runtime, "_compute_units", lambda: 1)
+    monkeypatch.setattr(runtime, "MID_MAX_BYTES", 0)           # (matrices of these sizes are the packed kernel's otherwise)
+    rng = np.random.default_rng(n + rows)
+    k = 72
+    head, w = output_head(rt, monkeypatch, n, k, rng)
+    x = t(rng.normal(size=(rows, k)), torch.bfloat16)
+    want = f64(x) @ w.T
+    many = 0 if rows > 64 else MANY_TILES[n][0 if rows <= 16 else 1 if rows <= 48 else 2]
+    wide = calls_of(monkeypatch, ops, "gemm_wide_packed_bf16")
+
+    plain = rt.pack(t(w, torch.bfloat16), always=True)
+    for dtype, bound in ((torch.bfloat16, 1e-2), (torch.float32, LIBRARY_F32)):
+        wide.clear()
+        assert rel_to_max(f64(rt.linear_packed(x, plain, out_dtype=dtype)), want) < bound
+        few = (3, 4) if 17 <= rows <= 48 else ()
+        assert [kw["waves"] for _, kw in wide] == ([many] if many and rows >= 17 else [runtime._wide_whole_waves(n, rows)] if few else [])
+        assert many or not wide or wide[0][1]["waves"] in few
+    wide.clear()
+    logits = head.forward(x)
+    assert logits.dtype == torch.float32 and rel_to_max(f64(logits), want) < LIBRARY_F32
+    assert [kw["waves"] for _, kw in wide] == ([many] if many else [4] if rows <= 48 else [])
+    assert (head.packed is not None) == bool(wide)
+    runtime._wide_many_waves.cache_clear()
