@@ -192,6 +192,7 @@ class OutputHead(Head):
     PACKED_MORE_ROWS = 48            # for rows of up to PACKED_MORE_DIM elements
     PACKED_MORE_DIM = 4096
     PAIRED_MAX_ROWS = 8
+    FEW_ROW_TILES = 4
 
     def forward(self, x):
         logits = self.uncapped(x)
@@ -204,7 +205,7 @@ class OutputHead(Head):
         most = self.PACKED_MORE_ROWS if self.dim <= self.PACKED_MORE_DIM else self.PACKED_MAX_ROWS
         many = None
         if self.PAIRED_MAX_ROWS < rows <= self.PACKED_MANY_ROWS and self.rt.dtype == torch.bfloat16:
-            many = self.rt.many_waves(self.vocab, self.dim, rows)
+            many = self.rt.many_waves(self.vocab, self.dim, rows, self.FEW_ROW_TILES)
             most = self.PACKED_MANY_ROWS if many else most
         if 2 <= rows <= most and self.dim % 8 == 0:
             packed = self._packed_copy()
@@ -212,7 +213,7 @@ class OutputHead(Head):
                 if rows <= self.PAIRED_MAX_ROWS:
                     return self.rt.linear_packed(x, packed, out_dtype=torch.float32)
                 return ops.gemm_wide_packed_bf16(self.rt.normed_now(x), packed.packed, self.vocab, torch.float32,
-                                                 depth=1, waves=many or 4)
+                                                 depth=1, waves=many or self.FEW_ROW_TILES)
         return self.rt.linear(x, self.weight, out_dtype=torch.float32)
 
 

@@ -47,7 +47,7 @@ SMALL_ONLY_ROWS = 64             # a matrix packed for small steps alone stays o
 WIDE_GATED_FILL = 0.75            # gate|up goes to the wide kernel where its workgroups fill this share of the rounds,
 WIDE_GATED_ROWS = 48             # and up to this many rows whatever they fill, if the packed kernel of 17 to 64 rows is no match:
 WIDE_GATED_BYTES = 64_000_000    # pairs larger than this (smaller ones, up to 32 tiled rows, are that kernel's)
-# 17 to 48 rows (to 64 where _wide_many_waves says so) against a plain matrix of many rows (all experts' gates and ups side by side: 4 row tiles a compute unit and
+# 17 to 48 rows (to 64 where _wide_many_waves below says so) against a plain matrix of many rows (all experts' gates and ups side by side: 4 row tiles a compute unit and
 # more): the wide kernel, K whole.  98,304 x 4,096 at 17 / 32 / 48 / 64 rows: 136 / 143 / 163 / 183 us against the library's 180 / 180 / 172 / 177;
 # 24,576 x 1,024: 13 / 15 / 17 / 20 against 32 / 32 / 18 / 18; 24,576 x 4,096 37 / 41 / 49 / 58 against 52 / 51 / 51 / 51; with fewer row
 # tiles level (12,288 x 4,096 at 32 rows 23 against 24).  Weights not in the caches, at 17 / 32 / 48 rows, the wide kernel : the library: 16,384 x 1,024
@@ -70,39 +70,58 @@ def _compute_units() -> int:
 
 
 # Row tiles a workgroup of the wide kernel with K whole: 3 or 4 (whole slices of x), or many in half slices, one a wavefront or (20) two.  A
-# compute unit fetches some 30 GB/s whatever it fetches, so the form is the one with which it fetches the fewest rows.  Many row tiles only where that saves a seventh, in a single round a fifth (few large workgroups
-# have a slow beginning and end: 32,768 x 4,096 at 32 rows, 0.83 of the rows, 56 us : 53), and a single round of them not for short rows (32,768 x 1,024 at 48 rows 19 : 17) nor
-# for up to 16 rows of x (24,576 x 4,096: 43.5 : 35.6).  us at 16 / 32 / 48 / 64 rows, many : three or four (the library, float32 results):
-# 151,936 x 4,096 in 20s 194 / 205 / 215 / 221 : 214 / 239 / 268 / 291 (259 / 270 / 267 / 274), x 1,024 57 / 61 / 65 / 69 : 60 / 67 / 74 / 85 (67 / 80 /
-# 82 / 86), x 5,120 238 / 261 / 268 / 279 : 262 / 302 / 342 / 377 (319 / 355 / 305 / 320); 98,304 x 4,096 in twelves from 32 rows on 142 / 146 / 144 : 151 /
-# 171 / 189 (166 / 178 / 183); 49,152 x 2,048 38 / 40 / 41 : 39 / 44 / 50 (49 / 49 / 54); 24,576 x 4,096 in sixes 39 / 38 / 46 : 40 / 48 / 58 (45 / 46 / 47).
-WIDE_MANY_TILES = (6, 8, 12, 20)
-WIDE_MANY_SAVES = 0.85
-WIDE_MANY_SAVES_ONE = 0.8        # in a single round, and there only for
-WIDE_MANY_MIN_K = 2048           # rows as long as this
+# compute unit fetches some 30 GB/s whatever it fetches, so the form is the one with which it fetches the fewest rows: of x (those that there are;
+# the rest of a tile comes from a kilobyte of zeros) for every round of workgroups, and of the matrix.  Many row tiles where their share of the
+# rows that three or four fetch is no more than below: in a single round (few large workgroups have a slow beginning and end), in several.  The limits are
+# where 1,800 sizes of 16,384 to 160,000 rows by 512 to 8,192 at 9 to 64 rows of x, weights from memory, stop gaining; 1,023 of them take many row tiles, 0.88 of
+# the time (at most 1.02 against three or four, 1.08 against the library).  us, many : three or four: 18,432 x 4,096 in sixes at 32 / 48 rows 34.5 : 35.9 / 32.3 : 42.5, at 17 (0.87
+# of the rows) 32.6 : 30.5; 73,728 x 4,096 in 20s at 17 / 32 93 : 104 / 95 : 111; 98,304 x 4,096 in twelves at 32 / 48 136 : 140 / 142 : 160; 151,936 in 20s,
+# float32 sums, at 9 / 16 / 32 / 48 / 64: x 4,096 188 / 193 / 204 / 215 / 221 : 203 / 212 / 237 / 265 / 287, x 1,024 51 / 53 / 58 / 63 / 66 : 52 / 56 / 64 / 72 / 80.
+WIDE_MANY = {6: (0.80, 0.88), 8: (0.83, 0.90), 12: (0.80, 0.86), 20: (0.92, 0.92)}
+# A single round not for up to 16 rows of x (24,576 x 4,096: 43.5 : 35.6) nor, but for 20s, for rows shorter than WIDE_MANY_MIN_K.  Eights whose rows are
+# a power of two of 1,024 to 4,096 elements lose whatever they fetch, below 4,096 always (65,536 x 2,048 at 17 / 32 / 48 rows 60 / 62 / 60 : 46 / 51 / 57; 20s of
+# it 46 / 49 / 50), at 4,096 past this share (65,536 at 17 rows, 0.90: 96 : 90).
+WIDE_MANY_MIN_K = 2048
+WIDE_EVEN_EIGHTS = 0.84
+# Past WIDE_PLAIN_ROWS the library takes the step otherwise.  With float32 results it is behind nearly everywhere (at 64 rows 151,936 x 4,096 221 : 267,
+# x 1,024 66 : 81; ahead at 50,304 x 5,120 105 : 100), with bfloat16 results ahead for short rows (57,344 x 1,024 32 : 26) and, but for the fewest rows fetched,
+# for rows past 4,096 (26,624 x 5,120 in eights 59 : 54, 122,880 x 5,120 in twelves 248 : 220; 81,920 x 5,120 in 20s 137 : 171).
+WIDE_LIBRARY_K = 4096
+WIDE_LIBRARY_SHARE = 0.70
 
 
 def _wide_rows(n: int, m: int, waves: int) -> tuple[int, int]:
     """Rounds of workgroups of that many row tiles, and the rows (of x and of the matrix) that a compute unit fetches in them."""
     rounds = -(-n // (16 * waves * _compute_units()))
-    return rounds, rounds * (-(-m // 16) * 16 + 16 * waves)
+    return rounds, rounds * (m + 16 * waves)
 
 
 def _wide_whole_waves(n: int, m: int) -> int:
     """Three or four row tiles a workgroup of the wide kernel with K whole: whichever has a compute unit fetch fewer rows (of
-    x for every round of workgroups, and of the matrix)."""
-    return 3 if _wide_rows(n, m, 3)[1] < _wide_rows(n, m, 4)[1] else 4
+    x in whole tiles for every round of workgroups, and of the matrix)."""
+    tiled = -(-m // 16) * 16
+    return 3 if _wide_rows(n, tiled, 3)[1] < _wide_rows(n, tiled, 4)[1] else 4
 
 
 @functools.lru_cache(maxsize=4096)
-def _wide_many_waves(n: int, k: int, m: int) -> int | None:
-    """Many row tiles a workgroup of the wide kernel with K whole (of WIDE_MANY_TILES), where they pay."""
-    few = _wide_rows(n, m, _wide_whole_waves(n, m))[1]
+def _wide_many_waves(n: int, k: int, m: int, wide_out: bool = False, few: int | None = None) -> int | None:
+    """Many row tiles a workgroup of the wide kernel with K whole (of WIDE_MANY), where they pay: against ``few`` (three or four by the rule
+    above), past WIDE_PLAIN_ROWS against the library's product with float32 (``wide_out``) or bfloat16 results."""
+    beside = _wide_rows(n, m, few or _wide_whole_waves(n, m))[1]
+    even = 1024 <= k <= 4096 and k & (k - 1) == 0
     best = None
-    for waves in WIDE_MANY_TILES:
+    for waves, limits in WIDE_MANY.items():
         rounds, rows = _wide_rows(n, m, waves)
-        one_ok = k >= WIDE_MANY_MIN_K and m > SKINNY_MAX_ROWS and rows <= WIDE_MANY_SAVES_ONE * few
-        if (one_ok if rounds == 1 else rows <= WIDE_MANY_SAVES * few) and (best is None or rows < best[0]):
+        limit = limits[rounds > 1]
+        if rounds == 1 and (m <= SKINNY_MAX_ROWS or (waves < 20 and k < WIDE_MANY_MIN_K)):
+            continue
+        if waves == 8 and even:
+            limit = min(limit, WIDE_EVEN_EIGHTS if k == 4096 else 0.0)
+        if m > WIDE_PLAIN_ROWS and not wide_out:
+            if k < WIDE_MANY_MIN_K or (k > WIDE_LIBRARY_K and waves < 12):
+                continue
+            limit = min(limit, WIDE_LIBRARY_SHARE) if k > WIDE_LIBRARY_K else limit
+        if rows <= limit * beside and (best is None or rows < best[0]):
             best = (rows, waves)
     return best[1] if best else None
 
@@ -276,9 +295,9 @@ class Runtime:
 
     # ---- products
     @staticmethod
-    def many_waves(n: int, k: int, m: int) -> int | None:
-        """``_wide_many_waves`` for parts that call the wide kernel themselves."""
-        return _wide_many_waves(n, k, m)
+    def many_waves(n: int, k: int, m: int, few: int) -> int | None:
+        """``_wide_many_waves`` for parts that call the wide kernel themselves, for float32 sums, with ``few`` row tiles otherwise."""
+        return _wide_many_waves(n, k, m, True, few)
 
     def linear(self, x: torch.Tensor, w: torch.Tensor, out_dtype=None) -> torch.Tensor:
         """``x @ w.T`` with float32 accumulation; no bias anywhere in this family
@@ -456,7 +475,7 @@ class Runtime:
                                                 tiled_out=tiled_out and out_dtype == torch.bfloat16)
             if (WIDE_MIN_ROWS <= m <= MID_MAX_ROWS and pw.packed is not None and not pw.swiglu and not pw.small_only
                     and pw.n >= 16 * WIDE_PLAIN_TILES * _compute_units()):
-                many = _wide_many_waves(pw.n, pw.k, m)
+                many = _wide_many_waves(pw.n, pw.k, m, out_dtype == torch.float32)
                 if many or m <= WIDE_PLAIN_ROWS:
                     x = self.normed_now(x) if later else x
                     return ops.gemm_wide_packed_bf16(x, pw.packed, pw.n, out_dtype, depth=1,

@@ -225,7 +225,7 @@ def test_products_of_one_size_together(m, dtype, monkeypatch):
 
 
 def test_many_row_tiles_of_a_whole_wide_product(monkeypatch):
-    """Many row tiles a workgroup where that saves a compute unit a fifth of the rows it fetches; not in a single round for few rows or short ones."""
+    """Many row tiles a workgroup where that saves a compute unit enough of the rows that it fetches; not in a single round for few rows or short ones."""
     from rust_inference_amd.parts import runtime
     monkeypatch.setattr(runtime, "_compute_units", lambda: 256)
     runtime._wide_many_waves.cache_clear()
@@ -236,6 +236,21 @@ def test_many_row_tiles_of_a_whole_wide_product(monkeypatch):
     assert [got[98304, 4096, m] for m in (16, 32, 64)] == [None, 12, 12]
     assert [got[32768, 4096, m] for m in (16, 32, 64)] == [None, None, 8]
     assert not any(got[n, k, m] for n, k in ((32768, 1024), (16384, 4096), (64, 4096)) for m in (16, 32, 64))
+
+
+def test_many_row_tiles_only_where_they_gain(monkeypatch):
+    """The rows of x that there are count, not those of whole tiles; eights not for short rows of a power of two; past 48 rows the library's product
+    stands beside, with bfloat16 results ahead for short and for long rows."""
+    from rust_inference_amd.parts import runtime
+    monkeypatch.setattr(runtime, "_compute_units", lambda: 256)
+    runtime._wide_many_waves.cache_clear()
+    many = runtime._wide_many_waves
+    assert [many(18432, 4096, m) for m in (17, 24, 31, 32, 48)] == [None, None, None, 6, 6]
+    assert [many(65536, k, 48) for k in (512, 1024, 1536, 2048, 4096)] == [8, 20, 8, 20, 8] and many(65536, 4096, 17) is None
+    assert many(57344, 1024, 64) is None and many(26624, 5120, 64) is None and many(122880, 5120, 64) is None
+    assert many(57344, 1024, 64, True, 4) and many(26624, 5120, 64, True, 4) and many(81920, 5120, 64) == 20
+    assert [many(98304, 4096, m) for m in (17, 18, 32, 64)] == [None, 12, 12, 12]
+    runtime._wide_many_waves.cache_clear()
 
 
 def test_tiled_rows_reach_every_kind_of_product():

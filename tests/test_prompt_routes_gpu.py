@@ -433,7 +433,7 @@ def test_output_matrix_without_room_for_a_second_copy(ops, monkeypatch, rows):
     for invariant in (False, True):
         rt = runtime_of(torch.bfloat16, invariant)
         head, w = output_head(rt, monkeypatch, 256 * 64, 64, rng)
-        monkeypatch.setattr(type(rt), "many_waves", staticmethod(lambda n, k, m: 8 if m > 16 else None))
+        monkeypatch.setattr(type(rt), "many_waves", staticmethod(lambda n, k, m, few: 8 if m > 16 else None))
         tried = []
 
         def full(*args, **kw):
@@ -449,13 +449,16 @@ def test_output_matrix_without_room_for_a_second_copy(ops, monkeypatch, rows):
         assert len(tried) == 1
 
 
-# results -> row tiles a workgroup on a machine of one compute unit, rows of 72: (9 and 16 rows of x, 17 to 48, 49 and 64); 0: not that kernel's choice
-MANY_TILES = {288: (0, 6, 6), 250: (0, 8, 8), 380: (0, 12, 12), 620: (20, 20, 20), 410: (0, 0, 0)}
+# (results, K) -> row tiles a workgroup on a machine of one compute unit: bfloat16 and float32 results at 17, 48, 49 and 64 rows, an output matrix at 9, 16
+# and those; 0: three or four up to 48 rows, then the library
+MANY_TILES = {(288, 72): ((20, 20, 0, 0), (20, 20, 20, 20), (6, 6, 20, 20, 20, 20)), (250, 72): ((8, 8, 0, 0), (8, 8, 8, 8), (0, 8, 8, 8, 8, 8)),
+              (250, 2056): ((8, 8, 8, 8), (8, 8, 8, 8), (0, 8, 8, 8, 8, 8)), (380, 72): ((8, 12, 0, 0), (8, 12, 12, 12), (0, 8, 8, 12, 12, 12)),
+              (620, 72): ((20, 20, 0, 0), (20, 20, 20, 20), (20,) * 6), (410, 72): ((0, 8, 0, 0), (0, 8, 8, 8), (0, 0, 0, 8, 8, 8))}
 
 
 @pytest.mark.parametrize("rows", [9, 16, 17, 48, 49, 64, 65])
-@pytest.mark.parametrize("n", list(MANY_TILES))
-def test_products_of_many_row_tiles_are_sent_to_the_form_that_is_chosen(ops, rt, monkeypatch, n, rows):
+@pytest.mark.parametrize("n, k", list(MANY_TILES))
+def test_products_of_many_row_tiles_are_sent_to_the_form_that_is_chosen(ops, rt, monkeypatch, n, k, rows):
     """A plain matrix and an output matrix at the edges of the rows that each form takes: what the kernel is given, and float64.  Where the rule
     has no form of many row tiles, a plain matrix has three or four from 17 to 48 rows, an output matrix four from 9 rows on, and others the rest."""
     from rust_inference_amd.parts import runtime
@@ -463,23 +466,23 @@ def test_products_of_many_row_tiles_are_sent_to_the_form_that_is_chosen(ops, rt,
     monkeypatch.setattr(runtime, "_compute_units", lambda: 1)
     monkeypatch.setattr(runtime, "MID_MAX_BYTES", 0)           # (matrices of these sizes are the packed kernel's otherwise)
     rng = np.random.default_rng(n + rows)
-    k = 72
     head, w = output_head(rt, monkeypatch, n, k, rng)
     x = t(rng.normal(size=(rows, k)), torch.bfloat16)
     want = f64(x) @ w.T
-    many = 0 if rows > 64 else MANY_TILES[n][0 if rows <= 16 else 1 if rows <= 48 else 2]
+    half, whole, logits = ({9: 0, 16: 0, 17: a[-4], 48: a[-3], 49: a[-2], 64: a[-1]}.get(rows, 0) for a in MANY_TILES[n, k])
+    logits = {9: MANY_TILES[n, k][2][0], 16: MANY_TILES[n, k][2][1]}.get(rows, logits)
     wide = calls_of(monkeypatch, ops, "gemm_wide_packed_bf16")
 
     plain = rt.pack(t(w, torch.bfloat16), always=True)
-    for dtype, bound in ((torch.bfloat16, 1e-2), (torch.float32, LIBRARY_F32)):
+    for dtype, bound, many in ((torch.bfloat16, 1e-2, half), (torch.float32, LIBRARY_F32, whole)):
         wide.clear()
         assert rel_to_max(f64(rt.linear_packed(x, plain, out_dtype=dtype)), want) < bound
-        few = (3, 4) if 17 <= rows <= 48 else ()
-        assert [kw["waves"] for _, kw in wide] == ([many] if many and rows >= 17 else [runtime._wide_whole_waves(n, rows)] if few else [])
-        assert many or not wide or wide[0][1]["waves"] in few
+        given = [kw["waves"] for _, kw in wide]
+        assert given == ([many] if many else [runtime._wide_whole_waves(n, rows)] if 17 <= rows <= 48 else [])
+        assert many or not given or given[0] in (3, 4)
     wide.clear()
-    logits = head.forward(x)
-    assert logits.dtype == torch.float32 and rel_to_max(f64(logits), want) < LIBRARY_F32
-    assert [kw["waves"] for _, kw in wide] == ([many] if many else [4] if rows <= 48 else [])
+    made = head.forward(x)
+    assert made.dtype == torch.float32 and rel_to_max(f64(made), want) < LIBRARY_F32
+    assert [kw["waves"] for _, kw in wide] == ([logits] if logits else [4] if rows <= 48 else [])
     assert (head.packed is not None) == bool(wide)
     runtime._wide_many_waves.cache_clear()
