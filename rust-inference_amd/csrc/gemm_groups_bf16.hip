@@ -4,9 +4,10 @@
 // A launch an expert is a round of tiles an expert, and its last tiles fill a part of the machine: of eight experts with some 1,230 rows each
 // (4,921 tokens, two experts a token; 6,144 x 4,096 gates and ups, 4,096 x 6,144 downs) gates and ups are 240 tiles a launch of 256 places, downs
 // 80, which the library cuts into smaller ones (69 to 72 us each, 0.86 PFLOP/s).  Workgroups that stay go from one group's tiles to the next one's
-// here, so only the last round of all is partly filled: gates and ups with the activation 734 us (8 launches 780), downs 436 (8 of the library's
-// 560; 392 where an expert's matrix lies in one piece and not, as the mixture's does, in rows 98,304 bytes apart).  Where a group's rows begin is read from memory, where the sort has left it: the host need
-// not know.
+// here, so only the last round of all is partly filled: gates and ups with the activation 756 us (8 launches 772, the
+// library's and an activation kernel 870), downs 414 (8 of the library's 551; 398 where an expert's matrix lies in one piece and not, as the mixture's
+// does, in rows 98,304 bytes apart); inside the model 729 and 419.  Where a group's rows begin is read from memory, where the sort has left it: the
+// host need not know.
 #include "gemm_tiles.h"
 
 template <int TM, int TN, int ACT>

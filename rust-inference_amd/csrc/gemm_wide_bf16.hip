@@ -31,8 +31,8 @@
 // bound, some 30 GB/s from memory and L2 cache together, and with four row tiles a workgroup of 64 rows half of it is x.
 // So six to twelve wavefronts share a copy of x, or ten with two row tiles each, in half slices: a workgroup's two
 // buffers of 64 rows are 32 KB then and two or three workgroups a compute unit cover one another's barriers, a wavefront
-// has four fragments (PAIR: eight) in flight.  151,936 x 4,096 at 64 rows: 221 us (5.6 TB/s of weights) in tens of pairs, 291
-// in fours, the library with float32 results 274; at 32 rows 205 : 239 : 270.  The sums are the same bits in every form.
+// has four fragments (PAIR: eight) in flight.  151,936 x 4,096 at 64 rows: 221 us (5.6 TB/s of weights) in tens of pairs, 287
+// in fours, the library with float32 results 267; at 32 rows 204 : 237 : 269.  The sums are the same bits in every form.
 #include "api.h"
 #include "common.h"
 

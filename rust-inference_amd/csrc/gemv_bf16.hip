@@ -211,7 +211,8 @@ gemv_bf16_kernel(TO* __restrict__ out, const bf16_t* __restrict__ x, const bf16_
 // above, bit for bit: in PARTS parts of a row, the first of (STEPS + 1) / 2 pieces if there are two.
 // us, weights from memory, with the norm of x left to it where the model leaves it, before : now: gate and up 3,072 x 1,024 6.4 : 5.0, 6,144 x 2,048
 // 13.6 : 10.7, 9,728 x 2,560 19.0 : 17.9, 12,288 x 4,096 33.6 : 32.6, 25,600 x 5,120 81 : 78; plain 1,024 x 2,048 3.5 : 2.9, 1,024 x 3,072 4.2 : 3.3, 4,096 x 1,024
-// 4.8 : 4.3, 6,144 x 2,560 11.3 : 8.2, 4,096 x 4,096 7.9 : 7.7, 151,936 x 1,024 56 : 48 (6.5 TB/s).  Rows of 6,144 and more are level.
+// 4.8 : 4.3, 6,144 x 2,560 11.3 : 8.2, 4,096 x 4,096 7.9 : 7.7, 151,936 x 1,024 56 : 48 (6.5 TB/s); few rows too, 64 x 1,024 2.5 : 2.2, 16 x 4,096
+// 2.9 : 2.4, though a matrix then has half the wavefronts.  Rows of 6,144 and more are level.
 // An empty launch takes 1.6 us of a chain: what bounds the small ones is that, a trip to memory, and the end of the launch.
 #define GV_ONE_STEPS 10
 

@@ -146,7 +146,8 @@ class RoutedExperts(FeedForward):
     # (one wavefront an output row: every assignment streams its expert's matrices once, so with as many assignments
     # as experts it would read what all experts hold); from SORTED_MIN_TOKENS tokens on a prompt's assignments are
     # sorted by expert and every expert is two products over its own rows (from four experts on of one launch for all, see grouped_tiles); between them, and in float32, all
-    # experts are computed for all tokens as two products, with zeros where a token did not choose.
+    # experts are computed for all tokens as two products, with zeros where a token did not choose.  The number, and the refusal
+    # under capture, are those of a launch an expert, for which the host waits.
     SORTED_MIN_TOKENS = 256
 
     def route(self, x, ctx):

@@ -181,12 +181,13 @@ class OutputHead(Head):
     # Rows of logits up to which the packed copy serves: 2 to 8 the packed kernel (one load of x serves two steps of
     # K there); from 9 on the wide kernel with four row tiles a workgroup, which shares the rows of x through LDS
     # (151,936 x 4,096 at 9, 16, 17 and 32 rows: 204, 213, 222 and 247 us against the packed kernel's 224 and 279
-    # and the library's 250 to 279; x 1,024 at 16 rows 57 against 78; x 5,120: 254 against 382; from 48 rows on the
-    # library is ahead, 266 against 279 us, with 39 MB of float32 logits to write).  33 to 48 rows with three tiles of
+    # and the library's 250 to 279; x 1,024 at 16 rows 57 against 78; x 5,120: 254 against 382; with four row tiles the
+    # library is ahead from 48 rows on, 257 against 265 us, with 29 MB of float32 logits to write).  33 to 48 rows with three tiles of
     # x, for rows of up to 4,096 elements: eight layers and this matrix at 33 / 40 / 47 sequences are 1.5 / 1.5 / 0.9%
     # shorter at Qwen3-0.6B sizes, 3.7 / 2.8 / 1.8% at 4B, 1.2 / 0.8 / 0% at 8B; with rows of 5,120 (32B) 0 to 0.7% longer.
-    # Vocabularies that many row tiles a workgroup serve better (parts/runtime.py has the figures) stay with the
-    # packed copy up to 64 rows: 151,936 x 4,096 at 64 rows 221 us against the library's 274.
+    # Vocabularies that many row tiles a workgroup serve better (parts/runtime.py has the rule and the figures; 151,936 in
+    # twenties, 32,768 x 4,096 in eights from 33 rows on, 32,768 x 1,024 never) take those, and stay with the packed copy up
+    # to 64 rows: 151,936 x 4,096 at 48 rows 215 us, at 64 rows 221 against the library's 267.
     PACKED_MANY_ROWS = 64
     PACKED_MAX_ROWS = 32
     PACKED_MORE_ROWS = 48            # for rows of up to PACKED_MORE_DIM elements

@@ -179,10 +179,11 @@ def _tiles_plan(m: int, n: int, k: int, wide_out: bool, activation: str | None) 
 
 
 # The same for rows in groups, a matrix each, in one launch (ops.gemm_tiles_groups), from four groups on (fewer fill the machine one by one).
-# us, in one launch : the library's product and the activation a group; rows in eight groups: 9,842; gate and up 6,144 x 4,096 761 : 847, down 4,096 x 6,144
-# 436 : 562; 2,048; the same 264 : 399 and 211 : 273; 512; 192 : 242 and 134 : 180; gate and up 1,536 x 1,024, down 1,024 x 1,536, 4,096 rows 30 : 113 and 34 : 71,
-# 512 18 : 90 and 20 : 60; in 64 groups, 1,024 rows 81 : 754 and 36 : 437.  The host does not know how the rows are shared out: half a tile a group more than
-# they fill, for the choice of the tile.  The smaller takes 0.6 to 0.72 of the larger's time (9,842 rows: 861 : 761 us and 521 : 436; 512: 192 : 212, 18 : 26).
+# us, in one launch : the library's product and the activation a group; rows in eight groups: 9,842; gate and up 6,144 x 4,096 756 : 870, down 4,096 x 6,144
+# 414 : 551; 2,048; the same 222 : 431 and 138 : 239; 512; 187 : 229 and 113 : 178; gate and up 1,536 x 1,024, down 1,024 x 1,536, 4,096 rows 30 : 113 and 34 : 71,
+# 512 18 : 90 and 20 : 60; in 64 groups, 1,024 rows 81 : 754 and 36 : 437.  Whole mixtures of 4 to 64 experts of drawn sizes, even and skewed, 256 to 5,900 tokens: 0.02
+# (launches of the host) to 0.93 of an expert a launch.  The host does not know how the rows are shared out: half a tile a group more than
+# they fill, for the choice of the tile.  A round of the smaller takes 0.53 to 0.75 of the larger's time where tiles are full (9,842 rows, 15 : 8 rounds 866 : 756 us, 5 : 3 rounds 493 : 414).
 GROUPS_LEAST = 4
 GROUPS_SMALLER = 0.68
 
